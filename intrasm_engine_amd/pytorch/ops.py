@@ -366,10 +366,12 @@ def _spmm(b, row_indices, values, row_offsets, column_indices, m, *, per_batch_v
         # the density only; what the first look at the pattern found about its structure decides here
         share = _known_dense_share(row_offsets, column_indices, k)
         if share is not None and batch * m * k >= (1 << 25):
-            force_variant = 10 if share >= _STRUCTURE_SHARE else 1
-            if force_variant == 10 and _lib.load().iex_spmm_workspace_kind(
-                    _DT[b.dtype], _IT[column_indices.dtype], _lib.SPMM_PER_BATCH_VALUES | (10 << 16), m, k, n, nonzeros, batch) != 10:
-                force_variant = 0      # (the kernel does not serve this call: another n, int16 indices)
+            kind = lambda variant: _lib.load().iex_spmm_workspace_kind(
+                _DT[b.dtype], _IT[column_indices.dtype], _lib.SPMM_PER_BATCH_VALUES | (variant << 16), m, k, n, nonzeros, batch)
+            if share >= _STRUCTURE_SHARE:
+                force_variant = 10 if kind(10) == 10 else 0      # (0: the kernel does not serve this call: another n, int16 indices)
+            elif kind(0) == 10:
+                force_variant = 1      # (only where the density rule would have picked that kernel: every other choice stays the library's)
     flags = (_lib.SPMM_PER_BATCH_VALUES if per_batch_values else 0) | (_lib.SPMM_ANY_COLUMN_ORDER if any_order else 0) | \
             (_lib.SPMM_BESIDE_GATHER_KERNEL if beside_gather else 0) | \
             (_lib.SPMM_ACCUMULATE if accumulate else 0) | (_lib.SPMM_RELU if relu else 0) | \
@@ -508,9 +510,13 @@ def _sddmm(a, b, row_indices, row_offsets, column_indices, *, sum_over_batch, dt
         # per-entry SDDMM = attention scores: by the pattern's structure where a look at it has told, not by its density
         share = _known_dense_share(row_offsets, column_indices, n)
         if share is not None and batch * m * n >= (1 << 25):
-            force_variant = 3 if share >= _STRUCTURE_SHARE else 1
-            if force_variant == 3 and _lib.load().iex_sddmm_workspace_kind(_DT[a.dtype], 3 << 16, m, k, n, nonzeros, batch) != 3:
-                force_variant = 0      # (the kernel does not serve this call: another k)
+            kind = lambda variant: _lib.load().iex_sddmm_workspace_kind(_DT[a.dtype], variant << 16, m, k, n, nonzeros, batch)
+            if share >= _STRUCTURE_SHARE:
+                force_variant = 3 if kind(3) == 3 else 0      # (0: the kernel does not serve this call: another k)
+            elif kind(0) == 3:
+                # only where the density rule would have picked that kernel: a long k (the gradient of a pruned weight:
+                # 11008 x 4096 at 90 %, k = 2048, fp16) keeps the dense product, 1691 -> 230 us
+                force_variant = 1
     flags = (_lib.SDDMM_SUM_OVER_BATCH if sum_over_batch else 0) | (_lib.SDDMM_ANY_COLUMN_ORDER if any_order else 0) | \
             (_lib.SDDMM_ACCUMULATE if accumulate else 0) | ((int(force_wpr) & 0xff) << 8) | \
             ((int(force_variant) & 0xf) << 16)
