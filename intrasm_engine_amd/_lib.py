@@ -38,6 +38,7 @@ SIGNATURES = {
     "iex_last_error": (_c.c_char_p, []),
     "iex_last_kernels": (_c.c_char_p, []),
     "iex_device_ok": (_i, []),
+    "iex_gather_values": (_i, [_i, _i, _vp, _vp, _vp, _vp]),
     "iex_copy_bytes": (_i, [_vp, _vp, _c.c_size_t, _vp]),
     "iex_spmm_ex": (_i, [_i, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "iex_spmm_ws": (_i, [_i, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _c.c_size_t]),

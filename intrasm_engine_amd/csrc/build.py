@@ -18,7 +18,7 @@ def build(force: bool = True, jobs: int = 8) -> str:
         sys.stderr.write("\n".join(lines) + "\n")
         raise RuntimeError("building libiex_hip.so failed")
     out = os.path.normpath(os.path.join(HERE, "..", "libiex_hip.so"))
-    assert os.path.exists(out)
+    assert os.path.exists(out) and os.path.exists(os.path.join(os.path.dirname(out), "_iex_host.so"))
     return out
 
 

@@ -52,6 +52,21 @@ __global__ __launch_bounds__(256) void copy_kernel(uint4* __restrict__ dst, cons
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) dst[i] = src[i];
 }
 
+// out[i] = values[index[i]]: four elements per thread, so that the 8-byte indices come as 16-byte loads and four gathers
+// are in flight; the gathers themselves hit L2 (the values of one matrix).  4.5 M fp16 values: 38 us by torch's indexing.
+template <typename E>
+__global__ __launch_bounds__(256) void gather_values_kernel(int n, const E* __restrict__ values, const long long* __restrict__ index, E* __restrict__ out) {
+  struct alignas(sizeof(E) * 4) Four { E v[4]; };
+  struct alignas(16) Two { long long v[2]; };
+  const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i + 4 <= n) {
+    const Two a = *reinterpret_cast<const Two*>(index + i), b = *reinterpret_cast<const Two*>(index + i + 2);
+    *reinterpret_cast<Four*>(out + i) = Four{{values[a.v[0]], values[a.v[1]], values[b.v[0]], values[b.v[1]]}};
+  } else {
+    for (int j = i; j < n; ++j) out[j] = values[index[j]];
+  }
+}
+
 // What is wrong with a CSR pattern, as bits ORed into *status: one wavefront per row.
 template <typename IT>
 __global__ __launch_bounds__(256) void csr_check_kernel(int m, int k, int nnz, const int* __restrict__ row_offsets, const IT* __restrict__ cols,
@@ -251,6 +266,21 @@ int iex_csr_row_histogram(int m, const int* row_offsets, int* histogram, void* s
   if (m == 0) return 0;
   hipLaunchKernelGGL(csr_row_histogram_kernel, dim3((m + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), m, row_offsets, histogram);
   return iex::check_hip(hipGetLastError(), "csr_row_histogram launch");
+}
+
+int iex_gather_values(int elem_bytes, int n, const void* values, const long long* index, void* out, void* stream) {
+  IEX_REQUIRE(elem_bytes == 2 || elem_bytes == 4, IEX_ERR_UNSUPPORTED, "gather_values: elements of 2 or 4 bytes (got %d)", elem_bytes);
+  IEX_REQUIRE(n >= 0 && n < (1 << 31) - 1024, IEX_ERR_BAD_ARGUMENT, "gather_values: bad number of elements");
+  if (n == 0) return 0;
+  IEX_REQUIRE(values && index && out && iex::aligned(index, 16) && iex::aligned(out, 16), IEX_ERR_BAD_ARGUMENT,
+              "gather_values: null pointer argument, or indices or output not 16-byte aligned");
+  const dim3 grid((n + 1023) / 1024);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (elem_bytes == 2)
+    hipLaunchKernelGGL(gather_values_kernel<uint16_t>, grid, dim3(256), 0, s, n, static_cast<const uint16_t*>(values), index, static_cast<uint16_t*>(out));
+  else
+    hipLaunchKernelGGL(gather_values_kernel<uint32_t>, grid, dim3(256), 0, s, n, static_cast<const uint32_t*>(values), index, static_cast<uint32_t*>(out));
+  return iex::check_hip(hipGetLastError(), "gather_values launch");
 }
 
 int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream) {

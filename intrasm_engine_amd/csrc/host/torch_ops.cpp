@@ -1,0 +1,371 @@
+// The operators' calls as native code: what stands between torch.ops.iex_ops.* (and the autograd functions built on
+// them) and the C entry points of libiex_hip.so.
+//
+// Small products are bound by the host: 1024 x 1024 at 90 %, n = 256 runs 7 us on the GPU, and a call whose checks,
+// allocation and launch are Python took 18.  So the call everybody makes -- operands that fit, a pattern that has been
+// looked at before, nothing forced -- is served here; everything else (operands to refuse, with the texts of the
+// checks; a pattern's first look; kernel choices forced by ops.kernel_params; plans) goes to the Python functions of
+// pytorch/ops.py, which stay the one place that raises and that looks at patterns.
+//
+// A pattern's note (what ops._look found) is kept here as well as on the column_indices tensor object: by the tensor's
+// address, with weak references to both index tensors and their version counters, so that a note never outlives its
+// tensors or passes for another pattern's, and keeps no memory of theirs alive.
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/utils/pybind.h>
+#include <torch/library.h>
+
+#include <array>
+#include <mutex>
+#include <optional>
+#include <shared_mutex>
+#include <unordered_map>
+
+#include "../../../include/iex_hip.h"
+
+namespace py = pybind11;
+using at::Tensor;
+
+namespace {
+
+// ---- the Python side -----------------------------------------------------------------------------------------
+// (leaked on purpose: they are used until the interpreter ends)
+py::object* python_ops = nullptr;   // the functions of pytorch/ops.py by operator name
+
+thread_local bool forced = false;   // an ops.kernel_params block is active on this thread
+
+template <typename Result, typename... Args>
+Result ask_python(const char* name, const Args&... args) {
+  py::gil_scoped_acquire gil;
+  TORCH_CHECK(python_ops, "iex_ops: the package has not been initialised");
+  return py::cast<Result>((*python_ops)[name](args...));
+}
+
+void check(int rc, const char* what) {
+  TORCH_CHECK(rc == 0, what, ": ", iex_last_error(), " (code ", rc, ")");
+}
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+// ---- notes about patterns --------------------------------------------------------------------------------------
+typedef c10::weak_intrusive_ptr<c10::TensorImpl> Weak;
+struct Note {
+  Weak columns, offsets;
+  int64_t columns_version, offsets_version, k;
+  int status;
+  bool has_histogram;
+  std::array<int, 16> histogram;
+  double dense_share;   // < 0: not known
+  Weak tables;          // of the kernels for patterns with structure; may be gone
+};
+struct Known {   // what a call needs of it
+  int status;
+  bool has_histogram;
+  std::array<int, 16> histogram;
+  double dense_share;
+  Tensor tables;
+};
+
+std::shared_mutex notes_mutex;
+std::unordered_map<const c10::TensorImpl*, Note>& notes() {
+  static auto* map = new std::unordered_map<const c10::TensorImpl*, Note>;   // (outlives every tensor)
+  return *map;
+}
+size_t notes_sweep_at = 256;
+
+int64_t version_of(const Tensor& t) { return t.is_inference() ? 0 : t._version(); }
+
+void set_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k, int status, const std::optional<std::vector<int>>& histogram,
+              const std::optional<double>& dense_share, const std::optional<Tensor>& tables) {
+  Note n{Weak(column_indices.getIntrusivePtr()), Weak(row_offsets.getIntrusivePtr()), version_of(column_indices), version_of(row_offsets), k, status,
+         histogram.has_value(), {}, dense_share.value_or(-1.0),
+         Weak(tables.has_value() ? tables->getIntrusivePtr() : c10::intrusive_ptr<c10::TensorImpl, c10::UndefinedTensorImpl>())};
+  if (histogram) std::copy_n(histogram->begin(), 16, n.histogram.begin());
+  std::unique_lock lock(notes_mutex);
+  auto& map = notes();
+  if (map.size() >= notes_sweep_at) {   // notes of tensors that are gone
+    for (auto it = map.begin(); it != map.end();) it = it->second.columns.expired() ? map.erase(it) : std::next(it);
+    notes_sweep_at = std::max<size_t>(256, 2 * map.size());
+  }
+  map.insert_or_assign(column_indices.unsafeGetTensorImpl(), std::move(n));
+}
+
+std::optional<Known> note_of(const Tensor& row_offsets, const Tensor& column_indices, int64_t k) {
+  std::shared_lock lock(notes_mutex);
+  const auto& map = notes();
+  const auto it = map.find(column_indices.unsafeGetTensorImpl());
+  if (it == map.end()) return {};
+  const Note& n = it->second;
+  // (a weak reference that has not expired holds the address: nobody else can have it)
+  if (n.k != k || n.columns.expired() || n.offsets.expired() || n.offsets._unsafe_get_target() != row_offsets.unsafeGetTensorImpl() ||
+      n.columns_version != version_of(column_indices) || n.offsets_version != version_of(row_offsets))
+    return {};
+  Known known{n.status, n.has_histogram, n.histogram, n.dense_share, Tensor()};
+  if (auto alive = n.tables.lock()) known.tables = Tensor(std::move(alive));
+  return known;
+}
+
+// ---- operands that fit -------------------------------------------------------------------------------------------
+int dtype_code(at::ScalarType t) { return t == at::kFloat ? IEX_F32 : t == at::kHalf ? IEX_F16 : t == at::kBFloat16 ? IEX_BF16 : -1; }
+
+bool plain(const Tensor& t, int64_t dim) { return t.is_cuda() && t.layout() == at::kStrided && t.dim() == dim && t.is_contiguous(); }
+
+bool plain_csr(const Tensor& row_indices, const Tensor& row_offsets, const Tensor& column_indices, const Tensor& with, int64_t m) {
+  return plain(row_indices, 1) && plain(row_offsets, 1) && plain(column_indices, 1) && row_indices.scalar_type() == at::kInt &&
+         row_offsets.scalar_type() == at::kInt && row_indices.size(0) == m && row_offsets.size(0) == m + 1 && column_indices.size(0) > 0 &&
+         row_indices.device() == with.device() && row_offsets.device() == with.device() && column_indices.device() == with.device();
+}
+
+constexpr int kBadPattern = IEX_CSR_BAD_OFFSETS | IEX_CSR_COLUMN_OUT_OF_RANGE;
+// Patterns of attention-sized products with at least this share of their nonzeros in dense 128 x 128 blocks go to the
+// kernels for patterns with structure (ops._STRUCTURE_SHARE).
+constexpr double kStructureShare = 0.5;
+constexpr double kStructureCells = 1 << 25;
+
+Tensor workspace(size_t bytes, const Tensor& like) {
+  return bytes ? at::empty({(int64_t)bytes}, like.options().dtype(at::kByte)) : Tensor();
+}
+
+// ---- SpMM ----------------------------------------------------------------------------------------------------------
+enum class Spmm { kSharedF32, kSharedHalf, kPerEntry, kAtomic };
+
+const char* spmm_name(Spmm kind) {
+  switch (kind) {
+    case Spmm::kSharedF32: return "spmm_sputnik_reuse_weight";
+    case Spmm::kSharedHalf: return "spmm_sputnik_reuse_weight_half";
+    case Spmm::kPerEntry: return "spmm_sputnik_batched_values";
+    default: return "spmm_sputnik_atomic";
+  }
+}
+
+// flat: b is (k, n) and the result (m, n), without the batch dimension
+template <Spmm kind, bool flat = false>
+Tensor spmm(const Tensor& b, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m) {
+  constexpr bool per_entry = kind == Spmm::kPerEntry || kind == Spmm::kAtomic, accumulate = kind == Spmm::kAtomic;
+  auto python = [&] {
+    const Tensor out = ask_python<Tensor>(spmm_name(kind), flat ? b.unsqueeze(0) : b, row_indices, values, row_offsets, column_indices, m);
+    return flat ? at::_unsafe_view(out, {out.size(1), out.size(2)}) : out;
+  };
+  if (forced || !plain(b, flat ? 2 : 3) || !plain(values, per_entry ? 2 : 1) || values.device() != b.device() || values.scalar_type() != b.scalar_type() ||
+      !plain_csr(row_indices, row_offsets, column_indices, b, m))
+    return python();
+  const int dtype = dtype_code(b.scalar_type());
+  const bool i16 = column_indices.scalar_type() == at::kShort;
+  const bool type_fits = kind == Spmm::kPerEntry ? dtype >= 0 : kind == Spmm::kSharedHalf ? (dtype == IEX_F16 || dtype == IEX_BF16) : dtype == IEX_F32;
+  const bool index_fits = i16 ? dtype == IEX_F16 : column_indices.scalar_type() == at::kInt;
+  const int64_t batch = flat ? 1 : b.size(0), k = b.size(-2), n = b.size(-1), nonzeros = column_indices.size(0);
+  const bool shape_fits = values.size(-1) == nonzeros && (!per_entry || values.size(0) == batch) && (!accumulate || batch == 1 || nonzeros % 4 == 0);
+  if (!type_fits || !index_fits || !shape_fits || batch * m * n == 0) return python();
+  const auto known = note_of(row_offsets, column_indices, k);
+  if (!known || (known->status & kBadPattern)) return python();
+  const bool any_order = known->status & IEX_CSR_NOT_ASCENDING;
+  const int itype = i16 ? IEX_I16 : IEX_I32;
+  int flags = (per_entry ? IEX_SPMM_PER_BATCH_VALUES : 0) | (accumulate ? IEX_SPMM_ACCUMULATE : 0) | (any_order ? IEX_SPMM_ANY_COLUMN_ORDER : 0);
+  auto kind_of = [&](int f) { return iex_spmm_workspace_kind(dtype, itype, f, m, k, n, nonzeros, batch); };
+  if (kind == Spmm::kPerEntry && !any_order && dtype != IEX_F32 && known->dense_share >= 0 && (double)batch * m * k >= kStructureCells) {
+    // by the pattern's structure where a look at it has told, not by its density (the library's rule)
+    if (known->dense_share >= kStructureShare) flags |= kind_of(flags | IEX_SPMM_FORCE_VARIANT(10)) == 10 ? IEX_SPMM_FORCE_VARIANT(10) : 0;
+    else if (kind_of(flags) == 10) flags |= IEX_SPMM_FORCE_VARIANT(1);
+  }
+  const c10::DeviceGuard guard(b.device());
+  const int64_t shape[3] = {batch, m, n};
+  const at::IntArrayRef out_shape(shape + flat, 3 - flat);
+  Tensor out = accumulate ? at::zeros(out_shape, b.options()) : at::empty(out_shape, b.options());
+  const size_t ws_bytes = iex_spmm_workspace_bytes(dtype, itype, flags, m, k, n, nonzeros, batch);
+  Tensor ws;
+  if (ws_bytes && kind_of(flags) == 10) {
+    if (!known->tables.defined() || (size_t)known->tables.numel() < ws_bytes) return python();   // (it makes them)
+    ws = known->tables;
+    flags |= IEX_SPMM_TABLES_READY | IEX_SPMM_LISTS_READY;
+  } else {
+    ws = workspace(ws_bytes, b);
+  }
+  check(iex_spmm_sched(dtype, itype, flags, m, k, n, nonzeros, row_indices.const_data_ptr<int>(), values.const_data_ptr(),
+                       row_offsets.const_data_ptr<int>(), column_indices.const_data_ptr(), b.const_data_ptr(), nullptr, out.data_ptr(), stream_of(b),
+                       batch, ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, known->has_histogram ? known->histogram.data() : nullptr),
+        "spmm");
+  return out;
+}
+
+// ---- SDDMM ---------------------------------------------------------------------------------------------------------
+// flat: a is (m, k), b (n, k) and the result (nnz), without the batch dimension
+template <bool summed, bool flat = false>
+Tensor sddmm(const Tensor& a, const Tensor& b, const Tensor& row_indices, const Tensor& row_offsets, const Tensor& column_indices) {
+  auto python = [&] {
+    const Tensor out = ask_python<Tensor>(summed ? "sddmm_sputnik_atomic_upd_weight" : "sddmm_sputnik_half", flat ? a.unsqueeze(0) : a,
+                                          flat ? b.unsqueeze(0) : b, row_indices, row_offsets, column_indices);
+    return flat && !summed ? at::_unsafe_view(out, {out.size(1)}) : out;
+  };
+  if (forced || !plain(a, flat ? 2 : 3) || !plain(b, flat ? 2 : 3) || b.device() != a.device() || b.scalar_type() != a.scalar_type() ||
+      (!flat && a.size(0) != b.size(0)) || a.size(-1) != b.size(-1) || !plain_csr(row_indices, row_offsets, column_indices, a, a.size(-2)) ||
+      column_indices.scalar_type() != at::kInt)
+    return python();
+  const int dtype = dtype_code(a.scalar_type());
+  const int64_t batch = flat ? 1 : a.size(0), m = a.size(-2), k = a.size(-1), n = b.size(-2), nonzeros = column_indices.size(0);
+  if (dtype < 0 || (summed && dtype != IEX_F32) || batch * m == 0) return python();
+  const auto known = note_of(row_offsets, column_indices, n);
+  if (!known || (known->status & kBadPattern)) return python();
+  const bool any_order = known->status & IEX_CSR_NOT_ASCENDING;
+  int flags = (summed ? IEX_SDDMM_SUM_OVER_BATCH : 0) | (any_order ? IEX_SDDMM_ANY_COLUMN_ORDER : 0);
+  auto kind_of = [&](int f) { return iex_sddmm_workspace_kind(dtype, f, m, k, n, nonzeros, batch); };
+  if (!summed && !any_order && dtype != IEX_F32 && known->dense_share >= 0 && (double)batch * m * n >= kStructureCells) {
+    if (known->dense_share >= kStructureShare) flags |= kind_of(flags | IEX_SDDMM_FORCE_VARIANT(3)) == 3 ? IEX_SDDMM_FORCE_VARIANT(3) : 0;
+    else if (kind_of(flags) == 3) flags |= IEX_SDDMM_FORCE_VARIANT(1);
+  }
+  const c10::DeviceGuard guard(a.device());
+  Tensor out = summed || flat ? at::empty({nonzeros}, a.options()) : at::empty({batch, nonzeros}, a.options());
+  const size_t ws_bytes = iex_sddmm_workspace_bytes(dtype, flags, m, k, n, nonzeros, batch);
+  Tensor ws;
+  if (ws_bytes && kind_of(flags) == 3) {
+    if (!known->tables.defined() || (size_t)known->tables.numel() < ws_bytes) return python();   // (it makes them)
+    ws = known->tables;
+    flags |= IEX_SDDMM_TABLES_READY | IEX_SDDMM_LISTS_READY;
+  } else {
+    ws = workspace(ws_bytes, a);
+  }
+  check(iex_sddmm_ws(dtype, flags, m, k, n, nonzeros, row_indices.const_data_ptr<int>(), row_offsets.const_data_ptr<int>(),
+                     column_indices.const_data_ptr<int>(), a.const_data_ptr(), b.const_data_ptr(), out.data_ptr(), stream_of(a), batch,
+                     ws.defined() ? ws.data_ptr() : nullptr, ws_bytes),
+        "sddmm");
+  return out;
+}
+
+// ---- softmax, GEMM -------------------------------------------------------------------------------------------------
+Tensor csr_softmax(Tensor values, const Tensor& row_indices, const Tensor& row_offsets, double scale) {
+  const int dtype = dtype_code(values.scalar_type());
+  const int64_t m = row_indices.dim() == 1 ? row_indices.size(0) : -1;
+  if (!plain(values, 2) || !plain(row_indices, 1) || !plain(row_offsets, 1) || dtype < 0 || row_indices.scalar_type() != at::kInt ||
+      row_offsets.scalar_type() != at::kInt || row_offsets.size(0) != m + 1 || row_indices.device() != values.device() ||
+      row_offsets.device() != values.device()) {
+    ask_python<py::object>("csr_softmax_", values, row_indices, row_offsets, scale);
+    return values;
+  }
+  const c10::DeviceGuard guard(values.device());
+  check(iex_csr_softmax(dtype, m, values.size(1), row_indices.const_data_ptr<int>(), row_offsets.const_data_ptr<int>(), values.data_ptr(), (float)scale,
+                        stream_of(values), values.size(0)),
+        "csr_softmax");
+  return values;
+}
+
+Tensor gemm(const Tensor& a, const Tensor& b, bool trans_b) {
+  const int dtype = dtype_code(a.scalar_type());
+  const bool fits = !forced && (a.dim() == 2 || a.dim() == 3) && (b.dim() == 2 || b.dim() == 3) && plain(a, a.dim()) && plain(b, b.dim()) &&
+                    a.device() == b.device() && (dtype == IEX_F16 || dtype == IEX_BF16) && b.scalar_type() == a.scalar_type() &&
+                    b.size(trans_b ? -1 : -2) == a.size(-1) && (a.dim() == 2 || b.dim() == 2 || a.size(0) == b.size(0));
+  if (!fits) return ask_python<Tensor>("gemm_mfma", a, b, trans_b);
+  const int64_t M = a.size(-2), K = a.size(-1), N = b.size(trans_b ? -2 : -1);
+  const bool batched = a.dim() == 3 || b.dim() == 3;
+  const int64_t batch = a.dim() == 3 ? a.size(0) : b.dim() == 3 ? b.size(0) : 1;
+  const c10::DeviceGuard guard(a.device());
+  Tensor out = batched ? at::empty({batch, M, N}, a.options()) : at::empty({M, N}, a.options());
+  const size_t ws_bytes = iex_gemm_workspace_bytes(dtype, trans_b, M, N, K, batch);
+  const Tensor ws = workspace(ws_bytes, a);
+  check(iex_gemm_ws(dtype, trans_b, M, N, K, a.const_data_ptr(), b.const_data_ptr(), out.data_ptr(), batch, a.dim() == 3 ? M * K : 0,
+                    b.dim() == 3 ? N * K : 0, M * N, stream_of(a), ws.defined() ? ws.data_ptr() : nullptr, ws_bytes),
+        "gemm");
+  return out;
+}
+
+// ---- autograd: the plain calls of MySpMM and MyLinear (no recording, no forced kernels) -----------------------------
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+Tensor spmm_shared(const Tensor& b, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m) {
+  return values.scalar_type() == at::kFloat ? spmm<Spmm::kSharedF32, true>(b, row_indices, values, row_offsets, column_indices, m)
+                                            : spmm<Spmm::kSharedHalf, true>(b, row_indices, values, row_offsets, column_indices, m);
+}
+
+// values[perm]: the values of the transposed matrix
+Tensor permuted(const Tensor& values, const Tensor& perm) {
+  const int64_t n = perm.numel();
+  if (!plain(values, 1) || !plain(perm, 1) || perm.scalar_type() != at::kLong || values.numel() != n || dtype_code(values.scalar_type()) < 0 ||
+      perm.device() != values.device())
+    return values.detach().index_select(0, perm);
+  const c10::DeviceGuard guard(values.device());
+  Tensor out = at::empty({n}, values.options());
+  check(iex_gather_values(values.element_size(), n, values.const_data_ptr(), reinterpret_cast<const long long*>(perm.const_data_ptr<int64_t>()),
+                          out.data_ptr(), stream_of(values)),
+        "gather_values");
+  return out;
+}
+
+struct TrainableSpmm : torch::autograd::Function<TrainableSpmm> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& b, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets,
+                        const Tensor& column_indices, int64_t m, const Tensor& row_indices_t, const Tensor& row_offsets_t,
+                        const Tensor& column_indices_t, const Tensor& perm) {
+    const Tensor dense = b.contiguous();
+    ctx->save_for_backward({dense, row_indices, values, row_offsets, column_indices, row_indices_t, row_offsets_t, column_indices_t, perm});
+    return spmm_shared(dense, row_indices, values, row_offsets, column_indices, m);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &dense = saved[0], &row_indices = saved[1], &values = saved[2], &row_offsets = saved[3], &column_indices = saved[4];
+    const Tensor grad = grads[0].contiguous();
+    variable_list out(10);
+    if (ctx->needs_input_grad(2)) {
+      // lhs = grad (m, n), rhs = b (k, n): rows of rhs are indexed by the CSR column
+      const Tensor columns = column_indices.scalar_type() == at::kInt ? column_indices : ask_python<Tensor>("int32_columns", column_indices);
+      out[2] = grad.scalar_type() == at::kFloat ? sddmm<true, true>(grad, dense, row_indices, row_offsets, columns)
+                                                : sddmm<false, true>(grad, dense, row_indices, row_offsets, columns);
+    }
+    if (ctx->needs_input_grad(0)) out[0] = spmm_shared(grad, saved[5], permuted(values, saved[8]), saved[6], saved[7], dense.size(0));
+    return out;
+  }
+};
+
+Tensor trainable_spmm(const Tensor& b, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m,
+                      const Tensor& row_indices_t, const Tensor& row_offsets_t, const Tensor& column_indices_t, const Tensor& perm) {
+  py::gil_scoped_release no_gil;
+  return TrainableSpmm::apply(b, row_indices, values, row_offsets, column_indices, m, row_indices_t, row_offsets_t, column_indices_t, perm);
+}
+
+struct TrainableLinear : torch::autograd::Function<TrainableLinear> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& input, const Tensor& weight) {
+    const Tensor x = input.contiguous(), w = weight.contiguous();
+    ctx->save_for_backward({x, w});
+    return gemm(x, w, true);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor grad = grads[0].contiguous();
+    variable_list out(2);
+    if (ctx->needs_input_grad(0)) out[0] = gemm(grad, saved[1], false);
+    if (ctx->needs_input_grad(1)) out[1] = gemm(grad.t().contiguous(), saved[0], false);
+    return out;
+  }
+};
+
+Tensor trainable_linear(const Tensor& input, const Tensor& weight) {
+  py::gil_scoped_release no_gil;
+  return TrainableLinear::apply(input, weight);
+}
+
+}  // namespace
+
+TORCH_LIBRARY(iex_ops, lib) {
+  const char* spmm_schema = "(Tensor b, Tensor row_indices, Tensor values, Tensor row_offsets, Tensor column_indices, int m) -> Tensor";
+  const char* sddmm_schema = "(Tensor a, Tensor b, Tensor row_indices, Tensor row_offsets, Tensor column_indices) -> Tensor";
+  // one implementation for every backend: operands that are not device tensors are refused with the reference's message
+  auto define = [&](const std::string& name, const char* schema, auto fn) {
+    lib.def((name + schema).c_str());
+    lib.impl(name.c_str(), torch::dispatch(c10::DispatchKey::CompositeExplicitAutograd, fn));
+  };
+  define("spmm_sputnik_reuse_weight", spmm_schema, TORCH_FN(spmm<Spmm::kSharedF32>));
+  define("spmm_sputnik_atomic", spmm_schema, TORCH_FN(spmm<Spmm::kAtomic>));
+  define("spmm_sputnik_reuse_weight_half", spmm_schema, TORCH_FN(spmm<Spmm::kSharedHalf>));
+  define("spmm_sputnik_batched_values", spmm_schema, TORCH_FN(spmm<Spmm::kPerEntry>));
+  define("sddmm_sputnik_atomic_upd_weight", sddmm_schema, TORCH_FN(sddmm<true>));
+  define("sddmm_sputnik_half", sddmm_schema, TORCH_FN(sddmm<false>));
+  define("csr_softmax_", "(Tensor(a!) values, Tensor row_indices, Tensor row_offsets, float scale) -> Tensor(a!)", TORCH_FN(csr_softmax));
+  define("gemm_mfma", "(Tensor a, Tensor b, bool trans_b=False) -> Tensor", TORCH_FN(gemm));
+}
+
+PYBIND11_MODULE(_iex_host, module) {
+  module.def("bind", [](py::object functions) { python_ops = new py::object(std::move(functions)); });
+  module.def("set_forced", [](bool on) { forced = on; });
+  module.def("set_note", &set_note);
+  module.def("trainable_spmm", &trainable_spmm);
+  module.def("trainable_linear", &trainable_linear);
+}

@@ -20,9 +20,10 @@ from __future__ import annotations
 
 import torch
 
+from .... import _iex_host
 from ... import ops as _ops
 from ...utils import _transpose_with_info, transpose_info
-from .utils import MyAutogradFunc, TunableItemCfg, maybe_captured
+from .utils import MyAutogradFunc, TunableItemCfg, maybe_captured, runs_plainly
 
 ops = torch.ops.iex_ops
 
@@ -106,6 +107,13 @@ class MySpMM(MyAutogradFunc):
     ``_transp_info`` is the tuple of :func:`transpose_info` (or None: it is then computed
     on the fly, outside any capture); ``column_indices`` may be int16 for half values in the
     forward pass, the backward pass uses int32 indices (the transposed matrix has m columns)."""
+
+    @classmethod
+    def apply(cls, fwd_kwargs, *inputs):
+        # nothing to record and nothing forced: the same node as native code (a small layer's training step is host time)
+        if cls is MySpMM and runs_plainly(fwd_kwargs) and len(inputs) == 7 and inputs[6] is not None:
+            return _iex_host.trainable_spmm(*inputs[:5], int(inputs[5]), *inputs[6])
+        return super().apply(fwd_kwargs, *inputs)
 
     @staticmethod
     def num_inputs(**kwargs) -> int:

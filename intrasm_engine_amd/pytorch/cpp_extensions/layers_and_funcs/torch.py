@@ -9,8 +9,9 @@ from __future__ import annotations
 
 import torch
 
+from .... import _iex_host
 from ... import ops as _ops
-from .utils import MyAutogradFunc, TunableItemCfg, maybe_captured
+from .utils import MyAutogradFunc, TunableItemCfg, maybe_captured, runs_plainly
 
 ops = torch.ops.iex_ops
 
@@ -27,6 +28,12 @@ def _gemm(a, b, trans_b, tile="auto"):
 
 class MyLinear(MyAutogradFunc):
     """``MyLinear.apply(fwd_kwargs, input, weight)``."""
+
+    @classmethod
+    def apply(cls, fwd_kwargs, *inputs):
+        if cls is MyLinear and runs_plainly(fwd_kwargs) and len(inputs) == 2:   # (as in MySpMM.apply)
+            return _iex_host.trainable_linear(*inputs)
+        return super().apply(fwd_kwargs, *inputs)
 
     @staticmethod
     def num_inputs(**kwargs) -> int:

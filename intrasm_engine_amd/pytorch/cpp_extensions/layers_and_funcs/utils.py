@@ -69,6 +69,14 @@ def normalise_kwargs(kwargs: dict | None) -> dict:
     return out
 
 
+def runs_plainly(fwd_kwargs: dict | None) -> bool:
+    """Whether a call with these (valid) options neither records into a constructor nor forces a kernel."""
+    if not fwd_kwargs:
+        return True
+    kwargs = normalise_kwargs(fwd_kwargs)
+    return not (kwargs["constructor_enabled"] or kwargs["params"])
+
+
 @contextlib.contextmanager
 def maybe_captured(constructor, enabled: bool, stream_beg: int):
     """Run the body on registered stream ``stream_beg`` of ``constructor`` inside a

@@ -7,6 +7,10 @@ operand's device (so a surrounding graph capture routes it to the capture's pool
 look up torch's *current* stream (never an argument, sputnik_kernels.cpp:81,151) and
 call the C ABI of ``libiex_hip.so``.  Nothing here computes on the CPU.
 
+The everyday call is served natively (``csrc/host/torch_ops.cpp``, ``_iex_host.so``): a small product is over on the GPU
+before a Python body has launched it.  The functions below are where it turns for the rest: operands to refuse, a
+pattern's first look, kernel choices forced by :func:`kernel_params`, plans, given outputs.
+
 Registered operators
     spmm_sputnik_reuse_weight        fp32, values (nnz)                     [reference :173-175]
     spmm_sputnik_atomic              fp32, values (batch, nnz)              [reference :170-172]
@@ -27,7 +31,7 @@ import weakref
 
 import torch
 
-from .. import _lib
+from .. import _iex_host, _lib
 
 _DT = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 _IT = {torch.int32: _lib.I32, torch.int16: _lib.I16}
@@ -60,10 +64,12 @@ def kernel_params(*, spmm: dict | None = None, sddmm: dict | None = None, gemm: 
     for name, given in (("spmm", spmm), ("sddmm", sddmm), ("gemm", gemm)):
         if given is not None:
             setattr(_TUNING, name, given or None)
+    _iex_host.set_forced(bool(_TUNING.__dict__.get("spmm") or _TUNING.__dict__.get("sddmm") or _TUNING.__dict__.get("gemm")))
     try:
         yield
     finally:
         _TUNING.spmm, _TUNING.sddmm, _TUNING.gemm = before["spmm"], before["sddmm"], before["gemm"]
+        _iex_host.set_forced(any(before.values()))
 
 
 def _version(t) -> int:
@@ -168,10 +174,12 @@ def _pattern_tables_host(row_offsets, column_indices, k):
     return ws
 
 
-def _set_note(row_offsets, column_indices, k, status, hist, share=None):
-    # (last field: the tables of the kernels for patterns with structure, made by the first call that wants them)
+def _set_note(row_offsets, column_indices, k, status, hist, share=None, tables=None):
+    """Keep what is known about a pattern on its ``column_indices`` and with the native side of the operators.
+    ``tables``: of the kernels for patterns with structure, made by the first call that wants them."""
     column_indices.__dict__["_iex_csr"] = (weakref.ref(row_offsets), _version(row_offsets), _version(column_indices), int(k), status, hist, share,
-                                           None)
+                                           tables)
+    _iex_host.set_note(row_offsets, column_indices, int(k), status, hist, share, tables)
 
 
 def mark_canonical(row_offsets, column_indices, k, measure=True):
@@ -265,7 +273,7 @@ def _known_tables(row_offsets, column_indices, k):
     if note[7] is None and not torch.cuda.is_current_stream_capturing():
         tables = _pattern_tables_host(row_offsets, column_indices, k)
         if tables is not None:
-            column_indices.__dict__["_iex_csr"] = note[:7] + (tables,)
+            _set_note(row_offsets, column_indices, k, *note[4:7], tables)
         return tables
     return note[7]
 
@@ -296,9 +304,10 @@ def carry_pattern_note(column_indices, copy):
     """``copy`` holds the same column indices as ``column_indices`` (another integer type, a clone): what is known about
     the one holds for the other."""
     note = column_indices.__dict__.get("_iex_csr")
-    if note is not None and note[2] == _version(column_indices):
+    row_offsets = note[0]() if note is not None and note[2] == _version(column_indices) else None
+    if row_offsets is not None and note[1] == _version(row_offsets):
         # (the tables were made from int32 indices: a copy of another integer type does not inherit them)
-        copy.__dict__["_iex_csr"] = note[:2] + (_version(copy),) + note[3:7] + (note[7] if copy.dtype == column_indices.dtype else None,)
+        _set_note(row_offsets, copy, *note[3:7], note[7] if copy.dtype == column_indices.dtype else None)
     return copy
 
 
@@ -723,38 +732,25 @@ def fused_spmm_gemm(b, row_indices, values, row_offsets, column_indices, m, ga, 
     return out, c
 
 
-_SPMM_SCHEMA = "(Tensor b, Tensor row_indices, Tensor values, Tensor row_offsets, Tensor column_indices, int m) -> Tensor"
-_SDDMM_SCHEMA = "(Tensor a, Tensor b, Tensor row_indices, Tensor row_offsets, Tensor column_indices) -> Tensor"
 _registered = False
 _library = None
 
 
 def register() -> None:
-    """Define the operators under ``torch.ops.iex_ops`` (idempotent)."""
+    """Complete the operators under ``torch.ops.iex_ops`` (idempotent): loading ``_iex_host`` has defined all but the
+    fused one; it gets the functions of this module that serve what it does not."""
     global _registered, _library
     if _registered:
         return
-    lib = torch.library.Library("iex_ops", "DEF")
-    table = [
-        ("spmm_sputnik_reuse_weight", _SPMM_SCHEMA, spmm_sputnik_reuse_weight),
-        ("spmm_sputnik_atomic", _SPMM_SCHEMA, spmm_sputnik_atomic),
-        ("spmm_sputnik_reuse_weight_half", _SPMM_SCHEMA, spmm_sputnik_reuse_weight_half),
-        ("spmm_sputnik_batched_values", _SPMM_SCHEMA, spmm_sputnik_batched_values),
-        ("sddmm_sputnik_atomic_upd_weight", _SDDMM_SCHEMA, sddmm_sputnik_atomic_upd_weight),
-        ("sddmm_sputnik_half", _SDDMM_SCHEMA, sddmm_sputnik_half),
-        ("csr_softmax_", "(Tensor(a!) values, Tensor row_indices, Tensor row_offsets, float scale) -> Tensor(a!)",
-         csr_softmax_),
-        ("gemm_mfma", "(Tensor a, Tensor b, bool trans_b=False) -> Tensor",
-         lambda a, b, trans_b=False: gemm_mfma(a, b, trans_b)),
-        ("fused_spmm_gemm",
-         "(Tensor b, Tensor row_indices, Tensor values, Tensor row_offsets, Tensor column_indices, int m, "
-         "Tensor ga, Tensor gb, bool trans_b=False, int? interleave=None) -> (Tensor, Tensor)",
-         fused_spmm_gemm),
-    ]
-    for name, schema, fn in table:
-        lib.define(name + schema)
-        # one implementation for every backend: the body itself rejects non-device
-        # tensors with the reference's message ("b must be a CUDA tensor")
-        lib.impl(name, fn, "CompositeExplicitAutograd")
+    functions = {f.__name__: f for f in (spmm_sputnik_reuse_weight, spmm_sputnik_atomic, spmm_sputnik_reuse_weight_half, spmm_sputnik_batched_values,
+                                         sddmm_sputnik_atomic_upd_weight, sddmm_sputnik_half, csr_softmax_, gemm_mfma)}
+    functions["int32_columns"] = lambda columns: carry_pattern_note(columns, columns.to(torch.int32))
+    _iex_host.bind(functions)
+    lib = torch.library.Library("iex_ops", "FRAGMENT")
+    lib.define("fused_spmm_gemm(Tensor b, Tensor row_indices, Tensor values, Tensor row_offsets, Tensor column_indices, int m, "
+               "Tensor ga, Tensor gb, bool trans_b=False, int? interleave=None) -> (Tensor, Tensor)")
+    # one implementation for every backend: the body itself rejects non-device
+    # tensors with the reference's message ("b must be a CUDA tensor")
+    lib.impl("fused_spmm_gemm", fused_spmm_gemm, "CompositeExplicitAutograd")
     _library = lib
     _registered = True
