@@ -33,7 +33,6 @@ struct SddmmParams {
   const void* rhs;
   void* out;
   int sum_over_batch, accumulate;
-  int deep = 0;  // generic-k path: keep four slices of both rows in flight (set by the launcher)
 };
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -56,6 +55,28 @@ __device__ __forceinline__ float dot_vec(const vec_t<T, VEC>& a, const vec_t<T, 
   }
 }
 
+// VEC elements of a row of k from element kk on.  TAIL: the vector may reach past the row's end: the VEC elements that
+// end there are read instead (k >= VEC, checked by the host) and `keep` clears those that are not kk .. kk + VEC - 1, in
+// both operands (a zero in one alone would turn an infinity of the other into a NaN).
+template <typename T, int VEC>
+struct tail_mask {
+  static constexpr int kWords = (int)sizeof(T) * VEC / 4;
+  uint32_t keep[kWords > 0 ? kWords : 1];
+  __device__ __forceinline__ explicit tail_mask(int valid) {   // the last `valid` elements of the vector stay
+    constexpr int per_word = 4 / (int)sizeof(T);
+#pragma unroll
+    for (int w = 0; w < kWords; ++w) {
+      const int dead = VEC - valid - w * per_word;   // elements of this word to clear
+      keep[w] = dead <= 0 ? 0xffffffffu : dead >= per_word ? 0u : 0xffff0000u;
+    }
+  }
+  __device__ __forceinline__ void apply(vec_t<T, VEC>& v) const {
+    uint32_t* w = reinterpret_cast<uint32_t*>(&v);
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) w[i] &= keep[i];
+  }
+};
+
 // PASSES > 0: k <= PASSES*LPN*VEC (EXACT: k equals it, so no load needs a predicate): the lhs
 //             fragment of a (row, batch entry) is one register load per pass; a chunk of 64
 //             nonzeros takes LPN steps of G nonzeros: all column indices are shuffled out and
@@ -63,12 +84,16 @@ __device__ __forceinline__ float dot_vec(const vec_t<T, VEC>& a, const vec_t<T, 
 //             every group, so each lane ends up with exactly one output (nonzero lane%LPN*G +
 //             lane/LPN) and the chunk is written with ONE store instruction that covers 64
 //             consecutive outputs.  Plain stores only (no accumulate mode).
-// PASSES == 0: generic k and accumulate mode, operands streamed in LPN*VEC slices.
+// PASSES == 0: generic k, accumulate mode and sums over a batch: operands streamed in LPN*VEC slices, a slice of lhs
+//             serving kSddmmSteps nonzeros per lane group at a time, two slices in flight.
+// RAGGED: k is no multiple of VEC (or the operands are not aligned to it): vectors at element alignment, the one past
+//         the row's end masked.  (By single elements: 631 x 3656 at 96 %, k = 1189, fp16 267 us.)
 // A block serves kSddmmZb batch entries (grid.z = ceil(batch / kSddmmZb)) in per-entry output
 // mode, so the row's column indices are fetched once and reused.
 constexpr int kSddmmZb = 4;
+constexpr int kSddmmSteps = 4;
 
-template <typename T, int VEC, int LPN, int PASSES, int WPR, bool EXACT>
+template <typename T, int VEC, int LPN, int PASSES, int WPR, bool EXACT, bool RAGGED>
 __global__ __launch_bounds__(256) void sddmm_kernel(SddmmParams p) {
   constexpr int G = kWave / LPN;
   constexpr int KT = LPN * VEC;
@@ -114,18 +139,21 @@ __global__ __launch_bounds__(256) void sddmm_kernel(SddmmParams p) {
         const T* __restrict__ rhs = rhs_all + (size_t)z * rhs_zstride;
         vec_t<T, VEC> lfrag[PASSES];
         vec_t<T, VEC> rv[LPN][PASSES];
+        // (ragged: every lane reads a vector, only the last pass can reach past the row's end)
+        const int last_kk = (PASSES - 1) * KT + sl * VEC;
+        const tail_mask<T, VEC> mask(RAGGED ? min(max(p.k - last_kk, 0), VEC) : VEC);
+        auto at = [&](int ps) { return RAGGED ? min(ps * KT + sl * VEC, p.k - VEC) : ps * KT + sl * VEC; };
 #pragma unroll
         for (int ps = 0; ps < PASSES; ++ps) {
-          const int kk = ps * KT + sl * VEC;
-          if (EXACT || kk < p.k) lfrag[ps] = load_vec<T, VEC>(lhs + kk);
+          if (EXACT || RAGGED || at(ps) < p.k) lfrag[ps] = load_vec<T, VEC, !RAGGED>(lhs + at(ps));
         }
+        if constexpr (RAGGED) mask.apply(lfrag[PASSES - 1]);
 #pragma unroll
         for (int st = 0; st < LPN; ++st) {
           const T* r = rhs + (size_t)cc[st] * p.k;
 #pragma unroll
           for (int ps = 0; ps < PASSES; ++ps) {
-            const int kk = ps * KT + sl * VEC;
-            if (EXACT || kk < p.k) rv[st][ps] = load_vec<T, VEC>(r + kk);
+            if (EXACT || RAGGED || at(ps) < p.k) rv[st][ps] = load_vec<T, VEC, !RAGGED>(r + at(ps));
           }
         }
         float res = 0.f;
@@ -133,8 +161,12 @@ __global__ __launch_bounds__(256) void sddmm_kernel(SddmmParams p) {
         for (int st = 0; st < LPN; ++st) {
           float acc = 0.f;
 #pragma unroll
-          for (int ps = 0; ps < PASSES; ++ps)
-            if (EXACT || ps * KT + sl * VEC < p.k) acc = dot_vec<T, VEC>(lfrag[ps], rv[st][ps], acc);
+          for (int ps = 0; ps < PASSES; ++ps) {
+            if constexpr (RAGGED) {
+              if (ps == PASSES - 1) mask.apply(rv[st][ps]);
+            }
+            if (EXACT || RAGGED || at(ps) < p.k) acc = dot_vec<T, VEC>(lfrag[ps], rv[st][ps], acc);
+          }
           acc = group_sum<LPN>(acc);
           res = (sl == st) ? acc : res;
         }
@@ -146,39 +178,58 @@ __global__ __launch_bounds__(256) void sddmm_kernel(SddmmParams p) {
         const T* __restrict__ rhs = rhs_all + (size_t)z * rhs_zstride;
         T* __restrict__ out = out_all + (p.sum_over_batch ? (size_t)0 : (size_t)z * p.nnz);
         const int steps = (cnt + G - 1) / G;
-        for (int st = 0; st < steps; ++st) {
-          const int t = st * G + sub;           // nonzero of this chunk handled by my lane group
-          const int col = __shfl(c, t, kWave);  // t < 64 always; slots past cnt carry column 0
-          float acc = 0.f;
+        for (int st = 0; st < steps; st += kSddmmSteps) {
+          // nonzero st * G + u * G + sub of this chunk is the u-th of my lane group; slots past cnt carry column 0
+          int t[kSddmmSteps];
+          const T* row_of[kSddmmSteps];
+          float acc[kSddmmSteps];
+#pragma unroll
+          for (int u = 0; u < kSddmmSteps; ++u) {
+            t[u] = (st + u) * G + sub;
+            row_of[u] = rhs + (size_t)__shfl(c, t[u] & (kWave - 1), kWave) * p.k;
+            acc[u] = 0.f;
+          }
           for (int zz = 0; zz < zn; ++zz) {
             const T* l = lhs + (size_t)zz * lhs_zstride;
-            const T* r = rhs + (size_t)zz * rhs_zstride + (size_t)col * p.k;
+            const size_t zoff = (size_t)zz * rhs_zstride;
             int kk = sl * VEC;
-            if (p.deep) {
-              // few wavefronts on the chip: a long k is a chain of load -> multiply -> load with one
-              // memory latency per slice unless several slices are in flight.  (With the chip full,
-              // other wavefronts hide that latency and the extra rows in flight only cost cache hits:
-              // 4096 x 4096 at 90 %, k = 2048, fp32: 1.16 ms plain, 1.67 ms this way; 1024 x 1024 at
-              // 95 %, k = 4096: 0.36 ms plain, 0.13 ms this way.)
-              for (; kk + 3 * KT < p.k; kk += 4 * KT) {
-                vec_t<T, VEC> lv[4], rv[4];
+            // two slices of lhs and of every nonzero's rhs row in flight: the chain load -> multiply -> load is what a
+            // launch with few wavefronts waits for, and a slice of lhs is read once for kSddmmSteps nonzeros
+            for (; kk + KT + VEC <= p.k; kk += 2 * KT) {
+              vec_t<T, VEC> lv[2], rv[2][kSddmmSteps];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                  lv[u] = load_vec<T, VEC>(l + kk + u * KT);
-                  rv[u] = load_vec<T, VEC>(r + kk + u * KT);
-                }
+              for (int h = 0; h < 2; ++h) {
+                lv[h] = load_vec<T, VEC, !RAGGED>(l + kk + h * KT);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) acc = dot_vec<T, VEC>(lv[u], rv[u], acc);
+                for (int u = 0; u < kSddmmSteps; ++u) rv[h][u] = load_vec<T, VEC, !RAGGED>(row_of[u] + zoff + kk + h * KT);
+              }
+#pragma unroll
+              for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int u = 0; u < kSddmmSteps; ++u) acc[u] = dot_vec<T, VEC>(lv[h], rv[h][u], acc[u]);
+            }
+            for (; kk < p.k; kk += KT) {
+              const int from = RAGGED ? min(kk, p.k - VEC) : kk;
+              const tail_mask<T, VEC> mask(RAGGED ? min(p.k - kk, VEC) : VEC);
+              vec_t<T, VEC> lv = load_vec<T, VEC, !RAGGED>(l + from), rv[kSddmmSteps];
+#pragma unroll
+              for (int u = 0; u < kSddmmSteps; ++u) rv[u] = load_vec<T, VEC, !RAGGED>(row_of[u] + zoff + from);
+              if constexpr (RAGGED) mask.apply(lv);
+#pragma unroll
+              for (int u = 0; u < kSddmmSteps; ++u) {
+                if constexpr (RAGGED) mask.apply(rv[u]);
+                acc[u] = dot_vec<T, VEC>(lv, rv[u], acc[u]);
               }
             }
-            for (; kk < p.k; kk += KT)
-              acc = dot_vec<T, VEC>(load_vec<T, VEC>(l + kk), load_vec<T, VEC>(r + kk), acc);
           }
-          acc = group_sum<LPN>(acc);
-          if (sl == 0 && t < cnt) {
-            const size_t o = (size_t)base + t;
-            if (p.accumulate) acc += elem<T>::to_float(out[o]);
-            out[o] = elem<T>::from_float(acc);
+#pragma unroll
+          for (int u = 0; u < kSddmmSteps; ++u) {
+            acc[u] = group_sum<LPN>(acc[u]);
+            if (sl == 0 && t[u] < cnt) {
+              const size_t o = (size_t)base + t[u];
+              if (p.accumulate) acc[u] += elem<T>::to_float(out[o]);
+              out[o] = elem<T>::from_float(acc[u]);
+            }
           }
         }
       }
@@ -187,47 +238,42 @@ __global__ __launch_bounds__(256) void sddmm_kernel(SddmmParams p) {
   }
 }
 
-template <typename T, int VEC, int LPN, int PASSES, int WPR, bool EXACT>
-int launch_one(const SddmmParams& p0, hipStream_t stream) {
-  SddmmParams p = p0;
+template <typename T, int VEC, int LPN, int PASSES, int WPR, bool EXACT, bool RAGGED>
+int launch_one(const SddmmParams& p, hipStream_t stream) {
   dim3 grid(ceil_div(p.m, 4 / WPR), 1, p.sum_over_batch ? 1 : ceil_div(p.batch, kSddmmZb));
-  p.deep = (long long)grid.x * grid.z * 4 <= 2048;  // at most two wavefronts per SIMD of the chip
-  note_kernel("sddmm_kernel<%s, %d, %d, %d, %d, %s>", type_name<T>(), VEC, LPN, PASSES, WPR, EXACT ? "true" : "false");
-  hipLaunchKernelGGL((sddmm_kernel<T, VEC, LPN, PASSES, WPR, EXACT>), grid, dim3(256), 0, stream, p);
+  note_kernel("sddmm_kernel<%s, %d, %d, %d, %d, %s, %s>", type_name<T>(), VEC, LPN, PASSES, WPR, EXACT ? "true" : "false", RAGGED ? "true" : "false");
+  hipLaunchKernelGGL((sddmm_kernel<T, VEC, LPN, PASSES, WPR, EXACT, RAGGED>), grid, dim3(256), 0, stream, p);
   return check_hip(hipGetLastError(), "sddmm launch");
 }
 
-template <typename T, int VEC, int LPN, int PASSES, bool EXACT>
+template <typename T, int VEC, int LPN, int PASSES, bool EXACT, bool RAGGED>
 int launch_wpr(const SddmmParams& p, int wpr, hipStream_t stream) {
-  if (wpr == 4) return launch_one<T, VEC, LPN, PASSES, 4, EXACT>(p, stream);
-  return launch_one<T, VEC, LPN, PASSES, 1, EXACT>(p, stream);
+  if (wpr == 4) return launch_one<T, VEC, LPN, PASSES, 4, EXACT, RAGGED>(p, stream);
+  return launch_one<T, VEC, LPN, PASSES, 1, EXACT, RAGGED>(p, stream);
 }
 
-template <typename T, int VEC, int LPN>
+template <typename T, int VEC, int LPN, bool RAGGED>
 int launch_passes(const SddmmParams& p, int wpr, hipStream_t stream) {
   // register-resident lhs needs one batch entry per dot product and plain stores
   const bool fast = !(p.sum_over_batch && p.batch > 1) && !p.accumulate;
   constexpr int kt = LPN * VEC;
-  if (fast && p.k == kt) return launch_wpr<T, VEC, LPN, 1, true>(p, wpr, stream);
-  if (fast && p.k == 2 * kt) return launch_wpr<T, VEC, LPN, 2, true>(p, wpr, stream);
-  if (fast && p.k < kt) return launch_wpr<T, VEC, LPN, 1, false>(p, wpr, stream);
-  if (fast && p.k < 2 * kt) return launch_wpr<T, VEC, LPN, 2, false>(p, wpr, stream);
-  return launch_wpr<T, VEC, LPN, 0, false>(p, wpr, stream);
+  if constexpr (!RAGGED) {
+    if (fast && p.k == kt) return launch_wpr<T, VEC, LPN, 1, true, RAGGED>(p, wpr, stream);
+    if (fast && p.k == 2 * kt) return launch_wpr<T, VEC, LPN, 2, true, RAGGED>(p, wpr, stream);
+  }
+  if (fast && p.k <= kt) return launch_wpr<T, VEC, LPN, 1, false, RAGGED>(p, wpr, stream);
+  if (fast && p.k <= 2 * kt) return launch_wpr<T, VEC, LPN, 2, false, RAGGED>(p, wpr, stream);
+  return launch_wpr<T, VEC, LPN, 0, false, RAGGED>(p, wpr, stream);
 }
 
 template <typename T>
 int launch_typed(const SddmmParams& p, int wpr, hipStream_t stream) {
   constexpr int kMax = 16 / (int)sizeof(T);
-  int vec = kMax;
-  while (vec > 1 && (p.k % vec != 0 || !aligned(p.lhs, sizeof(T) * vec) || !aligned(p.rhs, sizeof(T) * vec)))
-    vec >>= 1;
+  if (p.k < kMax) return launch_passes<T, 1, 16, false>(p, wpr, stream);   // (no whole vector in a row)
   // lanes per nonzero: enough to cover k in one or two passes, at most 16 (one DPP row)
-  if (vec == kMax) {
-    if (p.k <= 8 * vec) return launch_passes<T, kMax, 8>(p, wpr, stream);
-    return launch_passes<T, kMax, 16>(p, wpr, stream);
-  }
-  if (vec >= 2) return launch_passes<T, 2, 16>(p, wpr, stream);
-  return launch_passes<T, 1, 16>(p, wpr, stream);
+  const bool ragged = p.k % kMax != 0 || !aligned(p.lhs, 16) || !aligned(p.rhs, 16);
+  if (p.k <= 8 * kMax) return ragged ? launch_passes<T, kMax, 8, true>(p, wpr, stream) : launch_passes<T, kMax, 8, false>(p, wpr, stream);
+  return ragged ? launch_passes<T, kMax, 16, true>(p, wpr, stream) : launch_passes<T, kMax, 16, false>(p, wpr, stream);
 }
 
 // ---- dense product, then sampling (16-bit types, caller's workspace of m * n * 2 bytes) ----

@@ -293,3 +293,23 @@ def test_dense_product_path_is_chosen_with_a_workspace_and_only_then(oracle, dev
     forced = (_lib.F16, 7 << 16) + args[2:]
     assert lib.iex_sddmm_ex(*forced) != 0 and "workspace" in _lib.last_error()
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("k", [3, 9, 31, 63, 65, 66, 127, 129, 250, 1189])
+def test_rows_of_no_whole_vectors(oracle, dev, dtype, k):
+    """k that is no multiple of the 128-bit vector, on either side of every change of path, and operands that are not
+    16-byte aligned; an infinity beyond a lane's share of a row must not turn its neighbours into NaNs."""
+    rng = np.random.default_rng(k)
+    a = W.config2_matrix(0.85, m=75, k=90)
+    lhs, rhs = (rng.standard_normal((2, rows, k)).astype(np.float32) for rows in (a.m, a.k))
+    ri, _, ro, ci = to_dev(a, dev)
+    lt, rt = (torch.from_numpy(x).to(dev).to(dtype) for x in (lhs, rhs))
+    want = oracle.sddmm(rounded(lhs, dtype), rounded(rhs, dtype), a.row_indices, a.row_offsets, a.column_indices, sum_over_batch=False)
+    scale = np.stack([oracle.sddmm_abs_scale(lhs[z:z + 1], rhs[z:z + 1], a.row_indices, a.row_offsets, a.column_indices) for z in range(2)])
+    got = ops.sddmm_sputnik_half(lt, rt, ri, ro, ci)
+    assert_close(got.float().cpu().numpy(), want, scale, RTOL[dtype], f"k={k}")
+    odd = torch.empty(lt.numel() + 1, dtype=dtype, device=dev)[1:].view_as(lt).copy_(lt)     # element-aligned only
+    assert_close(ops.sddmm_sputnik_half(odd, rt, ri, ro, ci).float().cpu().numpy(), want, scale, RTOL[dtype], f"k={k}, unaligned")
+    rt[0, :, k - 1] = float("inf")
+    assert not torch.isnan(ops.sddmm_sputnik_half(lt, rt, ri, ro, ci)).any()
