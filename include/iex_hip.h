@@ -124,6 +124,10 @@ int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream);
  * units by hand (tests/test_interleaving.py:434-476); this is the same choice, made by the callee.  Ignored when bits
  * 16..19 force a family, with IEX_SPMM_ANY_COLUMN_ORDER, and for every other element type.                      */
 #define IEX_SPMM_BESIDE_GATHER_KERNEL 0x40
+/* iex_spmm_ws and its workspace queries: the dense-form path (IEX_SPMM_FORCE_VARIANT(7), and where it is chosen) also
+ * serves k, n and dense operands that are no whole 16-byte vectors, by copying the dense operand into the workspace with
+ * zeros around it where it has to; the size asked for then holds that copy.  16-bit values shared by the batch. */
+#define IEX_SPMM_PAD_OPERANDS 0x80
 /* bits 8..15: force waves-per-row (1, 4 or 8); 0 = choose from nnz/m.  For tuning.    */
 #define IEX_SPMM_FORCE_WPR(w) (((w) & 0xff) << 8)
 /* bits 16..19: force the kernel family: 1 = row kernel gathering from L2, 2 = LDS-staged
@@ -238,6 +242,15 @@ int iex_spmm_static(int dtype, int itype, int flags, int m, int k, int n, int no
                     void* out, void* stream, int batch);
 size_t iex_spmm_static_scratch_bytes(void);
 
+/* out (k x n) = A^T * dense for the m x k matrix A in canonical CSR form (no transposed pattern, no permuted values) and
+ * dense (m x n), fp16 / bf16, by way of A's dense form.  Counterpart of the backward product of the reference's MySpMM
+ * (layers_and_funcs/sputnik.py:93-122), which transposes the CSR first.  The workspace query returns 0 where a SpMM on the
+ * transposed CSR would not take the dense-form path (the call runs all the same, with spmm_transposed's own need of
+ * bytes); the workspace is 256-byte aligned. */
+size_t iex_spmm_transposed_workspace_bytes(int dtype, int m, int k, int n, int nonzeros);
+int iex_spmm_transposed(int dtype, int itype, int m, int k, int n, int nonzeros, const void* values, const int* row_offsets,
+                        const void* column_indices, const void* dense, void* out, void* stream, void* workspace, size_t workspace_bytes);
+
 /* Drop-ins for the three launchers the reference declares in csrc/extensions.h:28-30.  Like the reference's they accept
  * column indices in any order inside a row, and duplicates (IEX_SPMM_ANY_COLUMN_ORDER is always set: the row kernel,
  * or the few-columns kernel); a caller that knows its CSR arrays to be canonical gets every family from iex_spmm_ex.
@@ -274,6 +287,9 @@ int iex_CudaSpmm5(int m, int k, int n, int nonzeros, const int* row_indices,
  * with nothing forced the call keeps to the gather kernel and the dense-product path, which take such input.
  * Ignored when bits 16..19 force a variant.                                                            */
 #define IEX_SDDMM_ANY_COLUMN_ORDER 0x10
+/* iex_sddmm_ws and its workspace queries: the dense product (IEX_SDDMM_FORCE_VARIANT(7), and where it is chosen) also
+ * serves k, n and operands that are no whole 16-byte vectors, by copies in the workspace. */
+#define IEX_SDDMM_PAD_OPERANDS 0x20
 /* bits 8..15: force wavefronts per row (1 or 4); 0 = choose from nnz/m.  For tuning.
  * With variant 3 the same bits set the number of nonzeros from which a 128 x 128 block of the
  * mask counts as dense: 0 = built in, 1 = every block, 255 = none, else 64 * value.       */
@@ -352,7 +368,8 @@ int iex_csr_softmax(int dtype, int m, int nonzeros, const int* row_indices,
                     int batch);
 
 /* ------------------------------------------------------------------ GEMM ---- */
-/* C[z] = A[z] * B[z] (trans_b == 0, B is (K,N)) or A[z] * B[z]^T (trans_b == 1, B is
+/* (bit 1 of trans_b: A is (K,M), any K, M a multiple of 8, B (K,N))
+ * C[z] = A[z] * B[z] (trans_b == 0, B is (K,N)) or A[z] * B[z]^T (trans_b == 1, B is
  * (N,K), the torch.nn.Linear weight layout used by MyLinear, layers_and_funcs/torch.py:17).
  * dtype is IEX_F16 or IEX_BF16 for A, B and C; accumulation is fp32 on the matrix cores.
  * stride_* are element strides between batch entries (0 = operand shared by the batch).

@@ -21,11 +21,13 @@ SPMM_TABLES_READY = 0x8
 SPMM_LISTS_READY = 0x10
 SPMM_BESIDE_GATHER_KERNEL = 0x40
 SPMM_ANY_COLUMN_ORDER = 0x20
+SPMM_PAD_OPERANDS = 0x80
 SDDMM_SUM_OVER_BATCH = 0x1
 SDDMM_ACCUMULATE = 0x2
 SDDMM_TABLES_READY = 0x4
 SDDMM_LISTS_READY = 0x8
 SDDMM_ANY_COLUMN_ORDER = 0x10
+SDDMM_PAD_OPERANDS = 0x20
 CSR_BAD_OFFSETS, CSR_COLUMN_OUT_OF_RANGE, CSR_NOT_ASCENDING = 0x1, 0x2, 0x4
 
 _c = ctypes
@@ -48,6 +50,8 @@ SIGNATURES = {
     "iex_csr_dense_share_scratch_bytes": (_c.c_size_t, [_i, _i]),
     "iex_spmm_workspace_bytes": (_c.c_size_t, [_i, _i, _i, _i, _i, _i, _i, _i]),
     "iex_spmm_workspace_kind": (_i, [_i, _i, _i, _i, _i, _i, _i, _i]),
+    "iex_spmm_transposed_workspace_bytes": (_c.c_size_t, [_i, _i, _i, _i, _i]),
+    "iex_spmm_transposed": (_i, [_i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c.c_size_t]),
     "iex_spmm_static": (_i, [_i, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "iex_spmm_static_scratch_bytes": (_c.c_size_t, []),
     "iex_CudaSpmm2": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i]),

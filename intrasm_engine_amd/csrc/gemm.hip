@@ -39,15 +39,15 @@ int launch(GemmParams p, int batch, hipStream_t stream) {
   return check_hip(hipGetLastError(), "gemm launch");
 }
 
-template <bool BF16, bool TRANS_B, int WM, int WN, int BK, int STAGES, int WCN>
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int BK, int STAGES, int WCN>
 __global__ __launch_bounds__(WCN * 128, (WCN == 2 && WM * WN <= 8 && gemm_dma_lds_bytes<WM, WN, WCN, BK, STAGES>() <= 80 * 1024 ? 2 : 1)) void gemm_dma_kernel(GemmParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   int tile_m, tile_n;
   if (!xcd_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;  // uniform per block
-  gemm_tile_dma<BF16, TRANS_B, WM, WN, WCN, BK, STAGES>(p, tile_m, tile_n, blockIdx.y, smem);
+  gemm_tile_dma<BF16, TRANS_B, WM, WN, WCN, BK, STAGES, 0, TRANS_A>(p, tile_m, tile_n, blockIdx.y, smem);
 }
 
-template <bool BF16, bool TRANS_B, int WM, int WN, int BK, int STAGES, int WCN = 2>
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int BK, int STAGES, int WCN = 2>
 int launch_dma(GemmParams p, int batch, hipStream_t stream) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32;
   p.tiles_m = ceil_div(p.M, BM);
@@ -55,7 +55,7 @@ int launch_dma(GemmParams p, int batch, hipStream_t stream) {
   const int total = p.tiles_m * p.tiles_n;
   const int per_xcd = (total + kXcds - 1) / kXcds;
   constexpr int lds = gemm_dma_lds_bytes<WM, WN, WCN, BK, STAGES>();
-  auto kern = gemm_dma_kernel<BF16, TRANS_B, WM, WN, BK, STAGES, WCN>;
+  auto kern = gemm_dma_kernel<BF16, TRANS_A, TRANS_B, WM, WN, BK, STAGES, WCN>;
   if (lds > 64 * 1024) {
     static thread_local bool raised = false;  // per instantiation
     if (!raised) {
@@ -66,22 +66,22 @@ int launch_dma(GemmParams p, int batch, hipStream_t stream) {
       raised = true;
     }
   }
-  note_kernel("gemm_dma_kernel<%s, %s, %d, %d, %d, %d, %d> (%d x %d tiles, %d waves)", BF16 ? "bf16" : "f16", TRANS_B ? "B(N,K)" : "B(K,N)", WM, WN,
+  note_kernel("gemm_dma_kernel<%s, %s%s, %d, %d, %d, %d, %d> (%d x %d tiles, %d waves)", BF16 ? "bf16" : "f16", TRANS_A ? "A(K,M), " : "", TRANS_B ? "B(N,K)" : "B(K,N)", WM, WN,
               BK, STAGES, WCN, BM, BN, 2 * WCN);
   hipLaunchKernelGGL(kern, dim3(per_xcd * kXcds, batch), dim3(WCN * 128), lds, stream, p);
   return check_hip(hipGetLastError(), "gemm launch");
 }
 
 // Eight wavefronts in two groups that alternate between reading / loading and multiplying (gemm_pp_device.cuh).
-template <bool BF16, bool TRANS_B, int WM, int WN, int WCN>
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN>
 __global__ __launch_bounds__(WCN * 128, 1) void gemm_pp_kernel(GemmParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   int tile_m, tile_n;
   if (!xcd_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;  // uniform per block
-  gemm_tile_pp<BF16, TRANS_B, WM, WN, WCN>(p, tile_m, tile_n, blockIdx.y, smem);
+  gemm_tile_pp<BF16, TRANS_B, WM, WN, WCN, TRANS_A>(p, tile_m, tile_n, blockIdx.y, smem);
 }
 
-template <bool BF16, bool TRANS_B, int WM, int WN, int WCN>
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN>
 int launch_pp(GemmParams p, int batch, hipStream_t stream) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32;
   p.tiles_m = ceil_div(p.M, BM);
@@ -89,7 +89,7 @@ int launch_pp(GemmParams p, int batch, hipStream_t stream) {
   const int total = p.tiles_m * p.tiles_n;
   const int per_xcd = (total + kXcds - 1) / kXcds;
   constexpr int lds = gemm_pp_lds_bytes<BF16, TRANS_B, WM, WN, WCN>();
-  auto kern = gemm_pp_kernel<BF16, TRANS_B, WM, WN, WCN>;
+  auto kern = gemm_pp_kernel<BF16, TRANS_A, TRANS_B, WM, WN, WCN>;
   static thread_local bool raised = false;  // per instantiation
   if (!raised) {
     if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds),
@@ -97,8 +97,8 @@ int launch_pp(GemmParams p, int batch, hipStream_t stream) {
       return rc;
     raised = true;
   }
-  note_kernel("gemm_pp_kernel<%s, %s, %d, %d, %d> (%d x %d tiles, two groups of 4 waves in alternating phases)", BF16 ? "bf16" : "f16",
-              TRANS_B ? "B(N,K)" : "B(K,N)", WM, WN, WCN, BM, BN);
+  note_kernel("gemm_pp_kernel<%s, %s%s, %d, %d, %d> (%d x %d tiles, two groups of 4 waves in alternating phases)", BF16 ? "bf16" : "f16",
+              TRANS_A ? "A(K,M), " : "", TRANS_B ? "B(N,K)" : "B(K,N)", WM, WN, WCN, BM, BN);
   hipLaunchKernelGGL(kern, dim3(per_xcd * kXcds, batch), dim3(WCN * 128), lds, stream, p);
   return check_hip(hipGetLastError(), "gemm launch");
 }
@@ -123,14 +123,14 @@ __global__ __launch_bounds__(WCN * 128, 1) void gemm_dma_splitk_kernel(GemmParam
   if (!xcd_tile(slot, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;  // uniform per block
   const int first = ((p.K + BK - 1) / BK / 2) * BK;   // K entries of the first half: whole steps
   GemmParams q = p;
-  q.ldk = p.K;
   if (part == 0) {
     q.K = first;
   } else {
     q.K = p.K - first;
     q.A = static_cast<const unsigned short*>(p.A) + first;
-    q.B = static_cast<const unsigned short*>(p.B) + (TRANS_B ? (size_t)first : (size_t)first * p.N);
+    q.B = static_cast<const unsigned short*>(p.B) + (TRANS_B ? (size_t)first : (size_t)first * p.ldb);
   }
+  q.kb = min(q.K, p.kb - (p.K - q.K) * part);
   gemm_tile_dma<BF16, TRANS_B, WM, WN, WCN, BK, STAGES, 1>(q, tile_m, tile_n, blockIdx.y, smem);
 }
 
@@ -170,7 +170,7 @@ int launch_dma_splitk(GemmParams p, int batch, void* ws, bool flags_are_zero, hi
 }
 
 // ---- K split over several workgroups per tile, every part on one XCD, the last to finish adds up (gemm_dma_device.cuh)
-template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, int BK, int STAGES>
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN, int BK, int STAGES>
 __global__ __launch_bounds__(WCN * 128, (WCN == 2 && WM * WN <= 8 && gemm_dma_lds_bytes<WM, WN, WCN, BK, STAGES>() <= 80 * 1024 ? 2 : 1)) void gemm_dma_parts_kernel(GemmParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int b = blockIdx.x, parts = p.split_parts;
@@ -180,12 +180,12 @@ __global__ __launch_bounds__(WCN * 128, (WCN == 2 && WM * WN <= 8 && gemm_dma_ld
   const int steps = (p.K + BK - 1) / BK, per = (steps + parts - 1) / parts * BK;   // K entries per part: whole steps
   const int k0 = part * per;   // (the host has chosen parts so that every part has a step)
   GemmParams q = p;
-  q.ldk = p.K;
   q.split_part = part;
   q.K = min(per, p.K - k0);
-  q.A = static_cast<const unsigned short*>(p.A) + k0;
-  q.B = static_cast<const unsigned short*>(p.B) + (TRANS_B ? (size_t)k0 : (size_t)k0 * p.N);
-  gemm_tile_dma<BF16, TRANS_B, WM, WN, WCN, BK, STAGES, 2>(q, tile_m, tile_n, blockIdx.y, smem);
+  q.kb = min(q.K, p.kb - k0);   // (the rows that are missing are fewer than a chunk: the last part has some)
+  q.A = static_cast<const unsigned short*>(p.A) + (TRANS_A ? (size_t)k0 * p.lda : (size_t)k0);
+  q.B = static_cast<const unsigned short*>(p.B) + (TRANS_B ? (size_t)k0 : (size_t)k0 * p.ldb);
+  gemm_tile_dma<BF16, TRANS_B, WM, WN, WCN, BK, STAGES, 2, TRANS_A>(q, tile_m, tile_n, blockIdx.y, smem);
 }
 
 // Parts per tile: as many as give every CU a workgroup, at most 8, every part at least 1024 of K, none empty.
@@ -204,7 +204,7 @@ inline size_t gemm_parts_bytes(int M, int N, int batch, int bm, int bn, int part
   return tiles * parts * bm * bn * sizeof(float) + ((tiles * sizeof(int) + 255) / 256) * 256;
 }
 
-template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, int BK, int STAGES>
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN, int BK, int STAGES>
 int launch_dma_parts(GemmParams p, int batch, int parts, void* ws, bool flags_are_zero, hipStream_t stream) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32;
   p.tiles_m = ceil_div(p.M, BM);
@@ -215,7 +215,7 @@ int launch_dma_parts(GemmParams p, int batch, int parts, void* ws, bool flags_ar
   p.split_ws = static_cast<float*>(ws);
   p.split_flags = reinterpret_cast<int*>(static_cast<unsigned char*>(ws) + (size_t)total * batch * parts * BM * BN * sizeof(float));
   constexpr int lds = gemm_dma_lds_bytes<WM, WN, WCN, BK, STAGES>();
-  auto kern = gemm_dma_parts_kernel<BF16, TRANS_B, WM, WN, WCN, BK, STAGES>;
+  auto kern = gemm_dma_parts_kernel<BF16, TRANS_A, TRANS_B, WM, WN, WCN, BK, STAGES>;
   if (lds > 64 * 1024) {
     static thread_local bool raised = false;  // per instantiation
     if (!raised) {
@@ -229,7 +229,7 @@ int launch_dma_parts(GemmParams p, int batch, int parts, void* ws, bool flags_ar
     note_kernel("fill_zero_kernel");
     hipLaunchKernelGGL(fill_zero_kernel, dim3(ceil_div(total * batch, 256)), dim3(256), 0, stream, p.split_flags, total * batch);
   }
-  note_kernel("gemm_dma_parts_kernel<%s, %s> (%d x %d tiles, K in %d parts)", BF16 ? "bf16" : "f16", TRANS_B ? "B(N,K)" : "B(K,N)", BM, BN, parts);
+  note_kernel("gemm_dma_parts_kernel<%s, %s%s> (%d x %d tiles, K in %d parts)", BF16 ? "bf16" : "f16", TRANS_A ? "A(K,M), " : "", TRANS_B ? "B(N,K)" : "B(K,N)", BM, BN, parts);
   hipLaunchKernelGGL(kern, dim3(per_xcd * kXcds * parts, batch), dim3(WCN * 128), lds, stream, p);
   return check_hip(hipGetLastError(), "gemm (K in parts) launch");
 }
@@ -248,34 +248,36 @@ inline bool auto_split_wanted(int M, int N, int K, int batch) {
   return split_parts_for(M, N, K, batch, 64, 128, 64) >= 2;
 }
 
-template <bool BF16, bool TRANS_B>
+template <bool BF16, bool TRANS_A, bool TRANS_B>
 int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, void* ws, size_t ws_bytes, bool flags_are_zero) {
-  if (force == 12) {
-    IEX_REQUIRE(p.K >= 64, IEX_ERR_UNSUPPORTED, "gemm: the K-split kernel needs two K steps (K >= 64; K=%d)", p.K);
-    IEX_REQUIRE(ws && aligned(ws, 256) && ws_bytes >= gemm_splitk_bytes(p.M, p.N, batch, 256, 256) && !p.accumulate, IEX_ERR_BAD_ARGUMENT,
-                "gemm: the K-split kernel needs a 256-byte aligned workspace of %zu bytes (iex_gemm_ws) and a plain store", gemm_splitk_bytes(p.M, p.N, batch, 256, 256));
-    return launch_dma_splitk<BF16, TRANS_B, 4, 4, 2, 32, 4>(p, batch, ws, flags_are_zero, stream);
+  if constexpr (!TRANS_A) {   // kernels that are never chosen
+    if (force == 12) {
+      IEX_REQUIRE(p.K >= 64, IEX_ERR_UNSUPPORTED, "gemm: the K-split kernel needs two K steps (K >= 64; K=%d)", p.K);
+      IEX_REQUIRE(ws && aligned(ws, 256) && ws_bytes >= gemm_splitk_bytes(p.M, p.N, batch, 256, 256), IEX_ERR_BAD_ARGUMENT,
+                  "gemm: the K-split kernel needs a 256-byte aligned workspace of %zu bytes (iex_gemm_ws)", gemm_splitk_bytes(p.M, p.N, batch, 256, 256));
+      return launch_dma_splitk<BF16, TRANS_B, 4, 4, 2, 32, 4>(p, batch, ws, flags_are_zero, stream);
+    }
+    if (force == 1) return launch<BF16, TRANS_B, 2, 2>(p, batch, stream);
+    if (force == 2) return launch<BF16, TRANS_B, 2, 4>(p, batch, stream);
+    if (force == 3) return launch<BF16, TRANS_B, 4, 4>(p, batch, stream);
+    if (force == 4) return launch<BF16, TRANS_B, 2, 2, 64>(p, batch, stream);
+    if (force == 6) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 4, 32, 4>(p, batch, stream);
+    if (force == 7) return launch_dma<BF16, TRANS_A, TRANS_B, 4, 4, 32, 4>(p, batch, stream);
+    if (force == 11) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 64, 3, 4>(p, batch, stream);
   }
   if (force == 14) {
     const int parts = std::max(2, split_parts_for(p.M, p.N, p.K, batch, 64, 128, 64)), steps = ceil_div(p.K, 64);
     IEX_REQUIRE(steps >= parts && (parts - 1) * ceil_div(steps, parts) < steps, IEX_ERR_UNSUPPORTED,
                 "gemm: K in %d parts needs a K step of 64 for every part (K=%d)", parts, p.K);
-    IEX_REQUIRE(ws && aligned(ws, 256) && ws_bytes >= gemm_parts_bytes(p.M, p.N, batch, 64, 128, parts) && !p.accumulate, IEX_ERR_BAD_ARGUMENT,
-                "gemm: K in parts needs a 256-byte aligned workspace of %zu bytes (iex_gemm_ws) and a plain store", gemm_parts_bytes(p.M, p.N, batch, 64, 128, parts));
-    return launch_dma_parts<BF16, TRANS_B, 1, 1, 4, 64, 4>(p, batch, parts, ws, flags_are_zero, stream);
+    IEX_REQUIRE(ws && aligned(ws, 256) && ws_bytes >= gemm_parts_bytes(p.M, p.N, batch, 64, 128, parts), IEX_ERR_BAD_ARGUMENT,
+                "gemm: K in parts needs a 256-byte aligned workspace of %zu bytes (iex_gemm_ws)", gemm_parts_bytes(p.M, p.N, batch, 64, 128, parts));
+    return launch_dma_parts<BF16, TRANS_A, TRANS_B, 1, 1, 4, 64, 4>(p, batch, parts, ws, flags_are_zero, stream);
   }
-  if (force == 1) return launch<BF16, TRANS_B, 2, 2>(p, batch, stream);
-  if (force == 2) return launch<BF16, TRANS_B, 2, 4>(p, batch, stream);
-  if (force == 3) return launch<BF16, TRANS_B, 4, 4>(p, batch, stream);
-  if (force == 4) return launch<BF16, TRANS_B, 2, 2, 64>(p, batch, stream);
-  if (force == 5) return launch_dma<BF16, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
-  if (force == 6) return launch_dma<BF16, TRANS_B, 2, 4, 32, 4>(p, batch, stream);
-  if (force == 7) return launch_dma<BF16, TRANS_B, 4, 4, 32, 4>(p, batch, stream);
-  if (force == 8) return launch_dma<BF16, TRANS_B, 2, 1, 64, 4, 4>(p, batch, stream);
-  if (force == 9) return launch_dma<BF16, TRANS_B, 1, 1, 64, 4, 4>(p, batch, stream);
-  if (force == 10) return launch_dma<BF16, TRANS_B, 2, 2, 32, 4, 4>(p, batch, stream);
-  if (force == 11) return launch_dma<BF16, TRANS_B, 2, 2, 64, 3, 4>(p, batch, stream);
-  if (force == 13) return launch_pp<BF16, TRANS_B, 4, 2, 4>(p, batch, stream);
+  if (force == 5) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
+  if (force == 8) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 1, 64, 4, 4>(p, batch, stream);
+  if (force == 9) return launch_dma<BF16, TRANS_A, TRANS_B, 1, 1, 64, 4, 4>(p, batch, stream);
+  if (force == 10) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4, 4>(p, batch, stream);
+  if (force == 13) return launch_pp<BF16, TRANS_A, TRANS_B, 4, 2, 4>(p, batch, stream);
   // Default: operands straight from global memory into LDS (gemm_dma_device.cuh).  The larger the
   // tile of a wave, the fewer LDS bytes each MFMA needs, and LDS time is what the main loop runs
   // against; the smaller the tile, the more workgroups there are to fill 256 CUs, and a tile wider
@@ -284,7 +286,7 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
   // A short K (at most 8 steps) is prologue and epilogue: small tiles, two workgroups per CU that cover for
   // each other (512 x (512 x 512 x 128), the attention scores of the decoder layer: 229 -> 123 us; 8192 x 8192 x
   // 128: 59 -> 48; from K = 512 the large tiles are ahead again).
-  if (p.K <= 256) return launch_dma<BF16, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
+  if (p.K <= 256) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
   const long long small_tiles = (long long)ceil_div(p.M, 128) * ceil_div(p.N, 128) * batch;
   if (small_tiles > 256) {
     // More 128 x 128 tiles than CUs: the tile shape that finishes first, counting whole rounds of workgroups (a
@@ -304,9 +306,9 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
     // warmed-up clocks: 8192^3 1250 / 1230, 4096 x 8192 x 4096 1109 / 1076, 11008 x 8192 x 4096 1151 / 1109,
     // 4096^3 1054 / 954; bit-equal results.  11008 x 2048 x 4096, where the two shapes are within 1 % in this count:
     // 218 us in two rounds of 256 x 256 tiles, 221-230 in three of 128 x 256)
-    if (huge <= wide && huge <= small) return launch_pp<BF16, TRANS_B, 4, 2, 4>(p, batch, stream);
-    if (wide <= small) return launch_dma<BF16, TRANS_B, 2, 2, 32, 4, 4>(p, batch, stream);
-    return launch_dma<BF16, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
+    if (huge <= wide && huge <= small) return launch_pp<BF16, TRANS_A, TRANS_B, 4, 2, 4>(p, batch, stream);
+    if (wide <= small) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4, 4>(p, batch, stream);
+    return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
   }
   // One round of at most one 128 x 128 tile per CU and a long K: eight waves (64 x 32 each) and K steps of 64
   // (4096 x 512 x 4096: 44 -> 34.5 us; eight waves with steps of 32 and eight stages 38.6; 64 x 128 tiles 36.8).
@@ -317,42 +319,41 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
   // (4096 x 256 x 4096: 35 -> 27.5 us, 4096 x 512 x 4096: 35 -> 30, 1024 x 2048 x 1024: 13.9 -> 12.4).
   const long long half_tiles = (long long)ceil_div(p.M, 64) * ceil_div(p.N, 128) * batch;
   // ... and with room for the partial sums, K in parts on as many CUs as there are
-  if (auto_split_wanted(p.M, p.N, p.K, batch) && !p.accumulate) {
+  if (auto_split_wanted(p.M, p.N, p.K, batch)) {
     const int parts = split_parts_for(p.M, p.N, p.K, batch, 64, 128, 64);
     if (ws && aligned(ws, 256) && ws_bytes >= gemm_parts_bytes(p.M, p.N, batch, 64, 128, parts))
-      return launch_dma_parts<BF16, TRANS_B, 1, 1, 4, 64, 4>(p, batch, parts, ws, flags_are_zero, stream);
+      return launch_dma_parts<BF16, TRANS_A, TRANS_B, 1, 1, 4, 64, 4>(p, batch, parts, ws, flags_are_zero, stream);
   }
-  if (half_tiles <= 256 && p.K >= 512) return launch_dma<BF16, TRANS_B, 1, 1, 64, 4, 4>(p, batch, stream);
-  if (p.K >= 2048) return launch_dma<BF16, TRANS_B, 2, 1, 64, 4, 4>(p, batch, stream);
-  return launch_dma<BF16, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
+  if (half_tiles <= 256 && p.K >= 512) return launch_dma<BF16, TRANS_A, TRANS_B, 1, 1, 64, 4, 4>(p, batch, stream);
+  if (p.K >= 2048) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 1, 64, 4, 4>(p, batch, stream);
+  return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
 }
 
 }  // namespace
 }  // namespace iex
 
-// trans_b: bit 0 = B is (N, K); bits 4..7 force the kernel for tuning.  Register-staged operands:
+// code: bit 0 = B is (N, K), bit 1 = A is (K, M); bits 4..7 force the kernel for tuning (A as (K, M): 5, 8, 9, 10, 13, 14).  Register-staged operands:
 // 1 = 128x128 tiles, 2 = 128x256, 3 = 256x256, 4 = 128x128 with K steps of 64.  Operands loaded
 // straight into LDS: 5 = 128x128, 6 = 128x256, 7 = 256x256, 8 = 128x128, 9 = 64x128 by eight waves with K steps of 64,
 // 10 = 128x256 by eight waves, 11 = the same with K steps of 64, 12 = 256x256 with K split over two workgroups per tile
 // (iex_gemm_ws only; never chosen), 13 = 256x256 by eight waves in two groups that alternate between loading and
 // multiplying, 14 = 64x128 by eight waves with K split over two to eight workgroups per tile (iex_gemm_ws only).
 // 0 = choose (one of 5, 8, 9, 10, 13, and 14 where iex_gemm_workspace_bytes asked for room and got it).
-extern "C" int iex_gemm(int dtype, int trans_b_and_shape, int M, int N, int K, const void* A, const void* B, void* C, int batch,
-                        long long stride_a, long long stride_b, long long stride_c, void* stream) {
-  iex::trail_reset();
-  return iex::gemm_dispatch(dtype, trans_b_and_shape, M, N, K, A, B, C, batch, stride_a, stride_b, stride_c, stream, nullptr, 0, 0);
-}
-
-extern "C" int iex_gemm_ws(int dtype, int trans_b_and_shape, int M, int N, int K, const void* A, const void* B, void* C, int batch,
+extern "C" int iex_gemm_ws(int dtype, int code, int M, int N, int K, const void* A, const void* B, void* C, int batch,
                            long long stride_a, long long stride_b, long long stride_c, void* stream, void* workspace, size_t workspace_bytes) {
   iex::trail_reset();
-  return iex::gemm_dispatch(dtype, trans_b_and_shape, M, N, K, A, B, C, batch, stride_a, stride_b, stride_c, stream, nullptr, 0, 0, workspace,
-                            workspace_bytes);
+  return iex::gemm_dispatch(dtype, code, iex::GemmParams{M, N, K, A, B, C, stride_a, stride_b, stride_c, 0, 0}, batch, static_cast<hipStream_t>(stream),
+                            workspace, workspace_bytes);
 }
 
-extern "C" size_t iex_gemm_workspace_bytes(int dtype, int trans_b_and_shape, int M, int N, int K, int batch) {
+extern "C" int iex_gemm(int dtype, int code, int M, int N, int K, const void* A, const void* B, void* C, int batch,
+                        long long stride_a, long long stride_b, long long stride_c, void* stream) {
+  return iex_gemm_ws(dtype, code, M, N, K, A, B, C, batch, stride_a, stride_b, stride_c, stream, nullptr, 0);
+}
+
+extern "C" size_t iex_gemm_workspace_bytes(int dtype, int code, int M, int N, int K, int batch) {
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || (dtype != IEX_F16 && dtype != IEX_BF16)) return 0;
-  const int force = (trans_b_and_shape >> 4) & 0xf;
+  const int force = (code >> 4) & 0xf;
   if (force == 12) return iex::gemm_splitk_bytes(M, N, batch, 256, 256);
   if (force == 14) return iex::gemm_parts_bytes(M, N, batch, 64, 128, 8);
   return force == 0 ? iex::gemm_auto_split_bytes(M, N, K, batch) : 0;
@@ -372,27 +373,34 @@ void iex::gemm_auto_split_flags(int M, int N, int K, int batch, size_t* offset_b
   *words = (int)tiles;
 }
 
-int iex::gemm_dispatch(int dtype, int trans_b_and_shape, int M, int N, int K, const void* A, const void* B, void* C, int batch,
-                       long long stride_a, long long stride_b, long long stride_c, void* stream, const float* row_bias, int relu,
-                       int accumulate, void* workspace, size_t workspace_bytes, bool workspace_flags_are_zero) {
-  const int trans_b = trans_b_and_shape & 1, force = (trans_b_and_shape >> 4) & 0xf;
-  IEX_REQUIRE(M >= 0 && N >= 0 && K >= 0 && batch >= 0, IEX_ERR_BAD_ARGUMENT, "gemm: negative dimension");
-  if (M == 0 || N == 0 || batch == 0) return 0;
-  IEX_REQUIRE(A && B && C, IEX_ERR_BAD_ARGUMENT, "gemm: null pointer argument");
+int iex::gemm_dispatch(int dtype, int code, const GemmParams& given, int batch, hipStream_t stream, void* workspace, size_t workspace_bytes,
+                       bool workspace_flags_are_zero) {
+  GemmParams p = given;
+  const int trans_b = code & 1, trans_a = (code >> 1) & 1, force = (code >> 4) & 0xf;
+  IEX_REQUIRE(p.M >= 0 && p.N >= 0 && p.K >= 0 && batch >= 0, IEX_ERR_BAD_ARGUMENT, "gemm: negative dimension");
+  if (p.M == 0 || p.N == 0 || batch == 0) return 0;
+  IEX_REQUIRE(p.A && p.B && p.C, IEX_ERR_BAD_ARGUMENT, "gemm: null pointer argument");
   IEX_REQUIRE(dtype == IEX_F16 || dtype == IEX_BF16, IEX_ERR_UNSUPPORTED, "gemm: dtype must be fp16 or bf16");
-  IEX_REQUIRE(K > 0 && K % 8 == 0, IEX_ERR_UNSUPPORTED, "gemm: K must be a positive multiple of 8 (K=%d)", K);
-  IEX_REQUIRE(trans_b || N % 8 == 0, IEX_ERR_UNSUPPORTED, "gemm: N must be a multiple of 8 when B is (K,N) (N=%d)", N);
-  IEX_REQUIRE(aligned(A, 16) && aligned(B, 16), IEX_ERR_UNSUPPORTED, "gemm: operands must be 16-byte aligned");
-  IEX_REQUIRE(stride_a % 8 == 0 && stride_b % 8 == 0, IEX_ERR_UNSUPPORTED, "gemm: batch strides must be multiples of 8");
+  IEX_REQUIRE(!(trans_a && trans_b), IEX_ERR_UNSUPPORTED, "gemm: A as (K,M) goes with B as (K,N) only");
+  IEX_REQUIRE(p.K > 0 && (p.K % 8 == 0 || trans_a), IEX_ERR_UNSUPPORTED, "gemm: K must be a positive multiple of 8 (K=%d)", p.K);
+  if (!p.lda) p.lda = trans_a ? p.M : p.K;
+  if (!p.ldb) p.ldb = trans_b ? p.K : p.N;
+  if (!p.ldc) p.ldc = p.N;
+  if (!p.kb) p.kb = p.K;
+  IEX_REQUIRE(p.ldb % 8 == 0, IEX_ERR_UNSUPPORTED, "gemm: N must be a multiple of 8 when B is (K,N) (N=%d)", p.ldb);
+  IEX_REQUIRE(p.lda % 8 == 0, IEX_ERR_UNSUPPORTED, "gemm: M must be a multiple of 8 when A is (K,M) (M=%d)", p.lda);
+  IEX_REQUIRE(p.lda >= (trans_a ? p.M : p.K) && p.ldb >= (trans_b ? p.K : p.N) && p.ldc >= p.N && p.kb > 0 && p.kb <= p.K && p.K - p.kb < 8, IEX_ERR_BAD_ARGUMENT,
+              "gemm: a row stride is shorter than its row");
+  IEX_REQUIRE(aligned(p.A, 16) && aligned(p.B, 16), IEX_ERR_UNSUPPORTED, "gemm: operands must be 16-byte aligned");
+  IEX_REQUIRE(p.stride_a % 8 == 0 && p.stride_b % 8 == 0, IEX_ERR_UNSUPPORTED, "gemm: batch strides must be multiples of 8");
   IEX_REQUIRE(batch <= 65535, IEX_ERR_TOO_LARGE, "gemm: batch %d exceeds 65535", batch);
-  IEX_REQUIRE((long long)M * K < (1ll << 31) && (long long)N * K < (1ll << 31) && (long long)M * N < (1ll << 31),
+  IEX_REQUIRE((long long)(trans_a ? p.K : p.M) * p.lda < (1ll << 31) && (long long)(trans_b ? p.N : p.K) * p.ldb < (1ll << 31) &&
+                  (long long)p.M * p.ldc < (1ll << 31),
               IEX_ERR_TOO_LARGE, "gemm: an operand exceeds 2^31 elements per batch entry");
-  GemmParams p{M, N, K, A, B, C, stride_a, stride_b, stride_c, 0, 0, row_bias, relu, accumulate};
-  p.stream_out = (double)M * N * batch * 2 >= 128e6;
-  hipStream_t s = static_cast<hipStream_t>(stream);
+  p.stream_out = (double)p.M * p.N * batch * 2 >= 128e6;
   const bool bf = dtype == IEX_BF16;
-  if (bf && trans_b) return launch_shape<true, true>(p, batch, force, s, workspace, workspace_bytes, workspace_flags_are_zero);
-  if (bf && !trans_b) return launch_shape<true, false>(p, batch, force, s, workspace, workspace_bytes, workspace_flags_are_zero);
-  if (!bf && trans_b) return launch_shape<false, true>(p, batch, force, s, workspace, workspace_bytes, workspace_flags_are_zero);
-  return launch_shape<false, false>(p, batch, force, s, workspace, workspace_bytes, workspace_flags_are_zero);
+  auto launch = [&](auto kernel) { return kernel(p, batch, force, stream, workspace, workspace_bytes, workspace_flags_are_zero); };
+  if (trans_a) return bf ? launch(launch_shape<true, true, false>) : launch(launch_shape<false, true, false>);
+  if (trans_b) return bf ? launch(launch_shape<true, false, true>) : launch(launch_shape<false, false, true>);
+  return bf ? launch(launch_shape<true, false, false>) : launch(launch_shape<false, false, false>);
 }

@@ -31,15 +31,18 @@ struct GemmParams {
   void* C;
   long long stride_a, stride_b, stride_c;
   int tiles_m, tiles_n;
-  // epilogue beyond C = A * B, for the SpMM path that hands its product to this kernel:
-  // C = relu?((accumulate ? C : 0) + A * B + row_bias[row])
+  // epilogue beyond C = A * B: C = relu?(A * B + row_bias[row]), then with an auxiliary operand of C's shape and strides
+  // (16-byte aligned where C is; it may be C itself) C = that + aux (kGemmAdd) or C = that * silu(aux) (kGemmTimesSilu)
   const float* row_bias = nullptr;
-  int relu = 0, accumulate = 0;
+  int relu = 0;
+  int aux_mode = 0;
+  const void* aux = nullptr;
   int stream_out = 0;  // C is far larger than the caches: store it with the streaming hint
-  // K split over two workgroups per tile (gemm.hip): the row stride of A and of an (N, K) B when K above is only a
-  // part of it (0: K is the stride), where the first workgroup to finish a tile leaves its fp32 partial sums, and
-  // per tile a ticket counter and a "partial sums written" flag (both zero at launch)
-  int ldk = 0;
+  // row strides in elements, 0 = the natural one (A: K, or M where it is given as (K,M); B: K, or N where it is given as
+  // (K,N); C: N), and the rows of a (K,N) B that exist where K has been rounded up (0 = K; A is zero beyond them)
+  int lda = 0, ldb = 0, ldc = 0, kb = 0;
+  // K split over two workgroups per tile (gemm.hip): where the first workgroup to finish a tile leaves its fp32 partial
+  // sums, and per tile a ticket counter and a "partial sums written" flag (both zero at launch)
   float* split_ws = nullptr;
   int* split_flags = nullptr;
   // K split over split_parts workgroups per tile, every one of which leaves its partial sums in the workspace and draws
@@ -47,10 +50,11 @@ struct GemmParams {
   int split_parts = 0, split_part = 0;
 };
 
-// iex_gemm with the epilogue options above (gemm.hip).
-int gemm_dispatch(int dtype, int trans_b_and_shape, int M, int N, int K, const void* A, const void* B, void* C, int batch,
-                  long long stride_a, long long stride_b, long long stride_c, void* stream, const float* row_bias, int relu,
-                  int accumulate, void* workspace = nullptr, size_t workspace_bytes = 0, bool workspace_flags_are_zero = false);
+constexpr int kGemmAdd = 1, kGemmTimesSilu = 2;
+
+// iex_gemm with the options above (gemm.hip).  code: bit 0 = B is (N,K), bit 1 = A is (K,M), bits 4..7 = forced kernel.
+int gemm_dispatch(int dtype, int code, const GemmParams& p, int batch, hipStream_t stream, void* workspace = nullptr, size_t workspace_bytes = 0,
+                  bool workspace_flags_are_zero = false);
 // Bytes of workspace with which gemm_dispatch, left to choose, splits K over two workgroups per tile (0: this shape is
 // not split), and where in such a workspace the words sit that must be zero at launch (gemm_dispatch zeroes them with a
 // launch of its own unless the caller says it has: workspace_flags_are_zero).
@@ -186,126 +190,107 @@ struct GemmStage {
   }
 };
 
-// Writes the WM x WN accumulator blocks of one wavefront to C (rounded to the 16-bit type).
-template <bool BF16, int WM, int WN>
-__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const f32x16 (&acc)[WM][WN], unsigned short* __restrict__ C,
-                                                int m0, int n0, int wm, int wn, int lane, const float* partial = nullptr) {
-  typedef unsigned short u16;
-  // Swapped-operand result layout: lane holds row (lane % 32) of the 32x32 block and, in
-  // accumulator quad q, columns q*8 + (lane / 32)*4 .. +3.
-  const bool vec_ok = (p.N % 4 == 0) && ((reinterpret_cast<uintptr_t>(C) & 7) == 0);
-#pragma unroll
-  for (int i = 0; i < WM; ++i) {
-    const int gm = m0 + (wm * WM + i) * 32 + (lane & 31);
-    if (gm >= p.M) continue;
-    const float bias = p.row_bias ? p.row_bias[gm] : 0.f;
-#pragma unroll
-    for (int j = 0; j < WN; ++j) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int gn = n0 + (wn * WN + j) * 32 + q * 8 + (lane >> 5) * 4;
-        if (gn >= p.N) continue;
-        u16* dst = C + (size_t)gm * p.N + gn;
-        float x[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = acc[i][j][q * 4 + e];
-        if (partial) {   // the other half of K: this lane's sums in the same order, 256 floats per (block, quad)
-          const f32x4 o = *reinterpret_cast<const f32x4*>(partial + ((i * WN + j) * 4 + q) * 256);
-          x[0] += o.x, x[1] += o.y, x[2] += o.z, x[3] += o.w;
-        }
-        if (p.accumulate) {
-          if (vec_ok) {
-            const u32x2 w = *reinterpret_cast<const u32x2*>(dst);
-            x[0] += f16_to_32((u16)(w.x & 0xffffu), BF16);
-            x[1] += f16_to_32((u16)(w.x >> 16), BF16);
-            x[2] += f16_to_32((u16)(w.y & 0xffffu), BF16);
-            x[3] += f16_to_32((u16)(w.y >> 16), BF16);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (gn + e < p.N) x[e] += f16_to_32(dst[e], BF16);
-          }
-        }
-        u16 h[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float y = x[e] + bias;
-          if (p.relu) y = fmaxf(y, 0.f);
-          h[e] = f32_to_16(y, BF16);
-        }
-        if (vec_ok) {
-          u32x2 w;
-          w.x = (unsigned)h[0] | ((unsigned)h[1] << 16);
-          w.y = (unsigned)h[2] | ((unsigned)h[3] << 16);
-          *reinterpret_cast<u32x2*>(dst) = w;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (gn + e < p.N) dst[e] = h[e];
-        }
-      }
-    }
-  }
-}
-
-// The same, through LDS: a lane's accumulators are 4 adjacent columns of 32 different rows, so the
-// direct store writes 32 pieces of 16 bytes per instruction; here each 32-row block of the wavefront's
-// tile is laid out in the wavefront's own slice of LDS (rows padded by 16 bytes) and read back 16 lanes
-// per row, so a store instruction writes 4 rows of WN * 64 contiguous bytes.  A GEMM with a short K is a
-// writer of its output: 16 x 4096 x 4096 outputs with K = 64 went from 1.7 TB/s to the rate of a fill.
-// `lds` = this wavefront's slice, gemm_store_lds_bytes<WN>() bytes, nobody else touches it (no barrier
-// needed: the LDS operations of one wavefront execute in order).  Needs N % 8 == 0, a 16-byte aligned
-// C and no accumulation; `stream`: store with the streaming hint.
+// Writes the WM x WN accumulator blocks of one wavefront to C (rounded to the 16-bit type), through LDS: a lane's
+// accumulators are 4 adjacent columns of 32 different rows, so a direct store would write 32 pieces of 16 bytes per
+// instruction; here each 32-row block of the wavefront's tile is laid out in the wavefront's own slice of LDS (rows padded
+// by 16 bytes) and read back 16 lanes per row, so a store instruction writes 4 rows of WN * 64 contiguous bytes.  A GEMM
+// with a short K is a writer of its output: 16 x 4096 x 4096 outputs with K = 64 went from 1.7 TB/s to the rate of a fill.
+// An auxiliary operand takes the same way in before: rows read 16 lanes at a time, picked up by the lanes that hold their
+// sums, combined in fp32 and rounded once.  Rows of C that are not 16-byte aligned (any N, any pointer) are stored with
+// vectors at element alignment, the columns past the last whole vector one by one.
+// `lds` = this wavefront's slice, gemm_store_lds_bytes<WN>() bytes, nobody else touches it (no barrier needed: the LDS
+// operations of one wavefront execute in order).  `stream`: store with the streaming hint.  `partial`: another half of the
+// sums in this lane's order, 256 floats per (block, quad).
 template <int WN>
 constexpr int gemm_store_lds_bytes() { return 32 * (WN * 64 + 16); }
 
 template <bool BF16, int WM, int WN>
-__device__ __forceinline__ void gemm_store_tile_lds(const GemmParams& p, const f32x16 (&acc)[WM][WN], unsigned short* __restrict__ C,
-                                                    int m0, int n0, int wm, int wn, int lane, unsigned char* lds, bool stream,
-                                                    const float* partial = nullptr) {
+__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const f32x16 (&acc)[WM][WN], unsigned short* __restrict__ C,
+                                                const unsigned short* aux, int m0, int n0, int wm, int wn, int lane, unsigned char* lds,
+                                                bool stream, const float* partial = nullptr) {
   typedef unsigned short u16;
+  typedef u32x4 u128_a2 __attribute__((aligned(2)));
   constexpr int ROWB = WN * 64 + 16;   // bytes of a padded row
   constexpr int CPR = WN * 4;          // 16-byte chunks per row
   constexpr int RPI = kWave / CPR;     // rows a store instruction covers
   static_assert(kWave % CPR == 0 && 32 % RPI == 0, "whole rows per instruction");
+  const int ldc = p.ldc ? p.ldc : p.N;
+  const int chunk = lane % CPR;
+  const int gn = n0 + wn * WN * 32 + chunk * 8;
+  const int here = min(p.N - gn, 8);   // columns of this lane's chunk that exist (none: <= 0)
+  const bool whole = p.N % 8 == 0 && ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;   // (uniform)
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
     const int row0 = m0 + (wm * WM + i) * 32;
     if (row0 >= p.M) break;  // (uniform)
     const int gm_w = min(row0 + (lane & 31), p.M - 1);
     const float bias = p.row_bias ? p.row_bias[gm_w] : 0.f;
+    if (aux) {
+#pragma unroll
+      for (int t = 0; t < 32 / RPI; ++t) {
+        const int r = t * RPI + lane / CPR;
+        const u16* src = aux + (size_t)min(row0 + r, p.M - 1) * ldc + gn;
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (here == 8) {
+          v = whole ? *reinterpret_cast<const u32x4*>(src) : *reinterpret_cast<const u128_a2*>(src);
+        } else {
+          unsigned w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (e < here) w[e / 2] |= (unsigned)src[e] << (16 * (e & 1));
+          v = u32x4{w[0], w[1], w[2], w[3]};
+        }
+        *reinterpret_cast<u32x4*>(lds + r * ROWB + chunk * 16) = v;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < WN; ++j) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         u16 h[4];
+        u32x2* at = reinterpret_cast<u32x2*>(lds + (lane & 31) * ROWB + (j * 32 + q * 8 + (lane >> 5) * 4) * 2);
         f32x4 o = {0.f, 0.f, 0.f, 0.f};
         if (partial) o = *reinterpret_cast<const f32x4*>(partial + ((i * WN + j) * 4 + q) * 256);   // the other half of K
+        float other[4] = {0.f, 0.f, 0.f, 0.f};
+        if (aux) {
+          const u32x2 w = *at;
+          other[0] = f16_to_32((u16)(w.x & 0xffffu), BF16);
+          other[1] = f16_to_32((u16)(w.x >> 16), BF16);
+          other[2] = f16_to_32((u16)(w.y & 0xffffu), BF16);
+          other[3] = f16_to_32((u16)(w.y >> 16), BF16);
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float y = acc[i][j][q * 4 + e] + o[e] + bias;
+          if (aux && p.aux_mode == kGemmAdd) y += other[e];
           if (p.relu) y = fmaxf(y, 0.f);
+          if (aux && p.aux_mode == kGemmTimesSilu) y *= other[e] / (1.f + __expf(-other[e]));
           h[e] = f32_to_16(y, BF16);
         }
         u32x2 w;
         w.x = (unsigned)h[0] | ((unsigned)h[1] << 16);
         w.y = (unsigned)h[2] | ((unsigned)h[3] << 16);
-        *reinterpret_cast<u32x2*>(lds + (lane & 31) * ROWB + (j * 32 + q * 8 + (lane >> 5) * 4) * 2) = w;
+        *at = w;
       }
     }
-    const int chunk = lane % CPR;
-    const int gn = n0 + wn * WN * 32 + chunk * 8;
 #pragma unroll
     for (int t = 0; t < 32 / RPI; ++t) {
       const int r = t * RPI + lane / CPR;
       const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * ROWB + chunk * 16);
-      if (row0 + r < p.M && gn < p.N) {
-        u16* dst = C + (size_t)(row0 + r) * p.N + gn;
-        if (stream) {
+      if (row0 + r < p.M && here > 0) {
+        u16* dst = C + (size_t)(row0 + r) * ldc + gn;
+        if (whole && stream) {
           asm volatile("" : "+v"(dst));  // (keeps the compiler from merging this store with the plain one and dropping the hint)
           __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));
-        } else {
+        } else if (whole) {
           *reinterpret_cast<u32x4*>(dst) = v;
+        } else if (here == 8) {
+          *reinterpret_cast<u128_a2*>(dst) = v;
+        } else {
+          const unsigned w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (e < here) dst[e] = (u16)(w[e / 2] >> (16 * (e & 1)));
         }
       }
     }
@@ -434,7 +419,9 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int tile_m, int t
     if (kt < KT) step(kt++, std::integral_constant<int, 0>{});
   }
 
-  gemm_store_tile<BF16, WM, WN>(p, acc, C, m0, n0, wm, wn, lane);
+  static_assert(2 * WCN * gemm_store_lds_bytes<WN>() <= gemm_lds_bytes<TRANS_B, WM, WN, WCN, BK>(), "the epilogue fits the buffers");
+  __syncthreads();  // everybody has read its last fragments
+  gemm_store_tile<BF16, WM, WN>(p, acc, C, nullptr, m0, n0, wm, wn, lane, smem + wave * gemm_store_lds_bytes<WN>(), p.stream_out != 0);
 }
 
 }  // namespace iex

@@ -13,9 +13,9 @@
 //   K-contiguous operands (A, and B given as (N, K)): LDS row = BK elements; position (row, c)
 //     holds global chunk c ^ sw(row), sw(row) = (row >> 2) & 3 for BK = 32 ((row >> 1) & 7 for 64):
 //     the 16 lanes of a 128-bit operand read hit 16 different 4-bank groups.
-//   B given as (K, N): LDS row = BN elements; position (k, c) holds global chunk c ^ ((k & 3) << 2):
-//     the 32 lanes of a transpose read (4 k rows x 2 column halves x 32 bytes) hit 8 different
-//     8-bank groups.
+//   B given as (K, N), A given as (K, M): LDS row = BN (BM) elements; position (k, c) holds global chunk
+//     c ^ ((k & 3) << 2): the 32 lanes of a transpose read (4 k rows x 2 column halves x 32 bytes) hit 8 different
+//     8-bank groups.  (64 elements per row, of which two share the 64 banks: c ^ ((k & 2) << 1).)
 // Pipeline: STAGES LDS stages; the operand fragments of a 16-wide sub-step are read from LDS while
 // the MFMAs of the sub-step before it run, and once per tile (before the first fragment read of
 // tile t+1): wait for my loads of tile t+1 | barrier | issue tile t+STAGES-1, between MFMAs, into
@@ -66,7 +66,31 @@ __device__ __forceinline__ bool xcd_tile(int block, int tiles_m, int tiles_n, in
   return true;
 }
 
-template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, int BK, int STAGES, int SPLIT = 0>
+// Chunk permutation of k row kr of an operand whose LDS rows hold ROW_ELEMS elements of one k.
+template <int ROW_ELEMS>
+__device__ __forceinline__ int kn_swizzle(int kr) { return ROW_ELEMS >= 128 ? (kr & 3) << 2 : (kr & 2) << 1; }
+
+// Operand fragment (8 k of a lane's row or column) out of LDS rows of ROW_BYTES that hold one k each, by two transpose reads.
+template <int ROW_BYTES>
+__device__ __forceinline__ u32x4 kn_fragment(const unsigned char* at) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 4 * ROW_BYTES));
+  const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+  return u32x4{l2.x, l2.y, h2.x, h2.y};
+}
+
+// Where, inside such a stage, a lane's fragment of the 32 rows (columns) `block` starts: lane group q = lane / 16 covers
+// column half (q % 2) and k half (q / 2) of a sub-step; lane r of a group points at k row r / 4 and columns
+// 4 * (r % 4) .. + 3 of its half.
+template <int ROW_ELEMS>
+__device__ __forceinline__ int kn_fragment_offset(int lane, int block) {
+  const int kr = (lane >> 5) * 8 + ((lane & 15) >> 2);
+  const int c = (block * 4 + ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) ^ kn_swizzle<ROW_ELEMS>(kr);
+  return kr * (ROW_ELEMS * 2) + c * 16 + (lane & 1) * 8;
+}
+
+template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, int BK, int STAGES, int SPLIT = 0, bool TRANS_A = false>
 __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, int tile_n, int z, unsigned char* smem) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32, WAVES = 2 * WCN;
   constexpr int CPR = BK / 8;          // 16-byte chunks per K-contiguous row
@@ -75,12 +99,13 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
   constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, STAGE_BYTES = A_BYTES + B_BYTES;
   constexpr int A_INSTR = A_BYTES / 1024 / WAVES, B_INSTR = B_BYTES / 1024 / WAVES;  // per wavefront and tile
   constexpr int LOADS = A_INSTR + B_INSTR;
-  constexpr int CPRB = BN / 8;         // (K,N) layout: chunks per k row
-  constexpr int RPIB = 64 / (CPRB < 64 ? CPRB : 64);  // (K,N) layout: k rows per instruction
+  constexpr int CPRB = BN / 8, CPRA = BM / 8;         // (K,N), (K,M) layout: chunks per k row
+  constexpr int RPIB = 64 / (CPRB < 64 ? CPRB : 64), RPIA = 64 / (CPRA < 64 ? CPRA : 64);  // ... k rows per instruction
   static_assert(BK == 32 || BK == 64, "K step");
   static_assert(A_INSTR >= 1 && B_INSTR >= 1 && A_BYTES % (1024 * WAVES) == 0 && B_BYTES % (1024 * WAVES) == 0,
                 "every wavefront fetches whole kilobytes of A and of B");
   static_assert(TRANS_B || (CPRB >= 16 && CPRB <= 64), "(K,N) layout: 128 <= BN <= 512");
+  static_assert(!TRANS_A || (CPRA >= 8 && CPRA <= 64), "(K,M) layout: 64 <= BM <= 512");
   static_assert(STAGES >= 3 && (BK / 16) % 2 == 0 && (STAGES - 2) * LOADS < 64, "stages in flight must fit the load counter");
   typedef unsigned short u16;
   typedef __attribute__((address_space(3))) unsigned char lds_u8;
@@ -94,17 +119,24 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
   const u16* __restrict__ B = static_cast<const u16*>(p.B) + (size_t)z * p.stride_b;
   u16* __restrict__ C = static_cast<u16*>(p.C) + (size_t)z * p.stride_c;
   const unsigned lds0 = (unsigned)(size_t)(lds_u8*)smem;  // LDS byte address of stage 0
-  const int ld = p.ldk ? p.ldk : p.K;  // row stride of the K-contiguous operands
+  const int lda = p.lda ? p.lda : TRANS_A ? p.M : p.K, ldb = p.ldb ? p.ldb : TRANS_B ? p.K : p.N;   // row strides
+  const int last_kb = (p.kb ? p.kb : p.K) - 1;   // the last k row of a (K,N) B
 
   // ---- what this lane fetches: per instruction a row pointer (or a column offset) and a chunk
-  const u16* a_row[A_INSTR];
-  int a_k8[A_INSTR];  // element offset of the chunk inside a K step
+  const u16* a_row[A_INSTR];  // (M,K): row pointer; (K,M): A + clamped row
+  int a_k8[A_INSTR];          // (M,K): element offset of the chunk inside a K step; (K,M): k row inside a K step
 #pragma unroll
   for (int q = 0; q < A_INSTR; ++q) {
-    const int row = (wave * A_INSTR + q) * RPI + lane / CPR;
-    const int sw = CPR == 4 ? (row >> 2) & 3 : (row >> 1) & 7;
-    a_row[q] = A + (size_t)min(m0 + row, p.M - 1) * ld;
-    a_k8[q] = ((lane % CPR) ^ sw) * 8;
+    if constexpr (TRANS_A) {
+      const int kr = (wave * A_INSTR + q) * RPIA + lane / CPRA;
+      a_row[q] = A + min(m0 + ((lane % CPRA) ^ kn_swizzle<BM>(kr)) * 8, lda - 8);
+      a_k8[q] = kr;
+    } else {
+      const int row = (wave * A_INSTR + q) * RPI + lane / CPR;
+      const int sw = CPR == 4 ? (row >> 2) & 3 : (row >> 1) & 7;
+      a_row[q] = A + (size_t)min(m0 + row, p.M - 1) * lda;
+      a_k8[q] = ((lane % CPR) ^ sw) * 8;
+    }
   }
   const u16* b_row[B_INSTR];  // (N,K): row pointer; (K,N): B + clamped column
   int b_k8[B_INSTR];          // (N,K): chunk offset inside a K step; (K,N): k row inside a K step
@@ -113,12 +145,11 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
     if constexpr (TRANS_B) {
       const int row = (wave * B_INSTR + q) * RPI + lane / CPR;
       const int sw = CPR == 4 ? (row >> 2) & 3 : (row >> 1) & 7;
-      b_row[q] = B + (size_t)min(n0 + row, p.N - 1) * ld;
+      b_row[q] = B + (size_t)min(n0 + row, p.N - 1) * ldb;
       b_k8[q] = ((lane % CPR) ^ sw) * 8;
     } else {
       const int kr = (wave * B_INSTR + q) * RPIB + lane / CPRB;
-      const int c = (lane % CPRB) ^ ((kr & 3) << 2);
-      b_row[q] = B + min(n0 + c * 8, p.N - 8);
+      b_row[q] = B + min(n0 + ((lane % CPRB) ^ kn_swizzle<BN>(kr)) * 8, ldb - 8);
       b_k8[q] = kr;
     }
   }
@@ -130,14 +161,17 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
     const int k0 = min(kt, KT - 1) * BK;  // past the end: the last tile again, into a stage nobody reads
     if (q < A_INSTR) {
       const unsigned base = lds0 + stage * STAGE_BYTES + wave * (A_INSTR * 1024);
-      lds_dma16(a_row[q] + min(k0 + a_k8[q], last_k8), __builtin_amdgcn_readfirstlane(base + q * 1024));
+      if constexpr (TRANS_A)
+        lds_dma16(a_row[q] + (size_t)min(k0 + a_k8[q], p.K - 1) * lda, __builtin_amdgcn_readfirstlane(base + q * 1024));
+      else
+        lds_dma16(a_row[q] + min(k0 + a_k8[q], last_k8), __builtin_amdgcn_readfirstlane(base + q * 1024));
     } else {
       const int qb = q - A_INSTR;
       const unsigned bbase = lds0 + stage * STAGE_BYTES + A_BYTES + wave * (B_INSTR * 1024);
       if constexpr (TRANS_B)
         lds_dma16(b_row[qb] + min(k0 + b_k8[qb], last_k8), __builtin_amdgcn_readfirstlane(bbase + qb * 1024));
       else
-        lds_dma16(b_row[qb] + (size_t)min(k0 + b_k8[qb], p.K - 1) * p.N, __builtin_amdgcn_readfirstlane(bbase + qb * 1024));
+        lds_dma16(b_row[qb] + (size_t)min(k0 + b_k8[qb], last_kb) * ldb, __builtin_amdgcn_readfirstlane(bbase + qb * 1024));
     }
   };
   auto issue = [&](int kt, int stage) {
@@ -170,42 +204,34 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
   constexpr int KS = BK / 16;
   const int frow = lane & 31, fkh = lane >> 5;
   const int fsw = CPR == 4 ? (frow >> 2) & 3 : (frow >> 1) & 7;
-  int a_off[KS];
+  int a_off[TRANS_A ? WM : KS];
+  if constexpr (TRANS_A) {
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) a_off[ks] = (wm * WM * 32 + frow) * RB + (((ks * 2 + fkh) ^ fsw) * 16);
-  constexpr int NB = TRANS_B ? KS : WN;
-  int b_off[NB];
+    for (int i = 0; i < WM; ++i) a_off[i] = kn_fragment_offset<BM>(lane, wm * WM + i);
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) a_off[ks] = (wm * WM * 32 + frow) * RB + (((ks * 2 + fkh) ^ fsw) * 16);
+  }
+  int b_off[TRANS_B ? KS : WN];
   if constexpr (TRANS_B) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) b_off[ks] = A_BYTES + (wn * WN * 32 + frow) * RB + (((ks * 2 + fkh) ^ fsw) * 16);
   } else {
-    // lane group q = lane / 16 covers column half (q % 2) and k half (q / 2) of a sub-step; lane r of a
-    // group points at k row r / 4 and columns 4 * (r % 4) .. + 3 of its half
-    const int kr = fkh * 8 + ((lane & 15) >> 2);
-    const int s = ((lane >> 2) & 3) << 2;
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      const int c = ((wn * WN + j) * 4 + ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) ^ s;
-      b_off[j] = A_BYTES + kr * (BN * 2) + c * 16 + (lane & 1) * 8;
-    }
+    for (int j = 0; j < WN; ++j) b_off[j] = A_BYTES + kn_fragment_offset<BN>(lane, wn * WN + j);
   }
 
   u32x4 fa[2][WM], fb[2][WN];  // operand fragments of two consecutive sub-steps
   auto read_frags = [&](const unsigned char* st, int ks, int buf) {
 #pragma unroll
-    for (int i = 0; i < WM; ++i) fa[buf][i] = *reinterpret_cast<const u32x4*>(st + a_off[ks] + i * 32 * RB);
+    for (int i = 0; i < WM; ++i) {
+      if constexpr (TRANS_A) fa[buf][i] = kn_fragment<BM * 2>(st + a_off[i] + ks * 16 * (BM * 2));
+      else fa[buf][i] = *reinterpret_cast<const u32x4*>(st + a_off[ks] + i * 32 * RB);
+    }
 #pragma unroll
     for (int j = 0; j < WN; ++j) {
-      if constexpr (TRANS_B) {
-        fb[buf][j] = *reinterpret_cast<const u32x4*>(st + b_off[ks] + j * 32 * RB);
-      } else {
-        typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-        const unsigned char* q0 = st + b_off[j] + ks * 16 * (BN * 2);
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(q0));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(q0 + 4 * (BN * 2)));
-        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
-        fb[buf][j] = u32x4{l2.x, l2.y, h2.x, h2.y};
-      }
+      if constexpr (TRANS_B) fb[buf][j] = *reinterpret_cast<const u32x4*>(st + b_off[ks] + j * 32 * RB);
+      else fb[buf][j] = kn_fragment<BN * 2>(st + b_off[j] + ks * 16 * (BN * 2));
     }
   };
 
@@ -359,14 +385,10 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
           }
     }
   }
-  // the stages are free now: row-contiguous stores through LDS where the shape allows
   static_assert(WAVES * gemm_store_lds_bytes<WN>() <= gemm_dma_lds_bytes<WM, WN, WCN, BK, STAGES>(), "the epilogue fits the stages");
-  if (!p.accumulate && p.N % 8 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0) {
-    __syncthreads();  // everybody has read its last fragments
-    gemm_store_tile_lds<BF16, WM, WN>(p, acc, C, m0, n0, wm, wn, lane, smem + wave * gemm_store_lds_bytes<WN>(), p.stream_out != 0, partial);
-  } else {
-    gemm_store_tile<BF16, WM, WN>(p, acc, C, m0, n0, wm, wn, lane, partial);
-  }
+  __syncthreads();  // everybody has read its last fragments: the stages are free
+  const u16* aux = p.aux ? static_cast<const u16*>(p.aux) + (size_t)z * p.stride_c : nullptr;
+  gemm_store_tile<BF16, WM, WN>(p, acc, C, aux, m0, n0, wm, wn, lane, smem + wave * gemm_store_lds_bytes<WN>(), p.stream_out != 0, partial);
 }
 
 }  // namespace iex

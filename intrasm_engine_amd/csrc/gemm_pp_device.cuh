@@ -37,7 +37,7 @@ namespace iex {
 template <bool BF16, bool TRANS_B, int WM, int WN, int WCN>
 constexpr int gemm_pp_lds_bytes() { return 3 * (2 * WM * 32) * 128 + 4 * (WCN * WN * 32) * 64; }
 
-template <bool BF16, bool TRANS_B, int WM, int WN, int WCN>
+template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, bool TRANS_A = false>
 __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, int tile_n, int z, unsigned char* smem) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32, WAVES = 2 * WCN;
   constexpr int SA = 3, SB = 4;                       // stages of A (64 k each) and of B (32 k each)
@@ -46,12 +46,13 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   constexpr int A_INSTR = A_STAGE / 1024 / WAVES;     // direct loads per wavefront and A tile
   constexpr int B_INSTR = B_STAGE / 1024 / WAVES;     // ... and B tile
   constexpr int LPP = A_INSTR / 2 + B_INSTR;          // loads per wavefront and phase
-  constexpr int CPRB = BN / 8;                        // (K,N) layout: chunks per k row
-  constexpr int RPIB = 64 / (CPRB < 64 ? CPRB : 64);  // (K,N) layout: k rows per instruction
+  constexpr int CPRB = BN / 8, CPRA = BM / 8;         // (K,N), (K,M) layout: chunks per k row
+  constexpr int RPIB = 64 / (CPRB < 64 ? CPRB : 64), RPIA = 64 / (CPRA < 64 ? CPRA : 64);  // ... k rows per instruction
   static_assert(WAVES == 8, "two wavefronts per SIMD");
   static_assert(A_INSTR >= 2 && A_INSTR % 2 == 0 && B_INSTR >= 1 && A_STAGE % (1024 * WAVES) == 0 && B_STAGE % (1024 * WAVES) == 0,
                 "every wavefront fetches whole kilobytes of A (in two halves) and of B");
   static_assert(TRANS_B || (CPRB >= 16 && CPRB <= 64), "(K,N) layout: 128 <= BN <= 512");
+  static_assert(!TRANS_A || (CPRA >= 16 && CPRA <= 64), "(K,M) layout: 128 <= BM <= 512");
   static_assert(3 * LPP < 64, "loads in flight must fit the load counter");
   typedef unsigned short u16;
   typedef __attribute__((address_space(3))) unsigned char lds_u8;
@@ -66,23 +67,25 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   const u16* __restrict__ B = static_cast<const u16*>(p.B) + (size_t)z * p.stride_b;
   u16* __restrict__ C = static_cast<u16*>(p.C) + (size_t)z * p.stride_c;
   const unsigned lds0 = (unsigned)(size_t)(lds_u8*)smem;
-  const int ld = p.ldk ? p.ldk : p.K;  // row stride of the K-contiguous operands
+  const int lda = p.lda ? p.lda : TRANS_A ? p.M : p.K, ldb = p.ldb ? p.ldb : TRANS_B ? p.K : p.N;   // row strides
+  const int last_kb = (p.kb ? p.kb : p.K) - 1;   // the last k row of a (K,N) B
 
   // ---- what this lane fetches.  A: 8 rows of 128 bytes per instruction, LDS position (row, c) holds global chunk
   // c ^ ((row >> 1) & 7).  B as (N,K): 16 rows of 64 bytes, chunk c ^ ((row >> 2) & 3).  B as (K,N): k rows of BN
-  // elements, chunk c ^ ((k & 3) << 2).
-  const u16* a_ptr[A_INSTR];   // row pointer + chunk offset, advanced by 64 k per A tile
+  // elements, chunk c ^ ((k & 3) << 2), and A as (K,M) likewise, 64 k rows of BM elements per stage.
+  const u16* a_ptr[A_INSTR];   // (M,K): row pointer + chunk offset, advanced by 64 k per A tile; (K,M): A + clamped row
+  int a_k8[A_INSTR];           // (M,K): chunk offset inside a tile; (K,M): k row inside a tile
 #pragma unroll
   for (int q = 0; q < A_INSTR; ++q) {
-    const int row = (wave * A_INSTR + q) * 8 + lane / 8;
-    const int sw = (row >> 1) & 7;
-    a_ptr[q] = A + (size_t)min(m0 + row, p.M - 1) * ld + ((lane % 8) ^ sw) * 8;
-  }
-  int a_k8[A_INSTR];
-#pragma unroll
-  for (int q = 0; q < A_INSTR; ++q) {
-    const int row = (wave * A_INSTR + q) * 8 + lane / 8;
-    a_k8[q] = ((lane % 8) ^ ((row >> 1) & 7)) * 8;
+    if constexpr (TRANS_A) {
+      const int kr = (wave * A_INSTR + q) * RPIA + lane / CPRA;
+      a_ptr[q] = A + min(m0 + ((lane % CPRA) ^ kn_swizzle<BM>(kr)) * 8, lda - 8);
+      a_k8[q] = kr;
+    } else {
+      const int row = (wave * A_INSTR + q) * 8 + lane / 8;
+      a_k8[q] = ((lane % 8) ^ ((row >> 1) & 7)) * 8;
+      a_ptr[q] = A + (size_t)min(m0 + row, p.M - 1) * lda + a_k8[q];
+    }
   }
   const u16* b_row[B_INSTR];
   int b_k8[B_INSTR];
@@ -91,12 +94,11 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
     if constexpr (TRANS_B) {
       const int row = (wave * B_INSTR + q) * 16 + lane / 4;
       const int sw = (row >> 2) & 3;
-      b_row[q] = B + (size_t)min(n0 + row, p.N - 1) * ld;
+      b_row[q] = B + (size_t)min(n0 + row, p.N - 1) * ldb;
       b_k8[q] = ((lane % 4) ^ sw) * 8;
     } else {
       const int kr = (wave * B_INSTR + q) * RPIB + lane / CPRB;
-      const int c = (lane % CPRB) ^ ((kr & 3) << 2);
-      b_row[q] = B + min(n0 + c * 8, p.N - 8);
+      b_row[q] = B + min(n0 + ((lane % CPRB) ^ kn_swizzle<BN>(kr)) * 8, ldb - 8);
       b_k8[q] = kr;
     }
   }
@@ -111,8 +113,12 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
     const unsigned base = lds0 + (t % SA) * A_STAGE + wave * (A_INSTR * 1024);
 #pragma unroll
     for (int q = h * (A_INSTR / 2); q < (h + 1) * (A_INSTR / 2); ++q) {
-      const int over = max(k0 + a_k8[q] - last_k8, 0);   // a chunk past the last one of the row: that one instead
-      lds_dma16(a_ptr[q] + (k0 - over), __builtin_amdgcn_readfirstlane(base + q * 1024));
+      if constexpr (TRANS_A) {
+        lds_dma16(a_ptr[q] + (size_t)min(k0 + a_k8[q], p.K - 1) * lda, __builtin_amdgcn_readfirstlane(base + q * 1024));
+      } else {
+        const int over = max(k0 + a_k8[q] - last_k8, 0);   // a chunk past the last one of the row: that one instead
+        lds_dma16(a_ptr[q] + (k0 - over), __builtin_amdgcn_readfirstlane(base + q * 1024));
+      }
     }
   };
   auto issue_b = [&](int t) {
@@ -123,7 +129,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
       if constexpr (TRANS_B)
         lds_dma16(b_row[q] + min(k0 + b_k8[q], last_k8), __builtin_amdgcn_readfirstlane(base + q * 1024));
       else
-        lds_dma16(b_row[q] + (size_t)min(k0 + b_k8[q], p.K - 1) * p.N, __builtin_amdgcn_readfirstlane(base + q * 1024));
+        lds_dma16(b_row[q] + (size_t)min(k0 + b_k8[q], last_kb) * ldb, __builtin_amdgcn_readfirstlane(base + q * 1024));
     }
   };
   // entries at k >= K must be zero: clamped addresses delivered copies of real data.  Phase ph is the last one.
@@ -150,24 +156,21 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
 
   // ---- operand read addresses inside a stage (bytes), one per 16-wide sub-step
   const int frow = lane & 31, fkh = lane >> 5;
-  int a_off[4];   // the four sub-steps of an A tile
+  int a_off[TRANS_A ? WM : 4];   // the four sub-steps of an A tile, or the row blocks of a (K,M) one
+  if constexpr (TRANS_A) {
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) a_off[ks] = (wm * WM * 32 + frow) * 128 + (((ks * 2 + fkh) ^ ((frow >> 1) & 7)) * 16);
-  constexpr int NB = TRANS_B ? 2 : WN;
-  int b_off[NB];
+    for (int i = 0; i < WM; ++i) a_off[i] = kn_fragment_offset<BM>(lane, wm * WM + i);
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) a_off[ks] = (wm * WM * 32 + frow) * 128 + (((ks * 2 + fkh) ^ ((frow >> 1) & 7)) * 16);
+  }
+  int b_off[TRANS_B ? 2 : WN];
   if constexpr (TRANS_B) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) b_off[ks] = B_BASE + (wn * WN * 32 + frow) * 64 + (((ks * 2 + fkh) ^ ((frow >> 2) & 3)) * 16);
   } else {
-    // lane group q = lane / 16 covers column half (q % 2) and k half (q / 2) of a sub-step; lane r of a
-    // group points at k row r / 4 and columns 4 * (r % 4) .. + 3 of its half
-    const int kr = fkh * 8 + ((lane & 15) >> 2);
-    const int s = ((lane >> 2) & 3) << 2;
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      const int c = ((wn * WN + j) * 4 + ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) ^ s;
-      b_off[j] = B_BASE + kr * (BN * 2) + c * 16 + (lane & 1) * 8;
-    }
+    for (int j = 0; j < WN; ++j) b_off[j] = B_BASE + kn_fragment_offset<BN>(lane, wn * WN + j);
   }
 
   u32x4 fa[2][WM], fb[2][WN];  // the operand fragments of one phase (two sub-steps of 16)
@@ -180,21 +183,15 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
     const unsigned char* sb = smem + (ph % SB) * B_STAGE;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const int ao = a_off[2 * h + s];
 #pragma unroll
-      for (int i = 0; i < WM; ++i) fa[s][i] = *reinterpret_cast<const u32x4*>(sa + ao + i * 32 * 128);
+      for (int i = 0; i < WM; ++i) {
+        if constexpr (TRANS_A) fa[s][i] = kn_fragment<BM * 2>(sa + a_off[i] + (2 * h + s) * 16 * (BM * 2));
+        else fa[s][i] = *reinterpret_cast<const u32x4*>(sa + a_off[2 * h + s] + i * 32 * 128);
+      }
 #pragma unroll
       for (int j = 0; j < WN; ++j) {
-        if constexpr (TRANS_B) {
-          fb[s][j] = *reinterpret_cast<const u32x4*>(sb + b_off[s] + j * 32 * 64);
-        } else {
-          typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-          const unsigned char* q0 = sb + b_off[j] + s * 16 * (BN * 2);
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(q0));
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(q0 + 4 * (BN * 2)));
-          const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
-          fb[s][j] = u32x4{l2.x, l2.y, h2.x, h2.y};
-        }
+        if constexpr (TRANS_B) fb[s][j] = *reinterpret_cast<const u32x4*>(sb + b_off[s] + j * 32 * 64);
+        else fb[s][j] = kn_fragment<BN * 2>(sb + b_off[j] + s * 16 * (BN * 2));
       }
     }
     issue_a((ph >> 1) + 2, parity);
@@ -281,12 +278,9 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   wait_vmcnt<0>();  // the re-fetched last tiles: nothing may still be writing LDS when the stages are reused
 
   static_assert(WAVES * gemm_store_lds_bytes<WN>() <= SA * A_STAGE, "the epilogue fits the stages");
-  if (!p.accumulate && p.N % 8 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0) {
-    __syncthreads();  // everybody has read its last fragments and nobody's loads are in flight
-    gemm_store_tile_lds<BF16, WM, WN>(p, acc, C, m0, n0, wm, wn, lane, smem + wave * gemm_store_lds_bytes<WN>(), p.stream_out != 0, nullptr);
-  } else {
-    gemm_store_tile<BF16, WM, WN>(p, acc, C, m0, n0, wm, wn, lane, nullptr);
-  }
+  __syncthreads();  // everybody has read its last fragments and nobody's loads are in flight
+  const u16* aux = p.aux ? static_cast<const u16*>(p.aux) + (size_t)z * p.stride_c : nullptr;
+  gemm_store_tile<BF16, WM, WN>(p, acc, C, aux, m0, n0, wm, wn, lane, smem + wave * gemm_store_lds_bytes<WN>(), p.stream_out != 0);
 }
 
 }  // namespace iex

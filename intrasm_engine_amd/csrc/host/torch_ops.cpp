@@ -162,7 +162,7 @@ Tensor spmm(const Tensor& b, const Tensor& row_indices, const Tensor& values, co
   if (!known || (known->status & kBadPattern)) return python();
   const bool any_order = known->status & IEX_CSR_NOT_ASCENDING;
   const int itype = i16 ? IEX_I16 : IEX_I32;
-  int flags = (per_entry ? IEX_SPMM_PER_BATCH_VALUES : 0) | (accumulate ? IEX_SPMM_ACCUMULATE : 0) | (any_order ? IEX_SPMM_ANY_COLUMN_ORDER : 0);
+  int flags = IEX_SPMM_PAD_OPERANDS | (per_entry ? IEX_SPMM_PER_BATCH_VALUES : 0) | (accumulate ? IEX_SPMM_ACCUMULATE : 0) | (any_order ? IEX_SPMM_ANY_COLUMN_ORDER : 0);
   auto kind_of = [&](int f) { return iex_spmm_workspace_kind(dtype, itype, f, m, k, n, nonzeros, batch); };
   if (kind == Spmm::kPerEntry && !any_order && dtype != IEX_F32 && known->dense_share >= 0 && (double)batch * m * k >= kStructureCells) {
     // by the pattern's structure where a look at it has told, not by its density (the library's rule)
@@ -208,7 +208,7 @@ Tensor sddmm(const Tensor& a, const Tensor& b, const Tensor& row_indices, const 
   const auto known = note_of(row_offsets, column_indices, n);
   if (!known || (known->status & kBadPattern)) return python();
   const bool any_order = known->status & IEX_CSR_NOT_ASCENDING;
-  int flags = (summed ? IEX_SDDMM_SUM_OVER_BATCH : 0) | (any_order ? IEX_SDDMM_ANY_COLUMN_ORDER : 0);
+  int flags = IEX_SDDMM_PAD_OPERANDS | (summed ? IEX_SDDMM_SUM_OVER_BATCH : 0) | (any_order ? IEX_SDDMM_ANY_COLUMN_ORDER : 0);
   auto kind_of = [&](int f) { return iex_sddmm_workspace_kind(dtype, f, m, k, n, nonzeros, batch); };
   if (!summed && !any_order && dtype != IEX_F32 && known->dense_share >= 0 && (double)batch * m * n >= kStructureCells) {
     if (known->dense_share >= kStructureShare) flags |= kind_of(flags | IEX_SDDMM_FORCE_VARIANT(3)) == 3 ? IEX_SDDMM_FORCE_VARIANT(3) : 0;
@@ -268,6 +268,23 @@ Tensor gemm(const Tensor& a, const Tensor& b, bool trans_b) {
   return out;
 }
 
+// a^T @ b for a (K, M), b (K, N): the gradient of a linear layer's weight, without a transposed copy of a
+Tensor gemm_transposed_a(const Tensor& a, const Tensor& b) {
+  const int dtype = dtype_code(a.scalar_type());
+  if (forced || !plain(a, 2) || !plain(b, 2) || (dtype != IEX_F16 && dtype != IEX_BF16) || b.scalar_type() != a.scalar_type() ||
+      b.device() != a.device() || b.size(0) != a.size(0) || a.size(0) == 0 || a.size(1) % 8 != 0 || b.size(1) % 8 != 0)
+    return gemm(a.t().contiguous(), b, false);
+  const int64_t K = a.size(0), M = a.size(1), N = b.size(1);
+  const c10::DeviceGuard guard(a.device());
+  Tensor out = at::empty({M, N}, a.options());
+  const size_t ws_bytes = iex_gemm_workspace_bytes(dtype, 2, M, N, K, 1);
+  const Tensor ws = workspace(ws_bytes, a);
+  check(iex_gemm_ws(dtype, 2, M, N, K, a.const_data_ptr(), b.const_data_ptr(), out.data_ptr(), 1, 0, 0, 0, stream_of(a),
+                    ws.defined() ? ws.data_ptr() : nullptr, ws_bytes),
+        "gemm");
+  return out;
+}
+
 // ---- autograd: the plain calls of MySpMM and MyLinear (no recording, no forced kernels) -----------------------------
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
@@ -291,6 +308,27 @@ Tensor permuted(const Tensor& values, const Tensor& perm) {
   return out;
 }
 
+// A^T * grad from the CSR form of A where the transposed pattern's product would go by its dense form anyway (undefined
+// elsewhere)
+Tensor transposed_product(const Tensor& grad, const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t k) {
+  const int dtype = dtype_code(values.scalar_type());
+  if (dtype == IEX_F32 || dtype < 0 || forced || !plain(grad, 2) || !plain(values, 1) || grad.scalar_type() != values.scalar_type() ||
+      grad.device() != values.device() || values.size(0) != column_indices.size(0))
+    return Tensor();
+  const int64_t m = grad.size(0), n = grad.size(1), nonzeros = values.size(0);
+  const size_t bytes = m * k * n ? iex_spmm_transposed_workspace_bytes(dtype, m, k, n, nonzeros) : 0;
+  const auto known = note_of(row_offsets, column_indices, k);
+  if (!bytes || !known || known->status != 0) return Tensor();   // (canonical CSR only)
+  const c10::DeviceGuard guard(grad.device());
+  const Tensor ws = workspace(bytes, grad);
+  Tensor out = at::empty({k, n}, grad.options());
+  check(iex_spmm_transposed(dtype, column_indices.scalar_type() == at::kShort ? IEX_I16 : IEX_I32, m, k, n, nonzeros, values.const_data_ptr(),
+                            row_offsets.const_data_ptr<int>(), column_indices.const_data_ptr(), grad.const_data_ptr(), out.data_ptr(), stream_of(grad),
+                            ws.data_ptr(), bytes),
+        "spmm (transposed)");
+  return out;
+}
+
 struct TrainableSpmm : torch::autograd::Function<TrainableSpmm> {
   static Tensor forward(AutogradContext* ctx, const Tensor& b, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets,
                         const Tensor& column_indices, int64_t m, const Tensor& row_indices_t, const Tensor& row_offsets_t,
@@ -310,7 +348,8 @@ struct TrainableSpmm : torch::autograd::Function<TrainableSpmm> {
       out[2] = grad.scalar_type() == at::kFloat ? sddmm<true, true>(grad, dense, row_indices, row_offsets, columns)
                                                 : sddmm<false, true>(grad, dense, row_indices, row_offsets, columns);
     }
-    if (ctx->needs_input_grad(0)) out[0] = spmm_shared(grad, saved[5], permuted(values, saved[8]), saved[6], saved[7], dense.size(0));
+    if (ctx->needs_input_grad(0)) out[0] = transposed_product(grad, values, row_offsets, column_indices, dense.size(0));
+    if (ctx->needs_input_grad(0) && !out[0].defined()) out[0] = spmm_shared(grad, saved[5], permuted(values, saved[8]), saved[6], saved[7], dense.size(0));
     return out;
   }
 };
@@ -332,7 +371,7 @@ struct TrainableLinear : torch::autograd::Function<TrainableLinear> {
     const Tensor grad = grads[0].contiguous();
     variable_list out(2);
     if (ctx->needs_input_grad(0)) out[0] = gemm(grad, saved[1], false);
-    if (ctx->needs_input_grad(1)) out[1] = gemm(grad.t().contiguous(), saved[0], false);
+    if (ctx->needs_input_grad(1)) out[1] = gemm_transposed_a(grad, saved[0]);
     return out;
   }
 };

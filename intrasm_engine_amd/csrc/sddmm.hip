@@ -20,6 +20,7 @@
 #include <cmath>
 #include "iex_common.h"
 #include "sddmm_mfma_device.cuh"
+#include "spmm_dense_device.cuh"
 
 namespace iex {
 namespace {
@@ -33,6 +34,7 @@ struct SddmmParams {
   const void* rhs;
   void* out;
   int sum_over_batch, accumulate;
+  int pad = 0;   // the dense product may copy operands into the workspace (IEX_SDDMM_PAD_OPERANDS)
 };
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -281,24 +283,30 @@ int launch_typed(const SddmmParams& p, int wpr, hipStream_t stream) {
 // the dense GEMM computes all m * n dot products on the matrix cores in less time than that takes
 // once the mask is not very sparse, and a small kernel then picks the nonzeros' entries.
 // Same arithmetic per output (fp32 accumulation over k, one rounding to the 16-bit type).
-__global__ __launch_bounds__(256) void sample_dense_kernel(int m, int n, const int* __restrict__ row_offsets,
+__global__ __launch_bounds__(256) void sample_dense_kernel(int m, int ld, const int* __restrict__ row_offsets,
                                                            const int* __restrict__ cols,
                                                            const uint16_t* __restrict__ dense,
                                                            uint16_t* __restrict__ out) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= m) return;
   const int start = row_offsets[row], end = row_offsets[row + 1];
-  const uint16_t* drow = dense + (size_t)row * n;
+  const uint16_t* drow = dense + (size_t)row * ld;
   for (int j = start + lane_id(); j < end; j += kWave) out[j] = drow[cols[j]];
 }
 
 inline bool sddmm_dense_fits(int dtype, const SddmmParams& p) {
-  return (dtype == IEX_F16 || dtype == IEX_BF16) && !p.accumulate && !(p.sum_over_batch && p.batch > 1) &&
-         p.k > 0 && p.k % 8 == 0 && p.n % 8 == 0 && (long long)p.m * p.n < (1ll << 31) && aligned(p.lhs, 16) &&
-         aligned(p.rhs, 16);
+  return (dtype == IEX_F16 || dtype == IEX_BF16) && !p.accumulate && !(p.sum_over_batch && p.batch > 1) && p.k > 0 &&
+         (p.pad || (p.k % 8 == 0 && p.n % 8 == 0 && aligned(p.lhs, 16) && aligned(p.rhs, 16))) && (long long)p.m * round8(p.n) < (1ll << 31) &&
+         (long long)std::max(p.m, p.n) * round8(p.k) < (1ll << 31);
 }
 
-inline size_t sddmm_dense_bytes(const SddmmParams& p) { return (size_t)p.m * p.n * 2; }
+// The workspace: the product (rows of round8(n)), then copies of lhs and rhs where k or their addresses are no whole vectors.
+inline bool sddmm_dense_pads(const SddmmParams& p) { return p.k % 8 != 0 || !aligned(p.lhs, 16) || !aligned(p.rhs, 16); }
+inline size_t sddmm_dense_lhs_offset(const SddmmParams& p) { return round256((size_t)p.m * round8(p.n) * 2); }
+inline size_t sddmm_dense_rhs_offset(const SddmmParams& p) { return round256(sddmm_dense_lhs_offset(p) + (size_t)p.m * round8(p.k) * 2); }
+inline size_t sddmm_dense_bytes(const SddmmParams& p) {
+  return sddmm_dense_pads(p) ? sddmm_dense_rhs_offset(p) + (size_t)p.n * round8(p.k) * 2 : (size_t)p.m * round8(p.n) * 2;
+}
 
 // Time model fitted on MI355X (fp16).  Dense product per batch entry: three launches, the GEMM at
 // 1000 TFLOP/s or, with few tiles, 0.23 us per K step of 32 per round of 512 tiles of 128 x 128,
@@ -313,7 +321,8 @@ inline bool sddmm_dense_wins(const SddmmParams& p) {
   const double flops = 2.0 * p.m * p.n * p.k;
   const double tiles = (double)ceil_div(p.m, 128) * ceil_div(p.n, 128);
   const double product = std::max(flops / 1000e12, std::ceil(tiles / 512.0) * (p.k / 32.0) * 0.23e-6);
-  const double dense = p.batch * (16e-6 + product + ((double)p.m * p.n * 2 + (double)p.nnz * 8) / 4e12);
+  const double pad = sddmm_dense_pads(p) ? 8e-6 + 4.0 * ((double)p.m + p.n) * p.k / 4e12 : 0.0;
+  const double dense = p.batch * (16e-6 + pad + product + ((double)p.m * p.n * 2 + (double)p.nnz * 8) / 4e12);
   const double row_nnz = (double)p.nnz / p.m;
   const double chain = p.k > 256 ? std::ceil(row_nnz / (row_nnz >= 64.0 ? 16.0 : 4.0)) * (p.k / 128.0) * 0.12e-6 : 0.0;
   const double gather = std::max(8e-6 + (double)p.batch * p.nnz * p.k * 2 / 15e12, chain);
@@ -321,13 +330,24 @@ inline bool sddmm_dense_wins(const SddmmParams& p) {
 }
 
 int launch_sddmm_dense(int dtype, const SddmmParams& p, void* ws, hipStream_t stream) {
+  const int kp = round8(p.k), ld = round8(p.n);
+  unsigned char* at = static_cast<unsigned char*>(ws);
   for (int z = 0; z < p.batch; ++z) {
-    const uint16_t* lhs = static_cast<const uint16_t*>(p.lhs) + (size_t)z * p.m * p.k;
-    const uint16_t* rhs = static_cast<const uint16_t*>(p.rhs) + (size_t)z * p.n * p.k;
+    const void* lhs = static_cast<const uint16_t*>(p.lhs) + (size_t)z * p.m * p.k;
+    const void* rhs = static_cast<const uint16_t*>(p.rhs) + (size_t)z * p.n * p.k;
+    if (sddmm_dense_pads(p)) {
+      void *lhs_copy = at + sddmm_dense_lhs_offset(p), *rhs_copy = at + sddmm_dense_rhs_offset(p);
+      if (int rc = launch_pad_rows(p.m, p.k, lhs, p.m, kp, lhs_copy, 1, 0, stream)) return rc;
+      if (int rc = launch_pad_rows(p.n, p.k, rhs, p.n, kp, rhs_copy, 1, 0, stream)) return rc;
+      lhs = lhs_copy;
+      rhs = rhs_copy;
+    }
     // (the dispatcher, not the public entry point: that one starts a new trail of kernel names)
-    if (int rc = gemm_dispatch(dtype, 1, p.m, p.n, p.k, lhs, rhs, ws, 1, 0, 0, 0, stream, nullptr, 0, 0)) return rc;
+    GemmParams g{p.m, p.n, kp, lhs, rhs, ws, 0, 0, 0, 0, 0};
+    g.ldc = ld;
+    if (int rc = gemm_dispatch(dtype, 1, g, 1, stream)) return rc;
     note_kernel("sample_dense_kernel");
-    hipLaunchKernelGGL(sample_dense_kernel, dim3(ceil_div(p.m, 4)), dim3(256), 0, stream, p.m, p.n, p.row_offsets, p.cols,
+    hipLaunchKernelGGL(sample_dense_kernel, dim3(ceil_div(p.m, 4)), dim3(256), 0, stream, p.m, ld, p.row_offsets, p.cols,
                        static_cast<const uint16_t*>(ws), static_cast<uint16_t*>(p.out) + (size_t)z * p.nnz);
     if (int rc = check_hip(hipGetLastError(), "sddmm sampling launch")) return rc;
   }
@@ -409,7 +429,7 @@ int sddmm_workspace_kind(int dtype, int flags, int m, int k, int n, int nonzeros
   if (variant != 0 && variant != 7 && variant != 3) return 0;
   void* const some_aligned = reinterpret_cast<void*>(size_t(256));
   SddmmParams p{m, k, n, nonzeros, batch, nullptr, nullptr, nullptr, some_aligned, some_aligned, nullptr,
-                (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0};
+                (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0, (flags & IEX_SDDMM_PAD_OPERANDS) != 0};
   const bool any_order = (flags & IEX_SDDMM_ANY_COLUMN_ORDER) != 0;
   if (variant != 7 && sddmm_mfma_fits(dtype, p) && (variant == 3 || (!any_order && sddmm_mfma_wins(p)))) return 3;
   if (variant == 3 || !sddmm_dense_fits(dtype, p)) return 0;
@@ -422,7 +442,7 @@ size_t sddmm_workspace_bytes(int dtype, int flags, int m, int k, int n, int nonz
   if (variant != 0 && variant != 7 && variant != 3) return 0;
   void* const some_aligned = reinterpret_cast<void*>(size_t(256));
   SddmmParams p{m, k, n, nonzeros, batch, nullptr, nullptr, nullptr, some_aligned, some_aligned, nullptr,
-                (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0};
+                (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0, (flags & IEX_SDDMM_PAD_OPERANDS) != 0};
   const bool any_order = (flags & IEX_SDDMM_ANY_COLUMN_ORDER) != 0;
   if (variant != 7 && sddmm_mfma_fits(dtype, p) && (variant == 3 || (!any_order && sddmm_mfma_wins(p)))) return sddmm_mfma_bytes(p);
   if (variant == 3) return 0;
@@ -445,7 +465,7 @@ int sddmm_dispatch(int dtype, int flags, int m, int k, int n, int nonzeros, cons
   IEX_REQUIRE((long long)m * k < (1ll << 31) && (long long)n * k < (1ll << 31), IEX_ERR_TOO_LARGE,
               "sddmm: a dense operand exceeds 2^31 elements per batch entry");
   SddmmParams p{m, k, n, nonzeros, batch, row_indices, row_offsets, column_indices, lhs, rhs, out,
-                (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0};
+                (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0, (flags & IEX_SDDMM_PAD_OPERANDS) != 0};
   int wpr = (flags >> 8) & 0xff;  // forced (1 or 4), else from the mean row length
   if (wpr != 1 && wpr != 4) wpr = ((double)nonzeros / m >= 64.0) ? 4 : 1;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -465,7 +485,7 @@ int sddmm_dispatch(int dtype, int flags, int m, int k, int n, int nonzeros, cons
     const bool fits = sddmm_dense_fits(dtype, p);
     const bool room = workspace && aligned(workspace, 16) && workspace_bytes >= sddmm_dense_bytes(p);
     if (variant == 7) {
-      IEX_REQUIRE(fits, IEX_ERR_UNSUPPORTED, "sddmm: the dense-product path needs fp16 / bf16, plain store, one batch entry per output, k and n multiples of 8 and 16-byte aligned operands");
+      IEX_REQUIRE(fits, IEX_ERR_UNSUPPORTED, "sddmm: the dense-product path needs fp16 / bf16, plain store, one batch entry per output and, without IEX_SDDMM_PAD_OPERANDS, k and n multiples of 8 and 16-byte aligned operands");
       IEX_REQUIRE(room, IEX_ERR_BAD_ARGUMENT, "sddmm: the dense-product path needs a 16-byte aligned workspace of %zu bytes (iex_sddmm_ws)", sddmm_dense_bytes(p));
     }
     if (fits && room && (variant == 7 || sddmm_dense_wins(p))) return launch_sddmm_dense(dtype, p, workspace, s);

@@ -3,11 +3,11 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include "spmm_dense_device.cuh"
 #include "spmm_lds_device.cuh"
 #include "spmm_mfma2_device.cuh"
 #include "spmm_mfma3_device.cuh"
 #include "spmm_mfma_f32_device.cuh"
-#include "spmm_dense_device.cuh"
 #include "spmm_smallk_device.cuh"
 
 namespace iex {
@@ -523,21 +523,27 @@ inline int mfma3_windows(const SpmmParams& p) {
   return (density <= 0.33 || 2.0 * p.nnz == cells) ? 2 : 4;
 }
 
-// Dense form of A in the caller's workspace, then the dense GEMM (16-bit types, values shared by
-// the batch, plain store, no bias / ReLU).  What the shapes must satisfy, the workspace aside.
+// Dense form of A in the caller's workspace, then the dense GEMM (16-bit types, values shared by the batch).  The GEMM
+// wants rows of whole 16-byte chunks: the dense form gets them by zero columns up to a multiple of 8, a dense operand that
+// has none (n or its address) is copied into the workspace first.
 inline bool dense_path_fits(int elem_size, const SpmmParams& p, bool flagged) {
-  return elem_size == 2 && !flagged && p.nnz > 0 && p.k % 8 == 0 && p.n % 8 == 0 &&
-         (long long)p.m * p.k < (1ll << 31) && aligned(p.dense, 16) && aligned(p.out, 16);
+  return elem_size == 2 && !flagged && p.nnz > 0 && (p.pad || (p.k % 8 == 0 && p.n % 8 == 0 && aligned(p.dense, 16) && aligned(p.out, 16))) && (long long)p.m * round8(p.k) < (1ll << 31) && (long long)round8(p.k) * round8(p.n) < (1ll << 31);
 }
 
-inline size_t dense_path_bytes(const SpmmParams& p) { return (size_t)p.m * p.k * 2; }
+inline bool dense_path_pads(const SpmmParams& p) { return p.n % 8 != 0 || !aligned(p.dense, 16); }
+inline size_t dense_path_pad_offset(const SpmmParams& p) { return round256((size_t)p.m * round8(p.k) * 2); }
+inline size_t dense_path_bytes(const SpmmParams& p, int batch) {
+  return dense_path_pads(p) ? dense_path_pad_offset(p) + (size_t)batch * round8(p.k) * round8(p.n) * 2 : (size_t)p.m * round8(p.k) * 2;
+}
 
 // Whether the dense-form path is the faster one, from a time model fitted on MI355X (fp16):
 //   dense form + GEMM: two launches (8 us), m * k * 2 bytes written at 4 TB/s, the product at
 //     1000 TFLOP/s or, when the tiles are few, one round of 128 x 128 tiles per 512 tiles at 0.23 us
 //     per K step of 32 (4096^2, n <= 512: 40-45 us whatever the sparsity; 1024^2, n = 2048: 21 us);
 //   matrix-core SpMM kernels: 720 dense-equivalent TFLOP/s (2:4 4096^2, n = 8192: 0.40 against 0.27 ms
-//     for the dense form; 80 % 11008 x 4096: 0.93 / 0.69; 90 %, n = 2048: 0.27 / 0.23);
+//     for the dense form; 80 % 11008 x 4096: 0.93 / 0.69; 90 %, n = 2048: 0.27 / 0.23), or with few tiles a
+//     workgroup's chain of chunks of 128 columns, per chunk 3.5 us + 7 us * density for 128 x 512 tiles and
+//     4.5 + 21 for 128 x 256 tiles by four wavefronts (2:4 4096^2, n = 928: 482 us; 2760 x 2231 at 13 %, n = 1336: 126);
 //   gather kernels: nnz * n * 2 bytes through the L2 -> CU path at 26 TB/s (4096^2 at 70 %, n = 256:
 //     110 against 58 us; at 90 %, n = 256: 40 against 58; 11008 x 4096 at 95 %, n = 2048: 0.35 / 0.21 ms).
 //   a short K makes the GEMM a writer of its output at 3 TB/s (16 x 4096 x 4096, k = 64: 0.18 ms) and the
@@ -547,47 +553,79 @@ inline size_t dense_path_bytes(const SpmmParams& p) { return (size_t)p.m * p.k *
 // The dense form has to win by 15 % to be taken.  `few_columns`: the alternative is the few-columns kernel.
 // split_room: the workspace has room for the GEMM to take k in parts where it would (few tiles, long k: the K loop of a
 // tile then runs on several CUs; 4096^2 at 70-90 %, n = 128 / 256: 40 / 41 -> 27 / 32 us).
+//   rows of n elements that are no whole vectors are gathered in full-width tiles.
 inline bool dense_path_wins(const SpmmParams& p, int batch, int matrix_core_kind, bool few_columns, bool split_room = true) {
-  const double cells = (double)p.m * p.k, flops = 2.0 * cells * p.n * batch;
+  const double cells = (double)p.m * p.k, flops = 2.0 * cells * p.n * batch, density = p.nnz / std::max(cells, 1.0);
   const double out_bytes = (double)p.m * p.n * batch * 2;
   const double tiles = (double)ceil_div(p.m, 128) * ceil_div(p.n, 128) * batch;
-  const int parts = split_room && !p.accumulate ? gemm_auto_split_parts(p.m, p.n, p.k, batch) : 1;
+  const int parts = split_room && !p.accumulate ? gemm_auto_split_parts(p.m, p.n, round8(p.k), batch) : 1;
   const double product = std::max({flops / 1000e12, std::ceil(tiles / 512.0) * (p.k / 32.0) * 0.23e-6 / parts, out_bytes / 3e12});
-  const double dense_form = 8e-6 + cells * 2 / 4e12 + product;
+  const double pad = dense_path_pads(p) ? 4e-6 + 4.0 * p.k * p.n * batch / 4e12 : 0.0;
+  const double dense_form = 8e-6 + cells * 2 / 4e12 + pad + product;
   double other;
-  if (few_columns) other = 8e-6 + out_bytes / 4.5e12 + (double)p.nnz * batch * ceil_div(p.n, 512) * 10.0 / (256 * 2.1e9);
-  else if (matrix_core_kind) other = 8e-6 + std::max(flops / 720e12, out_bytes / 1.2e12);
-  else other = 8e-6 + (double)p.nnz * p.n * batch * 2 / 26e12 + out_bytes / 4e12;
+  if (few_columns) {
+    other = 8e-6 + out_bytes / 4.5e12 + (double)p.nnz * batch * ceil_div(p.n, 512) * 10.0 / (256 * 2.1e9);
+  } else if (matrix_core_kind) {
+    const bool wide = matrix_core_kind == 4;
+    const double rounds = std::ceil((double)ceil_div(p.m, kMfmaBM) * ceil_div(p.n, wide ? kMfma2BN : kMfmaBN) * batch / (wide ? 256.0 : 512.0));
+    const double chain = rounds * (p.k / 128.0) * (wide ? 3.5e-6 + 7e-6 * density : 4.5e-6 + 21e-6 * density);
+    other = 8e-6 + std::max({flops / 720e12, chain, out_bytes / 1.2e12});
+  } else {
+    const double columns = p.n % 8 == 0 || p.n < 256 ? p.n : ceil_div(p.n, 512) * 512;
+    other = 8e-6 + (double)p.nnz * columns * batch * 2 / 26e12 + out_bytes / 4e12;
+  }
   return 1.15 * dense_form < other;
 }
 
-// Behind the dense form (rounded up to 256 bytes) the workspace may hold what the GEMM wants for splitting K over two
+// Behind dense form and copy (rounded up to 256 bytes) the workspace may hold what the GEMM wants for splitting K over two
 // workgroups per tile (few tiles, long k: gemm_auto_split_bytes); the words it wants zero are zeroed by the kernel
 // that writes the dense form.
-inline size_t dense_path_split_offset(const SpmmParams& p) { return (dense_path_bytes(p) + 255) & ~size_t(255); }
-inline size_t dense_path_split_bytes(const SpmmParams& p, int batch) { return p.accumulate ? 0 : gemm_auto_split_bytes(p.m, p.n, p.k, batch); }
+inline size_t dense_path_split_offset(const SpmmParams& p, int batch) { return round256(dense_path_bytes(p, batch)); }
+inline size_t dense_path_split_bytes(const SpmmParams& p, int batch) { return p.accumulate ? 0 : gemm_auto_split_bytes(p.m, p.n, round8(p.k), batch); }
 
 inline bool dense_path_has_split_room(const SpmmParams& p, int batch, const Choice& ch) {
   const size_t split = dense_path_split_bytes(p, batch);
-  return split > 0 && ch.ws && aligned(ch.ws, 256) && ch.ws_bytes >= dense_path_split_offset(p) + split;
+  return split > 0 && ch.ws && aligned(ch.ws, 256) && ch.ws_bytes >= dense_path_split_offset(p, batch) + split;
+}
+
+template <typename IT>
+int launch_dense_form(int m, int ld, const int* row_offsets, const void* cols, const void* values, void* out, int* zero_words, int n_zero_words,
+                      hipStream_t stream) {
+  note_kernel("csr_to_dense_kernel<%s>", type_name<IT>());
+  hipLaunchKernelGGL((csr_to_dense_kernel<IT>), dim3(ceil_div(m, kDenseRows)), dim3(kDenseThreads), 0, stream, m, ld, row_offsets,
+                     static_cast<const IT*>(cols), static_cast<const uint16_t*>(values), static_cast<uint16_t*>(out), zero_words, n_zero_words);
+  return check_hip(hipGetLastError(), "spmm dense-form launch");
 }
 
 template <typename T, typename IT>
 int launch_dense_path(const SpmmParams& p, int batch, const Choice& ch, hipStream_t stream) {
-  const size_t split = dense_path_split_bytes(p, batch), offset = dense_path_split_offset(p);
+  const int kp = round8(p.k), np = round8(p.n);
+  const size_t split = dense_path_split_bytes(p, batch), offset = dense_path_split_offset(p, batch);
   const bool with_split = dense_path_has_split_room(p, batch, ch);
-  unsigned char* split_ws = with_split ? static_cast<unsigned char*>(ch.ws) + offset : nullptr;
+  unsigned char* ws = static_cast<unsigned char*>(ch.ws);
+  unsigned char* split_ws = with_split ? ws + offset : nullptr;
   size_t flags_at = 0;
   int flag_words = 0;
-  if (with_split) gemm_auto_split_flags(p.m, p.n, p.k, batch, &flags_at, &flag_words);
-  note_kernel("csr_to_dense_kernel<%s>", type_name<IT>());
-  hipLaunchKernelGGL((csr_to_dense_kernel<IT>), dim3(ceil_div(p.m, kDenseRows)), dim3(kDenseThreads), 0, stream, p.m, p.k,
-                     p.row_offsets, static_cast<const IT*>(p.cols), static_cast<const uint16_t*>(p.values),
-                     static_cast<uint16_t*>(ch.ws), with_split ? reinterpret_cast<int*>(split_ws + flags_at) : nullptr, flag_words);
-  if (int rc = check_hip(hipGetLastError(), "spmm dense-form launch")) return rc;
+  if (with_split) gemm_auto_split_flags(p.m, p.n, kp, batch, &flags_at, &flag_words);
+  if (int rc = launch_dense_form<IT>(p.m, kp, p.row_offsets, p.cols, p.values, ws, with_split ? reinterpret_cast<int*>(split_ws + flags_at) : nullptr,
+                                     flag_words, stream))
+    return rc;
+  GemmParams g{p.m, p.n, kp, ws, p.dense, p.out, 0, (long long)p.k * p.n, (long long)p.m * p.n, 0, 0};
+  g.row_bias = p.bias;
+  g.relu = p.relu;
+  g.aux = p.accumulate ? p.out : p.aux;
+  g.aux_mode = p.accumulate ? kGemmAdd : p.aux_mode;
+  g.kb = p.k;
+  if (dense_path_pads(p)) {
+    unsigned char* padded = ws + dense_path_pad_offset(p);
+    if (int rc = launch_pad_rows(p.k, p.n, p.dense, kp, np, padded, batch, (long long)p.k * p.n, stream)) return rc;
+    g.B = padded;
+    g.ldb = np;
+    g.kb = kp;
+    g.stride_b = (long long)kp * np;
+  }
   const int dtype = std::is_same<T, __half>::value ? IEX_F16 : IEX_BF16;
-  return gemm_dispatch(dtype, 0, p.m, p.n, p.k, ch.ws, p.dense, p.out, batch, 0, (long long)p.k * p.n, (long long)p.m * p.n, stream,
-                       p.bias, p.relu, p.accumulate, split_ws, with_split ? split : 0, with_split);
+  return gemm_dispatch(dtype, 0, g, batch, stream, split_ws, with_split ? split : 0, with_split);
 }
 
 template <typename T, typename IT>
@@ -604,7 +642,7 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
   // dense enough go to the dense-form path first (time model above).
   if (ch.variant == 0 && smallk_wanted<T>(p, batch)) {
     if constexpr (sizeof(T) == 2) {
-      const bool room = ch.ws && aligned(ch.ws, 16) && ch.ws_bytes >= dense_path_bytes(p);
+      const bool room = ch.ws && aligned(ch.ws, 16) && ch.ws_bytes >= dense_path_bytes(p, batch);
       if (room && dense_path_fits(2, p, p.per_batch_values) && dense_path_wins(p, batch, 0, true, dense_path_has_split_room(p, batch, ch)))
         return launch_dense_path<T, IT>(p, batch, ch, stream);
     }
@@ -619,10 +657,10 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
   const MfmaChoice mc = mfma_variant<T>(p, batch, ch);
   if constexpr (sizeof(T) == 2) {
     const bool fits = dense_path_fits(2, p, p.per_batch_values);
-    const bool room = ch.ws && aligned(ch.ws, 16) && ch.ws_bytes >= dense_path_bytes(p);
+    const bool room = ch.ws && aligned(ch.ws, 16) && ch.ws_bytes >= dense_path_bytes(p, batch);
     if (ch.variant == 7) {
-      IEX_REQUIRE(fits, IEX_ERR_UNSUPPORTED, "spmm: the dense-form path needs 16-bit values shared by the batch, k and n multiples of 8 and 16-byte aligned operands");
-      IEX_REQUIRE(room, IEX_ERR_BAD_ARGUMENT, "spmm: the dense-form path needs a 16-byte aligned workspace of %zu bytes (iex_spmm_ws)", dense_path_bytes(p));
+      IEX_REQUIRE(fits, IEX_ERR_UNSUPPORTED, "spmm: the dense-form path needs 16-bit values shared by the batch and, without IEX_SPMM_PAD_OPERANDS, k and n multiples of 8 and 16-byte aligned operands");
+      IEX_REQUIRE(room, IEX_ERR_BAD_ARGUMENT, "spmm: the dense-form path needs a 16-byte aligned workspace of %zu bytes (iex_spmm_ws)", dense_path_bytes(p, batch));
       return launch_dense_path<T, IT>(p, batch, ch, stream);
     }
     if (ch.variant == 0 && fits && room && dense_path_wins(p, batch, mc.kind, false, dense_path_has_split_room(p, batch, ch))) return launch_dense_path<T, IT>(p, batch, ch, stream);
@@ -724,6 +762,7 @@ int spmm_dispatch(int dtype, int itype, int flags, int m, int k, int n, int nonz
   SpmmParams p{m, k, n, nonzeros, row_indices, values, row_offsets, column_indices, dense, bias, out,
                (flags & IEX_SPMM_PER_BATCH_VALUES) != 0, (flags & IEX_SPMM_ACCUMULATE) != 0,
                (flags & IEX_SPMM_RELU) != 0};
+  p.pad = (flags & IEX_SPMM_PAD_OPERANDS) != 0;
   // beyond the 256 MB last-level cache an output can only stream; the hint is worth 15-25 % of the write rate
   p.stream_out = (double)m * n * batch * (dtype == IEX_F32 ? 4 : 2) >= 128e6;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -764,6 +803,7 @@ static size_t workspace_plan(int dtype, int itype, int flags, int m, int k, int 
   if (variant != 0 && variant != 7 && variant != 10) return 0;
   SpmmParams p{m, k, n, nonzeros, nullptr, nullptr, nullptr, nullptr, some_aligned, nullptr, some_aligned,
                (flags & IEX_SPMM_PER_BATCH_VALUES) != 0, (flags & IEX_SPMM_ACCUMULATE) != 0, (flags & IEX_SPMM_RELU) != 0};
+  p.pad = (flags & IEX_SPMM_PAD_OPERANDS) != 0;
   if (variant != 7 && nonzeros >= 8 && spmm_blocks_fits(dtype, itype, p) && (variant == 10 || spmm_blocks_wins(p, batch))) {
     *kind = 10;
     return spmm_blocks_bytes(p);
@@ -779,7 +819,7 @@ static size_t workspace_plan(int dtype, int itype, int flags, int m, int k, int 
   }
   *kind = 7;
   const size_t split = dense_path_split_bytes(p, batch);
-  return split ? dense_path_split_offset(p) + split : dense_path_bytes(p);
+  return split ? dense_path_split_offset(p, batch) + split : dense_path_bytes(p, batch);
 }
 
 size_t spmm_workspace_bytes(int dtype, int itype, int flags, int m, int k, int n, int nonzeros, int batch) {
@@ -791,6 +831,63 @@ int spmm_workspace_kind(int dtype, int itype, int flags, int m, int k, int n, in
   int kind;
   workspace_plan(dtype, itype, flags, m, k, n, nonzeros, batch, &kind);
   return kind;
+}
+
+// ---- A^T * G (the gradient of a sparse layer's input) from the CSR form of A, where the dense-form path would run it:
+// the dense form of A is its transpose's, read as a (K,M) operand, so neither the values nor the pattern of the
+// transposed matrix are needed.  ws = dense form (m x round8(k)), copy of G where its rows are no whole chunks, GEMM's room.
+struct TransposedPlan {
+  bool wanted;
+  bool pads;
+  size_t pad_at, split_at, split_bytes, bytes;
+};
+static TransposedPlan transposed_plan(int dtype, int m, int k, int n, int nonzeros, const void* dense) {
+  TransposedPlan t{};
+  if (!(dtype == IEX_F16 || dtype == IEX_BF16) || m <= 0 || k <= 0 || n <= 0 || nonzeros <= 0) return t;
+  void* const some_aligned = reinterpret_cast<void*>(size_t(256));
+  SpmmParams p{k, m, n, nonzeros, nullptr, nullptr, nullptr, nullptr, dense, nullptr, some_aligned, 0, 0, 0};   // (the product as the SpMM it replaces)
+  p.pad = 1;
+  if (!dense_path_fits(2, p, false) || (long long)m * round8(k) >= (1ll << 31) || (long long)m * round8(n) >= (1ll << 31)) return t;
+  const bool few = smallk_wanted<__half>(p, 1);
+  t.wanted = dense_path_wins(p, 1, few ? 0 : mfma_variant<__half>(p, 1, Choice{}).kind, few);
+  t.pads = dense_path_pads(p);
+  t.pad_at = round256((size_t)m * round8(k) * 2);
+  t.split_at = t.pads ? round256(t.pad_at + (size_t)m * round8(n) * 2) : t.pad_at;
+  t.split_bytes = gemm_auto_split_bytes(k, n, m, 1);
+  t.bytes = t.split_at + t.split_bytes;
+  return t;
+}
+
+size_t spmm_transposed_workspace_bytes(int dtype, int m, int k, int n, int nonzeros) {
+  const TransposedPlan t = transposed_plan(dtype, m, k, n, nonzeros, reinterpret_cast<void*>(size_t(256)));
+  return t.wanted ? t.bytes : 0;
+}
+
+int spmm_transposed(int dtype, int itype, int m, int k, int n, int nonzeros, const void* values, const int* row_offsets, const void* cols, const void* dense,
+                    void* out, hipStream_t stream, void* workspace, size_t workspace_bytes) {
+  trail_reset();
+  const TransposedPlan t = transposed_plan(dtype, m, k, n, nonzeros, dense);
+  IEX_REQUIRE(t.bytes > 0, IEX_ERR_UNSUPPORTED, "spmm (transposed): needs fp16 / bf16 operands, at least one nonzero and fewer than 2^31 elements");
+  IEX_REQUIRE(itype == IEX_I32 || itype == IEX_I16, IEX_ERR_UNSUPPORTED, "spmm (transposed): column indices must be int32 or int16");
+  IEX_REQUIRE(values && row_offsets && cols && dense && out, IEX_ERR_BAD_ARGUMENT, "spmm (transposed): null pointer argument");
+  IEX_REQUIRE(workspace && aligned(workspace, 256) && workspace_bytes >= t.bytes, IEX_ERR_BAD_ARGUMENT,
+              "spmm (transposed): needs a 256-byte aligned workspace of %zu bytes", t.bytes);
+  unsigned char* ws = static_cast<unsigned char*>(workspace);
+  size_t flags_at = 0;
+  int flag_words = 0;
+  if (t.split_bytes) gemm_auto_split_flags(k, n, m, 1, &flags_at, &flag_words);
+  int* flags = t.split_bytes ? reinterpret_cast<int*>(ws + t.split_at + flags_at) : nullptr;
+  if (int rc = itype == IEX_I16 ? launch_dense_form<short>(m, round8(k), row_offsets, cols, values, ws, flags, flag_words, stream)
+                                : launch_dense_form<int>(m, round8(k), row_offsets, cols, values, ws, flags, flag_words, stream))
+    return rc;
+  GemmParams g{k, n, m, ws, dense, out, 0, 0, 0, 0, 0};
+  g.lda = round8(k);
+  if (t.pads) {
+    if (int rc = launch_pad_rows(m, n, dense, m, round8(n), ws + t.pad_at, 1, 0, stream)) return rc;
+    g.B = ws + t.pad_at;
+    g.ldb = round8(n);
+  }
+  return gemm_dispatch(dtype, 2, g, 1, stream, t.split_bytes ? ws + t.split_at : nullptr, t.split_bytes, t.split_bytes > 0);
 }
 
 // ---- the library's own scratch memory, for callers that cannot allocate ---------------------------------
@@ -878,6 +975,16 @@ size_t iex_spmm_workspace_bytes(int dtype, int itype, int flags, int m, int k, i
 
 int iex_spmm_workspace_kind(int dtype, int itype, int flags, int m, int k, int n, int nonzeros, int batch) {
   return iex::spmm_workspace_kind(dtype, itype, flags, m, k, n, nonzeros, batch);
+}
+
+size_t iex_spmm_transposed_workspace_bytes(int dtype, int m, int k, int n, int nonzeros) {
+  return iex::spmm_transposed_workspace_bytes(dtype, m, k, n, nonzeros);
+}
+
+int iex_spmm_transposed(int dtype, int itype, int m, int k, int n, int nonzeros, const void* values, const int* row_offsets, const void* column_indices,
+                        const void* dense, void* out, void* stream, void* workspace, size_t workspace_bytes) {
+  return iex::spmm_transposed(dtype, itype, m, k, n, nonzeros, values, row_offsets, column_indices, dense, out, static_cast<hipStream_t>(stream), workspace,
+                              workspace_bytes);
 }
 
 int iex_CudaSpmm2(int m, int k, int n, int nonzeros, const int* row_indices, const float* values,

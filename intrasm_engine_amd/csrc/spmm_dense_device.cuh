@@ -10,8 +10,9 @@
 // "load 256 nonzeros, scatter them" steps of its wavefronts, each a round trip to memory: with one wavefront per row
 // the longest row set the kernel's time (4096 nonzeros: 16 steps, 24 us where the bytes written take 8).
 // Rows longer than kDenseSeg columns are done in segments, every wavefront with a cursor into its quarter of the
-// row's ascending column indices.  Needs k % 8 == 0 and a 16-byte aligned workspace; column indices inside a row must
-// ascend strictly (canonical CSR).
+// row's ascending column indices.  k, here the row stride of the dense form, is a multiple of 8 and no less than the number
+// of columns (the rest is zero); the workspace is 16-byte aligned; column indices inside a row must ascend strictly
+// (canonical CSR).
 #pragma once
 #include "iex_common.h"
 
@@ -93,6 +94,41 @@ __global__ __launch_bounds__(kDenseThreads) void csr_to_dense_kernel(int m, int 
           *reinterpret_cast<uint4*>(out + (size_t)row * k + c0 + i) = *reinterpret_cast<const uint4*>(srow[r] + i);
     }
   }
+}
+
+// dst (dst_rows x ld, ld a multiple of 8, 16-byte aligned) = src (rows x cols, at element alignment) with zeros around it:
+// a dense operand of any shape as the GEMM's direct loads want it.  One 16-byte chunk of dst per thread.
+static __global__ __launch_bounds__(256) void pad_rows_kernel(int rows, int cols, const uint16_t* __restrict__ src, int dst_rows, int ld, uint16_t* __restrict__ dst,
+                                                              long long src_stride) {
+  struct alignas(2) Any { uint16_t v[8]; };
+  struct alignas(16) Whole { uint16_t v[8]; };
+  const int chunks = ld / 8;
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long long)dst_rows * chunks) return;
+  const int r = (int)(i / chunks), c = (int)(i % chunks) * 8;
+  src += (size_t)blockIdx.y * src_stride + (size_t)r * cols;
+  dst += (size_t)blockIdx.y * dst_rows * ld + (size_t)r * ld;
+  Whole w{};
+  if (r < rows && c + 8 <= cols) {
+    const Any a = *reinterpret_cast<const Any*>(src + c);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w.v[e] = a.v[e];
+  } else if (r < rows) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w.v[e] = c + e < cols ? src[c + e] : (uint16_t)0;
+  }
+  *reinterpret_cast<Whole*>(dst + c) = w;
+}
+
+inline int round8(int x) { return (x + 7) & ~7; }
+inline size_t round256(size_t x) { return (x + 255) & ~size_t(255); }
+
+// rows x cols (`batch` of them, src_stride elements apart) into dst_rows x ld, as above.
+inline int launch_pad_rows(int rows, int cols, const void* src, int dst_rows, int ld, void* dst, int batch, long long src_stride, hipStream_t stream) {
+  note_kernel("pad_rows_kernel");
+  hipLaunchKernelGGL(pad_rows_kernel, dim3(ceil_div((long long)dst_rows * (ld / 8), 256), batch), dim3(256), 0, stream, rows, cols,
+                     static_cast<const uint16_t*>(src), dst_rows, ld, static_cast<uint16_t*>(dst), src_stride);
+  return check_hip(hipGetLastError(), "padding launch");
 }
 
 }  // namespace iex

@@ -33,6 +33,9 @@ struct SpmmParams {
   const float* bias;
   void* out;
   int per_batch_values, accumulate, relu;
+  int pad = 0;                // the dense-form path may copy operands into the workspace (IEX_SPMM_PAD_OPERANDS)
+  int aux_mode = 0;           // epilogue of the dense-form path: see GemmParams (gemm_device.cuh)
+  const void* aux = nullptr;
   int stream_out = 0;  // the output is far larger than the caches: store it with the streaming hint
 };
 

@@ -381,7 +381,7 @@ def _spmm(b, row_indices, values, row_offsets, column_indices, m, *, per_batch_v
                 force_variant = 10 if kind(10) == 10 else 0      # (0: the kernel does not serve this call: another n, int16 indices)
             elif kind(0) == 10:
                 force_variant = 1      # (only where the density rule would have picked that kernel: every other choice stays the library's)
-    flags = (_lib.SPMM_PER_BATCH_VALUES if per_batch_values else 0) | (_lib.SPMM_ANY_COLUMN_ORDER if any_order else 0) | \
+    flags = _lib.SPMM_PAD_OPERANDS | (_lib.SPMM_PER_BATCH_VALUES if per_batch_values else 0) | (_lib.SPMM_ANY_COLUMN_ORDER if any_order else 0) | \
             (_lib.SPMM_BESIDE_GATHER_KERNEL if beside_gather else 0) | \
             (_lib.SPMM_ACCUMULATE if accumulate else 0) | (_lib.SPMM_RELU if relu else 0) | \
             ((int(force_wpr) & 0xff) << 8) | ((int(force_variant) & 0xf) << 16) | ((int(force_rpw) & 0xf) << 20) | \
@@ -526,7 +526,7 @@ def _sddmm(a, b, row_indices, row_offsets, column_indices, *, sum_over_batch, dt
                 # only where the density rule would have picked that kernel: a long k (the gradient of a pruned weight:
                 # 11008 x 4096 at 90 %, k = 2048, fp16) keeps the dense product, 1691 -> 230 us
                 force_variant = 1
-    flags = (_lib.SDDMM_SUM_OVER_BATCH if sum_over_batch else 0) | (_lib.SDDMM_ANY_COLUMN_ORDER if any_order else 0) | \
+    flags = _lib.SDDMM_PAD_OPERANDS | (_lib.SDDMM_SUM_OVER_BATCH if sum_over_batch else 0) | (_lib.SDDMM_ANY_COLUMN_ORDER if any_order else 0) | \
             (_lib.SDDMM_ACCUMULATE if accumulate else 0) | ((int(force_wpr) & 0xff) << 8) | \
             ((int(force_variant) & 0xf) << 16)
     lib = _lib.load()
