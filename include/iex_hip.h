@@ -65,6 +65,13 @@ int iex_device_ok(void);
 int iex_csr_check(int itype, int m, int k, int nonzeros, const int* row_offsets, const void* column_indices,
                   int* status, void* stream);
 
+/* iex_spmm_sched with an element-wise epilogue against a second operand of the output's shape (16-bit types, shared values,
+ * plain store): mode 1: out = A*b + aux; mode 2: out = (A*b) * aux / (1 + exp(-aux)), the gate of a SiLU.  One kernel less
+ * and, where the product ends in the dense GEMM, no pass over memory: it happens before the sums are rounded. */
+int iex_spmm_aux(int dtype, int itype, int flags, int m, int k, int n, int nonzeros, const int* row_indices, const void* values,
+                 const int* row_offsets, const void* column_indices, const void* dense, const void* aux, int aux_mode, void* out,
+                 void* stream, int batch, void* workspace, size_t workspace_bytes, const int* row_histogram);
+
 /* Row lengths of a pattern on a coarse scale, for iex_spmm_sched: adds to histogram[j] (device memory, 16 ints that the
  * caller has set to 0; the launch is asynchronous on `stream`) the number of rows with more than 64 << j nonzeros,
  * j = 0 .. 15.  A function of row_offsets alone; a caller reads it back once per pattern, as set-up.
@@ -358,6 +365,15 @@ int iex_CudaSddmm2(int m, int k, int n, int nonzeros, const int* row_indices,
                    const int* row_offsets, const int* column_indices,
                    const float* lhs_matrix, const float* rhs_matrix, float* output_values,
                    void* stream, int batch_size);
+
+/* Dense attention, softmax(scale * q^T k) over the keys of a sequence, times v: q, k, v and out are feature-major
+ * (heads * head_dim, seqs * length) matrices of fp16 / bf16, the columns seqs sequences of length tokens; no mask.  fp32
+ * scores and sums, probabilities rounded to the type.  head_dim 64 or 128, length a multiple of 8, scale > 0, operands
+ * 16-byte aligned (iex_attention_fits says so for the first three).  The middle of the decoder layer of the reference's
+ * models, which runs it as two batched products around a softmax (nn.functional). */
+int iex_attention_fits(int dtype, int head_dim, int length);
+int iex_attention(int dtype, int heads, int head_dim, int seqs, int length, const void* q, const void* k, const void* v, float scale,
+                  void* out, void* stream);
 
 /* In-place row-wise softmax over the stored entries of a CSR matrix:
  * values[z, j] = exp(scale*values[z, j] - max_row) / sum_row.  values is (batch, nnz).

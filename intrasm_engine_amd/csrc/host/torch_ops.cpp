@@ -140,11 +140,14 @@ const char* spmm_name(Spmm kind) {
   }
 }
 
-// flat: b is (k, n) and the result (m, n), without the batch dimension
-template <Spmm kind, bool flat = false>
-Tensor spmm(const Tensor& b, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m) {
+// flat: b is (k, n) and the result (m, n), without the batch dimension.  aux: (16-bit, shared values) an operand of the
+// result's shape, mode 1 added, mode 2 its SiLU multiplied; undefined is returned where the call is not served here
+template <Spmm kind, bool flat>
+Tensor spmm_call(const Tensor& b, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m,
+                 const Tensor& aux = Tensor(), int aux_mode = 0) {
   constexpr bool per_entry = kind == Spmm::kPerEntry || kind == Spmm::kAtomic, accumulate = kind == Spmm::kAtomic;
   auto python = [&] {
+    if (aux.defined()) return Tensor();
     const Tensor out = ask_python<Tensor>(spmm_name(kind), flat ? b.unsqueeze(0) : b, row_indices, values, row_offsets, column_indices, m);
     return flat ? at::_unsafe_view(out, {out.size(1), out.size(2)}) : out;
   };
@@ -182,11 +185,25 @@ Tensor spmm(const Tensor& b, const Tensor& row_indices, const Tensor& values, co
   } else {
     ws = workspace(ws_bytes, b);
   }
+  if (aux.defined()) {
+    if (!plain(aux, 3 - flat) || aux.sizes() != out_shape || aux.scalar_type() != b.scalar_type() || aux.device() != b.device()) return Tensor();
+    check(iex_spmm_aux(dtype, itype, flags, m, k, n, nonzeros, row_indices.const_data_ptr<int>(), values.const_data_ptr(),
+                       row_offsets.const_data_ptr<int>(), column_indices.const_data_ptr(), b.const_data_ptr(), aux.const_data_ptr(), aux_mode,
+                       out.data_ptr(), stream_of(b), batch, ws.defined() ? ws.data_ptr() : nullptr, ws_bytes,
+                       known->has_histogram ? known->histogram.data() : nullptr),
+          "spmm");
+    return out;
+  }
   check(iex_spmm_sched(dtype, itype, flags, m, k, n, nonzeros, row_indices.const_data_ptr<int>(), values.const_data_ptr(),
                        row_offsets.const_data_ptr<int>(), column_indices.const_data_ptr(), b.const_data_ptr(), nullptr, out.data_ptr(), stream_of(b),
                        batch, ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, known->has_histogram ? known->histogram.data() : nullptr),
         "spmm");
   return out;
+}
+
+template <Spmm kind>
+Tensor spmm(const Tensor& b, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m) {
+  return spmm_call<kind, false>(b, row_indices, values, row_offsets, column_indices, m);
 }
 
 // ---- SDDMM ---------------------------------------------------------------------------------------------------------
@@ -285,13 +302,40 @@ Tensor gemm_transposed_a(const Tensor& a, const Tensor& b) {
   return out;
 }
 
+// ---- the steps of a decoder layer around its products --------------------------------------------------------------
+// W_csr @ x combined with a second operand (see spmm above); None where that is not served natively
+std::optional<Tensor> spmm_with(const Tensor& x, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices,
+                                int64_t m, const Tensor& aux, int mode) {
+  if (at::GradMode::is_enabled() && (x.requires_grad() || values.requires_grad() || aux.requires_grad())) return {};
+  const Tensor out = spmm_call<Spmm::kSharedHalf, true>(x, row_indices, values, row_offsets, column_indices, m, aux, mode);
+  return out.defined() ? std::optional<Tensor>(out) : std::nullopt;
+}
+
+// softmax(scale * q^T k) v per head and sequence on feature-major operands; None where the kernel does not serve them
+std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, int64_t seqs, double scale) {
+  const int dtype = dtype_code(q.scalar_type());
+  if (forced || !plain(q, 2) || !plain(k, 2) || !plain(v, 2) || k.sizes() != q.sizes() || v.sizes() != q.sizes() || k.scalar_type() != q.scalar_type() ||
+      v.scalar_type() != q.scalar_type() || k.device() != q.device() || v.device() != q.device() || heads <= 0 || seqs <= 0 || q.size(0) % heads != 0 ||
+      q.size(1) % seqs != 0 || !(scale > 0) || !iex_attention_fits(dtype, q.size(0) / heads, q.size(1) / seqs))
+    return {};
+  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) return {};
+  for (const Tensor* t : {&q, &k, &v})
+    if (reinterpret_cast<uintptr_t>(t->const_data_ptr()) % 16) return {};
+  const c10::DeviceGuard guard(q.device());
+  Tensor out = at::empty_like(q);
+  check(iex_attention(dtype, heads, q.size(0) / heads, seqs, q.size(1) / seqs, q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), (float)scale,
+                      out.data_ptr(), stream_of(q)),
+        "attention");
+  return out;
+}
+
 // ---- autograd: the plain calls of MySpMM and MyLinear (no recording, no forced kernels) -----------------------------
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
 Tensor spmm_shared(const Tensor& b, const Tensor& row_indices, const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m) {
-  return values.scalar_type() == at::kFloat ? spmm<Spmm::kSharedF32, true>(b, row_indices, values, row_offsets, column_indices, m)
-                                            : spmm<Spmm::kSharedHalf, true>(b, row_indices, values, row_offsets, column_indices, m);
+  return values.scalar_type() == at::kFloat ? spmm_call<Spmm::kSharedF32, true>(b, row_indices, values, row_offsets, column_indices, m)
+                                            : spmm_call<Spmm::kSharedHalf, true>(b, row_indices, values, row_offsets, column_indices, m);
 }
 
 // values[perm]: the values of the transposed matrix
@@ -405,6 +449,8 @@ PYBIND11_MODULE(_iex_host, module) {
   module.def("bind", [](py::object functions) { python_ops = new py::object(std::move(functions)); });
   module.def("set_forced", [](bool on) { forced = on; });
   module.def("set_note", &set_note);
+  module.def("spmm_with", &spmm_with);
+  module.def("attention", &attention);
   module.def("trainable_spmm", &trainable_spmm);
   module.def("trainable_linear", &trainable_linear);
 }

@@ -384,6 +384,26 @@ inline int launch_mfma_f32(const SpmmParams& p, int batch, int arrangement, int 
   return fail(IEX_ERR_BAD_ARGUMENT, "spmm: arrangement of the fp32 matrix-core variant must be 1, 2, 4, 5 or 6 (got %d)", arrangement);
 }
 
+// out = out + aux, or out * silu(aux), over n 16-bit elements: the epilogue of the products that have none of their own.
+template <bool BF16>
+__global__ __launch_bounds__(256) void combine_kernel(size_t n, const uint16_t* aux, int mode, uint16_t* out) {
+  struct alignas(2) Any { uint16_t v[8]; };
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  auto one = [&](uint16_t o, uint16_t a) {
+    const float x = f16_to_32(o, BF16), y = f16_to_32(a, BF16);
+    return f32_to_16(mode == kGemmAdd ? x + y : x * (y / (1.f + __expf(-y))), BF16);
+  };
+  if (i + 8 <= n) {
+    Any o = *reinterpret_cast<const Any*>(out + i);
+    const Any a = *reinterpret_cast<const Any*>(aux + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o.v[e] = one(o.v[e], a.v[e]);
+    *reinterpret_cast<Any*>(out + i) = o;
+  } else {
+    for (size_t j = i; j < n; ++j) out[j] = one(out[j], aux[j]);
+  }
+}
+
 struct Choice {
   int wpr = 0;      // wavefronts per row of the row kernel
   bool wpr_forced = false;
@@ -395,6 +415,7 @@ struct Choice {
   size_t ws_bytes = 0;
   bool any_order = false;   // columns of a row in any order, possibly repeated: families 1 and 8 only
   const int* hist = nullptr;   // host: rows with more than 64 << j nonzeros, j = 0 .. 15 (iex_spmm_sched), may be null
+  bool* aux_done = nullptr;    // set by a path whose own epilogue takes the auxiliary operand
   bool beside_gather = false;  // the launch shares the chip with a gather-bound one (IEX_SPMM_BESIDE_GATHER_KERNEL)
 };
 
@@ -553,7 +574,8 @@ inline size_t dense_path_bytes(const SpmmParams& p, int batch) {
 // The dense form has to win by 15 % to be taken.  `few_columns`: the alternative is the few-columns kernel.
 // split_room: the workspace has room for the GEMM to take k in parts where it would (few tiles, long k: the K loop of a
 // tile then runs on several CUs; 4096^2 at 70-90 %, n = 128 / 256: 40 / 41 -> 27 / 32 us).
-//   rows of n elements that are no whole vectors are gathered in full-width tiles.
+//   Wide rows are gathered in tiles of 512 columns, the last one as slow as the others (3449 x 8696 at 94 %, n = 552: 185
+//     against 72 us).
 inline bool dense_path_wins(const SpmmParams& p, int batch, int matrix_core_kind, bool few_columns, bool split_room = true) {
   const double cells = (double)p.m * p.k, flops = 2.0 * cells * p.n * batch, density = p.nnz / std::max(cells, 1.0);
   const double out_bytes = (double)p.m * p.n * batch * 2;
@@ -571,7 +593,7 @@ inline bool dense_path_wins(const SpmmParams& p, int batch, int matrix_core_kind
     const double chain = rounds * (p.k / 128.0) * (wide ? 3.5e-6 + 7e-6 * density : 4.5e-6 + 21e-6 * density);
     other = 8e-6 + std::max({flops / 720e12, chain, out_bytes / 1.2e12});
   } else {
-    const double columns = p.n % 8 == 0 || p.n < 256 ? p.n : ceil_div(p.n, 512) * 512;
+    const double columns = p.n <= 256 ? p.n : ceil_div(p.n, 512) * 512;   // (whole tiles: a last tile of few columns costs like a full one)
     other = 8e-6 + (double)p.nnz * columns * batch * 2 / 26e12 + out_bytes / 4e12;
   }
   return 1.15 * dense_form < other;
@@ -615,6 +637,7 @@ int launch_dense_path(const SpmmParams& p, int batch, const Choice& ch, hipStrea
   g.relu = p.relu;
   g.aux = p.accumulate ? p.out : p.aux;
   g.aux_mode = p.accumulate ? kGemmAdd : p.aux_mode;
+  if (p.aux && ch.aux_done) *ch.aux_done = true;
   g.kb = p.k;
   if (dense_path_pads(p)) {
     unsigned char* padded = ws + dense_path_pad_offset(p);
@@ -732,7 +755,8 @@ int spmm_matrix_core_windows(const SpmmParams& p) {
 int spmm_dispatch(int dtype, int itype, int flags, int m, int k, int n, int nonzeros,
                   const int* row_indices, const void* values, const int* row_offsets,
                   const void* column_indices, const void* dense, const float* bias, void* out,
-                  void* stream, int batch, void* workspace, size_t workspace_bytes, const int* row_histogram = nullptr) {
+                  void* stream, int batch, void* workspace, size_t workspace_bytes, const int* row_histogram = nullptr,
+                  const void* aux = nullptr, int aux_mode = 0, bool* aux_done = nullptr) {
   IEX_REQUIRE(m >= 0 && k >= 0 && n >= 0 && nonzeros >= 0 && batch >= 0, IEX_ERR_BAD_ARGUMENT,
               "spmm: negative dimension (m=%d k=%d n=%d nnz=%d batch=%d)", m, k, n, nonzeros, batch);
   trail_reset();
@@ -763,6 +787,9 @@ int spmm_dispatch(int dtype, int itype, int flags, int m, int k, int n, int nonz
                (flags & IEX_SPMM_PER_BATCH_VALUES) != 0, (flags & IEX_SPMM_ACCUMULATE) != 0,
                (flags & IEX_SPMM_RELU) != 0};
   p.pad = (flags & IEX_SPMM_PAD_OPERANDS) != 0;
+  p.aux = aux;
+  p.aux_mode = aux_mode;
+  ch.aux_done = aux_done;
   // beyond the 256 MB last-level cache an output can only stream; the hint is worth 15-25 % of the write rate
   p.stream_out = (double)m * n * batch * (dtype == IEX_F32 ? 4 : 2) >= 128e6;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -959,6 +986,27 @@ int iex_spmm_ws(int dtype, int itype, int flags, int m, int k, int n, int nonzer
                 void* stream, int batch, void* workspace, size_t workspace_bytes) {
   return iex::spmm_dispatch(dtype, itype, flags, m, k, n, nonzeros, row_indices, values, row_offsets,
                             column_indices, dense, bias, out, stream, batch, workspace, workspace_bytes);
+}
+
+int iex_spmm_aux(int dtype, int itype, int flags, int m, int k, int n, int nonzeros, const int* row_indices, const void* values,
+                 const int* row_offsets, const void* column_indices, const void* dense, const void* aux, int aux_mode, void* out,
+                 void* stream, int batch, void* workspace, size_t workspace_bytes, const int* row_histogram) {
+  using namespace iex;
+  IEX_REQUIRE(dtype == IEX_F16 || dtype == IEX_BF16, IEX_ERR_UNSUPPORTED, "spmm: an auxiliary operand goes with fp16 / bf16");
+  IEX_REQUIRE(!(flags & (IEX_SPMM_PER_BATCH_VALUES | IEX_SPMM_ACCUMULATE | IEX_SPMM_RELU)), IEX_ERR_UNSUPPORTED,
+              "spmm: an auxiliary operand goes with shared values, a plain store and no ReLU");
+  IEX_REQUIRE(aux && (aux_mode == kGemmAdd || aux_mode == kGemmTimesSilu), IEX_ERR_BAD_ARGUMENT, "spmm: null auxiliary operand or unknown mode %d", aux_mode);
+  bool done = false;
+  if (int rc = spmm_dispatch(dtype, itype, flags, m, k, n, nonzeros, row_indices, values, row_offsets, column_indices, dense, nullptr, out, stream, batch,
+                             workspace, workspace_bytes, row_histogram, aux, aux_mode, &done))
+    return rc;
+  const size_t total = (size_t)m * n * batch;
+  if (done || total == 0) return 0;
+  note_kernel("combine_kernel");
+  auto kernel = dtype == IEX_BF16 ? combine_kernel<true> : combine_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((total + 2047) / 2048)), dim3(256), 0, static_cast<hipStream_t>(stream), total,
+                     static_cast<const uint16_t*>(aux), aux_mode, static_cast<uint16_t*>(out));
+  return check_hip(hipGetLastError(), "spmm combine launch");
 }
 
 int iex_spmm_sched(int dtype, int itype, int flags, int m, int k, int n, int nonzeros,

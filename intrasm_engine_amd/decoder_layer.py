@@ -2,9 +2,11 @@
 this package -- the workload of benchmark configuration 5.
 
 Every projection is ``W_csr @ X`` (SpMM) with activations stored feature-major
-``(features, tokens)``; attention scores and context are batched MFMA GEMMs.  Included
-element-wise steps, done by PyTorch between the launches: softmax(QK^T / sqrt(d)) over
-keys, SiLU(gate) * up, and the two residual additions.  Not included (the configuration
+``(features, tokens)``; the attention reads and writes them as they are, scores and
+probabilities in registers (heads of 64 or 128; else heads are split off and scores and
+context are batched MFMA GEMMs around PyTorch's softmax).  Included element-wise steps,
+done by the epilogues of the products before them: SiLU(gate) * up and the two residual
+additions.  Not included (the configuration
 names none of them): RoPE, normalisation layers, causal masking, KV cache.
 
 Three ways to run the same arithmetic, mirroring how the reference's harness compares
@@ -14,8 +16,8 @@ Three ways to run the same arithmetic, mirroring how the reference's harness com
   multistream  the batch is split into two halves that are captured on two streams of one
                graph (two branches joined at the end), so the sparse projections of one half
                can overlap the dense attention of the other;
-  fused        the same two halves on one stream, with each dense attention GEMM of one half
-               launched together with a sparse projection of the other half through the
+  fused        the same two halves on one stream; where attention runs as batched GEMMs, each of
+               them is launched together with a sparse projection of the other half through the
                horizontally fused kernel.
 """
 from __future__ import annotations
@@ -25,6 +27,7 @@ import math
 import torch
 
 from . import interleaving as IL
+from . import _iex_host, _lib
 from .pytorch import ops as _pyops
 from .pytorch.cpp_extensions.cuda_graph_constructor import TorchCUDAGraphConstructor
 
@@ -38,6 +41,9 @@ class SparseDecoderLayer:
         self.hidden, self.heads, self.mlp = hidden, heads, mlp
         self.head_dim = hidden // heads
         self.device = device
+        # whether the attention kernel serves these heads; the layer then has no dense product of its own, and the steps
+        # after its sparse products go into their epilogues
+        self._one_attention = bool(_lib.load().iex_attention_fits(_lib.F16, self.head_dim, 8))
         self.w = {}
         for name, csr in weights.items():
             idt = index_dtype if csr.k <= 32768 else torch.int32
@@ -54,6 +60,15 @@ class SparseDecoderLayer:
         """(k, tokens) -> (m, tokens)."""
         ri, v, ro, ci, m = self.w[name]
         return ops.spmm_sputnik_reuse_weight_half(x.unsqueeze(0), ri, v, ro, ci, m)[0]
+
+    def _proj_with(self, name: str, x: torch.Tensor, other: torch.Tensor, mode: int):
+        """``proj`` combined with ``other`` before it is rounded: plus it (mode 1), times its SiLU (mode 2)."""
+        ri, v, ro, ci, m = self.w[name]
+        out = _iex_host.spmm_with(x, ri, v, ro, ci, m, other, mode) if self._one_attention else None
+        if out is None:
+            out = self.proj(name, x)
+            out = other + out if mode == 1 else torch.nn.functional.silu(other) * out
+        return out
 
     def _split_heads(self, t: torch.Tensor, seqs: int, scale: float = 1.0) -> torch.Tensor:
         """(hidden, seqs*L) feature-major -> (seqs*heads, L, head_dim), times ``scale`` in the same pass."""
@@ -82,18 +97,20 @@ class SparseDecoderLayer:
                 self._split_heads(v, seqs))
 
     def attention(self, q, k, v, seqs: int) -> torch.Tensor:
+        out = _iex_host.attention(q, k, v, self.heads, seqs, 1.0 / math.sqrt(self.head_dim)) if self._one_attention else None
+        if out is not None:
+            return out
         Q, K, V = self._split_qkv(q, k, v, seqs)
         P = self._softmax(ops.gemm_mfma(Q, K, True))      # (B, L, L)
         return self._merge_heads(ops.gemm_mfma(P, V, False), seqs)
 
     def mlp_block(self, h: torch.Tensor) -> torch.Tensor:
-        act = torch.nn.functional.silu(self.proj("gate", h)) * self.proj("up", h)
-        return h + self.proj("down", act)
+        return self._proj_with("down", self._proj_with("up", h, self.proj("gate", h), 2), h, 1)
 
     def forward(self, x: torch.Tensor, seqs: int) -> torch.Tensor:
         """x: (hidden, seqs*L) fp16, contiguous -> same shape."""
         q, k, v = self.proj("q", x), self.proj("k", x), self.proj("v", x)
-        h = x + self.proj("o", self.attention(q, k, v, seqs))
+        h = self._proj_with("o", self.attention(q, k, v, seqs), x, 1)
         return self.mlp_block(h)
 
     # ---- fused schedule over two half-batches ----------------------------------------------
@@ -104,7 +121,10 @@ class SparseDecoderLayer:
 
     def forward_fused(self, xa: torch.Tensor, xb: torch.Tensor, seqs_half: int, group=None):
         """Halves a and b of the batch; the dense GEMMs of one half ride along with sparse
-        projections of the other half."""
+        projections of the other half.  With the attention kernel there are none: one half after the other, ``group``
+        then orders nothing (16 x 512 tokens, hidden 4096: 4.4 ms by fused launches before that kernel, 3.0 now)."""
+        if self._one_attention:
+            return self.forward(xa, seqs_half), self.forward(xb, seqs_half)
         qa, ka, va = self.proj("q", xa), self.proj("k", xa), self.proj("v", xa)
         Qa, Ka, Va = self._split_qkv(qa, ka, va, seqs_half)
         qb, Sa = self._fused("q", xb, Qa, Ka, True, group)              # b.q  ||  a.QK^T
