@@ -96,6 +96,52 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(u32x4 a, u32x4 b, f32x16 c) {
   }
 }
 
+// Half the accumulator traffic per flop of the 32 x 32 form: under the power limit random operands run at 2100 instead of
+// 1875 TFLOP/s (a loop of MFMAs and nothing else, every CU; all-zero operands 2440 / 2470).
+template <bool BF16>
+__device__ __forceinline__ f32x4 mfma_16x16x32(u32x4 a, u32x4 b, f32x4 c) {
+  if constexpr (BF16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+}
+
+// The accumulators of a wavefront's WM x WN blocks of 32 x 32 (operands swapped: a quad is 4 adjacent columns of one row),
+// as quads: quad t of 4 * WN of row block i, with the row and the first column it has inside the block row.
+template <int WM, int WN>
+struct Acc32 {   // one 32 x 32 MFMA per block
+  f32x16 v[WM][WN];
+  __device__ __forceinline__ f32x4 quad(int i, int t) const {
+    const f32x16& a = v[i][t / 4];
+    return f32x4{a[t % 4 * 4], a[t % 4 * 4 + 1], a[t % 4 * 4 + 2], a[t % 4 * 4 + 3]};
+  }
+  static __device__ __forceinline__ int row(int, int lane) { return lane & 31; }
+  static __device__ __forceinline__ int col(int t, int lane) { return t * 8 + (lane >> 5) * 4; }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[i][j][r] = 0.f;
+  }
+};
+template <int WM, int WN>
+struct Acc16 {   // 2 x 2 MFMAs of 16 x 16 per block
+  f32x4 v[2 * WM][2 * WN];
+  __device__ __forceinline__ f32x4 quad(int i, int t) const { return v[2 * i + t / (2 * WN)][t % (2 * WN)]; }
+  __device__ __forceinline__ void add(int i, int t, f32x4 x) { v[2 * i + t / (2 * WN)][t % (2 * WN)] += x; }
+  static __device__ __forceinline__ int row(int t, int lane) { return t / (2 * WN) * 16 + (lane & 15); }
+  static __device__ __forceinline__ int col(int t, int lane) { return t % (2 * WN) * 16 + (lane >> 4) * 4; }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < 2 * WM; ++i)
+#pragma unroll
+      for (int j = 0; j < 2 * WN; ++j) v[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+};
+
 __device__ __forceinline__ float f16_to_32(unsigned short h, bool bf16) {
   if (bf16) return __uint_as_float((unsigned)h << 16);
   return (float)__builtin_bit_cast(_Float16, h);
@@ -204,8 +250,8 @@ struct GemmStage {
 template <int WN>
 constexpr int gemm_store_lds_bytes() { return 32 * (WN * 64 + 16); }
 
-template <bool BF16, int WM, int WN>
-__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const f32x16 (&acc)[WM][WN], unsigned short* __restrict__ C,
+template <bool BF16, int WM, int WN, typename Acc>
+__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const Acc& acc, unsigned short* __restrict__ C,
                                                 const unsigned short* aux, int m0, int n0, int wm, int wn, int lane, unsigned char* lds,
                                                 bool stream, const float* partial = nullptr) {
   typedef unsigned short u16;
@@ -223,8 +269,11 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const f32x1
   for (int i = 0; i < WM; ++i) {
     const int row0 = m0 + (wm * WM + i) * 32;
     if (row0 >= p.M) break;  // (uniform)
-    const int gm_w = min(row0 + (lane & 31), p.M - 1);
-    const float bias = p.row_bias ? p.row_bias[gm_w] : 0.f;
+    float bias[2] = {0.f, 0.f};   // of the row(s) this lane holds sums of
+    if (p.row_bias) {
+      bias[0] = p.row_bias[min(row0 + Acc::row(0, lane), p.M - 1)];
+      bias[1] = p.row_bias[min(row0 + Acc::row(4 * WN - 1, lane), p.M - 1)];
+    }
     if (aux) {
 #pragma unroll
       for (int t = 0; t < 32 / RPI; ++t) {
@@ -244,34 +293,32 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const f32x1
       }
     }
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        u16 h[4];
-        u32x2* at = reinterpret_cast<u32x2*>(lds + (lane & 31) * ROWB + (j * 32 + q * 8 + (lane >> 5) * 4) * 2);
-        f32x4 o = {0.f, 0.f, 0.f, 0.f};
-        if (partial) o = *reinterpret_cast<const f32x4*>(partial + ((i * WN + j) * 4 + q) * 256);   // the other half of K
-        float other[4] = {0.f, 0.f, 0.f, 0.f};
-        if (aux) {
-          const u32x2 w = *at;
-          other[0] = f16_to_32((u16)(w.x & 0xffffu), BF16);
-          other[1] = f16_to_32((u16)(w.x >> 16), BF16);
-          other[2] = f16_to_32((u16)(w.y & 0xffffu), BF16);
-          other[3] = f16_to_32((u16)(w.y >> 16), BF16);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float y = acc[i][j][q * 4 + e] + o[e] + bias;
-          if (aux && p.aux_mode == kGemmAdd) y += other[e];
-          if (p.relu) y = fmaxf(y, 0.f);
-          if (aux && p.aux_mode == kGemmTimesSilu) y *= other[e] / (1.f + __expf(-other[e]));
-          h[e] = f32_to_16(y, BF16);
-        }
-        u32x2 w;
-        w.x = (unsigned)h[0] | ((unsigned)h[1] << 16);
-        w.y = (unsigned)h[2] | ((unsigned)h[3] << 16);
-        *at = w;
+    for (int t = 0; t < 4 * WN; ++t) {
+      u16 h[4];
+      u32x2* at = reinterpret_cast<u32x2*>(lds + Acc::row(t, lane) * ROWB + Acc::col(t, lane) * 2);
+      const f32x4 mine = acc.quad(i, t);
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+      if (partial) o = *reinterpret_cast<const f32x4*>(partial + (i * 4 * WN + t) * 256);   // the other half of K
+      float other[4] = {0.f, 0.f, 0.f, 0.f};
+      if (aux) {
+        const u32x2 w = *at;
+        other[0] = f16_to_32((u16)(w.x & 0xffffu), BF16);
+        other[1] = f16_to_32((u16)(w.x >> 16), BF16);
+        other[2] = f16_to_32((u16)(w.y & 0xffffu), BF16);
+        other[3] = f16_to_32((u16)(w.y >> 16), BF16);
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float y = mine[e] + o[e] + bias[t / (2 * WN)];
+        if (aux && p.aux_mode == kGemmAdd) y += other[e];
+        if (p.relu) y = fmaxf(y, 0.f);
+        if (aux && p.aux_mode == kGemmTimesSilu) y *= other[e] / (1.f + __expf(-other[e]));
+        h[e] = f32_to_16(y, BF16);
+      }
+      u32x2 w;
+      w.x = (unsigned)h[0] | ((unsigned)h[1] << 16);
+      w.y = (unsigned)h[2] | ((unsigned)h[3] << 16);
+      *at = w;
     }
 #pragma unroll
     for (int t = 0; t < 32 / RPI; ++t) {
@@ -323,13 +370,8 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int tile_m, int t
   const u16* __restrict__ B = static_cast<const u16*>(p.B) + (size_t)z * p.stride_b;
   u16* __restrict__ C = static_cast<u16*>(p.C) + (size_t)z * p.stride_c;
 
-  f32x16 acc[WM][WN];
-#pragma unroll
-  for (int i = 0; i < WM; ++i)
-#pragma unroll
-    for (int j = 0; j < WN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  Acc32<WM, WN> acc;
+  acc.clear();
 
   Stage regs[SETS];  // regs[t % SETS] carries tile t (statically indexed below)
 
@@ -387,7 +429,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int tile_m, int t
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
-          for (int j = 0; j < WN; ++j) acc[i][j] = mfma_32x32x16<BF16>(fb[h][j], fa[h][i], acc[i][j]);
+          for (int j = 0; j < WN; ++j) acc.v[i][j] = mfma_32x32x16<BF16>(fb[h][j], fa[h][i], acc.v[i][j]);
     }
     // unconditional on purpose (see GemmStage::load): past the last tile this writes zeros to the
     // idle buffer and fetches clamped addresses

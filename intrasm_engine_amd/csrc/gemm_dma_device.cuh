@@ -90,6 +90,19 @@ __device__ __forceinline__ int kn_fragment_offset(int lane, int block) {
   return kr * (ROW_ELEMS * 2) + c * 16 + (lane & 1) * 8;
 }
 
+// The same for fragments of 16 rows (columns) x 32 k: a read of 32 lanes covers 4 k rows and the 4 k rows 8 further, 32
+// bytes of each, and the permutation puts them into the eight different 8-bank groups.
+template <int ROW_ELEMS>
+__device__ __forceinline__ int kn16_swizzle(int kr) {
+  return ROW_ELEMS >= 128 ? ((kr & 3) << 1) | (kr & 8) : (kr & 2) | ((kr & 8) >> 1);
+}
+template <int ROW_ELEMS>
+__device__ __forceinline__ int kn16_fragment_offset(int lane, int block) {
+  const int kr = (lane >> 4) * 8 + ((lane & 15) >> 2);
+  const int c = (block * 2 + ((lane & 3) >> 1)) ^ kn16_swizzle<ROW_ELEMS>(kr);
+  return kr * (ROW_ELEMS * 2) + c * 16 + (lane & 1) * 8;
+}
+
 template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, int BK, int STAGES, int SPLIT = 0, bool TRANS_A = false>
 __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, int tile_n, int z, unsigned char* smem) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32, WAVES = 2 * WCN;
@@ -106,7 +119,7 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
                 "every wavefront fetches whole kilobytes of A and of B");
   static_assert(TRANS_B || (CPRB >= 16 && CPRB <= 64), "(K,N) layout: 128 <= BN <= 512");
   static_assert(!TRANS_A || (CPRA >= 8 && CPRA <= 64), "(K,M) layout: 64 <= BM <= 512");
-  static_assert(STAGES >= 3 && (BK / 16) % 2 == 0 && (STAGES - 2) * LOADS < 64, "stages in flight must fit the load counter");
+  static_assert(STAGES >= 3 && (STAGES - 2) * LOADS < 64, "stages in flight must fit the load counter");
   typedef unsigned short u16;
   typedef __attribute__((address_space(3))) unsigned char lds_u8;
 
@@ -129,7 +142,7 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
   for (int q = 0; q < A_INSTR; ++q) {
     if constexpr (TRANS_A) {
       const int kr = (wave * A_INSTR + q) * RPIA + lane / CPRA;
-      a_row[q] = A + min(m0 + ((lane % CPRA) ^ kn_swizzle<BM>(kr)) * 8, lda - 8);
+      a_row[q] = A + min(m0 + ((lane % CPRA) ^ kn16_swizzle<BM>(kr)) * 8, lda - 8);
       a_k8[q] = kr;
     } else {
       const int row = (wave * A_INSTR + q) * RPI + lane / CPR;
@@ -149,7 +162,7 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
       b_k8[q] = ((lane % CPR) ^ sw) * 8;
     } else {
       const int kr = (wave * B_INSTR + q) * RPIB + lane / CPRB;
-      b_row[q] = B + min(n0 + ((lane % CPRB) ^ kn_swizzle<BN>(kr)) * 8, ldb - 8);
+      b_row[q] = B + min(n0 + ((lane % CPRB) ^ kn16_swizzle<BN>(kr)) * 8, ldb - 8);
       b_k8[q] = kr;
     }
   }
@@ -191,47 +204,43 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
       if (k0 + b_k8[q] >= p.K) *reinterpret_cast<u32x4*>(st + A_BYTES + ((wave * B_INSTR + q) * 64 + lane) * 16) = zero;
   };
 
-  f32x16 acc[WM][WN];
-#pragma unroll
-  for (int i = 0; i < WM; ++i)
-#pragma unroll
-    for (int j = 0; j < WN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  Acc16<WM, WN> acc;
+  acc.clear();
 
-  // ---- operand read addresses inside a stage (bytes), one per 16-wide sub-step (and per column
-  // block for the transpose reads): the chunk permutation makes them differ by more than a constant
-  constexpr int KS = BK / 16;
-  const int frow = lane & 31, fkh = lane >> 5;
-  const int fsw = CPR == 4 ? (frow >> 2) & 3 : (frow >> 1) & 7;
-  int a_off[TRANS_A ? WM : KS];
+  // ---- operand read addresses inside a stage (bytes), one per 32-wide sub-step (and per row or column block for the
+  // transpose reads): the chunk permutation makes them differ by more than a constant.  A fragment is 16 rows (columns) x
+  // 32 k, lane l has row l % 16 and the 8 k of chunk l / 16.
+  constexpr int KS = BK / 32;
+  const int frow = lane & 15, fch = lane >> 4;
+  const int fsw = CPR == 4 ? frow >> 2 : frow >> 1;
+  int a_off[TRANS_A ? 2 * WM : KS];
   if constexpr (TRANS_A) {
 #pragma unroll
-    for (int i = 0; i < WM; ++i) a_off[i] = kn_fragment_offset<BM>(lane, wm * WM + i);
+    for (int i = 0; i < 2 * WM; ++i) a_off[i] = kn16_fragment_offset<BM>(lane, wm * 2 * WM + i);
   } else {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) a_off[ks] = (wm * WM * 32 + frow) * RB + (((ks * 2 + fkh) ^ fsw) * 16);
+    for (int ks = 0; ks < KS; ++ks) a_off[ks] = (wm * WM * 32 + frow) * RB + (((ks * 4 + fch) ^ fsw) * 16);
   }
-  int b_off[TRANS_B ? KS : WN];
+  int b_off[TRANS_B ? KS : 2 * WN];
   if constexpr (TRANS_B) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) b_off[ks] = A_BYTES + (wn * WN * 32 + frow) * RB + (((ks * 2 + fkh) ^ fsw) * 16);
+    for (int ks = 0; ks < KS; ++ks) b_off[ks] = A_BYTES + (wn * WN * 32 + frow) * RB + (((ks * 4 + fch) ^ fsw) * 16);
   } else {
 #pragma unroll
-    for (int j = 0; j < WN; ++j) b_off[j] = A_BYTES + kn_fragment_offset<BN>(lane, wn * WN + j);
+    for (int j = 0; j < 2 * WN; ++j) b_off[j] = A_BYTES + kn16_fragment_offset<BN>(lane, wn * 2 * WN + j);
   }
 
-  u32x4 fa[2][WM], fb[2][WN];  // operand fragments of two consecutive sub-steps
+  u32x4 fa[2][2 * WM], fb[2][2 * WN];  // operand fragments of two consecutive sub-steps
   auto read_frags = [&](const unsigned char* st, int ks, int buf) {
 #pragma unroll
-    for (int i = 0; i < WM; ++i) {
-      if constexpr (TRANS_A) fa[buf][i] = kn_fragment<BM * 2>(st + a_off[i] + ks * 16 * (BM * 2));
-      else fa[buf][i] = *reinterpret_cast<const u32x4*>(st + a_off[ks] + i * 32 * RB);
+    for (int i = 0; i < 2 * WM; ++i) {
+      if constexpr (TRANS_A) fa[buf][i] = kn_fragment<BM * 2>(st + a_off[i] + ks * 32 * (BM * 2));
+      else fa[buf][i] = *reinterpret_cast<const u32x4*>(st + a_off[ks] + i * 16 * RB);
     }
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      if constexpr (TRANS_B) fb[buf][j] = *reinterpret_cast<const u32x4*>(st + b_off[ks] + j * 32 * RB);
-      else fb[buf][j] = kn_fragment<BN * 2>(st + b_off[j] + ks * 16 * (BN * 2));
+    for (int j = 0; j < 2 * WN; ++j) {
+      if constexpr (TRANS_B) fb[buf][j] = *reinterpret_cast<const u32x4*>(st + b_off[ks] + j * 16 * RB);
+      else fb[buf][j] = kn_fragment<BN * 2>(st + b_off[j] + ks * 32 * (BN * 2));
     }
   };
 
@@ -248,19 +257,20 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
   // a tile): wait for my loads of that tile, barrier (everybody's have landed and everybody has
   // read the previous tile for the last time), and then the next direct loads are issued between
   // the MFMAs of this sub-step, into the stage the previous tile just left.
-  constexpr int NM = WM * WN;
-  for (int kt = 0; kt < KT; ++kt) {
+  constexpr int NM = 4 * WM * WN;
+  // parity: which buffer the tile's first sub-step is in (compile-time, so that the fragments stay in registers)
+  auto tile_step = [&](int kt, auto parity) {
     const unsigned char* st = smem + (kt % STAGES) * STAGE_BYTES;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const int cur = ks & 1;
+      const int cur = (decltype(parity)::value + ks) & 1;
       if (ks + 1 < KS) {
         read_frags(st, ks + 1, cur ^ 1);
         __builtin_amdgcn_sched_barrier(0);  // reads first: the compiler would sink them behind the MFMAs
 #pragma unroll
-        for (int i = 0; i < WM; ++i)
+        for (int i = 0; i < 2 * WM; ++i)
 #pragma unroll
-          for (int j = 0; j < WN; ++j) acc[i][j] = mfma_32x32x16<BF16>(fb[cur][j], fa[cur][i], acc[i][j]);
+          for (int j = 0; j < 2 * WN; ++j) acc.v[i][j] = mfma_16x16x32<BF16>(fb[cur][j], fa[cur][i], acc.v[i][j]);
       } else {
         wait_vmcnt<(STAGES - 3) * LOADS>();  // my loads of tile kt + 1 have landed
         if (tail && kt + 2 == KT) zero_tail(kt + 1, (kt + 1) % STAGES);
@@ -269,18 +279,26 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
         __builtin_amdgcn_sched_barrier(0);
         const int next = kt + STAGES - 1;
 #pragma unroll
-        for (int i = 0; i < WM; ++i)
+        for (int i = 0; i < 2 * WM; ++i)
 #pragma unroll
-          for (int j = 0; j < WN; ++j) {
-            acc[i][j] = mfma_32x32x16<BF16>(fb[cur][j], fa[cur][i], acc[i][j]);
-            const int m = i * WN + j;
+          for (int j = 0; j < 2 * WN; ++j) {
+            acc.v[i][j] = mfma_16x16x32<BF16>(fb[cur][j], fa[cur][i], acc.v[i][j]);
+            const int m = i * 2 * WN + j;
 #pragma unroll
             for (int q = m * LOADS / NM; q < (m + 1) * LOADS / NM; ++q)
               issue_one(next, next % STAGES, q);
           }
       }
     }
+  };
+  const std::integral_constant<int, 0> first;
+  const std::integral_constant<int, KS & 1> second;
+  int kt = 0;
+  for (; kt + 2 <= KT; kt += 2) {
+    tile_step(kt, first);
+    tile_step(kt + 1, second);
   }
+  if (kt < KT) tile_step(kt, first);
   wait_vmcnt<0>();  // the re-fetched last tiles: nothing may still be writing LDS when the workgroup ends
 
   const float* partial = nullptr;
@@ -302,13 +320,10 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int j = 0; j < WN; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const f32x4 v = {acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
-            *reinterpret_cast<f32x4*>(mine + ((i * WN + j) * 4 + q) * 256) = v;
-            if (q == 3) __builtin_amdgcn_sched_barrier(0);
-          }
+        for (int t = 0; t < 4 * WN; ++t) {
+          *reinterpret_cast<f32x4*>(mine + (i * 4 * WN + t) * 256) = acc.quad(i, t);
+          if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
       // The two workgroups of a tile run on one XCD (the launcher's numbering; one partition spanning the whole GPU,
       // ids dealt round-robin to the XCDs), whose L2 both see.  Every wavefront waits until L2 has acknowledged its own
       // stores (vmcnt counts stores until then), the barrier collects all of them, and only then the flag goes up.
@@ -348,12 +363,7 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
-      for (int j = 0; j < WN; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4 v = {acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
-          *reinterpret_cast<f32x4*>(mine + ((i * WN + j) * 4 + q) * 256) = v;
-        }
+      for (int t = 0; t < 4 * WN; ++t) *reinterpret_cast<f32x4*>(mine + (i * 4 * WN + t) * 256) = acc.quad(i, t);
     wait_vmcnt<0>();   // (vmcnt counts a store until L2 has acknowledged it)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();   // everybody's sums are in L2, and everybody has read its last fragments: the stages are free
@@ -365,24 +375,13 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
     // stay at workgroup scope: a device-scope acquire here invalidates the XCD's L2 under every workgroup still
     // multiplying (measured: 4096 x 256 x 4096 21.8 -> 28.7 us), a device-scope release writes it back.
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-      for (int j = 0; j < WN; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    acc.clear();
     for (int s = 0; s < parts; ++s) {
       const float* from = all + (size_t)s * (BM * BN);
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int j = 0; j < WN; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(from + ((i * WN + j) * 4 + q) * 256);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[i][j][q * 4 + e] += v[e];
-          }
+        for (int t = 0; t < 4 * WN; ++t) acc.add(i, t, *reinterpret_cast<const f32x4*>(from + (i * 4 * WN + t) * 256));
     }
   }
   static_assert(WAVES * gemm_store_lds_bytes<WN>() <= gemm_dma_lds_bytes<WM, WN, WCN, BK, STAGES>(), "the epilogue fits the stages");

@@ -79,7 +79,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   for (int q = 0; q < A_INSTR; ++q) {
     if constexpr (TRANS_A) {
       const int kr = (wave * A_INSTR + q) * RPIA + lane / CPRA;
-      a_ptr[q] = A + min(m0 + ((lane % CPRA) ^ kn_swizzle<BM>(kr)) * 8, lda - 8);
+      a_ptr[q] = A + min(m0 + ((lane % CPRA) ^ kn16_swizzle<BM>(kr)) * 8, lda - 8);
       a_k8[q] = kr;
     } else {
       const int row = (wave * A_INSTR + q) * 8 + lane / 8;
@@ -98,7 +98,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
       b_k8[q] = ((lane % 4) ^ sw) * 8;
     } else {
       const int kr = (wave * B_INSTR + q) * RPIB + lane / CPRB;
-      b_row[q] = B + min(n0 + ((lane % CPRB) ^ kn_swizzle<BN>(kr)) * 8, ldb - 8);
+      b_row[q] = B + min(n0 + ((lane % CPRB) ^ kn16_swizzle<BN>(kr)) * 8, ldb - 8);
       b_k8[q] = kr;
     }
   }
@@ -146,34 +146,29 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
       if (ph * 32 + b_k8[q] >= p.K) *reinterpret_cast<u32x4*>(sb + ((wave * B_INSTR + q) * 64 + lane) * 16) = zero;
   };
 
-  f32x16 acc[WM][WN];
-#pragma unroll
-  for (int i = 0; i < WM; ++i)
-#pragma unroll
-    for (int j = 0; j < WN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  Acc16<WM, WN> acc;
+  acc.clear();
 
-  // ---- operand read addresses inside a stage (bytes), one per 16-wide sub-step
-  const int frow = lane & 31, fkh = lane >> 5;
-  int a_off[TRANS_A ? WM : 4];   // the four sub-steps of an A tile, or the row blocks of a (K,M) one
+  // ---- operand read addresses inside a stage (bytes): a fragment is 16 rows (columns) x 32 k, lane l has row l % 16 and
+  // the 8 k of chunk l / 16
+  const int frow = lane & 15, fch = lane >> 4;
+  int a_off[TRANS_A ? 2 * WM : 2];   // the two halves of an A tile, or the row blocks of a (K,M) one
   if constexpr (TRANS_A) {
 #pragma unroll
-    for (int i = 0; i < WM; ++i) a_off[i] = kn_fragment_offset<BM>(lane, wm * WM + i);
+    for (int i = 0; i < 2 * WM; ++i) a_off[i] = kn16_fragment_offset<BM>(lane, wm * 2 * WM + i);
   } else {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) a_off[ks] = (wm * WM * 32 + frow) * 128 + (((ks * 2 + fkh) ^ ((frow >> 1) & 7)) * 16);
+    for (int h = 0; h < 2; ++h) a_off[h] = (wm * WM * 32 + frow) * 128 + (((h * 4 + fch) ^ (frow >> 1)) * 16);
   }
-  int b_off[TRANS_B ? 2 : WN];
+  int b_off[TRANS_B ? 1 : 2 * WN];
   if constexpr (TRANS_B) {
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) b_off[ks] = B_BASE + (wn * WN * 32 + frow) * 64 + (((ks * 2 + fkh) ^ ((frow >> 2) & 3)) * 16);
+    b_off[0] = B_BASE + (wn * WN * 32 + frow) * 64 + ((fch ^ (frow >> 2)) * 16);
   } else {
 #pragma unroll
-    for (int j = 0; j < WN; ++j) b_off[j] = B_BASE + kn_fragment_offset<BN>(lane, wn * WN + j);
+    for (int j = 0; j < 2 * WN; ++j) b_off[j] = B_BASE + kn16_fragment_offset<BN>(lane, wn * 2 * WN + j);
   }
 
-  u32x4 fa[2][WM], fb[2][WN];  // the operand fragments of one phase (two sub-steps of 16)
+  u32x4 fa[2 * WM], fb[2 * WN];  // the operand fragments of one phase
   const std::integral_constant<int, 0> even;
   const std::integral_constant<int, 1> odd;
   // parity = ph % 2 at compile time: which half of the A tile
@@ -182,17 +177,14 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
     const unsigned char* sa = smem + ((ph >> 1) % SA) * A_STAGE;
     const unsigned char* sb = smem + (ph % SB) * B_STAGE;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+    for (int i = 0; i < 2 * WM; ++i) {
+      if constexpr (TRANS_A) fa[i] = kn_fragment<BM * 2>(sa + a_off[i] + h * 32 * (BM * 2));
+      else fa[i] = *reinterpret_cast<const u32x4*>(sa + a_off[h] + i * 16 * 128);
+    }
 #pragma unroll
-      for (int i = 0; i < WM; ++i) {
-        if constexpr (TRANS_A) fa[s][i] = kn_fragment<BM * 2>(sa + a_off[i] + (2 * h + s) * 16 * (BM * 2));
-        else fa[s][i] = *reinterpret_cast<const u32x4*>(sa + a_off[2 * h + s] + i * 32 * 128);
-      }
-#pragma unroll
-      for (int j = 0; j < WN; ++j) {
-        if constexpr (TRANS_B) fb[s][j] = *reinterpret_cast<const u32x4*>(sb + b_off[s] + j * 32 * 64);
-        else fb[s][j] = kn_fragment<BN * 2>(sb + b_off[j] + s * 16 * (BN * 2));
-      }
+    for (int j = 0; j < 2 * WN; ++j) {
+      if constexpr (TRANS_B) fb[j] = *reinterpret_cast<const u32x4*>(sb + b_off[0] + j * 16 * 64);
+      else fb[j] = kn_fragment<BN * 2>(sb + b_off[j]);
     }
     issue_a((ph >> 1) + 2, parity);
     issue_b(ph + 3);
@@ -200,11 +192,9 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   auto compute_phase = [&]() {
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int i = 0; i < 2 * WM; ++i)
 #pragma unroll
-      for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j) acc[i][j] = mfma_32x32x16<BF16>(fb[s][j], fa[s][i], acc[i][j]);
+      for (int j = 0; j < 2 * WN; ++j) acc.v[i][j] = mfma_16x16x32<BF16>(fb[j], fa[i], acc.v[i][j]);
     __builtin_amdgcn_s_setprio(0);
   };
   // at the end of phase ph: my loads of what phase ph + 1 reads have landed (two phases' worth may still fly)
