@@ -1,5 +1,5 @@
 // Dense GEMM tile for gfx950 whose operands travel from global memory straight into LDS
-// (global_load_lds_dwordx4): no staging registers and no ds_write in the main loop.
+// (buffer_load_dwordx4 ... lds): no staging registers and no ds_write in the main loop.
 //
 // Why: a ds_write_b128 stream runs at 64 bytes/clock/CU and, while it runs, takes a quarter of
 // the LDS read rate away from the MFMA operand reads; with register staging the writes of one K
@@ -12,11 +12,13 @@
 // chunk of global memory each lane fetches instead:
 //   K-contiguous operands (A, and B given as (N, K)): LDS row = BK elements; position (row, c)
 //     holds global chunk c ^ sw(row), sw(row) = (row >> 2) & 3 for BK = 32 ((row >> 1) & 7 for 64):
-//     the 16 lanes of a 128-bit operand read hit 16 different 4-bank groups.
-//   B given as (K, N), A given as (K, M): LDS row = BN (BM) elements; position (k, c) holds global chunk
-//     c ^ ((k & 3) << 2): the 32 lanes of a transpose read (4 k rows x 2 column halves x 32 bytes) hit 8 different
-//     8-bank groups.  (64 elements per row, of which two share the 64 banks: c ^ ((k & 2) << 1).)
-// Pipeline: STAGES LDS stages; the operand fragments of a 16-wide sub-step are read from LDS while
+//     the 16 rows of a fragment's chunk hit 16 different 4-bank groups.
+//   B given as (K, N), A given as (K, M): LDS row = BN (BM) elements, permuted by kn16_swizzle (k row): the 32 lanes of a
+//     transpose read hit 8 different 8-bank groups.
+// The addresses are buffer addresses: what changes from K step to K step is one scalar offset.  With 64-bit addresses per
+// lane (global_load_lds) a load cost four vector instructions and twice the address registers read, and the loads, not the
+// bytes, were what the loop waited for: 8192^3 1319 -> 1465 TFLOP/s (bf16, B as (K, N)), 4096 x 8192 x 4096 1269 -> 1397.
+// Pipeline: STAGES LDS stages; the operand fragments of a 32-wide sub-step are read from LDS while
 // the MFMAs of the sub-step before it run, and once per tile (before the first fragment read of
 // tile t+1): wait for my loads of tile t+1 | barrier | issue tile t+STAGES-1, between MFMAs, into
 // the stage that tile t-1 just left.
@@ -31,6 +33,17 @@ namespace iex {
 
 __device__ __forceinline__ void lds_dma16(const void* g, unsigned lds_base_uniform) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_base_uniform) : "memory", "m0");
+}
+
+// The same by buffer address: base, size and scalar offset in scalar registers, one 32-bit offset per lane that never changes, so a load of the loop
+// costs no vector instruction; what lies past the end is not read (zeros arrive).
+__device__ __forceinline__ void lds_dma16(u32x4 rsrc, unsigned lane_offset, unsigned uniform_offset, unsigned lds_base_uniform) {
+  asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(lane_offset), "s"(rsrc), "s"(uniform_offset), "s"(lds_base_uniform) : "memory", "m0");
+}
+__device__ __forceinline__ u32x4 buffer_of(const void* base_uniform, size_t bytes) {
+  const size_t at = reinterpret_cast<size_t>(base_uniform);
+  return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((unsigned)at), (unsigned)__builtin_amdgcn_readfirstlane((unsigned)(at >> 32) & 0xffffu),
+               (unsigned)__builtin_amdgcn_readfirstlane((unsigned)(bytes < 0xffffffffu ? bytes : 0xffffffffu)), 4u << 15};   // raw buffer of 32-bit words
 }
 
 template <int N>
@@ -135,63 +148,56 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
   const int lda = p.lda ? p.lda : TRANS_A ? p.M : p.K, ldb = p.ldb ? p.ldb : TRANS_B ? p.K : p.N;   // row strides
   const int last_kb = (p.kb ? p.kb : p.K) - 1;   // the last k row of a (K,N) B
 
-  // ---- what this lane fetches: per instruction a row pointer (or a column offset) and a chunk
-  const u16* a_row[A_INSTR];  // (M,K): row pointer; (K,M): A + clamped row
-  int a_k8[A_INSTR];          // (M,K): element offset of the chunk inside a K step; (K,M): k row inside a K step
+  // ---- what this lane fetches, as byte offsets at k = 0.  Rows past M (columns past N) are the last one's: they feed rows
+  // (columns) of C that are not stored.
+  const u32x4 a_buf = TRANS_A ? buffer_of(A, (size_t)p.K * lda * 2) : buffer_of(A + (size_t)m0 * lda, (size_t)(p.M - m0) * lda * 2);
+  const u32x4 b_buf = TRANS_B ? buffer_of(B + (size_t)n0 * ldb, (size_t)(p.N - n0) * ldb * 2) : buffer_of(B, (size_t)(last_kb + 1) * ldb * 2);
+  unsigned a_lane[A_INSTR];
+  int a_k8[A_INSTR];          // (M,K): first k of the chunk inside a K step; (K,M): k row inside a K step
 #pragma unroll
   for (int q = 0; q < A_INSTR; ++q) {
     if constexpr (TRANS_A) {
       const int kr = (wave * A_INSTR + q) * RPIA + lane / CPRA;
-      a_row[q] = A + min(m0 + ((lane % CPRA) ^ kn16_swizzle<BM>(kr)) * 8, lda - 8);
       a_k8[q] = kr;
+      a_lane[q] = ((unsigned)kr * lda + min(m0 + ((lane % CPRA) ^ kn16_swizzle<BM>(kr)) * 8, lda - 8)) * 2u;
     } else {
       const int row = (wave * A_INSTR + q) * RPI + lane / CPR;
-      const int sw = CPR == 4 ? (row >> 2) & 3 : (row >> 1) & 7;
-      a_row[q] = A + (size_t)min(m0 + row, p.M - 1) * lda;
-      a_k8[q] = ((lane % CPR) ^ sw) * 8;
+      a_k8[q] = ((lane % CPR) ^ (CPR == 4 ? (row >> 2) & 3 : (row >> 1) & 7)) * 8;
+      a_lane[q] = ((unsigned)min(row, p.M - 1 - m0) * lda + a_k8[q]) * 2u;
     }
   }
-  const u16* b_row[B_INSTR];  // (N,K): row pointer; (K,N): B + clamped column
-  int b_k8[B_INSTR];          // (N,K): chunk offset inside a K step; (K,N): k row inside a K step
+  unsigned b_lane[B_INSTR];
+  int b_k8[B_INSTR];
 #pragma unroll
   for (int q = 0; q < B_INSTR; ++q) {
     if constexpr (TRANS_B) {
       const int row = (wave * B_INSTR + q) * RPI + lane / CPR;
-      const int sw = CPR == 4 ? (row >> 2) & 3 : (row >> 1) & 7;
-      b_row[q] = B + (size_t)min(n0 + row, p.N - 1) * ldb;
-      b_k8[q] = ((lane % CPR) ^ sw) * 8;
+      b_k8[q] = ((lane % CPR) ^ (CPR == 4 ? (row >> 2) & 3 : (row >> 1) & 7)) * 8;
+      b_lane[q] = ((unsigned)min(row, p.N - 1 - n0) * ldb + b_k8[q]) * 2u;
     } else {
       const int kr = (wave * B_INSTR + q) * RPIB + lane / CPRB;
-      b_row[q] = B + min(n0 + ((lane % CPRB) ^ kn16_swizzle<BN>(kr)) * 8, ldb - 8);
       b_k8[q] = kr;
+      b_lane[q] = ((unsigned)kr * ldb + min(n0 + ((lane % CPRB) ^ kn16_swizzle<BN>(kr)) * 8, ldb - 8)) * 2u;
     }
   }
-  const int last_k8 = p.K - 8;
+  const unsigned a_step = (TRANS_A ? (unsigned)BK * lda : (unsigned)BK) * 2u, b_step = (TRANS_B ? (unsigned)BK : (unsigned)BK * ldb) * 2u;
   const int KT = (p.K + BK - 1) / BK;
 
-  // instruction q of a tile: A for q < A_INSTR, then B
+  // instruction q of a tile: A for q < A_INSTR, then B.  Past the end: the last tile again, into a stage nobody reads.  (A
+  // chunk past a row's end is the next row's, or nothing: zero_tail.)
   auto issue_one = [&](int kt, int stage, int q) {
-    const int k0 = min(kt, KT - 1) * BK;  // past the end: the last tile again, into a stage nobody reads
-    if (q < A_INSTR) {
-      const unsigned base = lds0 + stage * STAGE_BYTES + wave * (A_INSTR * 1024);
-      if constexpr (TRANS_A)
-        lds_dma16(a_row[q] + (size_t)min(k0 + a_k8[q], p.K - 1) * lda, __builtin_amdgcn_readfirstlane(base + q * 1024));
-      else
-        lds_dma16(a_row[q] + min(k0 + a_k8[q], last_k8), __builtin_amdgcn_readfirstlane(base + q * 1024));
-    } else {
-      const int qb = q - A_INSTR;
-      const unsigned bbase = lds0 + stage * STAGE_BYTES + A_BYTES + wave * (B_INSTR * 1024);
-      if constexpr (TRANS_B)
-        lds_dma16(b_row[qb] + min(k0 + b_k8[qb], last_k8), __builtin_amdgcn_readfirstlane(bbase + qb * 1024));
-      else
-        lds_dma16(b_row[qb] + (size_t)min(k0 + b_k8[qb], last_kb) * ldb, __builtin_amdgcn_readfirstlane(bbase + qb * 1024));
-    }
+    const unsigned t = min(kt, KT - 1);
+    if (q < A_INSTR)
+      lds_dma16(a_buf, a_lane[q], t * a_step, __builtin_amdgcn_readfirstlane(lds0 + stage * STAGE_BYTES + (wave * A_INSTR + q) * 1024));
+    else
+      lds_dma16(b_buf, b_lane[q - A_INSTR], t * b_step,
+                __builtin_amdgcn_readfirstlane(lds0 + stage * STAGE_BYTES + A_BYTES + (wave * B_INSTR + q - A_INSTR) * 1024));
   };
   auto issue = [&](int kt, int stage) {
 #pragma unroll
     for (int q = 0; q < LOADS; ++q) issue_one(kt, stage, q);
   };
-  // entries at k >= K of the last tile must be zero: clamped addresses delivered copies of real data
+  // entries at k >= K of the last tile must be zero: what was loaded there is other data
   auto zero_tail = [&](int kt, int stage) {
     const int k0 = kt * BK;
     unsigned char* st = smem + stage * STAGE_BYTES;

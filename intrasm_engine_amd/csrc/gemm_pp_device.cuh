@@ -12,10 +12,13 @@
 //
 //   M(p)  = memory phase p: read the operand fragments of 32 k of the tile from LDS into registers,
 //           issue my share of the direct loads (global memory -> LDS) of the tile STAGES - 1 ahead;
-//   C(p)  = compute phase p: the WM x WN x 2 MFMAs on those fragments, nothing else.
+//   C(p)  = compute phase p: the 4 * WM * WN MFMAs (16 x 16 x 32) on those fragments, nothing else.
 // Intervals are separated by workgroup barriers, so on every SIMD one wavefront feeds the matrix cores while
 // the other one waits for LDS and issues loads, and all waits hide behind the other group's MFMAs.
-// A wavefront owns WM x WN MFMA tiles of 32 x 32 (128 x 64 of a 256 x 256 tile with WM = 4, WN = 2, WCN = 4).
+// A wavefront owns WM x WN blocks of 32 x 32 (128 x 64 of a 256 x 256 tile with WM = 4, WN = 2, WCN = 4).
+// What bounds it (8192^3, bf16, TFLOP/s): 1440 as it is, 1650 without the loads, 1540 with fragments read once, 1760 with
+// neither (MFMAs and barriers; MFMAs alone run at 2100, the card's power limit on random operands).  One barrier per phase
+// instead of strict alternation: 1315; loads before the fragment reads: the same; multiplying at raised priority: 1-2 % slower.
 //
 // Stage reuse: what phase p reads was last needed by phase p (group 1 reads it one interval after group 0), and the
 // loads that overwrite it go out in later M phases.  A wavefront waits for its own loads of what phase p + 1 reads at
@@ -72,67 +75,57 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
 
   // ---- what this lane fetches.  A: 8 rows of 128 bytes per instruction, LDS position (row, c) holds global chunk
   // c ^ ((row >> 1) & 7).  B as (N,K): 16 rows of 64 bytes, chunk c ^ ((row >> 2) & 3).  B as (K,N): k rows of BN
-  // elements, chunk c ^ ((k & 3) << 2), and A as (K,M) likewise, 64 k rows of BM elements per stage.
-  const u16* a_ptr[A_INSTR];   // (M,K): row pointer + chunk offset, advanced by 64 k per A tile; (K,M): A + clamped row
-  int a_k8[A_INSTR];           // (M,K): chunk offset inside a tile; (K,M): k row inside a tile
+  // elements, chunk c ^ kn16_swizzle(k), and A as (K,M) likewise, 64 k rows of BM elements per stage.
+  // Rows past M (columns past N) are the last one's: they feed rows (columns) of C that are not stored.
+  const u32x4 a_buf = TRANS_A ? buffer_of(A, (size_t)p.K * lda * 2) : buffer_of(A + (size_t)m0 * lda, (size_t)(p.M - m0) * lda * 2);
+  const u32x4 b_buf = TRANS_B ? buffer_of(B + (size_t)n0 * ldb, (size_t)(p.N - n0) * ldb * 2) : buffer_of(B, (size_t)(last_kb + 1) * ldb * 2);
+  unsigned a_lane[A_INSTR];    // byte offset inside the buffer at k = 0
+  int a_k8[A_INSTR];           // (M,K): first k of the chunk inside a tile; (K,M): k row inside a tile
 #pragma unroll
   for (int q = 0; q < A_INSTR; ++q) {
     if constexpr (TRANS_A) {
       const int kr = (wave * A_INSTR + q) * RPIA + lane / CPRA;
-      a_ptr[q] = A + min(m0 + ((lane % CPRA) ^ kn16_swizzle<BM>(kr)) * 8, lda - 8);
       a_k8[q] = kr;
+      a_lane[q] = ((unsigned)kr * lda + min(m0 + ((lane % CPRA) ^ kn16_swizzle<BM>(kr)) * 8, lda - 8)) * 2u;
     } else {
       const int row = (wave * A_INSTR + q) * 8 + lane / 8;
       a_k8[q] = ((lane % 8) ^ ((row >> 1) & 7)) * 8;
-      a_ptr[q] = A + (size_t)min(m0 + row, p.M - 1) * lda + a_k8[q];
+      a_lane[q] = ((unsigned)min(row, p.M - 1 - m0) * lda + a_k8[q]) * 2u;
     }
   }
-  const u16* b_row[B_INSTR];
+  unsigned b_lane[B_INSTR];
   int b_k8[B_INSTR];
 #pragma unroll
   for (int q = 0; q < B_INSTR; ++q) {
     if constexpr (TRANS_B) {
       const int row = (wave * B_INSTR + q) * 16 + lane / 4;
-      const int sw = (row >> 2) & 3;
-      b_row[q] = B + (size_t)min(n0 + row, p.N - 1) * ldb;
-      b_k8[q] = ((lane % 4) ^ sw) * 8;
+      b_k8[q] = ((lane % 4) ^ ((row >> 2) & 3)) * 8;
+      b_lane[q] = ((unsigned)min(row, p.N - 1 - n0) * ldb + b_k8[q]) * 2u;
     } else {
       const int kr = (wave * B_INSTR + q) * RPIB + lane / CPRB;
-      b_row[q] = B + min(n0 + ((lane % CPRB) ^ kn16_swizzle<BN>(kr)) * 8, ldb - 8);
       b_k8[q] = kr;
+      b_lane[q] = ((unsigned)kr * ldb + min(n0 + ((lane % CPRB) ^ kn16_swizzle<BN>(kr)) * 8, ldb - 8)) * 2u;
     }
   }
-  const int last_k8 = p.K - 8;
   const int P = (p.K + 31) / 32;       // phases
   const int TA = (p.K + 63) / 64;      // A tiles
+  const unsigned a_step = (TRANS_A ? 64u * lda : 64u) * 2u, b_step = (TRANS_B ? 32u : 32u * ldb) * 2u;   // bytes per tile
 
-  // half h (instructions h * A_INSTR / 2 ...) of A tile t; past the end: the last tile again, into a stage nobody reads
-  auto issue_a = [&](int t, auto half) {
-    constexpr int h = decltype(half)::value;   // (compile-time: a_ptr stays in registers)
-    const int k0 = min(t, TA - 1) * 64;
-    const unsigned base = lds0 + (t % SA) * A_STAGE + wave * (A_INSTR * 1024);
+  // half h (instructions h * A_INSTR / 2 ...) of A tile t into stage `base`; past the end: the last tile again, into a
+  // stage nobody reads.  (A chunk past a row's end is the next row's, or nothing: zero_tail.)
+  auto issue_a = [&](int t, unsigned base, auto half) {
+    constexpr int h = decltype(half)::value;
+    const unsigned at = (unsigned)min(t, TA - 1) * a_step;
 #pragma unroll
-    for (int q = h * (A_INSTR / 2); q < (h + 1) * (A_INSTR / 2); ++q) {
-      if constexpr (TRANS_A) {
-        lds_dma16(a_ptr[q] + (size_t)min(k0 + a_k8[q], p.K - 1) * lda, __builtin_amdgcn_readfirstlane(base + q * 1024));
-      } else {
-        const int over = max(k0 + a_k8[q] - last_k8, 0);   // a chunk past the last one of the row: that one instead
-        lds_dma16(a_ptr[q] + (k0 - over), __builtin_amdgcn_readfirstlane(base + q * 1024));
-      }
-    }
+    for (int q = h * (A_INSTR / 2); q < (h + 1) * (A_INSTR / 2); ++q)
+      lds_dma16(a_buf, a_lane[q], at, __builtin_amdgcn_readfirstlane(lds0 + base + (wave * A_INSTR + q) * 1024));
   };
   auto issue_b = [&](int t) {
-    const int k0 = min(t, P - 1) * 32;
-    const unsigned base = lds0 + B_BASE + (t % SB) * B_STAGE + wave * (B_INSTR * 1024);
+    const unsigned at = (unsigned)min(t, P - 1) * b_step, base = B_BASE + (t % SB) * B_STAGE;
 #pragma unroll
-    for (int q = 0; q < B_INSTR; ++q) {
-      if constexpr (TRANS_B)
-        lds_dma16(b_row[q] + min(k0 + b_k8[q], last_k8), __builtin_amdgcn_readfirstlane(base + q * 1024));
-      else
-        lds_dma16(b_row[q] + (size_t)min(k0 + b_k8[q], last_kb) * ldb, __builtin_amdgcn_readfirstlane(base + q * 1024));
-    }
+    for (int q = 0; q < B_INSTR; ++q) lds_dma16(b_buf, b_lane[q], at, __builtin_amdgcn_readfirstlane(lds0 + base + (wave * B_INSTR + q) * 1024));
   };
-  // entries at k >= K must be zero: clamped addresses delivered copies of real data.  Phase ph is the last one.
+  // entries at k >= K must be zero: what was loaded there is other data.  Phase ph is the last one.
   auto zero_tail = [&](int ph) {
     const u32x4 zero = {0u, 0u, 0u, 0u};
     const int ta = ph / 2;
@@ -171,10 +164,11 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   u32x4 fa[2 * WM], fb[2 * WN];  // the operand fragments of one phase
   const std::integral_constant<int, 0> even;
   const std::integral_constant<int, 1> odd;
-  // parity = ph % 2 at compile time: which half of the A tile
+  // parity = ph % 2 at compile time: which half of the A tile.  a_rd, a_wr: the stages of A tiles ph / 2 and ph / 2 + 2
+  unsigned a_rd = 0, a_wr = 2 * A_STAGE;
   auto mem_phase = [&](int ph, auto parity) {
     constexpr int h = decltype(parity)::value;
-    const unsigned char* sa = smem + ((ph >> 1) % SA) * A_STAGE;
+    const unsigned char* sa = smem + a_rd;
     const unsigned char* sb = smem + (ph % SB) * B_STAGE;
 #pragma unroll
     for (int i = 0; i < 2 * WM; ++i) {
@@ -186,16 +180,18 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
       if constexpr (TRANS_B) fb[j] = *reinterpret_cast<const u32x4*>(sb + b_off[0] + j * 16 * 64);
       else fb[j] = kn_fragment<BN * 2>(sb + b_off[j]);
     }
-    issue_a((ph >> 1) + 2, parity);
+    issue_a((ph >> 1) + 2, a_wr, parity);
     issue_b(ph + 3);
+    if constexpr (h) {
+      a_rd = a_rd == 2 * A_STAGE ? 0 : a_rd + A_STAGE;
+      a_wr = a_wr == 2 * A_STAGE ? 0 : a_wr + A_STAGE;
+    }
   };
   auto compute_phase = [&]() {
-    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int i = 0; i < 2 * WM; ++i)
 #pragma unroll
       for (int j = 0; j < 2 * WN; ++j) acc.v[i][j] = mfma_16x16x32<BF16>(fb[j], fa[i], acc.v[i][j]);
-    __builtin_amdgcn_s_setprio(0);
   };
   // at the end of phase ph: my loads of what phase ph + 1 reads have landed (two phases' worth may still fly)
   const bool tail = (p.K % 32) != 0;
@@ -210,10 +206,10 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   };
 
   // prologue = the loads that phases -4 .. -1 would have issued
-  issue_a(0, even);
-  issue_a(0, odd); issue_b(0);
-  issue_a(1, even); issue_b(1);
-  issue_a(1, odd); issue_b(2);
+  issue_a(0, 0, even);
+  issue_a(0, 0, odd); issue_b(0);
+  issue_a(1, A_STAGE, even); issue_b(1);
+  issue_a(1, A_STAGE, odd); issue_b(2);
   wait_vmcnt<2 * LPP>();  // A tile 0 and B tile 0 have landed
   if (tail && P == 1) zero_tail(0);
   __syncthreads();
