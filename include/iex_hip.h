@@ -393,6 +393,7 @@ int iex_csr_softmax(int dtype, int m, int nonzeros, const int* row_indices,
  * 8 = 128x128 and 9 = 64x128 by eight waves with K steps of 64 (few tiles, long K), 10 = 128x256 by eight waves
  * (11: with K steps of 64), 12 = 256x256 with K split over two workgroups per tile (iex_gemm_ws only), 13 = 256x256 by
  * eight waves in two groups that take turns: one reads operand fragments and issues loads while the other multiplies,
+ * 15 = 128x256 by eight waves like 13, in phases of 64 k,
  * 14 = 64x128 by eight waves with K split over two to eight workgroups per tile (iex_gemm_ws only),
  * all with the operands loaded from global memory straight into LDS (0 = choose picks among 5, 8, 9, 10 and 13, and
  * 14 where iex_gemm_ws got the room iex_gemm_workspace_bytes asks for);

@@ -73,23 +73,23 @@ int launch_dma(GemmParams p, int batch, hipStream_t stream) {
 }
 
 // Eight wavefronts in two groups that alternate between reading / loading and multiplying (gemm_pp_device.cuh).
-template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN>
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN, int KP>
 __global__ __launch_bounds__(WCN * 128, 1) void gemm_pp_kernel(GemmParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   int tile_m, tile_n;
   if (!xcd_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;  // uniform per block
-  gemm_tile_pp<BF16, TRANS_B, WM, WN, WCN, TRANS_A>(p, tile_m, tile_n, blockIdx.y, smem);
+  gemm_tile_pp<BF16, TRANS_B, WM, WN, WCN, TRANS_A, KP>(p, tile_m, tile_n, blockIdx.y, smem);
 }
 
-template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN>
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN, int KP = 32>
 int launch_pp(GemmParams p, int batch, hipStream_t stream) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32;
   p.tiles_m = ceil_div(p.M, BM);
   p.tiles_n = ceil_div(p.N, BN);
   const int total = p.tiles_m * p.tiles_n;
   const int per_xcd = (total + kXcds - 1) / kXcds;
-  constexpr int lds = gemm_pp_lds_bytes<BF16, TRANS_B, WM, WN, WCN>();
-  auto kern = gemm_pp_kernel<BF16, TRANS_A, TRANS_B, WM, WN, WCN>;
+  constexpr int lds = gemm_pp_lds_bytes<WM, WN, WCN, KP>();
+  auto kern = gemm_pp_kernel<BF16, TRANS_A, TRANS_B, WM, WN, WCN, KP>;
   static thread_local bool raised = false;  // per instantiation
   if (!raised) {
     if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds),
@@ -277,6 +277,7 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
   if (force == 8) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 1, 64, 4, 4>(p, batch, stream);
   if (force == 9) return launch_dma<BF16, TRANS_A, TRANS_B, 1, 1, 64, 4, 4>(p, batch, stream);
   if (force == 10) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4, 4>(p, batch, stream);
+  if (force == 15) return launch_pp<BF16, TRANS_A, TRANS_B, 2, 2, 4, 64>(p, batch, stream);
   if (force == 13) return launch_pp<BF16, TRANS_A, TRANS_B, 4, 2, 4>(p, batch, stream);
   // Default: operands straight from global memory into LDS (gemm_dma_device.cuh).  The larger the
   // tile of a wave, the fewer LDS bytes each MFMA needs, and LDS time is what the main loop runs
@@ -291,20 +292,22 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
   if (small_tiles > 256) {
     // More 128 x 128 tiles than CUs: the tile shape that finishes first, counting whole rounds of workgroups (a
     // workgroup of the last round takes as long as any other) at the rate each shape reaches with every CU busy.
-    // TFLOP/s measured (bf16): 256 x 256 (one workgroup per CU, eight waves in two alternating groups) 1450; 128 x 256 by
-    // eight waves (64 x 64 each, two per SIMD that cover for each other at the barrier and the waits of every K step; one
-    // workgroup per CU) 1110; 128 x 128 (two workgroups per CU) 1050.
-    //   4096 x 2048 x 4096: 947 / 1056 / 932      4096 x 8192 x 4096: 1459 / 1079 / 1009      8192^3: 1490 / 1125 / 1067
+    // TFLOP/s measured (8192^3, bf16, B as (K, N) / B as (N, K) / A as (K, M)): 256 x 256 by eight waves in two alternating
+    // groups 1460 / 1490 / 1385; 128 x 256 by the same in phases of 64 k (64 x 64 per wave) 1214 / 1334 / 1147, where eight waves
+    // in phase reach 1151 / 1078 / 1135; 128 x 128 by four waves, two workgroups per CU, 1080 / 959 / 1190.
+    //   4096 x 2048 x 4096: 829 / 858 / 729, 1115 / 1208 / 999 (in phase 1011 / 889 / 979), 950 / 806 / 1082
+    // (128 x 128 and 64 x 128 in alternating phases: no faster than codes 8 and 9.)
     // A last round with a share f of the CUs at work takes 0.65 + 0.35 f of a full one: those that work have the way from L2
     // and the power to themselves (11008 x 2048 x 4096, 1.34 rounds of 256 x 256: 175 against 195 for 2.69 of 128 x 256).
-    // A as (K, M): 128 x 128 tiles lose less (8192^3 1372 / 1118 / 1172).
     auto cost = [&](int bm, int bn, int slots, double rate) {
       const long long tiles = (long long)ceil_div(p.M, bm) * ceil_div(p.N, bn) * batch, full = tiles / slots, rest = tiles % slots;
       return ((double)full + (rest ? 0.65 + 0.35 * rest / slots : 0.0)) * slots * bm * bn / rate;
     };
-    const double huge = cost(256, 256, 256, TRANS_A ? 1400.0 : 1450.0), wide = cost(128, 256, 256, 1110.0), small = cost(128, 128, 512, TRANS_A ? 1170.0 : 1050.0);
+    const double huge = cost(256, 256, 256, TRANS_A ? 1385.0 : TRANS_B ? 1490.0 : 1460.0);
+    const double wide = cost(128, 256, 256, TRANS_A ? 1147.0 : TRANS_B ? 1334.0 : 1180.0);
+    const double small = cost(128, 128, 512, TRANS_A ? 1190.0 : TRANS_B ? 959.0 : 1080.0);
     if (huge <= wide && huge <= small) return launch_pp<BF16, TRANS_A, TRANS_B, 4, 2, 4>(p, batch, stream);
-    if (wide <= small) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4, 4>(p, batch, stream);
+    if (wide <= small) return launch_pp<BF16, TRANS_A, TRANS_B, 2, 2, 4, 64>(p, batch, stream);
     return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
   }
   // One round of at most one 128 x 128 tile per CU and a long K: eight waves (64 x 32 each) and K steps of 64
@@ -329,13 +332,13 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
 }  // namespace
 }  // namespace iex
 
-// code: bit 0 = B is (N, K), bit 1 = A is (K, M); bits 4..7 force the kernel for tuning (A as (K, M): 5, 8, 9, 10, 13, 14).  Register-staged operands:
+// code: bit 0 = B is (N, K), bit 1 = A is (K, M); bits 4..7 force the kernel for tuning (A as (K, M): 5, 8, 9, 10, 13, 14, 15).  Register-staged operands:
 // 1 = 128x128 tiles, 2 = 128x256, 3 = 256x256, 4 = 128x128 with K steps of 64.  Operands loaded
 // straight into LDS: 5 = 128x128, 6 = 128x256, 7 = 256x256, 8 = 128x128, 9 = 64x128 by eight waves with K steps of 64,
 // 10 = 128x256 by eight waves, 11 = the same with K steps of 64, 12 = 256x256 with K split over two workgroups per tile
 // (iex_gemm_ws only; never chosen), 13 = 256x256 by eight waves in two groups that alternate between loading and
-// multiplying, 14 = 64x128 by eight waves with K split over two to eight workgroups per tile (iex_gemm_ws only).
-// 0 = choose (one of 5, 8, 9, 10, 13, and 14 where iex_gemm_workspace_bytes asked for room and got it).
+// multiplying, 14 = 64x128 by eight waves with K split over two to eight workgroups per tile (iex_gemm_ws only), 15 = 128x256 like 13 in
+// phases of 64 k.  0 = choose (one of 5, 8, 9, 13, 15, and 14 where iex_gemm_workspace_bytes asked for room and got it).
 extern "C" int iex_gemm_ws(int dtype, int code, int M, int N, int K, const void* A, const void* B, void* C, int batch,
                            long long stride_a, long long stride_b, long long stride_c, void* stream, void* workspace, size_t workspace_bytes) {
   iex::trail_reset();

@@ -37,26 +37,32 @@ namespace iex {
 // 160 KB for 256 x 256 tiles.  Phase p reads the half p % 2 of A tile p / 2 and B tile p, and issues half of the loads
 // of A tile p / 2 + 2 and all loads of B tile p + 3; every wavefront issues the same number of loads LPP in every
 // phase, so "my loads of everything that phase p + 1 reads have landed" is vmcnt(2 * LPP) at the end of phase p.
-template <bool BF16, bool TRANS_B, int WM, int WN, int WCN>
-constexpr int gemm_pp_lds_bytes() { return 3 * (2 * WM * 32) * 128 + 4 * (WCN * WN * 32) * 64; }
+// KP = 64: phases of 64 k, three stages of A and B tiles of 64 k, tile p + 2 loaded in phase p (one phase's loads may fly at
+// its end).  For 128 x 256 tiles: half the rows leave a phase of 32 k too short for what a memory phase has to wait for.
+template <int WM, int WN, int WCN, int KP>
+constexpr int gemm_pp_lds_bytes() { return 3 * (2 * WM * 32) * 128 + (KP == 32 ? 4 * 64 : 3 * 128) * (WCN * WN * 32); }
 
-template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, bool TRANS_A = false>
+template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, bool TRANS_A = false, int KP = 32>
 __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, int tile_n, int z, unsigned char* smem) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32, WAVES = 2 * WCN;
-  constexpr int SA = 3, SB = 4;                       // stages of A (64 k each) and of B (32 k each)
-  constexpr int A_STAGE = BM * 128, B_STAGE = BN * 64;
+  constexpr int SA = 3, SB = KP == 32 ? 4 : 3;        // stages of A (64 k each) and of B (KP each)
+  constexpr int A_STAGE = BM * 128, B_STAGE = BN * KP * 2;
   constexpr int B_BASE = SA * A_STAGE;
+  constexpr int HALVES = 64 / KP, SUB = KP / 32;      // phases per A tile, MFMA sub-steps per phase
   constexpr int A_INSTR = A_STAGE / 1024 / WAVES;     // direct loads per wavefront and A tile
   constexpr int B_INSTR = B_STAGE / 1024 / WAVES;     // ... and B tile
-  constexpr int LPP = A_INSTR / 2 + B_INSTR;          // loads per wavefront and phase
+  constexpr int LPP = A_INSTR / HALVES + B_INSTR;     // loads per wavefront and phase
+  constexpr int FLY = (KP == 32 ? 2 : 1) * LPP;       // ... that may be in flight where one phase ends
   constexpr int CPRB = BN / 8, CPRA = BM / 8;         // (K,N), (K,M) layout: chunks per k row
   constexpr int RPIB = 64 / (CPRB < 64 ? CPRB : 64), RPIA = 64 / (CPRA < 64 ? CPRA : 64);  // ... k rows per instruction
+  constexpr int CPKB = KP / 8;                        // (N,K) layout: chunks per row
   static_assert(WAVES == 8, "two wavefronts per SIMD");
-  static_assert(A_INSTR >= 2 && A_INSTR % 2 == 0 && B_INSTR >= 1 && A_STAGE % (1024 * WAVES) == 0 && B_STAGE % (1024 * WAVES) == 0,
-                "every wavefront fetches whole kilobytes of A (in two halves) and of B");
+  static_assert(KP == 32 || KP == 64, "k per phase");
+  static_assert(A_INSTR >= HALVES && A_INSTR % HALVES == 0 && B_INSTR >= 1 && A_STAGE % (1024 * WAVES) == 0 && B_STAGE % (1024 * WAVES) == 0,
+                "every wavefront fetches whole kilobytes of A (in HALVES parts) and of B");
   static_assert(TRANS_B || (CPRB >= 16 && CPRB <= 64), "(K,N) layout: 128 <= BN <= 512");
   static_assert(!TRANS_A || (CPRA >= 16 && CPRA <= 64), "(K,M) layout: 128 <= BM <= 512");
-  static_assert(3 * LPP < 64, "loads in flight must fit the load counter");
+  static_assert(FLY + LPP < 64, "loads in flight must fit the load counter");
   typedef unsigned short u16;
   typedef __attribute__((address_space(3))) unsigned char lds_u8;
 
@@ -74,7 +80,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   const int last_kb = (p.kb ? p.kb : p.K) - 1;   // the last k row of a (K,N) B
 
   // ---- what this lane fetches.  A: 8 rows of 128 bytes per instruction, LDS position (row, c) holds global chunk
-  // c ^ ((row >> 1) & 7).  B as (N,K): 16 rows of 64 bytes, chunk c ^ ((row >> 2) & 3).  B as (K,N): k rows of BN
+  // c ^ ((row >> 1) & 7).  B as (N,K): the same, or 16 rows of 64 bytes, chunk c ^ ((row >> 2) & 3).  B as (K,N): k rows of BN
   // elements, chunk c ^ kn16_swizzle(k), and A as (K,M) likewise, 64 k rows of BM elements per stage.
   // Rows past M (columns past N) are the last one's: they feed rows (columns) of C that are not stored.
   const u32x4 a_buf = TRANS_A ? buffer_of(A, (size_t)p.K * lda * 2) : buffer_of(A + (size_t)m0 * lda, (size_t)(p.M - m0) * lda * 2);
@@ -98,8 +104,8 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
 #pragma unroll
   for (int q = 0; q < B_INSTR; ++q) {
     if constexpr (TRANS_B) {
-      const int row = (wave * B_INSTR + q) * 16 + lane / 4;
-      b_k8[q] = ((lane % 4) ^ ((row >> 2) & 3)) * 8;
+      const int row = (wave * B_INSTR + q) * (64 / CPKB) + lane / CPKB;
+      b_k8[q] = ((lane % CPKB) ^ (KP == 32 ? (row >> 2) & 3 : (row >> 1) & 7)) * 8;
       b_lane[q] = ((unsigned)min(row, p.N - 1 - n0) * ldb + b_k8[q]) * 2u;
     } else {
       const int kr = (wave * B_INSTR + q) * RPIB + lane / CPRB;
@@ -107,28 +113,28 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
       b_lane[q] = ((unsigned)kr * ldb + min(n0 + ((lane % CPRB) ^ kn16_swizzle<BN>(kr)) * 8, ldb - 8)) * 2u;
     }
   }
-  const int P = (p.K + 31) / 32;       // phases
+  const int P = (p.K + KP - 1) / KP;   // phases
   const int TA = (p.K + 63) / 64;      // A tiles
-  const unsigned a_step = (TRANS_A ? 64u * lda : 64u) * 2u, b_step = (TRANS_B ? 32u : 32u * ldb) * 2u;   // bytes per tile
+  const unsigned a_step = (TRANS_A ? 64u * lda : 64u) * 2u, b_step = (TRANS_B ? (unsigned)KP : (unsigned)KP * ldb) * 2u;   // bytes per tile
 
-  // half h (instructions h * A_INSTR / 2 ...) of A tile t into stage `base`; past the end: the last tile again, into a
+  // part h (instructions h * A_INSTR / HALVES ...) of A tile t into stage `base`; past the end: the last tile again, into a
   // stage nobody reads.  (A chunk past a row's end is the next row's, or nothing: zero_tail.)
   auto issue_a = [&](int t, unsigned base, auto half) {
     constexpr int h = decltype(half)::value;
     const unsigned at = (unsigned)min(t, TA - 1) * a_step;
 #pragma unroll
-    for (int q = h * (A_INSTR / 2); q < (h + 1) * (A_INSTR / 2); ++q)
+    for (int q = h * (A_INSTR / HALVES); q < (h + 1) * (A_INSTR / HALVES); ++q)
       lds_dma16(a_buf, a_lane[q], at, __builtin_amdgcn_readfirstlane(lds0 + base + (wave * A_INSTR + q) * 1024));
   };
-  auto issue_b = [&](int t) {
-    const unsigned at = (unsigned)min(t, P - 1) * b_step, base = B_BASE + (t % SB) * B_STAGE;
+  auto issue_b = [&](int t, unsigned stage) {
+    const unsigned at = (unsigned)min(t, P - 1) * b_step, base = B_BASE + stage;
 #pragma unroll
     for (int q = 0; q < B_INSTR; ++q) lds_dma16(b_buf, b_lane[q], at, __builtin_amdgcn_readfirstlane(lds0 + base + (wave * B_INSTR + q) * 1024));
   };
   // entries at k >= K must be zero: what was loaded there is other data.  Phase ph is the last one.
   auto zero_tail = [&](int ph) {
     const u32x4 zero = {0u, 0u, 0u, 0u};
-    const int ta = ph / 2;
+    const int ta = ph / HALVES;
     unsigned char* sa = smem + (ta % SA) * A_STAGE;
 #pragma unroll
     for (int q = 0; q < A_INSTR; ++q)
@@ -136,7 +142,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
     unsigned char* sb = smem + B_BASE + (ph % SB) * B_STAGE;
 #pragma unroll
     for (int q = 0; q < B_INSTR; ++q)
-      if (ph * 32 + b_k8[q] >= p.K) *reinterpret_cast<u32x4*>(sb + ((wave * B_INSTR + q) * 64 + lane) * 16) = zero;
+      if (ph * KP + b_k8[q] >= p.K) *reinterpret_cast<u32x4*>(sb + ((wave * B_INSTR + q) * 64 + lane) * 16) = zero;
   };
 
   Acc16<WM, WN> acc;
@@ -153,50 +159,60 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
 #pragma unroll
     for (int h = 0; h < 2; ++h) a_off[h] = (wm * WM * 32 + frow) * 128 + (((h * 4 + fch) ^ (frow >> 1)) * 16);
   }
-  int b_off[TRANS_B ? 1 : 2 * WN];
+  int b_off[TRANS_B ? SUB : 2 * WN];
   if constexpr (TRANS_B) {
-    b_off[0] = B_BASE + (wn * WN * 32 + frow) * 64 + ((fch ^ (frow >> 2)) * 16);
+#pragma unroll
+    for (int s = 0; s < SUB; ++s)
+      b_off[s] = B_BASE + (wn * WN * 32 + frow) * (KP * 2) + (((s * 4 + fch) ^ (KP == 32 ? frow >> 2 : frow >> 1)) * 16);
   } else {
 #pragma unroll
     for (int j = 0; j < 2 * WN; ++j) b_off[j] = B_BASE + kn16_fragment_offset<BN>(lane, wn * 2 * WN + j);
   }
 
-  u32x4 fa[2 * WM], fb[2 * WN];  // the operand fragments of one phase
+  u32x4 fa[SUB][2 * WM], fb[SUB][2 * WN];  // the operand fragments of one phase
   const std::integral_constant<int, 0> even;
-  const std::integral_constant<int, 1> odd;
-  // parity = ph % 2 at compile time: which half of the A tile.  a_rd, a_wr: the stages of A tiles ph / 2 and ph / 2 + 2
-  unsigned a_rd = 0, a_wr = 2 * A_STAGE;
+  const std::integral_constant<int, HALVES - 1> odd;
+  // parity = ph % HALVES at compile time: which part of the A tile.  a_rd, a_wr: the stages of A tiles ph / HALVES and two
+  // further; b_rd, b_wr: of B tiles ph and SB - 1 further (the stage before, going round)
+  unsigned a_rd = 0, a_wr = 2 * A_STAGE, b_rd = 0, b_wr = (SB - 1) * B_STAGE;
   auto mem_phase = [&](int ph, auto parity) {
     constexpr int h = decltype(parity)::value;
     const unsigned char* sa = smem + a_rd;
-    const unsigned char* sb = smem + (ph % SB) * B_STAGE;
+    const unsigned char* sb = smem + b_rd;
 #pragma unroll
-    for (int i = 0; i < 2 * WM; ++i) {
-      if constexpr (TRANS_A) fa[i] = kn_fragment<BM * 2>(sa + a_off[i] + h * 32 * (BM * 2));
-      else fa[i] = *reinterpret_cast<const u32x4*>(sa + a_off[h] + i * 16 * 128);
-    }
+    for (int s = 0; s < SUB; ++s) {
 #pragma unroll
-    for (int j = 0; j < 2 * WN; ++j) {
-      if constexpr (TRANS_B) fb[j] = *reinterpret_cast<const u32x4*>(sb + b_off[0] + j * 16 * 64);
-      else fb[j] = kn_fragment<BN * 2>(sb + b_off[j]);
+      for (int i = 0; i < 2 * WM; ++i) {
+        if constexpr (TRANS_A) fa[s][i] = kn_fragment<BM * 2>(sa + a_off[i] + (h + s) * 32 * (BM * 2));
+        else fa[s][i] = *reinterpret_cast<const u32x4*>(sa + a_off[h + s] + i * 16 * 128);
+      }
+#pragma unroll
+      for (int j = 0; j < 2 * WN; ++j) {
+        if constexpr (TRANS_B) fb[s][j] = *reinterpret_cast<const u32x4*>(sb + b_off[s] + j * 16 * (KP * 2));
+        else fb[s][j] = kn_fragment<BN * 2>(sb + b_off[j] + s * 32 * (BN * 2));
+      }
     }
-    issue_a((ph >> 1) + 2, a_wr, parity);
-    issue_b(ph + 3);
-    if constexpr (h) {
+    issue_a(ph / HALVES + 2, a_wr, parity);
+    issue_b(ph + SB - 1, b_wr);
+    b_wr = b_rd;
+    b_rd = b_rd == (SB - 1) * B_STAGE ? 0 : b_rd + B_STAGE;
+    if constexpr (h == HALVES - 1) {
+      a_wr = a_rd;
       a_rd = a_rd == 2 * A_STAGE ? 0 : a_rd + A_STAGE;
-      a_wr = a_wr == 2 * A_STAGE ? 0 : a_wr + A_STAGE;
     }
   };
   auto compute_phase = [&]() {
 #pragma unroll
-    for (int i = 0; i < 2 * WM; ++i)
+    for (int s = 0; s < SUB; ++s)
 #pragma unroll
-      for (int j = 0; j < 2 * WN; ++j) acc.v[i][j] = mfma_16x16x32<BF16>(fb[j], fa[i], acc.v[i][j]);
+      for (int i = 0; i < 2 * WM; ++i)
+#pragma unroll
+        for (int j = 0; j < 2 * WN; ++j) acc.v[i][j] = mfma_16x16x32<BF16>(fb[s][j], fa[s][i], acc.v[i][j]);
   };
-  // at the end of phase ph: my loads of what phase ph + 1 reads have landed (two phases' worth may still fly)
-  const bool tail = (p.K % 32) != 0;
+  // at the end of phase ph: my loads of what phase ph + 1 reads have landed
+  const bool tail = (p.K % KP) != 0;
   auto landed = [&](int ph) {
-    wait_vmcnt<2 * LPP>();
+    wait_vmcnt<FLY>();
     if (tail && ph + 2 == P) zero_tail(ph + 1);
   };
   auto interval_end = [&]() {
@@ -205,12 +221,17 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // prologue = the loads that phases -4 .. -1 would have issued
-  issue_a(0, 0, even);
-  issue_a(0, 0, odd); issue_b(0);
-  issue_a(1, A_STAGE, even); issue_b(1);
-  issue_a(1, A_STAGE, odd); issue_b(2);
-  wait_vmcnt<2 * LPP>();  // A tile 0 and B tile 0 have landed
+  // prologue = the loads that the phases before phase 0 would have issued
+  if constexpr (KP == 32) {
+    issue_a(0, 0, even);
+    issue_a(0, 0, odd); issue_b(0, 0);
+    issue_a(1, A_STAGE, even); issue_b(1, B_STAGE);
+    issue_a(1, A_STAGE, odd); issue_b(2, 2 * B_STAGE);
+  } else {
+    issue_a(0, 0, even); issue_b(0, 0);
+    issue_a(1, A_STAGE, even); issue_b(1, B_STAGE);
+  }
+  wait_vmcnt<FLY>();  // what phase 0 reads has landed
   if (tail && P == 1) zero_tail(0);
   __syncthreads();
 
