@@ -389,13 +389,13 @@ int iex_csr_softmax(int dtype, int m, int nonzeros, const int* row_indices,
  * (N,K), the torch.nn.Linear weight layout used by MyLinear, layers_and_funcs/torch.py:17).
  * dtype is IEX_F16 or IEX_BF16 for A, B and C; accumulation is fp32 on the matrix cores.
  * stride_* are element strides between batch entries (0 = operand shared by the batch).
- * Bits 4..7 of trans_b force the kernel for tuning: 5 = 128x128, 6 = 128x256, 7 = 256x256 tiles,
+ * Bits 4..8 of trans_b force the kernel for tuning: 5 = 128x128, 6 = 128x256, 7 = 256x256 tiles,
  * 8 = 128x128 and 9 = 64x128 by eight waves with K steps of 64 (few tiles, long K), 10 = 128x256 by eight waves
  * (11: with K steps of 64), 12 = 256x256 with K split over two workgroups per tile (iex_gemm_ws only), 13 = 256x256 by
  * eight waves in two groups that take turns: one reads operand fragments and issues loads while the other multiplies,
- * 15 = 128x256 by eight waves like 13, in phases of 64 k,
+ * 15 = 128x256 by eight waves like 13, in phases of 64 k, 16 = 192x256 like 13 (not with A as (K,M)),
  * 14 = 64x128 by eight waves with K split over two to eight workgroups per tile (iex_gemm_ws only),
- * all with the operands loaded from global memory straight into LDS (0 = choose picks among 5, 8, 9, 10 and 13, and
+ * all with the operands loaded from global memory straight into LDS (0 = choose picks among 5, 8, 9, 13, 15 and 16, and
  * 14 where iex_gemm_ws got the room iex_gemm_workspace_bytes asks for);
  * 1 = 128x128, 2 = 128x256, 3 = 256x256, 4 = 128x128 with K steps of 64, operands staged through
  * registers.  K % 8 == 0, N % 8 == 0 for a (K,N) B, 16-byte aligned operands.

@@ -250,7 +250,7 @@ inline bool auto_split_wanted(int M, int N, int K, int batch) {
 
 template <bool BF16, bool TRANS_A, bool TRANS_B>
 int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, void* ws, size_t ws_bytes, bool flags_are_zero) {
-  if constexpr (!TRANS_A) {   // kernels that are never chosen
+  if constexpr (!TRANS_A) {   // kernels that are never chosen, or not for A as (K, M)
     if (force == 12) {
       IEX_REQUIRE(p.K >= 64, IEX_ERR_UNSUPPORTED, "gemm: the K-split kernel needs two K steps (K >= 64; K=%d)", p.K);
       IEX_REQUIRE(ws && aligned(ws, 256) && ws_bytes >= gemm_splitk_bytes(p.M, p.N, batch, 256, 256), IEX_ERR_BAD_ARGUMENT,
@@ -263,6 +263,7 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
     if (force == 4) return launch<BF16, TRANS_B, 2, 2, 64>(p, batch, stream);
     if (force == 6) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 4, 32, 4>(p, batch, stream);
     if (force == 7) return launch_dma<BF16, TRANS_A, TRANS_B, 4, 4, 32, 4>(p, batch, stream);
+    if (force == 16) return launch_pp<BF16, TRANS_A, TRANS_B, 3, 2, 4>(p, batch, stream);
     if (force == 11) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 64, 3, 4>(p, batch, stream);
   }
   if (force == 14) {
@@ -296,6 +297,8 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
     // groups 1460 / 1490 / 1385; 128 x 256 by the same in phases of 64 k (64 x 64 per wave) 1214 / 1334 / 1147, where eight waves
     // in phase reach 1151 / 1078 / 1135; 128 x 128 by four waves, two workgroups per CU, 1080 / 959 / 1190.
     //   4096 x 2048 x 4096: 829 / 858 / 729, 1115 / 1208 / 999 (in phase 1011 / 889 / 979), 950 / 806 / 1082
+    // 192 x 256 as 256 x 256 (not with A as (K, M)) 1303 / 1295: between the two where whole rounds are few, 11008 x 2048 x 4096
+    // 172 / 155 / 176 us for 256 / 192 / 128 rows, 9000 x 2048 x 4096 166 / 147 / 168, 5528 x 1600 x 2224 50 / 45 / 64.
     // (128 x 128 and 64 x 128 in alternating phases: no faster than codes 8 and 9.)
     // A last round with a share f of the CUs at work takes 0.65 + 0.35 f of a full one: those that work have the way from L2
     // and the power to themselves (11008 x 2048 x 4096, 1.34 rounds of 256 x 256: 175 against 195 for 2.69 of 128 x 256).
@@ -306,6 +309,9 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
     const double huge = cost(256, 256, 256, TRANS_A ? 1385.0 : TRANS_B ? 1490.0 : 1460.0);
     const double wide = cost(128, 256, 256, TRANS_A ? 1147.0 : TRANS_B ? 1334.0 : 1180.0);
     const double small = cost(128, 128, 512, TRANS_A ? 1190.0 : TRANS_B ? 959.0 : 1080.0);
+    if constexpr (!TRANS_A) {
+      if (cost(192, 256, 256, 1300.0) <= std::min({huge, wide, small})) return launch_pp<BF16, TRANS_A, TRANS_B, 3, 2, 4>(p, batch, stream);
+    }
     if (huge <= wide && huge <= small) return launch_pp<BF16, TRANS_A, TRANS_B, 4, 2, 4>(p, batch, stream);
     if (wide <= small) return launch_pp<BF16, TRANS_A, TRANS_B, 2, 2, 4, 64>(p, batch, stream);
     return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
@@ -332,13 +338,13 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
 }  // namespace
 }  // namespace iex
 
-// code: bit 0 = B is (N, K), bit 1 = A is (K, M); bits 4..7 force the kernel for tuning (A as (K, M): 5, 8, 9, 10, 13, 14, 15).  Register-staged operands:
+// code: bit 0 = B is (N, K), bit 1 = A is (K, M); bits 4..8 force the kernel for tuning (A as (K, M): 5, 8, 9, 10, 13, 14, 15).  Register-staged operands:
 // 1 = 128x128 tiles, 2 = 128x256, 3 = 256x256, 4 = 128x128 with K steps of 64.  Operands loaded
 // straight into LDS: 5 = 128x128, 6 = 128x256, 7 = 256x256, 8 = 128x128, 9 = 64x128 by eight waves with K steps of 64,
 // 10 = 128x256 by eight waves, 11 = the same with K steps of 64, 12 = 256x256 with K split over two workgroups per tile
 // (iex_gemm_ws only; never chosen), 13 = 256x256 by eight waves in two groups that alternate between loading and
 // multiplying, 14 = 64x128 by eight waves with K split over two to eight workgroups per tile (iex_gemm_ws only), 15 = 128x256 like 13 in
-// phases of 64 k.  0 = choose (one of 5, 8, 9, 13, 15, and 14 where iex_gemm_workspace_bytes asked for room and got it).
+// phases of 64 k, 16 = 192x256 like 13.  0 = choose (one of 5, 8, 9, 13, 15, 16, and 14 where iex_gemm_workspace_bytes asked for room and got it).
 extern "C" int iex_gemm_ws(int dtype, int code, int M, int N, int K, const void* A, const void* B, void* C, int batch,
                            long long stride_a, long long stride_b, long long stride_c, void* stream, void* workspace, size_t workspace_bytes) {
   iex::trail_reset();
@@ -353,7 +359,7 @@ extern "C" int iex_gemm(int dtype, int code, int M, int N, int K, const void* A,
 
 extern "C" size_t iex_gemm_workspace_bytes(int dtype, int code, int M, int N, int K, int batch) {
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0 || (dtype != IEX_F16 && dtype != IEX_BF16)) return 0;
-  const int force = (code >> 4) & 0xf;
+  const int force = (code >> 4) & 0x1f;
   if (force == 12) return iex::gemm_splitk_bytes(M, N, batch, 256, 256);
   if (force == 14) return iex::gemm_parts_bytes(M, N, batch, 64, 128, 8);
   return force == 0 ? iex::gemm_auto_split_bytes(M, N, K, batch) : 0;
@@ -376,7 +382,7 @@ void iex::gemm_auto_split_flags(int M, int N, int K, int batch, size_t* offset_b
 int iex::gemm_dispatch(int dtype, int code, const GemmParams& given, int batch, hipStream_t stream, void* workspace, size_t workspace_bytes,
                        bool workspace_flags_are_zero) {
   GemmParams p = given;
-  const int trans_b = code & 1, trans_a = (code >> 1) & 1, force = (code >> 4) & 0xf;
+  const int trans_b = code & 1, trans_a = (code >> 1) & 1, force = (code >> 4) & 0x1f;
   IEX_REQUIRE(p.M >= 0 && p.N >= 0 && p.K >= 0 && batch >= 0, IEX_ERR_BAD_ARGUMENT, "gemm: negative dimension");
   if (p.M == 0 || p.N == 0 || batch == 0) return 0;
   IEX_REQUIRE(p.A && p.B && p.C, IEX_ERR_BAD_ARGUMENT, "gemm: null pointer argument");

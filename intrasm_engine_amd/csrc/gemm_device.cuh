@@ -52,7 +52,7 @@ struct GemmParams {
 
 constexpr int kGemmAdd = 1, kGemmTimesSilu = 2;
 
-// iex_gemm with the options above (gemm.hip).  code: bit 0 = B is (N,K), bit 1 = A is (K,M), bits 4..7 = forced kernel.
+// iex_gemm with the options above (gemm.hip).  code: bit 0 = B is (N,K), bit 1 = A is (K,M), bits 4..8 = forced kernel.
 int gemm_dispatch(int dtype, int code, const GemmParams& p, int batch, hipStream_t stream, void* workspace = nullptr, size_t workspace_bytes = 0,
                   bool workspace_flags_are_zero = false);
 // Bytes of workspace with which gemm_dispatch, left to choose, splits K over two workgroups per tile (0: this shape is

@@ -35,8 +35,8 @@ namespace iex {
 // requested from L2 for 8.6 GB of operands, the texture-data unit busy 83 % of the cycles at 20 bytes per clock).  So A is
 // staged 64 k at a time (whole lines, three stages), B 32 k at a time (four stages): 3 * BM * 128 + 4 * BN * 64 bytes,
 // 160 KB for 256 x 256 tiles.  Phase p reads the half p % 2 of A tile p / 2 and B tile p, and issues half of the loads
-// of A tile p / 2 + 2 and all loads of B tile p + 3; every wavefront issues the same number of loads LPP in every
-// phase, so "my loads of everything that phase p + 1 reads have landed" is vmcnt(2 * LPP) at the end of phase p.
+// of A tile p / 2 + 2 and all loads of B tile p + 3; every wavefront issues the same number of loads in every two
+// phases, so "my loads of everything that phase p + 1 reads have landed" is vmcnt(that number) at the end of phase p.
 // KP = 64: phases of 64 k, three stages of A and B tiles of 64 k, tile p + 2 loaded in phase p (one phase's loads may fly at
 // its end).  For 128 x 256 tiles: half the rows leave a phase of 32 k too short for what a memory phase has to wait for.
 template <int WM, int WN, int WCN, int KP>
@@ -51,18 +51,18 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   constexpr int HALVES = 64 / KP, SUB = KP / 32;      // phases per A tile, MFMA sub-steps per phase
   constexpr int A_INSTR = A_STAGE / 1024 / WAVES;     // direct loads per wavefront and A tile
   constexpr int B_INSTR = B_STAGE / 1024 / WAVES;     // ... and B tile
-  constexpr int LPP = A_INSTR / HALVES + B_INSTR;     // loads per wavefront and phase
-  constexpr int FLY = (KP == 32 ? 2 : 1) * LPP;       // ... that may be in flight where one phase ends
+  // Loads per wavefront that may be in flight where a phase ends: those of two phases (one, for KP = 64).
+  constexpr int FLY = A_INSTR + HALVES * B_INSTR;
   constexpr int CPRB = BN / 8, CPRA = BM / 8;         // (K,N), (K,M) layout: chunks per k row
   constexpr int RPIB = 64 / (CPRB < 64 ? CPRB : 64), RPIA = 64 / (CPRA < 64 ? CPRA : 64);  // ... k rows per instruction
   constexpr int CPKB = KP / 8;                        // (N,K) layout: chunks per row
   static_assert(WAVES == 8, "two wavefronts per SIMD");
   static_assert(KP == 32 || KP == 64, "k per phase");
-  static_assert(A_INSTR >= HALVES && A_INSTR % HALVES == 0 && B_INSTR >= 1 && A_STAGE % (1024 * WAVES) == 0 && B_STAGE % (1024 * WAVES) == 0,
+  static_assert(A_INSTR >= HALVES && B_INSTR >= 1 && A_STAGE % (1024 * WAVES) == 0 && B_STAGE % (1024 * WAVES) == 0,
                 "every wavefront fetches whole kilobytes of A (in HALVES parts) and of B");
   static_assert(TRANS_B || (CPRB >= 16 && CPRB <= 64), "(K,N) layout: 128 <= BN <= 512");
-  static_assert(!TRANS_A || (CPRA >= 16 && CPRA <= 64), "(K,M) layout: 128 <= BM <= 512");
-  static_assert(FLY + LPP < 64, "loads in flight must fit the load counter");
+  static_assert(!TRANS_A || CPRA == 16 || CPRA == 32 || CPRA == 64, "(K,M) layout: BM is 128, 256 or 512");
+  static_assert(FLY + A_INSTR + B_INSTR < 64, "loads in flight must fit the load counter");
   typedef unsigned short u16;
   typedef __attribute__((address_space(3))) unsigned char lds_u8;
 
@@ -117,13 +117,13 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   const int TA = (p.K + 63) / 64;      // A tiles
   const unsigned a_step = (TRANS_A ? 64u * lda : 64u) * 2u, b_step = (TRANS_B ? (unsigned)KP : (unsigned)KP * ldb) * 2u;   // bytes per tile
 
-  // part h (instructions h * A_INSTR / HALVES ...) of A tile t into stage `base`; past the end: the last tile again, into a
+  // part h (of HALVES; of an odd number of instructions the second has one more) of A tile t into stage `base`; past the end: the last tile again, into a
   // stage nobody reads.  (A chunk past a row's end is the next row's, or nothing: zero_tail.)
   auto issue_a = [&](int t, unsigned base, auto half) {
     constexpr int h = decltype(half)::value;
     const unsigned at = (unsigned)min(t, TA - 1) * a_step;
 #pragma unroll
-    for (int q = h * (A_INSTR / HALVES); q < (h + 1) * (A_INSTR / HALVES); ++q)
+    for (int q = h * (A_INSTR / HALVES); q < (h == HALVES - 1 ? A_INSTR : A_INSTR / HALVES); ++q)
       lds_dma16(a_buf, a_lane[q], at, __builtin_amdgcn_readfirstlane(lds0 + base + (wave * A_INSTR + q) * 1024));
   };
   auto issue_b = [&](int t, unsigned stage) {

@@ -10,12 +10,14 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("layout", [0, 1, 2])   # B as (K, N), B as (N, K), A as (K, M)
-@pytest.mark.parametrize("tile", [13, 15])      # 256 x 256 in phases of 32 k, 128 x 256 in phases of 64
+@pytest.mark.parametrize("tile", [13, 15, 16])  # 256 x 256 in phases of 32 k, 128 x 256 in phases of 64, 192 x 256 in phases of 32
 @pytest.mark.parametrize("mnk", [(8, 8, 8), (128, 256, 64), (136, 264, 72), (256, 256, 96), (264, 520, 192), (72, 1000, 1032)])
 def test_layouts_at_the_edges_of_the_stages(oracle, dev, dtype, layout, tile, mnk):
     """One, two, three phases and more, the last one whole or with 8 k; tiles of which one row of chunks exists."""
     from intrasm_engine_amd import _lib
     M, N, K = mnk
+    if tile == 16 and layout == 2:
+        pytest.skip("a (K, M) operand has no rows of 192")
     rng = np.random.default_rng(M + K)
     a_np, b_np = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
     a, b = torch.from_numpy(a_np).to(dev).to(dtype), torch.from_numpy(b_np).to(dev).to(dtype)
