@@ -375,6 +375,17 @@ int iex_attention_fits(int dtype, int head_dim, int length);
 int iex_attention(int dtype, int heads, int head_dim, int seqs, int length, const void* q, const void* k, const void* v, float scale,
                   void* out, void* stream);
 
+/* ---- sparse attention over a CSR mask in one kernel: out = softmax(scale * q k^T at the mask's entries) v, operands
+ * (heads, tokens, head_dim), mask tokens x tokens in canonical CSR (columns ascend inside a row).  iex_mask_tables writes,
+ * from the index arrays alone, what the kernel reads of the mask (256-byte aligned memory of iex_mask_tables_bytes(tokens,
+ * tokens, nonzeros), 0: not served); they serve every call of that dtype on the mask.  A row without entries gives zeros. */
+size_t iex_mask_tables_bytes(int m, int n, int nonzeros);
+int iex_mask_tables(int dtype, int m, int n, int nonzeros, const int* row_offsets, const int* column_indices, void* tables,
+                    size_t bytes, void* stream);
+int iex_sparse_attention_fits(int dtype, int head_dim, int tokens);
+int iex_sparse_attention(int dtype, int heads, int tokens, int head_dim, int nonzeros, const int* row_offsets, const void* q,
+                         const void* k, const void* v, float scale, void* out, const void* tables, size_t bytes, void* stream);
+
 /* In-place row-wise softmax over the stored entries of a CSR matrix:
  * values[z, j] = exp(scale*values[z, j] - max_row) / sum_row.  values is (batch, nnz).
  * The middle step of sparse attention between SDDMM and SpMM (no reference

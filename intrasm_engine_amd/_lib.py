@@ -68,6 +68,10 @@ SIGNATURES = {
     "iex_CudaSddmm2": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "iex_attention_fits": (_i, [_i, _i, _i]),
     "iex_attention": (_i, [_i, _i, _i, _i, _i, _vp, _vp, _vp, _f, _vp, _vp]),
+    "iex_mask_tables_bytes": (_c.c_size_t, [_i, _i, _i]),
+    "iex_mask_tables": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _c.c_size_t, _vp]),
+    "iex_sparse_attention_fits": (_i, [_i, _i, _i]),
+    "iex_sparse_attention": (_i, [_i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _f, _vp, _vp, _c.c_size_t, _vp]),
     "iex_csr_softmax": (_i, [_i, _i, _i, _vp, _vp, _vp, _f, _vp, _i]),
     "iex_gemm": (_i, [_i, _i, _i, _i, _i, _vp, _vp, _vp, _i, _ll, _ll, _ll, _vp]),
     "iex_gemm_ws": (_i, [_i, _i, _i, _i, _i, _vp, _vp, _vp, _i, _ll, _ll, _ll, _vp, _vp, _c.c_size_t]),

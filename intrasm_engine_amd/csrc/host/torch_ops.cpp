@@ -59,7 +59,11 @@ struct Note {
   std::array<int, 16> histogram;
   double dense_share;   // < 0: not known
   Weak tables;          // of the kernels for patterns with structure; may be gone
+  Weak mask_tables[2];  // of sparse attention in one kernel, for 16-bit types and fp32; may be gone
 };
+Weak weak_of(const std::optional<Tensor>& t) {
+  return Weak(t.has_value() ? t->getIntrusivePtr() : c10::intrusive_ptr<c10::TensorImpl, c10::UndefinedTensorImpl>());
+}
 struct Known {   // what a call needs of it
   int status;
   bool has_histogram;
@@ -81,7 +85,7 @@ void set_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k
               const std::optional<double>& dense_share, const std::optional<Tensor>& tables) {
   Note n{Weak(column_indices.getIntrusivePtr()), Weak(row_offsets.getIntrusivePtr()), version_of(column_indices), version_of(row_offsets), k, status,
          histogram.has_value(), {}, dense_share.value_or(-1.0),
-         Weak(tables.has_value() ? tables->getIntrusivePtr() : c10::intrusive_ptr<c10::TensorImpl, c10::UndefinedTensorImpl>())};
+         weak_of(tables), {weak_of({}), weak_of({})}};
   if (histogram) std::copy_n(histogram->begin(), 16, n.histogram.begin());
   std::unique_lock lock(notes_mutex);
   auto& map = notes();
@@ -92,16 +96,38 @@ void set_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k
   map.insert_or_assign(column_indices.unsafeGetTensorImpl(), std::move(n));
 }
 
-std::optional<Known> note_of(const Tensor& row_offsets, const Tensor& column_indices, int64_t k) {
-  std::shared_lock lock(notes_mutex);
-  const auto& map = notes();
+// (with notes_mutex held; null: nothing is known)
+Note* find_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k) {
+  auto& map = notes();
   const auto it = map.find(column_indices.unsafeGetTensorImpl());
-  if (it == map.end()) return {};
-  const Note& n = it->second;
+  if (it == map.end()) return nullptr;
+  Note& n = it->second;
   // (a weak reference that has not expired holds the address: nobody else can have it)
   if (n.k != k || n.columns.expired() || n.offsets.expired() || n.offsets._unsafe_get_target() != row_offsets.unsafeGetTensorImpl() ||
       n.columns_version != version_of(column_indices) || n.offsets_version != version_of(row_offsets))
-    return {};
+    return nullptr;
+  return &n;
+}
+
+void set_mask_tables(const Tensor& row_offsets, const Tensor& column_indices, int64_t k, int which, const Tensor& tables) {
+  std::unique_lock lock(notes_mutex);
+  if (Note* n = find_note(row_offsets, column_indices, k)) n->mask_tables[which] = weak_of(tables);
+}
+
+// of a canonical pattern; undefined where there are none
+Tensor mask_tables_of(const Tensor& row_offsets, const Tensor& column_indices, int64_t k, int which) {
+  std::shared_lock lock(notes_mutex);
+  const Note* n = find_note(row_offsets, column_indices, k);
+  if (!n || n->status != 0) return Tensor();
+  auto alive = n->mask_tables[which].lock();
+  return alive ? Tensor(std::move(alive)) : Tensor();
+}
+
+std::optional<Known> note_of(const Tensor& row_offsets, const Tensor& column_indices, int64_t k) {
+  std::shared_lock lock(notes_mutex);
+  const Note* found = find_note(row_offsets, column_indices, k);
+  if (!found) return {};
+  const Note& n = *found;
   Known known{n.status, n.has_histogram, n.histogram, n.dense_share, Tensor()};
   if (auto alive = n.tables.lock()) known.tables = Tensor(std::move(alive));
   return known;
@@ -329,6 +355,28 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
   return out;
 }
 
+// sparse attention over a mask whose tables exist; None where the kernel does not serve the call
+std::optional<Tensor> sparse_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& row_indices, const Tensor& row_offsets,
+                                       const Tensor& column_indices, double scale) {
+  const int dtype = dtype_code(q.scalar_type());
+  if (forced || dtype < 0 || !plain(q, 3) || !plain(k, 3) || !plain(v, 3) || k.sizes() != q.sizes() || v.sizes() != q.sizes() ||
+      k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() || k.device() != q.device() || v.device() != q.device() || q.size(0) == 0 ||
+      !(scale > 0) || !iex_sparse_attention_fits(dtype, q.size(2), q.size(1)) || !plain_csr(row_indices, row_offsets, column_indices, q, q.size(1)) ||
+      column_indices.scalar_type() != at::kInt)
+    return {};
+  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) return {};
+  for (const Tensor* t : {&q, &k, &v})
+    if (reinterpret_cast<uintptr_t>(t->const_data_ptr()) % 16) return {};
+  const Tensor tables = mask_tables_of(row_offsets, column_indices, q.size(1), dtype == IEX_F32);
+  if (!tables.defined()) return {};
+  const c10::DeviceGuard guard(q.device());
+  Tensor out = at::empty_like(q);
+  check(iex_sparse_attention(dtype, q.size(0), q.size(1), q.size(2), column_indices.size(0), row_offsets.const_data_ptr<int>(), q.const_data_ptr(),
+                             k.const_data_ptr(), v.const_data_ptr(), (float)scale, out.data_ptr(), tables.const_data_ptr(), tables.numel(), stream_of(q)),
+        "sparse attention");
+  return out;
+}
+
 // ---- autograd: the plain calls of MySpMM and MyLinear (no recording, no forced kernels) -----------------------------
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
@@ -451,6 +499,8 @@ PYBIND11_MODULE(_iex_host, module) {
   module.def("set_note", &set_note);
   module.def("spmm_with", &spmm_with);
   module.def("attention", &attention);
+  module.def("sparse_attention", &sparse_attention);
+  module.def("set_mask_tables", &set_mask_tables);
   module.def("trainable_spmm", &trainable_spmm);
   module.def("trainable_linear", &trainable_linear);
 }

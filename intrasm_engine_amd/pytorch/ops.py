@@ -285,6 +285,46 @@ def structured_tables(row_offsets, column_indices, k):
     return _known_tables(row_offsets, column_indices, k) if share is not None and share >= _STRUCTURE_SHARE else None
 
 
+def prepare_mask(q, row_offsets, column_indices):
+    """Make what sparse attention in one kernel reads of a mask (``iex_mask_tables``) and keep it with the mask's note, so
+    that calls on the mask with operands like ``q`` (heads, tokens, head_dim) are served by that kernel.  False where they
+    are not: other shapes, a pattern that is not canonical CSR or that nobody may look at (``mark_canonical(..., measure=False)``: it changes from call to call),
+    an active :func:`kernel_params` block, a running stream capture.  A mask whose first call was captured keeps to the
+    kernels that were recorded, so that replays and eager calls give the same bits."""
+    tokens, dtype = q.shape[1], q.dtype
+    if dtype not in _DT or not q.is_cuda:
+        return False
+    if torch.cuda.is_current_stream_capturing():
+        column_indices.__dict__.setdefault("_iex_mask_tables", None)
+        return False
+    if any(getattr(_TUNING, name, None) for name in ("spmm", "sddmm", "gemm")) or \
+            not all(t.dtype == torch.int32 and t.dim() == 1 and t.device == q.device and t.is_contiguous() for t in (row_offsets, column_indices)) or \
+            row_offsets.numel() != tokens + 1 or not _lib.load().iex_sparse_attention_fits(_DT[dtype], q.shape[2], tokens):
+        return False
+    status, hist = _pattern_note(row_offsets, column_indices, tokens)
+    if status != 0 or hist is None:
+        return False
+    which = int(dtype == torch.float32)
+    kept = column_indices.__dict__.setdefault("_iex_mask_tables", [None, None])
+    if kept is None:
+        return False
+    key = (weakref.ref(row_offsets), _version(row_offsets), _version(column_indices))
+    if kept[which] is None or kept[which][0][0]() is not row_offsets or kept[which][0][1:] != key[1:]:
+        nonzeros = column_indices.numel()
+        nbytes = _lib.load().iex_mask_tables_bytes(tokens, tokens, nonzeros)
+        if nbytes == 0:
+            return False
+        tables = torch.empty(nbytes, dtype=torch.uint8, device=row_offsets.device)
+        with torch.cuda.device(row_offsets.device):
+            rc = _lib.load().iex_mask_tables(_DT[dtype], tokens, tokens, nonzeros, row_offsets.data_ptr(), column_indices.data_ptr(), tables.data_ptr(),
+                                             nbytes, _stream_ptr(row_offsets.device))
+            _lib.check(rc, "mask_tables")
+            torch.cuda.current_stream(row_offsets.device).synchronize()      # (every later call, on any stream, only reads them)
+        kept[which] = (key, tables)
+    _iex_host.set_mask_tables(row_offsets, column_indices, tokens, which, kept[which][1])
+    return True
+
+
 def prepare_pattern(row_offsets, column_indices, k, tables=True):
     """Look at a pattern now (see :func:`_csr_status`) so that later calls -- under stream capture too, where nothing can
     be looked at -- take every kernel family for canonical CSR.  Returns the status bits; raises for offsets or columns

@@ -9,14 +9,18 @@ form the attention of one layer:
     probs        = softmax over each CSR row of scores * scale        (in place)
     out[h]       = probs[h] (as CSR values) @ v[h]
 
-All heads share the index arrays; values are per head.  Three launches on the current stream,
-nothing leaves the device, no dense tokens x tokens matrix exists at any point.
+All heads share the index arrays; values are per head.  One launch on the current stream where neither scores nor
+probabilities are asked for (heads of 32, 64 or 128, up to 16384 tokens), three otherwise; nothing leaves the device, no
+dense tokens x tokens matrix exists at any point.
 """
 from __future__ import annotations
 
 import math
 
 import torch
+
+from .. import _iex_host
+from . import ops as _pyops
 
 ops = torch.ops.iex_ops
 
@@ -38,7 +42,14 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_indi
         raise RuntimeError("the mask must be tokens x tokens")
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[2])
-    from . import ops as _pyops
+    if plan is None and not return_probs:
+        # one kernel, scores and probabilities in registers, where it serves the call (its tables of the mask are made by the
+        # first call on it)
+        out = _iex_host.sparse_attention(q, k, v, row_indices, row_offsets, column_indices, scale)
+        if out is None and v.shape == q.shape and _pyops.prepare_mask(q, row_offsets, column_indices):
+            out = _iex_host.sparse_attention(q, k, v, row_indices, row_offsets, column_indices, scale)
+        if out is not None:
+            return out
     if plan is None and q.dtype in (torch.float16, torch.bfloat16) and \
             _pyops.structured_tables(row_offsets, column_indices, tokens) is None:
         # for this call only: what the first product derives from the mask serves the second too.  (Not needed for a
