@@ -58,10 +58,10 @@ int launch_ragged(const SpmmParams& p, int batch, int wpr, hipStream_t stream) {
 }
 
 // ---- few columns in A, wide output: the dense operand's tile lives in LDS ---------------------
-template <typename T, typename IT, int VEC, bool RAGGED, int WAVES>
+template <typename T, typename IT, int VEC, bool RAGGED, int WAVES, int MOST, bool PLAIN>
 __global__ __launch_bounds__(WAVES * kWave) void spmm_smallk_kernel(SpmmParams p, int rows_per_wave) {
   extern __shared__ __align__(16) unsigned char smem[];
-  spmm_smallk_block<T, IT, VEC, RAGGED, WAVES>(p, rows_per_wave, blockIdx.x, blockIdx.y, blockIdx.z, smem);
+  spmm_smallk_block<T, IT, VEC, RAGGED, WAVES, MOST, PLAIN>(p, rows_per_wave, blockIdx.x, blockIdx.y, blockIdx.z, smem);
 }
 
 // full vectors at their natural alignment, or (ragged) any n at element alignment
@@ -95,33 +95,60 @@ bool smallk_wanted(const SpmmParams& p, int batch) {
   return p.m >= 8 * p.k && (double)p.nnz >= (smallk_aligned<T>(p) ? 1.8 : 2.5) * p.m;
 }
 
+template <typename T, typename IT, bool RAGGED, int WAVES, int MOST, bool PLAIN>
+int launch_smallk_one(const SpmmParams& p, int batch, int tiles_n, int lds, hipStream_t stream) {
+  constexpr int kMax = 16 / (int)sizeof(T);
+  const long long tiles = (long long)tiles_n * batch;
+  int rows;   // per wavefront
+  if constexpr (WAVES == 8) {
+    // two workgroups per CU cover for each other's tile load: enough rows for it to be a fraction of what they write
+    rows = std::min(64, std::max(16, p.k / 2));
+    while (rows > 4 && (long long)ceil_div(p.m, WAVES * rows) * tiles < 1024) rows >>= 1;
+  } else {
+    // One per CU: rows are dealt evenly to as many as finish first, rounds of workgroups times the rows of a wavefront plus
+    // four, about what the tile load costs.  (384 x 785 x 785: one workgroup with 50 rows per wavefront, 301 us, not one of 512
+    // rows and one of 273, 328; 96 x 1536 x 1536: four of 24 rows, not two of 48, which are 2.25 rounds: 191 / 227.)
+    double least = 0;
+    rows = 0;
+    for (int blocks = ceil_div(p.m, WAVES * 64), upto = std::max(blocks, ceil_div(p.m, WAVES * 4)); blocks <= upto && blocks < 65536; ++blocks) {
+      const int r = ceil_div(p.m, WAVES * blocks);
+      const double cost = (double)ceil_div(blocks * tiles, 256) * (r + 4);
+      if (rows == 0 || cost < least) rows = r, least = cost;
+      if (blocks >= 64) blocks += blocks / 16;   // (long operands: not every count)
+    }
+  }
+  auto kern = spmm_smallk_kernel<T, IT, kMax, RAGGED, WAVES, MOST, PLAIN>;
+  if (lds > 64 * 1024) {
+    static thread_local bool raised = false;  // per instantiation
+    if (!raised) {
+      if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
+                             "hipFuncSetAttribute(LDS size)"))
+        return rc;
+      raised = true;
+    }
+  }
+  dim3 grid(ceil_div(p.m, WAVES * rows), tiles_n, batch);
+  note_kernel("spmm_smallk_kernel<%s, %s, %d, %s, %d, %d>", type_name<T>(), type_name<IT>(), kMax, RAGGED ? "true" : "false", WAVES, MOST);
+  hipLaunchKernelGGL(kern, grid, dim3(WAVES * kWave), lds, stream, p, rows);
+  return check_hip(hipGetLastError(), "spmm (few columns) launch");
+}
+
+// Two vectors per lane where the output is wider than one and two of every dense row fit the LDS.
 template <typename T, typename IT>
 int launch_smallk(const SpmmParams& p, int batch, hipStream_t stream) {
   constexpr int kMax = 16 / (int)sizeof(T);
-  // rows per wavefront: enough for the tile load (k KB per workgroup) to be a fraction of the output
-  // (8 * rows KB), as long as that leaves every CU several workgroups
-  const long long tiles = (long long)ceil_div(p.n, kWave * kMax) * batch;
-  const int waves = smallk_waves(p.k);
-  int rows = std::min(64, std::max(16, p.k / 2));
-  while (rows > 4 && (long long)ceil_div(p.m, waves * rows) * tiles < 1024) rows >>= 1;
-  const int lds = p.k * kWave * 16;
-  const bool ragged = !smallk_aligned<T>(p);
-  auto kern = waves == 8 ? (ragged ? spmm_smallk_kernel<T, IT, kMax, true, 8> : spmm_smallk_kernel<T, IT, kMax, false, 8>)
-                         : (ragged ? spmm_smallk_kernel<T, IT, kMax, true, 16> : spmm_smallk_kernel<T, IT, kMax, false, 16>);
-  if (lds > 64 * 1024) {
-    static thread_local bool raised[2] = {false, false};  // per instantiation and alignment variant
-    if (!raised[ragged]) {
-      if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 kSmallKMax * kWave * 16),
-                             "hipFuncSetAttribute(LDS size)"))
-        return rc;
-      raised[ragged] = true;
-    }
-  }
-  dim3 grid(ceil_div(p.m, waves * rows), ceil_div(p.n, kWave * kMax), batch);
-  note_kernel("spmm_smallk_kernel<%s, %s, %d, %s, %d>", type_name<T>(), type_name<IT>(), kMax, ragged ? "true" : "false", waves);
-  hipLaunchKernelGGL(kern, grid, dim3(waves * kWave), lds, stream, p, rows);
-  return check_hip(hipGetLastError(), "spmm (few columns) launch");
+  const bool plain = !p.bias && !p.relu && !p.accumulate;
+  const int most = plain && p.n > kWave * kMax && 2 * p.k <= kSmallKMax ? 2 : 1;
+  const SmallkTiles t = smallk_tiles(p.n, most, kMax);
+  const int last = smallk_row_bytes(t.nv, t.single, sizeof(T)), lds = p.k * (t.tiles > 1 ? std::max(last, smallk_row_bytes(most, false, sizeof(T))) : last);
+  const bool eight = smallk_waves(lds) == 8;
+  auto pick = [&](auto ragged) {
+    constexpr bool R = decltype(ragged)::value;
+    if (most == 2) return eight ? launch_smallk_one<T, IT, R, 8, 2, true>(p, batch, t.tiles, lds, stream) : launch_smallk_one<T, IT, R, 16, 2, true>(p, batch, t.tiles, lds, stream);
+    if (plain) return eight ? launch_smallk_one<T, IT, R, 8, 1, true>(p, batch, t.tiles, lds, stream) : launch_smallk_one<T, IT, R, 16, 1, true>(p, batch, t.tiles, lds, stream);
+    return eight ? launch_smallk_one<T, IT, R, 8, 1, false>(p, batch, t.tiles, lds, stream) : launch_smallk_one<T, IT, R, 16, 1, false>(p, batch, t.tiles, lds, stream);
+  };
+  return smallk_aligned<T>(p) ? pick(std::false_type{}) : pick(std::true_type{});
 }
 
 template <typename T, typename IT, int VEC, int LPG>
