@@ -143,7 +143,7 @@ int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream);
  * (v_mfma_f32_32x32x2, 32-row tiles), 6 = family 4's tile with the dense operand loaded from
  * global memory straight into LDS and A expanded 64 columns at a time (fp16 / bf16), 7 = dense
  * form of A in the caller's workspace, then the dense GEMM (iex_spmm_ws only), 8 = A with at most
- * 128 columns and an output at least one tile (64 128-bit vectors) wide: the dense operand's tile
+ * 128 columns and an output at least 256 (16-bit: 64) columns wide: the dense operand's tile
  * in LDS, rows streamed in natural order (bit-equal to family 1 with one wavefront per row; fails
  * on other shapes), 9 = unused,
  * 10 = sparse operands with structure (attention probabilities: bands, blocks, windows) times a dense

@@ -74,8 +74,11 @@ bool smallk_aligned(const SpmmParams& p) {
 template <typename T>
 bool smallk_fits(const SpmmParams& p) {
   constexpr int kMax = 16 / (int)sizeof(T);
-  return p.k >= 1 && p.k <= kSmallKMax && p.n >= kWave * kMax && aligned(p.dense, sizeof(T)) && aligned(p.out, sizeof(T));
+  return p.k >= 1 && p.k <= kSmallKMax && p.n >= (sizeof(T) == 2 ? kWave : kWave * kMax) && aligned(p.dense, sizeof(T)) && aligned(p.out, sizeof(T));
 }
+
+template <typename T>
+bool matrix_core_kernel_applies(const SpmmParams& p, int batch);
 
 // ... and where the library takes it by itself: up to 64 columns (two workgroups per CU), enough rows for
 // the tile load (k KB per workgroup) to be a fraction of what the workgroup writes, and rows that gather:
@@ -83,16 +86,31 @@ bool smallk_fits(const SpmmParams& p) {
 // k = 32, 2 per row: 107 against 127 us; 8 x 4096 x 4096, k = 64, 6 per row: 126 / 172, 32 per row: 344 / 535);
 // almost empty rows are a plain write, which the row kernel does at 6 TB/s with streaming stores
 // (96 x 3136 x 3136, 0.5 per row: 627 against 711).
+//   (rows that are no multiple of the vector: from 2.5 per row -- 384 x 785 x 785, k = 64: 3.2 per row 377 -> 322 us,
+//   1.9 per row 290 -> 313)
+// k = 65 .. 128 (one workgroup of 16 wavefronts per CU), fewer rows per dense row, and outputs narrower than a vector per lane
+// (fp32 / 16-bit; us by the other kernels -> here, for outputs large enough to fill the chip):
+//   k = 128, fp32: 60 x 1000 x 1000, 13 per row 136 -> 99, 2.6 per row 68 -> 91; 24 x 3136 x 3136, 13 per row 450 -> 361, 38 per row
+//     2083 -> 782; 200 x 333 x 333, 13 per row 76 -> 72;
+//   k = 128, fp16: 24 x 785 x 785, 13 per row 45 -> 30; 200 x 333 x 333, 2.6 per row 30 -> 26, 13 per row 77 -> 49; but where the
+//     matrix-core kernels apply they stay ahead (24 x 3136 x 3136, 13 per row 214 / 230, 38 per row 244 / 590);
+//   k = 64, m = 333: 13 per row 71 -> 47 (fp32), 78 -> 49 (fp16), 1.9 per row 26 / 28;
+//   rows of fp16 narrower than half a tile and no whole vectors, which the row kernel takes in single elements: 384 x 197 x 197
+//     64 - 177 -> 26 - 116 whatever k and density; fp32 there: 46 / 53 at 13 per row.
 template <typename T>
 bool smallk_wanted(const SpmmParams& p, int batch) {
-  (void)batch;
-  // (rows that are no multiple of the vector: from 2.5 per row -- 384 x 785 x 785, k = 64: 3.2 per row 377 -> 322 us,
-  // 1.9 per row 290 -> 313)
-  // k = 65 .. 128 (one workgroup of 16 wavefronts per CU): from 4 per row and 32 k rows -- 8 x 4096 x 4096, k = 128:
-  // 6.4 per row 166 -> 137 us, 1.3 per row 102 -> 120.
+  constexpr int kMax = 16 / (int)sizeof(T);
   if (!smallk_fits<T>(p)) return false;
-  if (p.k > 64) return p.m >= 32 * p.k && (double)p.nnz >= 4.0 * p.m;
-  return p.m >= 8 * p.k && (double)p.nnz >= (smallk_aligned<T>(p) ? 1.8 : 2.5) * p.m;
+  const double per_row = (double)p.nnz / std::max(p.m, 1);
+  const bool whole = smallk_aligned<T>(p), large = (double)batch * p.m * p.n >= 8e6;
+  const bool wide = p.n >= kWave * kMax / (sizeof(T) == 2 ? 2 : 1);
+  if (wide && p.k <= 64 && p.m >= 8 * p.k) return per_row >= (whole ? 1.8 : 2.5);
+  if (wide && p.k > 64 && p.m >= 32 * p.k && per_row >= 4.0) return true;
+  if (!large) return false;
+  if (sizeof(T) == 2 && matrix_core_kernel_applies<T>(p, batch)) return false;
+  if (sizeof(T) == 2 && p.n % 8 != 0 && p.n < kWave * kMax / 2) return per_row >= 1.5;
+  if (!wide || p.m < 2 * p.k) return false;
+  return per_row >= (p.k <= 64 ? 8.0 : sizeof(T) == 2 ? 2.5 : 8.0);
 }
 
 template <typename T, typename IT, bool RAGGED, int WAVES, int MOST, bool PLAIN>
@@ -528,6 +546,9 @@ MfmaChoice mfma_variant(const SpmmParams& p, int batch, const Choice& ch) {
   return mc;
 }
 
+template <typename T>
+bool matrix_core_kernel_applies(const SpmmParams& p, int batch) { return mfma_variant<T>(p, batch, Choice{}).kind != 0; }
+
 // fp32 on the matrix cores: int32 indices, n a multiple of 4, 16-byte aligned dense operands.
 // Returns the arrangement code (0 = use a gather kernel) and sets the number of register windows.
 template <typename T, typename IT>
@@ -723,7 +744,7 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
   if (mc.kind == 4) return launch_mfma2<T, IT>(p, batch, mc.param, stream);
   if (mc.kind == 3) return launch_mfma<T, IT>(p, batch, mc.param, stream);
   if (ch.variant == 8) {
-    IEX_REQUIRE(smallk_fits<T>(p), IEX_ERR_UNSUPPORTED, "spmm: the few-columns kernel needs k <= %d and an output at least one tile (64 128-bit vectors) wide", kSmallKMax);
+    IEX_REQUIRE(smallk_fits<T>(p), IEX_ERR_UNSUPPORTED, "spmm: the few-columns kernel needs k <= %d and an output at least %d columns wide", kSmallKMax, sizeof(T) == 2 ? kWave : kWave * kMax);
     return launch_smallk<T, IT>(p, batch, stream);
   }
   int lvec = 0, rpw = 0;
