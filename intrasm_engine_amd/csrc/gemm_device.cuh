@@ -265,6 +265,26 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const Acc& 
   const int gn = n0 + wn * WN * 32 + chunk * 8;
   const int here = min(p.N - gn, 8);   // columns of this lane's chunk that exist (none: <= 0)
   const bool whole = p.N % 8 == 0 && ldc % 8 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;   // (uniform)
+  // the auxiliary operand of the whole tile, all loads in flight together (the fragments' registers are free by now)
+  u32x4 held[WM][32 / RPI];
+  if (aux) {
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int t = 0; t < 32 / RPI; ++t) {
+        const u16* src = aux + (size_t)min(m0 + (wm * WM + i) * 32 + t * RPI + lane / CPR, p.M - 1) * ldc + gn;
+        held[i][t] = u32x4{0u, 0u, 0u, 0u};
+        if (here == 8) {
+          held[i][t] = whole ? *reinterpret_cast<const u32x4*>(src) : *reinterpret_cast<const u128_a2*>(src);
+        } else {
+          unsigned w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (e < here) w[e / 2] |= (unsigned)src[e] << (16 * (e & 1));
+          held[i][t] = u32x4{w[0], w[1], w[2], w[3]};
+        }
+      }
+  }
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
     const int row0 = m0 + (wm * WM + i) * 32;
@@ -276,21 +296,7 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const Acc& 
     }
     if (aux) {
 #pragma unroll
-      for (int t = 0; t < 32 / RPI; ++t) {
-        const int r = t * RPI + lane / CPR;
-        const u16* src = aux + (size_t)min(row0 + r, p.M - 1) * ldc + gn;
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (here == 8) {
-          v = whole ? *reinterpret_cast<const u32x4*>(src) : *reinterpret_cast<const u128_a2*>(src);
-        } else {
-          unsigned w[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (e < here) w[e / 2] |= (unsigned)src[e] << (16 * (e & 1));
-          v = u32x4{w[0], w[1], w[2], w[3]};
-        }
-        *reinterpret_cast<u32x4*>(lds + r * ROWB + chunk * 16) = v;
-      }
+      for (int t = 0; t < 32 / RPI; ++t) *reinterpret_cast<u32x4*>(lds + (t * RPI + lane / CPR) * ROWB + chunk * 16) = held[i][t];
     }
 #pragma unroll
     for (int t = 0; t < 4 * WN; ++t) {
