@@ -121,16 +121,12 @@ __global__ __launch_bounds__(WCN * 128, 1) void gemm_dma_splitk_kernel(GemmParam
   const int part = (b >> 3) & 1, slot = (b >> 4) * kXcds + (b & 7);
   int tile_m, tile_n;
   if (!xcd_tile(slot, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;  // uniform per block
-  const int first = ((p.K + BK - 1) / BK / 2) * BK;   // K entries of the first half: whole steps
+  const KPart half = k_in_halves(p.K, p.kb, BK, part);
   GemmParams q = p;
-  if (part == 0) {
-    q.K = first;
-  } else {
-    q.K = p.K - first;
-    q.A = static_cast<const unsigned short*>(p.A) + first;
-    q.B = static_cast<const unsigned short*>(p.B) + (TRANS_B ? (size_t)first : (size_t)first * p.ldb);
-  }
-  q.kb = min(q.K, p.kb - (p.K - q.K) * part);
+  q.K = half.K;
+  q.kb = half.kb;
+  q.A = static_cast<const unsigned short*>(p.A) + half.k0;
+  q.B = static_cast<const unsigned short*>(p.B) + (TRANS_B ? (size_t)half.k0 : (size_t)half.k0 * p.ldb);
   gemm_tile_dma<BF16, TRANS_B, WM, WN, WCN, BK, STAGES, 1>(q, tile_m, tile_n, blockIdx.y, smem);
 }
 
@@ -177,14 +173,13 @@ __global__ __launch_bounds__(WCN * 128, (WCN == 2 && WM * WN <= 8 && gemm_dma_ld
   const int part = (b >> 3) % parts, slot = ((b >> 3) / parts) * kXcds + (b & 7);
   int tile_m, tile_n;
   if (!xcd_tile(slot, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;  // uniform per block
-  const int steps = (p.K + BK - 1) / BK, per = (steps + parts - 1) / parts * BK;   // K entries per part: whole steps
-  const int k0 = part * per;   // (the host has chosen parts so that every part has a step)
+  const KPart mine = k_in_parts(p.K, p.kb, BK, parts, part);
   GemmParams q = p;
   q.split_part = part;
-  q.K = min(per, p.K - k0);
-  q.kb = min(q.K, p.kb - k0);   // (the rows that are missing are fewer than a chunk: the last part has some)
-  q.A = static_cast<const unsigned short*>(p.A) + (TRANS_A ? (size_t)k0 * p.lda : (size_t)k0);
-  q.B = static_cast<const unsigned short*>(p.B) + (TRANS_B ? (size_t)k0 : (size_t)k0 * p.ldb);
+  q.K = mine.K;
+  q.kb = mine.kb;
+  q.A = static_cast<const unsigned short*>(p.A) + (TRANS_A ? (size_t)mine.k0 * p.lda : (size_t)mine.k0);
+  q.B = static_cast<const unsigned short*>(p.B) + (TRANS_B ? (size_t)mine.k0 : (size_t)mine.k0 * p.ldb);
   gemm_tile_dma<BF16, TRANS_B, WM, WN, WCN, BK, STAGES, 2, TRANS_A>(q, tile_m, tile_n, blockIdx.y, smem);
 }
 

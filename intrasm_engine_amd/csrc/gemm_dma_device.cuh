@@ -27,6 +27,7 @@
 // fixed number of loads per step: past the last tile the last tile is fetched again.
 // A K tail (K % BK != 0) is zeroed in LDS by the threads that fetched it, before the barrier.
 #pragma once
+#include "gemm_addresses.h"
 #include "gemm_device.cuh"
 
 namespace iex {
@@ -103,12 +104,7 @@ __device__ __forceinline__ int kn_fragment_offset(int lane, int block) {
   return kr * (ROW_ELEMS * 2) + c * 16 + (lane & 1) * 8;
 }
 
-// The same for fragments of 16 rows (columns) x 32 k: a read of 32 lanes covers 4 k rows and the 4 k rows 8 further, 32
-// bytes of each, and the permutation puts them into the eight different 8-bank groups.
-template <int ROW_ELEMS>
-__device__ __forceinline__ int kn16_swizzle(int kr) {
-  return ROW_ELEMS >= 128 ? ((kr & 3) << 1) | (kr & 8) : (kr & 2) | ((kr & 8) >> 1);
-}
+// The same for fragments of 16 rows (columns) x 32 k.
 template <int ROW_ELEMS>
 __device__ __forceinline__ int kn16_fragment_offset(int lane, int block) {
   const int kr = (lane >> 4) * 8 + ((lane & 15) >> 2);
@@ -121,12 +117,10 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32, WAVES = 2 * WCN;
   constexpr int CPR = BK / 8;          // 16-byte chunks per K-contiguous row
   constexpr int RB = BK * 2;           // bytes per K-contiguous row
-  constexpr int RPI = 64 / CPR;        // rows one wavefront instruction fills
   constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, STAGE_BYTES = A_BYTES + B_BYTES;
   constexpr int A_INSTR = A_BYTES / 1024 / WAVES, B_INSTR = B_BYTES / 1024 / WAVES;  // per wavefront and tile
   constexpr int LOADS = A_INSTR + B_INSTR;
   constexpr int CPRB = BN / 8, CPRA = BM / 8;         // (K,N), (K,M) layout: chunks per k row
-  constexpr int RPIB = 64 / (CPRB < 64 ? CPRB : 64), RPIA = 64 / (CPRA < 64 ? CPRA : 64);  // ... k rows per instruction
   static_assert(BK == 32 || BK == 64, "K step");
   static_assert(A_INSTR >= 1 && B_INSTR >= 1 && A_BYTES % (1024 * WAVES) == 0 && B_BYTES % (1024 * WAVES) == 0,
                 "every wavefront fetches whole kilobytes of A and of B");
@@ -146,39 +140,29 @@ __device__ __forceinline__ void gemm_tile_dma(const GemmParams& p, int tile_m, i
   u16* __restrict__ C = static_cast<u16*>(p.C) + (size_t)z * p.stride_c;
   const unsigned lds0 = (unsigned)(size_t)(lds_u8*)smem;  // LDS byte address of stage 0
   const int lda = p.lda ? p.lda : TRANS_A ? p.M : p.K, ldb = p.ldb ? p.ldb : TRANS_B ? p.K : p.N;   // row strides
-  const int last_kb = (p.kb ? p.kb : p.K) - 1;   // the last k row of a (K,N) B
+  const int kb = p.kb ? p.kb : p.K;   // the k rows of a (K,N) B
 
-  // ---- what this lane fetches, as byte offsets at k = 0.  Rows past M (columns past N) are the last one's: they feed rows
-  // (columns) of C that are not stored.
-  const u32x4 a_buf = TRANS_A ? buffer_of(A, (size_t)p.K * lda * 2) : buffer_of(A + (size_t)m0 * lda, (size_t)(p.M - m0) * lda * 2);
-  const u32x4 b_buf = TRANS_B ? buffer_of(B + (size_t)n0 * ldb, (size_t)(p.N - n0) * ldb * 2) : buffer_of(B, (size_t)(last_kb + 1) * ldb * 2);
-  unsigned a_lane[A_INSTR];
-  int a_k8[A_INSTR];          // (M,K): first k of the chunk inside a K step; (K,M): k row inside a K step
+  // ---- what this lane fetches (gemm_addresses.h).  Rows past M (columns past N) are the last one's: they feed rows (columns)
+  // of C that are not stored.
+  const u32x4 a_buf = TRANS_A ? buffer_of(A, rows_bytes(p.K, p.M, lda)) : buffer_of(A + (size_t)m0 * lda, rows_bytes(p.M - m0, p.K, lda));
+  const u32x4 b_buf = TRANS_B ? buffer_of(B + (size_t)n0 * ldb, rows_bytes(p.N - n0, p.K, ldb)) : buffer_of(B, rows_bytes(kb, p.N, ldb));
+  unsigned a_lane[A_INSTR], b_lane[B_INSTR];
+  int a_k8[A_INSTR], b_k8[B_INSTR];   // K-contiguous: first k of the chunk inside a K step; else k row inside a K step
 #pragma unroll
   for (int q = 0; q < A_INSTR; ++q) {
-    if constexpr (TRANS_A) {
-      const int kr = (wave * A_INSTR + q) * RPIA + lane / CPRA;
-      a_k8[q] = kr;
-      a_lane[q] = ((unsigned)kr * lda + min(m0 + ((lane % CPRA) ^ kn16_swizzle<BM>(kr)) * 8, lda - 8)) * 2u;
-    } else {
-      const int row = (wave * A_INSTR + q) * RPI + lane / CPR;
-      a_k8[q] = ((lane % CPR) ^ (CPR == 4 ? (row >> 2) & 3 : (row >> 1) & 7)) * 8;
-      a_lane[q] = ((unsigned)min(row, p.M - 1 - m0) * lda + a_k8[q]) * 2u;
-    }
+    DirectChunk c;
+    if constexpr (TRANS_A) c = column_chunk<BM>(wave * A_INSTR + q, lane, m0, lda);
+    else c = row_chunk<BK>(wave * A_INSTR + q, lane, p.M - m0, lda);
+    a_lane[q] = c.offset;
+    a_k8[q] = c.k;
   }
-  unsigned b_lane[B_INSTR];
-  int b_k8[B_INSTR];
 #pragma unroll
   for (int q = 0; q < B_INSTR; ++q) {
-    if constexpr (TRANS_B) {
-      const int row = (wave * B_INSTR + q) * RPI + lane / CPR;
-      b_k8[q] = ((lane % CPR) ^ (CPR == 4 ? (row >> 2) & 3 : (row >> 1) & 7)) * 8;
-      b_lane[q] = ((unsigned)min(row, p.N - 1 - n0) * ldb + b_k8[q]) * 2u;
-    } else {
-      const int kr = (wave * B_INSTR + q) * RPIB + lane / CPRB;
-      b_k8[q] = kr;
-      b_lane[q] = ((unsigned)kr * ldb + min(n0 + ((lane % CPRB) ^ kn16_swizzle<BN>(kr)) * 8, ldb - 8)) * 2u;
-    }
+    DirectChunk c;
+    if constexpr (TRANS_B) c = row_chunk<BK>(wave * B_INSTR + q, lane, p.N - n0, ldb);
+    else c = column_chunk<BN>(wave * B_INSTR + q, lane, n0, ldb);
+    b_lane[q] = c.offset;
+    b_k8[q] = c.k;
   }
   const unsigned a_step = (TRANS_A ? (unsigned)BK * lda : (unsigned)BK) * 2u, b_step = (TRANS_B ? (unsigned)BK : (unsigned)BK * ldb) * 2u;
   const int KT = (p.K + BK - 1) / BK;

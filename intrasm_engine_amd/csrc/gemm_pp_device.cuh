@@ -54,8 +54,6 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   // Loads per wavefront that may be in flight where a phase ends: those of two phases (one, for KP = 64).
   constexpr int FLY = A_INSTR + HALVES * B_INSTR;
   constexpr int CPRB = BN / 8, CPRA = BM / 8;         // (K,N), (K,M) layout: chunks per k row
-  constexpr int RPIB = 64 / (CPRB < 64 ? CPRB : 64), RPIA = 64 / (CPRA < 64 ? CPRA : 64);  // ... k rows per instruction
-  constexpr int CPKB = KP / 8;                        // (N,K) layout: chunks per row
   static_assert(WAVES == 8, "two wavefronts per SIMD");
   static_assert(KP == 32 || KP == 64, "k per phase");
   static_assert(A_INSTR >= HALVES && B_INSTR >= 1 && A_STAGE % (1024 * WAVES) == 0 && B_STAGE % (1024 * WAVES) == 0,
@@ -77,41 +75,31 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   u16* __restrict__ C = static_cast<u16*>(p.C) + (size_t)z * p.stride_c;
   const unsigned lds0 = (unsigned)(size_t)(lds_u8*)smem;
   const int lda = p.lda ? p.lda : TRANS_A ? p.M : p.K, ldb = p.ldb ? p.ldb : TRANS_B ? p.K : p.N;   // row strides
-  const int last_kb = (p.kb ? p.kb : p.K) - 1;   // the last k row of a (K,N) B
+  const int kb = p.kb ? p.kb : p.K;   // the k rows of a (K,N) B
 
-  // ---- what this lane fetches.  A: 8 rows of 128 bytes per instruction, LDS position (row, c) holds global chunk
+  // ---- what this lane fetches (gemm_addresses.h).  A: 8 rows of 128 bytes per instruction, LDS position (row, c) holds global chunk
   // c ^ ((row >> 1) & 7).  B as (N,K): the same, or 16 rows of 64 bytes, chunk c ^ ((row >> 2) & 3).  B as (K,N): k rows of BN
   // elements, chunk c ^ kn16_swizzle(k), and A as (K,M) likewise, 64 k rows of BM elements per stage.
   // Rows past M (columns past N) are the last one's: they feed rows (columns) of C that are not stored.
-  const u32x4 a_buf = TRANS_A ? buffer_of(A, (size_t)p.K * lda * 2) : buffer_of(A + (size_t)m0 * lda, (size_t)(p.M - m0) * lda * 2);
-  const u32x4 b_buf = TRANS_B ? buffer_of(B + (size_t)n0 * ldb, (size_t)(p.N - n0) * ldb * 2) : buffer_of(B, (size_t)(last_kb + 1) * ldb * 2);
-  unsigned a_lane[A_INSTR];    // byte offset inside the buffer at k = 0
-  int a_k8[A_INSTR];           // (M,K): first k of the chunk inside a tile; (K,M): k row inside a tile
+  const u32x4 a_buf = TRANS_A ? buffer_of(A, rows_bytes(p.K, p.M, lda)) : buffer_of(A + (size_t)m0 * lda, rows_bytes(p.M - m0, p.K, lda));
+  const u32x4 b_buf = TRANS_B ? buffer_of(B + (size_t)n0 * ldb, rows_bytes(p.N - n0, p.K, ldb)) : buffer_of(B, rows_bytes(kb, p.N, ldb));
+  unsigned a_lane[A_INSTR], b_lane[B_INSTR];   // byte offset inside the buffer at k = 0
+  int a_k8[A_INSTR], b_k8[B_INSTR];            // K-contiguous: first k of the chunk inside a tile; else k row inside a tile
 #pragma unroll
   for (int q = 0; q < A_INSTR; ++q) {
-    if constexpr (TRANS_A) {
-      const int kr = (wave * A_INSTR + q) * RPIA + lane / CPRA;
-      a_k8[q] = kr;
-      a_lane[q] = ((unsigned)kr * lda + min(m0 + ((lane % CPRA) ^ kn16_swizzle<BM>(kr)) * 8, lda - 8)) * 2u;
-    } else {
-      const int row = (wave * A_INSTR + q) * 8 + lane / 8;
-      a_k8[q] = ((lane % 8) ^ ((row >> 1) & 7)) * 8;
-      a_lane[q] = ((unsigned)min(row, p.M - 1 - m0) * lda + a_k8[q]) * 2u;
-    }
+    DirectChunk c;
+    if constexpr (TRANS_A) c = column_chunk<BM>(wave * A_INSTR + q, lane, m0, lda);
+    else c = row_chunk<64>(wave * A_INSTR + q, lane, p.M - m0, lda);
+    a_lane[q] = c.offset;
+    a_k8[q] = c.k;
   }
-  unsigned b_lane[B_INSTR];
-  int b_k8[B_INSTR];
 #pragma unroll
   for (int q = 0; q < B_INSTR; ++q) {
-    if constexpr (TRANS_B) {
-      const int row = (wave * B_INSTR + q) * (64 / CPKB) + lane / CPKB;
-      b_k8[q] = ((lane % CPKB) ^ (KP == 32 ? (row >> 2) & 3 : (row >> 1) & 7)) * 8;
-      b_lane[q] = ((unsigned)min(row, p.N - 1 - n0) * ldb + b_k8[q]) * 2u;
-    } else {
-      const int kr = (wave * B_INSTR + q) * RPIB + lane / CPRB;
-      b_k8[q] = kr;
-      b_lane[q] = ((unsigned)kr * ldb + min(n0 + ((lane % CPRB) ^ kn16_swizzle<BN>(kr)) * 8, ldb - 8)) * 2u;
-    }
+    DirectChunk c;
+    if constexpr (TRANS_B) c = row_chunk<KP>(wave * B_INSTR + q, lane, p.N - n0, ldb);
+    else c = column_chunk<BN>(wave * B_INSTR + q, lane, n0, ldb);
+    b_lane[q] = c.offset;
+    b_k8[q] = c.k;
   }
   const int P = (p.K + KP - 1) / KP;   // phases
   const int TA = (p.K + 63) / 64;      // A tiles

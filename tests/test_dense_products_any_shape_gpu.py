@@ -91,3 +91,32 @@ def test_sddmm_by_the_dense_product(oracle, dev, dtype, m, n, k, batch):
     args = (csr.row_indices, csr.row_offsets, csr.column_indices)
     scale = np.stack([oracle.sddmm_abs_scale(ar[z:z + 1], br[z:z + 1], *args) for z in range(batch)])
     assert_close(got.float().cpu().numpy(), oracle.sddmm(ar, br, *args, sum_over_batch=False), scale, RTOL[dtype], "sampled")
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])      # B (K,N), B (N,K), A (K,M)
+@pytest.mark.parametrize("tile,mnk", [(0, (1000, 200, 4104)), (14, (72, 136, 1160)), (12, (264, 264, 104)), (13, (264, 264, 72)), (15, (136, 264, 72))])
+def test_operands_that_end_where_their_memory_does(oracle, dev, layout, tile, mnk):
+    """K with a tail, in parts and whole, on operands that are the last bytes of a memory block of their own."""
+    if tile == 12 and layout == 2:
+        pytest.skip("K in halves has no A as (K, M)")
+    M, N, K = mnk
+    rng = np.random.default_rng(M + K)
+    a, b = _normal(rng, M, K), _normal(rng, K, N)
+
+    def at_the_end(x):
+        block = torch.full((12 << 20,), float("nan"), dtype=torch.bfloat16, device=dev)      # (24 MiB: a segment of its own)
+        view = block[block.numel() - x.size:].view(x.shape)
+        view.copy_(torch.from_numpy(np.ascontiguousarray(x)).bfloat16())
+        return view
+
+    at, bt = at_the_end(a.T if layout == 2 else a), at_the_end(b.T if layout == 1 else b)
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+    lib = _lib.load()
+    code = layout | (tile << 4)
+    need = lib.iex_gemm_workspace_bytes(_lib.BF16, code, M, N, K, 1)
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
+    _lib.check(lib.iex_gemm_ws(_lib.BF16, code, M, N, K, at.data_ptr(), bt.data_ptr(), out.data_ptr(), 1, 0, 0, 0, torch.cuda.current_stream().cuda_stream,
+                               ws.data_ptr(), need))
+    assert ("parts" in _lib.last_kernels()) == (tile in (0, 14))
+    ar, br = rounded(a, torch.bfloat16), rounded(b, torch.bfloat16)
+    assert_close(out.float().cpu().numpy(), oracle.gemm(ar, br), np.abs(ar) @ np.abs(br), RTOL[torch.bfloat16], f"{mnk} tile {tile} layout {layout}")
