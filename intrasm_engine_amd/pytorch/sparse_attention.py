@@ -34,7 +34,7 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_indi
     Rows of the mask without entries give zero output rows.
     ``plan``: an ``ops.SddmmPlan`` that the caller keeps for this mask; with it the tables and lists that the two sparse
     products derive from the mask are written by the first call only (16-bit inputs; ignored where those kernels are not
-    the ones that run)."""
+    the ones that run: in the one launch too, unless the plan names its kernels, by ``analyze()`` or its ``variant``)."""
     if q.dim() != 3 or k.shape != q.shape or v.dim() != 3 or v.shape[:2] != q.shape[:2]:
         raise RuntimeError("q, k must be (heads, tokens, d) and v (heads, tokens, dv)")
     tokens = q.shape[1]
@@ -42,7 +42,7 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_indi
         raise RuntimeError("the mask must be tokens x tokens")
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[2])
-    if plan is None and not return_probs:
+    if not return_probs and (plan is None or plan.variant == 0):
         # one kernel, scores and probabilities in registers, where it serves the call (its tables of the mask are made by the
         # first call on it)
         out = _iex_host.sparse_attention(q, k, v, row_indices, row_offsets, column_indices, scale)
