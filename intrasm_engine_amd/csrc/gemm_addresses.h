@@ -5,6 +5,7 @@
 #include <cstddef>
 
 #ifdef __HIPCC__
+#include <hip/hip_runtime.h>
 #define IEX_HD __host__ __device__ __forceinline__
 #else
 #define IEX_HD inline
