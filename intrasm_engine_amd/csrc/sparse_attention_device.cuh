@@ -4,7 +4,7 @@
 // By three kernels (SDDMM, softmax over CSR rows, SpMM) the scores of 16 heads over 287 entries per row of 4096 went
 // through memory five times (38 MB each way), the gather kernels read 2 * HD * size bytes per entry through the L2 -> CU path,
 // and a short prompt was three launches of 5 - 20 us.  Us per call before / here: 8 heads x 1000 tokens, causal band of 256,
-// bf16: 37 / 7.4; 16 x 4096, band 256 + 32 scattered, fp16: 81 / 44; 32 x 2048 x 128, causal band of 512, fp32: 1121 / 182.
+// bf16: 37 / 6.8; 16 x 4096, band 256 + 32 scattered, fp16: 81 / 38.7; 32 x 2048 x 128, causal band of 512, fp32: 1121 / 182.
 //
 // The mask's tables (made once per mask by mask_tables_kernel): per block of 128 rows the 64-column tiles that hold at
 // least dense_min entries ("dense"), for each of them a 64-bit word per row, and per row the columns outside dense tiles.
@@ -173,6 +173,26 @@ __device__ __forceinline__ float sa_dot(u32x4 a, u32x4 b) {
   return acc;
 }
 
+// The whole row's product out of its CPR lanes' chunks; every one of them gets it.
+template <int TYPE, int CPR>
+__device__ __forceinline__ float sa_row_dot(u32x4 a, u32x4 b) {
+  float x = group_sum<(CPR > 16 ? 16 : CPR)>(sa_dot<TYPE>(a, b));
+  if constexpr (CPR == 32) x += __shfl_xor(x, 16);
+  return x;
+}
+
+// acc += w * the elements of a chunk
+template <int TYPE>
+__device__ __forceinline__ void sa_add_row(float* acc, float w, u32x4 chunk) {
+#pragma unroll
+  for (int e = 0; e < (TYPE == 2 ? 4 : 8); ++e) {
+    float x;
+    if constexpr (TYPE == 2) x = __uint_as_float(chunk[e]);
+    else x = f16_to_32((unsigned short)(chunk[e / 2] >> (16 * (e & 1))), TYPE == 1);
+    acc[e] = fmaf(w, x, acc[e]);
+  }
+}
+
 template <int TYPE>
 __device__ __forceinline__ unsigned sa_pack(float a, float b) {
   typedef float f2 __attribute__((ext_vector_type(2)));
@@ -197,7 +217,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
   constexpr int INSTR = TILE / 1024 / QW;           // direct loads per wavefront, operand and stage
   static_assert(TILE % (1024 * QW) == 0, "whole kilobytes per wavefront");
   static_assert(QW == 1 || KW == 1, "either queries or keys are shared out");
-  constexpr float kNone = -1e30f;                   // the maximum of no entries
+  constexpr float kNone = -1e30f;                   // the maximum of no entries (finite: differences of it are)
   typedef __attribute__((address_space(3))) unsigned char lds_u8;
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int STAGE = 2 * TILE, MASKS = 2 * STAGE;
@@ -400,11 +420,14 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
       i32x4_a4 next[U / 4];
 #pragma unroll
       for (int x = 0; x < U / 4; ++x) next[x] = *reinterpret_cast<const i32x4_a4*>(at_cols + x * 4);
+      // Past the row's last entry: its first one again, with weight 0.  Another token's V there would turn a row that is finite
+      // into NaN (and be computed once more, below).  Zeroes in the registers instead: 16 x 4096, 32 scattered, 40.3 -> 41.4 us.
+      const int past = count > 0 ? next[0][0] : 0;
       for (int c0 = 0; c0 < most; c0 += U) {
         u32x4 kv[U], vv[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {   // (an entry past the row's last: row 0)
-          const int c = c0 + u < count ? next[u / 4][u % 4] : 0;
+        for (int u = 0; u < U; ++u) {
+          const int c = c0 + u < count ? next[u / 4][u % 4] : past;
           kv[u] = *reinterpret_cast<const u32x4*>(k + ((size_t)c * CPR + part) * 16);
           vv[u] = *reinterpret_cast<const u32x4*>(v + ((size_t)c * CPR + part) * 16);
         }
@@ -416,9 +439,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
         float d[U], m = -INFINITY;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          float x = sa_dot<TYPE>(qv, kv[u]);
-          x = group_sum<(CPR > 16 ? 16 : CPR)>(x);
-          if constexpr (CPR == 32) x += __shfl_xor(x, 16);
+          const float x = sa_row_dot<TYPE, CPR>(qv, kv[u]);
           d[u] = c0 + u < count ? x : -INFINITY;
           m = fmaxf(m, d[u]);
         }
@@ -431,13 +452,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
         for (int u = 0; u < U; ++u) {
           const float w = __builtin_amdgcn_exp2f(fmaf(d[u], p.scale_log2, shift));
           sum_r += w;
-#pragma unroll
-          for (int e = 0; e < E; ++e) {
-            float x;
-            if constexpr (F32) x = __uint_as_float(vv[u][e]);
-            else x = f16_to_32((unsigned short)(vv[u][e / 2] >> (16 * (e & 1))), TYPE == 1);
-            acc[e] = fmaf(w, x, acc[e]);
-          }
+          sa_add_row<TYPE>(acc, w, vv[u]);
         }
       }
 #pragma unroll
@@ -474,11 +489,13 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
         for (int r = 0; r < 16; ++r) o[d][r] = o[d][r] * keep + theirs[(d * 16 + r) * kWave] * keep_w;
     }
   }
+  float top_all = top;
   if (__ballot(my_count > 0)) {   // (uniform) the sums over entries outside dense tiles
     __builtin_amdgcn_wave_barrier();   // (the LDS operations of one wavefront execute in order)
     const float top_t = state[col * 2], sum_t = state[col * 2 + 1];
     const float now = fmaxf(top, top_t);
     const float keep = __builtin_amdgcn_exp2f((top - now) * p.scale_log2), keep_t = __builtin_amdgcn_exp2f((top_t - now) * p.scale_log2);
+    top_all = now;
     sum = sum * keep + sum_t * keep_t;
 #pragma unroll
     for (int d = 0; d < DT; ++d)
@@ -490,7 +507,78 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
       }
   }
 
-  const float inv = sum > 0.f ? 1.f / sum : 0.f;   // (a row without entries: zeros)
+  // ---- rows whose result the above does not give, once more, entry by entry, by the mask's words and lists: a masked key's
+  // infinity or NaN in V times its weight 0 is NaN for all 32 queries (so any row that is not finite); scores that are all at
+  // or below kNone, or infinite, left nothing in the sum.  Two passes over a row, its maximum first.  Looking costs 0.1 us (8
+  // heads x 424 of 128: 7.96 -> 8.07); clean V in every tile would cost every tile.
+  bool again = false;
+  {
+    float all[4] = {sum, 0.f, 0.f, 0.f};   // not finite where anything in it is not (or where products are beyond 1e38: no harm)
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) all[r / 2 % 4] = fmaf(o[d][r], o[d][r + 1], all[r / 2 % 4]);
+    again = query < T && !(fabsf((all[0] + all[1]) + (all[2] + all[3])) < INFINITY && sum > 0.f && top_all > kNone);
+  }
+  if (__ballot(again)) {   // (uniform)
+    if (again && p.row_offsets[query] == p.row_offsets[query + 1]) {   // a row without entries: zeros
+      again = false;
+      sum = 0.f;
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] = 0.f;
+    }
+    const unsigned long long lanes = __ballot(again);
+    const unsigned todo = (unsigned)lanes | (unsigned)(lanes >> 32);
+    constexpr int G = kWave / CPR, E = 16 / ES;
+    const int* thin_cols = reinterpret_cast<const int*>(p.tables + mt.thin_cols);
+    const int sub = lane / CPR, part = lane % CPR;
+    for (int r0 = 0; r0 < 32; r0 += G) {
+      const unsigned these = todo >> r0 & (unsigned)((1ull << G) - 1);
+      if (!these) continue;   // (uniform)
+      if (these >> sub & 1) {
+        const int r = r0 + sub, row = row0 + r, nd = list[0], nt = thin_counts[row], first = p.row_offsets[row];
+        const u32x4 qv = *reinterpret_cast<const u32x4*>(q + ((size_t)row * CPR + part) * 16);
+        auto entries = [&](auto each) {   // (the same for the CPR lanes of a row)
+          for (int i = 0; i < nd; ++i) {
+            unsigned long long word = *reinterpret_cast<const unsigned long long*>(bits + ((size_t)i * kMaRows + r) * 8);
+            const int c0 = (list[1 + i] & 0xffff) * kMaCols;
+            for (; word; word &= word - 1) each(c0 + __ffsll((long long)word) - 1);
+          }
+          for (int i = 0; i < nt; ++i) each(thin_cols[first + i]);
+        };
+        auto score = [&](int c) { return sa_row_dot<TYPE, CPR>(qv, *reinterpret_cast<const u32x4*>(k + ((size_t)c * CPR + part) * 16)); };
+        float m = -INFINITY, total = 0.f, acc[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[e] = 0.f;
+        entries([&](int c) { m = fmaxf(m, score(c)); });
+        entries([&](int c) {
+          const float w = __builtin_amdgcn_exp2f((score(c) - m) * p.scale_log2);
+          total += w;
+          sa_add_row<TYPE>(acc, w, *reinterpret_cast<const u32x4*>(v + ((size_t)c * CPR + part) * 16));
+        });
+#pragma unroll
+        for (int e = 0; e < E; e += 4) *reinterpret_cast<f32x4*>(rows + r * TLD + part * E + e) = f32x4{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
+        if (part == 0) state[r * 2 + 1] = total;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (todo >> col & 1) {
+      sum = state[col * 2 + 1];
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(rows + col * TLD + d * 32 + g * 8 + half * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[d][g * 4 + e] = x[e];
+        }
+    }
+  }
+
+  const float inv = sum != 0.f ? 1.f / sum : 0.f;   // (a row without entries: zeros)
   if (query < T) {
     unsigned char* to = static_cast<unsigned char*>(p.out) + at + (size_t)query * HD * ES;
 #pragma unroll
