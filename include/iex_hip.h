@@ -378,7 +378,8 @@ int iex_attention(int dtype, int heads, int head_dim, int seqs, int length, cons
 /* ---- sparse attention over a CSR mask in one kernel: out = softmax(scale * q k^T at the mask's entries) v, operands
  * (heads, tokens, head_dim), mask tokens x tokens in canonical CSR (columns ascend inside a row).  iex_mask_tables writes,
  * from the index arrays alone, what the kernel reads of the mask (256-byte aligned memory of iex_mask_tables_bytes(tokens,
- * tokens, nonzeros), 0: not served); they serve every call of that dtype on the mask.  A row without entries gives zeros.
+ * tokens, nonzeros), 0: not served); they serve every call of that dtype on the mask, and are
+ * all that those read of it.  A row without entries gives zeros.
  * What a row does not attend to leaves no trace in it, infinities and NaN included; what it attends to shows as in the
  * formula (a row of scores that are all -infinity is NaN). */
 size_t iex_mask_tables_bytes(int m, int n, int nonzeros);

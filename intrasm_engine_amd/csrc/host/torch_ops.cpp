@@ -12,6 +12,7 @@
 // tensors or passes for another pattern's, and keeps no memory of theirs alive.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
@@ -43,11 +44,24 @@ Result ask_python(const char* name, const Args&... args) {
   return py::cast<Result>((*python_ops)[name](args...));
 }
 
+// The same for what is called for its effect: its result goes while the interpreter's lock is held.
+template <typename... Args>
+void tell_python(const char* name, const Args&... args) {
+  py::gil_scoped_acquire gil;
+  TORCH_CHECK(python_ops, "iex_ops: the package has not been initialised");
+  (*python_ops)[name](args...);
+}
+
+int dtype_code(at::ScalarType t) { return t == at::kFloat ? IEX_F32 : t == at::kHalf ? IEX_F16 : t == at::kBFloat16 ? IEX_BF16 : -1; }
+
 void check(int rc, const char* what) {
   TORCH_CHECK(rc == 0, what, ": ", iex_last_error(), " (code ", rc, ")");
 }
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+// (of the current device)
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 
 // ---- notes about patterns --------------------------------------------------------------------------------------
 typedef c10::weak_intrusive_ptr<c10::TensorImpl> Weak;
@@ -59,7 +73,9 @@ struct Note {
   std::array<int, 16> histogram;
   double dense_share;   // < 0: not known
   Weak tables;          // of the kernels for patterns with structure; may be gone
+  int64_t tables_stream;   // ... the stream whose memory they are, -1: not known
   Weak mask_tables[2];  // of sparse attention in one kernel, for 16-bit types and fp32; may be gone
+  int64_t mask_stream[2];
 };
 Weak weak_of(const std::optional<Tensor>& t) {
   return Weak(t.has_value() ? t->getIntrusivePtr() : c10::intrusive_ptr<c10::TensorImpl, c10::UndefinedTensorImpl>());
@@ -70,6 +86,7 @@ struct Known {   // what a call needs of it
   std::array<int, 16> histogram;
   double dense_share;
   Tensor tables;
+  int64_t tables_stream;
 };
 
 std::shared_mutex notes_mutex;
@@ -80,21 +97,6 @@ std::unordered_map<const c10::TensorImpl*, Note>& notes() {
 size_t notes_sweep_at = 256;
 
 int64_t version_of(const Tensor& t) { return t.is_inference() ? 0 : t._version(); }
-
-void set_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k, int status, const std::optional<std::vector<int>>& histogram,
-              const std::optional<double>& dense_share, const std::optional<Tensor>& tables) {
-  Note n{Weak(column_indices.getIntrusivePtr()), Weak(row_offsets.getIntrusivePtr()), version_of(column_indices), version_of(row_offsets), k, status,
-         histogram.has_value(), {}, dense_share.value_or(-1.0),
-         weak_of(tables), {weak_of({}), weak_of({})}};
-  if (histogram) std::copy_n(histogram->begin(), 16, n.histogram.begin());
-  std::unique_lock lock(notes_mutex);
-  auto& map = notes();
-  if (map.size() >= notes_sweep_at) {   // notes of tensors that are gone
-    for (auto it = map.begin(); it != map.end();) it = it->second.columns.expired() ? map.erase(it) : std::next(it);
-    notes_sweep_at = std::max<size_t>(256, 2 * map.size());
-  }
-  map.insert_or_assign(column_indices.unsafeGetTensorImpl(), std::move(n));
-}
 
 // (with notes_mutex held; null: nothing is known)
 Note* find_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k) {
@@ -109,18 +111,33 @@ Note* find_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t
   return &n;
 }
 
-void set_mask_tables(const Tensor& row_offsets, const Tensor& column_indices, int64_t k, int which, const Tensor& tables) {
+void set_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k, int status, const std::optional<std::vector<int>>& histogram,
+              const std::optional<double>& dense_share, const std::optional<Tensor>& tables, int64_t tables_stream) {
+  Note n{Weak(column_indices.getIntrusivePtr()), Weak(row_offsets.getIntrusivePtr()), version_of(column_indices), version_of(row_offsets), k, status,
+         histogram.has_value(), {}, dense_share.value_or(-1.0),
+         weak_of(tables), tables_stream, {weak_of({}), weak_of({})}, {-1, -1}};
+  if (histogram) std::copy_n(histogram->begin(), 16, n.histogram.begin());
   std::unique_lock lock(notes_mutex);
-  if (Note* n = find_note(row_offsets, column_indices, k)) n->mask_tables[which] = weak_of(tables);
+  if (const Note* before = find_note(row_offsets, column_indices, k)) {   // more is known about the same arrays
+    std::copy_n(before->mask_tables, 2, n.mask_tables);
+    std::copy_n(before->mask_stream, 2, n.mask_stream);
+  }
+  auto& map = notes();
+  if (map.size() >= notes_sweep_at) {   // notes of tensors that are gone
+    for (auto it = map.begin(); it != map.end();) it = it->second.columns.expired() ? map.erase(it) : std::next(it);
+    notes_sweep_at = std::max<size_t>(256, 2 * map.size());
+  }
+  map.insert_or_assign(column_indices.unsafeGetTensorImpl(), std::move(n));
 }
 
-// of a canonical pattern; undefined where there are none
-Tensor mask_tables_of(const Tensor& row_offsets, const Tensor& column_indices, int64_t k, int which) {
-  std::shared_lock lock(notes_mutex);
-  const Note* n = find_note(row_offsets, column_indices, k);
-  if (!n || n->status != 0) return Tensor();
-  auto alive = n->mask_tables[which].lock();
-  return alive ? Tensor(std::move(alive)) : Tensor();
+// for calls of q's type on the mask
+void set_mask_tables(const Tensor& q, const Tensor& row_offsets, const Tensor& column_indices, const Tensor& tables, int64_t stream) {
+  std::unique_lock lock(notes_mutex);
+  Note* n = find_note(row_offsets, column_indices, q.size(1));
+  const int dtype = dtype_code(q.scalar_type()), which = dtype == IEX_F32;
+  if (!n || dtype < 0) return;
+  n->mask_tables[which] = weak_of(tables);
+  n->mask_stream[which] = stream;
 }
 
 std::optional<Known> note_of(const Tensor& row_offsets, const Tensor& column_indices, int64_t k) {
@@ -128,14 +145,23 @@ std::optional<Known> note_of(const Tensor& row_offsets, const Tensor& column_ind
   const Note* found = find_note(row_offsets, column_indices, k);
   if (!found) return {};
   const Note& n = *found;
-  Known known{n.status, n.has_histogram, n.histogram, n.dense_share, Tensor()};
+  Known known{n.status, n.has_histogram, n.histogram, n.dense_share, Tensor(), n.tables_stream};
   if (auto alive = n.tables.lock()) known.tables = Tensor(std::move(alive));
   return known;
 }
 
-// ---- operands that fit -------------------------------------------------------------------------------------------
-int dtype_code(at::ScalarType t) { return t == at::kFloat ? IEX_F32 : t == at::kHalf ? IEX_F16 : t == at::kBFloat16 ? IEX_BF16 : -1; }
+// Tables that outlive a call are memory of the stream they were made on.  Work on another one is told to their allocator;
+// a call that is captured has them kept as long as the pattern's tensor, also where later calls replace them.
+void use_tables(const Tensor& tables, int64_t tables_stream, const Tensor& column_indices, bool captured) {
+  if (captured) {
+    tell_python("keep_recorded", column_indices, tables);
+    return;
+  }
+  const auto stream = c10::hip::getCurrentHIPStream(tables.get_device());
+  if (stream.id() != tables_stream) tables.record_stream(c10::Stream(c10::Stream::UNSAFE, tables.device(), stream.id()));   // (a tensor's device is "cuda", the stream's "hip")
+}
 
+// ---- operands that fit -------------------------------------------------------------------------------------------
 bool plain(const Tensor& t, int64_t dim) { return t.is_cuda() && t.layout() == at::kStrided && t.dim() == dim && t.is_contiguous(); }
 
 bool plain_csr(const Tensor& row_indices, const Tensor& row_offsets, const Tensor& column_indices, const Tensor& with, int64_t m) {
@@ -207,6 +233,7 @@ Tensor spmm_call(const Tensor& b, const Tensor& row_indices, const Tensor& value
   if (ws_bytes && kind_of(flags) == 10) {
     if (!known->tables.defined() || (size_t)known->tables.numel() < ws_bytes) return python();   // (it makes them)
     ws = known->tables;
+    use_tables(ws, known->tables_stream, column_indices, capturing());
     flags |= IEX_SPMM_TABLES_READY | IEX_SPMM_LISTS_READY;
   } else {
     ws = workspace(ws_bytes, b);
@@ -264,6 +291,7 @@ Tensor sddmm(const Tensor& a, const Tensor& b, const Tensor& row_indices, const 
   if (ws_bytes && kind_of(flags) == 3) {
     if (!known->tables.defined() || (size_t)known->tables.numel() < ws_bytes) return python();   // (it makes them)
     ws = known->tables;
+    use_tables(ws, known->tables_stream, column_indices, capturing());
     flags |= IEX_SDDMM_TABLES_READY | IEX_SDDMM_LISTS_READY;
   } else {
     ws = workspace(ws_bytes, a);
@@ -282,7 +310,7 @@ Tensor csr_softmax(Tensor values, const Tensor& row_indices, const Tensor& row_o
   if (!plain(values, 2) || !plain(row_indices, 1) || !plain(row_offsets, 1) || dtype < 0 || row_indices.scalar_type() != at::kInt ||
       row_offsets.scalar_type() != at::kInt || row_offsets.size(0) != m + 1 || row_indices.device() != values.device() ||
       row_offsets.device() != values.device()) {
-    ask_python<py::object>("csr_softmax_", values, row_indices, row_offsets, scale);
+    tell_python("csr_softmax_", values, row_indices, row_offsets, scale);
     return values;
   }
   const c10::DeviceGuard guard(values.device());
@@ -356,25 +384,36 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
 }
 
 // sparse attention over a mask whose tables exist; None where the kernel does not serve the call
-std::optional<Tensor> sparse_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& row_indices, const Tensor& row_offsets,
-                                       const Tensor& column_indices, double scale) {
+py::object sparse_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& row_indices, const Tensor& row_offsets,
+                            const Tensor& column_indices, double scale) {
   const int dtype = dtype_code(q.scalar_type());
   if (forced || dtype < 0 || !plain(q, 3) || !plain(k, 3) || !plain(v, 3) || k.sizes() != q.sizes() || v.sizes() != q.sizes() ||
       k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() || k.device() != q.device() || v.device() != q.device() || q.size(0) == 0 ||
       !(scale > 0) || !iex_sparse_attention_fits(dtype, q.size(2), q.size(1)) || !plain_csr(row_indices, row_offsets, column_indices, q, q.size(1)) ||
       column_indices.scalar_type() != at::kInt)
-    return {};
-  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) return {};
+    return py::none();
+  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) return py::none();
   for (const Tensor* t : {&q, &k, &v})
-    if (reinterpret_cast<uintptr_t>(t->const_data_ptr()) % 16) return {};
-  const Tensor tables = mask_tables_of(row_offsets, column_indices, q.size(1), dtype == IEX_F32);
-  if (!tables.defined()) return {};
+    if (reinterpret_cast<uintptr_t>(t->const_data_ptr()) % 16) return py::none();
   const c10::DeviceGuard guard(q.device());
+  const bool captured = capturing();
+  const int which = dtype == IEX_F32;
+  Tensor tables;
+  int64_t tables_stream = -1;
+  {
+    std::shared_lock lock(notes_mutex);
+    const Note* n = find_note(row_offsets, column_indices, q.size(1));
+    if (!n || n->status != 0) return py::none();
+    if (auto alive = n->mask_tables[which].lock()) tables = Tensor(std::move(alive));
+    tables_stream = n->mask_stream[which];
+    if (!tables.defined()) return py::none();
+  }
+  use_tables(tables, tables_stream, column_indices, captured);
   Tensor out = at::empty_like(q);
   check(iex_sparse_attention(dtype, q.size(0), q.size(1), q.size(2), column_indices.size(0), row_offsets.const_data_ptr<int>(), q.const_data_ptr(),
                              k.const_data_ptr(), v.const_data_ptr(), (float)scale, out.data_ptr(), tables.const_data_ptr(), tables.numel(), stream_of(q)),
         "sparse attention");
-  return out;
+  return py::cast(out);
 }
 
 // ---- autograd: the plain calls of MySpMM and MyLinear (no recording, no forced kernels) -----------------------------

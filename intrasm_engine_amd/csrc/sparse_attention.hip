@@ -87,7 +87,7 @@ extern "C" int iex_sparse_attention(int dtype, int heads, int tokens, int head_d
   const size_t need = iex_mask_tables_bytes(tokens, tokens, nonzeros);
   IEX_REQUIRE(need > 0 && tables && aligned(tables, 256) && bytes >= need, IEX_ERR_BAD_ARGUMENT, "sparse attention: needs the mask's tables (iex_mask_tables, same dtype)");
   IEX_REQUIRE((long long)ceil_div(tokens, 32) * heads < (1ll << 31), IEX_ERR_TOO_LARGE, "sparse attention: too many blocks of queries");
-  SparseAttentionParams p{heads, tokens, nonzeros, q, k, v, out, scale * 1.44269504088896340736f, row_offsets, static_cast<const unsigned char*>(tables)};
+  SparseAttentionParams p{heads, tokens, nonzeros, q, k, v, out, scale * 1.44269504088896340736f, static_cast<const unsigned char*>(tables)};
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == IEX_F32) return launch_type<2>(p, head_dim, s);
   return dtype == IEX_BF16 ? launch_type<1>(p, head_dim, s) : launch_type<0>(p, head_dim, s);

@@ -24,19 +24,21 @@
 namespace iex {
 
 constexpr int kMaRows = 128, kMaCols = 64, kMaMaxTokens = 16384;
+constexpr int kMaEntries = 1 << 31;
 
-// Where the parts of a mask's tables lie in their memory.
+// Where the parts of a mask's tables lie in their memory.  They hold all that the kernel reads of the mask: a recorded launch
+// works on the mask as it was, whatever becomes of the index arrays.
 struct MaskTables {
   int blocks, tiles;            // blocks of 128 rows, tiles of 64 columns
-  size_t list, thin_count, thin_cols, bits, bytes;   // byte offsets and the total
+  size_t list, thin, thin_cols, bits, bytes;   // byte offsets and the total
 };
 inline __host__ __device__ MaskTables mask_tables_layout(int m, int n, int nnz) {
   MaskTables t;
   t.blocks = (m + kMaRows - 1) / kMaRows;
   t.tiles = (n + kMaCols - 1) / kMaCols;
   t.list = 0;                                                              // int [blocks][tiles + 1]: how many; tile | wavefronts of 32 rows << 16
-  t.thin_count = t.list + (size_t)t.blocks * (t.tiles + 1) * 4;            // int [blocks * 128]
-  t.thin_cols = t.thin_count + (size_t)t.blocks * kMaRows * 4;             // int [nnz]: row r's from row_offsets[r]
+  t.thin = (t.list + (size_t)t.blocks * (t.tiles + 1) * 4 + 7) / 8 * 8;    // int2 [blocks * 128]: where a row's begin (kMaEntries: it has entries); how many
+  t.thin_cols = t.thin + (size_t)t.blocks * kMaRows * 8;                   // int [nnz]: row r's from row_offsets[r]
   t.bits = (t.thin_cols + (size_t)nnz * 4 + 255) / 256 * 256;              // u64 [blocks][tiles][128]: by position in the list
   t.bytes = t.bits + (size_t)t.blocks * t.tiles * kMaRows * 8;
   return t;
@@ -56,7 +58,7 @@ __global__ __launch_bounds__(kMtWaves * kWave) void mask_tables_kernel(int m, in
   int* dense = groups + tiles;      // [tiles]: the list
   unsigned* map = reinterpret_cast<unsigned*>(dense + tiles) + wave * tiles * 2;   // [tiles * 2]: this wavefront's row, a bit per column
   int* list = reinterpret_cast<int*>(ws + t.list) + (size_t)rb * (tiles + 1);
-  int* thin_count = reinterpret_cast<int*>(ws + t.thin_count) + (size_t)rb * kMaRows;
+  int2* thin_of = reinterpret_cast<int2*>(ws + t.thin) + (size_t)rb * kMaRows;
   int* thin_cols = reinterpret_cast<int*>(ws + t.thin_cols);
   unsigned long long* bits = reinterpret_cast<unsigned long long*>(ws + t.bits) + (size_t)rb * tiles * kMaRows;
   for (int i = threadIdx.x; i < 2 * tiles; i += blockDim.x) count[i] = 0;
@@ -104,9 +106,10 @@ __global__ __launch_bounds__(kMtWaves * kWave) void mask_tables_kernel(int m, in
   for (int r = wave; r < kMaRows; r += kMtWaves) {
     const int row = rb * kMaRows + r;
     for (int i = lane; i < 2 * tiles; i += kWave) map[i] = 0;
-    int thin = 0;
+    int thin = 0, begin = 0;
     if (row < m) {
       const int start = row_offsets[row], end = row_offsets[row + 1];
+      begin = start | (start < end ? kMaEntries : 0);
       for (int j0 = start; j0 < end; j0 += kWave) {
         const int j = j0 + lane, col = j < end ? cols[j] : -1;
         const bool to_thin = col >= 0 && count[col >> 6] < 0;
@@ -116,7 +119,7 @@ __global__ __launch_bounds__(kMtWaves * kWave) void mask_tables_kernel(int m, in
         thin += __popcll(them);
       }
     }
-    if (lane == 0) thin_count[r] = thin;
+    if (lane == 0) thin_of[r] = int2{begin, thin};
     __builtin_amdgcn_wave_barrier();   // (the LDS operations of one wavefront execute in order)
     for (int s = lane; s < nd; s += kWave) {
       const int tile = dense[s];
@@ -133,7 +136,6 @@ struct SparseAttentionParams {
   const void* v;
   void* out;
   float scale_log2;        // scale * log2(e), > 0
-  const int* row_offsets;
   const unsigned char* tables;
 };
 
@@ -398,8 +400,8 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
   float* state = rows + 32 * TLD;
   const int row0 = q0 + wave * 32;
   const int my_row = min(row0 + col, T - 1);
-  const int* thin_counts = reinterpret_cast<const int*>(p.tables + mt.thin_count);
-  const int my_count = row0 + col < T ? thin_counts[my_row] : 0;
+  const int2* thin_of = reinterpret_cast<const int2*>(p.tables + mt.thin);
+  const int my_count = row0 + col < T ? thin_of[my_row].y : 0;
   if (__ballot(my_count > 0)) {   // (uniform)
     constexpr int G = kWave / CPR, U = HD * ES >= 256 ? 4 : 8, E = 16 / ES;
     typedef int i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -407,8 +409,9 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
     const int sub = lane / CPR, part = lane % CPR;
     for (int r0 = kw * G; r0 < 32; r0 += KW * G) {
       const int row = row0 + r0 + sub, safe = min(row, T - 1);
-      const int count = row < T ? thin_counts[safe] : 0;
-      const int* at_cols = thin_cols + p.row_offsets[safe];   // (what follows the columns in the tables may be read, not used)
+      const int2 thin = thin_of[safe];
+      const int count = row < T ? thin.y : 0;
+      const int* at_cols = thin_cols + (thin.x & ~kMaEntries);   // (what follows the columns in the tables may be read, not used)
       int most = count;   // of the G rows
 #pragma unroll
       for (int x = CPR; x < kWave; x <<= 1) most = max(most, __shfl_xor(most, x));
@@ -509,7 +512,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
 
   // ---- rows whose result the above does not give, once more, entry by entry, by the mask's words and lists: a masked key's
   // infinity or NaN in V times its weight 0 is NaN for all 32 queries (so any row that is not finite); scores that are all at
-  // or below kNone, or infinite, left nothing in the sum.  Two passes over a row, its maximum first.  Looking costs 0.1 us (8
+  // or below kNone, or infinite, left nothing in the sum.  Two passes over a row, its maximum first.  Looking costs 0.1 us (12
   // heads x 424 of 128: 7.96 -> 8.07); clean V in every tile would cost every tile.
   bool again = false;
   {
@@ -521,7 +524,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
     again = query < T && !(fabsf((all[0] + all[1]) + (all[2] + all[3])) < INFINITY && sum > 0.f && top_all > kNone);
   }
   if (__ballot(again)) {   // (uniform)
-    if (again && p.row_offsets[query] == p.row_offsets[query + 1]) {   // a row without entries: zeros
+    if (again && !(thin_of[query].x & kMaEntries)) {   // a row without entries: zeros
       again = false;
       sum = 0.f;
 #pragma unroll
@@ -538,7 +541,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
       const unsigned these = todo >> r0 & (unsigned)((1ull << G) - 1);
       if (!these) continue;   // (uniform)
       if (these >> sub & 1) {
-        const int r = r0 + sub, row = row0 + r, nd = list[0], nt = thin_counts[row], first = p.row_offsets[row];
+        const int r = r0 + sub, row = row0 + r, nd = list[0], nt = thin_of[row].y, first = thin_of[row].x & ~kMaEntries;
         const u32x4 qv = *reinterpret_cast<const u32x4*>(q + ((size_t)row * CPR + part) * 16);
         auto entries = [&](auto each) {   // (the same for the CPR lanes of a row)
           for (int i = 0; i < nd; ++i) {

@@ -38,6 +38,7 @@ _IT = {torch.int32: _lib.I32, torch.int16: _lib.I16}
 
 
 _TUNING = threading.local()
+_MASK_LOCK = threading.Lock()      # one thread at a time makes a mask's tables
 _SPMM_KEYS = ("force_wpr", "force_variant", "force_rpw", "force_nt", "force_lpg")
 
 
@@ -156,6 +157,31 @@ def _dense_share_host(row_offsets, column_indices, k, dense_min=None):
     return int(count.item()) / nonzeros
 
 
+def _table_memory(nbytes, device):
+    """Memory for tables that outlive the call: it is the current stream's, which the allocator has to be told where they
+    are used on another one (:func:`_use_tables`)."""
+    memory = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    memory._iex_stream = torch.cuda.current_stream(device).stream_id
+    return memory
+
+
+def _keep_recorded(column_indices, tables):
+    """A captured call reads ``tables``: they live as long as the pattern's tensor, also where later calls replace them."""
+    recorded = column_indices.__dict__.setdefault("_iex_recorded", [])
+    if not any(t is tables for t in recorded):
+        recorded.append(tables)
+
+
+def _use_tables(tables, column_indices):
+    """The current stream is about to read ``tables`` that are kept with a pattern (``use_tables`` of csrc/host/torch_ops.cpp)."""
+    if torch.cuda.is_current_stream_capturing():
+        _keep_recorded(column_indices, tables)
+        return
+    stream = torch.cuda.current_stream(tables.device)
+    if stream.stream_id != tables._iex_stream:
+        tables.record_stream(stream)
+
+
 def _pattern_tables_host(row_offsets, column_indices, k):
     """The tables and lists of the kernels for patterns with structure, written once (``iex_pattern_tables``) into a
     tensor that lives as long as the pattern's note; the stream is waited for, so every later call on any stream finds
@@ -165,7 +191,7 @@ def _pattern_tables_host(row_offsets, column_indices, k):
     nbytes = lib.iex_pattern_tables_bytes(m, int(k), nonzeros) if column_indices.dtype == torch.int32 else 0
     if nbytes == 0:
         return None
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=row_offsets.device)
+    ws = _table_memory(nbytes, row_offsets.device)
     with torch.cuda.device(row_offsets.device):
         rc = lib.iex_pattern_tables(m, int(k), nonzeros, row_offsets.data_ptr(), column_indices.data_ptr(), ws.data_ptr(), nbytes,
                                     _stream_ptr(row_offsets.device))
@@ -179,7 +205,7 @@ def _set_note(row_offsets, column_indices, k, status, hist, share=None, tables=N
     ``tables``: of the kernels for patterns with structure, made by the first call that wants them."""
     column_indices.__dict__["_iex_csr"] = (weakref.ref(row_offsets), _version(row_offsets), _version(column_indices), int(k), status, hist, share,
                                            tables)
-    _iex_host.set_note(row_offsets, column_indices, int(k), status, hist, share, tables)
+    _iex_host.set_note(row_offsets, column_indices, int(k), status, hist, share, tables, tables._iex_stream if tables is not None else -1)
 
 
 def mark_canonical(row_offsets, column_indices, k, measure=True):
@@ -305,23 +331,25 @@ def prepare_mask(q, row_offsets, column_indices):
     if status != 0 or hist is None:
         return False
     which = int(dtype == torch.float32)
-    kept = column_indices.__dict__.setdefault("_iex_mask_tables", [None, None])
-    if kept is None:
-        return False
-    key = (weakref.ref(row_offsets), _version(row_offsets), _version(column_indices))
-    if kept[which] is None or kept[which][0][0]() is not row_offsets or kept[which][0][1:] != key[1:]:
-        nonzeros = column_indices.numel()
-        nbytes = _lib.load().iex_mask_tables_bytes(tokens, tokens, nonzeros)
-        if nbytes == 0:
+    with _MASK_LOCK:
+        kept = column_indices.__dict__.setdefault("_iex_mask_tables", [None, None])
+        if kept is None:
             return False
-        tables = torch.empty(nbytes, dtype=torch.uint8, device=row_offsets.device)
-        with torch.cuda.device(row_offsets.device):
-            rc = _lib.load().iex_mask_tables(_DT[dtype], tokens, tokens, nonzeros, row_offsets.data_ptr(), column_indices.data_ptr(), tables.data_ptr(),
-                                             nbytes, _stream_ptr(row_offsets.device))
-            _lib.check(rc, "mask_tables")
-            torch.cuda.current_stream(row_offsets.device).synchronize()      # (every later call, on any stream, only reads them)
-        kept[which] = (key, tables)
-    _iex_host.set_mask_tables(row_offsets, column_indices, tokens, which, kept[which][1])
+        key = (weakref.ref(row_offsets), _version(row_offsets), _version(column_indices))
+        if kept[which] is None or kept[which][0][0]() is not row_offsets or kept[which][0][1:] != key[1:]:
+            nonzeros = column_indices.numel()
+            nbytes = _lib.load().iex_mask_tables_bytes(tokens, tokens, nonzeros)
+            if nbytes == 0:
+                return False
+            tables = _table_memory(nbytes, row_offsets.device)
+            with torch.cuda.device(row_offsets.device):
+                rc = _lib.load().iex_mask_tables(_DT[dtype], tokens, tokens, nonzeros, row_offsets.data_ptr(), column_indices.data_ptr(), tables.data_ptr(),
+                                                 nbytes, _stream_ptr(row_offsets.device))
+                _lib.check(rc, "mask_tables")
+                torch.cuda.current_stream(row_offsets.device).synchronize()      # (every later call, on any stream, only reads them)
+            kept[which] = (key, tables)
+        tables = kept[which][1]
+        _iex_host.set_mask_tables(q, row_offsets, column_indices, tables, tables._iex_stream)
     return True
 
 
@@ -453,6 +481,7 @@ def _spmm(b, row_indices, values, row_offsets, column_indices, m, *, per_batch_v
                 (((flags >> 16) & 0xf) != 10 or ((flags >> 8) & 0xff) == 0) else None
             if tables is not None and tables.numel() >= ws_bytes and tables.device == b.device:
                 # written when the pattern was first looked at, with the built-in threshold, and read-only since
+                _use_tables(tables, column_indices)
                 ws = tables
                 flags |= _lib.SPMM_TABLES_READY | _lib.SPMM_LISTS_READY
             else:
@@ -592,6 +621,7 @@ def _sddmm(a, b, row_indices, row_offsets, column_indices, *, sum_over_batch, dt
             tables = _known_tables(row_offsets, column_indices, n) if kind3 and (((flags >> 16) & 0xf) != 3 or ((flags >> 8) & 0xff) == 0) else None
             if tables is not None and tables.numel() >= ws_bytes and tables.device == a.device:
                 # written when the pattern was first looked at, with the built-in threshold, and read-only since
+                _use_tables(tables, column_indices)
                 ws = tables
                 flags |= _lib.SDDMM_TABLES_READY | _lib.SDDMM_LISTS_READY
             else:
@@ -784,6 +814,7 @@ def register() -> None:
         return
     functions = {f.__name__: f for f in (spmm_sputnik_reuse_weight, spmm_sputnik_atomic, spmm_sputnik_reuse_weight_half, spmm_sputnik_batched_values,
                                          sddmm_sputnik_atomic_upd_weight, sddmm_sputnik_half, csr_softmax_, gemm_mfma)}
+    functions["keep_recorded"] = _keep_recorded
     functions["int32_columns"] = lambda columns: carry_pattern_note(columns, columns.to(torch.int32))
     _iex_host.bind(functions)
     lib = torch.library.Library("iex_ops", "FRAGMENT")

@@ -34,7 +34,13 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_indi
     Rows of the mask without entries give zero output rows.
     ``plan``: an ``ops.SddmmPlan`` that the caller keeps for this mask; with it the tables and lists that the two sparse
     products derive from the mask are written by the first call only (16-bit inputs; ignored where those kernels are not
-    the ones that run: in the one launch too, unless the plan names its kernels, by ``analyze()`` or its ``variant``)."""
+    the ones that run: in the one launch too, unless the plan names its kernels, by ``analyze()`` or its ``variant``).
+
+    Under stream capture: the one launch is recorded where a call on the mask has come before, else three, and further calls
+    on the mask then keep to the same three.  Either way the graph works on the mask as it was when it was captured, and its index
+    tensors have to live as long as the graph: what is derived from them lives with ``column_indices``.  A mask that changes
+    between replays is one to vouch for with ``ops.mark_canonical(..., measure=False)``: nothing derived from it is kept, and
+    captured calls derive what they need when they are replayed."""
     if q.dim() != 3 or k.shape != q.shape or v.dim() != 3 or v.shape[:2] != q.shape[:2]:
         raise RuntimeError("q, k must be (heads, tokens, d) and v (heads, tokens, dv)")
     tokens = q.shape[1]
