@@ -76,7 +76,10 @@ struct Note {
   int64_t tables_stream;   // ... the stream whose memory they are, -1: not known
   Weak mask_tables[2];  // of sparse attention in one kernel, for 16-bit types and fp32; may be gone
   int64_t mask_stream[2];
+  unsigned recorded;    // attention_form()s whose first call was captured, by three launches
 };
+// A type and head size that sparse attention in one kernel serves, as a bit.
+unsigned attention_form(int dtype, int64_t head_dim) { return 1u << (dtype * 3 + (head_dim == 32 ? 0 : head_dim == 64 ? 1 : 2)); }
 Weak weak_of(const std::optional<Tensor>& t) {
   return Weak(t.has_value() ? t->getIntrusivePtr() : c10::intrusive_ptr<c10::TensorImpl, c10::UndefinedTensorImpl>());
 }
@@ -115,12 +118,13 @@ void set_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k
               const std::optional<double>& dense_share, const std::optional<Tensor>& tables, int64_t tables_stream) {
   Note n{Weak(column_indices.getIntrusivePtr()), Weak(row_offsets.getIntrusivePtr()), version_of(column_indices), version_of(row_offsets), k, status,
          histogram.has_value(), {}, dense_share.value_or(-1.0),
-         weak_of(tables), tables_stream, {weak_of({}), weak_of({})}, {-1, -1}};
+         weak_of(tables), tables_stream, {weak_of({}), weak_of({})}, {-1, -1}, 0};
   if (histogram) std::copy_n(histogram->begin(), 16, n.histogram.begin());
   std::unique_lock lock(notes_mutex);
   if (const Note* before = find_note(row_offsets, column_indices, k)) {   // more is known about the same arrays
     std::copy_n(before->mask_tables, 2, n.mask_tables);
     std::copy_n(before->mask_stream, 2, n.mask_stream);
+    n.recorded = before->recorded;
   }
   auto& map = notes();
   if (map.size() >= notes_sweep_at) {   // notes of tensors that are gone
@@ -130,7 +134,7 @@ void set_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k
   map.insert_or_assign(column_indices.unsafeGetTensorImpl(), std::move(n));
 }
 
-// for calls of q's type on the mask
+// for calls of q's type on the mask; lifts what an earlier capture has settled for calls like q
 void set_mask_tables(const Tensor& q, const Tensor& row_offsets, const Tensor& column_indices, const Tensor& tables, int64_t stream) {
   std::unique_lock lock(notes_mutex);
   Note* n = find_note(row_offsets, column_indices, q.size(1));
@@ -138,6 +142,7 @@ void set_mask_tables(const Tensor& q, const Tensor& row_offsets, const Tensor& c
   if (!n || dtype < 0) return;
   n->mask_tables[which] = weak_of(tables);
   n->mask_stream[which] = stream;
+  n->recorded &= ~attention_form(dtype, q.size(2));
 }
 
 std::optional<Known> note_of(const Tensor& row_offsets, const Tensor& column_indices, int64_t k) {
@@ -383,7 +388,8 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
   return out;
 }
 
-// sparse attention over a mask whose tables exist; None where the kernel does not serve the call
+// sparse attention in one kernel.  None where it does not serve the call, True where it will once the mask has its tables
+// (ops.prepare_mask).
 py::object sparse_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& row_indices, const Tensor& row_offsets,
                             const Tensor& column_indices, double scale) {
   const int dtype = dtype_code(q.scalar_type());
@@ -401,12 +407,20 @@ py::object sparse_attention(const Tensor& q, const Tensor& k, const Tensor& v, c
   Tensor tables;
   int64_t tables_stream = -1;
   {
-    std::shared_lock lock(notes_mutex);
-    const Note* n = find_note(row_offsets, column_indices, q.size(1));
-    if (!n || n->status != 0) return py::none();
+    std::unique_lock lock(notes_mutex);
+    Note* n = find_note(row_offsets, column_indices, q.size(1));
+    if (!n) return captured ? py::object(py::none()) : py::object(py::bool_(true));   // (nobody has looked at it)
+    const unsigned form = attention_form(dtype, q.size(2));
+    // (columns in any order; a pattern that nobody may look at: it changes from call to call; one whose first call like this
+    // was captured before it had tables: replays and eager calls give the same bits)
+    if (n->status != 0 || !n->has_histogram || (n->recorded & form)) return py::none();
     if (auto alive = n->mask_tables[which].lock()) tables = Tensor(std::move(alive));
     tables_stream = n->mask_stream[which];
-    if (!tables.defined()) return py::none();
+    if (!tables.defined()) {
+      if (!captured) return py::bool_(true);
+      n->recorded |= form;
+      return py::none();
+    }
   }
   use_tables(tables, tables_stream, column_indices, captured);
   Tensor out = at::empty_like(q);

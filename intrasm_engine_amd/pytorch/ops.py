@@ -313,17 +313,13 @@ def structured_tables(row_offsets, column_indices, k):
 
 def prepare_mask(q, row_offsets, column_indices):
     """Make what sparse attention in one kernel reads of a mask (``iex_mask_tables``) and keep it with the mask's note, so
-    that calls on the mask with operands like ``q`` (heads, tokens, head_dim) are served by that kernel.  False where they
-    are not: other shapes, a pattern that is not canonical CSR or that nobody may look at (``mark_canonical(..., measure=False)``: it changes from call to call),
-    an active :func:`kernel_params` block, a running stream capture.  A mask whose first call was captured keeps to the
-    kernels that were recorded, so that replays and eager calls give the same bits."""
+    that calls on the mask with operands like ``q`` (heads, tokens, head_dim) are served by that kernel, captured ones too.
+    False where they are not: other shapes, a pattern that is not canonical CSR or that nobody may look at
+    (``mark_canonical(..., measure=False)``: it changes from call to call), an active :func:`kernel_params` block, a running
+    stream capture."""
     tokens, dtype = q.shape[1], q.dtype
-    if dtype not in _DT or not q.is_cuda:
-        return False
-    if torch.cuda.is_current_stream_capturing():
-        column_indices.__dict__.setdefault("_iex_mask_tables", None)
-        return False
-    if any(getattr(_TUNING, name, None) for name in ("spmm", "sddmm", "gemm")) or \
+    if dtype not in _DT or not q.is_cuda or torch.cuda.is_current_stream_capturing() or \
+            any(getattr(_TUNING, name, None) for name in ("spmm", "sddmm", "gemm")) or \
             not all(t.dtype == torch.int32 and t.dim() == 1 and t.device == q.device and t.is_contiguous() for t in (row_offsets, column_indices)) or \
             row_offsets.numel() != tokens + 1 or not _lib.load().iex_sparse_attention_fits(_DT[dtype], q.shape[2], tokens):
         return False
@@ -333,8 +329,6 @@ def prepare_mask(q, row_offsets, column_indices):
     which = int(dtype == torch.float32)
     with _MASK_LOCK:
         kept = column_indices.__dict__.setdefault("_iex_mask_tables", [None, None])
-        if kept is None:
-            return False
         key = (weakref.ref(row_offsets), _version(row_offsets), _version(column_indices))
         if kept[which] is None or kept[which][0][0]() is not row_offsets or kept[which][0][1:] != key[1:]:
             nonzeros = column_indices.numel()

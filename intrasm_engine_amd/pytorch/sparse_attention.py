@@ -36,8 +36,9 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_indi
     products derive from the mask are written by the first call only (16-bit inputs; ignored where those kernels are not
     the ones that run: in the one launch too, unless the plan names its kernels, by ``analyze()`` or its ``variant``).
 
-    Under stream capture: the one launch is recorded where a call on the mask has come before, else three, and further calls
-    on the mask then keep to the same three.  Either way the graph works on the mask as it was when it was captured, and its index
+    Under stream capture: the one launch is recorded where a call on the mask (or ``ops.prepare_mask``) has come before,
+    else three, and further calls on the mask with operands of this type and head size then keep to the same three
+    (``ops.prepare_mask`` lifts that).  Either way the graph works on the mask as it was when it was captured, and its index
     tensors have to live as long as the graph: what is derived from them lives with ``column_indices``.  A mask that changes
     between replays is one to vouch for with ``ops.mark_canonical(..., measure=False)``: nothing derived from it is kept, and
     captured calls derive what they need when they are replayed."""
@@ -52,8 +53,10 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_indi
         # one kernel, scores and probabilities in registers, where it serves the call (its tables of the mask are made by the
         # first call on it)
         out = _iex_host.sparse_attention(q, k, v, row_indices, row_offsets, column_indices, scale)
-        if out is None and v.shape == q.shape and _pyops.prepare_mask(q, row_offsets, column_indices):
-            out = _iex_host.sparse_attention(q, k, v, row_indices, row_offsets, column_indices, scale)
+        if out is True:
+            prepared = _pyops.prepare_mask(q, row_offsets, column_indices)
+            out = _iex_host.sparse_attention(q, k, v, row_indices, row_offsets, column_indices, scale) if prepared else None
+            out = None if out is True else out      # (somebody has changed the mask since)
         if out is not None:
             return out
     if plan is None and q.dtype in (torch.float16, torch.bfloat16) and \

@@ -94,6 +94,42 @@ def test_replays_follow_a_mask_that_nobody_may_look_at(dev, heads, tokens, band,
     constructor.destroy_graph_exec()
 
 
+def test_a_capture_that_comes_first_settles_calls_like_it_only(dev):
+    tokens = 300
+    ri, ro, ci = _arrays(tokens, 40, dev)
+    pyops.prepare_pattern(ro, ci, tokens)
+    q, k, v = _operands(dev, 2, tokens, 64, torch.float16)
+    constructor, out = _captured(lambda: sparse_attention(q, k, v, ri, ro, ci))
+    assert "sparse_attention_kernel" not in _lib.last_kernels()
+    constructor.execute_graph()
+    constructor.synchronize()
+    for _ in range(2):
+        assert torch.equal(out, sparse_attention(q, k, v, ri, ro, ci)) and "sparse_attention_kernel" not in _lib.last_kernels()
+    constructor.destroy_graph_exec()
+    for dtype, d in ((torch.float32, 64), (torch.bfloat16, 64), (torch.float16, 32)):
+        sparse_attention(*_operands(dev, 2, tokens, d, dtype), ri, ro, ci)
+        assert "sparse_attention_kernel" in _lib.last_kernels(), (dtype, d)
+    sparse_attention(q, k, v, ri, ro, ci)
+    assert "sparse_attention_kernel" not in _lib.last_kernels()
+    assert pyops.prepare_mask(q, ro, ci)
+    got = sparse_attention(q, k, v, ri, ro, ci)
+    assert "sparse_attention_kernel" in _lib.last_kernels() and torch.allclose(got.float(), out.float(), atol=1e-2)
+
+
+def test_no_tables_for_calls_that_do_not_use_them(dev):
+    tokens = 200
+    ri, ro, ci = _arrays(tokens, 30, dev)
+    q, k, v = _operands(dev, 2, tokens, 64, torch.float16)
+    want = sparse_attention(q, k, v, *_arrays(tokens, 30, dev))
+    flat = torch.empty(q.numel() + 1, dtype=q.dtype, device=dev)
+    off = flat[1:].view_as(q)                   # not 16-byte aligned
+    off.copy_(q)
+    for call in (lambda: sparse_attention(off, k, v, ri, ro, ci), lambda: sparse_attention(q.clone().requires_grad_(), k, v, ri, ro, ci),
+                 lambda: sparse_attention(q, k, v, ri, ro, ci, return_probs=True)[0]):
+        assert torch.allclose(call().detach().float(), want.float(), atol=1e-2)
+        assert "_iex_mask_tables" not in ci.__dict__
+
+
 def test_tables_outlive_their_mask_on_another_stream(dev):
     """The mask's tensor goes while a call on another stream has not run yet: its tables' memory is not handed out before."""
     tokens = 1024
