@@ -98,7 +98,7 @@ int iex_csr_dense_share(int itype, int m, int k, int nonzeros, const int* row_of
 size_t iex_csr_dense_share_scratch_bytes(int m, int k);
 
 /* out[i] = values[index[i]] for i < n, elements of elem_bytes (2 or 4) bytes: a CSR matrix' values in the order of its
- * transpose.  Every index must lie in the values. */
+ * transpose (values are n too).  index and out 16-byte aligned.  An index outside [0, n) gives an element of all set bits (NaN). */
 int iex_gather_values(int elem_bytes, int n, const void* values, const long long* index, void* out, void* stream);
 /* dst[0:nbytes] = src[0:nbytes] with a plain 128-bit-per-lane streaming kernel (nbytes and both
  * pointers multiples of 16).  Measurement aid with no counterpart in the reference: hardware

@@ -443,7 +443,7 @@ Tensor spmm_shared(const Tensor& b, const Tensor& row_indices, const Tensor& val
 Tensor permuted(const Tensor& values, const Tensor& perm) {
   const int64_t n = perm.numel();
   if (!plain(values, 1) || !plain(perm, 1) || perm.scalar_type() != at::kLong || values.numel() != n || dtype_code(values.scalar_type()) < 0 ||
-      perm.device() != values.device())
+      perm.device() != values.device() || reinterpret_cast<uintptr_t>(perm.const_data_ptr()) % 16 != 0)
     return values.detach().index_select(0, perm);
   const c10::DeviceGuard guard(values.device());
   Tensor out = at::empty({n}, values.options());

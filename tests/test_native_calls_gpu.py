@@ -55,3 +55,37 @@ def test_notes_follow_the_tensors(dev):
     ci[start] = 256
     with pytest.raises(RuntimeError, match="every column index must lie in"):
         ops.spmm_sputnik_reuse_weight(b, ri, v, ro, ci, 256)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_gather_values_outside_the_values_is_nan(dev, dtype):
+    n = 1027
+    values = torch.randn(n, device=dev).to(dtype)
+    index = torch.randperm(n, device=dev)
+    wrong = [0, 513, 1023, 1024, n - 1]
+    index[wrong] = torch.tensor([n, -1, 1 << 40, -(1 << 62), n + 5], device=dev)
+    out = torch.zeros_like(values)
+    _lib.check(_lib.load().iex_gather_values(values.element_size(), n, values.data_ptr(), index.data_ptr(), out.data_ptr(),
+                                             torch.cuda.current_stream().cuda_stream))
+    good = torch.ones(n, dtype=torch.bool, device=dev)
+    good[wrong] = False
+    assert out[wrong].isnan().all() and torch.equal(out[good], values[index[good]])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_training_step_with_a_permutation_that_is_a_slice(dev, dtype):
+    """The permutation of the transpose as part of a larger tensor: 8-byte aligned only."""
+    from intrasm_engine_amd.pytorch.cpp_extensions.layers_and_funcs.sputnik import spmm
+    from intrasm_engine_amd.pytorch.utils import transpose_info
+    a = W.config2_matrix(0.9, m=300, k=200)
+    ri, v, ro, ci = to_dev(a, dev, dtype)
+    info = transpose_info(300, 200, ro, ci)
+    larger = torch.cat([torch.zeros(1, dtype=torch.int64, device=dev), info[3]])
+    b, grad = torch.randn(200, 17, device=dev).to(dtype), torch.randn(300, 17, device=dev).to(dtype)
+    got = []
+    for perm in (info[3], larger[1:]):
+        b.requires_grad_(), v.requires_grad_()
+        out = spmm(b, ri, v, ro, ci, 300, (*info[:3], perm))
+        got.append(torch.autograd.grad(out, (b, v), grad))
+    assert larger[1:].data_ptr() % 16 == 8
+    assert all(torch.equal(x, y) for x, y in zip(*got))
