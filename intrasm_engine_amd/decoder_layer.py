@@ -16,9 +16,10 @@ Three ways to run the same arithmetic, mirroring how the reference's harness com
   multistream  the batch is split into two halves that are captured on two streams of one
                graph (two branches joined at the end), so the sparse projections of one half
                can overlap the dense attention of the other;
-  fused        the same two halves on one stream; where attention runs as batched GEMMs, each of
-               them is launched together with a sparse projection of the other half through the
-               horizontally fused kernel.
+  fused        the same two halves on one stream; where attention runs as batched GEMMs (heads of
+               other sizes than 64 and 128), each of them is launched together with a sparse
+               projection of the other half through the horizontally fused kernel; where it is one
+               kernel there is nothing to fuse, and the halves run one after the other.
 """
 from __future__ import annotations
 
@@ -43,7 +44,7 @@ class SparseDecoderLayer:
         self.device = device
         # whether the attention kernel serves these heads; the layer then has no dense product of its own, and the steps
         # after its sparse products go into their epilogues
-        self._one_attention = bool(_lib.load().iex_attention_fits(_lib.F16, self.head_dim, 8))
+        self._heads_fit = bool(_lib.load().iex_attention_fits(_lib.F16, self.head_dim, 8))
         self.w = {}
         for name, csr in weights.items():
             idt = index_dtype if csr.k <= 32768 else torch.int32
@@ -61,10 +62,15 @@ class SparseDecoderLayer:
         ri, v, ro, ci, m = self.w[name]
         return ops.spmm_sputnik_reuse_weight_half(x.unsqueeze(0), ri, v, ro, ci, m)[0]
 
+    def _one_attention(self, length: int) -> bool:
+        """Whether ``attention`` over sequences of ``length`` tokens is the one kernel: heads and length that it serves, and no
+        :func:`ops.kernel_params` block that names the kernels of the products it stands for."""
+        return self._heads_fit and not _pyops.kernels_forced() and bool(_lib.load().iex_attention_fits(_lib.F16, self.head_dim, length))
+
     def _proj_with(self, name: str, x: torch.Tensor, other: torch.Tensor, mode: int):
         """``proj`` combined with ``other`` before it is rounded: plus it (mode 1), times its SiLU (mode 2)."""
         ri, v, ro, ci, m = self.w[name]
-        out = _iex_host.spmm_with(x, ri, v, ro, ci, m, other, mode) if self._one_attention else None
+        out = _iex_host.spmm_with(x, ri, v, ro, ci, m, other, mode) if self._heads_fit else None
         if out is None:
             out = self.proj(name, x)
             out = other + out if mode == 1 else torch.nn.functional.silu(other) * out
@@ -97,7 +103,7 @@ class SparseDecoderLayer:
                 self._split_heads(v, seqs))
 
     def attention(self, q, k, v, seqs: int) -> torch.Tensor:
-        out = _iex_host.attention(q, k, v, self.heads, seqs, 1.0 / math.sqrt(self.head_dim)) if self._one_attention else None
+        out = _iex_host.attention(q, k, v, self.heads, seqs, 1.0 / math.sqrt(self.head_dim)) if self._heads_fit else None
         if out is not None:
             return out
         Q, K, V = self._split_qkv(q, k, v, seqs)
@@ -121,9 +127,10 @@ class SparseDecoderLayer:
 
     def forward_fused(self, xa: torch.Tensor, xb: torch.Tensor, seqs_half: int, group=None):
         """Halves a and b of the batch; the dense GEMMs of one half ride along with sparse
-        projections of the other half.  With the attention kernel there are none: one half after the other, ``group``
-        then orders nothing (16 x 512 tokens, hidden 4096: 4.4 ms by fused launches before that kernel, 3.0 now)."""
-        if self._one_attention:
+        projections of the other half, in the order that ``group`` names.  Where attention is one kernel there are none, and
+        the halves go one after the other whatever ``group`` is (16 x 512 tokens, hidden 4096: 4.4 ms by fused launches before
+        that kernel, FUSEDMS now)."""
+        if self._one_attention(xa.shape[1] // seqs_half):
             return self.forward(xa, seqs_half), self.forward(xb, seqs_half)
         qa, ka, va = self.proj("q", xa), self.proj("k", xa), self.proj("v", xa)
         Qa, Ka, Va = self._split_qkv(qa, ka, va, seqs_half)

@@ -65,12 +65,17 @@ def kernel_params(*, spmm: dict | None = None, sddmm: dict | None = None, gemm: 
     for name, given in (("spmm", spmm), ("sddmm", sddmm), ("gemm", gemm)):
         if given is not None:
             setattr(_TUNING, name, given or None)
-    _iex_host.set_forced(bool(_TUNING.__dict__.get("spmm") or _TUNING.__dict__.get("sddmm") or _TUNING.__dict__.get("gemm")))
+    _iex_host.set_forced(kernels_forced())
     try:
         yield
     finally:
         _TUNING.spmm, _TUNING.sddmm, _TUNING.gemm = before["spmm"], before["sddmm"], before["gemm"]
         _iex_host.set_forced(any(before.values()))
+
+
+def kernels_forced() -> bool:
+    """Whether a :func:`kernel_params` block that names a kernel is active on this thread."""
+    return any(getattr(_TUNING, name, None) for name in ("spmm", "sddmm", "gemm"))
 
 
 def _version(t) -> int:
@@ -319,7 +324,7 @@ def prepare_mask(q, row_offsets, column_indices):
     stream capture."""
     tokens, dtype = q.shape[1], q.dtype
     if dtype not in _DT or not q.is_cuda or torch.cuda.is_current_stream_capturing() or \
-            any(getattr(_TUNING, name, None) for name in ("spmm", "sddmm", "gemm")) or \
+            kernels_forced() or \
             not all(t.dtype == torch.int32 and t.dim() == 1 and t.device == q.device and t.is_contiguous() for t in (row_offsets, column_indices)) or \
             row_offsets.numel() != tokens + 1 or not _lib.load().iex_sparse_attention_fits(_DT[dtype], q.shape[2], tokens):
         return False

@@ -88,3 +88,26 @@ def test_three_variants_agree(dev):
     constructor.synchronize()
     assert torch.equal(keep[0], full)
     constructor.destroy_graph_exec()
+
+
+@pytest.mark.parametrize("heads, forced", [(8, False), (HEADS, True)])
+def test_fused_launches_agree_with_the_plain_layer(dev, heads, forced):
+    """Heads of 32 that the attention kernel does not serve, and heads of 64 under a named GEMM tile: the fused schedule
+    launches the attention's products together with projections, four of them, and gives the layer's result."""
+    from intrasm_engine_amd.pytorch import ops as pyops
+    _, weights = _layer(dev)
+    layer = SparseDecoderLayer(weights, HIDDEN, heads, MLP, dev)
+    x = torch.relu(torch.randn(HIDDEN, 2 * L, generator=torch.Generator().manual_seed(2))).half().to(dev)
+    xa, xb = x[:, :L].contiguous(), x[:, L:].contiguous()
+    launches, fused = [], layer._fused
+    layer._fused = lambda name, *args: (launches.append(name), fused(name, *args))[1]
+    with pyops.kernel_params(gemm={"tile": 5} if forced else None):
+        want = layer.forward(xa, 1), layer.forward(xb, 1)
+        for group in (None, 0, 8):
+            got = layer.forward_fused(xa, xb, 1, group)
+            # (one rounding of a residual sum or a gate more or less on either side: a few fp16 units of the largest value)
+            assert all((g.float() - w.float()).abs().max() <= 4 * 2.0 ** -11 * w.float().abs().max() for g, w in zip(got, want)), group
+    assert launches == ["q", "k", "o", "gate"] * 3
+    one = SparseDecoderLayer(weights, HIDDEN, HEADS, MLP, dev)
+    one._fused = None                           # (never called: attention is one kernel)
+    assert all(torch.equal(g, one.forward(h, 1)) for g, h in zip(one.forward_fused(xa, xb, 1), (xa, xb)))
