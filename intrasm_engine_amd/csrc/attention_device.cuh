@@ -130,6 +130,14 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attention_kernel(AttentionPar
   issue(0, 0);
   for (int t = 0; t < tiles; ++t) {
     wait_vmcnt<0>();
+    if (t * kAttnKeys + kAttnKeys > L) {   // (uniform) v of the keys past the end, that a lane has fetched: their weight 0 times a real key's infinity would be NaN
+#pragma unroll
+      for (int i = 0; i < INSTR; ++i) {
+        const int g = wave * INSTR + i, d = g * 8 + row_in;
+        if (t * kAttnKeys + (chunk_in ^ ((d >> 1) & 7)) * 8 >= L)
+          *reinterpret_cast<u32x4*>(smem + (t & 1) * 2 * TILE + TILE + g * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+      }
+    }
     __syncthreads();   // everybody's loads of tile t have landed, and everybody is done with the other stage
     if (t + 1 < tiles) issue(t + 1, (t + 1) & 1);
     const unsigned char* sk = smem + (t & 1) * 2 * TILE;

@@ -39,7 +39,7 @@ def _check(dev, mask, q, k, v, dtype, scale=None):
     endless = np.isinf(want)
     assert np.array_equal(np.isinf(got), endless) and np.array_equal(got[endless], want[endless])
     rest = np.isfinite(want)
-    assert np.linalg.norm((got - want)[rest]) <= TOL[dtype] * np.linalg.norm(want[rest])
+    assert np.linalg.norm(got[rest] - want[rest]) <= TOL[dtype] * np.linalg.norm(want[rest])
     return want
 
 
@@ -94,3 +94,26 @@ def test_infinite_scores(dev, dtype, heads, extra):
     k[:, 100], k[:, 101] = -np.inf, np.inf
     want = _check(dev, mask, q, k, v, dtype)
     assert np.isnan(want[:, [10, 12]]).all() and np.isfinite(want[:, 11]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d, length", [(64, 8), (128, 72), (64, 136), (128, 200), (64, 64)])
+def test_dense_attention_with_infinite_values(dev, dtype, d, length):
+    """Infinities in v show as infinities in their sequence, head and feature, also at the last keys of a length off the tile."""
+    from intrasm_engine_amd import _iex_host
+    heads, seqs, g = 2, 2, torch.Generator(dev).manual_seed(length)
+    q, k, v = (torch.randn(heads * d, seqs * length, device=dev, generator=g).to(dtype) for _ in range(3))
+    v[3, length - 1], v[d + 5, length - 8], v[7, 2 * length - 1] = np.inf, -np.inf, np.nan
+    scale = d ** -0.5
+    out = _iex_host.attention(q, k, v, heads, seqs, scale)
+    assert "attention_kernel" in _lib.last_kernels()
+    split = lambda t: t.double().cpu().view(heads, d, seqs, length).permute(2, 0, 3, 1)
+    Q, K, V = split(q), split(k), split(v)
+    p = torch.softmax(torch.matmul(Q, K.transpose(-1, -2).contiguous()) * scale, dim=-1)
+    want = (p[..., None] * V[:, :, None]).sum(dim=3).permute(1, 3, 0, 2).reshape(heads * d, seqs * length).numpy()
+    got = out.float().cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want).any()
+    endless = np.isinf(want)
+    assert np.array_equal(np.isinf(got), endless) and np.array_equal(got[endless], want[endless]) and endless.any()
+    rest = np.isfinite(want)
+    assert np.linalg.norm(got[rest] - want[rest]) <= TOL[dtype] * np.linalg.norm(want[rest])
