@@ -20,6 +20,7 @@
 // instructions (exponentials at a quarter rate among them) on two wavefronts per SIMD.
 #pragma once
 #include "gemm_dma_device.cuh"
+#include "online_softmax_device.cuh"
 
 namespace iex {
 
@@ -32,23 +33,13 @@ struct AttentionParams {
   float scale_log2;   // scale * log2(e), > 0
 };
 
+// v of keys past a sequence's end: weight 0 times an infinity would be NaN.
+static __device__ __align__(16) const unsigned attention_no_values[4] = {0u, 0u, 0u, 0u};
+
 constexpr int kAttnQ = 128, kAttnKeys = 64, kAttnThreads = 256;
 
 template <int HD>
 constexpr int attention_lds_bytes() { return 2 * 2 * HD * kAttnKeys * 2; }
-
-template <bool BF16>
-__device__ __forceinline__ unsigned pack_16(float a, float b) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  const f2 ab = {a, b};
-  if constexpr (BF16) {
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(ab, b2));
-  } else {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(ab, h2));
-  }
-}
 
 template <bool BF16, int HD>
 __global__ __launch_bounds__(kAttnThreads, 2) void attention_kernel(AttentionParams p) {
@@ -104,7 +95,8 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attention_kernel(AttentionPar
       const int g = wave * INSTR + i, d = g * 8 + row_in;
       const unsigned base = lds0 + stage * 2 * TILE + g * 1024;
       lds_dma16(k + d * T + min(k0 + (chunk_in ^ kn_swizzle<kAttnKeys>(d)) * 8, L - 8), __builtin_amdgcn_readfirstlane(base));
-      lds_dma16(v + d * T + min(k0 + (chunk_in ^ ((d >> 1) & 7)) * 8, L - 8), __builtin_amdgcn_readfirstlane(base + TILE));
+      const int at_v = k0 + (chunk_in ^ ((d >> 1) & 7)) * 8;
+      lds_dma16(at_v < L ? static_cast<const void*>(v + d * T + at_v) : attention_no_values, __builtin_amdgcn_readfirstlane(base + TILE));
     }
   };
   // where a lane's fragments start: k by transpose reads with the middle quads of every 16 keys exchanged, v as 16 bytes
@@ -130,14 +122,6 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attention_kernel(AttentionPar
   issue(0, 0);
   for (int t = 0; t < tiles; ++t) {
     wait_vmcnt<0>();
-    if (t * kAttnKeys + kAttnKeys > L) {   // (uniform) v of the keys past the end, that a lane has fetched: their weight 0 times a real key's infinity would be NaN
-#pragma unroll
-      for (int i = 0; i < INSTR; ++i) {
-        const int g = wave * INSTR + i, d = g * 8 + row_in;
-        if (t * kAttnKeys + (chunk_in ^ ((d >> 1) & 7)) * 8 >= L)
-          *reinterpret_cast<u32x4*>(smem + (t & 1) * 2 * TILE + TILE + g * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
-      }
-    }
     __syncthreads();   // everybody's loads of tile t have landed, and everybody is done with the other stage
     if (t + 1 < tiles) issue(t + 1, (t + 1) & 1);
     const unsigned char* sk = smem + (t & 1) * 2 * TILE;
@@ -159,35 +143,13 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attention_kernel(AttentionPar
         for (int r = 0; r < 16; ++r)
           if (t * kAttnKeys + b * 32 + (r / 8) * 16 + half * 8 + r % 8 >= L) s[b][r] = -INFINITY;
     }
-    float m = s[0][0];
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) m = fmaxf(m, s[b][r]);
-    m = fmaxf(m, __shfl_xor(m, 32));
-    if (__ballot(m > top)) {   // (the first tile always; later ones ever more rarely)
-      const float now = fmaxf(top, m), keep = __builtin_amdgcn_exp2f((top - now) * p.scale_log2);
-      top = now;
-      sum *= keep;
-#pragma unroll
-      for (int d = 0; d < DT; ++d)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[d][r] *= keep;
-    }
-    const float shift = -top * p.scale_log2;
+    softmax_maximum(s, o, top, sum, p.scale_log2);
     u32x4 fp[4];   // the probabilities as MFMA operand: 16 keys each
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        float x[8];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          x[r] = __builtin_amdgcn_exp2f(fmaf(s[b][h * 8 + r], p.scale_log2, shift));
-          sum += x[r];
-        }
-        fp[b * 2 + h] = u32x4{pack_16<BF16>(x[0], x[1]), pack_16<BF16>(x[2], x[3]), pack_16<BF16>(x[4], x[5]), pack_16<BF16>(x[6], x[7])};
-      }
+    for (int e = 0; e < 4; ++e) {
+      softmax_weights<8>(s[e / 2], e % 2 * 8, top, sum, p.scale_log2);
+      fp[e] = probability_operand<BF16>(s[e / 2], e % 2 * 8);
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll

@@ -50,6 +50,20 @@ template <> struct elem<__hip_bfloat16> {
   static __device__ __forceinline__ __hip_bfloat16 from_float(float v) { return __float2bfloat16(v); }
 };
 
+// Two floats rounded to nearest even and packed (a, then b in the upper half): one conversion instruction on this part.
+template <bool BF16>
+__device__ __forceinline__ unsigned pack_pair(float a, float b) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  const f2 ab = {a, b};
+  if constexpr (BF16) {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(ab, b2));
+  } else {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(ab, h2));
+  }
+}
+
 // A VEC-wide register vector of T moved with one load/store instruction.
 template <typename T, int VEC> struct alignas(sizeof(T) * VEC) vec_t { T v[VEC]; };
 

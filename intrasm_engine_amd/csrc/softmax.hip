@@ -59,20 +59,6 @@ __device__ __forceinline__ void softmax_row_in_registers(T* v, int start, int en
   }
 }
 
-// Two floats rounded to nearest even and packed (a, then b in the upper half): one conversion instruction on this part.
-template <typename T>
-__device__ __forceinline__ unsigned pack_pair(float a, float b) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  const f2 ab = {a, b};
-  if constexpr (std::is_same<T, __half>::value) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(ab, h2));
-  } else {
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(ab, b2));
-  }
-}
-
 // 16-bit entries, rows of up to 512 entries: four rows per wavefront, 16 lanes per row, P pairs of neighbouring entries
 // per lane (one 4-byte access at 2-byte alignment each; the pair that would pass the end of the tensor is read one
 // entry earlier).  The one-row-per-wavefront kernel below spends 160 vector instructions per row of 280 entries, most
@@ -116,7 +102,7 @@ __device__ __forceinline__ void softmax_four_rows(T* v, int start, int end, int 
 #pragma unroll
   for (int i = 0; i < P; ++i) {
     const int j = start + (i * 16 + gl) * 2;
-    const unsigned both = pack_pair<T>(x[i][0] * inv, x[i][1] * inv);
+    const unsigned both = pack_pair<std::is_same<T, __hip_bfloat16>::value>(x[i][0] * inv, x[i][1] * inv);
     if (j + 1 < end)
       *reinterpret_cast<u32_a2*>(v + j) = both;
     else if (j < end)

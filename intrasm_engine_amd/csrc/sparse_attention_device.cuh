@@ -20,6 +20,7 @@
 // 512 of MFMAs), for fp32 the MFMAs (4096 clocks per half tile of HD = 64), for scattered entries the way from L2.
 #pragma once
 #include "gemm_dma_device.cuh"
+#include "online_softmax_device.cuh"
 
 namespace iex {
 
@@ -195,19 +196,6 @@ __device__ __forceinline__ void sa_add_row(float* acc, float w, u32x4 chunk) {
   }
 }
 
-template <int TYPE>
-__device__ __forceinline__ unsigned sa_pack(float a, float b) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  const f2 ab = {a, b};
-  if constexpr (TYPE == 1) {
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(ab, b2));
-  } else {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(ab, h2));
-  }
-}
-
 template <int TYPE, int HD, int QW, int KW>
 __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attention_kernel(SparseAttentionParams p) {
   typedef SparseAttentionShape<TYPE, HD> Shape;
@@ -315,29 +303,9 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
         }
       }
     }
-    float m = s[0][0];
+    softmax_maximum(s, o, top, sum, p.scale_log2);
 #pragma unroll
-    for (int b = 0; b < KB; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) m = fmaxf(m, s[b][r]);
-    m = fmaxf(m, __shfl_xor(m, 32));
-    if (__ballot(m > top)) {   // (the first tile always; later ones ever more rarely)
-      const float now = fmaxf(top, m), keep = __builtin_amdgcn_exp2f((top - now) * p.scale_log2);
-      top = now;
-      sum *= keep;
-#pragma unroll
-      for (int d = 0; d < DT; ++d)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[d][r] *= keep;
-    }
-    const float shift = -top * p.scale_log2;
-#pragma unroll
-    for (int b = 0; b < KB; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        s[b][r] = __builtin_amdgcn_exp2f(fmaf(s[b][r], p.scale_log2, shift));   // (exp2(-infinity) = 0)
-        sum += s[b][r];
-      }
+    for (int b = 0; b < KB; ++b) softmax_weights<16>(s[b], 0, top, sum, p.scale_log2);
     // ---- times V: rows = features
     if constexpr (F32) {
 #pragma unroll
@@ -353,10 +321,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
     } else {
 #pragma unroll
       for (int e = 0; e < KEYS / 16; ++e) {
-        const f32x16& x = s[e / 2];
-        const int r0 = e % 2 * 8;
-        const u32x4 fp = {sa_pack<TYPE>(x[r0], x[r0 + 1]), sa_pack<TYPE>(x[r0 + 2], x[r0 + 3]), sa_pack<TYPE>(x[r0 + 4], x[r0 + 5]),
-                          sa_pack<TYPE>(x[r0 + 6], x[r0 + 7])};
+        const u32x4 fp = probability_operand<TYPE == 1>(s[e / 2], e % 2 * 8);
         const int kr = half * 8 + ((lane & 15) >> 2);
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
@@ -591,7 +556,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
         const float x0 = o[d][g * 4] * inv, x1 = o[d][g * 4 + 1] * inv, x2 = o[d][g * 4 + 2] * inv, x3 = o[d][g * 4 + 3] * inv;
         unsigned char* there = to + (d * 32 + g * 8 + half * 4) * ES;
         if constexpr (F32) *reinterpret_cast<f32x4*>(there) = f32x4{x0, x1, x2, x3};
-        else *reinterpret_cast<u32x2*>(there) = u32x2{sa_pack<TYPE>(x0, x1), sa_pack<TYPE>(x2, x3)};
+        else *reinterpret_cast<u32x2*>(there) = u32x2{pack_pair<TYPE == 1>(x0, x1), pack_pair<TYPE == 1>(x2, x3)};
       }
   }
 }
