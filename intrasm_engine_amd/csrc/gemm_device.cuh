@@ -1,5 +1,7 @@
 // Dense companion GEMM for gfx950: C = A * B (or A * B^T), fp16 / bf16 in, fp32
-// accumulate on the matrix cores (v_mfma_f32_32x32x16_{f16,bf16}), LDS double-buffered.
+// accumulate on the matrix cores, LDS double-buffered.  Here: what the GEMM kernels share (the matrix-core forms, their
+// accumulators, the epilogue), and the tile whose operands travel through registers (tile codes 1 - 4, v_mfma_f32_32x32x16);
+// the tiles that are chosen are those of gemm_dma_device.cuh and gemm_pp_device.cuh (v_mfma_f32_16x16x32).
 //
 // Tiling: a workgroup of 2 x WCN wavefronts (WCN = 2, or 4 for the 512-thread workgroups of
 // the fused launch) owns a (2*WM*32) x (WCN*WN*32) tile of C; a wavefront owns WM x WN MFMA
@@ -96,8 +98,8 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(u32x4 a, u32x4 b, f32x16 c) {
   }
 }
 
-// Half the accumulator traffic per flop of the 32 x 32 form: under the power limit random operands run at 2100 instead of
-// 1875 TFLOP/s (a loop of MFMAs and nothing else, every CU; all-zero operands 2440 / 2470).
+// Half the accumulator traffic per flop of the 32 x 32 form: under the power limit random operands run at 1930 instead of
+// 1710 TFLOP/s, all-zero ones at 2430 / 2460 (benchmarks/mfma_rates.hip: MFMAs and nothing else on every CU).
 template <bool BF16>
 __device__ __forceinline__ f32x4 mfma_16x16x32(u32x4 a, u32x4 b, f32x4 c) {
   if constexpr (BF16) {

@@ -16,9 +16,11 @@
 // Intervals are separated by workgroup barriers, so on every SIMD one wavefront feeds the matrix cores while
 // the other one waits for LDS and issues loads, and all waits hide behind the other group's MFMAs.
 // A wavefront owns WM x WN blocks of 32 x 32 (128 x 64 of a 256 x 256 tile with WM = 4, WN = 2, WCN = 4).
-// What bounds it (8192^3, bf16, TFLOP/s): 1440 as it is, 1650 without the loads, 1540 with fragments read once, 1760 with
-// neither (MFMAs and barriers; MFMAs alone run at 2100, the card's power limit on random operands).  One barrier per phase
-// instead of strict alternation: 1315; loads before the fragment reads: the same; multiplying at raised priority: 1-2 % slower.
+// What bounds it (8192^3, bf16): the matrix cores are busy 78 % of the cycles, at the 1.64 GHz that the card's power limit leaves
+// them on random operands (MFMAs and nothing else: 1930 TFLOP/s); 14 % of the wavefronts' time is waiting, LDS is in use 31 %.
+// One round of 128 x 256 tiles: busy 46 % at 2.25 GHz, a workgroup's only tile being mostly prologue and epilogue.
+// (profiles/kernel_counters_of_the_cases.txt.)  One barrier per phase instead of strict alternation: 1315 TFLOP/s for 1440;
+// loads before the fragment reads: the same; multiplying at raised priority: 1-2 % slower.
 //
 // Stage reuse: what phase p reads was last needed by phase p (group 1 reads it one interval after group 0), and the
 // loads that overwrite it go out in later M phases.  A wavefront waits for its own loads of what phase p + 1 reads at

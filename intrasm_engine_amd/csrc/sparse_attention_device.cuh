@@ -16,8 +16,10 @@
 //     O^T += V^T P^T with the probabilities as they lie in the lanes.  fp32 goes by v_mfma_f32_32x32x2, tiles in halves.
 //   * other entries: HD * size / 16 lanes per row walk the row's list, 4 or 8 entries at a time, 16 bytes of each K and V
 //     row per lane, dot products across the lanes, a softmax state per row; rows' results meet the dense part's in LDS.
-// What bounds it: for 16-bit types the vector instructions of the softmax (about 1100 clocks per wavefront and tile beside
-// 512 of MFMAs), for fp32 the MFMAs (4096 clocks per half tile of HD = 64), for scattered entries the way from L2.
+// What bounds it (profiles/kernel_counters_of_the_cases.txt): for 16-bit types vector instructions, 270 - 300 per wavefront and
+// tile for the softmax (1100 - 1200 clocks beside 512 of MFMAs) and 4 per scattered entry, on the two wavefronts per SIMD that
+// LDS leaves room for; a short prompt is the chain of a wavefront's few tiles (59 % waiting); for fp32 the MFMAs (4096 clocks
+// per half tile of HD = 64; busy 60 %).
 #pragma once
 #include "gemm_dma_device.cuh"
 #include "online_softmax_device.cuh"
