@@ -420,7 +420,7 @@ int iex_gemm(int dtype, int trans_b, int M, int N, int K, const void* A, const v
 
 /* iex_gemm with a workspace in device memory that the call may use (and overwrite) until the work it
  * puts on `stream` has run.  Used by the kernels that split K over several workgroups per tile.
- * Shape code 14 (bits 4..7 of trans_b): 64 x 128 tiles with K in two to eight parts, which the library also picks by
+ * Shape code 14 (bits 4..8 of trans_b): 64 x 128 tiles with K in two to eight parts, which the library also picks by
  * itself for products with few tiles and a long K (64 tiles or fewer, or 128 or fewer and K >= 4096; every part at
  * least 1024 of K; as many parts as give every CU a workgroup: 4096 x 128 x 4096 23.8 -> 17.1 us in 4 parts, 512 x 512 x
  * 8192 42.5 -> 17.6 us in 8).  Every workgroup leaves its fp32 partial sums in the workspace and draws a ticket; the one
