@@ -111,3 +111,13 @@ def test_fused_launches_agree_with_the_plain_layer(dev, heads, forced):
     one = SparseDecoderLayer(weights, HIDDEN, HEADS, MLP, dev)
     one._fused = None                           # (never called: attention is one kernel)
     assert all(torch.equal(g, one.forward(h, 1)) for g, h in zip(one.forward_fused(xa, xb, 1), (xa, xb)))
+
+
+def test_lengths_off_eight_are_refused_by_every_schedule(dev):
+    """The attention kernel steps aside for them, and so do the products it would fall back to (their inner dimension)."""
+    layer, _ = _layer(dev)
+    x = torch.relu(torch.randn(HIDDEN, 2 * 12, generator=torch.Generator().manual_seed(3))).half().to(dev)
+    xa, xb = x[:, :12].contiguous(), x[:, 12:].contiguous()
+    for call in (lambda: layer.forward(x, 2), lambda: layer.forward_fused(xa, xb, 1)):
+        with pytest.raises(RuntimeError, match="multiple of 8"):
+            call()
