@@ -34,7 +34,7 @@ struct GemmParams {
   long long stride_a, stride_b, stride_c;
   int tiles_m, tiles_n;
   // epilogue beyond C = A * B: C = relu?(A * B + row_bias[row]), then with an auxiliary operand of C's shape and strides
-  // (16-byte aligned where C is; it may be C itself) C = that + aux (kGemmAdd) or C = that * silu(aux) (kGemmTimesSilu)
+  // (any alignment; it may be C itself) C = that + aux (kGemmAdd) or C = that * silu(aux) (kGemmTimesSilu)
   const float* row_bias = nullptr;
   int relu = 0;
   int aux_mode = 0;
@@ -270,6 +270,7 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const Acc& 
   // the auxiliary operand of the whole tile, all loads in flight together (the fragments' registers are free by now)
   u32x4 held[WM][32 / RPI];
   if (aux) {
+    const bool whole_aux = whole && (reinterpret_cast<uintptr_t>(aux) & 15) == 0;   // (uniform)
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -277,7 +278,7 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const Acc& 
         const u16* src = aux + (size_t)min(m0 + (wm * WM + i) * 32 + t * RPI + lane / CPR, p.M - 1) * ldc + gn;
         held[i][t] = u32x4{0u, 0u, 0u, 0u};
         if (here == 8) {
-          held[i][t] = whole ? *reinterpret_cast<const u32x4*>(src) : *reinterpret_cast<const u128_a2*>(src);
+          held[i][t] = whole_aux ? *reinterpret_cast<const u32x4*>(src) : *reinterpret_cast<const u128_a2*>(src);
         } else {
           unsigned w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll

@@ -53,3 +53,20 @@ def test_product_with_an_auxiliary_operand(oracle, dev, dtype, m, k, n, dense):
         assert ("combine_kernel" in _lib.last_kernels()) != ("csr_to_dense_kernel" in _lib.last_kernels())
         # (without an epilogue of its own the product is rounded before it is combined: twice the type's half step)
         assert_close(got.float().cpu().numpy(), want, 5 * bound, RTOL[dtype], f"mode {mode}")
+
+
+@pytest.mark.parametrize("offset", [1, 2, 4])
+def test_auxiliary_operand_at_any_alignment(dev, offset):
+    """The other operand as a slice that starts 2, 4 or 8 bytes past an aligned address: the same bits as from a copy of it."""
+    m, k, n = 640, 512, 264
+    ro, ci = W.csr_from_row_lengths(np.random.default_rng(1), m, k, np.full(m, k // 2))
+    csr = W.CSR(m, k, np.random.default_rng(2).standard_normal(ci.shape[0]).astype(np.float32), W.swizzle_from_offsets(ro), ro, ci)
+    ri, v, ro, ci = to_dev(csr, dev, torch.float16)
+    x = torch.randn(k, n, device=dev).half()
+    flat = torch.randn(m * n + 8, device=dev).half()
+    aux = flat[offset:offset + m * n].view(m, n)
+    assert aux.data_ptr() % 16 == 2 * offset
+    for mode in (1, 2):
+        got = _iex_host.spmm_with(x, ri, v, ro, ci, m, aux, mode)
+        assert "csr_to_dense_kernel" in _lib.last_kernels()
+        assert torch.equal(got, _iex_host.spmm_with(x, ri, v, ro, ci, m, aux.clone(), mode))
