@@ -24,6 +24,13 @@ class TorchCUDAGraphConstructor:
         self.notifier = iex.CUDAGraphCaptureNotifier()
         self.constructor = iex.CUDAExperimentalGraphConstructor()
         self.constructor.register_stream(self.registeredStreams[0].handle)
+        self._kept: list[torch.Tensor] = []
+
+    def keep(self, *tensors: torch.Tensor) -> None:
+        """What recorded kernels read at every replay lives as long as the constructor: copies, transposes and gathered
+        values are made outside the capture, and the allocator would hand their memory to the next allocation while the
+        graph still reads it.  (Detached: a kept tensor must not keep the autograd node that keeps the constructor.)"""
+        self._kept.extend(t.detach() for t in tensors)
 
     def get_primary_stream(self) -> CompoundStream:
         """The first stream: where streams join and where the graph is executed."""

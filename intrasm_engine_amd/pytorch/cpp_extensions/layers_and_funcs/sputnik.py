@@ -155,7 +155,8 @@ class MySpMM(MyAutogradFunc):
         k = b3.shape[1]
         if _transp_info is None:
             _transp_info = transpose_info(int(m), k, row_offsets, column_indices)
-        with maybe_captured(kwargs["constructor"], kwargs["constructor_enabled"], kwargs["stream_beg"]):
+        with maybe_captured(kwargs["constructor"], kwargs["constructor_enabled"], kwargs["stream_beg"],
+                            reads=(b3, row_indices, values, row_offsets, column_indices)):
             out = _spmm(b3, row_indices, values, row_offsets, column_indices, int(m), params.get("spmm_kernel", "auto"))
         ctx_dict = {"m": int(m), "k": k, "backward_constructor": kwargs["backward_constructor"],
                     "constructor_enabled": kwargs["constructor_enabled"] and kwargs["backward_constructor"] is not None,
@@ -172,12 +173,14 @@ class MySpMM(MyAutogradFunc):
         ci32 = column_indices if column_indices.dtype == torch.int32 else _ops.carry_pattern_note(column_indices, column_indices.to(torch.int32))
         if needs_input_grad[2]:
             # lhs = grad (m, tokens), rhs = b (k, tokens): rhs rows are indexed by the CSR column
-            with maybe_captured(backward_constructor, constructor_enabled, stream_beg):
+            with maybe_captured(backward_constructor, constructor_enabled, stream_beg,
+                                reads=(grad3, b3, row_indices, row_offsets, ci32)):
                 grad_sparse = _sddmm(grad3, b3, row_indices, row_offsets, ci32, params.get("grad_values_wpr", 0))
         if needs_input_grad[0]:
             # gather outside the capture zone, as the reference notes for its transposes (:93-95)
             _, values_t, _, _ = _transpose_with_info(values, (row_indices_t, row_offsets_t, column_indices_t, perm))
-            with maybe_captured(backward_constructor, constructor_enabled, stream_beg):
+            with maybe_captured(backward_constructor, constructor_enabled, stream_beg,
+                                reads=(grad3, row_indices_t, values_t, row_offsets_t, column_indices_t)):
                 grad_dense = _spmm(grad3, row_indices_t, values_t, row_offsets_t, column_indices_t, k,
                                    params.get("grad_dense_kernel", "auto")).squeeze(0)
         return grad_dense, None, grad_sparse, None, None, None, None

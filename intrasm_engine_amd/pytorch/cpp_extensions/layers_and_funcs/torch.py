@@ -67,7 +67,7 @@ class MyLinear(MyAutogradFunc):
         params = kwargs.get("params") or {}
         input = input.contiguous()
         weight = weight.contiguous()
-        with maybe_captured(kwargs["constructor"], kwargs["constructor_enabled"], kwargs["stream_beg"]):
+        with maybe_captured(kwargs["constructor"], kwargs["constructor_enabled"], kwargs["stream_beg"], reads=(input, weight)):
             output = _gemm(input, weight, True, params.get("gemm_tile", "auto"))
         ctx_dict = {"backward_constructor": kwargs["backward_constructor"],
                     "constructor_enabled": kwargs["constructor_enabled"] and kwargs["backward_constructor"] is not None,
@@ -80,11 +80,11 @@ class MyLinear(MyAutogradFunc):
         grad_output = grad_output.contiguous()
         grad_input = grad_weight = None
         if needs_input_grad[0]:
-            with maybe_captured(backward_constructor, constructor_enabled, stream_beg):
+            with maybe_captured(backward_constructor, constructor_enabled, stream_beg, reads=(grad_output, weight)):
                 grad_input = _gemm(grad_output, weight, False, params.get("grad_input_tile", "auto"))
         if needs_input_grad[1]:
             go_t = grad_output.t().contiguous()          # outside the capture zone
-            with maybe_captured(backward_constructor, constructor_enabled, stream_beg):
+            with maybe_captured(backward_constructor, constructor_enabled, stream_beg, reads=(go_t, input)):
                 grad_weight = _gemm(go_t, input, False, params.get("grad_weight_tile", "auto"))
         return grad_input, grad_weight
 

@@ -78,12 +78,14 @@ def runs_plainly(fwd_kwargs: dict | None) -> bool:
 
 
 @contextlib.contextmanager
-def maybe_captured(constructor, enabled: bool, stream_beg: int):
+def maybe_captured(constructor, enabled: bool, stream_beg: int, reads=()):
     """Run the body on registered stream ``stream_beg`` of ``constructor`` inside a
-    ``capture_library_call_begin/end`` pair, or plainly when capture is off."""
+    ``capture_library_call_begin/end`` pair, or plainly when capture is off.  ``reads``: the tensors that
+    the recorded kernels will read at every replay; the constructor keeps them."""
     if not enabled or constructor is None:
         yield
         return
+    constructor.keep(*reads)
     with constructor.registeredStreams[stream_beg]:
         constructor.capture_library_call_begin()
         try:

@@ -109,6 +109,36 @@ def test_pair_recorded_as_parallel_branches(dev):
     bwd.destroy_graph_exec()
 
 
+@pytest.mark.parametrize("index", [torch.int32, torch.int16])
+def test_recorded_kernels_keep_what_they_read(dev, index):
+    """The gathered values, the transposed gradient and the converted indices of a recorded backward pass are made outside
+    the capture: memory that the allocator hands out between recording and replay is not theirs."""
+    case = _Case(dev, seed=7)
+    _, want_grads = case.one_by_one()
+    pair = make_kernel_pair_or_triple_autograd_function(MySpMM, MyLinear)
+    bwd = TorchCUDAGraphConstructor()
+    fwd = TorchCUDAGraphConstructor()
+    bwd.register_new_stream()
+    fwd.register_new_stream()
+    opts = {f"fwd_kwargs_{i + 1}": {"constructor": fwd, "backward_constructor": bwd, "constructor_enabled": True,
+                                    "stream_beg": i} for i in range(2)}
+    b, v, x, w = case.leaves()
+    case.ci = U.to_int16_indices(case.ci, case.a.k) if index == torch.int16 else case.ci
+    y1, y2 = pair.apply(opts, *case.spmm_inputs(b, v), x, w)
+    torch.autograd.backward([y1, y2], [case.g_sparse, case.g_dense])
+    del y1, y2
+    other = [torch.ones(size, device=dev) for size in (1, 2048, 8192, 16384) for _ in range(64)]
+    for t in other:
+        t.zero_()
+    bwd.instantiate_graph_exec()
+    for _ in range(3):
+        bwd.execute_graph()
+        bwd.synchronize()
+        for got, want in zip((b.grad, v.grad, x.grad, w.grad), want_grads):
+            assert torch.equal(got, want)
+    bwd.destroy_graph_exec()
+
+
 def test_triple_node(dev):
     case, other = _Case(dev, seed=5), _Case(dev, seed=6)
     want_out, want_grads = case.one_by_one()
