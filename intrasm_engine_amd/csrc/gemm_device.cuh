@@ -252,6 +252,76 @@ struct GemmStage {
 template <int WN>
 constexpr int gemm_store_lds_bytes() { return 32 * (WN * 64 + 16); }
 
+// Two sums as one word of the 16-bit type.
+template <bool BF16>
+__device__ __forceinline__ unsigned pack_16(float x, float y) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  if constexpr (BF16) return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x, y}), bf16x2));
+  else return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x, y}), f16x2));
+}
+template <bool BF16>
+__device__ __forceinline__ void unpack_16(unsigned w, float& x, float& y) {
+  if constexpr (BF16) {
+    x = __uint_as_float(w << 16);
+    y = __uint_as_float(w & 0xffff0000u);
+  } else {
+    x = (float)__builtin_bit_cast(_Float16, (unsigned short)(w & 0xffffu));
+    y = (float)__builtin_bit_cast(_Float16, (unsigned short)(w >> 16));
+  }
+}
+
+// The plain case of gemm_store_tile below: rows of whole 16-byte vectors, no row bias, no ReLU; AUX = its aux_mode (0: none).  Without a branch:
+// stores are buffer stores, which drop what lies outside C (a lane whose row or column does not exist asks for the buffer's end).
+// That is what an epilogue costs: its instructions run once per tile, out of a cold instruction cache, and the general code below
+// is 60 KB of them for a 128 x 64 wavefront tile (one 256 x 256 tile and nothing else: 12.4 us, 4.8 without its epilogue, 8.0 with this one).
+template <bool BF16, int WM, int WN, int AUX, bool STREAM, typename Acc>
+__device__ __forceinline__ void gemm_store_whole(const GemmParams& p, const Acc& acc, unsigned short* C, const unsigned short* aux, int m0, int n0, int wm,
+                                                 int wn, int lane, unsigned char* lds) {
+  constexpr int ROWB = WN * 64 + 16, CPR = WN * 4, RPI = kWave / CPR;   // as below
+  const int ldc = p.ldc ? p.ldc : p.N;
+  const int chunk = lane % CPR, first = m0 + wm * WM * 32 + lane / CPR, gn = n0 + wn * WN * 32 + chunk * 8;
+  const unsigned bytes = ((unsigned)(p.M - 1) * ldc + p.N) * 2u;   // (below 2^32: the host's limits)
+  const auto c_buf = __builtin_amdgcn_make_buffer_rsrc(C, 0, bytes, 4 << 15);
+  const auto aux_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(AUX ? aux : C), 0, bytes, 4 << 15);
+  auto at = [&](int i, int t) {
+    const int row = first + i * 32 + t * RPI;
+    return row < p.M && gn < p.N ? ((unsigned)row * ldc + gn) * 2u : 0xfffffff0u;
+  };
+  u32x4 held[WM][32 / RPI];
+  if constexpr (AUX != 0) {   // all of the tile's in flight together
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int t = 0; t < 32 / RPI; ++t) held[i][t] = __builtin_amdgcn_raw_buffer_load_b128(aux_buf, at(i, t), 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < WM; ++i) {
+    if constexpr (AUX != 0) {
+#pragma unroll
+      for (int t = 0; t < 32 / RPI; ++t) *reinterpret_cast<u32x4*>(lds + (t * RPI + lane / CPR) * ROWB + chunk * 16) = held[i][t];
+    }
+#pragma unroll
+    for (int t = 0; t < 4 * WN; ++t) {
+      u32x2* to = reinterpret_cast<u32x2*>(lds + Acc::row(t, lane) * ROWB + Acc::col(t, lane) * 2);
+      f32x4 y = acc.quad(i, t);
+      if constexpr (AUX != 0) {
+        const u32x2 w = *to;
+        float other[4];
+        unpack_16<BF16>(w.x, other[0], other[1]);
+        unpack_16<BF16>(w.y, other[2], other[3]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = AUX == kGemmAdd ? y[e] + other[e] : y[e] * (other[e] / (1.f + __expf(-other[e])));
+      }
+      *to = u32x2{pack_16<BF16>(y[0], y[1]), pack_16<BF16>(y[2], y[3])};
+    }
+#pragma unroll
+    for (int t = 0; t < 32 / RPI; ++t)
+      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4*>(lds + (t * RPI + lane / CPR) * ROWB + chunk * 16), c_buf, at(i, t), 0, STREAM ? 2 : 0);
+  }
+}
+
 template <bool BF16, int WM, int WN, typename Acc>
 __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const Acc& acc, unsigned short* __restrict__ C,
                                                 const unsigned short* aux, int m0, int n0, int wm, int wn, int lane, unsigned char* lds,
@@ -263,6 +333,20 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, const Acc& 
   constexpr int RPI = kWave / CPR;     // rows a store instruction covers
   static_assert(kWave % CPR == 0 && 32 % RPI == 0, "whole rows per instruction");
   const int ldc = p.ldc ? p.ldc : p.N;
+  // rows of whole vectors and nothing but an auxiliary operand to do (uniform)
+  if (p.N % 8 == 0 && ldc % 8 == 0 && ((reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(aux)) & 15) == 0 && !p.row_bias && !p.relu && !partial &&
+      (long long)(p.M + 256) * ldc < (1ll << 31)) {
+    const int mode = aux ? p.aux_mode : 0;
+    auto store = [&](auto m, auto s) { gemm_store_whole<BF16, WM, WN, decltype(m)::value, decltype(s)::value>(p, acc, C, aux, m0, n0, wm, wn, lane, lds); };
+    auto by_mode = [&](auto s) {
+      if (mode == 0) store(std::integral_constant<int, 0>{}, s);
+      else if (mode == kGemmAdd) store(std::integral_constant<int, kGemmAdd>{}, s);
+      else store(std::integral_constant<int, kGemmTimesSilu>{}, s);
+    };
+    if (stream) by_mode(std::true_type{});
+    else by_mode(std::false_type{});
+    return;
+  }
   const int chunk = lane % CPR;
   const int gn = n0 + wn * WN * 32 + chunk * 8;
   const int here = min(p.N - gn, 8);   // columns of this lane's chunk that exist (none: <= 0)

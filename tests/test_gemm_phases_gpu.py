@@ -28,3 +28,24 @@ def test_layouts_at_the_edges_of_the_stages(oracle, dev, dtype, layout, tile, mn
     assert rc == 0, _lib.last_error()
     a_r, b_r = rounded(a_np, dtype), rounded(b_np, dtype)
     assert_close(out.float().cpu().numpy(), oracle.gemm(a_r, b_r), oracle.gemm(np.abs(a_r), np.abs(b_r)), 1e-2, f"tile {tile} layout {layout} {mnk}")
+
+
+@pytest.mark.parametrize("tile", [5, 9, 13, 15, 16])
+@pytest.mark.parametrize("M,N", [(255, 256), (257, 248), (193, 264), (1, 8), (256, 512)])
+def test_stores_end_where_the_output_does(oracle, dev, tile, M, N):
+    """Rows of whole vectors are stored without branches, by buffer stores that drop what lies outside: every entry of both batch
+    entries is written and nothing around them."""
+    rng = np.random.default_rng(M + N)
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((2, M, 72), (2, 72, N)))
+    at, bt = (torch.from_numpy(x).to(dev).bfloat16() for x in (a, b))
+    around = torch.full((4 * 256 * 512 + 2 * M * N,), 7.0, dtype=torch.bfloat16, device=dev)
+    out = around[2 * 256 * 512:][:2 * M * N].view(2, M, N)
+    out.fill_(float("nan"))
+    lib = _lib.load()
+    _lib.check(lib.iex_gemm(_lib.BF16, tile << 4, M, N, 72, at.data_ptr(), bt.data_ptr(), out.data_ptr(), 2, M * 72, 72 * N, M * N,
+                            torch.cuda.current_stream().cuda_stream))
+    for z in range(2):
+        ar, br = rounded(a[z], torch.bfloat16), rounded(b[z], torch.bfloat16)
+        assert_close(out[z].float().cpu().numpy(), oracle.gemm(ar, br), np.abs(ar) @ np.abs(br), RTOL[torch.bfloat16], f"{M} x {N} tile {tile}")
+    rest = torch.cat([around[:2 * 256 * 512], around[2 * 256 * 512 + 2 * M * N:]])
+    assert bool((rest == 7.0).all())
