@@ -3,7 +3,8 @@ import numpy as np
 import pytest
 import torch
 
-from _util import assert_close, rounded
+from intrasm_engine_amd import _lib
+from _util import RTOL, assert_close, rounded
 
 pytestmark = pytest.mark.gpu
 
