@@ -258,6 +258,35 @@ size_t iex_spmm_transposed_workspace_bytes(int dtype, int m, int k, int n, int n
 int iex_spmm_transposed(int dtype, int itype, int m, int k, int n, int nonzeros, const void* values, const int* row_offsets,
                         const void* column_indices, const void* dense, void* out, void* stream, void* workspace, size_t workspace_bytes);
 
+/* A sparse 16-bit weight laid out once, for a program that keeps it and multiplies it again and again (out (m x n) = A * dense
+ * (k x n), row-major): the products then launch one kernel and read no CSR array.  No counterpart in the reference, whose kernels read the
+ * CSR arrays in every call.  A form is memory of the caller's, 256-byte aligned, of one kind:
+ *   0              A's dense form (m rows of round8(k)), multiplied by the dense GEMM;
+ *   128, 192, 256  two-of-four: the first two entries of every four neighbouring columns with two index bits each, multiplied by
+ *                  the structured-sparsity matrix instructions at twice the dense rate, in tiles of that many rows; entries
+ *                  beyond them ("spilled") as a narrow dense operand of the columns that have any, per half tile.  k <= 65536.
+ * The CSR must be canonical (rows' columns ascend strictly).  What was laid out stands for A's values at that time.
+ *   iex_form_measure  adds to spill_phases (device memory, six ints that the caller has set to 0) the phases of 32 spilled columns of all
+ *                     blocks of 64 / 96 / 128 rows (half tiles of kinds 128 / 192 / 256), and takes the largest of any block:
+ *                     0 0 0 0 0 0 for a 2:4 weight.  scratch: iex_form_scratch_bytes, 16-byte aligned.
+ *   iex_form_bytes    for a two-of-four form with room for `spill_phases` phases per half tile, the measured maximum (0: no such form)
+ *   iex_form_build    needs the scratch memory for the two-of-four kinds; at least three nonzeros, fewer than 2^29.
+ *   iex_form_choose   which of `kinds` (bit 0: kind 0, bits 1, 2, 3: kinds 128, 192, 256) is estimated fastest for n columns (host code;
+ *                     spill_phases: the first three measured numbers, host memory), -1 where a SpMM that reads the CSR arrays is.
+ *   iex_form_product  aux / aux_mode as in iex_spmm_aux (aux NULL: none).  n a multiple of 8, dense 16-byte aligned; workspace
+ *                     (256-byte aligned, iex_form_product_workspace_bytes, may be NULL) lets the dense product take K in parts.
+ *                     Non-finite entries of dense rows that A does not reference may reach the output, as with the dense form. */
+size_t iex_form_scratch_bytes(int m, int k);
+int iex_form_measure(int itype, int m, int k, int nonzeros, const int* row_offsets, const void* column_indices, void* scratch, size_t scratch_bytes,
+                     int* spill_phases, void* stream);
+size_t iex_form_bytes(int kind, int m, int k, int spill_phases);
+int iex_form_build(int itype, int kind, int m, int k, int nonzeros, const int* row_offsets, const void* column_indices, const void* values,
+                   int spill_phases, void* form, size_t form_bytes, void* scratch, size_t scratch_bytes, void* stream);
+int iex_form_choose(int kinds, int m, int k, int n, int nonzeros, const int* spill_phases);
+size_t iex_form_product_workspace_bytes(int kind, int m, int k, int n);
+int iex_form_product(int dtype, int kind, int m, int k, int n, int spill_phases, const void* form, const void* dense, const void* aux, int aux_mode,
+                     void* out, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Drop-ins for the three launchers the reference declares in csrc/extensions.h:28-30.  Like the reference's they accept
  * column indices in any order inside a row, and duplicates (IEX_SPMM_ANY_COLUMN_ORDER is always set: the row kernel,
  * or the few-columns kernel); a caller that knows its CSR arrays to be canonical gets every family from iex_spmm_ex.

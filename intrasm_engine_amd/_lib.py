@@ -58,6 +58,13 @@ SIGNATURES = {
     "iex_CudaSpmm2": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "iex_CudaSpmm3": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "iex_CudaSpmm5": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i]),
+    "iex_form_scratch_bytes": (_c.c_size_t, [_i, _i]),
+    "iex_form_measure": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _c.c_size_t, _vp, _vp]),
+    "iex_form_bytes": (_c.c_size_t, [_i, _i, _i, _i]),
+    "iex_form_build": (_i, [_i, _i, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _c.c_size_t, _vp, _c.c_size_t, _vp]),
+    "iex_form_choose": (_i, [_i, _i, _i, _i, _i, _vp]),
+    "iex_form_product_workspace_bytes": (_c.c_size_t, [_i, _i, _i, _i]),
+    "iex_form_product": (_i, [_i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _c.c_size_t, _vp]),
     "iex_csr_check": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "iex_sddmm_ex": (_i, [_i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "iex_sddmm_ws": (_i, [_i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _c.c_size_t]),

@@ -243,6 +243,12 @@ inline bool auto_split_wanted(int M, int N, int K, int batch) {
   return split_parts_for(M, N, K, batch, 64, 128, 64) >= 2;
 }
 
+// What a tile shape takes, per K and in units of 1 / rate: whole rounds of `slots` workgroups, the last one by the share that works (see launch_shape).
+inline double tile_cost(int M, int N, int batch, int bm, int bn, int slots, double rate) {
+  const long long tiles = (long long)ceil_div(M, bm) * ceil_div(N, bn) * batch, full = tiles / slots, rest = tiles % slots;
+  return ((double)full + (rest ? 0.65 + 0.35 * rest / slots : 0.0)) * slots * bm * bn / rate;
+}
+
 template <bool BF16, bool TRANS_A, bool TRANS_B>
 int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, void* ws, size_t ws_bytes, bool flags_are_zero) {
   if constexpr (!TRANS_A) {   // kernels that are never chosen, or not for A as (K, M)
@@ -297,10 +303,7 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
     // (128 x 128 and 64 x 128 in alternating phases: no faster than codes 8 and 9.)
     // A last round with a share f of the CUs at work takes 0.65 + 0.35 f of a full one: those that work have the way from L2
     // and the power to themselves (11008 x 2048 x 4096, 1.34 rounds of 256 x 256: 175 against 195 for 2.69 of 128 x 256).
-    auto cost = [&](int bm, int bn, int slots, double rate) {
-      const long long tiles = (long long)ceil_div(p.M, bm) * ceil_div(p.N, bn) * batch, full = tiles / slots, rest = tiles % slots;
-      return ((double)full + (rest ? 0.65 + 0.35 * rest / slots : 0.0)) * slots * bm * bn / rate;
-    };
+    auto cost = [&](int bm, int bn, int slots, double rate) { return tile_cost(p.M, p.N, batch, bm, bn, slots, rate); };
     const double huge = cost(256, 256, 256, TRANS_A ? 1385.0 : TRANS_B ? 1490.0 : 1460.0);
     const double wide = cost(128, 256, 256, TRANS_A ? 1147.0 : TRANS_B ? 1334.0 : 1180.0);
     const double small = cost(128, 128, 512, TRANS_A ? 1190.0 : TRANS_B ? 959.0 : 1080.0);
@@ -362,6 +365,17 @@ extern "C" size_t iex_gemm_workspace_bytes(int dtype, int code, int M, int N, in
 
 size_t iex::gemm_auto_split_bytes(int M, int N, int K, int batch) {
   return auto_split_wanted(M, N, K, batch) ? gemm_parts_bytes(M, N, batch, 64, 128, split_parts_for(M, N, K, batch, 64, 128, 64)) : 0;
+}
+
+// Seconds of C = A B with B as (K, N), as launch_shape would run it with a workspace, with launch, prologue and epilogue.
+double iex::gemm_seconds(int M, int N, int K) {
+  if ((long long)ceil_div(M, 128) * ceil_div(N, 128) > 256 && K > 256) {
+    const double best = std::min({tile_cost(M, N, 1, 256, 256, 256, 1460.0), tile_cost(M, N, 1, 192, 256, 256, 1300.0), tile_cost(M, N, 1, 128, 256, 256, 1180.0),
+                                  tile_cost(M, N, 1, 128, 128, 512, 1080.0)});
+    return 6e-6 + best * K * 2e-12;
+  }
+  const double tiles = (double)ceil_div(M, 128) * ceil_div(N, 128);
+  return 6e-6 + std::max(std::ceil(tiles / 512.0) * (K / 32.0) * 0.23e-6 / gemm_auto_split_parts(M, N, K, 1), (double)M * N * 2 / 3e12);
 }
 
 int iex::gemm_auto_split_parts(int M, int N, int K, int batch) {

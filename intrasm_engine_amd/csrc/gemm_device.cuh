@@ -63,6 +63,7 @@ int gemm_dispatch(int dtype, int code, const GemmParams& p, int batch, hipStream
 size_t gemm_auto_split_bytes(int M, int N, int K, int batch);
 int gemm_auto_split_parts(int M, int N, int K, int batch);   // parts of K that gemm_dispatch would use with that workspace (1: no split)
 void gemm_auto_split_flags(int M, int N, int K, int batch, size_t* offset_bytes, int* words);
+double gemm_seconds(int M, int N, int K);   // an estimate, for choices between a dense product and others
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));

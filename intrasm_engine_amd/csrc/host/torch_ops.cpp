@@ -371,6 +371,59 @@ std::optional<Tensor> spmm_with(const Tensor& x, const Tensor& row_indices, cons
 }
 
 // softmax(scale * q^T k) v per head and sequence on feature-major operands; None where the kernel does not serve them
+// A sparse weight laid out once (ops.WeightForm makes it): the product with x, combined with `other` as in spmm_with.  Nothing is returned where the
+// call is not served here -- operands that do not fit, a gradient wanted, kernels forced, an operator on the CSR arrays that is faster.  A captured
+// call lays the weight out inside the graph: replays follow the CSR arrays, and give the same bits as a call.
+struct WeightForm {
+  static constexpr int kAnyRoom = 1 << 20;
+  int dtype;
+  int64_t m, k, nonzeros;
+  std::array<Tensor, 4> forms;   // kinds 0, 128, 192, 256
+  std::array<int, 3> phases, rooms;
+  int kinds = 0;
+  Tensor values, row_offsets, column_indices;
+
+  WeightForm(const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m, int64_t k,
+             const std::vector<std::optional<Tensor>>& given, const std::vector<int>& measured)
+      : dtype(dtype_code(values.scalar_type())), m(m), k(k), nonzeros(column_indices.numel()), values(values), row_offsets(row_offsets), column_indices(column_indices) {
+    TORCH_CHECK(given.size() == 4 && measured.size() == 6, "WeightForm: four forms and six numbers");
+    for (int i = 0; i < 4; ++i)
+      if (given[i]) forms[i] = *given[i], kinds |= 1 << i;
+    std::copy_n(measured.begin(), 3, phases.begin());
+    std::copy_n(measured.begin() + 3, 3, rooms.begin());
+  }
+
+  std::optional<Tensor> product(const Tensor& x, const std::optional<Tensor>& other, int mode) const {
+    const int64_t n = x.dim() == 2 ? x.size(1) : 0;
+    if (forced || !plain(x, 2) || x.size(0) != k || n == 0 || n % 8 || k * n >= (1ll << 31) || m * n >= (1ll << 31) || dtype_code(x.scalar_type()) != dtype ||
+        reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 || (at::GradMode::is_enabled() && (x.requires_grad() || (other && other->requires_grad()))))
+      return {};
+    if (other && (!plain(*other, 2) || other->size(0) != m || other->size(1) != n || other->scalar_type() != x.scalar_type() || other->device() != x.device())) return {};
+    const c10::DeviceGuard guard(x.device());
+    const int kind = iex_form_choose(kinds, m, k, n, nonzeros, phases.data());
+    if (kind < 0) return {};
+    Tensor form = forms[kind ? kind / 64 - 1 : 0];
+    if (form.device() != x.device()) return {};
+    int room = kind ? rooms[kind / 64 - 2] : 0;
+    if (capturing()) {
+      room = kind ? kAnyRoom : 0;   // (the pattern of a later replay may spill more)
+      form = workspace(iex_form_bytes(kind, m, k, room), x);
+      const Tensor scratch = workspace(kind ? iex_form_scratch_bytes(m, k) : 0, x);
+      check(iex_form_build(column_indices.scalar_type() == at::kShort ? IEX_I16 : IEX_I32, kind, m, k, nonzeros, row_offsets.const_data_ptr<int>(),
+                           column_indices.const_data_ptr(), values.const_data_ptr(), room, form.data_ptr(), form.numel(),
+                           scratch.defined() ? scratch.data_ptr() : nullptr, scratch.defined() ? scratch.numel() : 0, stream_of(x)),
+            "form");
+    }
+    const size_t ws_bytes = iex_form_product_workspace_bytes(kind, m, k, n);
+    const Tensor ws = workspace(ws_bytes, x);
+    Tensor out = at::empty({m, n}, x.options());
+    check(iex_form_product(dtype, kind, m, k, n, room, form.const_data_ptr(), x.const_data_ptr(), other ? other->const_data_ptr() : nullptr, mode,
+                           out.data_ptr(), ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, stream_of(x)),
+          "form product");
+    return out;
+  }
+};
+
 std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, int64_t seqs, double scale) {
   const int dtype = dtype_code(q.scalar_type());
   if (forced || !plain(q, 2) || !plain(k, 2) || !plain(v, 2) || k.sizes() != q.sizes() || v.sizes() != q.sizes() || k.scalar_type() != q.scalar_type() ||
@@ -552,6 +605,10 @@ PYBIND11_MODULE(_iex_host, module) {
   module.def("set_note", &set_note);
   module.def("spmm_with", &spmm_with);
   module.def("attention", &attention);
+  py::class_<WeightForm>(module, "WeightForm")
+      .def(py::init<const Tensor&, const Tensor&, const Tensor&, int64_t, int64_t, const std::vector<std::optional<Tensor>>&, const std::vector<int>&>())
+      .def_readonly("kinds", &WeightForm::kinds)
+      .def("product", &WeightForm::product, py::arg("x"), py::arg("other") = std::nullopt, py::arg("mode") = 0);
   module.def("sparse_attention", &sparse_attention);
   module.def("set_mask_tables", &set_mask_tables);
   module.def("trainable_spmm", &trainable_spmm);

@@ -624,14 +624,8 @@ inline size_t dense_path_bytes(const SpmmParams& p, int batch) {
 // tile then runs on several CUs; 4096^2 at 70-90 %, n = 128 / 256: 40 / 41 -> 27 / 32 us).
 //   Wide rows are gathered in tiles of 512 columns, the last one as slow as the others (3449 x 8696 at 94 %, n = 552: 185
 //     against 72 us).
-inline bool dense_path_wins(const SpmmParams& p, int batch, int matrix_core_kind, bool few_columns, bool split_room = true) {
-  const double cells = (double)p.m * p.k, flops = 2.0 * cells * p.n * batch, density = p.nnz / std::max(cells, 1.0);
-  const double out_bytes = (double)p.m * p.n * batch * 2;
-  const double tiles = (double)ceil_div(p.m, 128) * ceil_div(p.n, 128) * batch;
-  const int parts = split_room && !p.accumulate ? gemm_auto_split_parts(p.m, p.n, round8(p.k), batch) : 1;
-  const double product = std::max({flops / 1000e12, std::ceil(tiles / 512.0) * (p.k / 32.0) * 0.23e-6 / parts, out_bytes / 3e12});
-  const double pad = dense_path_pads(p) ? 4e-6 + 4.0 * p.k * p.n * batch / 4e12 : 0.0;
-  const double dense_form = 8e-6 + cells * 2 / 4e12 + pad + product;
+inline double other_families_seconds(const SpmmParams& p, int batch, int matrix_core_kind, bool few_columns) {
+  const double cells = (double)p.m * p.k, flops = 2.0 * cells * p.n * batch, density = p.nnz / std::max(cells, 1.0), out_bytes = (double)p.m * p.n * batch * 2;
   double other;
   if (few_columns) {
     other = 8e-6 + out_bytes / 4.5e12 + (double)p.nnz * batch * ceil_div(p.n, 512) * 10.0 / (256 * 2.1e9);
@@ -644,7 +638,17 @@ inline bool dense_path_wins(const SpmmParams& p, int batch, int matrix_core_kind
     const double columns = p.n <= 256 ? p.n : ceil_div(p.n, 512) * 512;   // (whole tiles: a last tile of few columns costs like a full one)
     other = 8e-6 + (double)p.nnz * columns * batch * 2 / 26e12 + out_bytes / 4e12;
   }
-  return 1.15 * dense_form < other;
+  return other;
+}
+inline bool dense_path_wins(const SpmmParams& p, int batch, int matrix_core_kind, bool few_columns, bool split_room = true) {
+  const double cells = (double)p.m * p.k, flops = 2.0 * cells * p.n * batch;
+  const double out_bytes = (double)p.m * p.n * batch * 2;
+  const double tiles = (double)ceil_div(p.m, 128) * ceil_div(p.n, 128) * batch;
+  const int parts = split_room && !p.accumulate ? gemm_auto_split_parts(p.m, p.n, round8(p.k), batch) : 1;
+  const double product = std::max({flops / 1000e12, std::ceil(tiles / 512.0) * (p.k / 32.0) * 0.23e-6 / parts, out_bytes / 3e12});
+  const double pad = dense_path_pads(p) ? 4e-6 + 4.0 * p.k * p.n * batch / 4e12 : 0.0;
+  const double dense_form = 8e-6 + cells * 2 / 4e12 + pad + product;
+  return 1.15 * dense_form < other_families_seconds(p, batch, matrix_core_kind, few_columns);
 }
 
 // Behind dense form and copy (rounded up to 256 bytes) the workspace may hold what the GEMM wants for splitting K over two
@@ -792,6 +796,14 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
 }
 
 }  // namespace
+
+// The estimate of the time model above for a 16-bit product by a family that reads the CSR arrays (no dense form).
+double spmm_seconds(int m, int k, int n, int nonzeros) {
+  void* const some_aligned = reinterpret_cast<void*>(size_t(256));
+  SpmmParams p{m, k, n, nonzeros, nullptr, nullptr, nullptr, nullptr, some_aligned, nullptr, some_aligned, 0, 0, 0};
+  const bool few = smallk_wanted<__half>(p, 1);
+  return other_families_seconds(p, 1, few ? 0 : mfma_variant<__half>(p, 1, Choice{}).kind, few);
+}
 
 // For the fused launcher: the number of register windows if the dispatcher would run this
 // fp16 SpMM (one batch entry, nothing forced) on the 8-wave matrix-core kernel, else 0.

@@ -55,10 +55,28 @@ class SparseDecoderLayer:
             # (looked at once, here: the layer's schedules run under capture, where a pattern nobody has looked at
             # keeps to the kernels that take columns in any order)
             _pyops.prepare_pattern(self.w[name][2], self.w[name][3], csr.k, tables=False)
+        # the weights as the schedules multiply them, laid out once (a capture lays them out inside the graph)
+        self._forms = {name: self._lay_out(name) for name in self.w}
+
+    def _lay_out(self, name: str) -> "_pyops.WeightForm":
+        _, v, ro, ci, m = self.w[name]
+        return _pyops.WeightForm(v, ro, ci, m, self.mlp if name == "down" else self.hidden)
 
     # ---- building blocks ---------------------------------------------------------------
+    def _by_form(self, name: str, x: torch.Tensor, other=None, mode: int = 0):
+        """The product by what was laid out, of the weight as it is now; None where the operators have to serve it."""
+        form, (_, v, ro, ci, _) = self._forms[name], self.w[name]
+        if not form.is_of(v, ro, ci):
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            form = self._forms[name] = self._lay_out(name)
+        return form.product(x, other, mode)
+
     def proj(self, name: str, x: torch.Tensor) -> torch.Tensor:
         """(k, tokens) -> (m, tokens)."""
+        out = self._by_form(name, x)
+        if out is not None:
+            return out
         ri, v, ro, ci, m = self.w[name]
         return ops.spmm_sputnik_reuse_weight_half(x.unsqueeze(0), ri, v, ro, ci, m)[0]
 
@@ -69,6 +87,9 @@ class SparseDecoderLayer:
 
     def _proj_with(self, name: str, x: torch.Tensor, other: torch.Tensor, mode: int):
         """``proj`` combined with ``other`` before it is rounded: plus it (mode 1), times its SiLU (mode 2)."""
+        out = self._by_form(name, x, other, mode) if self._heads_fit else None
+        if out is not None:
+            return out
         ri, v, ro, ci, m = self.w[name]
         out = _iex_host.spmm_with(x, ri, v, ro, ci, m, other, mode) if self._heads_fit else None
         if out is None:

@@ -367,6 +367,57 @@ def prepare_pattern(row_offsets, column_indices, k, tables=True):
     return status
 
 
+class WeightForm:
+    """A 16-bit sparse weight laid out once for products with many dense columns (``iex_form_build``), for a program that keeps the weight:
+    its dense form and, where a row holds at most two of (nearly) every four neighbouring columns, the two-of-four form that the
+    structured-sparsity matrix instructions take.  Costs a synchronisation and about 2-4 bytes a cell of the weight.
+
+    What was laid out stands for the CSR tensors as they were: :meth:`is_of` tells whether they are still those."""
+
+    KINDS = (0, 128, 192, 256)
+
+    def __init__(self, values, row_offsets, column_indices, m, k):
+        self._tensors = (values, row_offsets, column_indices)
+        self._versions = tuple(_version(t) for t in self._tensors)
+        self._form = None
+        nonzeros, device, lib = column_indices.numel(), values.device, _lib.load()
+        if values.dtype not in (torch.float16, torch.bfloat16) or not 3 <= nonzeros < 1 << 29 or torch.cuda.is_current_stream_capturing() or \
+                _csr_status(row_offsets, column_indices, k) != 0 or lib.iex_form_bytes(0, m, k, 0) == 0:
+            return
+        itype = _IT[column_indices.dtype]
+        with torch.cuda.device(device):
+            stream = _stream_ptr(device)
+            scratch = torch.empty(lib.iex_form_scratch_bytes(m, k), dtype=torch.uint8, device=device)
+            measured = [0] * 6
+            if scratch.numel():
+                counts = torch.zeros(6, dtype=torch.int32, device=device)
+                _lib.check(lib.iex_form_measure(itype, m, k, nonzeros, row_offsets.data_ptr(), column_indices.data_ptr(), scratch.data_ptr(), scratch.numel(),
+                                                counts.data_ptr(), stream), "form")
+                measured = counts.tolist()
+            phases = (ctypes.c_int * 3)(*measured[:3])
+            # the kinds that some width wants
+            wanted = {0} | {lib.iex_form_choose(15 if scratch.numel() else 1, m, k, n, nonzeros, phases) for n in (256, 512, 1024, 2048, 4096, 8192)}
+            forms = [None] * 4
+            for i, kind in enumerate(self.KINDS):
+                if kind not in wanted:
+                    continue
+                room = measured[2 + i] if kind else 0
+                forms[i] = torch.empty(lib.iex_form_bytes(kind, m, k, room), dtype=torch.uint8, device=device)
+                _lib.check(lib.iex_form_build(itype, kind, m, k, nonzeros, row_offsets.data_ptr(), column_indices.data_ptr(), values.data_ptr(), room,
+                                              forms[i].data_ptr(), forms[i].numel(), scratch.data_ptr(), scratch.numel(), stream), "form")
+            torch.cuda.current_stream(device).synchronize()      # (products on any stream find it complete)
+        self._form = _iex_host.WeightForm(values, row_offsets, column_indices, m, k, forms, measured)
+
+    def is_of(self, values, row_offsets, column_indices) -> bool:
+        """Whether these are the tensors that were laid out, unchanged since."""
+        return all(a is b and _version(b) == v for a, b, v in zip(self._tensors, (values, row_offsets, column_indices), self._versions))
+
+    def product(self, x, other=None, mode=0):
+        """``weight @ x``, plus ``other`` (mode 1) or times its SiLU (mode 2) before it is rounded; None where an operator on the CSR tensors has to
+        serve the call (``WeightForm::product`` of csrc/host/torch_ops.cpp)."""
+        return self._form.product(x, other, mode) if self._form is not None else None
+
+
 def carry_pattern_note(column_indices, copy):
     """``copy`` holds the same column indices as ``column_indices`` (another integer type, a clone): what is known about
     the one holds for the other."""

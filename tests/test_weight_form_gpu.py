@@ -1,0 +1,170 @@
+"""A sparse 16-bit weight laid out once (dense form, two-of-four form with spilled entries) and multiplied by what was laid out: every
+kind at the edges of tiles, phases and spill blocks, against the oracle; when a form may stand for the CSR arrays."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from intrasm_engine_amd import _iex_host, _lib
+from intrasm_engine_amd import workloads as W
+from intrasm_engine_amd.decoder_layer import SparseDecoderLayer
+from intrasm_engine_amd.pytorch import ops as pyops
+from _util import RTOL, assert_close, rounded, to_dev
+
+pytestmark = pytest.mark.gpu
+CODE = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
+
+
+def _two_four(rng, m, k):
+    """Two of every four neighbouring columns (one of them, or none, in some groups)."""
+    keep = np.zeros((m, (k + 3) // 4, 4), bool)
+    order = rng.random(keep.shape).argsort(axis=2)
+    np.put_along_axis(keep, order[:, :, :2], True, axis=2)
+    keep &= rng.random(keep.shape) < 0.9
+    return keep.reshape(m, -1)[:, :k]
+
+
+def _csr(rng, m, k, density):
+    mask = _two_four(rng, m, k) if density == "2:4" else rng.random((m, k)) < density
+    mask[0, :min(k, 7)] = True           # (at least three entries; a row that spills)
+    if m > 2:
+        mask[2] = False
+    ro = np.concatenate([[0], np.cumsum(mask.sum(axis=1))]).astype(np.int32)
+    ci = np.nonzero(mask)[1].astype(np.int32)
+    return W.CSR(m, k, rng.standard_normal(ci.shape[0]).astype(np.float32), W.swizzle_from_offsets(ro), ro, ci)
+
+
+def _spilled_phases(csr, half):
+    """What iex_form_measure counts, from the definition: columns with entries beyond the first two of their group, per block of rows."""
+    phases = []
+    for r0 in range(0, csr.m, half):
+        cols = set()
+        for r in range(r0, min(r0 + half, csr.m)):
+            c = csr.column_indices[csr.row_offsets[r]:csr.row_offsets[r + 1]]
+            cols.update(c[2:][c[2:] // 4 == c[:-2] // 4].tolist())
+        phases.append((len(cols) + 31) // 32)
+    return sum(phases), max(phases)
+
+
+@pytest.mark.parametrize("dtype,idtype", [(torch.float16, torch.int16), (torch.bfloat16, torch.int32)])
+@pytest.mark.parametrize("m,k,n,density", [(1, 7, 8, 1.0), (127, 64, 256, "2:4"), (300, 200, 264, 0.3), (257, 129, 520, 0.5), (193, 1000, 40, 0.1),
+                                           (385, 65, 248, 0.05), (130, 260, 264, 1.0), (640, 4100, 264, 0.1)])
+def test_every_kind(oracle, dev, dtype, idtype, m, k, n, density):
+    rng = np.random.default_rng(m + k)
+    csr = _csr(rng, m, k, density)
+    _, v, ro, ci = to_dev(csr, dev, dtype, idtype)
+    x, aux = rng.standard_normal((k, n)).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    xt, at = (torch.from_numpy(t).to(dev).to(dtype) for t in (x, aux))
+    vr, xr, ar = rounded(csr.values, dtype), rounded(x, dtype), rounded(aux, dtype).astype(np.float64)
+    base = oracle.spmm(xr[None], csr.row_indices, vr, csr.row_offsets, csr.column_indices, m)[0]
+    scale = oracle.spmm_abs_scale(xr[None], csr.row_indices, vr, csr.row_offsets, csr.column_indices, m)[0]
+    silu = ar / (1 + np.exp(-ar))
+    lib, it, nnz, stream = _lib.load(), 1 if idtype == torch.int16 else 0, ci.numel(), torch.cuda.current_stream().cuda_stream
+    scratch = torch.empty(lib.iex_form_scratch_bytes(m, k), dtype=torch.uint8, device=dev)
+    counts = torch.zeros(6, dtype=torch.int32, device=dev)
+    _lib.check(lib.iex_form_measure(it, m, k, nnz, ro.data_ptr(), ci.data_ptr(), scratch.data_ptr(), scratch.numel(), counts.data_ptr(), stream))
+    counts = counts.tolist()
+    for i, half in enumerate((64, 96, 128)):
+        assert (counts[i], counts[3 + i]) == _spilled_phases(csr, half)
+    for i, kind in enumerate((0, 128, 192, 256)):
+        room = counts[2 + i] if kind else 0
+        form = torch.full((lib.iex_form_bytes(kind, m, k, room),), 0xff, dtype=torch.uint8, device=dev)      # (NaN where nothing is written)
+        _lib.check(lib.iex_form_build(it, kind, m, k, nnz, ro.data_ptr(), ci.data_ptr(), v.data_ptr(), room, form.data_ptr(), form.numel(),
+                                      scratch.data_ptr(), scratch.numel(), stream))
+        need = lib.iex_form_product_workspace_bytes(kind, m, k, n)
+        ws = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
+        for mode, want, bound in ((0, base, scale), (1, base + ar, scale + np.abs(ar)), (2, base * silu, scale * np.abs(silu) + 1e-3)):
+            out = torch.full((m, n), float("nan"), dtype=dtype, device=dev)
+            _lib.check(lib.iex_form_product(CODE[dtype], kind, m, k, n, room, form.data_ptr(), xt.data_ptr(), at.data_ptr() if mode else None, mode,
+                                            out.data_ptr(), ws.data_ptr(), need, stream))
+            assert ("two_four_kernel" in _lib.last_kernels()) == (kind > 0)
+            assert_close(out.float().cpu().numpy(), want, 5 * bound, RTOL[dtype], f"kind {kind} mode {mode}")
+
+
+def test_values_that_mark_an_empty_place_and_infinities(dev):
+    """Every bit pattern is a value; an infinity a row refers to shows as itself in that row."""
+    m, k, n = 130, 128, 256
+    rng = np.random.default_rng(1)
+    csr = _csr(rng, m, k, "2:4")
+    _, v, ro, ci = to_dev(csr, dev, torch.float16)
+    x = torch.randn(k, n, device=dev).half()
+    x[5, 3] = float("inf")
+    v[torch.nonzero(ci == 9)[0]] = float("nan")
+    form = pyops.WeightForm(v, ro, ci, m, k)
+    dense = torch.zeros(m, k, device=dev, dtype=torch.float64)
+    rows = torch.repeat_interleave(torch.arange(m, device=dev), ro.long().diff())
+    dense[rows, ci.long()] = v.double()
+    refers = dense[:, 5] != 0
+    lib, kinds = _lib.load(), form._form.kinds
+    assert kinds & 1
+    for kind in (128, 256):
+        counts = torch.zeros(6, dtype=torch.int32, device=dev)
+        scratch = torch.empty(lib.iex_form_scratch_bytes(m, k), dtype=torch.uint8, device=dev)
+        stream = torch.cuda.current_stream().cuda_stream
+        _lib.check(lib.iex_form_measure(0, m, k, ci.numel(), ro.data_ptr(), ci.data_ptr(), scratch.data_ptr(), scratch.numel(), counts.data_ptr(), stream))
+        room = counts.tolist()[2 + (kind // 64 - 1)]
+        memory = torch.empty(lib.iex_form_bytes(kind, m, k, room), dtype=torch.uint8, device=dev)
+        _lib.check(lib.iex_form_build(0, kind, m, k, ci.numel(), ro.data_ptr(), ci.data_ptr(), v.data_ptr(), room, memory.data_ptr(), memory.numel(),
+                                      scratch.data_ptr(), scratch.numel(), stream))
+        out = torch.empty(m, n, device=dev, dtype=torch.float16)
+        _lib.check(lib.iex_form_product(_lib.F16, kind, m, k, n, room, memory.data_ptr(), x.data_ptr(), None, 0, out.data_ptr(), None, 0, stream))
+        with_nan = dense.isnan().any(dim=1)
+        assert bool(out[with_nan].isnan().all())
+        assert bool(out[refers & ~with_nan][:, 3].isinf().all())
+        others = torch.ones(n, dtype=torch.bool, device=dev)
+        others[3] = False
+        want = (torch.nan_to_num(dense) @ torch.nan_to_num(x.double(), posinf=0.0))[~with_nan][:, others]
+        assert torch.allclose(out[~with_nan][:, others].double(), want, rtol=1e-2, atol=1e-1)
+
+
+def _layer(dev, hidden=256, mlp=512, seed=0):
+    rng = np.random.default_rng(seed)
+    weights = {}
+    for name, (m, k) in {**{x: (hidden, hidden) for x in "qkvo"}, "gate": (mlp, hidden), "up": (mlp, hidden), "down": (hidden, mlp)}.items():
+        csr = _csr(rng, m, k, "2:4" if len(name) == 1 else 0.2)
+        weights[name] = W.CSR(m, k, csr.values * 0.05, csr.row_indices, csr.row_offsets, csr.column_indices)
+    return SparseDecoderLayer(weights, hidden, hidden // 64, mlp, dev)
+
+
+def test_layer_by_forms_follows_its_weights(dev):
+    """By what was laid out and by the operators: the same result up to rounding, also after a weight was changed in place or replaced;
+    replays of a captured call give the same bits and follow the weights, too; a kernel_params block and a gradient keep to the operators."""
+    layer = _layer(dev)
+    x = torch.randn(256, 1024, device=dev).half()
+
+    def by_operators():
+        with pyops.kernel_params(gemm={"tile": 13}):
+            return layer.forward(x, 2)
+
+    first = layer.forward(x, 2)
+    assert torch.allclose(first.float(), by_operators().float(), rtol=2e-2, atol=2e-2)
+    layer.w["q"][1].mul_(3.0)
+    ri, v, ro, ci, m = layer.w["down"]
+    layer.w["down"] = (ri, v * 0.5, ro, ci, m)
+    second = layer.forward(x, 2)
+    assert not torch.allclose(second.float(), first.float(), rtol=2e-2, atol=2e-2)
+    assert torch.allclose(second.float(), by_operators().float(), rtol=2e-2, atol=2e-2)
+    assert torch.equal(layer.forward(x, 2), second)
+    assert layer._by_form("q", x.clone().requires_grad_()) is None and layer._by_form("q", x[:, :1021].contiguous()) is None
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = layer.forward(x, 2)
+    for factor in (1.0, 0.25, 2.0):
+        layer.w["gate"][1].mul_(factor)
+        graph.replay()
+        assert torch.equal(out, layer.forward(x, 2))
+
+
+def test_forms_are_refused_on_the_host(dev):
+    lib = _lib.load()
+    one = torch.zeros(1024, dtype=torch.int32, device=dev)
+    at = one.data_ptr()
+    assert lib.iex_form_bytes(64, 256, 256, 0) == 0 and lib.iex_form_bytes(256, 256, 70000, 0) == 0 and lib.iex_form_bytes(0, 1 << 16, 1 << 16, 0) == 0
+    assert lib.iex_form_build(0, 256, 256, 256, 2, at, at, at, 0, at, 1 << 30, at, 1 << 30, None) != 0             # two nonzeros
+    assert lib.iex_form_build(0, 256, 256, 256, 5, at, at, at, 0, at, 16, at, 1 << 30, None) != 0                  # no room
+    assert lib.iex_form_product(_lib.F16, 256, 256, 256, 12, 0, at, at, None, 0, at, None, 0, None) != 0           # n off 8
+    assert lib.iex_form_product(_lib.F32, 256, 256, 256, 16, 0, at, at, None, 0, at, None, 0, None) != 0
+    assert lib.iex_form_choose(15, 256, 256, 0, 100, (ctypes.c_int * 3)()) == -1
+    fp32 = torch.zeros(8, device=dev)
+    assert pyops.WeightForm(fp32, one[:2], one[:8], 1, 16).product(torch.zeros(16, 8, device=dev)) is None
