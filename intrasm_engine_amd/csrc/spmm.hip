@@ -58,10 +58,17 @@ int launch_ragged(const SpmmParams& p, int batch, int wpr, hipStream_t stream) {
 }
 
 // ---- few columns in A, wide output: the dense operand's tile lives in LDS ---------------------
-template <typename T, typename IT, int VEC, bool RAGGED, int WAVES, int MOST, bool PLAIN>
+template <typename T, typename IT, int VEC, bool RAGGED, int WAVES, int MOST, bool PLAIN, bool SCALAR>
 __global__ __launch_bounds__(WAVES * kWave) void spmm_smallk_kernel(SpmmParams p, int rows_per_wave) {
   extern __shared__ __align__(16) unsigned char smem[];
-  spmm_smallk_block<T, IT, VEC, RAGGED, WAVES, MOST, PLAIN>(p, rows_per_wave, blockIdx.x, blockIdx.y, blockIdx.z, smem);
+  spmm_smallk_block<T, IT, VEC, RAGGED, WAVES, MOST, PLAIN, SCALAR>(p, rows_per_wave, blockIdx.x, blockIdx.y, blockIdx.z, smem);
+}
+
+// The same with every line of the output written by one wavefront (fp32, no bias, ReLU or accumulation).
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void spmm_smallk_kernel_lines(SpmmParams p, SmallkLines t, int rows_per_wave) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  spmm_smallk_lines_block<WAVES>(p, t, rows_per_wave, blockIdx.x, blockIdx.y, blockIdx.z, smem);
 }
 
 // full vectors at their natural alignment, or (ragged) any n at element alignment
@@ -69,6 +76,14 @@ template <typename T>
 bool smallk_aligned(const SpmmParams& p) {
   constexpr int kMax = 16 / (int)sizeof(T);
   return p.n % kMax == 0 && aligned(p.dense, 16) && aligned(p.out, 16);
+}
+
+// Whole lines per wavefront: fp32 rows that do not start at multiples of 64 bytes.  A dword of LDS per lane, nonzero and 64 columns costs more
+// instructions than 128-bit vectors: up to 9 nonzeros a row (us, this / vectors: 384 x 785 x 785, 3.2 per row 252 / 283, 6.4 218 / 295, 9.6
+// 331 / 265, 19 429 / 411; 24 x 3133 x 3133, 6.4 215 / 283, 12.8 366 / 344; 64 x 1004 x 1004, 6.4 53 / 89, 12.8 104 / 101).
+template <typename T>
+bool smallk_by_lines(const SpmmParams& p) {
+  return sizeof(T) == 4 && !p.bias && !p.relu && !p.accumulate && (p.n % 16 != 0 || !aligned(p.out, 64)) && p.nnz <= 9ll * p.m && smallk_lines(p.n, p.k).rest > 0;
 }
 
 template <typename T>
@@ -97,6 +112,10 @@ bool matrix_core_kernel_applies(const SpmmParams& p, int batch);
 //   k = 64, m = 333: 13 per row 71 -> 47 (fp32), 78 -> 49 (fp16), 1.9 per row 26 / 28;
 //   rows of fp16 narrower than half a tile and no whole vectors, which the row kernel takes in single elements: 384 x 197 x 197
 //     64 - 177 -> 26 - 116 whatever k and density; fp32 there: 46 / 53 at 13 per row.
+// Where lines are written whole (smallk_by_lines) it is ahead from fewer nonzeros on, outputs of 80 MB and more: any number in rows of 700
+// columns, else one a row, three for k > 64 (384 x 785 x 785, k = 64: 1.9 per row 289 -> 203, 0.7 233 -> 201; k = 128, 6.4 437 -> 348, 1.3
+// 282 -> 238; 200 x 333 x 333, k = 64, 1 per row 32 -> 28, k = 128, 3.8 47 -> 40; 300 x 500 x 500, k = 64, 1.9 89 -> 79, 0.7 67 / 76, k = 128,
+// 1.9 97 / 105; rows of fewer than 256 columns stay with the row kernel: 384 x 197 x 197, k = 64, 6.6 per row 34 / 44).
 template <typename T>
 bool smallk_wanted(const SpmmParams& p, int batch) {
   constexpr int kMax = 16 / (int)sizeof(T);
@@ -104,6 +123,7 @@ bool smallk_wanted(const SpmmParams& p, int batch) {
   const double per_row = (double)p.nnz / std::max(p.m, 1);
   const bool whole = smallk_aligned<T>(p), large = (double)batch * p.m * p.n >= 8e6;
   const bool wide = p.n >= kWave * kMax / (sizeof(T) == 2 ? 2 : 1);
+  if (smallk_by_lines<T>(p) && (double)batch * p.m * p.n >= 2e7 && p.m >= 2 * p.k && per_row >= (p.n >= 700 ? 0.0 : p.k > 64 ? 3.0 : 1.0)) return true;
   if (wide && p.k <= 64 && p.m >= 8 * p.k) return per_row >= (whole ? 1.8 : 2.5);
   if (wide && p.k > 64 && p.m >= 32 * p.k && per_row >= 4.0) return true;
   if (!large) return false;
@@ -113,11 +133,10 @@ bool smallk_wanted(const SpmmParams& p, int batch) {
   return per_row >= (p.k <= 64 ? 8.0 : sizeof(T) == 2 ? 2.5 : 8.0);
 }
 
-template <typename T, typename IT, bool RAGGED, int WAVES, int MOST, bool PLAIN>
-int launch_smallk_one(const SpmmParams& p, int batch, int tiles_n, int lds, hipStream_t stream) {
-  constexpr int kMax = 16 / (int)sizeof(T);
-  const long long tiles = (long long)tiles_n * batch;
-  int rows;   // per wavefront
+// Rows per wavefront of the few-columns kernels, `tiles` column tiles (of all batch entries) and WAVES wavefronts per workgroup.
+template <int WAVES>
+int smallk_rows(const SpmmParams& p, long long tiles) {
+  int rows;
   if constexpr (WAVES == 8) {
     // two workgroups per CU cover for each other's tile load: enough rows for it to be a fraction of what they write
     rows = std::min(64, std::max(16, p.k / 2));
@@ -135,7 +154,17 @@ int launch_smallk_one(const SpmmParams& p, int batch, int tiles_n, int lds, hipS
       if (blocks >= 64) blocks += blocks / 16;   // (long operands: not every count)
     }
   }
-  auto kern = spmm_smallk_kernel<T, IT, kMax, RAGGED, WAVES, MOST, PLAIN>;
+  return rows;
+}
+
+template <typename T, typename IT, bool RAGGED, int WAVES, int MOST, bool PLAIN, bool SCALAR = false>
+int launch_smallk_one(const SpmmParams& p, int batch, int tiles_n, int lds, hipStream_t stream) {
+  constexpr int kMax = 16 / (int)sizeof(T);
+  if constexpr (!SCALAR && std::is_same<T, float>::value && std::is_same<IT, int>::value) {
+    if (p.nnz > (long long)kSmallkScalarRows * p.m) return launch_smallk_one<T, IT, RAGGED, WAVES, MOST, PLAIN, true>(p, batch, tiles_n, lds, stream);
+  }
+  const int rows = smallk_rows<WAVES>(p, (long long)tiles_n * batch);
+  auto kern = spmm_smallk_kernel<T, IT, kMax, RAGGED, WAVES, MOST, PLAIN, SCALAR>;
   if (lds > 64 * 1024) {
     static thread_local bool raised = false;  // per instantiation
     if (!raised) {
@@ -152,10 +181,33 @@ int launch_smallk_one(const SpmmParams& p, int batch, int tiles_n, int lds, hipS
 }
 
 // Two vectors per lane where the output is wider than one and two of every dense row fit the LDS.
+template <int WAVES>
+int launch_smallk_lines(const SpmmParams& p, int batch, const SmallkLines& t, int lds, hipStream_t stream) {
+  auto kern = spmm_smallk_kernel_lines<WAVES>;
+  static thread_local bool raised = false;  // per instantiation
+  if (!raised) {
+    if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
+                           "hipFuncSetAttribute(LDS size)"))
+      return rc;
+    raised = true;
+  }
+  const int rows = smallk_rows<WAVES>(p, (long long)(t.tiles + 1) * batch);
+  note_kernel("spmm_smallk_kernel_lines<%d> (%d tiles of %d columns, %d at the edges)", WAVES, t.tiles, t.width, t.rest);
+  hipLaunchKernelGGL(kern, dim3(ceil_div(p.m, WAVES * rows), t.tiles + 1, batch), dim3(WAVES * kWave), lds, stream, p, t, rows);
+  return check_hip(hipGetLastError(), "spmm (few columns, whole lines) launch");
+}
+
 template <typename T, typename IT>
 int launch_smallk(const SpmmParams& p, int batch, hipStream_t stream) {
   constexpr int kMax = 16 / (int)sizeof(T);
   const bool plain = !p.bias && !p.relu && !p.accumulate;
+  if constexpr (std::is_same<T, float>::value && std::is_same<IT, int>::value) {
+    if (smallk_by_lines<T>(p)) {
+      const SmallkLines t = smallk_lines(p.n, p.k);
+      const int lds = smallk_lines_lds(t, p.k);
+      return smallk_waves(lds) == 8 ? launch_smallk_lines<8>(p, batch, t, lds, stream) : launch_smallk_lines<16>(p, batch, t, lds, stream);
+    }
+  }
   const int most = plain && p.n > kWave * kMax && 2 * p.k <= kSmallKMax ? 2 : 1;
   const SmallkTiles t = smallk_tiles(p.n, most, kMax);
   const int last = smallk_row_bytes(t.nv, t.single, sizeof(T)), lds = p.k * (t.tiles > 1 ? std::max(last, smallk_row_bytes(most, false, sizeof(T))) : last);
