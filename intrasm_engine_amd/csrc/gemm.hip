@@ -1,5 +1,6 @@
 // Host side of the dense companion GEMM: kernel wrapper, tile-shape choice, XCD-aware
 // tile order, argument checks and the C entry point.  Device code: gemm_device.cuh.
+#include "gemm_il_device.cuh"
 #include "gemm_pp_device.cuh"
 
 namespace iex {
@@ -73,15 +74,15 @@ int launch_dma(GemmParams p, int batch, hipStream_t stream) {
 }
 
 // Eight wavefronts in two groups that alternate between reading / loading and multiplying (gemm_pp_device.cuh).
-template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN, int KP>
+template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, int KP>
 __global__ __launch_bounds__(WCN * 128, 1) void gemm_pp_kernel(GemmParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   int tile_m, tile_n;
   if (!xcd_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;  // uniform per block
-  gemm_tile_pp<BF16, TRANS_B, WM, WN, WCN, TRANS_A, KP>(p, tile_m, tile_n, blockIdx.y, smem);
+  gemm_tile_pp<BF16, TRANS_B, WM, WN, WCN, KP>(p, tile_m, tile_n, blockIdx.y, smem);
 }
 
-template <bool BF16, bool TRANS_A, bool TRANS_B, int WM, int WN, int WCN, int KP = 32>
+template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, int KP = 32>
 int launch_pp(GemmParams p, int batch, hipStream_t stream) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32;
   p.tiles_m = ceil_div(p.M, BM);
@@ -89,7 +90,7 @@ int launch_pp(GemmParams p, int batch, hipStream_t stream) {
   const int total = p.tiles_m * p.tiles_n;
   const int per_xcd = (total + kXcds - 1) / kXcds;
   constexpr int lds = gemm_pp_lds_bytes<WM, WN, WCN, KP>();
-  auto kern = gemm_pp_kernel<BF16, TRANS_A, TRANS_B, WM, WN, WCN, KP>;
+  auto kern = gemm_pp_kernel<BF16, TRANS_B, WM, WN, WCN, KP>;
   static thread_local bool raised = false;  // per instantiation
   if (!raised) {
     if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds),
@@ -97,9 +98,40 @@ int launch_pp(GemmParams p, int batch, hipStream_t stream) {
       return rc;
     raised = true;
   }
-  note_kernel("gemm_pp_kernel<%s, %s%s, %d, %d, %d> (%d x %d tiles, two groups of 4 waves in alternating phases)", BF16 ? "bf16" : "f16",
-              TRANS_A ? "A(K,M), " : "", TRANS_B ? "B(N,K)" : "B(K,N)", WM, WN, WCN, BM, BN);
+  note_kernel("gemm_pp_kernel<%s, %s, %d, %d, %d> (%d x %d tiles, two groups of 4 waves in alternating phases)", BF16 ? "bf16" : "f16",
+              TRANS_B ? "B(N,K)" : "B(K,N)", WM, WN, WCN, BM, BN);
   hipLaunchKernelGGL(kern, dim3(per_xcd * kXcds, batch), dim3(WCN * 128), lds, stream, p);
+  return check_hip(hipGetLastError(), "gemm launch");
+}
+
+// Eight wavefronts in phase, with single instructions between the MFMAs (gemm_il_device.cuh).
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM>
+__global__ __launch_bounds__(512, 1) void gemm_il_kernel(GemmParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  int tile_m, tile_n;
+  if (!xcd_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;  // uniform per block
+  gemm_tile_il<BF16, TRANS_B, WM, 2, 4, TRANS_A>(p, tile_m, tile_n, blockIdx.y, smem);
+}
+
+template <bool BF16, bool TRANS_A, bool TRANS_B, int WM>
+int launch_il(GemmParams p, int batch, hipStream_t stream) {
+  constexpr int BM = 2 * WM * 32, BN = 256;
+  p.tiles_m = ceil_div(p.M, BM);
+  p.tiles_n = ceil_div(p.N, BN);
+  const int total = p.tiles_m * p.tiles_n;
+  const int per_xcd = (total + kXcds - 1) / kXcds;
+  constexpr int lds = gemm_il_lds_bytes<WM, 2, 4>();
+  auto kern = gemm_il_kernel<BF16, TRANS_A, TRANS_B, WM>;
+  static thread_local bool raised = false;  // per instantiation
+  if (!raised) {
+    if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds),
+                           "hipFuncSetAttribute(LDS size)"))
+      return rc;
+    raised = true;
+  }
+  note_kernel("gemm_il_kernel<%s, %s%s, %d> (%d x %d tiles, 8 waves, single instructions between the MFMAs)", BF16 ? "bf16" : "f16",
+              TRANS_A ? "A(K,M), " : "", TRANS_B ? "B(N,K)" : "B(K,N)", WM, BM, BN);
+  hipLaunchKernelGGL(kern, dim3(per_xcd * kXcds, batch), dim3(512), lds, stream, p);
   return check_hip(hipGetLastError(), "gemm launch");
 }
 
@@ -264,7 +296,7 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
     if (force == 4) return launch<BF16, TRANS_B, 2, 2, 64>(p, batch, stream);
     if (force == 6) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 4, 32, 4>(p, batch, stream);
     if (force == 7) return launch_dma<BF16, TRANS_A, TRANS_B, 4, 4, 32, 4>(p, batch, stream);
-    if (force == 16) return launch_pp<BF16, TRANS_A, TRANS_B, 3, 2, 4>(p, batch, stream);
+    if (force == 16) return launch_il<BF16, TRANS_A, TRANS_B, 3>(p, batch, stream);
     if (force == 11) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 64, 3, 4>(p, batch, stream);
   }
   if (force == 14) {
@@ -279,8 +311,18 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
   if (force == 8) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 1, 64, 4, 4>(p, batch, stream);
   if (force == 9) return launch_dma<BF16, TRANS_A, TRANS_B, 1, 1, 64, 4, 4>(p, batch, stream);
   if (force == 10) return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4, 4>(p, batch, stream);
-  if (force == 15) return launch_pp<BF16, TRANS_A, TRANS_B, 2, 2, 4, 64>(p, batch, stream);
-  if (force == 13) return launch_pp<BF16, TRANS_A, TRANS_B, 4, 2, 4>(p, batch, stream);
+  // The schedule of the eight wavefronts: single instructions between the MFMAs where A is (K, M), alternating groups where
+  // it is not (measured side by side at the top of gemm_il_device.cuh)
+  auto rows_256 = [&] {
+    if constexpr (TRANS_A) return launch_il<BF16, TRANS_A, TRANS_B, 4>(p, batch, stream);
+    else return launch_pp<BF16, TRANS_B, 4, 2, 4>(p, batch, stream);
+  };
+  auto rows_128 = [&] {
+    if constexpr (TRANS_A) return launch_il<BF16, TRANS_A, TRANS_B, 2>(p, batch, stream);
+    else return launch_pp<BF16, TRANS_B, 2, 2, 4, 64>(p, batch, stream);
+  };
+  if (force == 15) return rows_128();
+  if (force == 13) return rows_256();
   // Default: operands straight from global memory into LDS (gemm_dma_device.cuh).  The larger the
   // tile of a wave, the fewer LDS bytes each MFMA needs, and LDS time is what the main loop runs
   // against; the smaller the tile, the more workgroups there are to fill 256 CUs, and a tile wider
@@ -294,24 +336,24 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
   if (small_tiles > 256) {
     // More 128 x 128 tiles than CUs: the tile shape that finishes first, counting whole rounds of workgroups (a
     // workgroup of the last round takes as long as any other) at the rate each shape reaches with every CU busy.
-    // TFLOP/s measured (8192^3, bf16, B as (K, N) / B as (N, K) / A as (K, M)): 256 x 256 by eight waves in two alternating
-    // groups 1460 / 1490 / 1385; 128 x 256 by the same in phases of 64 k (64 x 64 per wave) 1214 / 1334 / 1147, where eight waves
-    // in phase reach 1151 / 1078 / 1135; 128 x 128 by four waves, two workgroups per CU, 1080 / 959 / 1190.
-    //   4096 x 2048 x 4096: 829 / 858 / 729, 1115 / 1208 / 999 (in phase 1011 / 889 / 979), 950 / 806 / 1082
-    // 192 x 256 as 256 x 256 (not with A as (K, M)) 1303 / 1295: between the two where whole rounds are few, 11008 x 2048 x 4096
-    // 172 / 155 / 176 us for 256 / 192 / 128 rows, 9000 x 2048 x 4096 166 / 147 / 168, 5528 x 1600 x 2224 50 / 45 / 64.
+    // TFLOP/s measured (8192^3, bf16, B as (K, N) / B as (N, K) / A as (K, M)): 256 x 256 by eight waves 1520 / 1534 / 1456;
+    // 128 x 256 by the same (64 x 64 per wave) 1219 / 1335 / 1207, in one round or three 1105 .. 1189 / 1178 .. 1266 / 1093 .. 1140;
+    // 128 x 128 by four waves, two workgroups per CU, 1076 / 934 / 1188; 192 x 256 (not with A as (K, M)) 1311 / 1329.
+    //   us of 256 / 192 / 128 rows / 128 x 128:  4096 x 2048 x 4096 73 63 58 70 / 71 62 54 79 / 83 - 60 63;
+    //   11008 x 2048 x 4096 161 144 167 190 / 166 145 157 223 / 175 - 169 174;  9000 x 2048 x 4096 158 132 157 166 /
+    //   159 132 143 189 / 168 - 160 156;  5528 x 1600 x 2224 45 41 59 61 / 51 47 65 76 / 47 - 61 56.
     // (128 x 128 and 64 x 128 in alternating phases: no faster than codes 8 and 9.)
     // A last round with a share f of the CUs at work takes 0.65 + 0.35 f of a full one: those that work have the way from L2
     // and the power to themselves (11008 x 2048 x 4096, 1.34 rounds of 256 x 256: 175 against 195 for 2.69 of 128 x 256).
     auto cost = [&](int bm, int bn, int slots, double rate) { return tile_cost(p.M, p.N, batch, bm, bn, slots, rate); };
-    const double huge = cost(256, 256, 256, TRANS_A ? 1385.0 : TRANS_B ? 1490.0 : 1460.0);
-    const double wide = cost(128, 256, 256, TRANS_A ? 1147.0 : TRANS_B ? 1334.0 : 1180.0);
-    const double small = cost(128, 128, 512, TRANS_A ? 1190.0 : TRANS_B ? 959.0 : 1080.0);
+    const double huge = cost(256, 256, 256, TRANS_A ? 1440.0 : TRANS_B ? 1490.0 : 1460.0);
+    const double wide = cost(128, 256, 256, TRANS_A ? 1215.0 : TRANS_B ? 1280.0 : 1180.0);
+    const double small = cost(128, 128, 512, TRANS_A ? 1180.0 : TRANS_B ? 959.0 : 1080.0);
     if constexpr (!TRANS_A) {
-      if (cost(192, 256, 256, 1300.0) <= std::min({huge, wide, small})) return launch_pp<BF16, TRANS_A, TRANS_B, 3, 2, 4>(p, batch, stream);
+      if (cost(192, 256, 256, 1320.0) <= std::min({huge, wide, small})) return launch_il<BF16, TRANS_A, TRANS_B, 3>(p, batch, stream);
     }
-    if (huge <= wide && huge <= small) return launch_pp<BF16, TRANS_A, TRANS_B, 4, 2, 4>(p, batch, stream);
-    if (wide <= small) return launch_pp<BF16, TRANS_A, TRANS_B, 2, 2, 4, 64>(p, batch, stream);
+    if (huge <= wide && huge <= small) return rows_256();
+    if (wide <= small) return rows_128();
     return launch_dma<BF16, TRANS_A, TRANS_B, 2, 2, 32, 4>(p, batch, stream);
   }
   // One round of at most one 128 x 128 tile per CU and a long K: eight waves (64 x 32 each) and K steps of 64
@@ -341,8 +383,8 @@ int launch_shape(const GemmParams& p, int batch, int force, hipStream_t stream, 
 // straight into LDS: 5 = 128x128, 6 = 128x256, 7 = 256x256, 8 = 128x128, 9 = 64x128 by eight waves with K steps of 64,
 // 10 = 128x256 by eight waves, 11 = the same with K steps of 64, 12 = 256x256 with K split over two workgroups per tile
 // (iex_gemm_ws only; never chosen), 13 = 256x256 by eight waves in two groups that alternate between loading and
-// multiplying, 14 = 64x128 by eight waves with K split over two to eight workgroups per tile (iex_gemm_ws only), 15 = 128x256 like 13 in
-// phases of 64 k, 16 = 192x256 like 13.  0 = choose (one of 5, 8, 9, 13, 15, 16, and 14 where iex_gemm_workspace_bytes asked for room and got it).
+// multiplying (A as (K, M): in phase), 14 = 64x128 by eight waves with K split over two to eight workgroups per tile (iex_gemm_ws only), 15 = 128x256 like 13 in
+// phases of 64 k, 16 = 192x256 by eight waves in phase.  0 = choose (one of 5, 8, 9, 13, 15, 16, and 14 where iex_gemm_workspace_bytes asked for room and got it).
 extern "C" int iex_gemm_ws(int dtype, int code, int M, int N, int K, const void* A, const void* B, void* C, int batch,
                            long long stride_a, long long stride_b, long long stride_c, void* stream, void* workspace, size_t workspace_bytes) {
   iex::trail_reset();
@@ -370,7 +412,7 @@ size_t iex::gemm_auto_split_bytes(int M, int N, int K, int batch) {
 // Seconds of C = A B with B as (K, N), as launch_shape would run it with a workspace, with launch, prologue and epilogue.
 double iex::gemm_seconds(int M, int N, int K) {
   if ((long long)ceil_div(M, 128) * ceil_div(N, 128) > 256 && K > 256) {
-    const double best = std::min({tile_cost(M, N, 1, 256, 256, 256, 1460.0), tile_cost(M, N, 1, 192, 256, 256, 1300.0), tile_cost(M, N, 1, 128, 256, 256, 1180.0),
+    const double best = std::min({tile_cost(M, N, 1, 256, 256, 256, 1460.0), tile_cost(M, N, 1, 192, 256, 256, 1320.0), tile_cost(M, N, 1, 128, 256, 256, 1180.0),
                                   tile_cost(M, N, 1, 128, 128, 512, 1080.0)});
     return 6e-6 + best * K * 2e-12;
   }

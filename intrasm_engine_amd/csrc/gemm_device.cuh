@@ -22,9 +22,22 @@
 // then holds 4 adjacent columns of one row of C per accumulator quad and stores them
 // with one 64-bit store.
 #pragma once
+#include <type_traits>
+#include <utility>
+
 #include "iex_common.h"
 
 namespace iex {
+
+// f(0), .., f(COUNT - 1), each number a type
+template <typename F, int... N>
+__device__ __forceinline__ void for_each_of(F&& f, std::integer_sequence<int, N...>) {
+  (f(std::integral_constant<int, N>{}), ...);
+}
+template <int COUNT, typename F>
+__device__ __forceinline__ void for_each_number(F&& f) {
+  for_each_of(f, std::make_integer_sequence<int, COUNT>{});
+}
 
 struct GemmParams {
   int M, N, K;

@@ -27,6 +27,7 @@
 // the end of the interval before group 0 reads it (group 0: after C(p), group 1: after M(p)) and the barrier publishes
 // them.  Chunk permutations and the hand-written load counts follow gemm_dma_device.cuh; per accumulator the MFMAs
 // run in the same k order, so results are bit-equal to that kernel's.
+// 192 rows, and A as (K, M), are faster with single instructions between the MFMAs: gemm_il_device.cuh, with the figures of both.
 #pragma once
 #include "gemm_dma_device.cuh"
 
@@ -44,7 +45,7 @@ namespace iex {
 template <int WM, int WN, int WCN, int KP>
 constexpr int gemm_pp_lds_bytes() { return 3 * (2 * WM * 32) * 128 + (KP == 32 ? 4 * 64 : 3 * 128) * (WCN * WN * 32); }
 
-template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, bool TRANS_A = false, int KP = 32>
+template <bool BF16, bool TRANS_B, int WM, int WN, int WCN, int KP = 32>
 __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, int tile_n, int z, unsigned char* smem) {
   constexpr int BM = 2 * WM * 32, BN = WCN * WN * 32, WAVES = 2 * WCN;
   constexpr int SA = 3, SB = KP == 32 ? 4 : 3;        // stages of A (64 k each) and of B (KP each)
@@ -55,13 +56,12 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   constexpr int B_INSTR = B_STAGE / 1024 / WAVES;     // ... and B tile
   // Loads per wavefront that may be in flight where a phase ends: those of two phases (one, for KP = 64).
   constexpr int FLY = A_INSTR + HALVES * B_INSTR;
-  constexpr int CPRB = BN / 8, CPRA = BM / 8;         // (K,N), (K,M) layout: chunks per k row
+  constexpr int CPRB = BN / 8;                        // (K,N) layout: chunks per k row
   static_assert(WAVES == 8, "two wavefronts per SIMD");
   static_assert(KP == 32 || KP == 64, "k per phase");
   static_assert(A_INSTR >= HALVES && B_INSTR >= 1 && A_STAGE % (1024 * WAVES) == 0 && B_STAGE % (1024 * WAVES) == 0,
                 "every wavefront fetches whole kilobytes of A (in HALVES parts) and of B");
   static_assert(TRANS_B || (CPRB >= 16 && CPRB <= 64), "(K,N) layout: 128 <= BN <= 512");
-  static_assert(!TRANS_A || CPRA == 16 || CPRA == 32 || CPRA == 64, "(K,M) layout: BM is 128, 256 or 512");
   static_assert(FLY + A_INSTR + B_INSTR < 64, "loads in flight must fit the load counter");
   typedef unsigned short u16;
   typedef __attribute__((address_space(3))) unsigned char lds_u8;
@@ -76,22 +76,20 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   const u16* __restrict__ B = static_cast<const u16*>(p.B) + (size_t)z * p.stride_b;
   u16* __restrict__ C = static_cast<u16*>(p.C) + (size_t)z * p.stride_c;
   const unsigned lds0 = (unsigned)(size_t)(lds_u8*)smem;
-  const int lda = p.lda ? p.lda : TRANS_A ? p.M : p.K, ldb = p.ldb ? p.ldb : TRANS_B ? p.K : p.N;   // row strides
+  const int lda = p.lda ? p.lda : p.K, ldb = p.ldb ? p.ldb : TRANS_B ? p.K : p.N;   // row strides
   const int kb = p.kb ? p.kb : p.K;   // the k rows of a (K,N) B
 
   // ---- what this lane fetches (gemm_addresses.h).  A: 8 rows of 128 bytes per instruction, LDS position (row, c) holds global chunk
   // c ^ ((row >> 1) & 7).  B as (N,K): the same, or 16 rows of 64 bytes, chunk c ^ ((row >> 2) & 3).  B as (K,N): k rows of BN
-  // elements, chunk c ^ kn16_swizzle(k), and A as (K,M) likewise, 64 k rows of BM elements per stage.
+  // elements, chunk c ^ kn16_swizzle(k).
   // Rows past M (columns past N) are the last one's: they feed rows (columns) of C that are not stored.
-  const u32x4 a_buf = TRANS_A ? buffer_of(A, rows_bytes(p.K, p.M, lda)) : buffer_of(A + (size_t)m0 * lda, rows_bytes(p.M - m0, p.K, lda));
+  const u32x4 a_buf = buffer_of(A + (size_t)m0 * lda, rows_bytes(p.M - m0, p.K, lda));
   const u32x4 b_buf = TRANS_B ? buffer_of(B + (size_t)n0 * ldb, rows_bytes(p.N - n0, p.K, ldb)) : buffer_of(B, rows_bytes(kb, p.N, ldb));
   unsigned a_lane[A_INSTR], b_lane[B_INSTR];   // byte offset inside the buffer at k = 0
   int a_k8[A_INSTR], b_k8[B_INSTR];            // K-contiguous: first k of the chunk inside a tile; else k row inside a tile
 #pragma unroll
   for (int q = 0; q < A_INSTR; ++q) {
-    DirectChunk c;
-    if constexpr (TRANS_A) c = column_chunk<BM>(wave * A_INSTR + q, lane, m0, lda);
-    else c = row_chunk<64>(wave * A_INSTR + q, lane, p.M - m0, lda);
+    const DirectChunk c = row_chunk<64>(wave * A_INSTR + q, lane, p.M - m0, lda);
     a_lane[q] = c.offset;
     a_k8[q] = c.k;
   }
@@ -105,7 +103,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   }
   const int P = (p.K + KP - 1) / KP;   // phases
   const int TA = (p.K + 63) / 64;      // A tiles
-  const unsigned a_step = (TRANS_A ? 64u * lda : 64u) * 2u, b_step = (TRANS_B ? (unsigned)KP : (unsigned)KP * ldb) * 2u;   // bytes per tile
+  const unsigned a_step = 64u * 2u, b_step = (TRANS_B ? (unsigned)KP : (unsigned)KP * ldb) * 2u;   // bytes per tile
 
   // part h (of HALVES; of an odd number of instructions the second has one more) of A tile t into stage `base`; past the end: the last tile again, into a
   // stage nobody reads.  (A chunk past a row's end is the next row's, or nothing: zero_tail.)
@@ -141,14 +139,9 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
   // ---- operand read addresses inside a stage (bytes): a fragment is 16 rows (columns) x 32 k, lane l has row l % 16 and
   // the 8 k of chunk l / 16
   const int frow = lane & 15, fch = lane >> 4;
-  int a_off[TRANS_A ? 2 * WM : 2];   // the two halves of an A tile, or the row blocks of a (K,M) one
-  if constexpr (TRANS_A) {
+  int a_off[2];   // the two halves of an A tile
 #pragma unroll
-    for (int i = 0; i < 2 * WM; ++i) a_off[i] = kn16_fragment_offset<BM>(lane, wm * 2 * WM + i);
-  } else {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) a_off[h] = (wm * WM * 32 + frow) * 128 + (((h * 4 + fch) ^ (frow >> 1)) * 16);
-  }
+  for (int h = 0; h < 2; ++h) a_off[h] = (wm * WM * 32 + frow) * 128 + (((h * 4 + fch) ^ (frow >> 1)) * 16);
   int b_off[TRANS_B ? SUB : 2 * WN];
   if constexpr (TRANS_B) {
 #pragma unroll
@@ -172,10 +165,7 @@ __device__ __forceinline__ void gemm_tile_pp(const GemmParams& p, int tile_m, in
 #pragma unroll
     for (int s = 0; s < SUB; ++s) {
 #pragma unroll
-      for (int i = 0; i < 2 * WM; ++i) {
-        if constexpr (TRANS_A) fa[s][i] = kn_fragment<BM * 2>(sa + a_off[i] + (h + s) * 32 * (BM * 2));
-        else fa[s][i] = *reinterpret_cast<const u32x4*>(sa + a_off[h + s] + i * 16 * 128);
-      }
+      for (int i = 0; i < 2 * WM; ++i) fa[s][i] = *reinterpret_cast<const u32x4*>(sa + a_off[h + s] + i * 16 * 128);
 #pragma unroll
       for (int j = 0; j < 2 * WN; ++j) {
         if constexpr (TRANS_B) fb[s][j] = *reinterpret_cast<const u32x4*>(sb + b_off[s] + j * 16 * (KP * 2));

@@ -291,16 +291,6 @@ __device__ __forceinline__ f32x4 smfmac_16x16x64(u32x4 a, u32x8 b, f32x4 c, unsi
   else return __builtin_amdgcn_smfmac_f32_16x16x64_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x16, b), c, (int)index, 0, HIGH);
 }
 
-// f(0), .., f(COUNT - 1), each number a type
-template <typename F, int... N>
-__device__ __forceinline__ void for_each_of(F&& f, std::integer_sequence<int, N...>) {
-  (f(std::integral_constant<int, N>{}), ...);
-}
-template <int COUNT, typename F>
-__device__ __forceinline__ void for_each_number(F&& f) {
-  for_each_of(f, std::make_integer_sequence<int, COUNT>{});
-}
-
 // 4 bytes per lane, lane i's at M0 + 4 * i (cf. lds_dma16)
 __device__ __forceinline__ void lds_dma4(u32x4 rsrc, unsigned lane_offset, unsigned uniform_offset, unsigned lds_base_uniform) {
   asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dword %0, %1, %2 offen lds" ::"v"(lane_offset), "s"(rsrc), "s"(uniform_offset), "s"(lds_base_uniform) : "memory", "m0");
