@@ -163,7 +163,7 @@ int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream);
  * input.  Families 3-6 and 10 multiply explicit zeros with the dense operand, so a non-finite entry
  * in a row of `dense` that no nonzero references still reaches the output (0 * inf = NaN).
  * bits 20..23: rows per wavefront of family 2 (2, 4 or 8); windows of nonzeros held in
- * registers per row of family 4 (1, 2, 4 or 5 windows of 16), 5 (2, 4 or 8 windows of 8) and
+ * registers per row of family 4 (1, 2, 4 or 5 windows of 16), 5 (2, 4 or 8, without effect) and
  * 6 (1, 2 or 4 windows of 16).  0 = choose.                                              */
 #define IEX_SPMM_FORCE_VARIANT(v) (((v) & 0xf) << 16)
 #define IEX_SPMM_FORCE_RPW(r) (((r) & 0xf) << 20)

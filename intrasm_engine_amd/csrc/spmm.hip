@@ -440,34 +440,29 @@ int launch_mfma3(const SpmmParams& p, int batch, int windows, hipStream_t stream
 // arrangement code = MFMA tile height and how the 4 multiplying waves split the C tile:
 //   1 = 32 x 64 (4 k slices)    2 = 32 x 128 as 2 x 64 columns (2 k slices)    4 = 32 x 128 (4 k slices)
 //   5 = 16 x 64 (4 k slices)    6 = 16 x 128 as 2 x 64 columns (2 k slices)
-template <int MT, int NJ, int WAVES_N, int W, bool SPLIT>
+template <int MT, int NJ, int WAVES_N, bool SPLIT>
 __global__ __launch_bounds__(kF32Threads + (SPLIT ? MT * 8 : 0), 2) void spmm_mfma_f32_kernel(SpmmParams p, int tiles_m) {
   extern __shared__ __align__(16) unsigned char smem[];
-  spmm_mfma_f32_block<MT, NJ, WAVES_N, W, SPLIT>(p, blockIdx.x % tiles_m, blockIdx.x / tiles_m, blockIdx.y, smem);
+  spmm_mfma_f32_block<MT, NJ, WAVES_N, SPLIT>(p, blockIdx.x % tiles_m, blockIdx.x / tiles_m, blockIdx.y, smem);
 }
 
-template <int MT, int NJ, int WAVES_N, int W, bool SPLIT>
+template <int MT, int NJ, int WAVES_N, bool SPLIT>
 int launch_mfma_f32_one(const SpmmParams& p, int batch, hipStream_t stream) {
   constexpr int kBN = MT * NJ * WAVES_N;
   const int tiles_m = ceil_div(p.m, MT), tiles_n = ceil_div(p.n, kBN);
   constexpr int kLds = spmm_mfma_f32_lds_bytes<MT, NJ, WAVES_N>();
-  note_kernel("spmm_mfma_f32_kernel<%d, %d, %d, %d, %s>", MT, NJ, WAVES_N, W, SPLIT ? "true" : "false");
-  hipLaunchKernelGGL((spmm_mfma_f32_kernel<MT, NJ, WAVES_N, W, SPLIT>), dim3(tiles_m * tiles_n, batch),
+  note_kernel("spmm_mfma_f32_kernel<%d, %d, %d, %s>", MT, NJ, WAVES_N, SPLIT ? "true" : "false");
+  hipLaunchKernelGGL((spmm_mfma_f32_kernel<MT, NJ, WAVES_N, SPLIT>), dim3(tiles_m * tiles_n, batch),
                      dim3(kF32Threads + (SPLIT ? MT * 8 : 0)), kLds, stream, p, tiles_m);
   return check_hip(hipGetLastError(), "spmm (matrix-core, fp32) launch");
 }
 
 template <int MT, int NJ, int WAVES_N>
 int launch_mfma_f32_w(const SpmmParams& p, int batch, int windows, bool split, hipStream_t stream) {
-  // with separate expanding waves there are registers for 16 windows (the kernel uses as many
-  // of them as the rows of a wave need); waves that do both hold 2, 4 or 8
-  if (split) return launch_mfma_f32_one<MT, NJ, WAVES_N, 16, true>(p, batch, stream);
-  switch (windows) {
-    case 2: return launch_mfma_f32_one<MT, NJ, WAVES_N, 2, false>(p, batch, stream);
-    case 4: return launch_mfma_f32_one<MT, NJ, WAVES_N, 4, false>(p, batch, stream);
-    case 8: return launch_mfma_f32_one<MT, NJ, WAVES_N, 8, false>(p, batch, stream);
-  }
-  return fail(IEX_ERR_BAD_ARGUMENT, "spmm: windows of the fp32 matrix-core variant must be 2, 4 or 8 (got %d)", windows);
+  if (split) return launch_mfma_f32_one<MT, NJ, WAVES_N, true>(p, batch, stream);
+  // (the number of windows is the kernel's own affair by now; what was refused still is)
+  IEX_REQUIRE(windows == 2 || windows == 4 || windows == 8, IEX_ERR_BAD_ARGUMENT, "spmm: windows of the fp32 matrix-core variant must be 2, 4 or 8 (got %d)", windows);
+  return launch_mfma_f32_one<MT, NJ, WAVES_N, false>(p, batch, stream);
 }
 
 inline int launch_mfma_f32(const SpmmParams& p, int batch, int arrangement, int windows, bool split, hipStream_t stream) {
@@ -608,6 +603,7 @@ int mfma_f32_variant(const SpmmParams& p, int batch, const Choice& ch, int& wind
   if (!std::is_same<T, float>::value || !std::is_same<IT, int>::value) return 0;
   if (ch.variant != 0 && ch.variant != 5) return 0;
   if (!(p.nnz > 0 && p.n % 4 == 0 && aligned(p.dense, 16) && aligned(p.out, 16))) return 0;  // (also when forced)
+  if (p.nnz >= 1 << 30 || ((long long)p.k + 1024) * p.n >= 1 << 30) return 0;                 // 32-bit byte offsets
   const double density = (p.m > 0 && p.k > 0) ? (double)p.nnz / ((double)p.m * p.k) : 0.0;
   // 32-row tiles with 128 columns per wave when that still gives most CUs a workgroup; else
   // 16-row tiles (twice the workgroups, twice the reads of the dense operand)
@@ -627,7 +623,8 @@ int mfma_f32_variant(const SpmmParams& p, int batch, const Choice& ch, int& wind
   if (density >= 0.27 && arrangement == 4 && fill >= 0.75) return arrangement;
   // Beside a kernel that is bound by gathers the tie at 20 % goes to the matrix cores, also with the 16-row tiles of
   // n = 128: alone 124 against 118 us (4096 x 4096 at 20 %, n = 256) and 90 against 84 us (30 %, n = 128), but the
-  // neighbour then has the L2 -> CU path to itself (the 15 cells of that sweep on two branches of a graph: 654 -> 600 us).
+  // neighbour then has the L2 -> CU path to itself (the 15 cells of that sweep on two branches of a graph: 654 -> 600 us).  (The
+  // expansion of today: 112 and 74.)
   if (ch.beside_gather && density >= 0.195 && p.n >= 128 && fill >= 0.75) return arrangement;
   return 0;
 }

@@ -6,10 +6,9 @@
 // and 16 k rows per group: a wave then has four k slots of 16 lanes instead of two of 32.)
 //
 // Workgroup = 4 multiplying wavefronts, C tile = MT rows (CSR rows in swizzled order) x BN columns.
-//   A   chunks of 128 columns, double-buffered [32][132] floats in LDS.  A group of 8 lanes
-//       owns one row: cursor, row end and W windows of 8 nonzeros in registers; chunk c+1 is
-//       expanded before the MFMAs of chunk c are issued and the windows are reloaded right
-//       after, so those loads land during the MFMAs.  One barrier per chunk.
+//   A   chunks of 128 columns, double-buffered [32][132] floats in LDS.  A wavefront expands 8 rows, a
+//       lane a nonzero: the next 64 of every row are in registers (128 where rows are that dense), so those loads land
+//       during the MFMAs of a chunk.  One barrier per chunk.
 //   B   (k x n row-major) never touches LDS: with a 32-row tile every element of B feeds
 //       exactly one MFMA of the workgroup, and the MFMA operand layout (lane = column, half
 //       wave = k) is a coalesced global load already.  A lane loads NJ adjacent columns
@@ -21,14 +20,19 @@
 //       128-bit LDS read of A per lane and group: lanes 0-31 take k .. k+3, lanes 32-63
 //       k+4 .. k+7, the B loads follow the same assignment); partial tiles are added through
 //       LDS at the end in a fixed order (deterministic).
-// Loads of B run four groups (4 x 4 loads per lane) ahead of the MFMAs.
-// SPLIT: the workgroup has 8 wavefronts with two roles.  Waves 0-3 only multiply, waves 4-7
-// only expand the next chunk; one of each shares a SIMD, so the vector-ALU work of the
-// expansion runs beside the other wave's MFMAs instead of in front of them, and the
-// multiplying waves carry no loop around loads (the compiler can then count their loads in
-// flight exactly).  Without SPLIT all 4 waves do both, one after the other.
+// Loads of B run four groups (4 x 4 loads per lane) ahead of the MFMAs, by buffer address: their positions are scalar.
+// SPLIT: the workgroup has 8 wavefronts with two roles, each with a loop of its own.  Waves 0-3 only multiply, waves 4-7
+// only expand the next chunk; one of each shares a SIMD.  Without SPLIT all 4 waves do both, one after the other.
+// What bounds it: the MFMAs, which hold the SIMD's vector ALU for 64 clocks each and slip into every gap between two vector
+// instructions of the expanding wavefront.  That wavefront's vector instructions were the longer chain (up to 160 per
+// chunk of 64 MFMAs, eight lanes to a row and windows of 8 nonzeros): with a lane per nonzero, the rows' instructions side by
+// side, positions and masks in scalar registers, they are 16 - 40.  MI355X, us before -> now: 4096 x 4096, n = 256, rows of
+// geometric lengths, 20 % and 30 % density 128 -> 112, rows of one length, 2 / 10 / 30 / 50 / 100 % 86 / 91 / 104 / 116 / 130 -> 90 / 91 /
+// 92 / 109 / 112; n = 128 (16 rows), geometric 92 -> 74, equal 30 % 68 -> 56; 11008 x 4096, n = 1024, 30 % 1051 -> 1023.  (Expanding wavefronts
+// at raised priority: 2 us more.)
 // Requirements (checked by the host): n % 4 == 0, 16-byte aligned dense operand and output,
-// strictly ascending column indices inside a row.
+// strictly ascending column indices inside a row, (k + 1024) n and
+// nnz below 2^30 (32-bit byte offsets).
 #pragma once
 #include "spmm_device.cuh"
 
@@ -54,7 +58,7 @@ struct F32Frag {
   float v[NJ];
 };
 
-template <int MT, int NJ, int WAVES_N, int W, bool SPLIT>
+template <int MT, int NJ, int WAVES_N, bool SPLIT>
 __device__ __forceinline__ void spmm_mfma_f32_block(const SpmmParams& p, int tile_m, int tile_n, int z, unsigned char* smem) {
   constexpr int BM = MT, BKA = spmm_mfma_f32_bka<MT>();
   constexpr int LDA = BKA + 4;            // floats: 16 consecutive rows start in distinct 4-bank groups
@@ -66,178 +70,198 @@ __device__ __forceinline__ void spmm_mfma_f32_block(const SpmmParams& p, int til
   constexpr int BN = WCOLS * WAVES_N;     // columns of the workgroup
   constexpr int GROUPS = BKA / GK;        // groups per chunk (16 or 8)
   constexpr int GPW = GROUPS / WAVES_K;   // groups per wave and chunk
-  constexpr int LPR = 8;                  // lanes per row of the expansion
-  constexpr int EXP_THREADS = MT * LPR;   // threads that expand (256 or 128)
+  constexpr int EXP_ROWS = 8;                       // rows an expanding wavefront owns
+  constexpr int EXP_THREADS = MT / EXP_ROWS * 64;   // threads that expand (256 or 128)
   typedef float acc_t __attribute__((ext_vector_type(ACC)));
   static_assert(MT == 32 || MT == 16, "MFMA tile height");
   constexpr int AHEAD = GPW < 4 ? GPW : 4;  // groups of B loads in flight
-  constexpr int kNoCol = 0x7fffffff;
   static_assert(NJ == 2 || NJ == 4, "a lane loads 2 or 4 adjacent columns");
   static_assert(GPW % AHEAD == 0, "the prefetch ring is unrolled over the groups of a chunk");
 
   float* sA = reinterpret_cast<float*>(smem);  // [2][BM][LDA]
 
   const int lane = threadIdx.x & 63;
-  const bool is_mma = threadIdx.x < kF32Threads;                                   // wave-uniform roles
-  const bool is_exp = SPLIT ? threadIdx.x >= kF32Threads : threadIdx.x < EXP_THREADS;
-  const int tid = threadIdx.x % kF32Threads;                // index inside the role
-  const int wave = tid >> 6;
+  const int wave_id = uniform(threadIdx.x >> 6);
+  const bool is_mma = wave_id < kF32Threads / 64;                                   // wave-uniform roles
+  const bool is_exp = SPLIT ? !is_mma : wave_id < EXP_THREADS / 64;
+  const int wave = wave_id % (kF32Threads / 64);
   const int wn = wave % WAVES_N, wk = wave / WAVES_N;
   const int half = lane / MT;  // k slot: which 4 of the GK k rows of a group this lane feeds
   const int l32 = lane % MT;   // row (A fragment) / column slot (B fragment) of this lane
   const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const float* __restrict__ values = static_cast<const float*>(p.values) + (p.per_batch_values ? (size_t)z * p.nnz : (size_t)0);
-  const int* __restrict__ cols = static_cast<const int*>(p.cols);
-  const float* __restrict__ B = static_cast<const float*>(p.dense) + (size_t)z * p.k * p.n;
+  const float* values = static_cast<const float*>(p.values) + (p.per_batch_values ? (size_t)z * p.nnz : (size_t)0);
+  const float* B = static_cast<const float*>(p.dense) + (size_t)z * p.k * p.n;
   float* __restrict__ C = static_cast<float*>(p.out) + (size_t)z * p.m * p.n;
+  // Raw buffers: what lies past their end reads as zero, and the position inside costs no vector instruction.
+  auto buffer = [](const void* at, size_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(at), 0, (int)(unsigned)bytes, 4 << 15); };
+  const auto vals_buf = buffer(values, (size_t)p.nnz * 4), cols_buf = buffer(p.cols, (size_t)p.nnz * 4), b_buf = buffer(B, (size_t)p.k * p.n * 4);
 
-  // ---- expansion: lane group tid / 8 owns local row tid / 8 -------------------------------
-  const int sub = tid % LPR;
-  const int erow = tid / LPR;
-  const int gshift = lane & ~(LPR - 1);
-  int pos = 0, end = 0;
-  if (is_exp) {
-    const int slot = m0 + erow;
-    if (slot < p.m) {
-      const int row = p.row_indices[slot];
-      pos = p.row_offsets[row];
-      end = p.row_offsets[row + 1];
-    }
-  }
-  // W register windows of 8 nonzeros per row; the first wcnt of them are used (wave-uniform:
-  // enough for 1.3 x the run a row of this wave would have per chunk if its nonzeros were
-  // spread evenly, plus one).  A denser stretch than that falls back to the loop in expand().
-  int wc[W];
-  float wv[W];
-  int wcnt = W;
-  if (W > 8) {
-    int need = (int)(((long long)(end - pos) * BKA * 13 / 10 / (p.k > 0 ? p.k : 1) + LPR - 1) / LPR) + 1;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) need = max(need, __shfl_xor(need, o));
-    wcnt = min(W, need);
-  }
-  // (loads are unconditional with a clamped index and no arithmetic on the result: no branches
-  // and no wait at the load, so they overlap the MFMAs; the host guarantees nnz > 0)
-  const int last_nz = p.nnz - 1;
+  // ---- expansion: wavefront w owns local rows 8 w .. 8 w + 7, a lane a nonzero.  The next 64 nonzeros of every row are in
+  // registers (128 where a row of the wavefront has more than 40 in a chunk on average); a chunk takes 128 at most.
+  int pos[EXP_ROWS], end[EXP_ROWS], c0[EXP_ROWS], c1[EXP_ROWS];
+  float v0[EXP_ROWS], v1[EXP_ROWS];
+  bool wide = false;
+  // (scalar offsets never pass a buffer's end: only up to there does the range check hold)
+  auto load_window = [&](int first, int skip, int& c, float& v) {
+    c = __builtin_amdgcn_raw_buffer_load_b32(cols_buf, (lane + skip) * 4, (unsigned)first * 4u, 0);
+    v = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(vals_buf, (lane + skip) * 4, (unsigned)first * 4u, 0));
+  };
   auto load_windows = [&]() {
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      if (w >= wcnt) break;  // wave-uniform
-      const int idx = pos + w * LPR + sub;
-      const int safe = min(idx, last_nz);
-      wc[w] = cols[safe];   // raw: whether idx < end is decided at use, so that nothing
-      wv[w] = values[safe]; // here waits for the loads
+    for (int r = 0; r < EXP_ROWS; ++r) load_window(pos[r], 0, c0[r], v0[r]);
+    if (wide) {
+#pragma unroll
+      for (int r = 0; r < EXP_ROWS; ++r) load_window(pos[r], 64, c1[r], v1[r]);
     }
   };
-  if (is_exp) load_windows();
-  // Columns [ka0, ka0 + BKA) of the row -> abuf.  Zero fill and scatter come from the same
-  // wavefront, and LDS keeps the order of a wavefront's accesses.
-  auto expand = [&](int ka0, float* abuf) {
-    float* rowp = abuf + erow * LDA;
+  if (is_exp) {
 #pragma unroll
-    for (int q = 0; q < BKA / 4 / LPR; ++q) *reinterpret_cast<f32x4_t*>(rowp + (q * LPR + sub) * 4) = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const int kend = ka0 + BKA;
-    int consumed = 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      if (w >= wcnt) break;  // wave-uniform
-      const bool in = pos + w * LPR + sub < end && wc[w] < kend;
-      if (in) rowp[wc[w] - ka0] = wv[w];
-      consumed += __popcll((__ballot(in) >> gshift) & 0xffull);
-    }
-    pos += consumed;
-    // every window consumed: the run may go on -- unless the windows already span a whole chunk
-    bool more = consumed == wcnt * LPR && wcnt * LPR < BKA;
-    while (__any(more)) {  // a run longer than the windows held in registers: loads are exposed here
-      int c = kNoCol;
-      float v = 0.f;
-      const int idx = pos + sub;
-      if (more && idx < end) {
-        c = cols[idx];
-        v = values[idx];
+    for (int r = 0; r < EXP_ROWS; ++r) {
+      const int slot = m0 + wave * EXP_ROWS + r;
+      pos[r] = end[r] = 0;
+      c1[r] = 0, v1[r] = 0.f;
+      if (slot < p.m) {
+        const int row = uniform(p.row_indices[slot]);
+        pos[r] = uniform(p.row_offsets[row]);
+        end[r] = uniform(p.row_offsets[row + 1]);
       }
-      const bool in = c < kend;
-      if (in) rowp[c - ka0] = v;
-      const int cnt = __popcll((__ballot(in) >> gshift) & 0xffull);
-      pos += cnt;
-      more = cnt == LPR;
+      wide = wide || (long long)(end[r] - pos[r]) * BKA > (long long)p.k * 40;
+    }
+    load_windows();
+  }
+  // Columns [ka0, ka0 + BKA) of the wavefront's rows -> abuf.  Zeros and nonzeros come from the same wavefront, and LDS keeps
+  // the order of a wavefront's accesses.  An MFMA holds the vector ALU for 64 clocks and slips into every gap between two
+  // vector instructions of this wavefront: so few of them, the rows' side by side, all else in scalar registers.
+  auto first_of = [](int left) { return left >= 64 ? ~0ull : left > 0 ? (1ull << left) - 1 : 0ull; };
+  auto expand = [&](int ka0, float* abuf) {
+    float* mine = abuf + wave * EXP_ROWS * LDA;
+    constexpr int QUADS = EXP_ROWS * LDA / 4;
+#pragma unroll
+    for (int q = 0; q < (QUADS + 63) / 64; ++q)
+      if (q * 64 + 63 < QUADS || q * 64 + lane < QUADS) reinterpret_cast<f32x4_t*>(mine)[q * 64 + lane] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int kend = ka0 + BKA;
+    unsigned long long in[EXP_ROWS];
+    bool more = false;
+#pragma unroll
+    for (int r = 0; r < EXP_ROWS; ++r) {
+      in[r] = __ballot(c0[r] < kend) & first_of(end[r] - pos[r]);
+      more = more || in[r] == ~0ull;
+    }
+#pragma unroll
+    for (int r = 0; r < EXP_ROWS; ++r)
+      if (__builtin_amdgcn_inverse_ballot_w64(in[r])) mine[r * LDA + (c0[r] - ka0)] = v0[r];
+#pragma unroll
+    for (int r = 0; r < EXP_ROWS; ++r) pos[r] += __popcll(in[r]);
+    if (more) {   // (uniform) the second half of a chunk with 64 and more
+      if (!wide) {
+#pragma unroll
+        for (int r = 0; r < EXP_ROWS; ++r) load_window(pos[r], 0, c1[r], v1[r]);   // (of the others: what follows, none of it in the chunk)
+      }
+#pragma unroll
+      for (int r = 0; r < EXP_ROWS; ++r) in[r] = in[r] == ~0ull ? __ballot(c1[r] < kend) & first_of(end[r] - pos[r]) : 0ull;
+#pragma unroll
+      for (int r = 0; r < EXP_ROWS; ++r)
+        if (__builtin_amdgcn_inverse_ballot_w64(in[r])) mine[r * LDA + (c1[r] - ka0)] = v1[r];
+#pragma unroll
+      for (int r = 0; r < EXP_ROWS; ++r) pos[r] += __popcll(in[r]);
     }
     load_windows();
   };
 
   // ---- B: the 4 k rows of group g (chunk-relative) that this lane feeds ----------------------
+  // A k row beyond the matrix reads as zeros and meets zeros of A; a column beyond n is computed and never stored.
   const int col = n0 + wn * WCOLS + l32 * NJ;  // first of the NJ columns of this lane
-  const bool col_ok = col < p.n;               // n % 4 == 0: the NJ columns are in or out together
-  // Loads are clamped to valid addresses instead of masked: a k row beyond the matrix meets
-  // zeros of A, a column beyond n is computed and never stored.
-  const float* __restrict__ bsafe = B + (col_ok ? col : 0);
-  const int last_k = p.k - 1;
+  unsigned b_lane[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b_lane[i] = (unsigned)((half * 4 + i) * p.n + (col < p.n ? col : 0)) * 4u;   // n % 4 == 0: the NJ columns are in or out together
   auto load_b = [&](F32Frag<NJ> (&f)[4], int kbase) {  // kbase = first k row of the group
+    const unsigned at = (unsigned)min(kbase, p.k) * (unsigned)p.n * 4u;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float* src = bsafe + (size_t)min(kbase + half * 4 + i, last_k) * p.n;
       if constexpr (NJ == 4) {
-        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(src);
+        typedef int i32x4_t __attribute__((ext_vector_type(4)));
+        const i32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(b_buf, b_lane[i], at, 0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) f[i].v[j] = v[j];
+        for (int j = 0; j < 4; ++j) f[i].v[j] = __int_as_float(v[j]);
       } else {
-        const float2 v = *reinterpret_cast<const float2*>(src);
-        f[i].v[0] = v.x;
-        f[i].v[1] = v.y;
+        typedef int i32x2_t __attribute__((ext_vector_type(2)));
+        const i32x2_t v = __builtin_amdgcn_raw_buffer_load_b64(b_buf, b_lane[i], at, 0);
+        f[i].v[0] = __int_as_float(v[0]);
+        f[i].v[1] = __int_as_float(v[1]);
       }
     }
   };
+
+  // group index of this wave, global over chunks: gi -> k row (gi / GPW) * BKA + ((gi % GPW) * WAVES_K + wk) * 8
+  auto group_k = [&](int gi) { return (gi / GPW) * BKA + ((gi % GPW) * WAVES_K + wk) * GK; };
+  const int n_chunks = (p.k + BKA - 1) / BKA;
+  auto buffer_of_chunk = [&](int c) { return sA + (c & 1) * BM * LDA; };
+
+  if (SPLIT && is_exp) {   // (a loop of its own: neither role's registers are live in the other's)
+    expand(0, sA);
+    __syncthreads();
+    for (int c = 0; c < n_chunks; ++c) {
+      if (c + 1 < n_chunks) expand((c + 1) * BKA, buffer_of_chunk(c + 1));
+      __syncthreads();
+    }
+    __syncthreads();
+    if constexpr (WAVES_K > 1) __syncthreads();   // (the partial tiles)
+    return;
+  }
 
   acc_t acc[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j)
 #pragma unroll
     for (int r = 0; r < ACC; ++r) acc[j][r] = 0.f;
-
-  // group index of this wave, global over chunks: gi -> k row (gi / GPW) * BKA + ((gi % GPW) * WAVES_K + wk) * 8
-  auto group_k = [&](int gi) { return (gi / GPW) * BKA + ((gi % GPW) * WAVES_K + wk) * GK; };
-  const int n_chunks = (p.k + BKA - 1) / BKA;
-
   F32Frag<NJ> ring[AHEAD][4];
-  if (is_mma) {
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a) load_b(ring[a], group_k(a));
-  }
-  if (is_exp) expand(0, sA);
+  for (int a = 0; a < AHEAD; ++a) load_b(ring[a], group_k(a));
+  if (!SPLIT && is_exp) expand(0, sA);
   __syncthreads();
 
   // The scheduling barriers pin the order "MFMAs of group g, then the loads that refill its
   // ring slot": left alone, the compiler sinks all loads of a chunk behind its last MFMA and
-  // the next chunk starts by waiting for them.
+  // the next chunk starts by waiting for them.  A's fragment of a group is read a group ahead, that of the next chunk's first
+  // group behind the barrier, which stands before the last group of a chunk: everything of the chunk is in registers there.
+  const float* a_lane = sA + l32 * LDA + half * 4 + wk * GK;
+  f32x4_t fa = *reinterpret_cast<const f32x4_t*>(a_lane);
   for (int c = 0; c < n_chunks; ++c) {
-    if (is_exp && c + 1 < n_chunks) expand((c + 1) * BKA, sA + ((c + 1) & 1) * BM * LDA);
+    if (!SPLIT && is_exp && c + 1 < n_chunks) expand((c + 1) * BKA, buffer_of_chunk(c + 1));
     __builtin_amdgcn_sched_barrier(0);
-    if (is_mma) {
-      const float* a = sA + (c & 1) * BM * LDA + l32 * LDA + half * 4 + wk * GK;
+    const float* a = a_lane + (c & 1) * BM * LDA;
+    const float* a_next = a_lane + ((c + 1) & 1) * BM * LDA;
 #pragma unroll
-      for (int g = 0; g < GPW; ++g) {
-        const f32x4_t fa = *reinterpret_cast<const f32x4_t*>(a + g * WAVES_K * GK);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) {
-            if constexpr (MT == 32) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ring[g % AHEAD][i].v[j], fa[i], acc[j], 0, 0, 0);
-            else acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ring[g % AHEAD][i].v[j], fa[i], acc[j], 0, 0, 0);
-          }
-        __builtin_amdgcn_sched_barrier(0);
-        load_b(ring[g % AHEAD], group_k(c * GPW + g + AHEAD));  // (past the end: clamped, unused)
-        __builtin_amdgcn_sched_barrier(0);
+    for (int g = 0; g < GPW; ++g) {
+      f32x4_t next;
+      if (g + 1 < GPW) {
+        next = *reinterpret_cast<const f32x4_t*>(a + (g + 1) * WAVES_K * GK);
+      } else {
+        __syncthreads();
+        next = *reinterpret_cast<const f32x4_t*>(a_next);   // (past the last chunk: read, never used)
       }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          if constexpr (MT == 32) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ring[g % AHEAD][i].v[j], fa[i], acc[j], 0, 0, 0);
+          else acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ring[g % AHEAD][i].v[j], fa[i], acc[j], 0, 0, 0);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+      load_b(ring[g % AHEAD], group_k(c * GPW + g + AHEAD));  // (past the end: zeros, unused)
+      __builtin_amdgcn_sched_barrier(0);
+      fa = next;
     }
-    __syncthreads();
   }
+  __syncthreads();   // everybody is done with A's buffers
 
   if constexpr (WAVES_K > 1) {
     // partial tiles of the k slices -> LDS (the A buffers are free after the last barrier),
     // added by the wavefront of slice 0 in slice order
     constexpr int Q = ACC / 4;  // 128-bit pieces of an accumulator tile per lane
     f32x4_t* red = reinterpret_cast<f32x4_t*>(smem);  // [WAVES_K - 1][WAVES_N][NJ * Q][64]
-    if (is_mma && wk > 0) {
+    if (wk > 0) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -246,7 +270,7 @@ __device__ __forceinline__ void spmm_mfma_f32_block(const SpmmParams& p, int til
               f32x4_t{acc[j][q * 4], acc[j][q * 4 + 1], acc[j][q * 4 + 2], acc[j][q * 4 + 3]};
     }
     __syncthreads();
-    if (!is_mma || wk > 0) return;
+    if (wk > 0) return;
 #pragma unroll
     for (int s = 1; s < WAVES_K; ++s)
 #pragma unroll
@@ -262,7 +286,7 @@ __device__ __forceinline__ void spmm_mfma_f32_block(const SpmmParams& p, int til
   // Swapped operands: lane holds row (lane % MT) of the tile; accumulator slot v of MFMA j is
   // column NJ * ((v / 4) * 4 * KSLOTS + (lane / MT) * 4 + v % 4) + j of the wave's column range.
   const int slot = m0 + l32;
-  if (!is_mma || slot >= p.m) return;
+  if (slot >= p.m) return;
   const int row = p.row_indices[slot];
   const float bias = p.bias ? p.bias[row] : 0.f;
 #pragma unroll
