@@ -271,7 +271,7 @@ __device__ __forceinline__ void spmm_mfma_f32_block(const SpmmParams& p, int til
     }
     __syncthreads();
     if (wk > 0) return;
-#pragma unroll
+#pragma unroll 1   // (unrolled, all the reads at once: more registers than there are)
     for (int s = 1; s < WAVES_K; ++s)
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
