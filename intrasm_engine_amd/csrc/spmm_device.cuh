@@ -19,6 +19,7 @@
 //     needs no atomics.
 // Accumulation is fp32 for every element type.  Padding slots are never dereferenced.
 #pragma once
+#include <type_traits>
 #include "iex_common.h"
 
 namespace iex {
@@ -67,7 +68,9 @@ struct row_slab {
 // give a correct partition of the row's nonzeros over the wpr wavefronts that call this for the row.
 // WIN = gathers a wave keeps in flight (rolling window); raise it where few waves fit a CU.
 // RAGGED = vectors at element alignment (n not a multiple of VEC).
-template <typename T, typename IT, int VEC, int LPG, int WIN, int NT, bool RAGGED>
+// TAIL = what is left of a chunk after whole windows goes in windows of four and of two, then one gather at a time (several
+// nonzeros per gather; a chunk of 31 with four to a gather: 4 round trips to L2 instead of 8).
+template <typename T, typename IT, int VEC, int LPG, int WIN, int NT, bool RAGGED, bool TAIL = true>
 __device__ __forceinline__ void spmm_range_partial(const SpmmParams& p, int z, int start, int end, int part, int wpr, const int (&col_ld)[NT],
                                                    float (&acc)[NT][VEC]) {
   // (the row's nonzeros are start .. end - 1, wave-uniform: for a caller that has read the row's offsets already)
@@ -177,6 +180,21 @@ __device__ __forceinline__ void spmm_range_partial(const SpmmParams& p, int z, i
 #pragma unroll
           for (int u = 0; u < kWin; ++u) fma_row(vv[u], bv[u]);
         }
+        if constexpr (TAIL) {
+          auto window = [&](auto size) {
+            constexpr int N = decltype(size)::value;
+            if (kWin <= N || s + N > steps) return;
+            Slab bv[N];
+            float vv[N];
+#pragma unroll
+            for (int u = 0; u < N; ++u) bv[u] = load_row(fetch(s + u, vv[u]));
+#pragma unroll
+            for (int u = 0; u < N; ++u) fma_row(vv[u], bv[u]);
+            s += N;
+          };
+          window(std::integral_constant<int, 4>{});
+          window(std::integral_constant<int, 2>{});
+        }
         for (; s * G < cnt; ++s) {
           float vu;
           const int cu = fetch(s, vu);
@@ -198,10 +216,10 @@ __device__ __forceinline__ void spmm_range_partial(const SpmmParams& p, int z, i
   }
 }
 
-template <typename T, typename IT, int VEC, int LPG, int WIN, int NT, bool RAGGED>
+template <typename T, typename IT, int VEC, int LPG, int WIN, int NT, bool RAGGED, bool TAIL>
 __device__ __forceinline__ void spmm_row_partial(const SpmmParams& p, int z, int row, int part, int wpr, const int (&col_ld)[NT],
                                                  float (&acc)[NT][VEC]) {
-  spmm_range_partial<T, IT, VEC, LPG, WIN, NT, RAGGED>(p, z, uniform(p.row_offsets[row]), uniform(p.row_offsets[row + 1]), part, wpr, col_ld, acc);
+  spmm_range_partial<T, IT, VEC, LPG, WIN, NT, RAGGED, TAIL>(p, z, uniform(p.row_offsets[row]), uniform(p.row_offsets[row + 1]), part, wpr, col_ld, acc);
 }
 
 // Bias, ReLU, accumulation and the store of one row's sums (lanes of group 0 only; col0 = first column of tile 0).
@@ -248,7 +266,7 @@ __device__ __forceinline__ void spmm_store_row(const SpmmParams& p, int z, int r
 // RAGGED = n is not a multiple of VEC: vectors are moved at element alignment, and the one lane of a
 //       row whose vector would reach past the row's end reads VEC elements ending at the row's end
 //       instead (shifted back by `shift`), sums all of them and stores only the ones it owns.
-template <typename T, typename IT, int VEC, int LPG, int WPR, int WIN = kSpmmUnroll, int NT = 1, bool RAGGED = false>
+template <typename T, typename IT, int VEC, int LPG, int WPR, int WIN = kSpmmUnroll, int NT = 1, bool RAGGED = false, bool TAIL = true>
 __device__ __forceinline__ void spmm_block(const SpmmParams& p, int bx, int by, int bz, float* red) {
   static_assert(!RAGGED || (NT == 1 && LPG == kWave), "ragged rows: one full-width tile per wave");
   constexpr int kWavesPerBlock = (WPR > 4) ? WPR : 4;
@@ -279,7 +297,7 @@ __device__ __forceinline__ void spmm_block(const SpmmParams& p, int bx, int by, 
   int row = 0;
   if (row_live) {
     row = uniform(p.row_indices[row_slot]);
-    spmm_row_partial<T, IT, VEC, LPG, WIN, NT, RAGGED>(p, z, row, part, WPR, col_ld, acc);
+    spmm_row_partial<T, IT, VEC, LPG, WIN, NT, RAGGED, TAIL>(p, z, row, part, WPR, col_ld, acc);
   }
 
   if constexpr (WPR > 1) {
