@@ -48,10 +48,12 @@ class SparseDecoderLayer:
         self.w = {}
         for name, csr in weights.items():
             idt = index_dtype if csr.k <= 32768 else torch.int32
-            self.w[name] = (torch.from_numpy(csr.row_indices).to(device),
-                            torch.from_numpy(csr.values).to(device).half(),
-                            torch.from_numpy(csr.row_offsets).to(device),
-                            torch.from_numpy(csr.column_indices).to(device).to(idt), csr.m)
+            # (tensors that count their changes, also where the layer is built under inference_mode())
+            with torch.inference_mode(False):
+                self.w[name] = (torch.from_numpy(csr.row_indices).to(device),
+                                torch.from_numpy(csr.values).to(device).half(),
+                                torch.from_numpy(csr.row_offsets).to(device),
+                                torch.from_numpy(csr.column_indices).to(device).to(idt), csr.m)
             # (looked at once, here: the layer's schedules run under capture, where a pattern nobody has looked at
             # keeps to the kernels that take columns in any order)
             _pyops.prepare_pattern(self.w[name][2], self.w[name][3], csr.k, tables=False)
@@ -67,7 +69,7 @@ class SparseDecoderLayer:
         """The product by what was laid out, of the weight as it is now; None where the operators have to serve it."""
         form, (_, v, ro, ci, _) = self._forms[name], self.w[name]
         if not form.is_of(v, ro, ci):
-            if torch.cuda.is_current_stream_capturing():
+            if torch.cuda.is_current_stream_capturing() or any(t.is_inference() for t in (v, ro, ci)):
                 return None
             form = self._forms[name] = self._lay_out(name)
         return form.product(x, other, mode)

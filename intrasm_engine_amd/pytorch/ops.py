@@ -79,8 +79,8 @@ def kernels_forced() -> bool:
 
 
 def _version(t) -> int:
-    """In-place-change counter of a tensor; tensors created under ``torch.inference_mode()`` keep none (reading it
-    raises) and cannot be changed in place either, so 0 serves."""
+    """In-place-change counter of a tensor.  Tensors created under ``torch.inference_mode()`` keep none (reading it raises):
+    0 for them, although they can be changed in place inside that mode.  Such a change shows nowhere."""
     if t.is_inference():
         return 0
     return t._version
@@ -409,8 +409,10 @@ class WeightForm:
         self._form = _iex_host.WeightForm(values, row_offsets, column_indices, m, k, forms, measured)
 
     def is_of(self, values, row_offsets, column_indices) -> bool:
-        """Whether these are the tensors that were laid out, unchanged since."""
-        return all(a is b and _version(b) == v for a, b, v in zip(self._tensors, (values, row_offsets, column_indices), self._versions))
+        """Whether these are the tensors that were laid out, unchanged since.  Never of tensors that count no changes (made under
+        ``torch.inference_mode()``)."""
+        return all(a is b and not b.is_inference() and _version(b) == v
+                   for a, b, v in zip(self._tensors, (values, row_offsets, column_indices), self._versions))
 
     def product(self, x, other=None, mode=0):
         """``weight @ x``, plus ``other`` (mode 1) or times its SiLU (mode 2) before it is rounded; None where an operator on the CSR tensors has to

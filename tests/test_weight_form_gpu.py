@@ -156,6 +156,38 @@ def test_layer_by_forms_follows_its_weights(dev):
         assert torch.equal(out, layer.forward(x, 2))
 
 
+def _by_operators(layer, x):
+    with pyops.kernel_params(gemm={"tile": 13}):
+        return layer.forward(x, 2)
+
+
+def _follows(layer, x):
+    """The layer's result is that of the operators on the weights as they are now, and another than before."""
+    got, want = layer.forward(x, 2).float(), _by_operators(layer, x).float()
+    return bool((got - want).norm() < 2e-3 * want.norm())
+
+
+def test_layer_under_inference_mode_follows_its_weights(dev):
+    """Built, changed in place and given replaced weights under inference mode, where tensors count no changes: a relative error of 3e-2
+    where a weight is stale, of 1e-4 (fp16 results rounded after sums in another order) where not."""
+    with torch.inference_mode():
+        layer = _layer(dev)
+        x = torch.randn(256, 1024, device=dev).half()
+        assert _follows(layer, x) and layer._by_form("q", x) is not None
+        layer.w["q"][1].mul_(3.0)
+        layer.w["down"][1].mul_(0.1)
+        assert _follows(layer, x)
+        ri, v, ro, ci, m = layer.w["down"]
+        layer.w["down"] = (ri, v * 10.0, ro, ci, m)
+        assert layer.w["down"][1].is_inference() and _follows(layer, x)
+        layer.w["down"][1].mul_(0.1)
+        assert _follows(layer, x) and layer._by_form("down", torch.randn(512, 1024, device=dev).half()) is None
+        form = pyops.WeightForm(layer.w["down"][1], ro, ci, m, 512)
+        assert not form.is_of(layer.w["down"][1], ro, ci)
+    layer.w["q"][1].mul_(0.5)
+    assert _follows(layer, x)
+
+
 def test_forms_are_refused_on_the_host(dev):
     lib = _lib.load()
     one = torch.zeros(1024, dtype=torch.int32, device=dev)
