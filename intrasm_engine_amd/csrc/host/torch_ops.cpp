@@ -134,6 +134,11 @@ void set_note(const Tensor& row_offsets, const Tensor& column_indices, int64_t k
   map.insert_or_assign(column_indices.unsafeGetTensorImpl(), std::move(n));
 }
 
+void forget_note(const Tensor& column_indices) {
+  std::unique_lock lock(notes_mutex);
+  notes().erase(column_indices.unsafeGetTensorImpl());
+}
+
 // for calls of q's type on the mask; lifts what an earlier capture has settled for calls like q
 void set_mask_tables(const Tensor& q, const Tensor& row_offsets, const Tensor& column_indices, const Tensor& tables, int64_t stream) {
   std::unique_lock lock(notes_mutex);
@@ -603,6 +608,7 @@ PYBIND11_MODULE(_iex_host, module) {
   module.def("bind", [](py::object functions) { python_ops = new py::object(std::move(functions)); });
   module.def("set_forced", [](bool on) { forced = on; });
   module.def("set_note", &set_note);
+  module.def("forget_note", &forget_note);
   module.def("spmm_with", &spmm_with);
   module.def("attention", &attention);
   py::class_<WeightForm>(module, "WeightForm")

@@ -36,9 +36,15 @@ ops = torch.ops.iex_ops
 
 
 class SparseDecoderLayer:
-    def __init__(self, weights: dict, hidden: int, heads: int, mlp: int, device, index_dtype=torch.int16):
+    def __init__(self, weights: dict, hidden: int, heads: int, mlp: int, device, index_dtype=torch.int16, keep_forms: bool = True):
         """``weights``: name -> workloads.CSR for q, k, v, o (hidden x hidden), gate, up
-        (mlp x hidden), down (hidden x mlp); values are cast to fp16."""
+        (mlp x hidden), down (hidden x mlp); values are cast to fp16.
+
+        ``w`` holds them on the device: name -> (row_indices, values, row_offsets, column_indices, m).  Eager passes follow
+        entries that are replaced and tensors changed by ordinary operations; for writes that no version counter shows
+        (``.data``, a replayed graph, a kernel that was given the address) call :meth:`lay_out_weights` afterwards.
+        ``keep_forms=False`` keeps no copy of the values (2 to 4 bytes a cell of every weight): every pass then reads the CSR
+        arrays through the operators."""
         self.hidden, self.heads, self.mlp = hidden, heads, mlp
         self.head_dim = hidden // heads
         self.device = device
@@ -54,19 +60,37 @@ class SparseDecoderLayer:
                                 torch.from_numpy(csr.values).to(device).half(),
                                 torch.from_numpy(csr.row_offsets).to(device),
                                 torch.from_numpy(csr.column_indices).to(device).to(idt), csr.m)
-            # (looked at once, here: the layer's schedules run under capture, where a pattern nobody has looked at
-            # keeps to the kernels that take columns in any order)
-            _pyops.prepare_pattern(self.w[name][2], self.w[name][3], csr.k, tables=False)
         # the weights as the schedules multiply them, laid out once (a capture lays them out inside the graph)
-        self._forms = {name: self._lay_out(name) for name in self.w}
+        self._keep_forms = keep_forms
+        self._forms = {}
+        self.lay_out_weights()
+
+    def _inner(self, name: str) -> int:
+        return self.mlp if name == "down" else self.hidden
 
     def _lay_out(self, name: str) -> "_pyops.WeightForm":
         _, v, ro, ci, m = self.w[name]
-        return _pyops.WeightForm(v, ro, ci, m, self.mlp if name == "down" else self.hidden)
+        return _pyops.WeightForm(v, ro, ci, m, self._inner(name))
+
+    def lay_out_weights(self, names=None) -> None:
+        """Take the weights (``names``; all of them) as they are now, patterns included: what was known of them goes.  Not under
+        stream capture."""
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("lay_out_weights: the current stream is being captured")
+        for name in self.w if names is None else names:
+            _, _, ro, ci, _ = self.w[name]
+            # (looked at here: the layer's schedules run under capture, where a pattern nobody has looked at
+            # keeps to the kernels that take columns in any order)
+            _pyops.forget_pattern(ci)
+            _pyops.prepare_pattern(ro, ci, self._inner(name), tables=False)
+            if self._keep_forms:
+                self._forms[name] = self._lay_out(name)
 
     # ---- building blocks ---------------------------------------------------------------
     def _by_form(self, name: str, x: torch.Tensor, other=None, mode: int = 0):
         """The product by what was laid out, of the weight as it is now; None where the operators have to serve it."""
+        if not self._keep_forms:
+            return None
         form, (_, v, ro, ci, _) = self._forms[name], self.w[name]
         if not form.is_of(v, ro, ci):
             if torch.cuda.is_current_stream_capturing() or any(t.is_inference() for t in (v, ro, ci)):

@@ -80,7 +80,7 @@ def kernels_forced() -> bool:
 
 def _version(t) -> int:
     """In-place-change counter of a tensor.  Tensors created under ``torch.inference_mode()`` keep none (reading it raises):
-    0 for them, although they can be changed in place inside that mode.  Such a change shows nowhere."""
+    0 for them, although they can be changed in place inside that mode.  Such a change shows nowhere: see :func:`forget_pattern`."""
     if t.is_inference():
         return 0
     return t._version
@@ -211,6 +211,15 @@ def _set_note(row_offsets, column_indices, k, status, hist, share=None, tables=N
     column_indices.__dict__["_iex_csr"] = (weakref.ref(row_offsets), _version(row_offsets), _version(column_indices), int(k), status, hist, share,
                                            tables)
     _iex_host.set_note(row_offsets, column_indices, int(k), status, hist, share, tables, tables._iex_stream if tables is not None else -1)
+
+
+def forget_pattern(column_indices) -> None:
+    """Drop what is known about a pattern, its tables included (graphs that read them keep theirs): the next call on it looks
+    again.  For index tensors written where no version counter shows it: made under ``torch.inference_mode()`` and changed
+    there, through ``.data``, by a replayed graph, by a kernel that was given the address."""
+    for name in ("_iex_csr", "_iex_mask_tables"):
+        column_indices.__dict__.pop(name, None)
+    _iex_host.forget_note(column_indices)
 
 
 def mark_canonical(row_offsets, column_indices, k, measure=True):
@@ -372,7 +381,8 @@ class WeightForm:
     its dense form and, where a row holds at most two of (nearly) every four neighbouring columns, the two-of-four form that the
     structured-sparsity matrix instructions take.  Costs a synchronisation and about 2-4 bytes a cell of the weight.
 
-    What was laid out stands for the CSR tensors as they were: :meth:`is_of` tells whether they are still those."""
+    What was laid out stands for the CSR tensors as they were: :meth:`is_of` tells whether they are still those, by identity and version
+    counters.  A program that writes them otherwise (``.data``, a replayed graph, a raw address) makes a new one."""
 
     KINDS = (0, 128, 192, 256)
 

@@ -118,13 +118,13 @@ def test_values_that_mark_an_empty_place_and_infinities(dev):
         assert torch.allclose(out[~with_nan][:, others].double(), want, rtol=1e-2, atol=1e-1)
 
 
-def _layer(dev, hidden=256, mlp=512, seed=0):
+def _layer(dev, hidden=256, mlp=512, seed=0, **options):
     rng = np.random.default_rng(seed)
     weights = {}
     for name, (m, k) in {**{x: (hidden, hidden) for x in "qkvo"}, "gate": (mlp, hidden), "up": (mlp, hidden), "down": (hidden, mlp)}.items():
         csr = _csr(rng, m, k, "2:4" if len(name) == 1 else 0.2)
         weights[name] = W.CSR(m, k, csr.values * 0.05, csr.row_indices, csr.row_offsets, csr.column_indices)
-    return SparseDecoderLayer(weights, hidden, hidden // 64, mlp, dev)
+    return SparseDecoderLayer(weights, hidden, hidden // 64, mlp, dev, **options)
 
 
 def test_layer_by_forms_follows_its_weights(dev):
@@ -186,6 +186,43 @@ def test_layer_under_inference_mode_follows_its_weights(dev):
         assert not form.is_of(layer.w["down"][1], ro, ci)
     layer.w["q"][1].mul_(0.5)
     assert _follows(layer, x)
+
+
+def test_writes_that_no_counter_shows(dev):
+    """Through .data and by a replayed graph, values and patterns: followed after lay_out_weights, and without it by a layer that keeps
+    no forms."""
+    layer, plain = _layer(dev), _layer(dev, keep_forms=False)
+    x = torch.randn(256, 1024, device=dev).half()
+    assert _follows(plain, x) and plain._by_form("q", x) is None
+    for it in (layer, plain):
+        it.w["down"][1].data.mul_(0.1)
+    assert _follows(plain, x)
+    layer.lay_out_weights(["down"])
+    assert _follows(layer, x) and layer._by_form("q", x) is not None
+    assert torch.allclose(plain.forward(x, 2).float(), layer.forward(x, 2).float(), rtol=2e-2, atol=2e-2)
+    for it in (layer, plain):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            it.w["gate"][1].mul_(3.0)
+        seen = it.w["gate"][1]._version        # (the counter shows the recording, not the replay)
+        it.forward(x, 2)
+        graph.replay()
+        assert it.w["gate"][1]._version == seen
+    assert _follows(plain, x)
+    layer.lay_out_weights()
+    assert _follows(layer, x)
+    # a pattern: the columns of every row in reverse, with them the values (same matrix, no canonical CSR)
+    ri, v, ro, ci, m = layer.w["up"]
+    order = torch.cat([torch.arange(e - 1, s - 1, -1) for s, e in zip(ro.tolist()[:-1], ro.tolist()[1:])]).to(dev)
+    before = layer.forward(x, 2)
+    ci.data.copy_(ci[order].clone())
+    v.data.copy_(v[order].clone())
+    layer.lay_out_weights(["up"])
+    assert layer._by_form("up", x) is None and _follows(layer, x)
+    assert torch.allclose(layer.forward(x, 2).float(), before.float(), rtol=2e-2, atol=2e-2)
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        with pytest.raises(RuntimeError):
+            layer.lay_out_weights()
 
 
 def test_forms_are_refused_on_the_host(dev):
