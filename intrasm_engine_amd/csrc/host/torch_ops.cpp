@@ -160,15 +160,17 @@ std::optional<Known> note_of(const Tensor& row_offsets, const Tensor& column_ind
   return known;
 }
 
-// Tables that outlive a call are memory of the stream they were made on.  Work on another one is told to their allocator;
-// a call that is captured has them kept as long as the pattern's tensor, also where later calls replace them.
+// Memory that outlives a call is memory of the stream it was made on.  Work on another one is told to its allocator.
+void use_memory(const Tensor& memory, int64_t made_on) {
+  const auto stream = c10::hip::getCurrentHIPStream(memory.get_device());
+  if (stream.id() != made_on) memory.record_stream(c10::Stream(c10::Stream::UNSAFE, memory.device(), stream.id()));   // (a tensor's device is "cuda", the stream's "hip")
+}
+
+// The same for tables kept with a pattern; a call that is captured has them kept as long as the pattern's tensor, also where later calls
+// replace them.
 void use_tables(const Tensor& tables, int64_t tables_stream, const Tensor& column_indices, bool captured) {
-  if (captured) {
-    tell_python("keep_recorded", column_indices, tables);
-    return;
-  }
-  const auto stream = c10::hip::getCurrentHIPStream(tables.get_device());
-  if (stream.id() != tables_stream) tables.record_stream(c10::Stream(c10::Stream::UNSAFE, tables.device(), stream.id()));   // (a tensor's device is "cuda", the stream's "hip")
+  if (captured) tell_python("keep_recorded", column_indices, tables);
+  else use_memory(tables, tables_stream);
 }
 
 // ---- operands that fit -------------------------------------------------------------------------------------------
@@ -386,11 +388,12 @@ struct WeightForm {
   std::array<Tensor, 4> forms;   // kinds 0, 128, 192, 256
   std::array<int, 3> phases, rooms;
   int kinds = 0;
+  int64_t made_on;   // the stream whose memory they are
   Tensor values, row_offsets, column_indices;
 
   WeightForm(const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m, int64_t k,
-             const std::vector<std::optional<Tensor>>& given, const std::vector<int>& measured)
-      : dtype(dtype_code(values.scalar_type())), m(m), k(k), nonzeros(column_indices.numel()), values(values), row_offsets(row_offsets), column_indices(column_indices) {
+             const std::vector<std::optional<Tensor>>& given, const std::vector<int>& measured, int64_t made_on)
+      : dtype(dtype_code(values.scalar_type())), m(m), k(k), nonzeros(column_indices.numel()), made_on(made_on), values(values), row_offsets(row_offsets), column_indices(column_indices) {
     TORCH_CHECK(given.size() == 4 && measured.size() == 6, "WeightForm: four forms and six numbers");
     for (int i = 0; i < 4; ++i)
       if (given[i]) forms[i] = *given[i], kinds |= 1 << i;
@@ -418,6 +421,8 @@ struct WeightForm {
                            column_indices.const_data_ptr(), values.const_data_ptr(), room, form.data_ptr(), form.numel(),
                            scratch.defined() ? scratch.data_ptr() : nullptr, scratch.defined() ? scratch.numel() : 0, stream_of(x)),
             "form");
+    } else {
+      use_memory(form, made_on);
     }
     const size_t ws_bytes = iex_form_product_workspace_bytes(kind, m, k, n);
     const Tensor ws = workspace(ws_bytes, x);
@@ -612,7 +617,7 @@ PYBIND11_MODULE(_iex_host, module) {
   module.def("spmm_with", &spmm_with);
   module.def("attention", &attention);
   py::class_<WeightForm>(module, "WeightForm")
-      .def(py::init<const Tensor&, const Tensor&, const Tensor&, int64_t, int64_t, const std::vector<std::optional<Tensor>>&, const std::vector<int>&>())
+      .def(py::init<const Tensor&, const Tensor&, const Tensor&, int64_t, int64_t, const std::vector<std::optional<Tensor>>&, const std::vector<int>&, int64_t>())
       .def_readonly("kinds", &WeightForm::kinds)
       .def("product", &WeightForm::product, py::arg("x"), py::arg("other") = std::nullopt, py::arg("mode") = 0);
   module.def("sparse_attention", &sparse_attention);

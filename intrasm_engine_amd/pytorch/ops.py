@@ -416,7 +416,7 @@ class WeightForm:
                 _lib.check(lib.iex_form_build(itype, kind, m, k, nonzeros, row_offsets.data_ptr(), column_indices.data_ptr(), values.data_ptr(), room,
                                               forms[i].data_ptr(), forms[i].numel(), scratch.data_ptr(), scratch.numel(), stream), "form")
             torch.cuda.current_stream(device).synchronize()      # (products on any stream find it complete)
-        self._form = _iex_host.WeightForm(values, row_offsets, column_indices, m, k, forms, measured)
+        self._form = _iex_host.WeightForm(values, row_offsets, column_indices, m, k, forms, measured, torch.cuda.current_stream(device).stream_id)
 
     def is_of(self, values, row_offsets, column_indices) -> bool:
         """Whether these are the tensors that were laid out, unchanged since.  Never of tensors that count no changes (made under

@@ -225,6 +225,26 @@ def test_writes_that_no_counter_shows(dev):
             layer.lay_out_weights()
 
 
+def test_a_replaced_weight_on_another_stream(dev):
+    """A weight is replaced while a pass on another stream has not run yet: the memory of what was laid out is not handed out before."""
+    layer = _layer(dev)
+    x = torch.randn(256, 1024, device=dev).half()
+    want = layer.proj("q", x)
+    assert layer._by_form("q", x) is not None
+    sizes = [_lib.load().iex_form_bytes(kind, 256, 256, room) for kind in pyops.WeightForm.KINDS for room in range(3)]
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(200_000_000)
+        out = layer.proj("q", x)
+    ri, v, ro, ci, m = layer.w["q"]
+    layer.w["q"] = (ri, v * 3.0, ro, ci, m)
+    layer.proj("q", x)
+    keep = [torch.zeros(n, dtype=torch.uint8, device=dev) for n in sizes for _ in range(4)]
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and len(keep) == 48
+
+
 def test_forms_are_refused_on_the_host(dev):
     lib = _lib.load()
     one = torch.zeros(1024, dtype=torch.int32, device=dev)
