@@ -11,6 +11,7 @@
 // address, with weak references to both index tensors and their version counters, so that a note never outlives its
 // tensors or passes for another pattern's, and keeps no memory of theirs alive.
 #include <ATen/ATen.h>
+#include <ATen/hip/HIPEvent.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
@@ -377,52 +378,78 @@ std::optional<Tensor> spmm_with(const Tensor& x, const Tensor& row_indices, cons
   return out.defined() ? std::optional<Tensor>(out) : std::nullopt;
 }
 
-// softmax(scale * q^T k) v per head and sequence on feature-major operands; None where the kernel does not serve them
-// A sparse weight laid out once (ops.WeightForm makes it): the product with x, combined with `other` as in spmm_with.  Nothing is returned where the
-// call is not served here -- operands that do not fit, a gradient wanted, kernels forced, an operator on the CSR arrays that is faster.  A captured
-// call lays the weight out inside the graph: replays follow the CSR arrays, and give the same bits as a call.
+// A sparse weight for a program that keeps it (ops.WeightForm makes it): the product with x, combined with `other` as in spmm_with.  Nothing is
+// returned where the call is not served here -- operands that do not fit, a gradient wanted, kernels forced, an operator on the CSR arrays that is
+// faster.  The first product that takes a kind of form lays it out, on its stream and without waiting; later ones find it, on other streams behind
+// an event.  A captured call lays the weight out inside the graph: replays follow the CSR arrays, and give the same bits as a call.
 struct WeightForm {
   static constexpr int kAnyRoom = 1 << 20;
+  struct Layout {
+    Tensor memory;
+    at::cuda::CUDAEvent ready;
+    int64_t made_on = -1;   // the stream whose memory it is
+  };
   int dtype;
   int64_t m, k, nonzeros;
-  std::array<Tensor, 4> forms;   // kinds 0, 128, 192, 256
+  std::array<Layout, 4> layouts;   // kinds 0, 128, 192, 256
+  std::mutex layouts_mutex;
   std::array<int, 3> phases, rooms;
-  int kinds = 0;
-  int64_t made_on;   // the stream whose memory they are
+  int kinds;                       // a bit for each that the weight can be laid out as
   Tensor values, row_offsets, column_indices;
 
-  WeightForm(const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m, int64_t k,
-             const std::vector<std::optional<Tensor>>& given, const std::vector<int>& measured, int64_t made_on)
-      : dtype(dtype_code(values.scalar_type())), m(m), k(k), nonzeros(column_indices.numel()), made_on(made_on), values(values), row_offsets(row_offsets), column_indices(column_indices) {
-    TORCH_CHECK(given.size() == 4 && measured.size() == 6, "WeightForm: four forms and six numbers");
-    for (int i = 0; i < 4; ++i)
-      if (given[i]) forms[i] = *given[i], kinds |= 1 << i;
+  WeightForm(const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m, int64_t k, int kinds, const std::vector<int>& measured)
+      : dtype(dtype_code(values.scalar_type())), m(m), k(k), nonzeros(column_indices.numel()), kinds(kinds), values(values), row_offsets(row_offsets), column_indices(column_indices) {
+    TORCH_CHECK(measured.size() == 6, "WeightForm: six numbers");
     std::copy_n(measured.begin(), 3, phases.begin());
     std::copy_n(measured.begin() + 3, 3, rooms.begin());
   }
 
-  std::optional<Tensor> product(const Tensor& x, const std::optional<Tensor>& other, int mode) const {
+  int laid_out() {   // a bit for each kind that is
+    std::lock_guard lock(layouts_mutex);
+    int bits = 0;
+    for (int i = 0; i < 4; ++i) bits |= layouts[i].memory.defined() << i;
+    return bits;
+  }
+
+  Tensor lay_out(int kind, int room, const Tensor& like) const {
+    Tensor form = workspace(iex_form_bytes(kind, m, k, room), like);
+    const Tensor scratch = workspace(kind ? iex_form_scratch_bytes(m, k) : 0, like);
+    check(iex_form_build(column_indices.scalar_type() == at::kShort ? IEX_I16 : IEX_I32, kind, m, k, nonzeros, row_offsets.const_data_ptr<int>(),
+                         column_indices.const_data_ptr(), values.const_data_ptr(), room, form.data_ptr(), form.numel(),
+                         scratch.defined() ? scratch.data_ptr() : nullptr, scratch.defined() ? scratch.numel() : 0, stream_of(like)),
+          "form");
+    return form;
+  }
+
+  std::optional<Tensor> product(const Tensor& x, const std::optional<Tensor>& other, int mode) {
     const int64_t n = x.dim() == 2 ? x.size(1) : 0;
     if (forced || !plain(x, 2) || x.size(0) != k || n == 0 || n % 8 || k * n >= (1ll << 31) || m * n >= (1ll << 31) || dtype_code(x.scalar_type()) != dtype ||
-        reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 || (at::GradMode::is_enabled() && (x.requires_grad() || (other && other->requires_grad()))))
+        x.device() != values.device() || reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 ||
+        (at::GradMode::is_enabled() && (x.requires_grad() || (other && other->requires_grad()))))
       return {};
     if (other && (!plain(*other, 2) || other->size(0) != m || other->size(1) != n || other->scalar_type() != x.scalar_type() || other->device() != x.device())) return {};
     const c10::DeviceGuard guard(x.device());
     const int kind = iex_form_choose(kinds, m, k, n, nonzeros, phases.data());
     if (kind < 0) return {};
-    Tensor form = forms[kind ? kind / 64 - 1 : 0];
-    if (form.device() != x.device()) return {};
     int room = kind ? rooms[kind / 64 - 2] : 0;
+    Tensor form;
     if (capturing()) {
       room = kind ? kAnyRoom : 0;   // (the pattern of a later replay may spill more)
-      form = workspace(iex_form_bytes(kind, m, k, room), x);
-      const Tensor scratch = workspace(kind ? iex_form_scratch_bytes(m, k) : 0, x);
-      check(iex_form_build(column_indices.scalar_type() == at::kShort ? IEX_I16 : IEX_I32, kind, m, k, nonzeros, row_offsets.const_data_ptr<int>(),
-                           column_indices.const_data_ptr(), values.const_data_ptr(), room, form.data_ptr(), form.numel(),
-                           scratch.defined() ? scratch.data_ptr() : nullptr, scratch.defined() ? scratch.numel() : 0, stream_of(x)),
-            "form");
+      form = lay_out(kind, room, x);
     } else {
-      use_memory(form, made_on);
+      std::lock_guard lock(layouts_mutex);
+      Layout& layout = layouts[kind ? kind / 64 - 1 : 0];
+      const auto stream = at::cuda::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device());
+      if (!layout.memory.defined()) {
+        const Tensor made = lay_out(kind, room, x);
+        layout.ready.record(stream);
+        layout.made_on = c10::hip::getCurrentHIPStream(x.get_device()).id();
+        layout.memory = made;
+      } else if (c10::hip::getCurrentHIPStream(x.get_device()).id() != layout.made_on) {
+        layout.ready.block(stream);
+        use_memory(layout.memory, layout.made_on);
+      }
+      form = layout.memory;
     }
     const size_t ws_bytes = iex_form_product_workspace_bytes(kind, m, k, n);
     const Tensor ws = workspace(ws_bytes, x);
@@ -434,6 +461,7 @@ struct WeightForm {
   }
 };
 
+// softmax(scale * q^T k) v per head and sequence on feature-major operands; None where the kernel does not serve them
 std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, int64_t seqs, double scale) {
   const int dtype = dtype_code(q.scalar_type());
   if (forced || !plain(q, 2) || !plain(k, 2) || !plain(v, 2) || k.sizes() != q.sizes() || v.sizes() != q.sizes() || k.scalar_type() != q.scalar_type() ||
@@ -617,9 +645,11 @@ PYBIND11_MODULE(_iex_host, module) {
   module.def("spmm_with", &spmm_with);
   module.def("attention", &attention);
   py::class_<WeightForm>(module, "WeightForm")
-      .def(py::init<const Tensor&, const Tensor&, const Tensor&, int64_t, int64_t, const std::vector<std::optional<Tensor>>&, const std::vector<int>&, int64_t>())
+      .def(py::init<const Tensor&, const Tensor&, const Tensor&, int64_t, int64_t, int, const std::vector<int>&>())
       .def_readonly("kinds", &WeightForm::kinds)
-      .def("product", &WeightForm::product, py::arg("x"), py::arg("other") = std::nullopt, py::arg("mode") = 0);
+      // (nobody waits for layouts_mutex with the interpreter's lock in hand)
+      .def_property_readonly("laid_out", &WeightForm::laid_out, py::call_guard<py::gil_scoped_release>())
+      .def("product", &WeightForm::product, py::arg("x"), py::arg("other") = std::nullopt, py::arg("mode") = 0, py::call_guard<py::gil_scoped_release>());
   module.def("sparse_attention", &sparse_attention);
   module.def("set_mask_tables", &set_mask_tables);
   module.def("trainable_spmm", &trainable_spmm);

@@ -43,8 +43,8 @@ class SparseDecoderLayer:
         ``w`` holds them on the device: name -> (row_indices, values, row_offsets, column_indices, m).  Eager passes follow
         entries that are replaced and tensors changed by ordinary operations; for writes that no version counter shows
         (``.data``, a replayed graph, a kernel that was given the address) call :meth:`lay_out_weights` afterwards.
-        ``keep_forms=False`` keeps no copy of the values (2 to 4 bytes a cell of every weight): every pass then reads the CSR
-        arrays through the operators."""
+        ``keep_forms=False`` keeps no copy of the values (1 to 2 bytes a cell of every weight for each kind of layout that the
+        widths at hand take, four at most): every pass then reads the CSR arrays through the operators."""
         self.hidden, self.heads, self.mlp = hidden, heads, mlp
         self.head_dim = hidden // heads
         self.device = device
@@ -60,7 +60,7 @@ class SparseDecoderLayer:
                                 torch.from_numpy(csr.values).to(device).half(),
                                 torch.from_numpy(csr.row_offsets).to(device),
                                 torch.from_numpy(csr.column_indices).to(device).to(idt), csr.m)
-        # the weights as the schedules multiply them, laid out once (a capture lays them out inside the graph)
+        # the weights as the schedules multiply them, laid out by the first pass that takes them (a capture lays them out inside the graph)
         self._keep_forms = keep_forms
         self._forms = {}
         self.lay_out_weights()
@@ -73,8 +73,8 @@ class SparseDecoderLayer:
         return _pyops.WeightForm(v, ro, ci, m, self._inner(name))
 
     def lay_out_weights(self, names=None) -> None:
-        """Take the weights (``names``; all of them) as they are now, patterns included: what was known of them goes.  Not under
-        stream capture."""
+        """Take the weights (``names``; all of them) as they are now, patterns included: what was known of them goes, the next
+        pass lays them out.  Not under stream capture."""
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("lay_out_weights: the current stream is being captured")
         for name in self.w if names is None else names:

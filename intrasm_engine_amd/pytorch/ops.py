@@ -217,7 +217,7 @@ def forget_pattern(column_indices) -> None:
     """Drop what is known about a pattern, its tables included (graphs that read them keep theirs): the next call on it looks
     again.  For index tensors written where no version counter shows it: made under ``torch.inference_mode()`` and changed
     there, through ``.data``, by a replayed graph, by a kernel that was given the address."""
-    for name in ("_iex_csr", "_iex_mask_tables"):
+    for name in ("_iex_csr", "_iex_mask_tables", "_iex_form_counts"):
         column_indices.__dict__.pop(name, None)
     _iex_host.forget_note(column_indices)
 
@@ -376,10 +376,32 @@ def prepare_pattern(row_offsets, column_indices, k, tables=True):
     return status
 
 
+def _form_counts(row_offsets, column_indices, m, k):
+    """What ``iex_form_measure`` counts of a pattern: one read, kept with ``column_indices``.  None where a weight of this pattern has a dense
+    form only."""
+    lib = _lib.load()
+    if not lib.iex_form_scratch_bytes(m, k):
+        return None
+    key = (_version(row_offsets), _version(column_indices), m, k)
+    kept = column_indices.__dict__.get("_iex_form_counts")
+    if kept is not None and kept[0]() is row_offsets and kept[1] == key:
+        return kept[2]
+    device = row_offsets.device
+    with torch.cuda.device(device):
+        scratch = torch.empty(lib.iex_form_scratch_bytes(m, k), dtype=torch.uint8, device=device)
+        counts = torch.zeros(6, dtype=torch.int32, device=device)
+        _lib.check(lib.iex_form_measure(_IT[column_indices.dtype], m, k, column_indices.numel(), row_offsets.data_ptr(), column_indices.data_ptr(),
+                                        scratch.data_ptr(), scratch.numel(), counts.data_ptr(), _stream_ptr(device)), "form")
+        measured = counts.tolist()
+    column_indices.__dict__["_iex_form_counts"] = (weakref.ref(row_offsets), key, measured)
+    return measured
+
+
 class WeightForm:
     """A 16-bit sparse weight laid out once for products with many dense columns (``iex_form_build``), for a program that keeps the weight:
-    its dense form and, where a row holds at most two of (nearly) every four neighbouring columns, the two-of-four form that the
-    structured-sparsity matrix instructions take.  Costs a synchronisation and about 2-4 bytes a cell of the weight.
+    its dense form or, where a row holds at most two of (nearly) every four neighbouring columns, the two-of-four form that the
+    structured-sparsity matrix instructions take, by tiles of 128, 192 or 256 rows.  The first product that takes a kind lays it out; each takes
+    about 2 bytes a cell of the weight (dense) or 1.1 and its spilled columns.  A pattern that was not measured before costs one synchronising read.
 
     What was laid out stands for the CSR tensors as they were: :meth:`is_of` tells whether they are still those, by identity and version
     counters.  A program that writes them otherwise (``.data``, a replayed graph, a raw address) makes a new one."""
@@ -390,33 +412,11 @@ class WeightForm:
         self._tensors = (values, row_offsets, column_indices)
         self._versions = tuple(_version(t) for t in self._tensors)
         self._form = None
-        nonzeros, device, lib = column_indices.numel(), values.device, _lib.load()
-        if values.dtype not in (torch.float16, torch.bfloat16) or not 3 <= nonzeros < 1 << 29 or torch.cuda.is_current_stream_capturing() or \
-                _csr_status(row_offsets, column_indices, k) != 0 or lib.iex_form_bytes(0, m, k, 0) == 0:
+        if values.dtype not in (torch.float16, torch.bfloat16) or not 3 <= column_indices.numel() < 1 << 29 or torch.cuda.is_current_stream_capturing() or \
+                _csr_status(row_offsets, column_indices, k) != 0 or _lib.load().iex_form_bytes(0, m, k, 0) == 0:
             return
-        itype = _IT[column_indices.dtype]
-        with torch.cuda.device(device):
-            stream = _stream_ptr(device)
-            scratch = torch.empty(lib.iex_form_scratch_bytes(m, k), dtype=torch.uint8, device=device)
-            measured = [0] * 6
-            if scratch.numel():
-                counts = torch.zeros(6, dtype=torch.int32, device=device)
-                _lib.check(lib.iex_form_measure(itype, m, k, nonzeros, row_offsets.data_ptr(), column_indices.data_ptr(), scratch.data_ptr(), scratch.numel(),
-                                                counts.data_ptr(), stream), "form")
-                measured = counts.tolist()
-            phases = (ctypes.c_int * 3)(*measured[:3])
-            # the kinds that some width wants
-            wanted = {0} | {lib.iex_form_choose(15 if scratch.numel() else 1, m, k, n, nonzeros, phases) for n in (256, 512, 1024, 2048, 4096, 8192)}
-            forms = [None] * 4
-            for i, kind in enumerate(self.KINDS):
-                if kind not in wanted:
-                    continue
-                room = measured[2 + i] if kind else 0
-                forms[i] = torch.empty(lib.iex_form_bytes(kind, m, k, room), dtype=torch.uint8, device=device)
-                _lib.check(lib.iex_form_build(itype, kind, m, k, nonzeros, row_offsets.data_ptr(), column_indices.data_ptr(), values.data_ptr(), room,
-                                              forms[i].data_ptr(), forms[i].numel(), scratch.data_ptr(), scratch.numel(), stream), "form")
-            torch.cuda.current_stream(device).synchronize()      # (products on any stream find it complete)
-        self._form = _iex_host.WeightForm(values, row_offsets, column_indices, m, k, forms, measured, torch.cuda.current_stream(device).stream_id)
+        measured = _form_counts(row_offsets, column_indices, m, k)
+        self._form = _iex_host.WeightForm(values, row_offsets, column_indices, m, k, 15 if measured else 1, measured or [0] * 6)
 
     def is_of(self, values, row_offsets, column_indices) -> bool:
         """Whether these are the tensors that were laid out, unchanged since.  Never of tensors that count no changes (made under

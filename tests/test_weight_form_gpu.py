@@ -245,6 +245,33 @@ def test_a_replaced_weight_on_another_stream(dev):
     assert torch.equal(out, want) and len(keep) == 48
 
 
+def test_a_form_is_laid_out_by_the_first_product_that_takes_it(dev):
+    """Not before, no other kind, and without a read back to the host once the pattern is known; products on another stream wait for it."""
+    layer = _layer(dev)
+    x = torch.randn(256, 1024, device=dev).half()
+    laid_out = lambda: [form._form.laid_out for form in layer._forms.values()]
+    assert laid_out() == [0] * 7
+    want = layer.forward(x, 2)
+    before = laid_out()
+    assert all(bin(bits).count("1") == 1 for bits in before)
+    layer.forward(x, 2)
+    assert laid_out() == before
+    side = torch.cuda.Stream()
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        for w in layer.w.values():
+            w[1].mul_(1.0)
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(50_000_000)
+            first = layer.forward(x, 2)
+        second = layer.forward(x, 2)                  # (laid out on the other stream, which has not run yet)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    torch.cuda.synchronize()
+    assert torch.equal(first, want) and torch.equal(second, want)
+
+
 def test_forms_are_refused_on_the_host(dev):
     lib = _lib.load()
     one = torch.zeros(1024, dtype=torch.int32, device=dev)
