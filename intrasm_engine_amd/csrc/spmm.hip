@@ -454,38 +454,37 @@ int launch_mfma3(const SpmmParams& p, int batch, int windows, hipStream_t stream
 // arrangement code = MFMA tile height and how the 4 multiplying waves split the C tile:
 //   1 = 32 x 64 (4 k slices)    2 = 32 x 128 as 2 x 64 columns (2 k slices)    4 = 32 x 128 (4 k slices)
 //   5 = 16 x 64 (4 k slices)    6 = 16 x 128 as 2 x 64 columns (2 k slices)
-template <int MT, int NJ, int WAVES_N, bool SPLIT>
+template <int MT, int NJ, int WAVES_N, bool SPLIT, bool FAR>
 __global__ __launch_bounds__(kF32Threads + (SPLIT ? MT * 8 : 0), 2) void spmm_mfma_f32_kernel(SpmmParams p, int tiles_m) {
   extern __shared__ __align__(16) unsigned char smem[];
-  spmm_mfma_f32_block<MT, NJ, WAVES_N, SPLIT>(p, blockIdx.x % tiles_m, blockIdx.x / tiles_m, blockIdx.y, smem);
+  spmm_mfma_f32_block<MT, NJ, WAVES_N, SPLIT, FAR>(p, blockIdx.x % tiles_m, blockIdx.x / tiles_m, blockIdx.y, smem);
 }
 
-template <int MT, int NJ, int WAVES_N, bool SPLIT>
+template <int MT, int NJ, int WAVES_N, bool SPLIT, bool FAR>
 int launch_mfma_f32_one(const SpmmParams& p, int batch, hipStream_t stream) {
   constexpr int kBN = MT * NJ * WAVES_N;
   const int tiles_m = ceil_div(p.m, MT), tiles_n = ceil_div(p.n, kBN);
   constexpr int kLds = spmm_mfma_f32_lds_bytes<MT, NJ, WAVES_N>();
-  note_kernel("spmm_mfma_f32_kernel<%d, %d, %d, %s>", MT, NJ, WAVES_N, SPLIT ? "true" : "false");
-  hipLaunchKernelGGL((spmm_mfma_f32_kernel<MT, NJ, WAVES_N, SPLIT>), dim3(tiles_m * tiles_n, batch),
+  note_kernel("spmm_mfma_f32_kernel<%d, %d, %d, %s, %s>", MT, NJ, WAVES_N, SPLIT ? "true" : "false", FAR ? "true" : "false");
+  hipLaunchKernelGGL((spmm_mfma_f32_kernel<MT, NJ, WAVES_N, SPLIT, FAR>), dim3(tiles_m * tiles_n, batch),
                      dim3(kF32Threads + (SPLIT ? MT * 8 : 0)), kLds, stream, p, tiles_m);
   return check_hip(hipGetLastError(), "spmm (matrix-core, fp32) launch");
 }
 
 template <int MT, int NJ, int WAVES_N>
-int launch_mfma_f32_w(const SpmmParams& p, int batch, int windows, bool split, hipStream_t stream) {
-  if (split) return launch_mfma_f32_one<MT, NJ, WAVES_N, true>(p, batch, stream);
-  // (the number of windows is the kernel's own affair by now; what was refused still is)
-  IEX_REQUIRE(windows == 2 || windows == 4 || windows == 8, IEX_ERR_BAD_ARGUMENT, "spmm: windows of the fp32 matrix-core variant must be 2, 4 or 8 (got %d)", windows);
-  return launch_mfma_f32_one<MT, NJ, WAVES_N, false>(p, batch, stream);
+int launch_mfma_f32_roles(const SpmmParams& p, int batch, bool split, hipStream_t stream) {
+  // what the kernel's 32-bit byte offsets reach (the dense operand's: up to a few chunks past its end)
+  if (p.nnz >= 1 << 30 || ((long long)p.k + 1024) * p.n >= 1 << 30) return launch_mfma_f32_one<MT, NJ, WAVES_N, true, true>(p, batch, stream);
+  return split ? launch_mfma_f32_one<MT, NJ, WAVES_N, true, false>(p, batch, stream) : launch_mfma_f32_one<MT, NJ, WAVES_N, false, false>(p, batch, stream);
 }
 
-inline int launch_mfma_f32(const SpmmParams& p, int batch, int arrangement, int windows, bool split, hipStream_t stream) {
+inline int launch_mfma_f32(const SpmmParams& p, int batch, int arrangement, bool split, hipStream_t stream) {
   switch (arrangement) {
-    case 1: return launch_mfma_f32_w<32, 2, 1>(p, batch, windows, split, stream);
-    case 2: return launch_mfma_f32_w<32, 2, 2>(p, batch, windows, split, stream);
-    case 4: return launch_mfma_f32_w<32, 4, 1>(p, batch, windows, split, stream);
-    case 5: return launch_mfma_f32_w<16, 4, 1>(p, batch, windows, split, stream);
-    case 6: return launch_mfma_f32_w<16, 4, 2>(p, batch, windows, split, stream);
+    case 1: return launch_mfma_f32_roles<32, 2, 1>(p, batch, split, stream);
+    case 2: return launch_mfma_f32_roles<32, 2, 2>(p, batch, split, stream);
+    case 4: return launch_mfma_f32_roles<32, 4, 1>(p, batch, split, stream);
+    case 5: return launch_mfma_f32_roles<16, 4, 1>(p, batch, split, stream);
+    case 6: return launch_mfma_f32_roles<16, 4, 2>(p, batch, split, stream);
   }
   return fail(IEX_ERR_BAD_ARGUMENT, "spmm: arrangement of the fp32 matrix-core variant must be 1, 2, 4, 5 or 6 (got %d)", arrangement);
 }
@@ -611,21 +610,18 @@ template <typename T>
 bool matrix_core_kernel_applies(const SpmmParams& p, int batch) { return mfma_variant<T>(p, batch, Choice{}).kind != 0; }
 
 // fp32 on the matrix cores: int32 indices, n a multiple of 4, 16-byte aligned dense operands.
-// Returns the arrangement code (0 = use a gather kernel) and sets the number of register windows.
+// Returns the arrangement code (0 = use a gather kernel).
 template <typename T, typename IT>
-int mfma_f32_variant(const SpmmParams& p, int batch, const Choice& ch, int& windows) {
+int mfma_f32_variant(const SpmmParams& p, int batch, const Choice& ch) {
   if (!std::is_same<T, float>::value || !std::is_same<IT, int>::value) return 0;
   if (ch.variant != 0 && ch.variant != 5) return 0;
   if (!(p.nnz > 0 && p.n % 4 == 0 && aligned(p.dense, 16) && aligned(p.out, 16))) return 0;  // (also when forced)
-  if (p.nnz >= 1 << 30 || ((long long)p.k + 1024) * p.n >= 1 << 30) return 0;                 // 32-bit byte offsets
   const double density = (p.m > 0 && p.k > 0) ? (double)p.nnz / ((double)p.m * p.k) : 0.0;
   // 32-row tiles with 128 columns per wave when that still gives most CUs a workgroup; else
   // 16-row tiles (twice the workgroups, twice the reads of the dense operand)
   const long long tiles_m = ceil_div(p.m, 32);
   int arrangement = tiles_m * ceil_div(p.n, 128) * batch >= 200 ? 4 : (p.n <= 64 ? 5 : 6);
   if (ch.nt) arrangement = ch.nt;
-  const double run = density * 128;  // nonzeros of a row per chunk
-  windows = ch.rpw ? ch.rpw : (run <= 12.0 ? 2 : run <= 40.0 ? 4 : 8);
   if (ch.variant == 5) return arrangement;
   // Measured on MI355X: 70-105 dense-equivalent TFLOP/s (the fp32 MFMA rate is 153; fp32 MFMAs
   // run on the vector ALUs, so the expansion's instructions add to their time instead of hiding
@@ -787,8 +783,12 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
     return launch_smallk<T, IT>(p, batch, stream);
   }
   if constexpr (std::is_same<T, float>::value && std::is_same<IT, int>::value) {
-    int windows = 0;
-    if (const int arr = mfma_f32_variant<T, IT>(p, batch, ch, windows)) return launch_mfma_f32(p, batch, arr, windows, ch.lpg != 8, stream);  // (lanes-per-group code 8 = no role split, for tuning)
+    if (const int arr = mfma_f32_variant<T, IT>(p, batch, ch)) {
+      const bool split = ch.lpg != 8;   // (lanes-per-group code 8 = no role split, for tuning)
+      // (a row's windows are the kernel's own affair; numbers that it never had are refused)
+      IEX_REQUIRE(split || ch.rpw == 0 || ch.rpw == 2 || ch.rpw == 4 || ch.rpw == 8, IEX_ERR_BAD_ARGUMENT, "spmm: windows of the fp32 matrix-core variant must be 2, 4 or 8 (got %d)", ch.rpw);
+      return launch_mfma_f32(p, batch, arr, split, stream);
+    }
   }
   if (ch.variant == 6 && sizeof(T) == 2 && p.nnz > 0 && p.n % 8 == 0 && aligned(p.dense, 16) && aligned(p.out, 16))
     return launch_mfma3<T, IT>(p, batch, ch.rpw ? ch.rpw : mfma3_windows(p), stream);

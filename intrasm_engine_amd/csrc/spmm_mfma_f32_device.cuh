@@ -30,9 +30,10 @@
 // geometric lengths, 20 % and 30 % density 128 -> 112, rows of one length, 2 / 10 / 30 / 50 / 100 % 86 / 91 / 104 / 116 / 130 -> 90 / 91 /
 // 92 / 109 / 112; n = 128 (16 rows), geometric 92 -> 74, equal 30 % 68 -> 56; 11008 x 4096, n = 1024, 30 % 1051 -> 1023.  (Expanding wavefronts
 // at raised priority: 2 us more.)
+// FAR: the dense operand or the nonzeros pass the 4 GiB that a buffer's offsets reach; they are read by 64-bit addresses then (1024 x 1024 at
+// 50 %, n = 2^20: 32 ms, the row kernel 68).
 // Requirements (checked by the host): n % 4 == 0, 16-byte aligned dense operand and output,
-// strictly ascending column indices inside a row, (k + 1024) n and
-// nnz below 2^30 (32-bit byte offsets).
+// strictly ascending column indices inside a row; without FAR (k + 1024) n and nnz below 2^30.
 #pragma once
 #include "spmm_device.cuh"
 
@@ -41,7 +42,7 @@ namespace iex {
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-// columns of A per chunk: at most 128 nonzeros of a row fall into one, which 16 windows of 8 hold
+// columns of A per chunk: at most 128 nonzeros of a row fall into one, which two windows of 64 hold
 template <int MT>
 constexpr int spmm_mfma_f32_bka() { return 128; }
 constexpr int kF32Threads = 256;       // per role
@@ -58,7 +59,7 @@ struct F32Frag {
   float v[NJ];
 };
 
-template <int MT, int NJ, int WAVES_N, bool SPLIT>
+template <int MT, int NJ, int WAVES_N, bool SPLIT, bool FAR>
 __device__ __forceinline__ void spmm_mfma_f32_block(const SpmmParams& p, int tile_m, int tile_n, int z, unsigned char* smem) {
   constexpr int BM = MT, BKA = spmm_mfma_f32_bka<MT>();
   constexpr int LDA = BKA + 4;            // floats: 16 consecutive rows start in distinct 4-bank groups
@@ -103,6 +104,12 @@ __device__ __forceinline__ void spmm_mfma_f32_block(const SpmmParams& p, int til
   bool wide = false;
   // (scalar offsets never pass a buffer's end: only up to there does the range check hold)
   auto load_window = [&](int first, int skip, int& c, float& v) {
+    if constexpr (FAR) {
+      const int at = min(lane + skip, p.nnz - 1 - first);   // (-1 behind the last nonzero)
+      c = (static_cast<const int*>(p.cols) + first)[at];
+      v = (values + first)[at];
+      return;
+    }
     c = __builtin_amdgcn_raw_buffer_load_b32(cols_buf, (lane + skip) * 4, (unsigned)first * 4u, 0);
     v = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(vals_buf, (lane + skip) * 4, (unsigned)first * 4u, 0));
   };
@@ -175,6 +182,16 @@ __device__ __forceinline__ void spmm_mfma_f32_block(const SpmmParams& p, int til
 #pragma unroll
   for (int i = 0; i < 4; ++i) b_lane[i] = (unsigned)((half * 4 + i) * p.n + (col < p.n ? col : 0)) * 4u;   // n % 4 == 0: the NJ columns are in or out together
   auto load_b = [&](F32Frag<NJ> (&f)[4], int kbase) {  // kbase = first k row of the group
+    if constexpr (FAR) {   // (past the matrix: its last row)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        typedef float vec __attribute__((ext_vector_type(NJ)));
+        const vec v = *reinterpret_cast<const vec*>(B + (size_t)min(kbase + half * 4 + i, p.k - 1) * p.n + (col < p.n ? col : 0));
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) f[i].v[j] = v[j];
+      }
+      return;
+    }
     const unsigned at = (unsigned)min(kbase, p.k) * (unsigned)p.n * 4u;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

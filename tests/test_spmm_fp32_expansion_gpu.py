@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from intrasm_engine_amd import workloads as W
+from intrasm_engine_amd import _lib, workloads as W
 from intrasm_engine_amd.pytorch import ops as pyops
 from _util import assert_close, to_dev
 
@@ -34,3 +34,30 @@ def test_runs_at_the_edges_of_the_windows(oracle, dev, arrangement, m, k, filler
     scale = oracle.spmm_abs_scale(b_np, csr.row_indices, csr.values, csr.row_offsets, csr.column_indices, m)
     # at most k roundings of a sum, each 2^-24 of it: k * 6e-8 of the sum of magnitudes
     assert_close(out.cpu().numpy(), want, scale, max(k, 16) * 6e-8, f"arrangement {arrangement} {m} x {k}")
+
+
+@pytest.mark.parametrize("m,k,n,density", [(72, 300, 1 << 22, 0.5),            # 5 GB of the dense operand
+                                           (32776, 32768, 128, 1.0)])          # 2^30 nonzeros and a few
+def test_beyond_a_buffers_reach(dev, m, k, n, density):
+    """Operands whose byte offsets take more than 32 bits stay with the matrix cores, and both ends of them are read."""
+    gen = torch.Generator(dev).manual_seed(m)
+    rows = torch.rand(m, k, device=dev, generator=gen) < density if density < 1 else None
+    ro = torch.cat([torch.zeros(1, device=dev, dtype=torch.int64), rows.sum(1).cumsum(0) if rows is not None else torch.arange(1, m + 1, device=dev) * k]).int()
+    ci = rows.nonzero()[:, 1].int() if rows is not None else torch.arange(k, device=dev, dtype=torch.int32).repeat(m)
+    v = torch.randn(ci.numel(), device=dev, generator=gen)
+    a = torch.zeros(m, k, device=dev).masked_scatter_(rows, v) if rows is not None else v.view(m, k)
+    b = torch.randn(1, k, n, device=dev, generator=gen)
+    ri = torch.arange(m, device=dev, dtype=torch.int32)
+    out = torch.empty(1, m, n, device=dev)
+    rc = _lib.load().iex_spmm_ex(_lib.F32, _lib.I32, 0, m, k, n, ci.numel(), ri.data_ptr(), v.data_ptr(), ro.data_ptr(), ci.data_ptr(), b.data_ptr(),
+                                 None, out.data_ptr(), torch.cuda.current_stream().cuda_stream, 1)
+    _lib.check(rc, "spmm")
+    assert "spmm_mfma_f32_kernel" in _lib.last_kernels()
+    for columns in (slice(0, 128), slice(n // 2, n // 2 + 128), slice(n - 128, n)):
+        part = b[0, :, columns].double()
+        want = torch.cat([r.double() @ part for r in a.split(1024)])
+        scale = torch.cat([r.double().abs() @ part.abs() for r in a.split(1024)])
+        # at most k roundings of a sum, each 2^-24 of it
+        assert bool(((out[0, :, columns].double() - want).abs() <= k * 6e-8 * scale).all())
+    del a, b, out, v, ci, rows
+    torch.cuda.empty_cache()
