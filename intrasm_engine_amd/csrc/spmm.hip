@@ -26,7 +26,6 @@ int launch_one(const SpmmParams& p, int batch, hipStream_t stream) {
   constexpr int kRowsPerBlock = kWavesPerBlock / WPR;
   dim3 grid(ceil_div(p.m, kRowsPerBlock), ceil_div(p.n, NT * LPG * VEC), batch);
   dim3 block(kWavesPerBlock * kWave);
-  note_kernel("spmm_kernel<%s, %s, %d, %d, %d, %d>", type_name<T>(), type_name<IT>(), VEC, LPG, WPR, NT);
   // Several nonzeros per gather and rows of at most 128 on average, more of them than are resident: windows of four gathers
   // instead of eight.  Fewer registers (63 instead of 94, 8 wavefronts per SIMD instead of 5), and a short share is mostly
   // its last, partial window.  MI355X, us, eight / four: 11008 x 1000, 90 / 95 % sparse, fp32 n = 64 21 / 16 and 21 / 13, n =
@@ -34,12 +33,15 @@ int launch_one(const SpmmParams& p, int batch, hipStream_t stream) {
   // flight (4096 x 4096, 90 %, fp16 n = 128 22 / 26, fp32 n = 64 22 / 27), few rows leave the registers idle (1024 x 1024, 95 %, fp16 n
   // = 256 4.7 / 5.1).  There the last gathers of a chunk go by fours and twos in 16 bits (1024 - 4096, 90 - 98 %: 3 - 9 % less time); in
   // 32 bits that costs the 4096 x 4096 cells with long rows 5 %.
+  const char* const name = "spmm_kernel<%s, %s, %d, %d, %d, %d, %s>";
   if constexpr (LPG < kWave && NT == 1) {
     if (p.nnz <= 128ll * p.m && (long long)p.m * grid.y * batch * WPR > 16384) {
+      note_kernel(name, type_name<T>(), type_name<IT>(), VEC, LPG, WPR, NT, "true");
       hipLaunchKernelGGL((spmm_kernel<T, IT, VEC, LPG, WPR, NT, true>), grid, block, 0, stream, p);
       return check_hip(hipGetLastError(), "spmm launch");
     }
   }
+  note_kernel(name, type_name<T>(), type_name<IT>(), VEC, LPG, WPR, NT, "false");
   hipLaunchKernelGGL((spmm_kernel<T, IT, VEC, LPG, WPR, NT, false>), grid, block, 0, stream, p);
   return check_hip(hipGetLastError(), "spmm launch");
 }

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from intrasm_engine_amd import workloads as W
+from intrasm_engine_amd import _lib, workloads as W
 from intrasm_engine_amd.pytorch import ops as pyops
 from _util import assert_close, rounded, to_dev
 
@@ -26,6 +26,7 @@ def test_shares_of_every_length(oracle, dev, dtype, wpr, n, m):
     ri, v, ro_t, ci_t = to_dev(csr, dev, dtype)
     b = torch.from_numpy(b_np).to(dev).to(dtype)
     out = pyops._spmm(b, ri, v, ro_t, ci_t, m, per_batch_values=False, accumulate=False, dtypes=(dtype,), allow_i16=False, force_variant=1, force_wpr=wpr)
+    assert (", true>" in _lib.last_kernels()) == (m > 66 and wpr == 4 and (n < 256 or dtype != torch.float32)), _lib.last_kernels()
     b_r, v_r = rounded(b_np, dtype), rounded(csr.values, dtype)
     want = oracle.spmm(b_r, csr.row_indices, v_r, csr.row_offsets, csr.column_indices, m)
     scale = oracle.spmm_abs_scale(b_r, csr.row_indices, v_r, csr.row_offsets, csr.column_indices, m)
