@@ -13,7 +13,7 @@ __global__ __launch_bounds__(512, 1) void two_four_kernel(GemmParams p, TwoFourO
   extern __shared__ __align__(16) unsigned char smem[];
   int tile_m, tile_n;
   if (!xcd_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;  // uniform per block
-  two_four_tile<BF16, WM>(p, f, tile_m, tile_n, blockIdx.y, smem);
+  two_four_tile<BF16, WM>(p, f, tile_m, tile_n, smem);
 }
 
 template <typename Kernel>
@@ -26,7 +26,7 @@ int allow_lds(Kernel kernel, int bytes, bool& raised) {
 }
 
 template <bool BF16, int WM>
-int launch_product(GemmParams p, const TwoFourOperand& f, int batch, hipStream_t stream) {
+int launch_product(GemmParams p, const TwoFourOperand& f, hipStream_t stream) {
   constexpr int BM = 64 * WM, lds = two_four_lds_bytes(BM);
   auto kern = two_four_kernel<BF16, WM>;
   static thread_local bool raised = false;   // per instantiation
@@ -35,7 +35,7 @@ int launch_product(GemmParams p, const TwoFourOperand& f, int batch, hipStream_t
   p.tiles_n = ceil_div(p.N, kTwoFourBN);
   const int per_xcd = ceil_div((long long)p.tiles_m * p.tiles_n, kXcds);
   note_kernel("two_four_kernel<%s> (%d x %d tiles)", BF16 ? "bf16" : "f16", BM, kTwoFourBN);
-  hipLaunchKernelGGL(kern, dim3(per_xcd * kXcds, batch), dim3(512), lds, stream, p, f);
+  hipLaunchKernelGGL(kern, dim3(per_xcd * kXcds), dim3(512), lds, stream, p, f);
   return check_hip(hipGetLastError(), "two-of-four product launch");
 }
 
@@ -52,13 +52,13 @@ template <typename IT>
 int launch_form(const TwoFourForm& f, int m, int k, const int* row_offsets, const void* cols, const void* values, unsigned char* form, unsigned* marks,
                 hipStream_t stream) {
   if (int rc = launch_marks<IT>(m, k, row_offsets, cols, marks, stream)) return rc;
-  const TwoFourSource s{m, k, row_offsets, cols, static_cast<const uint16_t*>(values), nullptr};
+  const TwoFourSource s{m, k, row_offsets, cols, static_cast<const uint16_t*>(values)};
   const TwoFourTarget t{form, reinterpret_cast<int*>(form + f.counts_at), reinterpret_cast<unsigned*>(form + f.lists_at), reinterpret_cast<uint2*>(form + f.ranks_at),
                         f.bm, f.phases, f.spill_phases, f.list_room, f.words, f.block, f.panel};
   note_kernel("two_four_rank_kernel");
   hipLaunchKernelGGL(two_four_rank_kernel, dim3(f.panels * 2), dim3(256), 0, stream, t, marks, ceil_div(m, 32));
   const int rows = two_four_rows(k), lds = two_four_rows_lds_bytes(rows, f.phases);
-  auto kern = two_four_form_kernel<IT, false>;
+  auto kern = two_four_form_kernel<IT>;
   static thread_local bool raised = false;   // per instantiation
   if (int rc = allow_lds(kern, 80 * 1024, raised)) return rc;
   note_kernel("two_four_form_kernel<%s>", type_name<IT>());
@@ -166,9 +166,9 @@ extern "C" int iex_form_product(int dtype, int kind, int m, int k, int n, int sp
   const unsigned char* at = static_cast<const unsigned char*>(form);
   const TwoFourOperand o{at, reinterpret_cast<const int*>(at + f.counts_at), reinterpret_cast<const unsigned*>(at + f.lists_at), f.phases, f.spill_phases, f.list_room, f.panel};
   const bool bf = dtype == IEX_BF16;
-  if (kind == 256) return bf ? launch_product<true, 4>(p, o, 1, s) : launch_product<false, 4>(p, o, 1, s);
-  if (kind == 192) return bf ? launch_product<true, 3>(p, o, 1, s) : launch_product<false, 3>(p, o, 1, s);
-  return bf ? launch_product<true, 2>(p, o, 1, s) : launch_product<false, 2>(p, o, 1, s);
+  if (kind == 256) return bf ? launch_product<true, 4>(p, o, s) : launch_product<false, 4>(p, o, s);
+  if (kind == 192) return bf ? launch_product<true, 3>(p, o, s) : launch_product<false, 3>(p, o, s);
+  return bf ? launch_product<true, 2>(p, o, s) : launch_product<false, 2>(p, o, s);
 }
 
 extern "C" int iex_form_choose(int kinds, int m, int k, int n, int nonzeros, const int* spill_phases) {

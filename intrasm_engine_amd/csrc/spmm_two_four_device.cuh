@@ -63,7 +63,6 @@ struct TwoFourSource {   // the CSR matrix
   const int* row_offsets;
   const void* cols;
   const uint16_t* values;
-  const long long* perm;   // entry j has the value values[perm[j]] (null: values[j])
 };
 struct TwoFourTarget {
   unsigned char* form;
@@ -190,7 +189,7 @@ inline int two_four_rows(int k) {   // rows per workgroup: about 36 KB of LDS, f
 }
 inline int two_four_rows_lds_bytes(int rows, int phases) { return rows * (phases * 64 + 16) + rows * (phases * 8 + 4); }
 
-template <typename IT, bool PERM>
+template <typename IT>
 __global__ __launch_bounds__(kTwoFourRowThreads) void two_four_form_kernel(TwoFourSource s, TwoFourTarget t, int rows) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int WAVES = kTwoFourRowThreads / 64, U = 4, STEP = 61;
@@ -207,8 +206,7 @@ __global__ __launch_bounds__(kTwoFourRowThreads) void two_four_form_kernel(TwoFo
   const int end = min(pos + share, entries);
 
   const IT* __restrict__ cols = static_cast<const IT*>(s.cols) + first;
-  const uint16_t* __restrict__ values = s.values + (PERM ? 0 : first);
-  const long long* __restrict__ perm = PERM ? s.perm + first : nullptr;
+  const uint16_t* __restrict__ values = s.values + first;
   int c[U];
   uint16_t v[U];
   auto load = [&]() {   // entries pos - 2 .. + 61 of every step
@@ -217,8 +215,7 @@ __global__ __launch_bounds__(kTwoFourRowThreads) void two_four_form_kernel(TwoFo
     for (int u = 0; u < U; ++u) {
       const unsigned j = (unsigned)max(min(pos + u * STEP - 2 + lane, entries - 1), 0);
       c[u] = (int)*reinterpret_cast<const IT*>(reinterpret_cast<const char*>(cols) + j * (unsigned)sizeof(IT));
-      v[u] = PERM ? values[*reinterpret_cast<const long long*>(reinterpret_cast<const char*>(perm) + j * 8u)]
-                  : *reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(values) + j * 2u);
+      v[u] = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(values) + j * 2u);
     }
   };
   load();
@@ -354,7 +351,7 @@ constexpr int two_four_lds_bytes(int bm) { return 3 * two_four_stage_bytes(bm); 
 // dense product are 64 k's work and here 32's.  This one with a step's loads in one burst 186, spread over the step 176,
 // with single MFMAs between the other instructions instead of four in a row 149.
 template <bool BF16, int WM>
-__device__ __forceinline__ void two_four_tile(const GemmParams& p, const TwoFourOperand& f, int tile_m, int tile_n, int z, unsigned char* smem) {
+__device__ __forceinline__ void two_four_tile(const GemmParams& p, const TwoFourOperand& f, int tile_m, int tile_n, unsigned char* smem) {
   constexpr int WN = 2, WCN = 4, WAVES = 8;
   constexpr int BM = 2 * WM * 32, BN = kTwoFourBN;
   constexpr int BLOCK = BM == 192 ? 14 * 1024 : BM * 72;
@@ -373,8 +370,8 @@ __device__ __forceinline__ void two_four_tile(const GemmParams& p, const TwoFour
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WCN, wn = wave % WCN;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const u16* __restrict__ B = static_cast<const u16*>(p.B) + (size_t)z * p.stride_b;
-  u16* __restrict__ C = static_cast<u16*>(p.C) + (size_t)z * p.stride_c;
+  const u16* __restrict__ B = static_cast<const u16*>(p.B);
+  u16* __restrict__ C = static_cast<u16*>(p.C);
   const unsigned lds0 = (unsigned)(size_t)(lds_u8*)smem;
   const int ldb = p.ldb, kb = p.kb;
 
@@ -541,7 +538,7 @@ __device__ __forceinline__ void two_four_tile(const GemmParams& p, const TwoFour
   wait_vmcnt<0>();   // the re-fetched last blocks: nothing may still be writing LDS when the stages are reused
   static_assert(WAVES * gemm_store_lds_bytes<WN>() <= two_four_lds_bytes(BM), "the epilogue fits the stages");
   __syncthreads();
-  const u16* aux = p.aux ? static_cast<const u16*>(p.aux) + (size_t)z * p.stride_c : nullptr;
+  const u16* aux = static_cast<const u16*>(p.aux);
   gemm_store_tile<BF16, WM, WN>(p, acc, C, aux, m0, n0, wm, wn, lane, smem + wave * gemm_store_lds_bytes<WN>(), p.stream_out != 0);
 }
 
