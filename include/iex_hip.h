@@ -273,6 +273,7 @@ int iex_spmm_transposed(int dtype, int itype, int m, int k, int n, int nonzeros,
  *   iex_form_build    needs the scratch memory for the two-of-four kinds; at least three nonzeros, fewer than 2^29.
  *   iex_form_choose   which of `kinds` (bit 0: kind 0, bits 1, 2, 3: kinds 128, 192, 256) is estimated fastest for n columns (host code;
  *                     spill_phases: the first three measured numbers, host memory), -1 where a SpMM that reads the CSR arrays is.
+ *                     | IEX_FORM_EACH_CALL: for a program that lays the weight out anew for every product; that time counts.
  *   iex_form_product  aux / aux_mode as in iex_spmm_aux (aux NULL: none).  n a multiple of 8, dense 16-byte aligned; workspace
  *                     (256-byte aligned, iex_form_product_workspace_bytes, may be NULL) lets the dense product take K in parts.
  *                     Non-finite entries of dense rows that A does not reference may reach the output, as with the dense form. */
@@ -282,6 +283,7 @@ int iex_form_measure(int itype, int m, int k, int nonzeros, const int* row_offse
 size_t iex_form_bytes(int kind, int m, int k, int spill_phases);
 int iex_form_build(int itype, int kind, int m, int k, int nonzeros, const int* row_offsets, const void* column_indices, const void* values,
                    int spill_phases, void* form, size_t form_bytes, void* scratch, size_t scratch_bytes, void* stream);
+#define IEX_FORM_EACH_CALL 0x10
 int iex_form_choose(int kinds, int m, int k, int n, int nonzeros, const int* spill_phases);
 size_t iex_form_product_workspace_bytes(int kind, int m, int k, int n);
 int iex_form_product(int dtype, int kind, int m, int k, int n, int spill_phases, const void* form, const void* dense, const void* aux, int aux_mode,

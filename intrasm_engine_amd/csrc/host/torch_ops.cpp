@@ -381,7 +381,8 @@ std::optional<Tensor> spmm_with(const Tensor& x, const Tensor& row_indices, cons
 // A sparse weight for a program that keeps it (ops.WeightForm makes it): the product with x, combined with `other` as in spmm_with.  Nothing is
 // returned where the call is not served here -- operands that do not fit, a gradient wanted, kernels forced, an operator on the CSR arrays that is
 // faster.  The first product that takes a kind of form lays it out, on its stream and without waiting; later ones find it, on other streams behind
-// an event.  A captured call lays the weight out inside the graph: replays follow the CSR arrays, and give the same bits as a call.
+// an event.  A captured call lays the weight out inside the graph, so that replays follow the CSR arrays; it takes another way through the product than a
+// call, with the sums in another order, where laying out at every replay would cost more than it gains.
 struct WeightForm {
   static constexpr int kAnyRoom = 1 << 20;
   struct Layout {
@@ -429,11 +430,12 @@ struct WeightForm {
       return {};
     if (other && (!plain(*other, 2) || other->size(0) != m || other->size(1) != n || other->scalar_type() != x.scalar_type() || other->device() != x.device())) return {};
     const c10::DeviceGuard guard(x.device());
-    const int kind = iex_form_choose(kinds, m, k, n, nonzeros, phases.data());
+    const bool captured = capturing();
+    const int kind = iex_form_choose(captured ? kinds | IEX_FORM_EACH_CALL : kinds, m, k, n, nonzeros, phases.data());
     if (kind < 0) return {};
     int room = kind ? rooms[kind / 64 - 2] : 0;
     Tensor form;
-    if (capturing()) {
+    if (captured) {
       room = kind ? kAnyRoom : 0;   // (the pattern of a later replay may spill more)
       form = lay_out(kind, room, x);
     } else {

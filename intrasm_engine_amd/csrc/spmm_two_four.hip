@@ -84,6 +84,13 @@ double two_four_seconds(int kind, int m, int n, double steps) {
   return 6e-6 + rounds * (4e-6 + steps * (kind == 256 ? 0.98e-6 : kind == 192 ? 0.80e-6 : 0.63e-6));
 }
 
+// Seconds of laying a form out (us measured: 4096^2 dense 8.5 at 10 % / 12.5 at 2:4, two-of-four 19 / 31; 11008 x 4096 18.4 / 28.3, 31 / 56; 4096 x
+// 11008 19.6 / 32.7, 50 / 69; 1024^2, 2:4 4.5, 12; the longer rows of the last one leave a workgroup of the two-of-four form two of them).
+double layout_seconds(int kind, int m, int k, int nonzeros) {
+  const double cells = (double)m * k;
+  return kind == 0 ? 3.5e-6 + cells * 3.2e-13 + nonzeros * 4.5e-13 : 10e-6 + cells * (two_four_rows(k) <= 2 ? 6e-13 : 3.5e-13) + nonzeros * 1.4e-12;
+}
+
 }  // namespace
 }  // namespace iex
 
@@ -175,13 +182,22 @@ extern "C" int iex_form_choose(int kinds, int m, int k, int n, int nonzeros, con
   int best = -1;
   double seconds = 1e9;
   if (m <= 0 || k <= 0 || n <= 0 || nonzeros <= 0) return best;
-  if ((kinds & 1) && form_shape_fits(0, m, k)) best = 0, seconds = gemm_seconds(m, n, round8(k));
+  // IEX_FORM_EACH_CALL: the laying out counts too.  A weight multiplied once as it is laid out: two-of-four forms pay from many columns on (us of
+  // the product, layout and all, dense / two-of-four, 2:4 11008 x 4096: n = 512 80 / 94, 1024 106 / 111, 2048 187 / 167), dense ones not for few (2752 x
+  // 1024, 2:4, n = 64 14.1, CSR 10.1; 4096 x 11008, 10 %, n = 64 45, CSR 24.5).  A weight of up to 2^17 cells keeps the kind, and the bits, of a call
+  // with a kept form: laying it out is one launch of less than 4 us.
+  const bool each_call = (kinds & IEX_FORM_EACH_CALL) && (long long)m * k > (1 << 17);
+  auto layout = [&](int kind) { return each_call ? layout_seconds(kind, m, k, nonzeros) : 0.0; };
+  if ((kinds & 1) && form_shape_fits(0, m, k)) best = 0, seconds = gemm_seconds(m, n, round8(k)) + layout(0);
   for (int i = 0; i < 3; ++i) {
     const int kind = 128 + 64 * i, half_panels = ceil_div(m, kind / 2);
     if (!(kinds >> (i + 1) & 1) || !form_shape_fits(kind, m, k) || !spill_phases) continue;
     const double steps = ceil_div(k, 128) * 2 + 1.1 * spill_phases[i] / half_panels;   // (a panel takes the longer of its halves)
-    const double mine = two_four_seconds(kind, m, n, steps);
+    const double mine = two_four_seconds(kind, m, n, steps) + layout(kind);
     if (mine < 0.95 * seconds || best < 0) best = kind, seconds = mine;
   }
-  return best >= 0 && spmm_seconds(m, k, n, nonzeros) < seconds ? -1 : best;
+  double by_rows = spmm_seconds(m, k, n, nonzeros);
+  // (narrow products: 250 nonzeros a ns whatever n is, 2:4 11008 x 4096, n = 8 .. 32 88 us; a near tie goes to the form, for the bits of a call)
+  if (each_call) by_rows = 1.15 * std::max(by_rows, 5e-6 + nonzeros * 4e-12);
+  return best >= 0 && by_rows < seconds ? -1 : best;
 }
