@@ -397,12 +397,21 @@ struct WeightForm {
   std::array<int, 3> phases, rooms;
   int kinds;                       // a bit for each that the weight can be laid out as
   Tensor values, row_offsets, column_indices;
+  std::array<int64_t, 3> versions;   // of the three, when the form was made for them
 
-  WeightForm(const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, int64_t m, int64_t k, int kinds, const std::vector<int>& measured)
-      : dtype(dtype_code(values.scalar_type())), m(m), k(k), nonzeros(column_indices.numel()), kinds(kinds), values(values), row_offsets(row_offsets), column_indices(column_indices) {
+  WeightForm(const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, const std::array<int64_t, 3>& versions, int64_t m, int64_t k, int kinds,
+             const std::vector<int>& measured)
+      : dtype(dtype_code(values.scalar_type())), m(m), k(k), nonzeros(column_indices.numel()), kinds(kinds), values(values), row_offsets(row_offsets), column_indices(column_indices),
+        versions(versions) {
     TORCH_CHECK(measured.size() == 6, "WeightForm: six numbers");
     std::copy_n(measured.begin(), 3, phases.begin());
     std::copy_n(measured.begin() + 3, 3, rooms.begin());
+  }
+
+  // whether these are the tensors it was made for, unchanged since (never of tensors that count no changes)
+  bool is_of(const Tensor& v, const Tensor& offsets, const Tensor& columns) const {
+    auto same = [](const Tensor& mine, const Tensor& given, int64_t version) { return given.is_same(mine) && !given.is_inference() && given._version() == version; };
+    return same(values, v, versions[0]) && same(row_offsets, offsets, versions[1]) && same(column_indices, columns, versions[2]);
   }
 
   int laid_out() {   // a bit for each kind that is
@@ -422,17 +431,40 @@ struct WeightForm {
     return form;
   }
 
-  std::optional<Tensor> product(const Tensor& x, const std::optional<Tensor>& other, int mode) {
+  // the kind of form that serves the call, -1: none; `captured` is looked up where it matters
+  int kind_for(const Tensor& x, const std::optional<Tensor>& other, bool& captured) const {
     const int64_t n = x.dim() == 2 ? x.size(1) : 0;
     if (forced || !plain(x, 2) || x.size(0) != k || n == 0 || n % 8 || k * n >= (1ll << 31) || m * n >= (1ll << 31) || dtype_code(x.scalar_type()) != dtype ||
         x.device() != values.device() || reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 ||
         (at::GradMode::is_enabled() && (x.requires_grad() || (other && other->requires_grad()))))
-      return {};
-    if (other && (!plain(*other, 2) || other->size(0) != m || other->size(1) != n || other->scalar_type() != x.scalar_type() || other->device() != x.device())) return {};
+      return -1;
+    if (other && (!plain(*other, 2) || other->size(0) != m || other->size(1) != n || other->scalar_type() != x.scalar_type() || other->device() != x.device())) return -1;
+    const int kept = iex_form_choose(kinds, m, k, n, nonzeros, phases.data()), each_call = iex_form_choose(kinds | IEX_FORM_EACH_CALL, m, k, n, nonzeros, phases.data());
+    captured = false;
+    if (kept < 0 && each_call < 0) return -1;
     const c10::DeviceGuard guard(x.device());
-    const bool captured = capturing();
-    const int kind = iex_form_choose(captured ? kinds | IEX_FORM_EACH_CALL : kinds, m, k, n, nonzeros, phases.data());
-    if (kind < 0) return {};
+    captured = capturing();
+    return captured ? each_call : kept;
+  }
+
+  // None: an operator on the CSR arrays serves the call.  False: the form is not of these tensors as they are now.
+  py::object serve(const Tensor& v, const Tensor& offsets, const Tensor& columns, const Tensor& x, const std::optional<Tensor>& other, int mode) {
+    if (!is_of(v, offsets, columns)) return py::bool_(false);
+    bool captured;
+    const int kind = kind_for(x, other, captured);
+    return kind < 0 ? py::object(py::none()) : py::cast(product_by(kind, captured, x, other, mode));
+  }
+
+  std::optional<Tensor> product(const Tensor& x, const std::optional<Tensor>& other, int mode) {
+    bool captured;
+    const int kind = kind_for(x, other, captured);
+    return kind < 0 ? std::nullopt : std::optional<Tensor>(product_by(kind, captured, x, other, mode));
+  }
+
+  Tensor product_by(int kind, bool captured, const Tensor& x, const std::optional<Tensor>& other, int mode) {
+    const py::gil_scoped_release nobody_waits_for_layouts_mutex_with_it;
+    const c10::DeviceGuard guard(x.device());
+    const int64_t n = x.size(1);
     int room = kind ? rooms[kind / 64 - 2] : 0;
     Tensor form;
     if (captured) {
@@ -647,11 +679,12 @@ PYBIND11_MODULE(_iex_host, module) {
   module.def("spmm_with", &spmm_with);
   module.def("attention", &attention);
   py::class_<WeightForm>(module, "WeightForm")
-      .def(py::init<const Tensor&, const Tensor&, const Tensor&, int64_t, int64_t, int, const std::vector<int>&>())
+      .def(py::init<const Tensor&, const Tensor&, const Tensor&, const std::array<int64_t, 3>&, int64_t, int64_t, int, const std::vector<int>&>())
+      .def("is_of", &WeightForm::is_of)
       .def_readonly("kinds", &WeightForm::kinds)
-      // (nobody waits for layouts_mutex with the interpreter's lock in hand)
       .def_property_readonly("laid_out", &WeightForm::laid_out, py::call_guard<py::gil_scoped_release>())
-      .def("product", &WeightForm::product, py::arg("x"), py::arg("other") = std::nullopt, py::arg("mode") = 0, py::call_guard<py::gil_scoped_release>());
+      .def("product", &WeightForm::product, py::arg("x"), py::arg("other") = std::nullopt, py::arg("mode") = 0)
+      .def("serve", &WeightForm::serve);
   module.def("sparse_attention", &sparse_attention);
   module.def("set_mask_tables", &set_mask_tables);
   module.def("trainable_spmm", &trainable_spmm);

@@ -91,12 +91,14 @@ class SparseDecoderLayer:
         """The product by what was laid out, of the weight as it is now; None where the operators have to serve it."""
         if not self._keep_forms:
             return None
-        form, (_, v, ro, ci, _) = self._forms[name], self.w[name]
-        if not form.is_of(v, ro, ci):
+        _, v, ro, ci, _ = self.w[name]
+        out = self._forms[name].serve(v, ro, ci, x, other, mode)
+        if out is False:
             if torch.cuda.is_current_stream_capturing() or any(t.is_inference() for t in (v, ro, ci)):
                 return None
             form = self._forms[name] = self._lay_out(name)
-        return form.product(x, other, mode)
+            out = form.product(x, other, mode)
+        return out
 
     def proj(self, name: str, x: torch.Tensor) -> torch.Tensor:
         """(k, tokens) -> (m, tokens)."""

@@ -416,7 +416,9 @@ class WeightForm:
                 _csr_status(row_offsets, column_indices, k) != 0 or _lib.load().iex_form_bytes(0, m, k, 0) == 0:
             return
         measured = _form_counts(row_offsets, column_indices, m, k)
-        self._form = _iex_host.WeightForm(values, row_offsets, column_indices, m, k, 15 if measured else 1, measured or [0] * 6)
+        self._form = _iex_host.WeightForm(values, row_offsets, column_indices, self._versions, m, k, 15 if measured else 1, measured or [0] * 6)
+        # (asked by every product of a layer: without a Python frame around it)
+        self.serve = self._form.serve
 
     def is_of(self, values, row_offsets, column_indices) -> bool:
         """Whether these are the tensors that were laid out, unchanged since.  Never of tensors that count no changes (made under
@@ -428,6 +430,10 @@ class WeightForm:
         """``weight @ x``, plus ``other`` (mode 1) or times its SiLU (mode 2) before it is rounded; None where an operator on the CSR tensors has to
         serve the call (``WeightForm::product`` of csrc/host/torch_ops.cpp)."""
         return self._form.product(x, other, mode) if self._form is not None else None
+
+    def serve(self, values, row_offsets, column_indices, x, other, mode):
+        """:meth:`is_of` and :meth:`product` in one call: False where the form is not of these tensors as they are."""
+        return None if self.is_of(values, row_offsets, column_indices) else False   # (of a weight of which there is no form)
 
 
 def carry_pattern_note(column_indices, copy):
