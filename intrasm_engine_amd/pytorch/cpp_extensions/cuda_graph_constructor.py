@@ -24,13 +24,15 @@ class TorchCUDAGraphConstructor:
         self.notifier = iex.CUDAGraphCaptureNotifier()
         self.constructor = iex.CUDAExperimentalGraphConstructor()
         self.constructor.register_stream(self.registeredStreams[0].handle)
-        self._kept: list[torch.Tensor] = []
+        self._kept: dict[int, torch.Tensor] = {}   # by their memory
 
     def keep(self, *tensors: torch.Tensor) -> None:
         """What recorded kernels read at every replay lives as long as the constructor: copies, transposes and gathered
         values are made outside the capture, and the allocator would hand their memory to the next allocation while the
-        graph still reads it.  (Detached: a kept tensor must not keep the autograd node that keeps the constructor.)"""
-        self._kept.extend(t.detach() for t in tensors)
+        graph still reads it.  (Detached: a kept tensor must not keep the autograd node that keeps the constructor.  Once per
+        memory: weights and patterns are the same in every recording.)"""
+        for t in tensors:
+            self._kept.setdefault(t.untyped_storage()._cdata, t.detach())
 
     def get_primary_stream(self) -> CompoundStream:
         """The first stream: where streams join and where the graph is executed."""

@@ -139,6 +139,19 @@ def test_recorded_kernels_keep_what_they_read(dev, index):
     bwd.destroy_graph_exec()
 
 
+def test_a_weight_recorded_again_is_kept_once(dev):
+    constructor = TorchCUDAGraphConstructor()
+    x, w = torch.randn(192, 64, device=dev).half(), torch.randn(80, 64, device=dev).half().requires_grad_()
+    with constructor.get_primary_stream():
+        for step in range(3):
+            constructor.keep(x[:64 * (step + 1)], w)
+            assert len(constructor._kept) == 2
+    constructor.keep(x.clone())
+    assert len(constructor._kept) == 3
+    assert not any(t.requires_grad for t in constructor._kept.values())
+    assert {t.data_ptr() for t in constructor._kept.values()} >= {x.data_ptr(), w.data_ptr()}
+
+
 def test_triple_node(dev):
     case, other = _Case(dev, seed=5), _Case(dev, seed=6)
     want_out, want_grads = case.one_by_one()
