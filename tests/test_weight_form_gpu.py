@@ -118,6 +118,53 @@ def test_values_that_mark_an_empty_place_and_infinities(dev):
         assert torch.allclose(out[~with_nan][:, others].double(), want, rtol=1e-2, atol=1e-1)
 
 
+@pytest.mark.parametrize("dtype,idtype", [(torch.float16, torch.int16), (torch.bfloat16, torch.int32)])
+@pytest.mark.parametrize("m,k,n,kind", [(1024, 4096, 8192, 128), (1536, 4096, 6144, 192), (2048, 4096, 6144, 256)])
+def test_a_weight_with_spill_kept_and_captured(dev, dtype, idtype, m, k, n, kind):
+    """A two-of-four weight some of whose groups hold more: kept, laid out by every replay, and after values and columns were written in place so
+    that every row spills half of its entries."""
+    rng = np.random.default_rng(kind)
+    mask = _two_four(rng, m, k) | (rng.random((m, k)) < 5e-4)
+    mask[5] = False
+    ro_np = np.concatenate([[0], np.cumsum(mask.sum(1))]).astype(np.int32)
+    csr = W.CSR(m, k, rng.standard_normal(ro_np[-1]).astype(np.float32), W.swizzle_from_offsets(ro_np), ro_np, np.nonzero(mask)[1].astype(np.int32))
+    _, v, ro, ci = to_dev(csr, dev, dtype, idtype)
+    x = torch.randn(k, n, device=dev, generator=torch.Generator(dev).manual_seed(kind)).to(dtype)
+    rows = torch.repeat_interleave(torch.arange(m, device=dev), (ro[1:] - ro[:-1]).long())
+
+    def close(out):
+        a = torch.zeros(m, k, device=dev)
+        a[rows, ci.long()] = v.float()
+        want, scale = a.double() @ x.double(), a.abs() @ x.float().abs()
+        # the result's rounding, and at most k roundings of a sum in fp32, each 2^-24 of the magnitudes
+        return bool(((out.double() - want).abs() <= (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8) * want.abs() + k * 2.0 ** -24 * scale).all())
+
+    form = pyops.WeightForm(v, ro, ci, m, k)
+    kept = form.product(x)
+    assert f"two_four_kernel<{'f16' if dtype == torch.float16 else 'bf16'}> ({kind} x" in _lib.last_kernels()
+    assert close(kept)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        replayed = form.product(x)
+    assert f"({kind} x" in _lib.last_kernels()
+    for _ in range(3):
+        replayed.zero_()
+        graph.replay()
+        assert torch.equal(replayed, kept) and torch.equal(form.product(x), kept)
+    lens = np.diff(ro_np)
+    first = rng.integers(0, k - lens + 1)                    # every row's entries side by side, from some column on
+    ci.copy_(torch.from_numpy(np.concatenate([np.arange(f, f + c) for f, c in zip(first, lens)])).to(dev))
+    v.mul_(-0.5)
+    assert not form.is_of(v, ro, ci) and form.serve(v, ro, ci, x, None, 0) is False
+    for _ in range(3):
+        replayed.zero_()
+        graph.replay()
+        assert close(replayed)
+    again = pyops.WeightForm(v, ro, ci, m, k)
+    out = again.product(x)
+    assert out is None or close(out)
+
+
 def _layer(dev, hidden=256, mlp=512, seed=0, **options):
     rng = np.random.default_rng(seed)
     weights = {}
