@@ -27,7 +27,8 @@ int launch_one(const SpmmParams& p, int batch, hipStream_t stream) {
   dim3 grid(ceil_div(p.m, kRowsPerBlock), ceil_div(p.n, NT * LPG * VEC), batch);
   dim3 block(kWavesPerBlock * kWave);
   // Several nonzeros per gather and rows of at most 128 on average, more of them than are resident: windows of four gathers
-  // instead of eight.  Fewer registers (63 instead of 94, 8 wavefronts per SIMD instead of 5), and a short share is mostly
+  // instead of eight.  Fewer registers (n = 64 62 instead of 82 in fp32, n = 128 62 instead of 94 in fp16: 8 wavefronts per SIMD instead of 5; n = 128
+  // in fp32 72 instead of 98, 7 instead of 4), and a short share is mostly
   // its last, partial window.  MI355X, us, eight / four: 11008 x 1000, 90 / 95 % sparse, fp32 n = 64 21 / 16 and 21 / 13, n =
   // 128 32 / 25 and 25 / 19, fp16 n = 128 25 / 21 and 25 / 17, n = 256 - and 30 / 24.  Longer rows want the gathers in
   // flight (4096 x 4096, 90 %, fp16 n = 128 22 / 26, fp32 n = 64 22 / 27), few rows leave the registers idle (1024 x 1024, 95 %, fp16 n
@@ -625,12 +626,16 @@ int mfma_f32_variant(const SpmmParams& p, int batch, const Choice& ch) {
   int arrangement = tiles_m * ceil_div(p.n, 128) * batch >= 200 ? 4 : (p.n <= 64 ? 5 : 6);
   if (ch.nt) arrangement = ch.nt;
   if (ch.variant == 5) return arrangement;
-  // Measured on MI355X: 70-105 dense-equivalent TFLOP/s (the fp32 MFMA rate is 153; fp32 MFMAs
-  // run on the vector ALUs, so the expansion's instructions add to their time instead of hiding
-  // behind them).  That beats the gather kernels from 25-30 % density (4096 x 4096 at 50 %,
-  // n = 8192: 5.0 -> 2.9 ms; at 30 %, n = 1024: 0.69 -> 0.38 ms; at 30 %, n = 256: 0.19 -> 0.13 ms),
-  // ties at 20 % and loses below (11008 x 4096 at 20 %: 6.6 vs 7.3 ms).  The 16-row arrangements
-  // for small outputs stay on request: at 30 % and n = 128 they only tie (0.096 vs 0.100 ms).
+  // MI355X, us, matrix cores / the faster gather kernel, 4096 x 4096:
+  //   rows of geometric lengths  n = 128       n = 256       n = 512       n = 1024      n = 2048     of one length  n = 128   n = 256   n = 1024   n = 2048
+  //   10 %                       73 / 42       105 / 69      188 / 307     373 / 460     724 / 778                   53 / 33   86 / 60   340 / 227  677 / 415
+  //   20 %                       72 / 61       113 / 114     195 / 325     386 / 638     747 / 1225                  52 / 61   86 / 117  340 / 388  677 / 668
+  //   25 %                       74 / 77       113 / 140     200 / 341     386 / 768     750 / 1440                  53 / 72   87 / 140  340 / 451  677 / 790
+  //   30 %                       75 / 93       112 / 165     201 / 363     388 / 829     753 / 1623                  53 / 87   88 / 171  341 / 518  677 / 921
+  //   (11008 x 4096, n = 1024: 10 % 951 / 711, 20 % 991 / 1207, 30 % 1023 / 1750; of one length 931 / 611, 934 / 1016, 933 / 1380)
+  // The limit is that of an expansion that took 6 - 20 % longer and tied at 20 %; today's is ahead from there on, and with rows of
+  // geometric lengths and 512 columns from 10 %.  What a lower limit costs beside that: explicit zeros, which carry non-finite entries of rows of the dense
+  // operand that no nonzero references into the output.  The 16-row arrangements (n = 128 here) stay on request.
   const double fill = (double)p.n / ((double)ceil_div(p.n, 128) * 128);  // share of the computed columns that exist
   if (density >= 0.27 && arrangement == 4 && fill >= 0.75) return arrangement;
   // Beside a kernel that is bound by gathers the tie at 20 % goes to the matrix cores, also with the 16-row tiles of
