@@ -13,6 +13,8 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPEvent.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -175,6 +177,14 @@ void use_tables(const Tensor& tables, int64_t tables_stream, const Tensor& colum
 }
 
 // ---- operands that fit -------------------------------------------------------------------------------------------
+// Whether a call may pass the dispatcher by: no tensor that wraps another (vmap, jvp, functionalize, a subclass with a dispatch of its own),
+// and nobody who follows the operators called (a dispatch mode, a tracer).
+bool unwatched(const Tensor& t) {
+  using K = c10::DispatchKey;
+  constexpr c10::DispatchKeySet wrappers({K::Python, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Functionalize});
+  return t.has_storage() && !t.key_set().has_any(wrappers) && !c10::impl::TorchDispatchModeTLS::any_modes_set() && !c10::impl::tls_is_dispatch_key_included(K::Tracer);
+}
+
 bool plain(const Tensor& t, int64_t dim) { return t.is_cuda() && t.layout() == at::kStrided && t.dim() == dim && t.is_contiguous(); }
 
 bool plain_csr(const Tensor& row_indices, const Tensor& row_offsets, const Tensor& column_indices, const Tensor& with, int64_t m) {
@@ -434,7 +444,7 @@ struct WeightForm {
   // the kind of form that serves the call, -1: none; `captured` is looked up where it matters
   int kind_for(const Tensor& x, const std::optional<Tensor>& other, bool& captured) const {
     const int64_t n = x.dim() == 2 ? x.size(1) : 0;
-    if (forced || !plain(x, 2) || x.size(0) != k || n == 0 || n % 8 || k * n >= (1ll << 31) || m * n >= (1ll << 31) || dtype_code(x.scalar_type()) != dtype ||
+    if (forced || !unwatched(x) || (other && !unwatched(*other)) || !plain(x, 2) || x.size(0) != k || n == 0 || n % 8 || k * n >= (1ll << 31) || m * n >= (1ll << 31) || dtype_code(x.scalar_type()) != dtype ||
         x.device() != values.device() || reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 ||
         (at::GradMode::is_enabled() && (x.requires_grad() || (other && other->requires_grad()))))
       return -1;

@@ -5,6 +5,7 @@ import ctypes
 import numpy as np
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from intrasm_engine_amd import _iex_host, _lib
 from intrasm_engine_amd import workloads as W
@@ -203,15 +204,37 @@ def test_layer_by_forms_follows_its_weights(dev):
         assert torch.equal(out, layer.forward(x, 2))
 
 
-def _by_operators(layer, x):
+def _by_operators(layer, x, call=None):
     with pyops.kernel_params(gemm={"tile": 13}):
-        return layer.forward(x, 2)
+        return layer.forward(x, 2) if call is None else call("q", x)
 
 
 def _follows(layer, x):
     """The layer's result is that of the operators on the weights as they are now, and another than before."""
     got, want = layer.forward(x, 2).float(), _by_operators(layer, x).float()
     return bool((got - want).norm() < 2e-3 * want.norm())
+
+
+def test_projections_where_the_dispatcher_is_followed(dev):
+    """A form serves calls past the dispatcher: not where a transform has wrapped the operand, or somebody follows the operators called."""
+    layer = _layer(dev)
+    xs = torch.randn(3, 256, 1024, device=dev).half()
+    want = torch.stack([_by_operators(layer, x, layer.proj) for x in xs])
+    assert layer._by_form("q", xs[0]) is not None
+    assert torch.equal(torch.vmap(lambda x: layer.proj("q", x))(xs), want)
+    assert torch.equal(torch.func.jvp(lambda x: layer.proj("q", x), (xs[0],), (xs[1],))[0], want[0])
+
+    class Names(TorchDispatchMode):
+        def __torch_dispatch__(self, function, types, args=(), kwargs=None):
+            seen.append(str(function))
+            return function(*args, **(kwargs or {}))
+
+    seen = []
+    with Names():
+        out = layer.proj("q", xs[0])
+    assert torch.equal(out, want[0]) and any("spmm_sputnik_reuse_weight_half" in name for name in seen)
+    traced = torch.jit.trace(lambda x: layer.proj("q", x), xs[0], check_trace=False)
+    assert torch.equal(traced(xs[1]), want[1])
 
 
 def test_layer_under_inference_mode_follows_its_weights(dev):
