@@ -399,6 +399,7 @@ struct WeightForm {
     Tensor memory;
     at::cuda::CUDAEvent ready;
     int64_t made_on = -1;   // the stream whose memory it is
+    uint64_t of = 0;        // the generation of the values that are laid out
   };
   int dtype;
   int64_t m, k, nonzeros;
@@ -406,32 +407,41 @@ struct WeightForm {
   std::mutex layouts_mutex;
   std::array<int, 3> phases, rooms;
   int kinds;                       // a bit for each that the weight can be laid out as
-  Tensor values, row_offsets, column_indices;
-  std::array<int64_t, 3> versions;   // of the three, when the form was made for them
+  Tensor row_offsets, column_indices;
+  std::array<int64_t, 2> pattern_versions;   // when the form was made for them
+  // the values, their version, how many there were before; for copies only, so that it may be waited for with the interpreter's lock in hand
+  mutable std::mutex values_mutex;
+  Tensor values;
+  int64_t values_version;
+  uint64_t generation = 1;
 
   WeightForm(const Tensor& values, const Tensor& row_offsets, const Tensor& column_indices, const std::array<int64_t, 3>& versions, int64_t m, int64_t k, int kinds,
              const std::vector<int>& measured)
-      : dtype(dtype_code(values.scalar_type())), m(m), k(k), nonzeros(column_indices.numel()), kinds(kinds), values(values), row_offsets(row_offsets), column_indices(column_indices),
-        versions(versions) {
+      : dtype(dtype_code(values.scalar_type())), m(m), k(k), nonzeros(column_indices.numel()), kinds(kinds), row_offsets(row_offsets), column_indices(column_indices),
+        pattern_versions{versions[1], versions[2]}, values(values), values_version(versions[0]) {
     TORCH_CHECK(measured.size() == 6, "WeightForm: six numbers");
     std::copy_n(measured.begin(), 3, phases.begin());
     std::copy_n(measured.begin() + 3, 3, rooms.begin());
   }
 
-  // whether these are the tensors it was made for, unchanged since (never of tensors that count no changes)
+  static bool unchanged(const Tensor& mine, const Tensor& given, int64_t version) { return given.is_same(mine) && !given.is_inference() && given._version() == version; }
+  bool is_of_pattern(const Tensor& offsets, const Tensor& columns) const {
+    return unchanged(row_offsets, offsets, pattern_versions[0]) && unchanged(column_indices, columns, pattern_versions[1]);
+  }
+  // whether these are its tensors, unchanged since (never of tensors that count no changes)
   bool is_of(const Tensor& v, const Tensor& offsets, const Tensor& columns) const {
-    auto same = [](const Tensor& mine, const Tensor& given, int64_t version) { return given.is_same(mine) && !given.is_inference() && given._version() == version; };
-    return same(values, v, versions[0]) && same(row_offsets, offsets, versions[1]) && same(column_indices, columns, versions[2]);
+    std::lock_guard lock(values_mutex);
+    return unchanged(values, v, values_version) && is_of_pattern(offsets, columns);
   }
 
   int laid_out() {   // a bit for each kind that is
-    std::lock_guard lock(layouts_mutex);
+    std::scoped_lock lock(layouts_mutex, values_mutex);
     int bits = 0;
-    for (int i = 0; i < 4; ++i) bits |= layouts[i].memory.defined() << i;
+    for (int i = 0; i < 4; ++i) bits |= (layouts[i].memory.defined() && layouts[i].of == generation) << i;
     return bits;
   }
 
-  Tensor lay_out(int kind, int room, const Tensor& like) const {
+  Tensor lay_out(int kind, int room, const Tensor& values, const Tensor& like) const {
     Tensor form = workspace(iex_form_bytes(kind, m, k, room), like);
     const Tensor scratch = workspace(kind ? iex_form_scratch_bytes(m, k) : 0, like);
     check(iex_form_build(column_indices.scalar_type() == at::kShort ? IEX_I16 : IEX_I32, kind, m, k, nonzeros, row_offsets.const_data_ptr<int>(),
@@ -445,7 +455,7 @@ struct WeightForm {
   int kind_for(const Tensor& x, const std::optional<Tensor>& other, bool& captured) const {
     const int64_t n = x.dim() == 2 ? x.size(1) : 0;
     if (forced || !unwatched(x) || (other && !unwatched(*other)) || !plain(x, 2) || x.size(0) != k || n == 0 || n % 8 || k * n >= (1ll << 31) || m * n >= (1ll << 31) || dtype_code(x.scalar_type()) != dtype ||
-        x.device() != values.device() || reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 ||
+        x.device() != row_offsets.device() || reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 16 ||
         (at::GradMode::is_enabled() && (x.requires_grad() || (other && other->requires_grad()))))
       return -1;
     if (other && (!plain(*other, 2) || other->size(0) != m || other->size(1) != n || other->scalar_type() != x.scalar_type() || other->device() != x.device())) return -1;
@@ -457,9 +467,26 @@ struct WeightForm {
     return captured ? each_call : kept;
   }
 
-  // None: an operator on the CSR arrays serves the call.  False: the form is not of these tensors as they are now.
+  // Takes values that were changed, or others, of the same pattern; the next product lays them out.  (Captured: the caller sees to it.)
+  bool renew(const Tensor& v, const Tensor& offsets, const Tensor& columns) {
+    if (v.is_inference() || !unwatched(v) || !plain(v, 1) || v.numel() != nonzeros || dtype_code(v.scalar_type()) != dtype || v.device() != row_offsets.device() ||
+        !is_of_pattern(offsets, columns))
+      return false;
+    {
+      const c10::DeviceGuard guard(v.device());
+      if (capturing()) return false;
+    }
+    Tensor taken = v;
+    std::lock_guard lock(values_mutex);
+    std::swap(values, taken);   // (what goes is released without the lock)
+    values_version = v._version();
+    ++generation;
+    return true;
+  }
+
+  // None: an operator on the CSR arrays serves the call.  False: the form is not of this pattern as it is now.
   py::object serve(const Tensor& v, const Tensor& offsets, const Tensor& columns, const Tensor& x, const std::optional<Tensor>& other, int mode) {
-    if (!is_of(v, offsets, columns)) return py::bool_(false);
+    if (!is_of(v, offsets, columns) && !renew(v, offsets, columns)) return py::bool_(false);
     bool captured;
     const int kind = kind_for(x, other, captured);
     return kind < 0 ? py::object(py::none()) : py::cast(product_by(kind, captured, x, other, mode));
@@ -471,21 +498,29 @@ struct WeightForm {
     return kind < 0 ? std::nullopt : std::optional<Tensor>(product_by(kind, captured, x, other, mode));
   }
 
-  Tensor product_by(int kind, bool captured, const Tensor& x, const std::optional<Tensor>& other, int mode) {
+  Tensor product_by(int kind, bool captured, const Tensor& x, const std::optional<Tensor>& aux, int mode) {
     const py::gil_scoped_release nobody_waits_for_layouts_mutex_with_it;
     const c10::DeviceGuard guard(x.device());
     const int64_t n = x.size(1);
     int room = kind ? rooms[kind / 64 - 2] : 0;
-    Tensor form;
+    Tensor form, v;
+    uint64_t now;
+    {
+      std::lock_guard lock(values_mutex);
+      v = values, now = generation;
+    }
     if (captured) {
       room = kind ? kAnyRoom : 0;   // (the pattern of a later replay may spill more)
-      form = lay_out(kind, room, x);
+      form = lay_out(kind, room, v, x);
     } else {
       std::lock_guard lock(layouts_mutex);
       Layout& layout = layouts[kind ? kind / 64 - 1 : 0];
       const auto stream = at::cuda::getCurrentHIPStreamMasqueradingAsCUDA(x.get_device());
-      if (!layout.memory.defined()) {
-        const Tensor made = lay_out(kind, room, x);
+      if (!layout.memory.defined() || layout.of != now) {
+        for (Layout& other : layouts)
+          if (other.of != now) other.memory = Tensor();
+        const Tensor made = lay_out(kind, room, v, x);
+        layout.of = now;
         layout.ready.record(stream);
         layout.made_on = c10::hip::getCurrentHIPStream(x.get_device()).id();
         layout.memory = made;
@@ -498,7 +533,7 @@ struct WeightForm {
     const size_t ws_bytes = iex_form_product_workspace_bytes(kind, m, k, n);
     const Tensor ws = workspace(ws_bytes, x);
     Tensor out = at::empty({m, n}, x.options());
-    check(iex_form_product(dtype, kind, m, k, n, room, form.const_data_ptr(), x.const_data_ptr(), other ? other->const_data_ptr() : nullptr, mode,
+    check(iex_form_product(dtype, kind, m, k, n, room, form.const_data_ptr(), x.const_data_ptr(), aux ? aux->const_data_ptr() : nullptr, mode,
                            out.data_ptr(), ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, stream_of(x)),
           "form product");
     return out;

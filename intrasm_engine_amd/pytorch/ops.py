@@ -417,12 +417,15 @@ class WeightForm:
             return
         measured = _form_counts(row_offsets, column_indices, m, k)
         self._form = _iex_host.WeightForm(values, row_offsets, column_indices, self._versions, m, k, 15 if measured else 1, measured or [0] * 6)
+        self._tensors = None                # (the form has them, and takes others)
         # (asked by every product of a layer: without a Python frame around it)
         self.serve = self._form.serve
 
     def is_of(self, values, row_offsets, column_indices) -> bool:
-        """Whether these are the tensors that were laid out, unchanged since.  Never of tensors that count no changes (made under
+        """Whether these are the tensors that the form is of, unchanged since.  Never of tensors that count no changes (made under
         ``torch.inference_mode()``)."""
+        if self._form is not None:
+            return self._form.is_of(values, row_offsets, column_indices)
         return all(a is b and not b.is_inference() and _version(b) == v
                    for a, b, v in zip(self._tensors, (values, row_offsets, column_indices), self._versions))
 
@@ -432,7 +435,8 @@ class WeightForm:
         return self._form.product(x, other, mode) if self._form is not None else None
 
     def serve(self, values, row_offsets, column_indices, x, other, mode):
-        """:meth:`is_of` and :meth:`product` in one call: False where the form is not of these tensors as they are."""
+        """:meth:`product` of these tensors, of which the form takes changed or other values of its pattern (not under stream capture, nor ones that
+        count no changes).  False where it is not of them."""
         return None if self.is_of(values, row_offsets, column_indices) else False   # (of a weight of which there is no form)
 
 
