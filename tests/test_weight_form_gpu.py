@@ -1,6 +1,7 @@
 """A sparse 16-bit weight laid out once (dense form, two-of-four form with spilled entries) and multiplied by what was laid out: every
 kind at the edges of tiles, phases and spill blocks, against the oracle; when a form may stand for the CSR arrays."""
 import ctypes
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -340,6 +341,39 @@ def test_a_form_is_laid_out_by_the_first_product_that_takes_it(dev):
         torch.cuda.set_sync_debug_mode("default")
     torch.cuda.synchronize()
     assert torch.equal(first, want) and torch.equal(second, want)
+
+
+def test_a_form_takes_other_values_of_its_pattern(dev):
+    """Changed in place or other tensors, in turn and from two threads; nothing else is taken."""
+    layer = _layer(dev)
+    _, v, ro, ci, m = layer.w["gate"]
+    form = pyops.WeightForm(v, ro, ci, m, 256)
+    x = torch.randn(256, 1024, device=dev).half()
+    weights = [v, v * 2, v * -0.5]
+    want = [pyops.WeightForm(w, ro, ci, m, 256).product(x) for w in weights]
+    for i in (1, 2, 0, 0, 1):
+        assert torch.equal(form.serve(weights[i], ro, ci, x, None, 0), want[i]) and form.is_of(weights[i], ro, ci)
+    v.mul_(2)                                    # (and back: exact)
+    assert torch.equal(form.serve(v, ro, ci, x, None, 0), want[1])
+    v.mul_(0.5)
+    other = v.clone()
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        assert form.serve(other, ro, ci, x, None, 0) is False
+    with torch.inference_mode():
+        assert form.serve(v.clone(), ro, ci, x, None, 0) is False
+    assert form.serve(v[1:], ro, ci, x, None, 0) is False and form.serve(v.bfloat16(), ro, ci, x, None, 0) is False
+    assert form.serve(v, ro.clone(), ci, x, None, 0) is False and form.serve(v, ro, ci.clone(), x, None, 0) is False
+    assert torch.equal(form.serve(v, ro, ci, x, None, 0), want[0])
+
+    def many(stream):
+        with torch.cuda.stream(stream):
+            return [form.serve(v, ro, ci, x, None, 0) for _ in range(50)]
+
+    torch.cuda.synchronize()
+    with ThreadPoolExecutor(2) as pool:
+        outs = [out for outs in pool.map(many, (torch.cuda.Stream(), torch.cuda.Stream())) for out in outs]
+    torch.cuda.synchronize()
+    assert len(outs) == 100 and all(torch.equal(out, want[0]) for out in outs)
 
 
 def test_forms_are_refused_on_the_host(dev):
