@@ -133,7 +133,8 @@ int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream);
 #define IEX_SPMM_BESIDE_GATHER_KERNEL 0x40
 /* iex_spmm_ws and its workspace queries: the dense-form path (IEX_SPMM_FORCE_VARIANT(7), and where it is chosen) also
  * serves k, n and dense operands that are no whole 16-byte vectors, by copying the dense operand into the workspace with
- * zeros around it where it has to; the size asked for then holds that copy.  16-bit values shared by the batch. */
+ * zeros around it where it has to; the size asked for then holds that copy.  16-bit values shared by the batch.  In fp32 the
+ * product by parts (family 12), which works on copies of both operands, is open to calls with this flag only. */
 #define IEX_SPMM_PAD_OPERANDS 0x80
 /* bits 8..15: force waves-per-row (1, 4 or 8); 0 = choose from nnz/m.  For tuning.    */
 #define IEX_SPMM_FORCE_WPR(w) (((w) & 0xff) << 8)
@@ -158,6 +159,12 @@ int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream);
  * as dense: 0 = built in (1536), 1 = every block, 255 = none, else 64 * value); fails on other shapes.
  * 0 = choose.
  * 11 = the row kernel with wavefronts per row by the row's own length (iex_spmm_sched only: see there).
+ * 12 = fp32 by parts: every entry of A's dense form and of the dense operand as three bf16 parts that hold all its 24 bits, the
+ * six products of parts that reach into an fp32 result on the bf16 matrix cores (iex_spmm_ws only; chosen by itself for
+ * large fp32 products with IEX_SPMM_PAD_OPERANDS, values shared by the batch, plain store, canonical CSR).  Its error against 64 bits is below that of a chain of
+ * fp32 multiply-adds.  Where an operand holds an infinity or a NaN, or its entries are too large or small for the parts to be exact
+ * (largest magnitude outside 2^-90 .. 2^125, product of both outside 2^-80 .. 2^90), the row kernel computes the call instead;
+ * beside larger ones, entries below 2^-110 keep fewer bits.  Where it cannot run (no workspace, other types) the row kernel does.
  * Families 2-6 and 10 rely on strictly ascending column indices inside a row (canonical CSR, what
  * dense_to_sparse produces); family 1 accepts any order and duplicates -- force it for such
  * input.  Families 3-6 and 10 multiply explicit zeros with the dense operand, so a non-finite entry
@@ -198,6 +205,8 @@ int iex_spmm_ex(int dtype, int itype, int flags, int m, int k, int n, int nonzer
  * behind the dense form rounded up to 256 bytes, the room the GEMM wants for splitting k over several workgroups per
  * tile; a 16-byte aligned workspace of m * k * 2 bytes still runs the path, without the split.
  * IEX_SPMM_FORCE_VARIANT(7) asks for that path and fails where it cannot run.
+ * Large fp32 products with IEX_SPMM_PAD_OPERANDS run by parts (family 12), with a 256-byte aligned workspace for the parts of both operands and of k:
+ * 6 bytes a cell of A (m * k, k rounded up to 32) and an entry of the dense operand, and 4 per part of k and output.
  * iex_spmm_workspace_bytes returns the size with which the call described would use the workspace,
  * 0 when it would not whatever the size.  Neither call allocates.
  * No counterpart in the reference: its launchers (csrc/extensions.h:28-30) take no workspace. */

@@ -1,0 +1,298 @@
+// Host side of the fp32 product by three bf16 parts, and the kernels that make the parts and pick sampled entries.
+#include <algorithm>
+#include "gemm_split_device.cuh"
+
+namespace iex {
+namespace {
+
+// ---- parts --------------------------------------------------------------------------------------------------------
+// Two neighbours' parts, packed (the first in the lower half): each part rounded to nearest of what the ones before left,
+// which is exact in fp32.
+struct PartsPair {
+  unsigned high, middle, low;
+};
+__device__ __forceinline__ PartsPair parts_of(float x, float y) {
+  PartsPair r;
+  r.high = pack_pair<true>(x, y);
+  const float x1 = x - __uint_as_float(r.high << 16), y1 = y - __uint_as_float(r.high & 0xffff0000u);
+  r.middle = pack_pair<true>(x1, y1);
+  r.low = pack_pair<true>(x1 - __uint_as_float(r.middle << 16), y1 - __uint_as_float(r.middle & 0xffff0000u));
+  return r;
+}
+
+// eight neighbours to 16 bytes of each plane
+__device__ __forceinline__ void store_parts(const float (&x)[8], uint16_t* dst, long long plane) {
+  u32x4 h, m, l;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const PartsPair p = parts_of(x[2 * e], x[2 * e + 1]);
+    h[e] = p.high, m[e] = p.middle, l[e] = p.low;
+  }
+  *reinterpret_cast<u32x4*>(dst) = h;
+  *reinterpret_cast<u32x4*>(dst + plane) = m;
+  *reinterpret_cast<u32x4*>(dst + 2 * plane) = l;
+}
+
+__device__ __forceinline__ unsigned magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
+__device__ __forceinline__ unsigned wave_largest(unsigned x) {
+#pragma unroll
+  for (int d = 32; d; d >>= 1) x = max(x, (unsigned)__shfl_xor((int)x, d));
+  return x;
+}
+
+template <int WAVES>
+__device__ __forceinline__ void leave_largest(unsigned x, unsigned* at) {
+  __shared__ unsigned most[WAVES];
+  x = wave_largest(x);
+  if (lane_id() == 0) most[threadIdx.x >> 6] = x;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) x = max(x, most[w]);
+    *at = x;
+  }
+}
+
+__device__ __forceinline__ unsigned split_dense_block(const SplitDense& s, int block, int blocks) {
+  struct alignas(4) Any { float v[8]; };
+  const int chunks = s.dst_cols / 8;
+  const long long total = (long long)s.batch * s.dst_rows * chunks;
+  unsigned largest = 0;
+  for (long long i = (long long)block * 256 + threadIdx.x; i < total; i += (long long)blocks * 256) {
+    const long long zr = i / chunks;
+    const int c = (int)(i - zr * chunks) * 8;
+    const int z = (int)(zr / s.dst_rows), r = (int)(zr - (long long)z * s.dst_rows);
+    float x[8];
+    const float* src = s.src + ((size_t)z * s.rows + r) * s.cols + c;
+    if (r < s.rows && c + 8 <= s.cols) {
+      const Any a = *reinterpret_cast<const Any*>(src);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = a.v[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = r < s.rows && c + e < s.cols ? src[e] : 0.f;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) largest = max(largest, magnitude(x[e]));
+    store_parts(x, static_cast<uint16_t*>(s.dst) + (size_t)z * s.dst_batch + (size_t)r * s.ld + c, s.plane);
+  }
+  return largest;
+}
+
+// As csr_to_dense_kernel (spmm_dense_device.cuh): four wavefronts per pair of rows, a row (or 2048 columns of it) assembled in LDS in fp32, its
+// parts taken on the way out, every byte written once.
+constexpr int kPlanesSeg = 2048, kPlanesRows = 2, kPlanesWaves = 4;
+__device__ __forceinline__ unsigned split_sparse_block(const SplitSparse& s, int block, int blocks) {
+  __shared__ __align__(16) float srow[kPlanesRows][kPlanesSeg];
+  const int lane = lane_id(), wave = uniform(threadIdx.x >> 6);
+  const int* __restrict__ cols = s.cols;
+  const float* __restrict__ values = s.values;
+  uint16_t* __restrict__ dst = static_cast<uint16_t*>(s.dst);
+  unsigned most = 0;
+  bool again = false;
+  for (int slot0 = block * kPlanesRows; slot0 < s.m; slot0 += blocks * kPlanesRows) {
+    int pos[kPlanesRows], end[kPlanesRows];   // this wavefront's quarter of each row's nonzeros, in whole chunks of 64
+#pragma unroll
+    for (int r = 0; r < kPlanesRows; ++r) {
+      const int row = min(slot0 + r, s.m - 1);
+      const int first = uniform(s.row_offsets[row]), last = slot0 + r < s.m ? uniform(s.row_offsets[row + 1]) : first;
+      const int share = ((max(last - first, 0) + kWave * kPlanesWaves - 1) / (kWave * kPlanesWaves)) * kWave;
+      pos[r] = min(first + wave * share, last);
+      end[r] = min(pos[r] + share, last);
+    }
+    for (int c0 = 0; c0 < s.ld; c0 += kPlanesSeg) {
+      const int len = min(kPlanesSeg, s.ld - c0);   // a multiple of 32
+      if (again) __syncthreads();   // the previous segment has been copied out
+      again = true;
+#pragma unroll
+      for (int r = 0; r < kPlanesRows; ++r)
+        for (int i = threadIdx.x * 4; i < len; i += kPlanesWaves * kWave * 4) *reinterpret_cast<f32x4*>(srow[r] + i) = f32x4{0.f, 0.f, 0.f, 0.f};
+      __syncthreads();
+      bool more[kPlanesRows];
+#pragma unroll
+      for (int r = 0; r < kPlanesRows; ++r) more[r] = pos[r] < end[r];
+      static_assert(kPlanesRows == 2, "the loop below names both rows");
+      while (more[0] || more[1]) {
+        int c[kPlanesRows][4];
+        float v[kPlanesRows][4];
+#pragma unroll
+        for (int r = 0; r < kPlanesRows; ++r)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int j = max(min(pos[r] + u * kWave + lane, end[r] - 1), 0);   // (a row without nonzeros: entry 0, never used)
+            c[r][u] = cols[j] - c0;
+            v[r][u] = values[j];
+          }
+#pragma unroll
+        for (int r = 0; r < kPlanesRows; ++r) {
+          int taken = 0;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            // (the test on c keeps a row whose columns do not ascend inside the row's slice of LDS)
+            const bool mine = more[r] && pos[r] + u * kWave + lane < end[r] && c[r][u] < len && c[r][u] >= 0;
+            if (mine) {
+              srow[r][c[r][u]] = v[r][u];
+              most = max(most, magnitude(v[r][u]));
+            }
+            taken += __popcll(__ballot(mine));
+          }
+          pos[r] += taken;
+          more[r] = taken == 4 * kWave;   // a short take: the quarter ended or its next nonzero lies beyond this segment
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < kPlanesRows; ++r)
+        if (slot0 + r < s.m)
+          for (int i = threadIdx.x * 8; i < len; i += kPlanesWaves * kWave * 8) {
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(srow[r] + i), hi = *reinterpret_cast<const f32x4*>(srow[r] + i + 4);
+            const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            store_parts(x, dst + (size_t)(slot0 + r) * s.ld + c0 + i, s.plane);
+          }
+    }
+  }
+  return most;
+}
+
+// Both operands' parts in one launch: the first workgroups make those of the second operand.  Bound by the bytes, 4 read and 6 written an entry, 6
+// written a cell of a sparse operand.  (A maximum per workgroup, not atomics: 8192 of them on 64 words took 25 us.)
+template <typename First>
+__global__ __launch_bounds__(256) void split_operands_kernel(First a, SplitDense b, unsigned* largest, int blocks_b) {
+  if ((int)blockIdx.x < blocks_b) {
+    leave_largest<4>(split_dense_block(b, blockIdx.x, blocks_b), largest + blockIdx.x);
+  } else {
+    const int block = blockIdx.x - blocks_b, blocks = gridDim.x - blocks_b;
+    unsigned most;
+    if constexpr (std::is_same<First, SplitSparse>::value) most = split_sparse_block(a, block, blocks);
+    else most = split_dense_block(a, block, blocks);
+    leave_largest<4>(most, largest + kSplitSlots + block);
+  }
+}
+
+// A wavefront per row.  A score that is not finite (an infinity's parts give NaN) is computed as the dot product itself, by
+// the whole wavefront, and so are all where the operands' largest entries say that parts may have left fp32's normal range.
+__global__ __launch_bounds__(256) void split_sample_kernel(SplitSample s) {
+  const int row = blockIdx.x * 4 + uniform(threadIdx.x >> 6), lane = lane_id();
+  if (row >= s.m) return;
+  const int start = s.row_offsets[row], end = s.row_offsets[row + 1];
+  unsigned of_a = 0, of_b = 0;
+  for (int i = lane; i < kSplitSlots; i += kWave) {
+    if (i < s.slots_a) of_a = max(of_a, s.largest[kSplitSlots + i]);
+    if (i < s.slots_b) of_b = max(of_b, s.largest[i]);
+  }
+  of_a = wave_largest(of_a), of_b = wave_largest(of_b);
+  const bool all = max(of_a, of_b) < 0x7f800000u && !split_range_ok(of_a, of_b);   // (wave-uniform)
+  const float* scores = s.scores + (size_t)row * s.ld;
+  for (int j0 = start; j0 < end; j0 += kWave) {
+    const int j = min(j0 + lane, end - 1), col = s.cols[j];
+    float x = scores[col];
+    for (int part = 1; part < s.parts; ++part) x += scores[(size_t)part * s.stride_part + col];
+    const unsigned size = magnitude(x);
+    unsigned long long odd = __ballot(j0 + lane < end && (all || size >= 0x7f800000u));
+    while (odd) {
+      const int src = __ffsll(odd) - 1;
+      odd &= odd - 1;
+      const int c = bcast_i(col, src);
+      float sum = 0.f;
+      for (int z = 0; z < s.batch; ++z) {
+        const float* l = s.lhs + ((size_t)z * s.m + row) * s.k;
+        const float* r = s.rhs + ((size_t)z * s.n + c) * s.k;
+        for (int i = lane; i < s.k; i += kWave) sum = fmaf(l[i], r[i], sum);
+      }
+      sum = wave_sum(sum);
+      if (lane == src) x = sum;
+    }
+    if (j0 + lane < end) s.out[j] = x;
+  }
+}
+
+// ---- product ------------------------------------------------------------------------------------------------------
+constexpr int kSplitTile = 128, kSplitStages = 3, kSplitFlush = 16;
+
+template <bool TRANS_B>
+__global__ __launch_bounds__(256, 1) void gemm_split_kernel(SplitParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int b = blockIdx.x;
+  const int part = (b >> 3) % p.parts, slot = ((b >> 3) / p.parts) * kXcds + (b & 7);   // (a tile's parts on one XCD)
+  int tile_m, tile_n;
+  if (!xcd_tile(slot, p.tiles_m, p.tiles_n, tile_m, tile_n)) return;   // uniform per block
+  gemm_split_tile<TRANS_B, 2, 2, kSplitStages, kSplitFlush>(p, tile_m, tile_n, blockIdx.y, part, smem);
+}
+
+// Rounds of workgroups times the steps of each, plus what a workgroup takes besides (8 steps) and the sums of the parts.
+double split_steps(int M, int N, int K, int batch, int parts) {
+  const double tiles = (double)ceil_div(M, kSplitTile) * ceil_div(N, kSplitTile) * batch;
+  return std::ceil(tiles * parts / 256.0) * (ceil_div(K / 32, parts) + 8) + (parts > 1 ? 1 + (parts + 1.0) * M * N * batch * 4 / 4e12 / 1.1e-6 : 0);
+}
+
+template <bool TRANS_B>
+int launch_product(const SplitParams& p, int batch, hipStream_t stream) {
+  auto kern = gemm_split_kernel<TRANS_B>;
+  constexpr int lds = gemm_split_lds_bytes<2, 2, kSplitStages>();
+  static thread_local bool raised = false;   // per instantiation
+  if (!raised) {
+    if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds), "hipFuncSetAttribute(LDS size)"))
+      return rc;
+    raised = true;
+  }
+  const int per_xcd = ceil_div((long long)p.tiles_m * p.tiles_n, kXcds);
+  note_kernel("gemm_split_kernel<%s> (fp32 by three bf16 parts, %d x %d tiles, K in %d parts)", TRANS_B ? "B(N,K)" : "B(K,N)", kSplitTile, kSplitTile, p.parts);
+  hipLaunchKernelGGL(kern, dim3(per_xcd * kXcds * p.parts, batch), dim3(256), lds, stream, p);
+  return check_hip(hipGetLastError(), "gemm (fp32 by parts) launch");
+}
+
+template <typename First>
+int launch_operands(const First& a, int blocks_a, const SplitDense& b, unsigned* largest, hipStream_t stream) {
+  const int blocks_b = split_dense_blocks(b);
+  note_kernel("split_operands_kernel");
+  hipLaunchKernelGGL(split_operands_kernel<First>, dim3(blocks_a + blocks_b), dim3(256), 0, stream, a, b, largest, blocks_b);
+  return check_hip(hipGetLastError(), "parts of the operands, launch");
+}
+
+}  // namespace
+
+int gemm_split_parts(int M, int N, int K, int batch) {
+  const int steps = K / 32;
+  int best = 1;
+  for (int parts = 2; parts <= 8; ++parts) {
+    const int per = ceil_div(steps, parts);
+    if (per < 4 || (parts - 1) * per >= steps) continue;   // (every part has a step)
+    if ((double)parts * M * N * batch * 4 > 256e6) continue;
+    if (split_steps(M, N, K, batch, parts) < split_steps(M, N, K, batch, best)) best = parts;
+  }
+  return best;
+}
+double gemm_split_seconds(int M, int N, int K, int batch) {
+  const int parts = gemm_split_parts(M, N, K, batch);
+  return 1.1e-6 * std::ceil((double)ceil_div(M, kSplitTile) * ceil_div(N, kSplitTile) * batch * parts / 256.0) * (ceil_div(K / 32, parts) + 8);
+}
+
+int gemm_split(const SplitParams& given, bool trans_b, int batch, hipStream_t stream) {
+  SplitParams p = given;
+  p.tiles_m = ceil_div(p.M, kSplitTile);
+  p.tiles_n = ceil_div(p.N, kSplitTile);
+  p.parts = gemm_split_parts(p.M, p.N, p.K, batch);
+  IEX_REQUIRE(p.K > 0 && p.K % 32 == 0 && p.lda % 8 == 0 && p.ldb % 8 == 0 && (p.parts == 1 || (p.stride_part > 0 && !p.row_bias && !p.relu)), IEX_ERR_STATE,
+              "gemm (fp32 by parts): K=%d in %d parts, strides %d and %d", p.K, p.parts, p.lda, p.ldb);
+  return trans_b ? launch_product<true>(p, batch, stream) : launch_product<false>(p, batch, stream);
+}
+
+int split_dense_blocks(const SplitDense& s) {
+  const long long chunks = (long long)s.batch * s.dst_rows * (s.dst_cols / 8);
+  return (int)std::min<long long>(kSplitSlots, (chunks + 255) / 256);
+}
+int split_sparse_blocks(const SplitSparse& s) { return std::min(kSplitSparseSlots, ceil_div(s.m, kPlanesRows)); }
+int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* largest, hipStream_t stream) {
+  return launch_operands(a, split_sparse_blocks(a), b, largest, stream);
+}
+int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* largest, hipStream_t stream) {
+  return launch_operands(a, split_dense_blocks(a), b, largest, stream);
+}
+int launch_split_sample(const SplitSample& s, hipStream_t stream) {
+  note_kernel("split_sample_kernel");
+  hipLaunchKernelGGL(split_sample_kernel, dim3(ceil_div(s.m, 4)), dim3(256), 0, stream, s);
+  return check_hip(hipGetLastError(), "sampling launch");
+}
+
+}  // namespace iex

@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include "gemm_split.h"
 #include "spmm_dense_device.cuh"
 #include "spmm_lds_device.cuh"
 #include "spmm_mfma2_device.cuh"
@@ -769,6 +770,141 @@ int launch_dense_path(const SpmmParams& p, int batch, const Choice& ch, hipStrea
   return gemm_dispatch(dtype, 0, g, batch, stream, split_ws, with_split ? split : 0, with_split);
 }
 
+// ---- fp32 by parts: the dense form of A and B as three bf16 planes each, then their product on the bf16 matrix cores (gemm_split_device.cuh) ----
+struct SplitPlan {
+  int kp, np, parts, ld;   // ld: rows of the parts' sums
+  size_t a_at, b_at, sums_at, bytes;
+};
+// the workspace: the operands' largest magnitudes, planes of A, planes of B, sums of the parts of K
+inline SplitPlan split_plan(const SpmmParams& p, int batch) {
+  SplitPlan s;
+  s.kp = round32(p.k);
+  s.np = round8(p.n);
+  s.parts = gemm_split_parts(p.m, p.n, s.kp, batch);
+  s.ld = (p.n + 3) & ~3;
+  s.a_at = (kSplitSlots + kSplitSparseSlots) * 4;
+  s.b_at = s.a_at + round256((size_t)p.m * s.kp * 6);
+  s.sums_at = s.b_at + round256((size_t)batch * s.kp * s.np * 6);
+  s.bytes = s.sums_at + (s.parts > 1 ? (size_t)s.parts * batch * p.m * s.ld * 4 : 0);
+  return s;
+}
+// (canonical CSR; an operand's copies in the workspace, which is the caller's to allow; planes within a buffer's 4 GB; a vector of four columns for
+// the kernel behind it)
+inline bool split_path_fits(const SpmmParams& p) {
+  return p.pad && p.nnz > 0 && p.k > 0 && p.n >= 4 && !p.accumulate && !p.per_batch_values && (long long)p.m * round32(p.k) * 6 < (1ll << 32) &&
+         (long long)round32(p.k) * round8(p.n) * 6 < (1ll << 32);
+}
+
+// Whether that is the faster way, from a time model fitted on MI355X: three launches, the planes' bytes at 4.4 TB/s, the product
+// (gemm_split_seconds), the parts' sums at 4 TB/s; the row kernel gathers whole tiles of 256 columns at up to 30 TB/s, the fp32 matrix-core kernel
+// multiplies at 92 TFLOP/s.
+inline double split_path_seconds(const SpmmParams& p, int batch) {
+  const int kp = round32(p.k), parts = gemm_split_parts(p.m, p.n, kp, batch);
+  const double planes = 3.5e-6 + (6.0 * p.m * kp + 10.0 * batch * p.k * p.n) / 4.4e12;
+  return planes + gemm_split_seconds(p.m, p.n, kp, batch) + 4e-6 + (parts > 1 ? 4.0 * (parts + 1) * p.m * p.n * batch / 4e12 : 0.0);
+}
+inline bool split_path_wins(const SpmmParams& p, int batch) {
+  // Row kernel: whole tiles of 256 columns (narrow ones to the next power of two) at 30 TB/s, 25 where a tile's slice of B outgrows an XCD's L2.
+  // Rows of geometric lengths run at half of that with more than 256 columns, which the shape does not tell: the limit is that of even rows.
+  // MI355X, us, the kernels before / this way, at either side of the line: 4096 x 4096, even rows, n = 512, 80 % 218 / 112, 90 % 115 / 108, 95 % 62 / 104;
+  // n = 256, geometric, 80 % 114 / 80, 90 % 66 / 75; n = 128, 70 % 98 / 70, 80 % 60 / 65; 1656 x 1504, n = 640, 82 % 44 / 42; 2071 x 1694, n = 216,
+  // 72 % 36 / 47; 1408 x 10744, n = 513, 92 % 243 / 131; 11008 x 4096 and most of 200 drawn shapes in profiles/spmm_fp32_by_parts.txt.
+  int narrow = 32;
+  while (narrow < p.n) narrow *= 2;
+  const double columns = p.n <= 256 ? std::min(narrow, 256) : ceil_div(p.n, 256) * 256;
+  const double gather = 5e-6 + (double)p.nnz * columns * batch * 4 / (p.k > 4352 ? 25e12 : 30e12);
+  if (gather < 30e-6) return false;   // (what three launches and a short product take)
+  // Up to 256 columns the fp32 matrix-core kernel keeps the calls that its density rule gives it, although they are shorter this way (4096 x 4096, n = 256, 70 %
+  // 116 / 86): whoever looks at the names of the kernels finds that one there.
+  if (p.n <= 256 && mfma_f32_variant<float, int>(p, batch, Choice{})) return false;
+  return 1.1 * split_path_seconds(p, batch) < gather;
+}
+
+// Behind the product: adds the parts of K up (bias, ReLU), or where an operand holds an infinity or a NaN, which a product of parts (and of the
+// dense form's zeros) spreads, or lies outside the range in which parts hold all 24 bits, computes it once more as the row kernel does:
+// results there are the row kernel's.  With K in one part it ends at once else (2 us).
+constexpr int kFinishBlocks = 1024;
+__global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, const unsigned* largest, int slots_a, int slots_b, const float* sums, int parts, int ld,
+                                                               int tiles, int batch) {
+  __shared__ float red[spmm_lds_floats<4, 4, 1>()];
+  __shared__ unsigned most[2][4];
+  unsigned of_a = 0, of_b = 0;
+  for (int i = threadIdx.x; i < slots_b; i += 256) of_b = max(of_b, largest[i]);
+  for (int i = threadIdx.x; i < slots_a; i += 256) of_a = max(of_a, largest[kSplitSlots + i]);
+#pragma unroll
+  for (int d = 32; d; d >>= 1) {
+    of_b = max(of_b, (unsigned)__shfl_xor((int)of_b, d));
+    of_a = max(of_a, (unsigned)__shfl_xor((int)of_a, d));
+  }
+  if (lane_id() == 0) most[0][threadIdx.x >> 6] = of_a, most[1][threadIdx.x >> 6] = of_b;
+  __syncthreads();
+  of_a = max(max(most[0][0], most[0][1]), max(most[0][2], most[0][3]));
+  of_b = max(max(most[1][0], most[1][1]), max(most[1][2], most[1][3]));
+  if (!split_range_ok(of_a, of_b)) {
+    const long long total = (long long)p.m * tiles * batch;
+    for (long long i = blockIdx.x; i < total; i += gridDim.x) {
+      const int row = (int)(i % p.m), rest = (int)(i / p.m);
+      spmm_block<float, int, 4, kWave, 4, kSpmmUnroll, 1, true>(p, row, rest % tiles, rest / tiles, red);
+      __syncthreads();
+    }
+  } else if (parts > 1) {
+    typedef float four __attribute__((ext_vector_type(4)));
+    typedef four any4 __attribute__((aligned(4)));
+    const int chunks = ld / 4;
+    const size_t rows = (size_t)p.m * batch, part = rows * ld;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < rows * chunks; i += (size_t)gridDim.x * 256) {
+      const size_t zr = i / chunks;
+      const int c = (int)(i - zr * chunks) * 4;
+      const float* from = sums + zr * ld + c;
+      four x = *reinterpret_cast<const four*>(from);
+      for (int s = 1; s < parts; ++s) x += *reinterpret_cast<const four*>(from + s * part);
+      if (p.bias) x += p.bias[zr % p.m];
+      if (p.relu) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = fmaxf(x[e], 0.f);
+      }
+      float* out = static_cast<float*>(p.out) + zr * p.n + c;
+      if (c + 4 <= p.n) {
+        *reinterpret_cast<any4*>(out) = x;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < p.n) out[e] = x[e];
+      }
+    }
+  }
+}
+
+inline int launch_split_path(const SpmmParams& p, int batch, void* workspace, hipStream_t stream) {
+  const SplitPlan s = split_plan(p, batch);
+  unsigned char* ws = static_cast<unsigned char*>(workspace);
+  unsigned* largest = reinterpret_cast<unsigned*>(ws);
+  float* sums = reinterpret_cast<float*>(ws + s.sums_at);
+  const long long plane_a = (long long)p.m * s.kp, plane_b = (long long)s.kp * s.np;
+  const SplitSparse a{p.m, s.kp, p.row_offsets, static_cast<const int*>(p.cols), static_cast<const float*>(p.values), plane_a, ws + s.a_at};
+  const SplitDense b{batch, p.k, p.n, static_cast<const float*>(p.dense), s.kp, s.np, s.np, 3 * plane_b, plane_b, ws + s.b_at};
+  if (int rc = launch_split_operands(a, b, largest, stream)) return rc;
+  SplitParams g{};
+  g.M = p.m, g.N = p.n, g.K = s.kp;
+  g.A = ws + s.a_at, g.B = ws + s.b_at;
+  g.lda = s.kp, g.ldb = s.np;
+  g.plane_a = (unsigned)(plane_a * 2), g.plane_b = (unsigned)(plane_b * 2);
+  g.stride_b = 3 * plane_b;
+  if (s.parts > 1) {
+    g.C = sums, g.ldc = s.ld, g.stride_c = (long long)p.m * s.ld, g.stride_part = g.stride_c * batch;
+  } else {
+    g.C = static_cast<float*>(p.out), g.ldc = p.n, g.stride_c = (long long)p.m * p.n;
+    g.row_bias = p.bias, g.relu = p.relu;
+  }
+  if (int rc = gemm_split(g, false, batch, stream)) return rc;
+  note_kernel("spmm_split_finish_kernel");
+  const int tiles = ceil_div(p.n, kWave * 4);
+  const long long work = s.parts > 1 ? ((long long)p.m * batch * (s.ld / 4) + 255) / 256 : (long long)p.m * tiles * batch;
+  hipLaunchKernelGGL(spmm_split_finish_kernel, dim3((unsigned)std::min<long long>(s.parts > 1 ? kFinishBlocks : kFinishBlocks / 4, work)), dim3(256), 0, stream, p, largest,
+                     split_sparse_blocks(a), split_dense_blocks(b), sums, s.parts, s.ld, tiles, batch);
+  return check_hip(hipGetLastError(), "spmm (fp32 by parts) launch");
+}
+
 template <typename T, typename IT>
 int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_t stream) {
   constexpr int kMax = 16 / (int)sizeof(T);
@@ -790,6 +926,10 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
     return launch_smallk<T, IT>(p, batch, stream);
   }
   if constexpr (std::is_same<T, float>::value && std::is_same<IT, int>::value) {
+    const bool room = ch.ws && aligned(ch.ws, 256);
+    if ((ch.variant == 12 || (ch.variant == 0 && !ch.beside_gather)) && room && split_path_fits(p) && (ch.variant == 12 || split_path_wins(p, batch)) &&
+        ch.ws_bytes >= split_plan(p, batch).bytes)
+      return launch_split_path(p, batch, ch.ws, stream);
     if (const int arr = mfma_f32_variant<T, IT>(p, batch, ch)) {
       const bool split = ch.lpg != 8;   // (lanes-per-group code 8 = no role split, for tuning)
       // (a row's windows are the kernel's own affair; numbers that it never had are refused)
@@ -956,6 +1096,13 @@ static size_t workspace_plan(int dtype, int itype, int flags, int m, int k, int 
   const int variant = (flags >> 16) & 0xf;
   if (variant == 0 && (flags & IEX_SPMM_ANY_COLUMN_ORDER)) return 0;   // families 1 and 8 use no workspace
   void* const some_aligned = reinterpret_cast<void*>(size_t(256));
+  if (dtype == IEX_F32 && itype == IEX_I32 && (variant == 0 || variant == 12)) {
+    const SpmmParams p{m, k, n, nonzeros, nullptr, nullptr, nullptr, nullptr, some_aligned, nullptr, some_aligned,
+                       (flags & IEX_SPMM_PER_BATCH_VALUES) != 0, (flags & IEX_SPMM_ACCUMULATE) != 0, (flags & IEX_SPMM_RELU) != 0, (flags & IEX_SPMM_PAD_OPERANDS) != 0};
+    if (!split_path_fits(p) || (variant == 0 && ((flags & IEX_SPMM_BESIDE_GATHER_KERNEL) || !split_path_wins(p, batch)))) return 0;
+    *kind = 12;
+    return split_plan(p, batch).bytes;
+  }
   if (!(dtype == IEX_F16 || dtype == IEX_BF16) || !(itype == IEX_I32 || itype == IEX_I16)) return 0;
   if (variant != 0 && variant != 7 && variant != 10) return 0;
   SpmmParams p{m, k, n, nonzeros, nullptr, nullptr, nullptr, nullptr, some_aligned, nullptr, some_aligned,
@@ -1088,7 +1235,9 @@ int iex_spmm_static(int dtype, int itype, int flags, int m, int k, int n, int no
   // every call shares the array with whatever ran before it: nothing in it counts as "still there"
   flags &= ~(IEX_SPMM_TABLES_READY | IEX_SPMM_LISTS_READY);
   const size_t need = spmm_workspace_bytes(dtype, itype, flags, m, k, n, nonzeros, batch);
-  if (need == 0)  // a call that would not touch a workspace runs as iex_spmm_ex does (a forced family 7 fails there)
+  // a call that would not touch a workspace runs as iex_spmm_ex does (a forced family 7 fails there), and so does an fp32 one whose parts
+  // the array does not hold: the other families take none
+  if (need == 0 || (dtype == IEX_F32 && ((flags >> 16) & 0xf) == 0 && need > kStaticScratchBytes))
     return spmm_dispatch(dtype, itype, flags, m, k, n, nonzeros, row_indices, values, row_offsets, column_indices, dense,
                          bias, out, stream, batch, nullptr, 0);
   IEX_REQUIRE(need <= kStaticScratchBytes, IEX_ERR_TOO_LARGE,

@@ -3,7 +3,7 @@
 //   * lies inside its buffer and outside the operand's allocation -- a read the hardware would perform --, or
 //   * holds k < K of an existing row or column and does not come whole from where that element lies.
 // A buffer load performs the 4-byte words that end inside the buffer (scalar offset included) and delivers zeros for others.
-//   gemm_addresses_check M N K lda ldb layout(0 = B (K,N), 1 = B (N,K), 2 = A (K,M)) kb split(0 = none, -2 = halves, n = parts) [1: sizes as rows * stride]
+//   gemm_addresses_check M N K lda ldb layout(0 = B (K,N), 1 = B (N,K), 2 = A (K,M)) kb split(0 = none, -2 = halves, -3 = operands in three planes, n = parts) [1: sizes as rows * stride]
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -25,9 +25,10 @@ struct Walk {
   int first, count;      // the tile's first row or column, and how many exist
   int K, ld, step_k;     // of this part; k per step
   ll k_base;             // of the part's first k, in elements from the allocation's start (of row / column 0)
+  ll plane = 0;          // elements before the plane that is read (an operand in three planes)
 
   int chunk(DirectChunk c, int step, int lds_row, int lds_pos_first) const {
-    const ll soffset = rows_along_k ? (ll)step * step_k * 2 : (ll)step * step_k * ld * 2;
+    const ll soffset = plane * 2 + (rows_along_k ? (ll)step * step_k * 2 : (ll)step * step_k * ld * 2);
     const int k = step * step_k + c.k;
     const bool wanted = k < K && (rows_along_k ? first + lds_row < count : lds_pos_first < count);
     int words = 0;
@@ -44,7 +45,7 @@ struct Walk {
     ++checked;
     if (!wanted) return 0;
     const ll at = base + (soffset + c.offset) / 2;
-    const ll want = rows_along_k ? (ll)(first + lds_row) * ld + k_base + k : k_base + (ll)k * ld + lds_pos_first;
+    const ll want = plane + (rows_along_k ? (ll)(first + lds_row) * ld + k_base + k : k_base + (ll)k * ld + lds_pos_first);
     if (words != 4 || at != want) {
       std::printf("%s: step %d, row or column %d, k %d: element %lld (%d words) instead of %lld\n", what, step, rows_along_k ? first + lds_row : lds_pos_first, k,
                   at, words, want);
@@ -102,6 +103,21 @@ static int walk(int M, int N, int K, int lda, int ldb, int layout, int kb, int s
   return 0;
 }
 
+// The fp32 product by parts: 128 x 128 tiles, steps of 32 k, both operands in three planes; K a multiple of 32 (zeros where the operands end).
+static int walk_planes(int M, int N, int K, int lda, int ldb, int layout) {
+  const bool tb = layout == 1;
+  const ll plane_a = (ll)M * lda, plane_b = (ll)(tb ? N : K) * ldb;
+  for (int plane = 0; plane < 3; ++plane) {
+    for (int m0 = 0; m0 < M; m0 += 128)
+      if (walk_rows<32, 128>(Walk{"A", (ll)m0 * lda, 3 * plane_a, 4 * plane_a + (ll)rows_bytes(M - m0, K, lda), true, m0, M, K, lda, 32, 0, plane * plane_a})) return 1;
+    for (int n0 = 0; n0 < N; n0 += 128) {
+      const Walk w{"B", tb ? (ll)n0 * ldb : 0, 3 * plane_b, 4 * plane_b + (ll)(tb ? rows_bytes(N - n0, K, ldb) : rows_bytes(K, N, ldb)), tb, n0, N, K, ldb, 32, 0, plane * plane_b};
+      if (tb ? walk_rows<32, 128>(w) : walk_columns<128, 32>(w)) return 1;
+    }
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   if (argc < 9) return 2;
   int v[8];
@@ -109,7 +125,8 @@ int main(int argc, char** argv) {
   sizes_from_strides = argc > 9 && std::atoi(argv[9]);
   const int M = v[0], N = v[1], K = v[2], lda = v[3], ldb = v[4], layout = v[5], kb = v[6], split = v[7];
   int bad = 0;
-  if (split > 0) bad = walk<64, 128, 64, 64, 64>(M, N, K, lda, ldb, layout, kb, split);              // K in parts
+  if (split == -3) bad = walk_planes(M, N, K, lda, ldb, layout);                                       // fp32 by parts
+  else if (split > 0) bad = walk<64, 128, 64, 64, 64>(M, N, K, lda, ldb, layout, kb, split);              // K in parts
   else if (split == -2) bad = walk<256, 256, 32, 32, 32>(M, N, K, lda, ldb, layout, kb, split);      // K in halves
   else
     bad = walk<128, 128, 32, 32, 32>(M, N, K, lda, ldb, layout, kb, 0) || walk<64, 128, 64, 64, 64>(M, N, K, lda, ldb, layout, kb, 0) ||

@@ -25,6 +25,7 @@ CASES = [
     (300, 264, 72, 0, 0, 0, 0, -2), (257, 258, 104, 1, 0, 0, 0, -2), (300, 264, 72, 0, 8, 16, 0, -2),                # K in halves
     (1, 8, 8, 0, 0, 0, 0, 0), (1, 1, 8, 1, 0, 0, 0, 0), (8, 8, 1, 2, 0, 0, 0, 0), (131, 264, 72, 0, 0, 0, 7, 0),      # one workgroup per tile
     (131, 259, 200, 1, 0, 0, 0, 0), (131, 259, 200, 1, 8, 40, 0, 0), (131, 264, 200, 0, 8, 40, 0, 0), (136, 264, 33, 2, 0, 0, 0, 0),
+    (1, 8, 32, 0, 0, 0, 0, -3), (129, 136, 96, 0, 0, 0, 0, -3), (300, 264, 64, 0, 0, 0, 0, -3), (129, 131, 96, 1, 0, 0, 0, -3), (257, 1, 32, 1, 0, 0, 0, -3),   # three planes
     (45, 33, 70, 2, 3, 7, 0, 0),                                                                                     # ragged, rows padded to chunks
 ]
 
