@@ -373,6 +373,10 @@ int iex_sddmm_ex(int dtype, int flags, int m, int k, int n, int nonzeros,
  * gradients of a sparse linear layer: k = tokens).  Same arithmetic per output (fp32 accumulation,
  * one rounding).  Needs plain store, (batch, nnz) output or batch 1, k and n multiples of 8;
  * anything else, and a NULL or short workspace, runs exactly as iex_sddmm_ex.
+ * fp32 calls with IEX_SDDMM_PAD_OPERANDS, a plain store and one output (batch 1, or summed over the batch) do the same by parts (12, with a
+ * 256-byte aligned workspace): lhs and rhs as three bf16 parts of every entry, all products on the bf16 matrix cores (SpMM family 12 says what
+ * that does to accuracy); scores that are not finite, and all of them where the operands are too large or small for it, are
+ * computed as the dot products themselves.
  * The workspace also serves variant 3 above (short k, masks with structure), which 0 = choose picks first.
  * iex_sddmm_workspace_bytes returns the size with which the call described would use the
  * workspace, 0 when it would not whatever the size.  Neither call allocates.
@@ -383,7 +387,7 @@ int iex_sddmm_ws(int dtype, int flags, int m, int k, int n, int nonzeros,
                  void* stream, int batch, void* workspace, size_t workspace_bytes);
 size_t iex_sddmm_workspace_bytes(int dtype, int flags, int m, int k, int n, int nonzeros, int batch);
 /* What the workspace would hold: 0 = nothing (not used), 3 = the tables of variant 3 (a function of m, n
- * and the index arrays only: see IEX_SDDMM_TABLES_READY), 7 = the dense product. */
+ * and the index arrays only: see IEX_SDDMM_TABLES_READY), 7 = the dense product, 12 = the dense product by parts. */
 int iex_sddmm_workspace_kind(int dtype, int flags, int m, int k, int n, int nonzeros, int batch);
 
 /* The tables and lists that SDDMM variant 3 and SpMM family 10 derive from a pattern (m rows, n columns: the SpMM's k),

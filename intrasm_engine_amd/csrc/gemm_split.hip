@@ -80,9 +80,9 @@ __device__ __forceinline__ unsigned split_dense_block(const SplitDense& s, int b
   return largest;
 }
 
-// As csr_to_dense_kernel (spmm_dense_device.cuh): four wavefronts per pair of rows, a row (or 2048 columns of it) assembled in LDS in fp32, its
-// parts taken on the way out, every byte written once.
-constexpr int kPlanesSeg = 2048, kPlanesRows = 2, kPlanesWaves = 4;
+// As csr_to_dense_kernel (spmm_dense_device.cuh): a workgroup per row, the row (or 4096 columns of it) assembled in LDS in fp32, its parts taken on
+// the way out, every byte written once.  (4096 x 4096: 27 us, of which 20 are the bytes; two rows side by side the same, four 40.)
+constexpr int kPlanesSeg = 4096, kPlanesRows = 1, kPlanesWaves = 4;
 __device__ __forceinline__ unsigned split_sparse_block(const SplitSparse& s, int block, int blocks) {
   __shared__ __align__(16) float srow[kPlanesRows][kPlanesSeg];
   const int lane = lane_id(), wave = uniform(threadIdx.x >> 6);
@@ -109,11 +109,11 @@ __device__ __forceinline__ unsigned split_sparse_block(const SplitSparse& s, int
       for (int r = 0; r < kPlanesRows; ++r)
         for (int i = threadIdx.x * 4; i < len; i += kPlanesWaves * kWave * 4) *reinterpret_cast<f32x4*>(srow[r] + i) = f32x4{0.f, 0.f, 0.f, 0.f};
       __syncthreads();
-      bool more[kPlanesRows];
+      bool more[kPlanesRows], any = false;
 #pragma unroll
-      for (int r = 0; r < kPlanesRows; ++r) more[r] = pos[r] < end[r];
-      static_assert(kPlanesRows == 2, "the loop below names both rows");
-      while (more[0] || more[1]) {
+      for (int r = 0; r < kPlanesRows; ++r) any |= more[r] = pos[r] < end[r];
+      while (any) {
+        any = false;
         int c[kPlanesRows][4];
         float v[kPlanesRows][4];
 #pragma unroll
@@ -138,7 +138,7 @@ __device__ __forceinline__ unsigned split_sparse_block(const SplitSparse& s, int
             taken += __popcll(__ballot(mine));
           }
           pos[r] += taken;
-          more[r] = taken == 4 * kWave;   // a short take: the quarter ended or its next nonzero lies beyond this segment
+          any |= more[r] = taken == 4 * kWave;   // a short take: the quarter ended or its next nonzero lies beyond this segment
         }
       }
       __syncthreads();
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(256) void split_sample_kernel(SplitSample s) {
 }
 
 // ---- product ------------------------------------------------------------------------------------------------------
-constexpr int kSplitTile = 128, kSplitStages = 3, kSplitFlush = 16;
+constexpr int kSplitTile = 128, kSplitStages = 3, kSplitFlush = 8;
 
 template <bool TRANS_B>
 __global__ __launch_bounds__(256, 1) void gemm_split_kernel(SplitParams p) {
@@ -220,10 +220,13 @@ __global__ __launch_bounds__(256, 1) void gemm_split_kernel(SplitParams p) {
   gemm_split_tile<TRANS_B, 2, 2, kSplitStages, kSplitFlush>(p, tile_m, tile_n, blockIdx.y, part, smem);
 }
 
-// Rounds of workgroups times the steps of each, plus what a workgroup takes besides (8 steps) and the sums of the parts.
+// Rounds of workgroups (32 on an XCD at a time, which gets whole tiles: 81 tiles in three parts are 33 for one of them, a second round) times the steps
+// of each, plus what a workgroup takes besides (8 steps) and the sums of the parts.
+double split_rounds(int M, int N, int batch, int parts) {
+  return std::ceil((double)ceil_div((long long)ceil_div(M, kSplitTile) * ceil_div(N, kSplitTile), kXcds) * batch * parts / 32.0);
+}
 double split_steps(int M, int N, int K, int batch, int parts) {
-  const double tiles = (double)ceil_div(M, kSplitTile) * ceil_div(N, kSplitTile) * batch;
-  return std::ceil(tiles * parts / 256.0) * (ceil_div(K / 32, parts) + 8) + (parts > 1 ? 1 + (parts + 1.0) * M * N * batch * 4 / 4e12 / 1.1e-6 : 0);
+  return split_rounds(M, N, batch, parts) * (ceil_div(K / 32, parts) + 8) + (parts > 1 ? 1 + (parts + 1.0) * M * N * batch * 4 / 4e12 / 1.1e-6 : 0);
 }
 
 template <bool TRANS_B>
@@ -265,7 +268,7 @@ int gemm_split_parts(int M, int N, int K, int batch) {
 }
 double gemm_split_seconds(int M, int N, int K, int batch) {
   const int parts = gemm_split_parts(M, N, K, batch);
-  return 1.1e-6 * std::ceil((double)ceil_div(M, kSplitTile) * ceil_div(N, kSplitTile) * batch * parts / 256.0) * (ceil_div(K / 32, parts) + 8);
+  return 1.1e-6 * split_rounds(M, N, batch, parts) * (ceil_div(K / 32, parts) + 8);
 }
 
 int gemm_split(const SplitParams& given, bool trans_b, int batch, hipStream_t stream) {

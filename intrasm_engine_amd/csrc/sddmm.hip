@@ -18,6 +18,7 @@
 // the (nnz) output is a deterministic sum.
 #include <algorithm>
 #include <cmath>
+#include "gemm_split.h"
 #include "iex_common.h"
 #include "sddmm_mfma_device.cuh"
 #include "spmm_dense_device.cuh"
@@ -354,6 +355,60 @@ int launch_sddmm_dense(int dtype, const SddmmParams& p, void* ws, hipStream_t st
   return 0;
 }
 
+// ---- fp32: the dense product by three bf16 parts of every entry (gemm_split_device.cuh), then sampling ----
+// A sum over the batch is one product with the batch's k side by side.
+struct SddmmSplit {
+  int kp, K, ld, parts;   // k rounded up, of all batch entries; rows of scores; parts of K
+  size_t lhs_at, rhs_at, scores_at, bytes;
+};
+inline SddmmSplit sddmm_split_plan(const SddmmParams& p) {
+  SddmmSplit s;
+  s.kp = round32(p.k);
+  s.K = s.kp * p.batch;
+  s.ld = (p.n + 3) & ~3;
+  s.parts = gemm_split_parts(p.m, p.n, s.K, 1);
+  s.lhs_at = 2 * kSplitSlots * 4;
+  s.rhs_at = s.lhs_at + round256((size_t)p.m * s.K * 6);
+  s.scores_at = s.rhs_at + round256((size_t)p.n * s.K * 6);
+  s.bytes = s.scores_at + (size_t)s.parts * p.m * s.ld * 4;
+  return s;
+}
+// (copies of the operands, which are the caller's to allow; planes within a buffer's 4 GB)
+inline bool sddmm_split_fits(int dtype, const SddmmParams& p) {
+  return dtype == IEX_F32 && p.pad && !p.accumulate && (p.sum_over_batch || p.batch == 1) && p.k > 0 && p.n > 0 &&
+         (long long)std::max(p.m, p.n) * round32(p.k) * p.batch < (1ll << 32) / 6 && (long long)p.m * p.n < (1ll << 30);
+}
+// Time model fitted on MI355X: three launches, the planes' bytes at 4.4 TB/s, the product (gemm_split_seconds), the scores of all parts written and read
+// once at 4 TB/s; the gather kernel at 18 TB/s, 13.5 where rhs outgrows an XCD's L2.  Us, gather kernel / this way, at either side of
+// the line: 2160 x 1449, k = 221, 81 % 43 / 36; 3711 x 1112, k = 296, 86 % 38 / 52; 10680 x 3436, k = 179, 89 % 143 / 167; 8463 x 3904, k = 252, 88 % 229 / 191;
+// 4296 x 1093, k = 997, 95 % 73 / 102; 5176 x 1344, k = 1197, 86 % 305 / 127; 1560 x 2069, k = 1517, 97 % 52 / 83; 986 x 10230, k = 1049, 85 % 603 / 176.
+inline bool sddmm_split_wins(const SddmmParams& p) {
+  const double bytes = (double)p.nnz * p.k * p.batch * 4, gather = 4e-6 + bytes / ((double)p.n * p.k * 4 <= 4.5e6 ? 18e12 : 13.5e12);
+  if (gather < 28e-6) return false;   // (what three launches and a short product take)
+  const SddmmSplit s = sddmm_split_plan(p);
+  const double sample = 4.5e-6 + (4.0 * s.parts * p.m * s.ld + 8.0 * p.nnz) / 4e12;
+  return 1.1 * (3.5e-6 + 10.0 * ((double)p.m + p.n) * s.K / 4.4e12 + gemm_split_seconds(p.m, p.n, s.K, 1) + sample) < gather;
+}
+int launch_sddmm_split(const SddmmParams& p, void* workspace, hipStream_t stream) {
+  const SddmmSplit s = sddmm_split_plan(p);
+  unsigned char* ws = static_cast<unsigned char*>(workspace);
+  unsigned* largest = reinterpret_cast<unsigned*>(ws);
+  const long long plane_a = (long long)p.m * s.K, plane_b = (long long)p.n * s.K;
+  const SplitDense a{p.batch, p.m, p.k, static_cast<const float*>(p.lhs), p.m, s.kp, s.K, s.kp, plane_a, ws + s.lhs_at};
+  const SplitDense b{p.batch, p.n, p.k, static_cast<const float*>(p.rhs), p.n, s.kp, s.K, s.kp, plane_b, ws + s.rhs_at};
+  if (int rc = launch_split_operands(a, b, largest, stream)) return rc;
+  SplitParams g{};
+  g.M = p.m, g.N = p.n, g.K = s.K;
+  g.A = a.dst, g.B = b.dst, g.C = reinterpret_cast<float*>(ws + s.scores_at);
+  g.lda = g.ldb = s.K, g.ldc = s.ld;
+  g.plane_a = (unsigned)(plane_a * 2), g.plane_b = (unsigned)(plane_b * 2);
+  g.stride_part = (long long)p.m * s.ld;
+  if (int rc = gemm_split(g, true, 1, stream)) return rc;
+  const SplitSample q{p.m, p.k, p.n, p.batch, s.ld, s.parts, g.stride_part, p.row_offsets, p.cols, g.C, static_cast<const float*>(p.lhs), static_cast<const float*>(p.rhs),
+                      static_cast<float*>(p.out), largest, split_dense_blocks(a), split_dense_blocks(b)};
+  return launch_split_sample(q, stream);
+}
+
 // ---- score tiles on the matrix cores, sampled inside the workgroup (sddmm_mfma_device.cuh) ----
 // 16-bit types, k = 32, 64 or 128, plain store, one output per batch entry, canonical CSR (columns ascending and
 // distinct inside a row), n <= 128 * kSdMaxTiles; the workspace holds (6 ceil(n / 128) + 1) * m words (per row and
@@ -426,10 +481,12 @@ int launch_sddmm_mfma(int dtype, const SddmmParams& p, void* ws, int dense_code,
 int sddmm_workspace_kind(int dtype, int flags, int m, int k, int n, int nonzeros, int batch) {
   if (m <= 0 || k <= 0 || n <= 0 || nonzeros <= 0 || batch <= 0) return 0;
   const int variant = (flags >> 16) & 0xf;
-  if (variant != 0 && variant != 7 && variant != 3) return 0;
+  if (variant != 0 && variant != 7 && variant != 3 && variant != 12) return 0;
   void* const some_aligned = reinterpret_cast<void*>(size_t(256));
   SddmmParams p{m, k, n, nonzeros, batch, nullptr, nullptr, nullptr, some_aligned, some_aligned, nullptr,
                 (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0, (flags & IEX_SDDMM_PAD_OPERANDS) != 0};
+  if (dtype == IEX_F32 && variant != 3 && variant != 7) return sddmm_split_fits(dtype, p) && (variant == 12 || sddmm_split_wins(p)) ? 12 : 0;
+  if (variant == 12) return 0;
   const bool any_order = (flags & IEX_SDDMM_ANY_COLUMN_ORDER) != 0;
   if (variant != 7 && sddmm_mfma_fits(dtype, p) && (variant == 3 || (!any_order && sddmm_mfma_wins(p)))) return 3;
   if (variant == 3 || !sddmm_dense_fits(dtype, p)) return 0;
@@ -439,10 +496,12 @@ int sddmm_workspace_kind(int dtype, int flags, int m, int k, int n, int nonzeros
 size_t sddmm_workspace_bytes(int dtype, int flags, int m, int k, int n, int nonzeros, int batch) {
   if (m <= 0 || k <= 0 || n <= 0 || nonzeros <= 0 || batch <= 0) return 0;
   const int variant = (flags >> 16) & 0xf;
-  if (variant != 0 && variant != 7 && variant != 3) return 0;
+  if (variant != 0 && variant != 7 && variant != 3 && variant != 12) return 0;
   void* const some_aligned = reinterpret_cast<void*>(size_t(256));
   SddmmParams p{m, k, n, nonzeros, batch, nullptr, nullptr, nullptr, some_aligned, some_aligned, nullptr,
                 (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0, (flags & IEX_SDDMM_PAD_OPERANDS) != 0};
+  if (dtype == IEX_F32 && variant != 3 && variant != 7) return sddmm_split_fits(dtype, p) && (variant == 12 || sddmm_split_wins(p)) ? sddmm_split_plan(p).bytes : 0;
+  if (variant == 12) return 0;
   const bool any_order = (flags & IEX_SDDMM_ANY_COLUMN_ORDER) != 0;
   if (variant != 7 && sddmm_mfma_fits(dtype, p) && (variant == 3 || (!any_order && sddmm_mfma_wins(p)))) return sddmm_mfma_bytes(p);
   if (variant == 3) return 0;
@@ -469,7 +528,7 @@ int sddmm_dispatch(int dtype, int flags, int m, int k, int n, int nonzeros, cons
   int wpr = (flags >> 8) & 0xff;  // forced (1 or 4), else from the mean row length
   if (wpr != 1 && wpr != 4) wpr = ((double)nonzeros / m >= 64.0) ? 4 : 1;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int variant = (flags >> 16) & 0xf;  // 0 = choose, 1 = gather kernel, 3 = score tiles on the matrix cores, 7 = dense product then sampling
+  const int variant = (flags >> 16) & 0xf;  // 0 = choose, 1 = gather kernel, 3 = score tiles on the matrix cores, 7 = dense product then sampling, 12 = the same by parts
   const bool any_order = (flags & IEX_SDDMM_ANY_COLUMN_ORDER) != 0;   // (the tables of variant 3 assume ascending, distinct columns)
   if ((variant == 0 && !any_order) || variant == 3) {
     const bool fits = sddmm_mfma_fits(dtype, p);
@@ -490,6 +549,9 @@ int sddmm_dispatch(int dtype, int flags, int m, int k, int n, int nonzeros, cons
     }
     if (fits && room && (variant == 7 || sddmm_dense_wins(p))) return launch_sddmm_dense(dtype, p, workspace, s);
   }
+  if ((variant == 0 || variant == 12) && workspace && aligned(workspace, 256) && sddmm_split_fits(dtype, p) && (variant == 12 || sddmm_split_wins(p)) &&
+      workspace_bytes >= sddmm_split_plan(p).bytes)
+    return launch_sddmm_split(p, workspace, s);
   switch (dtype) {
     case IEX_F32: return launch_typed<float>(p, wpr, s);
     case IEX_F16: return launch_typed<__half>(p, wpr, s);
