@@ -311,6 +311,27 @@ int launch_rows(const SpmmParams& p, int batch, int lpg, const int* hist, int ro
   }
 }
 
+// Wavefronts per row of the kernel for narrow ragged rows (spmm_ragged.hip), 0 = a single nonzero per gather stays ahead: rows with few nonzeros leave it nothing to
+// share out, few rows nothing to fill the chip with.  Even rows by one wavefront each where there are many (the histogram tells: none longer than two to four
+// times the mean), rows of several hundred nonzeros and uneven ones by four.  MI355X, us, one nonzero per gather / one wavefront a row / four:
+//   even     9904 x 1000 at 97 %, n = 138 fp16, 31 a row 20.6 / 12.0 / 26.3;  5137 x 1040, n = 52, 97 a row 10.6 / 7.1 / 11.5;  10704 x 2846, n = 14, 302 43 / 20 / 27;
+//            fp32 8616 x 1800, n = 67, 365 84 / 57 / 60;  1064 x 3912, n = 177, 223 11.9 / 21.4 / 14.0;  752 x 792, n = 95, 82 4.8 / 5.7 / 5.0;  2558 x 1400, n = 31, 137 8.1 / 8.7 / 8.0
+//   uneven   1632 x 3347, n = 68, 418 29 / 41 / 16.5;  4248 x 800, n = 67, 89 15.8 / 21.9 / 12.7;  8768 x 3344, n = 12, 1000 87 / 64 / 50;  690 x 392, n = 246 fp32, 46 6.3 / 14.8 / 6.3
+inline int ragged_narrow_waves(const SpmmParams& p, int batch, const int* hist, int elem_size) {
+  const double mean = (double)p.nnz / std::max(p.m, 1), rows = (double)p.m * batch;
+  bool even = false;
+  if (hist) {
+    int j = 0;
+    while (j < 15 && (kWave << j) < 2 * mean) ++j;
+    even = hist[j] == 0;
+  }
+  if (elem_size == 2 && p.n % 2 != 0 && mean > 1000) return 0;   // (16-byte gathers at odd addresses: 4086 x 8048 at 71 %, n = 9 118 / - / 189)
+  if (even && mean >= 24 && rows >= 2700) return 1;
+  if (p.n > 256 / elem_size) return 0;   // (two nonzeros per gather: 568 x 2832 at 71 %, n = 137 fp16 21 / - / 31)
+  if (mean >= 250) return 4;
+  return hist && !even && mean >= 80 ? 4 : 0;
+}
+
 // ---- LDS-staged variant -----------------------------------------------------------------
 template <typename T, typename IT, int VEC, int RPW>
 __global__ __launch_bounds__(kLdsThreads, 4) void spmm_lds_kernel(SpmmParams p) {
@@ -812,7 +833,7 @@ inline bool split_path_wins(const SpmmParams& p, int batch) {
   int narrow = 32;
   while (narrow < p.n) narrow *= 2;
   const double columns = p.n <= 256 ? std::min(narrow, 256) : ceil_div(p.n, 256) * 256;
-  const double gather = 5e-6 + (double)p.nnz * columns * batch * 4 / (p.k > 4352 ? 25e12 : 30e12);
+  const double gather = 5e-6 + (double)p.nnz * columns * batch * 4 / ((double)p.k * std::min(p.n, 256) > 1.1e6 ? 25e12 : 30e12);
   if (gather < 30e-6) return false;   // (what three launches and a short product take)
   // Up to 256 columns the fp32 matrix-core kernel keeps the calls that its density rule gives it, although they are shorter this way (4096 x 4096, n = 256, 70 %
   // 116 / 86): whoever looks at the names of the kernels finds that one there.
@@ -998,6 +1019,11 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
   // the reference's ViT sweep shapes (fp32, batch 384, 97 % sparse): 785 x 785 outputs 865 -> 516 us,
   // 197 x 197 outputs 64 -> 33 us.
   if (p.n % kMax != 0 && p.n >= kWave * kMax / 2 && ch.lpg == 0) return launch_ragged<T, IT, kMax>(p, batch, wpr, stream);
+  // ... and narrower ones, several nonzeros per gather
+  if (p.n >= kMax && p.n < kWave * kMax / 2 && ch.lpg == 0 && nt == 1 && !ch.wpr_forced) {
+    if (const int waves = ragged_narrow_waves(p, batch, ch.hist, sizeof(T)))
+      return launch_spmm_ragged(std::is_same<T, float>::value ? IEX_F32 : std::is_same<T, __half>::value ? IEX_F16 : IEX_BF16, sizeof(IT) == 2 ? IEX_I16 : IEX_I32, p, batch, waves, stream);
+  }
   if constexpr (kMax == 8) {
     if (sh.vec == 4) return launch_wpr<T, IT, 4, 64>(p, batch, wpr, nt, stream);
   }

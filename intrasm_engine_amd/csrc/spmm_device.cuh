@@ -46,6 +46,9 @@ bool spmm_blocks_wins(const SpmmParams& p, int batch);
 size_t spmm_blocks_bytes(const SpmmParams& p);
 int launch_spmm_blocks(int dtype, const SpmmParams& p, int batch, void* ws, int dense_code, int ready, hipStream_t stream);
 
+// Narrow outputs whose rows are no whole 128-bit vectors (spmm_ragged.hip): n at least a vector and less than half of a wavefront's
+int launch_spmm_ragged(int dtype, int itype, const SpmmParams& p, int batch, int wpr, hipStream_t stream);
+
 constexpr int kSpmmUnroll = 8;
 
 template <int VEC, int WPR, int NT = 1>
@@ -268,7 +271,7 @@ __device__ __forceinline__ void spmm_store_row(const SpmmParams& p, int z, int r
 //       instead (shifted back by `shift`), sums all of them and stores only the ones it owns.
 template <typename T, typename IT, int VEC, int LPG, int WPR, int WIN = kSpmmUnroll, int NT = 1, bool RAGGED = false, bool TAIL = true>
 __device__ __forceinline__ void spmm_block(const SpmmParams& p, int bx, int by, int bz, float* red) {
-  static_assert(!RAGGED || (NT == 1 && LPG == kWave), "ragged rows: one full-width tile per wave");
+  static_assert(!RAGGED || NT == 1, "ragged rows: one tile per wave");
   constexpr int kWavesPerBlock = (WPR > 4) ? WPR : 4;
   constexpr int kRowsPerBlock = kWavesPerBlock / WPR;
   constexpr int G = kWave / LPG;
