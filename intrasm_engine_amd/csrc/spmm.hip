@@ -707,7 +707,7 @@ inline size_t dense_path_bytes(const SpmmParams& p, int batch) {
 //     matrix-core SpMM kernels at 1.2 TB/s (8 x 4096 x 4096, k = 128: 0.24 ms), the gather kernels write it at 4 TB/s, the few-columns kernel at 4.5 TB/s plus 10 clocks of a CU's LDS
 //     per nonzero and tile (same shape at 93 % sparsity: 0.15 ms; 8 x 4096 x 4096, k = 128 at 50 %: 0.58
 //     against 0.17 for the dense form).
-// The dense form has to win by 15 % to be taken.  `few_columns`: the alternative is the few-columns kernel.
+// The dense form has to win by 15 % to be taken, by 20 % with a copy of B.  `few_columns`: the alternative is the few-columns kernel.
 // split_room: the workspace has room for the GEMM to take k in parts where it would (few tiles, long k: the K loop of a
 // tile then runs on several CUs; 4096^2 at 70-90 %, n = 128 / 256: 40 / 41 -> 27 / 32 us).
 //   Wide rows are gathered in tiles of 512 columns, the last one as slow as the others (3449 x 8696 at 94 %, n = 552: 185
@@ -724,7 +724,21 @@ inline double other_families_seconds(const SpmmParams& p, int batch, int matrix_
     other = 8e-6 + std::max({flops / 720e12, chain, out_bytes / 1.2e12});
   } else {
     const double columns = p.n <= 256 ? p.n : ceil_div(p.n, 512) * 512;   // (whole tiles: a last tile of few columns costs like a full one)
-    other = 8e-6 + (double)p.nnz * columns * batch * 2 / 26e12 + out_bytes / 4e12;
+    double per_nonzero = columns * 2 / 26e12;
+    // Rows of no whole vectors: 16-byte gathers that start at multiples of 2, 4 or 8 bytes.  Us, gathers / dense form: 800 x 9672 at 91 %, n = 859 114 / 50;
+    // 1747 x 752 at 81 %, n = 406 13 / 16; 2783 x 3163 at 98 %, n = 1028 30 / 44; few rows of B stay in L1: 2472 x 389 at 84 %, n = 286 11 / 18.
+    const int vec = p.n % 4 == 0 ? 4 : p.n % 2 == 0 ? 2 : 1;
+    if (p.n % 8 != 0 && p.n >= 256) {
+      per_nonzero = columns * 2 / (p.k <= 512 || vec == 4 ? 26e12 : vec == 2 ? 22e12 : 13e12);
+    } else if (p.n % 8 != 0) {
+      // one nonzero per gather, 90 G of them a second (10680 x 3436 at 89 %, n = 179: 134 / 55), or several (ragged_narrow_waves; 9903 x 2825 at 88 %, n = 79:
+      // 94 / 37; 5043 x 4044 at 80 %, n = 26 24 / 38)
+      const double mean = (double)p.nnz / std::max(p.m, 1);
+      per_nonzero = std::max(ceil_div(p.n, kWave * vec) / 90e9, columns * 2 / 26e12);
+      if ((p.n <= 128 || (double)p.m * batch >= 2700) && (vec > 1 || mean <= 1000))
+        per_nonzero = std::min(per_nonzero, std::max(1 / (vec > 1 ? 150e9 : 80e9), columns * 2 / ((vec == 4 ? 18e12 : vec == 2 ? 12e12 : 6.5e12) * (p.k <= 512 ? 2 : 1))));
+    }
+    other = 8e-6 + (double)p.nnz * batch * per_nonzero + out_bytes / 4e12;
   }
   return other;
 }
@@ -736,7 +750,7 @@ inline bool dense_path_wins(const SpmmParams& p, int batch, int matrix_core_kind
   const double product = std::max({flops / 1000e12, std::ceil(tiles / 512.0) * (p.k / 32.0) * 0.23e-6 / parts, out_bytes / 3e12});
   const double pad = dense_path_pads(p) ? 4e-6 + 4.0 * p.k * p.n * batch / 4e12 : 0.0;
   const double dense_form = 8e-6 + cells * 2 / 4e12 + pad + product;
-  return 1.15 * dense_form < other_families_seconds(p, batch, matrix_core_kind, few_columns);
+  return (dense_path_pads(p) ? 1.2 : 1.15) * dense_form < other_families_seconds(p, batch, matrix_core_kind, few_columns);
 }
 
 // Behind dense form and copy (rounded up to 256 bytes) the workspace may hold what the GEMM wants for splitting K over two

@@ -62,3 +62,13 @@ def test_what_stays_with_one_nonzero_per_gather():
         assert "ragged_narrow" not in _lib.last_kernels()
         call(force_wpr=4)
         assert "ragged_narrow" not in _lib.last_kernels()
+
+
+@pytest.mark.parametrize("m,k,n,density,dense_form", [(1500, 4000, 315, 0.08, True), (1500, 300, 315, 0.08, False), (2000, 5000, 67, 0.1, True), (2600, 3100, 26, 0.18, False)])
+def test_rows_at_element_alignment_count_in_the_choice_of_the_dense_form(oracle, m, k, n, density, dense_form):
+    (values, row_indices, row_offsets, columns), b = operands(m, k, n, density, torch.float16)
+    got = torch.ops.iex_ops.spmm_sputnik_reuse_weight_half(b, row_indices, values, row_offsets, columns, m)
+    assert ("csr_to_dense" in _lib.last_kernels()) == dense_form, _lib.last_kernels()
+    v, ri, ro, ci = (t.float().cpu().numpy() if t.is_floating_point() else t.cpu().numpy() for t in (values, row_indices, row_offsets, columns))
+    x = b.float().cpu().numpy()
+    assert_close(got.float().cpu().numpy(), oracle.spmm(x, ri, v, ro, ci, m), oracle.spmm_abs_scale(x, ri, v, ro, ci, m), 1e-2, f"{m} x {k} x {n}")
