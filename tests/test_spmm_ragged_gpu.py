@@ -64,7 +64,7 @@ def test_what_stays_with_one_nonzero_per_gather():
         assert "ragged_narrow" not in _lib.last_kernels()
 
 
-@pytest.mark.parametrize("m,k,n,density,dense_form", [(1500, 4000, 315, 0.08, True), (1500, 300, 315, 0.08, False), (2000, 5000, 67, 0.1, True), (2600, 3100, 26, 0.18, False)])
+@pytest.mark.parametrize("m,k,n,density,dense_form", [(1500, 4000, 315, 0.15, True), (1500, 300, 315, 0.15, False), (2000, 5000, 67, 0.25, True), (2600, 3100, 26, 0.18, False)])
 def test_rows_at_element_alignment_count_in_the_choice_of_the_dense_form(oracle, m, k, n, density, dense_form):
     (values, row_indices, row_offsets, columns), b = operands(m, k, n, density, torch.float16)
     got = torch.ops.iex_ops.spmm_sputnik_reuse_weight_half(b, row_indices, values, row_offsets, columns, m)
