@@ -158,7 +158,8 @@ int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream);
  * IEX_SPMM_TABLES_READY / IEX_SPMM_LISTS_READY; bits 8..15 set the number of nonzeros from which a block counts
  * as dense: 0 = built in (1536), 1 = every block, 255 = none, else 64 * value); fails on other shapes.
  * 0 = choose.
- * 11 = the row kernel with wavefronts per row by the row's own length (iex_spmm_sched only: see there).
+ * 11 = the row kernel with wavefronts per row by the row's own length (iex_spmm_sched only: see there); with four waves per row
+ * forced too: a wavefront per row, four for rows of more than 64 << (code of bits 20..23 less one) nonzeros.
  * 12 = fp32 by parts: every entry of A's dense form and of the dense operand as three bf16 parts that hold all its 24 bits, the
  * six products of parts that reach into an fp32 result on the bf16 matrix cores (iex_spmm_ws only; chosen by itself for
  * large fp32 products with IEX_SPMM_PAD_OPERANDS, values shared by the batch, plain store, canonical CSR).  Its error against 64 bits is below that of a chain of
@@ -228,6 +229,8 @@ size_t iex_spmm_workspace_bytes(int dtype, int itype, int flags, int m, int k, i
  * summed completely, and to the same bits, whatever the histogram and whatever the order of row_indices: a wrong
  * histogram or another order costs time only.  IEX_SPMM_FORCE_VARIANT(11) asks for this kernel and fails without a histogram
  * (bits 20..23 then force the chunks of 64 nonzeros a wavefront may get: 1 + log2, 0 = choose).
+ * Where many rows fill the chip as it is, workgroups of four wavefronts serve one long row or four others each, n of no whole vectors too (family 11 with four
+ * waves per row forced), to the same promise.  With nothing forced the histogram settles which of these arrangements runs, or one number for all rows.
  * No counterpart in the reference. */
 int iex_spmm_sched(int dtype, int itype, int flags, int m, int k, int n, int nonzeros,
                    const int* row_indices, const void* values, const int* row_offsets,

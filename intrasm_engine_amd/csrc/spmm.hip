@@ -311,6 +311,81 @@ int launch_rows(const SpmmParams& p, int batch, int lpg, const int* hist, int ro
   }
 }
 
+// ---- ... by workgroups of four: a wavefront per row, four for the long ones ---------------------------------
+// Bound like the row kernel by the gathers' way from L2 into the CUs and, where rows are uneven, by the chain of the longest one.  A whole row per
+// wavefront needs no partial sums and lets the wavefronts of an XCD walk through the dense operand's rows together (2048 x 8192, even rows of 409,
+// n = 512 fp32: 125 us by four wavefronts a row, 68 by one); four for a long row shorten its chain without the cost for the others.
+// (Registers for four wavefronts per SIMD, six with full fp32 tiles: what a row by one wavefront has.)
+template <typename T, typename IT, int VEC, int LPG, bool RAGGED>
+__global__ __launch_bounds__(4 * kWave, LPG < kWave ? 4 : sizeof(T) == 2 ? 4 : 6) void spmm_rows_kernel4(SpmmParams p, LongRows lr) {
+  __shared__ float red[spmm_lds_floats<VEC, 4>()];
+  spmm_long_rows_block<T, IT, VEC, LPG, RAGGED>(p, lr, blockIdx.x, blockIdx.y, blockIdx.z, red);
+}
+
+template <typename T, typename IT, int LPG, bool RAGGED>
+int launch_long_rows_one(const SpmmParams& p, int batch, const LongRows& lr, hipStream_t stream) {
+  constexpr int kMax = 16 / (int)sizeof(T);
+  note_kernel("spmm_rows_kernel4<%s, %s, %d, %d, %s> (%d rows by four waves)", type_name<T>(), type_name<IT>(), kMax, LPG, RAGGED ? "true" : "false", lr.long_rows);
+  hipLaunchKernelGGL((spmm_rows_kernel4<T, IT, kMax, LPG, RAGGED>), dim3(lr.long_rows + ceil_div(p.m - lr.long_rows, 4), ceil_div(p.n, LPG * kMax), batch),
+                     dim3(4 * kWave), 0, stream, p, lr);
+  return check_hip(hipGetLastError(), "spmm (long rows) launch");
+}
+
+template <typename T, typename IT>
+int launch_long_rows(const SpmmParams& p, int batch, int lpg, bool ragged, const int* hist, int log2_chunks, hipStream_t stream) {
+  const LongRows lr{std::min(p.m, std::max(0, hist[log2_chunks])), kWave << log2_chunks};
+  if (ragged) return launch_long_rows_one<T, IT, kWave, true>(p, batch, lr, stream);
+  switch (lpg) {
+    case 8: return launch_long_rows_one<T, IT, 8, false>(p, batch, lr, stream);
+    case 16: return launch_long_rows_one<T, IT, 16, false>(p, batch, lr, stream);
+    case 32: return launch_long_rows_one<T, IT, 32, false>(p, batch, lr, stream);
+    default: return launch_long_rows_one<T, IT, kWave, false>(p, batch, lr, stream);
+  }
+}
+
+// How the wavefronts go to the rows of a pattern whose row lengths are known: log2(limit / 64) of the kernel above, or one of the names below
+// (kRowsAsBefore: by the mean alone, or by 16).  Even = no row longer than two to four times the mean.  MI355X, us, four wavefronts a row / one / the kernel above
+// at its limit (* = 16 wavefronts a workgroup, one chunk each):
+//  several nonzeros per gather, even: a row to a wavefront from 2000 rows up; long rows only where the workgroups fill whole rounds of the CUs (level)
+//   11008 x 4096 at 97 %, n = 64 fp16 20.8 / 11.6 / 11.9, fp32 18.2 / 17.7 / 15.9, at 90 % n = 128 fp32 82 / 79 / 78;  6000 x 3000 at 90 %, n = 128 41 / 34 / 36
+//   1024 x 2000 at 90 %, n = 128 fp32 7.3 / 8.9 / 8.3, 8.3*;  n = 256 fp16 8.0 / 9.1 / 8.6, 9.7*;  not level: 4552 x 3880 at 80 %, n = 80 fp16 39 / 44 / -
+//  ... uneven (geometric lengths)
+//   11008 x 4096 at 97 %, n = 64 fp16 20.8 / 14.5 / 12.0;  6000 x 3000 at 90 %, n = 32 fp16 16.4 / 31 / 12.9;  4096 x 4096 at 97 %, n = 128 fp32 16.2 / 32.5 / 14.3, 18.4*
+//   1024 x 2000 at 90 %, n = 128 fp32 16.3 / 45 / 15.3, 12.3*;  4096 x 4096 at 90 %, n = 64 fp32 21.6 / 53 / 22 - 24;  3752 x 416, 11 a row, n = 24 fp16 - / 5.2 / 5.4
+//  one nonzero per gather, even
+//   4096 x 4096 at 90 %, n = 256 fp32 61 / 60 / 60;  2000 x 4096 at 97 %, n = 512 26 / 24 / -;  4096 x 1000 at 97 %, n = 512 fp16 12.7 / 9.0 / -;  512 x 8192 at 95 %, n = 1024
+//   fp32 65 / 43 / -;  424 x 1104 at 93 %, n = 1540 15.3 / 16.1 / -;  not level: 4872 x 5176 at 97 %, n = 176 29 / 32 / -
+//  ... uneven
+//   4096 x 4096 at 95 %, n = 512 fp32 68 / 154 / 66, n = 2048 247 / 396 / 239;  98 %, n = 512 34 / 65 / 33, fp16 n = 2048 74 / 87 / 66;  10000 x 600 at 90 %, n = 256 25 / 30 / 23
+//   4096 x 4096 at 90 %, n = 256 fp32 68 / 168 / 67 - 75;  256 x 4096 at 90 %, n = 1024 136 / - / -, 57*;  512 x 1024 at 90 %, n = 512 16.2 / - / -, 11.7*;
+//   2048 x 1024 at 90 %, n = 256 15.6 / - / -, 18.1*;  1024 x 1024 at 90 %, n = 1024 fp16 19.4 / - / -, 21.6*
+// The limit grows with the rows, which are what a long row's chain hides behind.
+constexpr int kRowsAsBefore = -1, kRowsOneWave = -2, kRowsFourWaves = -3, kRowsSixteenWaves = -4;
+inline int rows_by_histogram(const SpmmParams& p, int batch, const int* hist, int elem_size, int lpg, int wpr) {
+  const double mean = (double)p.nnz / std::max(p.m, 1), rows = (double)p.m * batch;
+  int twice = 0;
+  while (twice < 15 && (kWave << twice) < 2 * mean) ++twice;
+  const bool even = hist[twice] <= 0;
+  const int tiles = ceil_div(p.n, lpg * 16 / elem_size);
+  const double groups = rows * tiles / (4 * 256);
+  const bool level = groups >= 0.96 * std::ceil(groups);
+  double ratio = 0.8 + rows / 4500;
+  if (lpg == kWave) {
+    if (even) return wpr == 4 && groups >= 1.9 && level && (rows >= 1900 || mean >= 250) ? kRowsOneWave : kRowsAsBefore;
+    if (mean < 24) return kRowsAsBefore;
+    if (wpr != 1 && !(elem_size == 2 && rows >= 4000 && mean <= 128)) {
+      if (rows < 256) return kRowsAsBefore;   // (not measured below)
+      if (mean >= 250 ? rows <= 1500 : mean >= 80 && tiles >= 2 && rows * tiles <= (elem_size == 4 ? 2100 : 1100)) return kRowsSixteenWaves;
+      return kRowsAsBefore;
+    }
+    if (elem_size == 4) ratio = std::max(hist[twice] < 0.01 * p.m ? 2.0 : 0.65, rows / 5500);
+  } else {
+    if (even) return wpr == 1 ? kRowsAsBefore : rows < 2000 || (mean > 250 && !level) || (mean > 500 && rows < 6000) ? kRowsFourWaves : elem_size == 4 ? twice : kRowsOneWave;
+    if (mean < 16 || (rows < 2000 && mean >= 100) || (rows < 5500 && mean > 250)) return kRowsAsBefore;
+  }
+  return std::min(15, std::max(0, (int)std::lround(std::log2(std::min(ratio, 4.0) * mean / kWave))));
+}
+
 // Wavefronts per row of the kernel for narrow ragged rows (spmm_ragged.hip), 0 = a single nonzero per gather stays ahead: rows with few nonzeros leave it nothing to
 // share out, few rows nothing to fill the chip with.  Even rows by one wavefront each where there are many (the histogram tells: none longer than two to four
 // times the mean), rows of several hundred nonzeros and uneven ones by four.  MI355X, us, one nonzero per gather / one wavefront a row / four:
@@ -326,10 +401,12 @@ inline int ragged_narrow_waves(const SpmmParams& p, int batch, const int* hist, 
     even = hist[j] == 0;
   }
   if (elem_size == 2 && p.n % 2 != 0 && mean > 1000) return 0;   // (16-byte gathers at odd addresses: 4086 x 8048 at 71 %, n = 9 118 / - / 189)
-  if (even && mean >= 24 && rows >= 2700) return 1;
+  const double groups = rows / (4 * 256);
+  if (even && mean >= 24 && rows >= 2700 && (mean <= 150 || groups >= 0.96 * std::ceil(groups))) return 1;
   if (p.n > 256 / elem_size) return 0;   // (two nonzeros per gather: 568 x 2832 at 71 %, n = 137 fp16 21 / - / 31)
-  if (mean >= 250) return 4;
-  return hist && !even && mean >= 80 ? 4 : 0;
+  const bool odd = elem_size == 2 && p.n % 2 != 0;
+  if (mean >= 250) return odd && even && rows >= 2700 ? 0 : 4;
+  return hist && !even && mean >= (odd ? 150 : 80) ? 4 : 0;
 }
 
 // ---- LDS-staged variant -----------------------------------------------------------------
@@ -707,7 +784,7 @@ inline size_t dense_path_bytes(const SpmmParams& p, int batch) {
 //     matrix-core SpMM kernels at 1.2 TB/s (8 x 4096 x 4096, k = 128: 0.24 ms), the gather kernels write it at 4 TB/s, the few-columns kernel at 4.5 TB/s plus 10 clocks of a CU's LDS
 //     per nonzero and tile (same shape at 93 % sparsity: 0.15 ms; 8 x 4096 x 4096, k = 128 at 50 %: 0.58
 //     against 0.17 for the dense form).
-// The dense form has to win by 15 % to be taken, by 20 % with a copy of B.  `few_columns`: the alternative is the few-columns kernel.
+// The dense form has to win by 15 % to be taken, by 20 % with a copy of B, 40 % if k is short too (10440 x 664 at 97 %, n = 1422: 47 against 39 us).  `few_columns`: the alternative is the few-columns kernel.
 // split_room: the workspace has room for the GEMM to take k in parts where it would (few tiles, long k: the K loop of a
 // tile then runs on several CUs; 4096^2 at 70-90 %, n = 128 / 256: 40 / 41 -> 27 / 32 us).
 //   Wide rows are gathered in tiles of 512 columns, the last one as slow as the others (3449 x 8696 at 94 %, n = 552: 185
@@ -750,7 +827,7 @@ inline bool dense_path_wins(const SpmmParams& p, int batch, int matrix_core_kind
   const double product = std::max({flops / 1000e12, std::ceil(tiles / 512.0) * (p.k / 32.0) * 0.23e-6 / parts, out_bytes / 3e12});
   const double pad = dense_path_pads(p) ? 4e-6 + 4.0 * p.k * p.n * batch / 4e12 : 0.0;
   const double dense_form = 8e-6 + cells * 2 / 4e12 + pad + product;
-  return (dense_path_pads(p) ? 1.2 : 1.15) * dense_form < other_families_seconds(p, batch, matrix_core_kind, few_columns);
+  return (!dense_path_pads(p) ? 1.15 : p.k < 1024 ? 1.4 : 1.2) * dense_form < other_families_seconds(p, batch, matrix_core_kind, few_columns);
 }
 
 // Behind dense form and copy (rounded up to 256 bytes) the workspace may hold what the GEMM wants for splitting K over two
@@ -840,13 +917,15 @@ inline double split_path_seconds(const SpmmParams& p, int batch) {
 }
 inline bool split_path_wins(const SpmmParams& p, int batch) {
   // Row kernel: whole tiles of 256 columns (narrow ones to the next power of two) at 30 TB/s, 25 where a tile's slice of B outgrows an XCD's L2.
-  // Rows of geometric lengths run at half of that with more than 256 columns, which the shape does not tell: the limit is that of even rows.
+  // Few rows of geometric lengths run at a third of that, which the shape does not tell: the limit is that of even rows.  A last tile of 208 columns or fewer
+  // costs less than a whole one (2779 x 1144 at 71 %, n = 153 31 / 37; 5305 x 7241 at 93 %, n = 358 209 / 231).
   // MI355X, us, the kernels before / this way, at either side of the line: 4096 x 4096, even rows, n = 512, 80 % 218 / 112, 90 % 115 / 108, 95 % 62 / 104;
   // n = 256, geometric, 80 % 114 / 80, 90 % 66 / 75; n = 128, 70 % 98 / 70, 80 % 60 / 65; 1656 x 1504, n = 640, 82 % 44 / 42; 2071 x 1694, n = 216,
   // 72 % 36 / 47; 1408 x 10744, n = 513, 92 % 243 / 131; 11008 x 4096 and most of 200 drawn shapes in profiles/spmm_fp32_by_parts.txt.
   int narrow = 32;
   while (narrow < p.n) narrow *= 2;
-  const double columns = p.n <= 256 ? std::min(narrow, 256) : ceil_div(p.n, 256) * 256;
+  const int last = p.n % 256;
+  const double columns = p.n <= 128 ? narrow : p.n - last + (last == 0 ? 0 : last <= 208 ? 216 : 256);
   const double gather = 5e-6 + (double)p.nnz * columns * batch * 4 / ((double)p.k * std::min(p.n, 256) > 1.1e6 ? 25e12 : 30e12);
   if (gather < 30e-6) return false;   // (what three launches and a short product take)
   // Up to 256 columns the fp32 matrix-core kernel keeps the calls that its density rule gives it, although they are shorter this way (4096 x 4096, n = 256, 70 %
@@ -1001,7 +1080,8 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
     if (lvec == kMax) return launch_lds_rpw<T, IT, kMax>(p, batch, rpw, stream);
     return launch_lds_rpw<T, IT, kMax / 2>(p, batch, rpw, stream);
   }
-  const int wpr = ch.wpr;
+  int wpr = ch.wpr;
+  bool by_length = true;   // (the rule for few chunks below)
   SpmmShape sh = spmm_pick_shape<T>(p.n, p.dense, p.out);
   if (ch.lpg && sh.vec == kMax && ch.lpg <= sh.lpg) sh.lpg = ch.lpg;  // narrower tiles on request
   // The caller knows the pattern's row lengths: wavefronts per row by the row's own length instead of one number for
@@ -1012,9 +1092,17 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
   // cell), not by its longest rows: four waves on every row keep more gathers in flight than a schedule that gives short
   // rows one wave, and that wins wherever the chip is full.  So this kernel is taken where it is not: fewer chunks
   // of 64 nonzeros than the chip holds wavefronts, and narrow tiles (several nonzeros per gather instruction).
-  if (ch.variant == 11) IEX_REQUIRE(ch.hist && sh.vec == kMax, IEX_ERR_BAD_ARGUMENT, "spmm: the rows-by-length kernel needs the row-length histogram (iex_spmm_sched) and full 128-bit vectors");
+  const bool ragged = p.n % kMax != 0 && p.n >= kWave * kMax / 2 && ch.lpg == 0;
+  if (ch.variant == 11) IEX_REQUIRE(ch.hist && (sh.vec == kMax || (ragged && ch.wpr_forced && wpr == 4)), IEX_ERR_BAD_ARGUMENT, "spmm: the rows-by-length kernel needs the row-length histogram (iex_spmm_sched) and full 128-bit vectors");
   const double chunk_count = (double)p.nnz / kWave * ceil_div(p.n, sh.lpg * sh.vec) * batch;
-  if (ch.hist && sh.vec == kMax && ch.nt <= 1 &&
+  if (ch.hist && ch.nt <= 1 && (sh.vec == kMax || ragged) && ((ch.variant == 11 && ch.wpr_forced && wpr == 4) || (ch.variant != 11 && flags_wpr_free(ch)))) {
+    const int way = ch.variant == 11 ? (ch.rpw ? ch.rpw - 1 : 0) : rows_by_histogram(p, batch, ch.hist, sizeof(T), sh.lpg, wpr);
+    if (way >= 0) return launch_long_rows<T, IT>(p, batch, sh.lpg, ragged, ch.hist, way, stream);
+    if (way == kRowsSixteenWaves && !ragged) return launch_rows<T, IT>(p, batch, kWave, ch.hist, 1, stream);
+    wpr = way == kRowsOneWave ? 1 : wpr;
+    by_length = way == kRowsAsBefore;
+  }
+  if (by_length && ch.hist && sh.vec == kMax && ch.nt <= 1 &&
       (ch.variant == 11 || (flags_wpr_free(ch) && ch.hist[0] > 0 && wpr != 1 && sh.lpg <= 32 && chunk_count <= 8192.0)))
     return launch_rows<T, IT>(p, batch, sh.lpg, ch.hist, ch.variant == 11 ? ch.rpw : 0, stream);
   // Two tiles per wave double the slice of the dense operand that the waves of an XCD share in
@@ -1032,7 +1120,7 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
   // half a tile wide: 128-bit accesses at element alignment instead of narrower vectors.  Measured on
   // the reference's ViT sweep shapes (fp32, batch 384, 97 % sparse): 785 x 785 outputs 865 -> 516 us,
   // 197 x 197 outputs 64 -> 33 us.
-  if (p.n % kMax != 0 && p.n >= kWave * kMax / 2 && ch.lpg == 0) return launch_ragged<T, IT, kMax>(p, batch, wpr, stream);
+  if (ragged) return launch_ragged<T, IT, kMax>(p, batch, wpr, stream);
   // ... and narrower ones, several nonzeros per gather
   if (p.n >= kMax && p.n < kWave * kMax / 2 && ch.lpg == 0 && nt == 1 && !ch.wpr_forced) {
     if (const int waves = ragged_narrow_waves(p, batch, ch.hist, sizeof(T)))

@@ -416,6 +416,59 @@ __device__ __forceinline__ void spmm_rows_block(const SpmmParams& p, const RowCl
   spmm_store_row<T, VEC, LPG, 1, false>(p, bz, row, col0, 0, acc);
 }
 
+// ... and by workgroups of four wavefronts, for as many rows as fill the chip: the first `long_rows` row slots get one each, the others four to a
+// workgroup.  As above the host counts the slots, and a row's own length settles its sum: more than `limit` nonzeros are added up as four shares, wherever
+// the row stands.
+struct LongRows {
+  int long_rows, limit;
+};
+
+template <typename T, typename IT, int VEC, int LPG, bool RAGGED>
+__device__ __forceinline__ void spmm_long_rows_block(const SpmmParams& p, const LongRows& lr, int bx, int by, int bz, float* red) {
+  constexpr int TW = LPG * VEC;
+  const int lane = lane_id();
+  const int wave = uniform(threadIdx.x >> 6);
+  const bool shared = bx < lr.long_rows;   // (uniform over the workgroup) the workgroup has one row slot
+  const int slot = shared ? bx : lr.long_rows + (bx - lr.long_rows) * 4 + wave;
+  const int col0 = by * TW + (lane % LPG) * VEC;
+  const int shift = (RAGGED && col0 < p.n && col0 + VEC > p.n) ? col0 + VEC - p.n : 0;  // (n >= VEC, checked by the host)
+  const int col_ld[1] = {col0 < p.n ? col0 - shift : 0};
+  float* const own = red + wave * VEC * kWave + lane;
+  float acc[1][VEC];
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) acc[0][i] = 0.f;
+  int row = 0;
+  if (slot < p.m) {
+    row = uniform(p.row_indices[slot]);
+    const int start = uniform(p.row_offsets[row]), end = uniform(p.row_offsets[row + 1]);
+    const int parts = end - start > lr.limit ? 4 : 1;
+    // a share for each wavefront of a workgroup that has one row, else all of them in their order (the sum so far waits in the wavefront's own part of LDS)
+    const int first = shared ? wave : 0, last = shared ? min(wave + 1, parts) : parts;
+    for (int q = first; q < last; ++q) {
+      spmm_range_partial<T, IT, VEC, LPG, kSpmmUnroll, 1, RAGGED>(p, bz, start, end, q, parts, col_ld, acc);
+      if (last - first == 1) break;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        if (q > first) acc[0][i] = own[i * kWave] + acc[0][i];
+        if (q + 1 < last) own[i * kWave] = acc[0][i], acc[0][i] = 0.f;
+      }
+    }
+  }
+  if (shared) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) own[i * kWave] = acc[0][i];
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+#pragma unroll
+      for (int w = 1; w < 4; ++w) acc[0][i] += own[(w * VEC + i) * kWave];
+    }
+  }
+  if (slot >= p.m || lane / LPG != 0) return;
+  spmm_store_row<T, VEC, LPG, 1, RAGGED>(p, bz, row, col0, shift, acc);
+}
+
 // Host-side shape choice shared by the stand-alone and the fused launcher.
 // VEC: widest per-lane vector that divides n and keeps rows aligned.  LPG: lanes per
 // nonzero; below 64 only for full 128-bit vectors (narrow outputs then run several

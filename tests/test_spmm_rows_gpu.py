@@ -138,3 +138,50 @@ def test_forcing_it_without_a_histogram_is_refused(dev):
                                  b.data_ptr(), None, out.data_ptr(), torch.cuda.current_stream().cuda_stream, 1)
     assert rc == _lib.load().iex_spmm_ex.restype(-1) or rc == -1
     assert "histogram" in _lib.last_error()
+
+
+@pytest.mark.parametrize("dtype,n", [(torch.float32, 32), (torch.float32, 64), (torch.float32, 100), (torch.float32, 256), (torch.float32, 130), (torch.float32, 301),
+                                     (torch.float16, 64), (torch.float16, 128), (torch.float16, 200), (torch.float16, 520), (torch.float16, 259)])
+@pytest.mark.parametrize("code", [1, 3, 15])                # more than 64 or 256 nonzeros are long, none is
+def test_four_wavefronts_for_the_long_rows_only(oracle, dev, dtype, n, code):
+    """Every tile width and rows of no whole vectors, empty rows, a ragged last workgroup; the order of the rows and a wrong histogram change no bit."""
+    rng = np.random.default_rng(n + code)
+    m, k = 205, 700
+    lens = rng.integers(0, 90, m)
+    lens[[3, 77, 150, 151]] = [700, 257, 65, 0]
+    ro, ci = W.csr_from_row_lengths(rng, m, k, lens)
+    c = W.CSR(m, k, rng.standard_normal(ci.shape[0]).astype(np.float32), W.swizzle_from_offsets(ro), ro, ci)
+    b_np = rng.standard_normal((2, k, n)).astype(np.float32)
+    flags = (11 << 16) | (4 << 8) | (code << 20)
+    hist = _histogram(c.row_offsets)
+    out = _call(c, dev, b_np, dtype, torch.int32, flags, hist, batch=2)
+    assert "spmm_rows_kernel4" in _lib.last_kernels()
+    v, b_r = rounded(c.values, dtype), rounded(b_np, dtype)
+    want = oracle.spmm(b_r, c.row_indices, v, c.row_offsets, c.column_indices, c.m)
+    scale = oracle.spmm_abs_scale(b_r, c.row_indices, v, c.row_offsets, c.column_indices, c.m)
+    half = dtype == torch.float16   # 700 roundings of a sum, each 2^-24 of the magnitudes; fp16: the result's rounding too, 2^-11 of it or 2^-25
+    assert_close(out.float().cpu().numpy(), want, scale, 2.0 ** -11 if half else 0.0, f"{dtype} n={n}", atol=700 * 2.0 ** -24 * scale + (2.0 ** -25 if half else 0.0))
+    for order in (None, np.arange(m, dtype=np.int32), rng.permutation(m).astype(np.int32)):
+        for h in (hist, [m] * 16, [0] * 16, [3, 2, 1] + [0] * 13, [-4] + [10 ** 9] * 15):
+            assert torch.equal(_call(c, dev, b_np, dtype, torch.int32, flags, h, batch=2, row_indices=order), out), (h[:3], order is None)
+
+
+@pytest.mark.parametrize("dtype,m,k,n,sparsity,even,kernel", [
+    (torch.float32, 11008, 1000, 64, 0.95, True, "spmm_rows_kernel4"), (torch.float16, 11008, 1000, 64, 0.95, True, "8, 8, 1, 1"), (torch.float16, 6144, 512, 128, 0.9, False, "spmm_rows_kernel4"),
+    (torch.float32, 4096, 1024, 512, 0.95, False, "spmm_rows_kernel4"), (torch.float32, 512, 1024, 512, 0.9, False, "spmm_rows_kernel<"), (torch.float32, 4096, 512, 256, 0.9, True, "64, 1, 1")])
+def test_operator_takes_the_wavefronts_per_row_from_the_row_lengths(oracle, dev, dtype, m, k, n, sparsity, even, kernel):
+    rng = np.random.default_rng(m + n)
+    mean = k * (1 - sparsity)
+    lens = np.full(m, int(mean)) if even else np.minimum(k, rng.geometric(1 / mean, m))
+    ro, ci = W.csr_from_row_lengths(rng, m, k, lens)
+    c = W.CSR(m, k, rng.standard_normal(ci.shape[0]).astype(np.float32), W.swizzle_from_offsets(ro), ro, ci)
+    ri, v, ro_t, ci_t = to_dev(c, dev, dtype)
+    b_np = rng.standard_normal((1, k, n)).astype(np.float32)
+    b = torch.from_numpy(b_np).to(dev).to(dtype)
+    out = (ops.spmm_sputnik_reuse_weight if dtype == torch.float32 else ops.spmm_sputnik_reuse_weight_half)(b, ri, v, ro_t, ci_t, m)
+    assert kernel in _lib.last_kernels(), _lib.last_kernels()
+    v, b_r = rounded(c.values, dtype), rounded(b_np, dtype)
+    want = oracle.spmm(b_r, c.row_indices, v, c.row_offsets, c.column_indices, c.m)
+    scale = oracle.spmm_abs_scale(b_r, c.row_indices, v, c.row_offsets, c.column_indices, c.m)
+    half = dtype == torch.float16
+    assert_close(out.float().cpu().numpy(), want, scale, 2.0 ** -11 if half else 0.0, kernel, atol=float(lens.max()) * 2.0 ** -24 * scale + (2.0 ** -25 if half else 0.0))
