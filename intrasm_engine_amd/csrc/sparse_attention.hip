@@ -4,11 +4,12 @@
 namespace iex {
 namespace {
 
-// Entries of a 128 x 64 tile from which it counts as dense.  A tile costs the matrix-core path about 1100 (16-bit) and 8200
-// (fp32, HD = 64) clocks of a wavefront for 32 rows, an entry on its own about 20 and 40 beside its two rows from L2.  (16
-// heads x 1500 tokens, 175 scattered entries per tile, fp16: 45 us from 128 on, 30 from 224 on; 8 x 1000, 260 per tile, fp32:
-// 28 from 224 on, 22 from 400 on.)
-inline int dense_min(int dtype) { return dtype == IEX_F32 ? 800 : 224; }
+// Entries of a 128 x 64 tile from which it counts as dense (fewer where only some groups of 32 rows have entries there).  A tile costs the matrix-core
+// path about 1100 (16-bit) and 8200 (fp32, HD = 64) clocks of a wavefront for 32 rows, an entry on its own about 20 and 40 beside its two rows from L2.  (16
+// heads x 1500 tokens, 175 scattered entries per tile, fp16: 45 us from 128 on, 30 from 224 on.  262 per tile, bf16, us from 224 / 288 / 512 on: 4 x 1000
+// of 128 20.5 / 14.4 / 13.1, 32 x 1000 of 32 21.8 / 17.3 / 16.4, of 64 27.2 / 25.2 / 24.8, of 128 42.7 / 43.5 / 43.5; 327 per tile, 32 x 800 of 128 37.8 / 37.9 / 41.5;
+// 655, 4 x 400 of 64 8.5 / - / 12.3.  8 x 1000, 260 per tile, fp32: 28 from 224 on, 22 from 400 on.)
+inline int dense_min(int dtype) { return dtype == IEX_F32 ? 800 : 288; }
 
 template <int TYPE, int HD, int QW, int KW>
 int launch(const SparseAttentionParams& p, hipStream_t stream) {
@@ -24,7 +25,7 @@ int launch(const SparseAttentionParams& p, hipStream_t stream) {
     }
   }
   note_kernel("sparse_attention_kernel<%s, %d, %d, %d>", TYPE == 2 ? "float" : TYPE == 1 ? "bf16" : "f16", HD, QW, KW);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(ceil_div(p.tokens, QW * 32) * (long long)p.heads)), dim3(QW * KW * kWave), lds, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(ceil_div(p.tokens, QW * 32) * (long long)p.heads)), dim3((QW * KW + SparseAttentionShape<TYPE, HD>::extra(KW)) * kWave), lds, stream, p);
   return check_hip(hipGetLastError(), "sparse attention launch");
 }
 

@@ -7,10 +7,12 @@
 // bf16: 37 / 6.8; 16 x 4096, band 256 + 32 scattered, fp16: 81 / 38.7; 32 x 2048 x 128, causal band of 512, fp32: 1121 / 182.
 //
 // The mask's tables (made once per mask by mask_tables_kernel): per block of 128 rows the 64-column tiles that hold at
-// least dense_min entries ("dense"), for each of them a 64-bit word per row, and per row the columns outside dense tiles.
+// least dense_min / 4 entries for each group of 32 rows that has any there ("dense"), for each of them a 64-bit word per row, and per row the columns outside dense tiles.
 // A wavefront owns 32 queries, a workgroup QW wavefronts (fewer where the heads are few: more workgroups, and fewer tiles
 // that only some of its wavefronts want), or KW wavefronts share 32 queries, each with every KW-th tile and stages of its own
-// (8 heads x 1000 tokens, fp32: 27.8 -> 16 us).
+// (8 heads x 1000 tokens, fp32: 27.8 -> 16 us), with more wavefronts beside them that do nothing but the other entries: their chains run
+// beside the tiles' on the SIMDs that the stages' LDS leaves empty (8 x 1500 of 128, band 64 + 32 scattered, bf16 44.9 -> 25.4 us, fp32 16 x 1214 of 128
+// + 16 118 -> 66, 12 x 3280 of 64 + 32 102 -> 81; by no scattered entries but the band's corners, 8 x 1000 of 64, 8.2 -> 7.7).
 //   * dense tiles as in attention_device.cuh: K and V rows of a tile straight into LDS, two stages; S^T = K Q^T on the
 //     matrix cores, entries outside the mask to -infinity by the row's word, running maximum and sum per query in registers,
 //     O^T += V^T P^T with the probabilities as they lie in the lanes.  fp32 goes by v_mfma_f32_32x32x2, tiles in halves.
@@ -88,7 +90,9 @@ __global__ __launch_bounds__(kMtWaves * kWave) void mask_tables_kernel(int m, in
     int had = 0;
     for (int base = 0; base < tiles; base += kWave) {
       const int tile = base + lane;
-      const bool is = tile < tiles && count[tile] >= dense_min;
+      // (a tile costs every group of 32 rows that has entries there: a band's corner with entries of one group is worth it from a quarter on; fp32, 8 x 1544 of
+      // 32, band 512 + 16 scattered, 31.5 -> 23 us, 16 x 1179 of 64, band 64, 33.8 -> 27.7)
+      const bool is = tile < tiles && 4 * count[tile] >= dense_min * __popc((unsigned)groups[tile]) && count[tile] > 0;
       const unsigned long long them = __ballot(is);
       if (tile < tiles) count[tile] = -1;
       if (is) {
@@ -149,10 +153,14 @@ struct SparseAttentionShape {
   static constexpr int CPR = HD * ES / 16;                  // 16-byte chunks per row
   static constexpr int TILE = KEYS * HD * ES;               // bytes of K or V per stage
   static constexpr int TLD = HD + 4;                        // floats per row of the scattered entries' results
+  static constexpr int stages(int qw, int kw) { return kw * 2 * (2 * TILE + qw * 256); }
+  // by several wavefronts to 32 queries the scattered entries' results lie behind the stages, else in their place
   static constexpr int lds(int qw, int kw) {
-    const int stages = kw * 2 * (2 * TILE + qw * 256), thin = qw * 32 * (TLD + 4) * 4 + (kw - 1) * (HD / 2 + 2) * 256;
-    return stages > thin ? stages : thin;
+    const int thin = qw * 32 * (TLD + 4) * 4;
+    return kw > 1 ? stages(qw, kw) + thin : stages(qw, kw) > thin ? stages(qw, kw) : thin;
   }
+  // wavefronts beside those KW, for the scattered entries alone
+  static constexpr int extra(int kw) { return kw == 1 ? 0 : kw == 2 ? 6 : 4; }
 };
 
 // LDS row of a key (or chunk permutation of a row): what keeps the operand reads of 16 consecutive lanes apart.
@@ -199,10 +207,11 @@ __device__ __forceinline__ void sa_add_row(float* acc, float w, u32x4 chunk) {
 }
 
 template <int TYPE, int HD, int QW, int KW>
-__global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attention_kernel(SparseAttentionParams p) {
+__global__ __launch_bounds__((QW * KW + SparseAttentionShape<TYPE, HD>::extra(KW)) * kWave, 2) void sparse_attention_kernel(SparseAttentionParams p) {
   typedef SparseAttentionShape<TYPE, HD> Shape;
   constexpr int ES = Shape::ES, KEYS = Shape::KEYS, CPR = Shape::CPR, TILE = Shape::TILE, TLD = Shape::TLD;
   constexpr bool F32 = TYPE == 2;
+  constexpr int XW = Shape::extra(KW);              // (wavefronts KW .. KW + XW - 1)
   constexpr int PER = kMaCols / KEYS;               // stages per tile of the mask
   constexpr int KB = KEYS / 32, DT = HD / 32;       // blocks of 32 keys, of 32 features
   constexpr int RPI = kWave / CPR;                  // rows per direct load
@@ -336,7 +345,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
   };
 
   // ---- dense tiles that any of this workgroup's rows have entries in
-  {
+  if (XW == 0 || kw < KW) {
     const int count = uniform(list[0]), mine = ((1 << QW) - 1) << group0;
     int entry = 0;   // of the tile that `next` has found
     auto next = [&](int i) {
@@ -359,11 +368,11 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
     }
   }
   sum += __shfl_xor(sum, 32);
-  __syncthreads();   // everybody is done with the stages
+  if constexpr (KW == 1) __syncthreads();   // everybody is done with the stages
 
   // ---- entries outside dense tiles: CPR lanes per row, G rows side by side, U entries of each at a time.  A lane holds the
   // same 16 bytes of every row of K and V, so nothing but the dot products crosses lanes.
-  float* rows = reinterpret_cast<float*>(smem) + wave * 32 * (TLD + 4);   // [32][TLD]: sums over them; then [32][2]: maximum, sum
+  float* rows = reinterpret_cast<float*>(smem + (KW > 1 ? Shape::stages(QW, KW) : 0)) + wave * 32 * (TLD + 4);   // [32][TLD]: sums over them; then [32][2]: maximum, sum
   float* state = rows + 32 * TLD;
   const int row0 = q0 + wave * 32;
   const int my_row = min(row0 + col, T - 1);
@@ -374,7 +383,7 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
     typedef int i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
     const int* thin_cols = reinterpret_cast<const int*>(p.tables + mt.thin_cols);
     const int sub = lane / CPR, part = lane % CPR;
-    for (int r0 = kw * G; r0 < 32; r0 += KW * G) {
+    for (int r0 = (kw + XW) % (KW + XW) * G; r0 < 32; r0 += (KW + XW) * G) {
       const int row = row0 + r0 + sub, safe = min(row, T - 1);
       const int2 thin = thin_of[safe];
       const int count = row < T ? thin.y : 0;
@@ -435,8 +444,10 @@ __global__ __launch_bounds__(QW * KW * kWave, KW > 1 ? 1 : 2) void sparse_attent
   }
   if constexpr (KW > 1) {   // the sums of the other wavefronts' tiles
     constexpr int N = 16 * DT;
-    float* parts = reinterpret_cast<float*>(smem) + 32 * (TLD + 4);   // [KW - 1][N + 2][64]
-    if (kw > 0) {
+    float* parts = reinterpret_cast<float*>(smem);   // [KW - 1][N + 2][64]
+    static_assert((KW - 1) * (N + 2) * kWave * 4 <= Shape::stages(QW, KW), "in the place of the stages");
+    __syncthreads();   // everybody is done with the stages
+    if (kw > 0 && kw < KW) {
       float* mine = parts + (kw - 1) * (N + 2) * kWave + lane;
 #pragma unroll
       for (int d = 0; d < DT; ++d)

@@ -57,6 +57,27 @@ def test_against_dense_masked_attention(dev, dtype, tol, heads, tokens, d, band,
     assert torch.equal(out, sparse_attention(*operands, ri, ro, ci))
 
 
+@pytest.mark.parametrize("dtype, tol", [(torch.bfloat16, 1e-2), (torch.float32, 1e-5)])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("tokens, group, corner", [(31, 0, 3), (160, 1, 80), (161, 4, 230), (420, 12, 300)])
+def test_lists_beside_tiles_that_few_rows_have(dev, dtype, tol, d, tokens, group, corner):
+    """Few heads (the entries outside dense tiles go to wavefronts of their own): rows with lists and tiles of which one group of 32 rows has entries, on either
+    side of the number that makes a tile dense, the last block of rows among them."""
+    rng = np.random.default_rng(tokens + d)
+    mask = _mask(tokens, 1, 5, rng)
+    first = min(group * 32, tokens - 1)
+    block = mask[first:first + 32, :64]
+    block.flat[rng.permutation(block.size)[:corner]] = True
+    ro, ci, _ = W.csr_from_mask(mask)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    ri, ro, ci = t(W.swizzle_from_offsets(ro)), t(ro), t(ci)
+    q, k, v = (rng.standard_normal((3, tokens, d)).astype(np.float32) for _ in range(3))
+    out = sparse_attention(*(t(x).to(dtype) for x in (q, k, v)), ri, ro, ci)
+    assert "sparse_attention_kernel" in _lib.last_kernels() and ", 1, " in _lib.last_kernels()
+    want = _reference(mask, *(rounded(x, dtype).astype(np.float64) for x in (q, k, v)))
+    assert np.linalg.norm(out.float().cpu().numpy() - want) <= tol * np.linalg.norm(want)
+
+
 def test_tables_follow_the_mask(dev):
     """A mask changed in place is looked at again; one that nobody may look at, and columns in another order, go by three kernels."""
     from intrasm_engine_amd.pytorch import ops as pyops
