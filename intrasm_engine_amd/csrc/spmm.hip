@@ -845,8 +845,7 @@ template <typename IT>
 int launch_dense_form(int m, int ld, const int* row_offsets, const void* cols, const void* values, void* out, int* zero_words, int n_zero_words,
                       hipStream_t stream) {
   note_kernel("csr_to_dense_kernel<%s>", type_name<IT>());
-  hipLaunchKernelGGL((csr_to_dense_kernel<IT>), dim3(ceil_div(m, kDenseRows)), dim3(kDenseThreads), 0, stream, m, ld, row_offsets,
-                     static_cast<const IT*>(cols), static_cast<const uint16_t*>(values), static_cast<uint16_t*>(out), zero_words, n_zero_words);
+  launch_csr_to_dense<IT>(m, ld, row_offsets, cols, values, out, zero_words, n_zero_words, stream);
   return check_hip(hipGetLastError(), "spmm dense-form launch");
 }
 

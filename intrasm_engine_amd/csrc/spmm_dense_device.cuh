@@ -9,8 +9,9 @@
 // workspace is written exactly once, by one kind of store, whatever the sparsity.  What a row costs is the chain of
 // "load 256 nonzeros, scatter them" steps of its wavefronts, each a round trip to memory: with one wavefront per row
 // the longest row set the kernel's time (4096 nonzeros: 16 steps, 24 us where the bytes written take 8).
-// Rows longer than kDenseSeg columns are done in segments, every wavefront with a cursor into its quarter of the
-// row's ascending column indices.  k, here the row stride of the dense form, is a multiple of 8 and no less than the number
+// Rows longer than the columns in LDS are done in segments, every wavefront with a cursor into its quarter of the
+// row's ascending column indices: quarters wait for their segment, so rows of more than 5120 columns have a workgroup and LDS for 12288 of them to themselves
+// (4096 x 11008 at 90 %, geometric lengths, 30.4 -> 20.8 us, even ones 21.9 -> 19.9; 500 x 8000 10.7 -> 6.2; not for 11008 x 4160, 20.6 -> 21.1).  k, here the row stride of the dense form, is a multiple of 8 and no less than the number
 // of columns (the rest is zero); the workspace is 16-byte aligned; column indices inside a row must ascend strictly
 // (canonical CSR).
 #pragma once
@@ -18,52 +19,51 @@
 
 namespace iex {
 
-constexpr int kDenseSeg = 4096;  // columns of a row assembled at a time (8 KB of LDS per wavefront)
+constexpr int kDenseSeg = 4096;       // columns of a row assembled at a time, two rows to a workgroup (16 KB of LDS)
+constexpr int kDenseLongSeg = 12288;  // ... of longer rows, one to a workgroup (24 KB)
 constexpr int kDenseWaves = 4;
 constexpr int kDenseThreads = kDenseWaves * kWave;
 
-constexpr int kDenseRows = 2;     // rows per workgroup, side by side: the loads of both are in flight together
-
-template <typename IT>
+template <typename IT, int ROWS, int SEG>
 __global__ __launch_bounds__(kDenseThreads) void csr_to_dense_kernel(int m, int k, const int* __restrict__ row_offsets,
                                                                      const IT* __restrict__ cols,
                                                                      const uint16_t* __restrict__ values,
                                                                      uint16_t* __restrict__ out, int* __restrict__ zero_words,
                                                                      int n_zero_words) {
-  __shared__ __align__(16) uint16_t srow[kDenseRows][kDenseSeg];
+  __shared__ __align__(16) uint16_t srow[ROWS][SEG];
   // (words that the kernel after this one wants zero at its launch, a few hundred at most: cheaper here than a launch)
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < n_zero_words; i += kDenseThreads) zero_words[i] = 0;
   const int lane = lane_id();
   const int wave = uniform(threadIdx.x >> 6);
   // this wavefront's quarter of each row's nonzeros, in whole chunks of 64
-  int pos[kDenseRows], end[kDenseRows];
+  int pos[ROWS], end[ROWS];
 #pragma unroll
-  for (int r = 0; r < kDenseRows; ++r) {
-    const int row = min((int)blockIdx.x * kDenseRows + r, m - 1);   // (the grid has ceil(m / kDenseRows) workgroups)
+  for (int r = 0; r < ROWS; ++r) {
+    const int row = min((int)blockIdx.x * ROWS + r, m - 1);   // (the grid has ceil(m / ROWS) workgroups)
     const int first = uniform(row_offsets[row]);
-    const int last = (int)blockIdx.x * kDenseRows + r < m ? uniform(row_offsets[row + 1]) : first;   // (past the matrix: an empty row, not stored)
+    const int last = (int)blockIdx.x * ROWS + r < m ? uniform(row_offsets[row + 1]) : first;   // (past the matrix: an empty row, not stored)
     const int share = ((max(last - first, 0) + kWave * kDenseWaves - 1) / (kWave * kDenseWaves)) * kWave;
     pos[r] = min(first + wave * share, last);
     end[r] = min(pos[r] + share, last);
   }
-  for (int c0 = 0; c0 < k; c0 += kDenseSeg) {
-    const int len = min(kDenseSeg, k - c0);  // a multiple of 8
+  for (int c0 = 0; c0 < k; c0 += SEG) {
+    const int len = min(SEG, k - c0);  // a multiple of 8
     if (c0) __syncthreads();   // the previous segment has been copied out
 #pragma unroll
-    for (int r = 0; r < kDenseRows; ++r)
+    for (int r = 0; r < ROWS; ++r)
       for (int i = threadIdx.x * 8; i < len; i += kDenseThreads * 8) *reinterpret_cast<uint4*>(srow[r] + i) = uint4{0u, 0u, 0u, 0u};
     __syncthreads();
     // the nonzeros of this segment: 64 at a time from the cursors, four chunks of each row in flight
-    bool more[kDenseRows];
+    bool more[ROWS];
 #pragma unroll
-    for (int r = 0; r < kDenseRows; ++r) more[r] = pos[r] < end[r];
-    static_assert(kDenseRows == 2, "the loop below names both rows");
-    while (more[0] || more[1]) {
-      int c[kDenseRows][4];
-      uint16_t v[kDenseRows][4];
+    for (int r = 0; r < ROWS; ++r) more[r] = pos[r] < end[r];
+    static_assert(ROWS <= 2, "the loop below names both rows");
+    while (more[0] || more[ROWS - 1]) {
+      int c[ROWS][4];
+      uint16_t v[ROWS][4];
 #pragma unroll
-      for (int r = 0; r < kDenseRows; ++r)
+      for (int r = 0; r < ROWS; ++r)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int j = max(min(pos[r] + u * kWave + lane, end[r] - 1), 0);   // (a row without nonzeros: entry 0, never used)
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(kDenseThreads) void csr_to_dense_kernel(int m, int 
           v[r][u] = values[j];
         }
 #pragma unroll
-      for (int r = 0; r < kDenseRows; ++r) {
+      for (int r = 0; r < ROWS; ++r) {
         int taken = 0;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -87,8 +87,8 @@ __global__ __launch_bounds__(kDenseThreads) void csr_to_dense_kernel(int m, int 
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kDenseRows; ++r) {
-      const int row = (int)blockIdx.x * kDenseRows + r;
+    for (int r = 0; r < ROWS; ++r) {
+      const int row = (int)blockIdx.x * ROWS + r;
       if (row < m)
         for (int i = threadIdx.x * 8; i < len; i += kDenseThreads * 8)
           *reinterpret_cast<uint4*>(out + (size_t)row * k + c0 + i) = *reinterpret_cast<const uint4*>(srow[r] + i);
@@ -118,6 +118,18 @@ static __global__ __launch_bounds__(256) void pad_rows_kernel(int rows, int cols
     for (int e = 0; e < 8; ++e) w.v[e] = c + e < cols ? src[c + e] : (uint16_t)0;
   }
   *reinterpret_cast<Whole*>(dst + c) = w;
+}
+
+// (k: the row stride of the dense form)
+template <typename IT>
+inline void launch_csr_to_dense(int m, int k, const int* row_offsets, const void* cols, const void* values, void* out, int* zero_words, int n_zero_words,
+                                hipStream_t stream) {
+  if (k < kDenseSeg + kDenseSeg / 4)
+    hipLaunchKernelGGL((csr_to_dense_kernel<IT, 2, kDenseSeg>), dim3(ceil_div(m, 2)), dim3(kDenseThreads), 0, stream, m, k, row_offsets, static_cast<const IT*>(cols),
+                       static_cast<const uint16_t*>(values), static_cast<uint16_t*>(out), zero_words, n_zero_words);
+  else
+    hipLaunchKernelGGL((csr_to_dense_kernel<IT, 1, kDenseLongSeg>), dim3(m), dim3(kDenseThreads), 0, stream, m, k, row_offsets, static_cast<const IT*>(cols),
+                       static_cast<const uint16_t*>(values), static_cast<uint16_t*>(out), zero_words, n_zero_words);
 }
 
 inline int round8(int x) { return (x + 7) & ~7; }

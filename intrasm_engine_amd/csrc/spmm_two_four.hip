@@ -133,12 +133,8 @@ extern "C" int iex_form_build(int itype, int kind, int m, int k, int nonzeros, c
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (kind == 0) {
     note_kernel("csr_to_dense_kernel");
-    if (itype == IEX_I16)
-      hipLaunchKernelGGL((csr_to_dense_kernel<short>), dim3(ceil_div(m, kDenseRows)), dim3(kDenseThreads), 0, s, m, round8(k), row_offsets,
-                         static_cast<const short*>(column_indices), static_cast<const uint16_t*>(values), static_cast<uint16_t*>(form), nullptr, 0);
-    else
-      hipLaunchKernelGGL((csr_to_dense_kernel<int>), dim3(ceil_div(m, kDenseRows)), dim3(kDenseThreads), 0, s, m, round8(k), row_offsets,
-                         static_cast<const int*>(column_indices), static_cast<const uint16_t*>(values), static_cast<uint16_t*>(form), nullptr, 0);
+    if (itype == IEX_I16) launch_csr_to_dense<short>(m, round8(k), row_offsets, column_indices, values, form, nullptr, 0, s);
+    else launch_csr_to_dense<int>(m, round8(k), row_offsets, column_indices, values, form, nullptr, 0, s);
     return check_hip(hipGetLastError(), "dense form launch");
   }
   IEX_REQUIRE(scratch && aligned(scratch, 16) && scratch_bytes >= iex_form_scratch_bytes(m, k), IEX_ERR_BAD_ARGUMENT, "form: needs %zu bytes of scratch memory", iex_form_scratch_bytes(m, k));

@@ -860,3 +860,23 @@ def test_csr_check_names_what_a_pattern_lacks(dev):
     rows[r] = False
     assert torch.equal(a[0, torch.from_numpy(rows)], b[0, torch.from_numpy(rows)])
     assert torch.allclose(a[0, r], b[0, r], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("k", [4096, 5112, 5120, 12288, 12296, 25000])   # two rows to a workgroup, one; one segment of columns, two, three
+@pytest.mark.parametrize("index", [torch.int32, torch.int16])
+def test_dense_form_of_long_rows(oracle, dev, k, index):
+    from intrasm_engine_amd.pytorch import ops as pyops
+    rng = np.random.default_rng(k)
+    m, n = 7, 16
+    lens = np.array([k, 0, 1, k // 2, 1025, 64, k - 1])
+    ro, ci = W.csr_from_row_lengths(rng, m, k, lens)
+    csr = W.CSR(m, k, rng.standard_normal(ci.shape[0]).astype(np.float32), W.swizzle_from_offsets(ro), ro, ci)
+    b_np = rng.standard_normal((1, k, n)).astype(np.float32)
+    ri, v, ro_t, ci_t = to_dev(csr, dev, torch.float16, index)
+    b = torch.from_numpy(b_np).to(dev).half()
+    out = pyops._spmm(b, ri, v, ro_t, ci_t, m, per_batch_values=False, accumulate=False, dtypes=(torch.float16,), allow_i16=True, force_variant=7)
+    assert "csr_to_dense" in pyops._lib.last_kernels()
+    vals_r, b_r = rounded(csr.values, torch.float16), rounded(b_np, torch.float16)
+    want = oracle.spmm(b_r, csr.row_indices, vals_r, csr.row_offsets, csr.column_indices, m)
+    scale = oracle.spmm_abs_scale(b_r, csr.row_indices, vals_r, csr.row_offsets, csr.column_indices, m)
+    assert_close(out.float().cpu().numpy(), want, scale, RTOL[torch.float16], f"k={k}")
