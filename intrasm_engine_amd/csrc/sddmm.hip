@@ -101,6 +101,10 @@ __global__ __launch_bounds__(256) void sddmm_kernel(SddmmParams p) {
   constexpr int G = kWave / LPN;
   constexpr int KT = LPN * VEC;
   constexpr int kRowsPerBlock = 4 / WPR;
+  // k below PASSES * KT: a predicate on each load, or loads that all lanes do.  In bf16, whose products widen both operands, the predicated loads' registers
+  // spill (us, predicates / without: 9709 x 632 at 86 %, k = 184 256 / 56; 4000 x 2000 at 95 %, k = 200 109 / 27; 10773 x 1185 at 95.5 %, k = 136 75 / 25); fp16
+  // and fp32 are as fast or faster with them (k = 96 13.5 / 15.5, 200 20.7 / 21.9; fp32 1200 x 3434, k = 44 11.4 / 13.6).
+  constexpr bool CLAMP = RAGGED || (!EXACT && VEC > 1 && __is_same(T, __hip_bfloat16));
   const int lane = lane_id();
   const int wave = uniform(threadIdx.x >> 6);
   const int sub = lane / LPN;
@@ -142,21 +146,21 @@ __global__ __launch_bounds__(256) void sddmm_kernel(SddmmParams p) {
         const T* __restrict__ rhs = rhs_all + (size_t)z * rhs_zstride;
         vec_t<T, VEC> lfrag[PASSES];
         vec_t<T, VEC> rv[LPN][PASSES];
-        // (ragged: every lane reads a vector, only the last pass can reach past the row's end)
+        // (CLAMP: every lane reads a vector, and what the last pass reads past the row's end is cleared)
         const int last_kk = (PASSES - 1) * KT + sl * VEC;
-        const tail_mask<T, VEC> mask(RAGGED ? min(max(p.k - last_kk, 0), VEC) : VEC);
-        auto at = [&](int ps) { return RAGGED ? min(ps * KT + sl * VEC, p.k - VEC) : ps * KT + sl * VEC; };
+        const tail_mask<T, VEC> mask(CLAMP ? min(max(p.k - last_kk, 0), VEC) : VEC);
+        auto at = [&](int ps) { return CLAMP ? min(ps * KT + sl * VEC, p.k - VEC) : ps * KT + sl * VEC; };
 #pragma unroll
         for (int ps = 0; ps < PASSES; ++ps) {
-          if (EXACT || RAGGED || at(ps) < p.k) lfrag[ps] = load_vec<T, VEC, !RAGGED>(lhs + at(ps));
+          if (EXACT || CLAMP || at(ps) < p.k) lfrag[ps] = load_vec<T, VEC, !RAGGED>(lhs + at(ps));
         }
-        if constexpr (RAGGED) mask.apply(lfrag[PASSES - 1]);
+        if constexpr (CLAMP) mask.apply(lfrag[PASSES - 1]);
 #pragma unroll
         for (int st = 0; st < LPN; ++st) {
           const T* r = rhs + (size_t)cc[st] * p.k;
 #pragma unroll
           for (int ps = 0; ps < PASSES; ++ps) {
-            if (EXACT || RAGGED || at(ps) < p.k) rv[st][ps] = load_vec<T, VEC, !RAGGED>(r + at(ps));
+            if (EXACT || CLAMP || at(ps) < p.k) rv[st][ps] = load_vec<T, VEC, !RAGGED>(r + at(ps));
           }
         }
         float res = 0.f;
@@ -165,10 +169,10 @@ __global__ __launch_bounds__(256) void sddmm_kernel(SddmmParams p) {
           float acc = 0.f;
 #pragma unroll
           for (int ps = 0; ps < PASSES; ++ps) {
-            if constexpr (RAGGED) {
+            if constexpr (CLAMP) {
               if (ps == PASSES - 1) mask.apply(rv[st][ps]);
             }
-            if (EXACT || RAGGED || at(ps) < p.k) acc = dot_vec<T, VEC>(lfrag[ps], rv[st][ps], acc);
+            if (EXACT || CLAMP || at(ps) < p.k) acc = dot_vec<T, VEC>(lfrag[ps], rv[st][ps], acc);
           }
           acc = group_sum<LPN>(acc);
           res = (sl == st) ? acc : res;
@@ -284,16 +288,22 @@ int launch_typed(const SddmmParams& p, int wpr, hipStream_t stream) {
 // the dense GEMM computes all m * n dot products on the matrix cores in less time than that takes
 // once the mask is not very sparse, and a small kernel then picks the nonzeros' entries.
 // Same arithmetic per output (fp32 accumulation over k, one rounding to the 16-bit type).
+// WIDE: a workgroup per row instead of a wavefront (rows of hundreds of nonzeros: their chain of steps is what few rows wait for).
+template <bool WIDE>
 __global__ __launch_bounds__(256) void sample_dense_kernel(int m, int ld, const int* __restrict__ row_offsets,
                                                            const int* __restrict__ cols,
                                                            const uint16_t* __restrict__ dense,
                                                            uint16_t* __restrict__ out) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int row = WIDE ? (int)blockIdx.x : (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
   if (row >= m) return;
   const int start = row_offsets[row], end = row_offsets[row + 1];
   const uint16_t* drow = dense + (size_t)row * ld;
-  for (int j = start + lane_id(); j < end; j += kWave) out[j] = drow[cols[j]];
+  for (int j = start + (WIDE ? (int)threadIdx.x : lane_id()); j < end; j += WIDE ? 256 : kWave) out[j] = drow[cols[j]];
 }
+
+// us of the whole product, a wavefront / a workgroup per row: 1128 x 10508 at 81 %, k = 248 45 / 33; 424 x 9043 at 88 %, k = 685 41 / 34; 696 x 2192 at 88 %, k = 248 11.8 / 10.4;
+// 4680 x 2144 at 88 %, k = 112 21.8 / 22.7
+inline bool sample_wide(const SddmmParams& p) { return p.nnz >= (p.m <= 2048 ? 128ll : 256ll) * p.m; }
 
 inline bool sddmm_dense_fits(int dtype, const SddmmParams& p) {
   return (dtype == IEX_F16 || dtype == IEX_BF16) && !p.accumulate && !(p.sum_over_batch && p.batch > 1) && p.k > 0 &&
@@ -309,24 +319,27 @@ inline size_t sddmm_dense_bytes(const SddmmParams& p) {
   return sddmm_dense_pads(p) ? sddmm_dense_rhs_offset(p) + (size_t)p.n * round8(p.k) * 2 : (size_t)p.m * round8(p.n) * 2;
 }
 
-// Time model fitted on MI355X (fp16).  Dense product per batch entry: three launches, the GEMM at
+// Time model fitted on MI355X (fp16).  Dense product per batch entry: two launches, the GEMM at
 // 1000 TFLOP/s or, with few tiles, 0.23 us per K step of 32 per round of 512 tiles of 128 x 128,
-// m * n * 2 bytes written and nnz entries picked at 4 TB/s.  Gather kernel: nnz * k * 2 bytes at
-// 15 TB/s (16 heads of 4096 x 4096 at 93 % sparsity, k = 64: 125 us; 2048 x 1024 at 80 %, k = 2048:
-// 117 us), and with a k beyond the register-resident fragments no less than one wave's chain of
+// m * n * 2 bytes written and nnz entries picked at 4 TB/s, two more launches where the operands are copied.  Gather kernel: nnz * k * 2 bytes at
+// 14 TB/s, at 9 (13 in registers) or 7 where rows start at odd multiples of 4 or 2 bytes, and half of that for k of a few dozen; with a k beyond the register-resident
+// fragments no less than one wave's chain of
 // loads (0.12 us per 128 elements of k and step of 4 nonzeros with four slices in flight:
-// 1024 x 1024 at 95 %, k = 4096: 50 us).  Measured: 11008 x 4096 at 80 %, k = 8192 (weight gradient of an MLP
-// projection) 16.5 -> 0.77 ms; 4096 x 4096 at 50 %, k = 8192 9.7 -> 0.32 ms; 4096 x 4096 at 90 %,
-// k = 512 120 -> 55 us.  The dense product has to win by 15 %.
+// 1024 x 1024 at 95 %, k = 4096: 50 us).  Us, gather / dense product: 11008 x 4096 at 80 %, k = 8192 (weight gradient of an MLP
+// projection) 16500 / 770; 4096 x 4096 at 90 %, k = 512 120 / 55; at either side of the line 1056 x 3184 at 80 %, k = 152 22.5 / 12.7; 1168 x 1248 at 81 %, k = 192 11.7 / 9.5;
+// 534 x 3173 at 88 %, k = 104 7.9 / 12.1; 696 x 2192 at 88 %, k = 248 10.8 / 10.4; 3304 x 494 at 90 %, k = 563 30 / 19; 1120 x 2184 at 80 %, k = 241 27 / 18; 422 x 2632 at 95 %, k = 667 16 / 20;
+// 958 x 2305 at 95 %, k = 438 12 / 23; 1529 x 6000 at 92 %, k = 242 27 / 33; 5472 x 7472 at 81 %, k = 23 109 / 47; 5043 x 4044 at 80 %, k = 26 30 / 40.  The dense product has to win by 15 %.
 inline bool sddmm_dense_wins(const SddmmParams& p) {
   const double flops = 2.0 * p.m * p.n * p.k;
   const double tiles = (double)ceil_div(p.m, 128) * ceil_div(p.n, 128);
   const double product = std::max(flops / 1000e12, std::ceil(tiles / 512.0) * (p.k / 32.0) * 0.23e-6);
-  const double pad = sddmm_dense_pads(p) ? 8e-6 + 4.0 * ((double)p.m + p.n) * p.k / 4e12 : 0.0;
-  const double dense = p.batch * (16e-6 + pad + product + ((double)p.m * p.n * 2 + (double)p.nnz * 8) / 4e12);
+  const double pad = sddmm_dense_pads(p) ? 7e-6 + 4.0 * ((double)p.m + p.n) * p.k / 4e12 : 0.0;
   const double row_nnz = (double)p.nnz / p.m;
+  const double sample = (p.nnz * 8.0) / 4e12 + row_nnz / (sample_wide(p) ? 256 : 64) * 0.35e-6;
+  const double dense = p.batch * (8.5e-6 + pad + product + (double)p.m * p.n * 2 / 4e12 + sample);
   const double chain = p.k > 256 ? std::ceil(row_nnz / (row_nnz >= 64.0 ? 16.0 : 4.0)) * (p.k / 128.0) * 0.12e-6 : 0.0;
-  const double gather = std::max(8e-6 + (double)p.batch * p.nnz * p.k * 2 / 15e12, chain);
+  const double rate = p.k % 4 == 0 ? 14e12 : p.k % 2 == 0 ? (p.k >= 64 && p.k <= 256 ? 13e12 : 9e12) : p.k < 64 ? 4e12 : 7e12;
+  const double gather = std::max(4e-6 + (double)p.batch * p.nnz * p.k * 2 / rate, chain);
   return 1.15 * dense < gather;
 }
 
@@ -348,8 +361,9 @@ int launch_sddmm_dense(int dtype, const SddmmParams& p, void* ws, hipStream_t st
     g.ldc = ld;
     if (int rc = gemm_dispatch(dtype, 1, g, 1, stream)) return rc;
     note_kernel("sample_dense_kernel");
-    hipLaunchKernelGGL(sample_dense_kernel, dim3(ceil_div(p.m, 4)), dim3(256), 0, stream, p.m, ld, p.row_offsets, p.cols,
-                       static_cast<const uint16_t*>(ws), static_cast<uint16_t*>(p.out) + (size_t)z * p.nnz);
+    uint16_t* out = static_cast<uint16_t*>(p.out) + (size_t)z * p.nnz;
+    if (sample_wide(p)) hipLaunchKernelGGL(sample_dense_kernel<true>, dim3(p.m), dim3(256), 0, stream, p.m, ld, p.row_offsets, p.cols, static_cast<const uint16_t*>(ws), out);
+    else hipLaunchKernelGGL(sample_dense_kernel<false>, dim3(ceil_div(p.m, 4)), dim3(256), 0, stream, p.m, ld, p.row_offsets, p.cols, static_cast<const uint16_t*>(ws), out);
     if (int rc = check_hip(hipGetLastError(), "sddmm sampling launch")) return rc;
   }
   return 0;

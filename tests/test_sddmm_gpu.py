@@ -313,3 +313,36 @@ def test_rows_of_no_whole_vectors(oracle, dev, dtype, k):
     assert_close(ops.sddmm_sputnik_half(odd, rt, ri, ro, ci).float().cpu().numpy(), want, scale, RTOL[dtype], f"k={k}, unaligned")
     rt[0, :, k - 1] = float("inf")
     assert not torch.isnan(ops.sddmm_sputnik_half(lt, rt, ri, ro, ci)).any()
+
+
+@pytest.mark.parametrize("k", [9, 24, 40, 72, 136, 184, 248])   # one or two vectors a lane, the last past the row's end or of it
+@pytest.mark.parametrize("mean", [20, 90])                      # a wavefront to a row, four
+def test_bf16_vectors_past_a_row_read_nothing_of_the_next(oracle, dev, k, mean):
+    rng = np.random.default_rng(k)
+    m, n = 65, 130
+    lens = rng.integers(mean - 15, mean + 15, m)
+    ro, ci = W.csr_from_row_lengths(rng, m, n, lens)
+    csr = W.CSR(m, n, np.ones(ci.shape[0], np.float32), W.swizzle_from_offsets(ro), ro, ci)
+    lhs = rng.standard_normal((1, m, k)).astype(np.float32)
+    rhs = rng.standard_normal((1, n, k)).astype(np.float32)
+    _check(oracle, csr, lhs, rhs, dev, torch.bfloat16, False, f"bf16 k={k}")
+    ri, _, ro_t, ci_t = to_dev(csr, dev, torch.bfloat16)
+    a, b = (torch.from_numpy(x).to(dev).bfloat16() for x in (lhs, rhs))
+    clean = ops.sddmm_sputnik_half(a, b, ri, ro_t, ci_t)
+    rows = torch.repeat_interleave(torch.arange(m, device=dev), (ro_t[1:] - ro_t[:-1]).long())
+    a[0, 7], b[0, 11] = float("inf"), float("nan")
+    got = ops.sddmm_sputnik_half(a, b, ri, ro_t, ci_t)
+    others = (rows != 7) & (ci_t.long() != 11)
+    assert torch.equal(got[0][others], clean[0][others]) and not got[0][~others].isfinite().any()
+
+
+@pytest.mark.parametrize("m,n,k,density,dense", [(1120, 2184, 241, 0.2, True), (560, 2400, 957, 0.17, True), (1100, 3200, 152, 0.2, True), (600, 3100, 104, 0.12, False), (960, 2300, 438, 0.05, False)])
+def test_the_dense_product_is_taken_where_gathers_take_longer(oracle, dev, m, n, k, density, dense):
+    from intrasm_engine_amd import _lib
+    rng = np.random.default_rng(m)
+    ro, ci = W.csr_from_row_lengths(rng, m, n, np.full(m, int(n * density)))     # (over and under the rows that get a workgroup each behind the product)
+    csr = W.CSR(m, n, np.ones(ci.shape[0], np.float32), W.swizzle_from_offsets(ro), ro, ci)
+    lhs = rng.standard_normal((1, m, k)).astype(np.float32)
+    rhs = rng.standard_normal((1, n, k)).astype(np.float32)
+    _check(oracle, csr, lhs, rhs, dev, torch.float16, False, f"{m} x {n} x {k}")
+    assert ("sample_dense_kernel" in _lib.last_kernels()) == dense, _lib.last_kernels()
