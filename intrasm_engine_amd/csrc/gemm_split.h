@@ -27,12 +27,12 @@ struct SplitSparse {
   long long plane;
   void* dst;
 };
-// Every workgroup leaves the largest magnitude it met, as its bits: at largest[0 ..] those of the second operand (a dense one), from
-// largest[kSplitSlots] on those of the first.  How many there are:
+// Every workgroup leaves the range of the entries it met, a SplitRange as a word: at ranges[0 ..] those of the second operand (a dense one), from
+// ranges[kSplitSlots] on those of the first.  How many there are:
 int split_dense_blocks(const SplitDense& s);
 int split_sparse_blocks(const SplitSparse& s);
-int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* largest, hipStream_t stream);
-int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* largest, hipStream_t stream);
+int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* ranges, hipStream_t stream);
+int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* ranges, hipStream_t stream);
 
 // C = A * B, or with K in parts (gemm_split_parts: more than one) part s's share of it at C + s * stride_part, which the caller adds up.
 struct SplitParams {
@@ -60,17 +60,39 @@ struct SplitSample {
   const float* scores;
   const float *lhs, *rhs;   // (batch, m, k), (batch, n, k)
   float* out;
-  const unsigned* largest;
+  const unsigned* ranges;
   int slots_a, slots_b;
 };
 int launch_split_sample(const SplitSample& s, hipStream_t stream);
 
-// From the largest magnitudes of both operands: whether the parts of every entry and product lie inside fp32's normal range (no
-// infinities or NaN either), so that the product of the parts stands for the fp32 one.
-__device__ __forceinline__ bool split_range_ok(unsigned a, unsigned b) {
-  const unsigned inf = 0x7f800000u, least = 37u << 23;   // 2^-90
-  if (a == 0u || b == 0u) return a < inf && b < inf;
-  if (a >= inf || b >= inf || a < least || b < least) return false;
+__device__ __forceinline__ unsigned magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
+// What is known of an operand's entries: the largest finite magnitude, as its bits, and whether there was an infinity or a NaN.
+struct SplitRange {
+  unsigned most = 0;
+  unsigned odd = 0;   // 0 or 1 << 31
+  __device__ __forceinline__ void add(float x) {
+    const unsigned size = magnitude(x);
+    if (size >= 0x7f800000u) odd = 1u << 31;
+    else most = max(most, size);
+  }
+  __device__ __forceinline__ unsigned word() const { return most | odd; }
+  __device__ __forceinline__ void add_word(unsigned w) {
+    most = max(most, w & 0x7fffffffu);
+    odd |= w & (1u << 31);
+  }
+  __device__ __forceinline__ void over_wave() {
+#pragma unroll
+    for (int d = 32; d; d >>= 1) add_word((unsigned)__shfl_xor((int)word(), d));
+  }
+};
+
+// Whether the largest entries of both operands and their product lie inside fp32's normal range, so that the product of the parts of finite
+// entries stands for the fp32 one.
+__device__ __forceinline__ bool split_range_ok(const SplitRange& of_a, const SplitRange& of_b) {
+  const unsigned a = of_a.most, b = of_b.most, least = 37u << 23;   // 2^-90
+  if (a == 0u || b == 0u) return true;
+  if (a < least || b < least) return false;
   const int ea = (int)(a >> 23) - 127, eb = (int)(b >> 23) - 127;
   return ea + eb > -80 && ea + eb < 90 && ea < 126 && eb < 126;
 }

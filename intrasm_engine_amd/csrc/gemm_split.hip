@@ -33,32 +33,24 @@ __device__ __forceinline__ void store_parts(const float (&x)[8], uint16_t* dst, 
   *reinterpret_cast<u32x4*>(dst + 2 * plane) = l;
 }
 
-__device__ __forceinline__ unsigned magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
-
-__device__ __forceinline__ unsigned wave_largest(unsigned x) {
-#pragma unroll
-  for (int d = 32; d; d >>= 1) x = max(x, (unsigned)__shfl_xor((int)x, d));
-  return x;
-}
-
 template <int WAVES>
-__device__ __forceinline__ void leave_largest(unsigned x, unsigned* at) {
-  __shared__ unsigned most[WAVES];
-  x = wave_largest(x);
-  if (lane_id() == 0) most[threadIdx.x >> 6] = x;
+__device__ __forceinline__ void leave_range(SplitRange x, unsigned* at) {
+  __shared__ unsigned of[WAVES];
+  x.over_wave();
+  if (lane_id() == 0) of[threadIdx.x >> 6] = x.word();
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) x = max(x, most[w]);
-    *at = x;
+    for (int w = 0; w < WAVES; ++w) x.add_word(of[w]);
+    *at = x.word();
   }
 }
 
-__device__ __forceinline__ unsigned split_dense_block(const SplitDense& s, int block, int blocks) {
+__device__ __forceinline__ SplitRange split_dense_block(const SplitDense& s, int block, int blocks) {
   struct alignas(4) Any { float v[8]; };
   const int chunks = s.dst_cols / 8;
   const long long total = (long long)s.batch * s.dst_rows * chunks;
-  unsigned largest = 0;
+  SplitRange range;
   for (long long i = (long long)block * 256 + threadIdx.x; i < total; i += (long long)blocks * 256) {
     const long long zr = i / chunks;
     const int c = (int)(i - zr * chunks) * 8;
@@ -74,22 +66,22 @@ __device__ __forceinline__ unsigned split_dense_block(const SplitDense& s, int b
       for (int e = 0; e < 8; ++e) x[e] = r < s.rows && c + e < s.cols ? src[e] : 0.f;
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) largest = max(largest, magnitude(x[e]));
+    for (int e = 0; e < 8; ++e) range.add(x[e]);
     store_parts(x, static_cast<uint16_t*>(s.dst) + (size_t)z * s.dst_batch + (size_t)r * s.ld + c, s.plane);
   }
-  return largest;
+  return range;
 }
 
 // As csr_to_dense_kernel (spmm_dense_device.cuh): a workgroup per row, the row (or 4096 columns of it) assembled in LDS in fp32, its parts taken on
 // the way out, every byte written once.  (4096 x 4096: 27 us, of which 20 are the bytes; two rows side by side the same, four 40.)
 constexpr int kPlanesSeg = 4096, kPlanesRows = 1, kPlanesWaves = 4;
-__device__ __forceinline__ unsigned split_sparse_block(const SplitSparse& s, int block, int blocks) {
+__device__ __forceinline__ SplitRange split_sparse_block(const SplitSparse& s, int block, int blocks) {
   __shared__ __align__(16) float srow[kPlanesRows][kPlanesSeg];
   const int lane = lane_id(), wave = uniform(threadIdx.x >> 6);
   const int* __restrict__ cols = s.cols;
   const float* __restrict__ values = s.values;
   uint16_t* __restrict__ dst = static_cast<uint16_t*>(s.dst);
-  unsigned most = 0;
+  SplitRange range;
   bool again = false;
   for (int slot0 = block * kPlanesRows; slot0 < s.m; slot0 += blocks * kPlanesRows) {
     int pos[kPlanesRows], end[kPlanesRows];   // this wavefront's quarter of each row's nonzeros, in whole chunks of 64
@@ -133,7 +125,7 @@ __device__ __forceinline__ unsigned split_sparse_block(const SplitSparse& s, int
             const bool mine = more[r] && pos[r] + u * kWave + lane < end[r] && c[r][u] < len && c[r][u] >= 0;
             if (mine) {
               srow[r][c[r][u]] = v[r][u];
-              most = max(most, magnitude(v[r][u]));
+              range.add(v[r][u]);
             }
             taken += __popcll(__ballot(mine));
           }
@@ -152,44 +144,43 @@ __device__ __forceinline__ unsigned split_sparse_block(const SplitSparse& s, int
           }
     }
   }
-  return most;
+  return range;
 }
 
 // Both operands' parts in one launch: the first workgroups make those of the second operand.  Bound by the bytes, 4 read and 6 written an entry, 6
-// written a cell of a sparse operand.  (A maximum per workgroup, not atomics: 8192 of them on 64 words took 25 us.)
+// written a cell of a sparse operand.  (A word per workgroup, not atomics: 8192 of them on 64 words took 25 us.)
 template <typename First>
-__global__ __launch_bounds__(256) void split_operands_kernel(First a, SplitDense b, unsigned* largest, int blocks_b) {
+__global__ __launch_bounds__(256) void split_operands_kernel(First a, SplitDense b, unsigned* ranges, int blocks_b) {
   if ((int)blockIdx.x < blocks_b) {
-    leave_largest<4>(split_dense_block(b, blockIdx.x, blocks_b), largest + blockIdx.x);
+    leave_range<4>(split_dense_block(b, blockIdx.x, blocks_b), ranges + blockIdx.x);
   } else {
     const int block = blockIdx.x - blocks_b, blocks = gridDim.x - blocks_b;
-    unsigned most;
-    if constexpr (std::is_same<First, SplitSparse>::value) most = split_sparse_block(a, block, blocks);
-    else most = split_dense_block(a, block, blocks);
-    leave_largest<4>(most, largest + kSplitSlots + block);
+    SplitRange range;
+    if constexpr (std::is_same<First, SplitSparse>::value) range = split_sparse_block(a, block, blocks);
+    else range = split_dense_block(a, block, blocks);
+    leave_range<4>(range, ranges + kSplitSlots + block);
   }
 }
 
 // A wavefront per row.  A score that is not finite (an infinity's parts give NaN) is computed as the dot product itself, by
-// the whole wavefront, and so are all where the operands' largest entries say that parts may have left fp32's normal range.
+// the whole wavefront, and so are all where the operands' largest finite entries say that parts may have left fp32's normal range.
 __global__ __launch_bounds__(256) void split_sample_kernel(SplitSample s) {
   const int row = blockIdx.x * 4 + uniform(threadIdx.x >> 6), lane = lane_id();
   if (row >= s.m) return;
   const int start = s.row_offsets[row], end = s.row_offsets[row + 1];
-  unsigned of_a = 0, of_b = 0;
+  SplitRange of_a, of_b;
   for (int i = lane; i < kSplitSlots; i += kWave) {
-    if (i < s.slots_a) of_a = max(of_a, s.largest[kSplitSlots + i]);
-    if (i < s.slots_b) of_b = max(of_b, s.largest[i]);
+    if (i < s.slots_a) of_a.add_word(s.ranges[kSplitSlots + i]);
+    if (i < s.slots_b) of_b.add_word(s.ranges[i]);
   }
-  of_a = wave_largest(of_a), of_b = wave_largest(of_b);
-  const bool all = max(of_a, of_b) < 0x7f800000u && !split_range_ok(of_a, of_b);   // (wave-uniform)
+  of_a.over_wave(), of_b.over_wave();
+  const bool all = !split_range_ok(of_a, of_b);   // (wave-uniform)
   const float* scores = s.scores + (size_t)row * s.ld;
   for (int j0 = start; j0 < end; j0 += kWave) {
     const int j = min(j0 + lane, end - 1), col = s.cols[j];
     float x = scores[col];
     for (int part = 1; part < s.parts; ++part) x += scores[(size_t)part * s.stride_part + col];
-    const unsigned size = magnitude(x);
-    unsigned long long odd = __ballot(j0 + lane < end && (all || size >= 0x7f800000u));
+    unsigned long long odd = __ballot(j0 + lane < end && (all || magnitude(x) >= 0x7f800000u));
     while (odd) {
       const int src = __ffsll(odd) - 1;
       odd &= odd - 1;
@@ -246,10 +237,10 @@ int launch_product(const SplitParams& p, int batch, hipStream_t stream) {
 }
 
 template <typename First>
-int launch_operands(const First& a, int blocks_a, const SplitDense& b, unsigned* largest, hipStream_t stream) {
+int launch_operands(const First& a, int blocks_a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
   const int blocks_b = split_dense_blocks(b);
   note_kernel("split_operands_kernel");
-  hipLaunchKernelGGL(split_operands_kernel<First>, dim3(blocks_a + blocks_b), dim3(256), 0, stream, a, b, largest, blocks_b);
+  hipLaunchKernelGGL(split_operands_kernel<First>, dim3(blocks_a + blocks_b), dim3(256), 0, stream, a, b, ranges, blocks_b);
   return check_hip(hipGetLastError(), "parts of the operands, launch");
 }
 
@@ -286,11 +277,11 @@ int split_dense_blocks(const SplitDense& s) {
   return (int)std::min<long long>(kSplitSlots, (chunks + 255) / 256);
 }
 int split_sparse_blocks(const SplitSparse& s) { return std::min(kSplitSparseSlots, ceil_div(s.m, kPlanesRows)); }
-int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* largest, hipStream_t stream) {
-  return launch_operands(a, split_sparse_blocks(a), b, largest, stream);
+int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
+  return launch_operands(a, split_sparse_blocks(a), b, ranges, stream);
 }
-int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* largest, hipStream_t stream) {
-  return launch_operands(a, split_dense_blocks(a), b, largest, stream);
+int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
+  return launch_operands(a, split_dense_blocks(a), b, ranges, stream);
 }
 int launch_split_sample(const SplitSample& s, hipStream_t stream) {
   note_kernel("split_sample_kernel");

@@ -406,11 +406,11 @@ inline bool sddmm_split_wins(const SddmmParams& p) {
 int launch_sddmm_split(const SddmmParams& p, void* workspace, hipStream_t stream) {
   const SddmmSplit s = sddmm_split_plan(p);
   unsigned char* ws = static_cast<unsigned char*>(workspace);
-  unsigned* largest = reinterpret_cast<unsigned*>(ws);
+  unsigned* ranges = reinterpret_cast<unsigned*>(ws);
   const long long plane_a = (long long)p.m * s.K, plane_b = (long long)p.n * s.K;
   const SplitDense a{p.batch, p.m, p.k, static_cast<const float*>(p.lhs), p.m, s.kp, s.K, s.kp, plane_a, ws + s.lhs_at};
   const SplitDense b{p.batch, p.n, p.k, static_cast<const float*>(p.rhs), p.n, s.kp, s.K, s.kp, plane_b, ws + s.rhs_at};
-  if (int rc = launch_split_operands(a, b, largest, stream)) return rc;
+  if (int rc = launch_split_operands(a, b, ranges, stream)) return rc;
   SplitParams g{};
   g.M = p.m, g.N = p.n, g.K = s.K;
   g.A = a.dst, g.B = b.dst, g.C = reinterpret_cast<float*>(ws + s.scores_at);
@@ -419,7 +419,7 @@ int launch_sddmm_split(const SddmmParams& p, void* workspace, hipStream_t stream
   g.stride_part = (long long)p.m * s.ld;
   if (int rc = gemm_split(g, true, 1, stream)) return rc;
   const SplitSample q{p.m, p.k, p.n, p.batch, s.ld, s.parts, g.stride_part, p.row_offsets, p.cols, g.C, static_cast<const float*>(p.lhs), static_cast<const float*>(p.rhs),
-                      static_cast<float*>(p.out), largest, split_dense_blocks(a), split_dense_blocks(b)};
+                      static_cast<float*>(p.out), ranges, split_dense_blocks(a), split_dense_blocks(b)};
   return launch_split_sample(q, stream);
 }
 

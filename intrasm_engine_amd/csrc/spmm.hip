@@ -886,7 +886,7 @@ struct SplitPlan {
   int kp, np, parts, ld;   // ld: rows of the parts' sums
   size_t a_at, b_at, sums_at, bytes;
 };
-// the workspace: the operands' largest magnitudes, planes of A, planes of B, sums of the parts of K
+// the workspace: the ranges of the operands' entries, planes of A, planes of B, sums of the parts of K
 inline SplitPlan split_plan(const SpmmParams& p, int batch) {
   SplitPlan s;
   s.kp = round32(p.k);
@@ -937,23 +937,19 @@ inline bool split_path_wins(const SpmmParams& p, int batch) {
 // dense form's zeros) spreads, or lies outside the range in which parts hold all 24 bits, computes it once more as the row kernel does:
 // results there are the row kernel's.  With K in one part it ends at once else (2 us).
 constexpr int kFinishBlocks = 1024;
-__global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, const unsigned* largest, int slots_a, int slots_b, const float* sums, int parts, int ld,
+__global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, const unsigned* ranges, int slots_a, int slots_b, const float* sums, int parts, int ld,
                                                                int tiles, int batch) {
   __shared__ float red[spmm_lds_floats<4, 4, 1>()];
-  __shared__ unsigned most[2][4];
-  unsigned of_a = 0, of_b = 0;
-  for (int i = threadIdx.x; i < slots_b; i += 256) of_b = max(of_b, largest[i]);
-  for (int i = threadIdx.x; i < slots_a; i += 256) of_a = max(of_a, largest[kSplitSlots + i]);
-#pragma unroll
-  for (int d = 32; d; d >>= 1) {
-    of_b = max(of_b, (unsigned)__shfl_xor((int)of_b, d));
-    of_a = max(of_a, (unsigned)__shfl_xor((int)of_a, d));
-  }
-  if (lane_id() == 0) most[0][threadIdx.x >> 6] = of_a, most[1][threadIdx.x >> 6] = of_b;
+  __shared__ unsigned of[2][4];
+  SplitRange of_a, of_b;
+  for (int i = threadIdx.x; i < slots_b; i += 256) of_b.add_word(ranges[i]);
+  for (int i = threadIdx.x; i < slots_a; i += 256) of_a.add_word(ranges[kSplitSlots + i]);
+  of_a.over_wave(), of_b.over_wave();
+  if (lane_id() == 0) of[0][threadIdx.x >> 6] = of_a.word(), of[1][threadIdx.x >> 6] = of_b.word();
   __syncthreads();
-  of_a = max(max(most[0][0], most[0][1]), max(most[0][2], most[0][3]));
-  of_b = max(max(most[1][0], most[1][1]), max(most[1][2], most[1][3]));
-  if (!split_range_ok(of_a, of_b)) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) of_a.add_word(of[0][w]), of_b.add_word(of[1][w]);
+  if (of_a.odd || of_b.odd || !split_range_ok(of_a, of_b)) {
     const long long total = (long long)p.m * tiles * batch;
     for (long long i = blockIdx.x; i < total; i += gridDim.x) {
       const int row = (int)(i % p.m), rest = (int)(i / p.m);
@@ -991,12 +987,12 @@ __global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, co
 inline int launch_split_path(const SpmmParams& p, int batch, void* workspace, hipStream_t stream) {
   const SplitPlan s = split_plan(p, batch);
   unsigned char* ws = static_cast<unsigned char*>(workspace);
-  unsigned* largest = reinterpret_cast<unsigned*>(ws);
+  unsigned* ranges = reinterpret_cast<unsigned*>(ws);
   float* sums = reinterpret_cast<float*>(ws + s.sums_at);
   const long long plane_a = (long long)p.m * s.kp, plane_b = (long long)s.kp * s.np;
   const SplitSparse a{p.m, s.kp, p.row_offsets, static_cast<const int*>(p.cols), static_cast<const float*>(p.values), plane_a, ws + s.a_at};
   const SplitDense b{batch, p.k, p.n, static_cast<const float*>(p.dense), s.kp, s.np, s.np, 3 * plane_b, plane_b, ws + s.b_at};
-  if (int rc = launch_split_operands(a, b, largest, stream)) return rc;
+  if (int rc = launch_split_operands(a, b, ranges, stream)) return rc;
   SplitParams g{};
   g.M = p.m, g.N = p.n, g.K = s.kp;
   g.A = ws + s.a_at, g.B = ws + s.b_at;
@@ -1013,7 +1009,7 @@ inline int launch_split_path(const SpmmParams& p, int batch, void* workspace, hi
   note_kernel("spmm_split_finish_kernel");
   const int tiles = ceil_div(p.n, kWave * 4);
   const long long work = s.parts > 1 ? ((long long)p.m * batch * (s.ld / 4) + 255) / 256 : (long long)p.m * tiles * batch;
-  hipLaunchKernelGGL(spmm_split_finish_kernel, dim3((unsigned)std::min<long long>(s.parts > 1 ? kFinishBlocks : kFinishBlocks / 4, work)), dim3(256), 0, stream, p, largest,
+  hipLaunchKernelGGL(spmm_split_finish_kernel, dim3((unsigned)std::min<long long>(s.parts > 1 ? kFinishBlocks : kFinishBlocks / 4, work)), dim3(256), 0, stream, p, ranges,
                      split_sparse_blocks(a), split_dense_blocks(b), sums, s.parts, s.ld, tiles, batch);
   return check_hip(hipGetLastError(), "spmm (fp32 by parts) launch");
 }

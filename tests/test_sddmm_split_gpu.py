@@ -68,6 +68,26 @@ def test_entries_outside_the_range_of_the_parts(of_lhs, of_rhs):
     assert error(sampled(args, 12), args) <= max(1.05 * error(sampled(args, 1), args), 8e-8)
 
 
+@pytest.mark.parametrize("what", [float("inf"), float("nan")])
+@pytest.mark.parametrize("of_lhs,of_rhs", [(1e-36, 1.0), (1.0, 1e-36), (1e-20, 1e-15), (1e25, 1e10)])
+def test_an_infinity_beside_entries_outside_the_range(what, of_lhs, of_rhs):
+    """The finite scores are the dot products themselves, as where there is no infinity."""
+    lhs, rhs, *pattern = operands(200, 150, 300, 0.2, seed=4)
+    clean = (lhs * of_lhs, rhs * of_rhs, *pattern)
+    args = (clean[0].clone(), clean[1].clone(), *pattern)
+    args[0][0, 7, 3] = what
+    args[1][0, 40, 9] = what
+    got, want = sampled(args, 12), sampled(args, 1)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    fine = want.isfinite()
+    _, _, _, row_offsets, columns = clean
+    rows = torch.repeat_interleave(torch.arange(200, device="cuda"), (row_offsets[1:] - row_offsets[:-1]).long())
+    exact = torch.matmul(clean[0][0].double(), clean[1][0].double().t().contiguous())[rows, columns.long()][fine]
+    of = lambda x: float((x[fine].double() - exact).norm() / exact.norm())
+    # (two fp32 chains over the same 300 terms, cut differently)
+    assert of(got) <= max(1.5 * of(want), 1.2e-7)
+
+
 def test_where_it_is_taken_and_where_not():
     args = operands(2000, 1500, 700, 0.2, seed=5)
     lhs, rhs, row_indices, row_offsets, columns = args
