@@ -91,7 +91,7 @@ struct SplitRange {
 // entries stands for the fp32 one.
 __device__ __forceinline__ bool split_range_ok(const SplitRange& of_a, const SplitRange& of_b) {
   const unsigned a = of_a.most, b = of_b.most, least = 37u << 23;   // 2^-90
-  if (a == 0u || b == 0u) return true;
+  if (a == 0u || b == 0u) return max(a, b) < 253u << 23;   // (beyond 2^126 a part may be an infinity, and its product with zero a NaN)
   if (a < least || b < least) return false;
   const int ea = (int)(a >> 23) - 127, eb = (int)(b >> 23) - 127;
   return ea + eb > -80 && ea + eb < 90 && ea < 126 && eb < 126;

@@ -101,6 +101,15 @@ def test_entries_outside_the_range_of_the_parts(of_values, of_dense):
     assert error(got, w, b) <= max(1.05 * error(want, w, b), 1.2e-7)
 
 
+def test_stored_zeros_beside_entries_that_round_to_an_infinity():
+    m, k, n = 130, 64, 40
+    w, csr, b = operands(m, k, n, 0.3, seed=9)
+    csr = (torch.zeros_like(csr[0]), *csr[1:])
+    b[0, 3, 7] = 3.4e38
+    got = product(csr, b, m, 12)
+    assert "gemm_split_kernel" in _lib.last_kernels() and not got.any()
+
+
 def test_where_it_is_taken_and_where_not():
     w, csr, b = operands(2048, 2048, 512, 0.2, seed=5)
     values, row_indices, row_offsets, columns = csr
