@@ -164,8 +164,8 @@ int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream);
  * six products of parts that reach into an fp32 result on the bf16 matrix cores (iex_spmm_ws only; chosen by itself for
  * large fp32 products with IEX_SPMM_PAD_OPERANDS, values shared by the batch, plain store, canonical CSR).  Its error against 64 bits is below that of a chain of
  * fp32 multiply-adds.  Where an operand holds an infinity or a NaN, or its entries are too large or small for the parts to be exact
- * (largest magnitude outside 2^-90 .. 2^125, product of both outside 2^-80 .. 2^90), the row kernel computes the call instead;
- * beside larger ones, entries below 2^-110 keep fewer bits.  Where it cannot run (no workspace, other types) the row kernel does.
+ * (a magnitude but zero outside 2^-110 .. 2^126, a product of two outside 2^-120 .. 2^90), the row kernel computes the call
+ * instead.  Where it cannot run (no workspace, other types) the row kernel does.
  * Families 2-6 and 10 rely on strictly ascending column indices inside a row (canonical CSR, what
  * dense_to_sparse produces); family 1 accepts any order and duplicates -- force it for such
  * input.  Families 3-6 and 10 multiply explicit zeros with the dense operand, so a non-finite entry

@@ -34,15 +34,15 @@ __device__ __forceinline__ void store_parts(const float (&x)[8], uint16_t* dst, 
 }
 
 template <int WAVES>
-__device__ __forceinline__ void leave_range(SplitRange x, unsigned* at) {
-  __shared__ unsigned of[WAVES];
+__device__ __forceinline__ void leave_range(SplitRange x, uint2* at) {
+  __shared__ uint2 of[WAVES];
   x.over_wave();
-  if (lane_id() == 0) of[threadIdx.x >> 6] = x.word();
+  if (lane_id() == 0) of[threadIdx.x >> 6] = x.words();
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) x.add_word(of[w]);
-    *at = x.word();
+    for (int w = 0; w < WAVES; ++w) x.add_words(of[w]);
+    *at = x.words();
   }
 }
 
@@ -148,9 +148,9 @@ __device__ __forceinline__ SplitRange split_sparse_block(const SplitSparse& s, i
 }
 
 // Both operands' parts in one launch: the first workgroups make those of the second operand.  Bound by the bytes, 4 read and 6 written an entry, 6
-// written a cell of a sparse operand.  (A word per workgroup, not atomics: 8192 of them on 64 words took 25 us.)
+// written a cell of a sparse operand.  (Two words per workgroup, not atomics: 8192 of them on 64 words took 25 us.)
 template <typename First>
-__global__ __launch_bounds__(256) void split_operands_kernel(First a, SplitDense b, unsigned* ranges, int blocks_b) {
+__global__ __launch_bounds__(256) void split_operands_kernel(First a, SplitDense b, uint2* ranges, int blocks_b) {
   if ((int)blockIdx.x < blocks_b) {
     leave_range<4>(split_dense_block(b, blockIdx.x, blocks_b), ranges + blockIdx.x);
   } else {
@@ -163,15 +163,15 @@ __global__ __launch_bounds__(256) void split_operands_kernel(First a, SplitDense
 }
 
 // A wavefront per row.  A score that is not finite (an infinity's parts give NaN) is computed as the dot product itself, by
-// the whole wavefront, and so are all where the operands' largest finite entries say that parts may have left fp32's normal range.
+// the whole wavefront, and so are all where the range of the operands' finite entries says that parts do not hold them.
 __global__ __launch_bounds__(256) void split_sample_kernel(SplitSample s) {
   const int row = blockIdx.x * 4 + uniform(threadIdx.x >> 6), lane = lane_id();
   if (row >= s.m) return;
   const int start = s.row_offsets[row], end = s.row_offsets[row + 1];
   SplitRange of_a, of_b;
   for (int i = lane; i < kSplitSlots; i += kWave) {
-    if (i < s.slots_a) of_a.add_word(s.ranges[kSplitSlots + i]);
-    if (i < s.slots_b) of_b.add_word(s.ranges[i]);
+    if (i < s.slots_a) of_a.add_words(s.ranges[kSplitSlots + i]);
+    if (i < s.slots_b) of_b.add_words(s.ranges[i]);
   }
   of_a.over_wave(), of_b.over_wave();
   const bool all = !split_range_ok(of_a, of_b);   // (wave-uniform)
@@ -237,7 +237,7 @@ int launch_product(const SplitParams& p, int batch, hipStream_t stream) {
 }
 
 template <typename First>
-int launch_operands(const First& a, int blocks_a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
+int launch_operands(const First& a, int blocks_a, const SplitDense& b, uint2* ranges, hipStream_t stream) {
   const int blocks_b = split_dense_blocks(b);
   note_kernel("split_operands_kernel");
   hipLaunchKernelGGL(split_operands_kernel<First>, dim3(blocks_a + blocks_b), dim3(256), 0, stream, a, b, ranges, blocks_b);
@@ -277,10 +277,10 @@ int split_dense_blocks(const SplitDense& s) {
   return (int)std::min<long long>(kSplitSlots, (chunks + 255) / 256);
 }
 int split_sparse_blocks(const SplitSparse& s) { return std::min(kSplitSparseSlots, ceil_div(s.m, kPlanesRows)); }
-int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
+int launch_split_operands(const SplitSparse& a, const SplitDense& b, uint2* ranges, hipStream_t stream) {
   return launch_operands(a, split_sparse_blocks(a), b, ranges, stream);
 }
-int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
+int launch_split_operands(const SplitDense& a, const SplitDense& b, uint2* ranges, hipStream_t stream) {
   return launch_operands(a, split_dense_blocks(a), b, ranges, stream);
 }
 int launch_split_sample(const SplitSample& s, hipStream_t stream) {

@@ -68,6 +68,21 @@ def test_entries_outside_the_range_of_the_parts(of_lhs, of_rhs):
     assert error(sampled(args, 12), args) <= max(1.05 * error(sampled(args, 1), args), 8e-8)
 
 
+@pytest.mark.parametrize("of_lhs,of_rhs", [(-126, 0), (0, -126), (-64, -64)])
+def test_rows_of_widely_different_scales(of_lhs, of_rhs):
+    lhs, rhs, *pattern = operands(128, 130, 300, 0.5, seed=11)
+    down = lambda rows, least: torch.exp2(-(torch.arange(rows, device="cuda").double() * 2).clamp(max=-least))[:, None].float()
+    args = (lhs * down(128, of_lhs), rhs * down(130, of_rhs), *pattern)
+    row_offsets, columns = pattern[1:]
+    rows = torch.repeat_interleave(torch.arange(128, device="cuda"), (row_offsets[1:] - row_offsets[:-1]).long())
+    pick = lambda x, y: torch.matmul(x[0].double(), y[0].double().t().contiguous())[rows, columns.long()]
+    exact, scale = pick(args[0], args[1]), pick(args[0].abs(), args[1].abs())
+    fine = scale >= 2.0 ** -120
+    of = lambda x: float(((x.double() - exact).abs() / scale)[fine].max())
+    # (2^-24 for each of 300 terms, were they all to add up)
+    assert of(sampled(args, 12)) <= max(1.05 * of(sampled(args, 1)), 2.0 ** -22)
+
+
 @pytest.mark.parametrize("what", [float("inf"), float("nan")])
 @pytest.mark.parametrize("of_lhs,of_rhs", [(1e-36, 1.0), (1.0, 1e-36), (1e-20, 1e-15), (1e25, 1e10)])
 def test_an_infinity_beside_entries_outside_the_range(what, of_lhs, of_rhs):

@@ -101,6 +101,22 @@ def test_entries_outside_the_range_of_the_parts(of_values, of_dense):
     assert error(got, w, b) <= max(1.05 * error(want, w, b), 1.2e-7)
 
 
+@pytest.mark.parametrize("of_rows,of_columns", [(-126, 0), (0, -126), (-64, -64), (-110, 0)])
+def test_rows_and_columns_of_widely_different_scales(of_rows, of_columns):
+    """Every row and column from 1 down to 2^of_rows and 2^of_columns in steps of two powers: each result beside its own row's and column's scale."""
+    m, k, n = 128, 320, 128
+    w, _, b = operands(m, k, n, 0.3, seed=10)
+    w *= torch.exp2(-(torch.arange(m, device="cuda").double() * 2).clamp(max=-of_rows))[:, None].float()
+    b *= torch.exp2(-(torch.arange(n, device="cuda").double() * 2).clamp(max=-of_columns)).float()
+    csr = dense_to_sparse(w)
+    got, want, exact = product(csr, b, m, 12)[0], product(csr, b, m, 1)[0], w.double() @ b[0].double()
+    # in fp32's normal range, each within rounding of the sum of its magnitudes: 2^-24 for each of some 100 terms, were they all to add up
+    scale = w.double().abs() @ b[0].double().abs()
+    fine = scale >= 2.0 ** -120
+    of = lambda x: float(((x.double() - exact).abs() / scale)[fine].max())
+    assert of(got) <= max(1.05 * of(want), 2.0 ** -22)
+
+
 def test_stored_zeros_beside_entries_that_round_to_an_infinity():
     m, k, n = 130, 64, 40
     w, csr, b = operands(m, k, n, 0.3, seed=9)
