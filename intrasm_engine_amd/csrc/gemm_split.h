@@ -7,6 +7,8 @@ namespace iex {
 constexpr int kSplitSlots = 512;         // workgroups that make a dense operand's parts, at most
 constexpr int kSplitSparseSlots = 2048;  // ... a sparse one's
 
+constexpr int kSplitVerdict = kSplitSlots + kSplitSparseSlots, kSplitRanges = kSplitVerdict + 64;   // (whole 256 bytes)
+
 inline int round32(int x) { return (x + 31) & ~31; }
 
 // src (batch x rows x cols, fp32, at element alignment) as three planes of bf16: high, middle and low parts.  Entry (z, r, c) of a plane lies at
@@ -27,12 +29,13 @@ struct SplitSparse {
   long long plane;
   void* dst;
 };
-// Every workgroup leaves the range of the entries it met, a SplitRange as two words: at ranges[0 ..] those of the second operand (a dense one), from
-// ranges[kSplitSlots] on those of the first.  How many there are:
+// Every workgroup leaves the range of the entries it met, a SplitRange as a word: at ranges[0 ..] those of the second operand (a dense one), from
+// ranges[kSplitSlots] on those of the first.  The product leaves at ranges[kSplitVerdict] whether it stands for the fp32 one; room for kSplitRanges in all.  How many
+// there are of each:
 int split_dense_blocks(const SplitDense& s);
 int split_sparse_blocks(const SplitSparse& s);
-int launch_split_operands(const SplitSparse& a, const SplitDense& b, uint2* ranges, hipStream_t stream);
-int launch_split_operands(const SplitDense& a, const SplitDense& b, uint2* ranges, hipStream_t stream);
+int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* ranges, hipStream_t stream);
+int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* ranges, hipStream_t stream);
 
 // C = A * B, or with K in parts (gemm_split_parts: more than one) part s's share of it at C + s * stride_part, which the caller adds up.
 struct SplitParams {
@@ -45,52 +48,55 @@ struct SplitParams {
   const float* row_bias;         // K in one part: C = relu?(A * B + row_bias[row])
   int relu;
   long long stride_part;
+  unsigned* ranges;                 // of the operands' entries, and the verdict: where the range says that the parts do not hold the entries nothing else is written
+  int slots_a, slots_b;
+  int finite;                    // ... and where there is an infinity or a NaN
   int tiles_m, tiles_n, parts;   // (set by the launcher)
 };
 int gemm_split_parts(int M, int N, int K, int batch);
 double gemm_split_seconds(int M, int N, int K, int batch);   // an estimate, for choices between this product and others
 int gemm_split(const SplitParams& p, bool trans_b, int batch, hipStream_t stream);
 
-// out[j] = scores[row of j][cols[j]] (of all parts) for every nonzero j, or the dot product itself where the scores do not stand for it.
+// out[j] = scores[row of j][cols[j]] (of all parts) for every nonzero j, or the dot product itself where the scores do not stand for it.  wide: a workgroup per row.
 struct SplitSample {
-  int m, k, n, batch, ld, parts;
+  int m, k, n, batch, ld, parts, wide;
   long long stride_part;
   const int* row_offsets;
   const int* cols;
   const float* scores;
   const float *lhs, *rhs;   // (batch, m, k), (batch, n, k)
   float* out;
-  const uint2* ranges;
-  int slots_a, slots_b;
+  const unsigned* ranges;
 };
 int launch_split_sample(const SplitSample& s, hipStream_t stream);
 
 __device__ __forceinline__ unsigned magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
 
-// What is known of an operand's entries: the largest finite magnitude and the smallest but zero, as their bits, and whether there was an
-// infinity or a NaN.
+// What is known of an operand's entries: the exponents of the largest finite magnitude and of the smallest but zero, and whether there was an
+// infinity or a NaN.  As a word: the first in the low byte, 255 less the second in the next one, the third above; 0 of no entries or zeros.
 struct SplitRange {
-  unsigned most = 0;
-  unsigned least = ~0u;   // less one: a zero is then the largest of all
-  unsigned odd = 0;       // 0 or 1 << 31
+  unsigned most = 0, small = 0, odd = 0;
+  __device__ __forceinline__ void add_word(unsigned w) {
+    most = max(most, w & 0xffu);
+    small = max(small, w & 0xff00u);
+    odd |= w & 0x10000u;
+  }
+  __device__ __forceinline__ unsigned word() const { return most | small | odd; }
+  __device__ __forceinline__ void over_wave() {
+    most = (unsigned)wave_max((float)most);
+    small = (unsigned)wave_max((float)small);
+    odd = __ballot(odd != 0) ? 0x10000u : 0u;
+  }
+};
+// ... and how it is found, entry by entry
+struct SplitExtent {
+  unsigned most = 0, least = ~0u, odd = 0;   // magnitudes as their bits (least: less one, a zero is then the largest of all)
   __device__ __forceinline__ void add(float x) {
     const unsigned size = magnitude(x);
-    if (size >= 0x7f800000u) odd = 1u << 31;
+    if (size >= 0x7f800000u) odd = 0x10000u;
     else most = max(most, size), least = min(least, size - 1u);
   }
-  __device__ __forceinline__ uint2 words() const { return uint2{most | odd, least}; }
-  __device__ __forceinline__ void add_words(uint2 w) {
-    most = max(most, w.x & 0x7fffffffu);
-    least = min(least, w.y);
-    odd |= w.x & (1u << 31);
-  }
-  __device__ __forceinline__ void over_wave() {
-#pragma unroll
-    for (int d = 32; d; d >>= 1) {
-      const uint2 w = words();
-      add_words(uint2{(unsigned)__shfl_xor((int)w.x, d), (unsigned)__shfl_xor((int)w.y, d)});
-    }
-  }
+  __device__ __forceinline__ SplitRange range() const { return SplitRange{most >> 23, least == ~0u ? 0u : (255u - ((least + 1u) >> 23)) << 8, odd}; }
 };
 
 // Whether the product of the parts of both operands' finite entries holds what an fp32 one does.  Entries from 2^-110 on have parts that hold
@@ -98,10 +104,10 @@ struct SplitRange {
 // sums, which end at 2^-149, keep to 2^-29 of them.  Rows of 2^-112 beside rows of 1 were off by 1.8e-7, of 2^-120 by 3.7e-5 (row kernel 1.0e-7).  At
 // the other end parts, products and their sums stay below infinity.
 __device__ __forceinline__ bool split_range_ok(const SplitRange& of_a, const SplitRange& of_b) {
-  if (of_a.most == 0u || of_b.most == 0u) return max(of_a.most, of_b.most) < 253u << 23;   // (beyond 2^126 a part may be an infinity, and its product with zero a NaN)
-  auto exponent = [](unsigned bits) { return (int)(bits >> 23) - 127; };
-  const int least_a = exponent(of_a.least + 1u), least_b = exponent(of_b.least + 1u), most_a = exponent(of_a.most), most_b = exponent(of_b.most);
-  return least_a >= -110 && least_b >= -110 && least_a + least_b >= -120 && most_a < 126 && most_b < 126 && most_a + most_b < 90;
+  const int most_a = (int)of_a.most - 127, most_b = (int)of_b.most - 127, least_a = 128 - (int)(of_a.small >> 8), least_b = 128 - (int)(of_b.small >> 8);
+  if (most_a >= 126 || most_b >= 126) return false;         // (beyond 2^126 a part may be an infinity, and its product with zero a NaN)
+  if (of_a.small == 0 || of_b.small == 0) return true;      // (zeros alone)
+  return least_a >= -110 && least_b >= -110 && least_a + least_b >= -120 && most_a + most_b < 90;
 }
 
 }  // namespace iex

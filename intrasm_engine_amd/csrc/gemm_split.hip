@@ -34,15 +34,15 @@ __device__ __forceinline__ void store_parts(const float (&x)[8], uint16_t* dst, 
 }
 
 template <int WAVES>
-__device__ __forceinline__ void leave_range(SplitRange x, uint2* at) {
-  __shared__ uint2 of[WAVES];
+__device__ __forceinline__ void leave_range(SplitRange x, unsigned* at) {
+  __shared__ unsigned of[WAVES];
   x.over_wave();
-  if (lane_id() == 0) of[threadIdx.x >> 6] = x.words();
+  if (lane_id() == 0) of[threadIdx.x >> 6] = x.word();
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) x.add_words(of[w]);
-    *at = x.words();
+    for (int w = 0; w < WAVES; ++w) x.add_word(of[w]);
+    *at = x.word();
   }
 }
 
@@ -50,7 +50,7 @@ __device__ __forceinline__ SplitRange split_dense_block(const SplitDense& s, int
   struct alignas(4) Any { float v[8]; };
   const int chunks = s.dst_cols / 8;
   const long long total = (long long)s.batch * s.dst_rows * chunks;
-  SplitRange range;
+  SplitExtent range;
   for (long long i = (long long)block * 256 + threadIdx.x; i < total; i += (long long)blocks * 256) {
     const long long zr = i / chunks;
     const int c = (int)(i - zr * chunks) * 8;
@@ -69,7 +69,7 @@ __device__ __forceinline__ SplitRange split_dense_block(const SplitDense& s, int
     for (int e = 0; e < 8; ++e) range.add(x[e]);
     store_parts(x, static_cast<uint16_t*>(s.dst) + (size_t)z * s.dst_batch + (size_t)r * s.ld + c, s.plane);
   }
-  return range;
+  return range.range();
 }
 
 // As csr_to_dense_kernel (spmm_dense_device.cuh): a workgroup per row, the row (or 4096 columns of it) assembled in LDS in fp32, its parts taken on
@@ -81,7 +81,7 @@ __device__ __forceinline__ SplitRange split_sparse_block(const SplitSparse& s, i
   const int* __restrict__ cols = s.cols;
   const float* __restrict__ values = s.values;
   uint16_t* __restrict__ dst = static_cast<uint16_t*>(s.dst);
-  SplitRange range;
+  SplitExtent range;
   bool again = false;
   for (int slot0 = block * kPlanesRows; slot0 < s.m; slot0 += blocks * kPlanesRows) {
     int pos[kPlanesRows], end[kPlanesRows];   // this wavefront's quarter of each row's nonzeros, in whole chunks of 64
@@ -144,13 +144,13 @@ __device__ __forceinline__ SplitRange split_sparse_block(const SplitSparse& s, i
           }
     }
   }
-  return range;
+  return range.range();
 }
 
 // Both operands' parts in one launch: the first workgroups make those of the second operand.  Bound by the bytes, 4 read and 6 written an entry, 6
-// written a cell of a sparse operand.  (Two words per workgroup, not atomics: 8192 of them on 64 words took 25 us.)
+// written a cell of a sparse operand.  (A word per workgroup, not atomics: 8192 of them on 64 words took 25 us.)
 template <typename First>
-__global__ __launch_bounds__(256) void split_operands_kernel(First a, SplitDense b, uint2* ranges, int blocks_b) {
+__global__ __launch_bounds__(256) void split_operands_kernel(First a, SplitDense b, unsigned* ranges, int blocks_b) {
   if ((int)blockIdx.x < blocks_b) {
     leave_range<4>(split_dense_block(b, blockIdx.x, blocks_b), ranges + blockIdx.x);
   } else {
@@ -162,37 +162,71 @@ __global__ __launch_bounds__(256) void split_operands_kernel(First a, SplitDense
   }
 }
 
-// A wavefront per row.  A score that is not finite (an infinity's parts give NaN) is computed as the dot product itself, by
-// the whole wavefront, and so are all where the range of the operands' finite entries says that parts do not hold them.
+// A wavefront per row, or (WIDE) a workgroup.  A score that is not finite (an infinity's parts give NaN) is computed as the dot product itself, and so are all where
+// the product has found that parts do not hold the operands' entries: eight scores side by side, by eight lanes each, four vectors of both operands in
+// flight, bound by the rows' way from L2 as the gather kernel is.  Us a call, 2160 x 1449 at 81 %, k = 221 / 986 x 10230 at 85 %, k = 1049 / 11008 x 4096 at 90 %,
+// k = 256: gather kernel 39 / 608 / 204, by parts 32 / 166 / 228; all computed here 58 / 714 / 306 (one score at a time by the whole wavefront: 228 / 5765 / 873); an
+// infinity in lhs, so one row of them, 49 / 386 / 230 (287 / 6436 / 673).
+constexpr int kDotLanes = 8, kDots = kWave / kDotLanes;
+__device__ __forceinline__ float dot_product(const SplitSample& s, int row, int col, int part) {
+  typedef float any4 __attribute__((ext_vector_type(4), aligned(4)));
+  float sums[4] = {0.f, 0.f, 0.f, 0.f};   // (short chains: the gather kernel's accuracy)
+  for (int z = 0; z < s.batch; ++z) {
+    const float* l = s.lhs + ((size_t)z * s.m + row) * s.k;
+    const float* r = s.rhs + ((size_t)z * s.n + col) * s.k;
+    int i = part * 4;
+    for (; i + 3 * kDotLanes * 4 + 4 <= s.k; i += 4 * kDotLanes * 4) {
+      any4 x[4], y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const any4*>(l + i + u * kDotLanes * 4), y[u] = *reinterpret_cast<const any4*>(r + i + u * kDotLanes * 4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sums[e] = fmaf(x[u][e], y[u][e], sums[e]);
+    }
+    for (; i < s.k; i += kDotLanes * 4) {
+      if (i + 4 <= s.k) {
+        const any4 x = *reinterpret_cast<const any4*>(l + i), y = *reinterpret_cast<const any4*>(r + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sums[e] = fmaf(x[e], y[e], sums[e]);
+      } else {
+        for (int e = i; e < s.k; ++e) sums[0] = fmaf(l[e], r[e], sums[0]);
+      }
+    }
+  }
+  float sum = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+#pragma unroll
+  for (int d = kDotLanes / 2; d; d >>= 1) sum += __shfl_xor(sum, d);
+  return sum;
+}
+
+template <bool WIDE>
 __global__ __launch_bounds__(256) void split_sample_kernel(SplitSample s) {
-  const int row = blockIdx.x * 4 + uniform(threadIdx.x >> 6), lane = lane_id();
+  const int wave = uniform(threadIdx.x >> 6), lane = lane_id();
+  const int row = WIDE ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave;
   if (row >= s.m) return;
   const int start = s.row_offsets[row], end = s.row_offsets[row + 1];
-  SplitRange of_a, of_b;
-  for (int i = lane; i < kSplitSlots; i += kWave) {
-    if (i < s.slots_a) of_a.add_words(s.ranges[kSplitSlots + i]);
-    if (i < s.slots_b) of_b.add_words(s.ranges[i]);
-  }
-  of_a.over_wave(), of_b.over_wave();
-  const bool all = !split_range_ok(of_a, of_b);   // (wave-uniform)
+  const bool all = s.ranges[kSplitVerdict] == 0;   // (uniform)
   const float* scores = s.scores + (size_t)row * s.ld;
-  for (int j0 = start; j0 < end; j0 += kWave) {
+  for (int j0 = start + (WIDE ? wave * kWave : 0); j0 < end; j0 += WIDE ? 4 * kWave : kWave) {
     const int j = min(j0 + lane, end - 1), col = s.cols[j];
-    float x = scores[col];
-    for (int part = 1; part < s.parts; ++part) x += scores[(size_t)part * s.stride_part + col];
-    unsigned long long odd = __ballot(j0 + lane < end && (all || magnitude(x) >= 0x7f800000u));
-    while (odd) {
-      const int src = __ffsll(odd) - 1;
-      odd &= odd - 1;
-      const int c = bcast_i(col, src);
-      float sum = 0.f;
-      for (int z = 0; z < s.batch; ++z) {
-        const float* l = s.lhs + ((size_t)z * s.m + row) * s.k;
-        const float* r = s.rhs + ((size_t)z * s.n + c) * s.k;
-        for (int i = lane; i < s.k; i += kWave) sum = fmaf(l[i], r[i], sum);
+    float x = 0.f;
+    if (!all) {
+      x = scores[col];
+      for (int part = 1; part < s.parts; ++part) x += scores[(size_t)part * s.stride_part + col];
+    }
+    const bool mine = j0 + lane < end && (all || magnitude(x) >= 0x7f800000u);
+    unsigned long long odd = __ballot(mine);
+    const int place = __popcll(odd & ((1ull << lane) - 1));   // of mine among them
+    for (int first = 0; odd; first += kDots) {
+      int src = __ffsll(odd) - 1;   // of the eight lanes that I am of: theirs is the next one, the one after ..., or the first again
+#pragma unroll
+      for (int d = 0; d < kDots; ++d) {
+        if (odd && lane / kDotLanes == d) src = __ffsll(odd) - 1;
+        odd &= odd - 1;
       }
-      sum = wave_sum(sum);
-      if (lane == src) x = sum;
+      const float sum = __shfl(dot_product(s, row, __shfl(col, src), lane % kDotLanes), (place - first) * kDotLanes & (kWave - 1));
+      if (mine && place >= first && place < first + kDots) x = sum;
     }
     if (j0 + lane < end) s.out[j] = x;
   }
@@ -237,7 +271,7 @@ int launch_product(const SplitParams& p, int batch, hipStream_t stream) {
 }
 
 template <typename First>
-int launch_operands(const First& a, int blocks_a, const SplitDense& b, uint2* ranges, hipStream_t stream) {
+int launch_operands(const First& a, int blocks_a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
   const int blocks_b = split_dense_blocks(b);
   note_kernel("split_operands_kernel");
   hipLaunchKernelGGL(split_operands_kernel<First>, dim3(blocks_a + blocks_b), dim3(256), 0, stream, a, b, ranges, blocks_b);
@@ -277,15 +311,16 @@ int split_dense_blocks(const SplitDense& s) {
   return (int)std::min<long long>(kSplitSlots, (chunks + 255) / 256);
 }
 int split_sparse_blocks(const SplitSparse& s) { return std::min(kSplitSparseSlots, ceil_div(s.m, kPlanesRows)); }
-int launch_split_operands(const SplitSparse& a, const SplitDense& b, uint2* ranges, hipStream_t stream) {
+int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
   return launch_operands(a, split_sparse_blocks(a), b, ranges, stream);
 }
-int launch_split_operands(const SplitDense& a, const SplitDense& b, uint2* ranges, hipStream_t stream) {
+int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
   return launch_operands(a, split_dense_blocks(a), b, ranges, stream);
 }
 int launch_split_sample(const SplitSample& s, hipStream_t stream) {
   note_kernel("split_sample_kernel");
-  hipLaunchKernelGGL(split_sample_kernel, dim3(ceil_div(s.m, 4)), dim3(256), 0, stream, s);
+  if (s.wide) hipLaunchKernelGGL(split_sample_kernel<true>, dim3(s.m), dim3(256), 0, stream, s);
+  else hipLaunchKernelGGL(split_sample_kernel<false>, dim3(ceil_div(s.m, 4)), dim3(256), 0, stream, s);
   return check_hip(hipGetLastError(), "sampling launch");
 }
 

@@ -21,6 +21,8 @@
 // Few tiles: K in parts, every part's sums in a matrix of their own; the kernel that comes next anyway (the check of the operands' range, or the
 // sampling) adds them up in their order.  (4096 x 256 x 4096 in four parts, us: the workgroup that draws a tile's last ticket reading
 // the others' sums, as in gemm_dma_device.cuh, 54; this way 47, and 3.5 in the next kernel.)
+// Every workgroup looks at the range of the operands' entries (10 KB, a word per workgroup that made parts) while its first tiles are on their way, and ends where
+// the product would not stand for the fp32 one: 4096 x 256 x 4096 47.7 -> 48.8 us, 5 where it ends, and the kernel behind it reads one word (7.6 -> 4.2).
 // Requirements (the caller's, who makes the planes): K a multiple of 32, planes zero where the operands end, row strides
 // multiples of 8, 16-byte aligned planes, three of them within 4 GB.
 #pragma once
@@ -31,7 +33,25 @@
 namespace iex {
 
 template <int WM, int WN, int STAGES>
-constexpr int gemm_split_lds_bytes() { return STAGES * 3 * (2 * WM * 32 + 2 * WN * 32) * 64; }
+constexpr int gemm_split_lds_bytes() { return STAGES * 3 * (2 * WM * 32 + 2 * WN * 32) * 64 + kSplitVerdict * 4 + 32; }
+
+// Whether the product of the parts stands for the fp32 one, by all 256 threads from the ranges' words in LDS, eight words of room behind them.  (An array of this
+// function's own would come first in LDS and shift the stages off the 128 bytes that direct loads write at a time: 4096 x 1024 x 4096 147 -> 154 us.)
+__device__ __forceinline__ bool split_stands(const SplitParams& p, unsigned* words) {
+  SplitRange a, b;
+#pragma unroll
+  for (int i = 0; i < kSplitVerdict; i += 256) {
+    const int at = (i < kSplitSlots ? i : i - kSplitSlots) + threadIdx.x;
+    if (at < (i < kSplitSlots ? p.slots_b : p.slots_a)) (i < kSplitSlots ? b : a).add_word(words[i + threadIdx.x]);
+  }
+  a.over_wave(), b.over_wave();
+  unsigned* of = words + kSplitVerdict;
+  if (lane_id() == 0) of[threadIdx.x >> 6] = a.word(), of[4 + (threadIdx.x >> 6)] = b.word();
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) a.add_word(of[w]), b.add_word(of[4 + w]);
+  return split_range_ok(a, b) && !(p.finite && (a.odd || b.odd));
+}
 
 // One tile's stretch `part` of K.  TRANS_B: B is (N, K), else (K, N).
 template <bool TRANS_B, int WM, int WN, int STAGES, int FLUSH>
@@ -96,12 +116,26 @@ __device__ __forceinline__ void gemm_split_tile(const SplitParams& p, int tile_m
   const std::integral_constant<int, 0> high;
   const std::integral_constant<int, 1> middle;
   const std::integral_constant<int, 2> low;
+  // the ranges' words, then the first tiles
+  static_assert(kSplitVerdict * 4 % 1024 == 0, "whole direct loads");
+  const u32x4 word_buf = buffer_of(p.ranges, kSplitVerdict * 4);
+#pragma unroll
+  for (int q = 0; q < (kSplitVerdict * 4 / 1024 + WAVES - 1) / WAVES; ++q) {
+    const unsigned at = min(q * WAVES + wave, kSplitVerdict * 4 / 1024 - 1) * 1024;   // (some come twice)
+    lds_dma16(word_buf, lane * 16, at, __builtin_amdgcn_readfirstlane(lds0 + STAGES * STAGE_BYTES + at));
+  }
 #pragma unroll
   for (int s = 0; s < STAGES; ++s)
 #pragma unroll
     for (int q = 0; q < LOADS; ++q) issue_one(s, s * STAGE_BYTES, q);
   wait_vmcnt<(STAGES - 1) * LOADS>();
   __syncthreads();
+  const bool stands = split_stands(p, reinterpret_cast<unsigned*>(smem + STAGES * STAGE_BYTES));
+  if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) p.ranges[kSplitVerdict] = stands;
+  if (!stands) {   // (uniform)
+    wait_vmcnt<0>();   // nothing may still be writing LDS when the workgroup ends
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) read_a(smem, low, al[i], i), read_a(smem, high, ah[0][i], i), read_a(smem, middle, am[i], i);
 #pragma unroll

@@ -381,7 +381,7 @@ inline SddmmSplit sddmm_split_plan(const SddmmParams& p) {
   s.K = s.kp * p.batch;
   s.ld = (p.n + 3) & ~3;
   s.parts = gemm_split_parts(p.m, p.n, s.K, 1);
-  s.lhs_at = 2 * kSplitSlots * sizeof(uint2);
+  s.lhs_at = kSplitRanges * 4;
   s.rhs_at = s.lhs_at + round256((size_t)p.m * s.K * 6);
   s.scores_at = s.rhs_at + round256((size_t)p.n * s.K * 6);
   s.bytes = s.scores_at + (size_t)s.parts * p.m * s.ld * 4;
@@ -406,7 +406,7 @@ inline bool sddmm_split_wins(const SddmmParams& p) {
 int launch_sddmm_split(const SddmmParams& p, void* workspace, hipStream_t stream) {
   const SddmmSplit s = sddmm_split_plan(p);
   unsigned char* ws = static_cast<unsigned char*>(workspace);
-  uint2* ranges = reinterpret_cast<uint2*>(ws);
+  unsigned* ranges = reinterpret_cast<unsigned*>(ws);
   const long long plane_a = (long long)p.m * s.K, plane_b = (long long)p.n * s.K;
   const SplitDense a{p.batch, p.m, p.k, static_cast<const float*>(p.lhs), p.m, s.kp, s.K, s.kp, plane_a, ws + s.lhs_at};
   const SplitDense b{p.batch, p.n, p.k, static_cast<const float*>(p.rhs), p.n, s.kp, s.K, s.kp, plane_b, ws + s.rhs_at};
@@ -417,9 +417,10 @@ int launch_sddmm_split(const SddmmParams& p, void* workspace, hipStream_t stream
   g.lda = g.ldb = s.K, g.ldc = s.ld;
   g.plane_a = (unsigned)(plane_a * 2), g.plane_b = (unsigned)(plane_b * 2);
   g.stride_part = (long long)p.m * s.ld;
+  g.ranges = ranges, g.slots_a = split_dense_blocks(a), g.slots_b = split_dense_blocks(b);
   if (int rc = gemm_split(g, true, 1, stream)) return rc;
-  const SplitSample q{p.m, p.k, p.n, p.batch, s.ld, s.parts, g.stride_part, p.row_offsets, p.cols, g.C, static_cast<const float*>(p.lhs), static_cast<const float*>(p.rhs),
-                      static_cast<float*>(p.out), ranges, split_dense_blocks(a), split_dense_blocks(b)};
+  const SplitSample q{p.m, p.k, p.n, p.batch, s.ld, s.parts, sample_wide(p), g.stride_part, p.row_offsets, p.cols, g.C, static_cast<const float*>(p.lhs), static_cast<const float*>(p.rhs),
+                      static_cast<float*>(p.out), ranges};
   return launch_split_sample(q, stream);
 }
 

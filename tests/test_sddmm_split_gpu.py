@@ -103,6 +103,24 @@ def test_an_infinity_beside_entries_outside_the_range(what, of_lhs, of_rhs):
     assert of(got) <= max(1.5 * of(want), 1.2e-7)
 
 
+# a wavefront and a workgroup to a row, rows of one score, of no whole eights and of several hundred; k of no whole vectors, below and beyond four vectors a lane
+@pytest.mark.parametrize("m,n,k,density,batch", [(5, 3, 1, 1.0, 1), (33, 70, 3, 0.4, 2), (40, 90, 31, 0.3, 1), (130, 600, 130, 0.5, 1), (300, 40, 257, 0.3, 3), (70, 1500, 300, 0.6, 2)])
+def test_scores_computed_one_by_one(oracle, m, n, k, density, batch):
+    """All of them (operands outside the range of the parts), or a row's and a column's (an infinity), as the dot products themselves."""
+    lhs, rhs, *pattern = operands(m, n, k, density, batch, seed=12)
+    args = (lhs * 1e-30, rhs * 1e-4, *pattern)
+    lhs_np, rhs_np, ri, ro, ci = (t.cpu().numpy() for t in args)
+    assert_close(sampled(args, 12).cpu().numpy(), oracle.sddmm(lhs_np, rhs_np, ri, ro, ci), oracle.sddmm_abs_scale(lhs_np, rhs_np, ri, ro, ci), 1e-5, f"{m}x{n}x{k}")
+    assert "split_sample_kernel" in _lib.last_kernels()
+    lhs[-1, m - 1, k - 1] = float("inf")
+    rhs[0, n - 1, 0] = float("-inf")
+    args = (lhs, rhs, *pattern)
+    got, want = sampled(args, 12), sampled(args, 1)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf()) and torch.equal(got[want.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    assert not fine.any() or float((got - want)[fine].double().norm() / want[fine].double().norm()) < 1e-6
+
+
 def test_where_it_is_taken_and_where_not():
     args = operands(2000, 1500, 700, 0.2, seed=5)
     lhs, rhs, row_indices, row_offsets, columns = args
