@@ -207,7 +207,8 @@ int iex_spmm_ex(int dtype, int itype, int flags, int m, int k, int n, int nonzer
  * tile; a 16-byte aligned workspace of m * k * 2 bytes still runs the path, without the split.
  * IEX_SPMM_FORCE_VARIANT(7) asks for that path and fails where it cannot run.
  * Large fp32 products with IEX_SPMM_PAD_OPERANDS run by parts (family 12), with a 256-byte aligned workspace for the parts of both operands and of k:
- * 6 bytes a cell of A (m * k, k rounded up to 32) and an entry of the dense operand, and 4 per part of k and output.
+ * 6 bytes a cell of A (m * k, k rounded up to 32) and an entry of the dense operand, and 4 per part of k and output; batch entries beyond 512 MB
+ * of these take turns, and a call that would need more than 4 GiB all the same does not go this way.
  * iex_spmm_workspace_bytes returns the size with which the call described would use the workspace,
  * 0 when it would not whatever the size.  Neither call allocates.
  * No counterpart in the reference: its launchers (csrc/extensions.h:28-30) take no workspace. */
@@ -379,7 +380,7 @@ int iex_sddmm_ex(int dtype, int flags, int m, int k, int n, int nonzeros,
  * fp32 calls with IEX_SDDMM_PAD_OPERANDS, a plain store and one output (batch 1, or summed over the batch) do the same by parts (12, with a
  * 256-byte aligned workspace): lhs and rhs as three bf16 parts of every entry, all products on the bf16 matrix cores (SpMM family 12 says what
  * that does to accuracy); scores that are not finite, and all of them where the operands are too large or small for it, are
- * computed as the dot products themselves.
+ * computed as the dot products themselves.  Calls that would need more than 4 GiB for it do not go this way.
  * The workspace also serves variant 3 above (short k, masks with structure), which 0 = choose picks first.
  * iex_sddmm_workspace_bytes returns the size with which the call described would use the
  * workspace, 0 when it would not whatever the size.  Neither call allocates.

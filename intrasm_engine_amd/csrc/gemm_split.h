@@ -9,6 +9,9 @@ constexpr int kSplitSparseSlots = 2048;  // ... a sparse one's
 
 constexpr int kSplitVerdict = kSplitSlots + kSplitSparseSlots, kSplitRanges = kSplitVerdict + 64;   // (whole 256 bytes)
 
+// The most that a call's workspace for parts may take: 1.4 % of the card's memory.  What would need more runs on the kernels without one.
+constexpr size_t kSplitWorkspaceMost = (size_t)4 << 30;
+
 inline int round32(int x) { return (x + 31) & ~31; }
 
 // src (batch x rows x cols, fp32, at element alignment) as three planes of bf16: high, middle and low parts.  Entry (z, r, c) of a plane lies at
@@ -36,6 +39,7 @@ int split_dense_blocks(const SplitDense& s);
 int split_sparse_blocks(const SplitSparse& s);
 int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* ranges, hipStream_t stream);
 int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* ranges, hipStream_t stream);
+int launch_split_operand(const SplitDense& b, unsigned* ranges, hipStream_t stream);   // the second one alone
 
 // C = A * B, or with K in parts (gemm_split_parts: more than one) part s's share of it at C + s * stride_part, which the caller adds up.
 struct SplitParams {
@@ -51,7 +55,8 @@ struct SplitParams {
   unsigned* ranges;                 // of the operands' entries, and the verdict: where the range says that the parts do not hold the entries nothing else is written
   int slots_a, slots_b;
   int finite;                    // ... and where there is an infinity or a NaN
-  int tiles_m, tiles_n, parts;   // (set by the launcher)
+  int parts;                     // of K, each with at least a step: gemm_split_parts
+  int tiles_m, tiles_n;          // (set by the launcher)
 };
 int gemm_split_parts(int M, int N, int K, int batch);
 double gemm_split_seconds(int M, int N, int K, int batch);   // an estimate, for choices between this product and others

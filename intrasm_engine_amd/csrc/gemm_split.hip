@@ -300,8 +300,8 @@ int gemm_split(const SplitParams& given, bool trans_b, int batch, hipStream_t st
   SplitParams p = given;
   p.tiles_m = ceil_div(p.M, kSplitTile);
   p.tiles_n = ceil_div(p.N, kSplitTile);
-  p.parts = gemm_split_parts(p.M, p.N, p.K, batch);
-  IEX_REQUIRE(p.K > 0 && p.K % 32 == 0 && p.lda % 8 == 0 && p.ldb % 8 == 0 && (p.parts == 1 || (p.stride_part > 0 && !p.row_bias && !p.relu)), IEX_ERR_STATE,
+  const int steps = p.K / 32, per = p.parts > 0 ? ceil_div(steps, p.parts) : 0;
+  IEX_REQUIRE(p.parts > 0 && (p.parts - 1) * per < steps && p.K > 0 && p.K % 32 == 0 && p.lda % 8 == 0 && p.ldb % 8 == 0 && (p.parts == 1 || (p.stride_part > 0 && !p.row_bias && !p.relu)), IEX_ERR_STATE,
               "gemm (fp32 by parts): K=%d in %d parts, strides %d and %d", p.K, p.parts, p.lda, p.ldb);
   return trans_b ? launch_product<true>(p, batch, stream) : launch_product<false>(p, batch, stream);
 }
@@ -317,6 +317,7 @@ int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* r
 int launch_split_operands(const SplitDense& a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
   return launch_operands(a, split_dense_blocks(a), b, ranges, stream);
 }
+int launch_split_operand(const SplitDense& b, unsigned* ranges, hipStream_t stream) { return launch_operands(b, 0, b, ranges, stream); }
 int launch_split_sample(const SplitSample& s, hipStream_t stream) {
   note_kernel("split_sample_kernel");
   if (s.wide) hipLaunchKernelGGL(split_sample_kernel<true>, dim3(s.m), dim3(256), 0, stream, s);

@@ -403,6 +403,12 @@ inline bool sddmm_split_wins(const SddmmParams& p) {
   const double sample = 4.5e-6 + (4.0 * s.parts * p.m * s.ld + 8.0 * p.nnz) / 4e12;
   return 1.1 * (3.5e-6 + 10.0 * ((double)p.m + p.n) * s.K / 4.4e12 + gemm_split_seconds(p.m, p.n, s.K, 1) + sample) < gather;
 }
+// What a call that goes this way wants of workspace; 0: it does not.
+inline size_t sddmm_split_bytes(int dtype, const SddmmParams& p, bool forced) {
+  if (!sddmm_split_fits(dtype, p) || (!forced && !sddmm_split_wins(p))) return 0;
+  const size_t bytes = sddmm_split_plan(p).bytes;
+  return bytes <= kSplitWorkspaceMost ? bytes : 0;
+}
 int launch_sddmm_split(const SddmmParams& p, void* workspace, hipStream_t stream) {
   const SddmmSplit s = sddmm_split_plan(p);
   unsigned char* ws = static_cast<unsigned char*>(workspace);
@@ -416,7 +422,7 @@ int launch_sddmm_split(const SddmmParams& p, void* workspace, hipStream_t stream
   g.A = a.dst, g.B = b.dst, g.C = reinterpret_cast<float*>(ws + s.scores_at);
   g.lda = g.ldb = s.K, g.ldc = s.ld;
   g.plane_a = (unsigned)(plane_a * 2), g.plane_b = (unsigned)(plane_b * 2);
-  g.stride_part = (long long)p.m * s.ld;
+  g.parts = s.parts, g.stride_part = (long long)p.m * s.ld;
   g.ranges = ranges, g.slots_a = split_dense_blocks(a), g.slots_b = split_dense_blocks(b);
   if (int rc = gemm_split(g, true, 1, stream)) return rc;
   const SplitSample q{p.m, p.k, p.n, p.batch, s.ld, s.parts, sample_wide(p), g.stride_part, p.row_offsets, p.cols, g.C, static_cast<const float*>(p.lhs), static_cast<const float*>(p.rhs),
@@ -500,7 +506,7 @@ int sddmm_workspace_kind(int dtype, int flags, int m, int k, int n, int nonzeros
   void* const some_aligned = reinterpret_cast<void*>(size_t(256));
   SddmmParams p{m, k, n, nonzeros, batch, nullptr, nullptr, nullptr, some_aligned, some_aligned, nullptr,
                 (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0, (flags & IEX_SDDMM_PAD_OPERANDS) != 0};
-  if (dtype == IEX_F32 && variant != 3 && variant != 7) return sddmm_split_fits(dtype, p) && (variant == 12 || sddmm_split_wins(p)) ? 12 : 0;
+  if (dtype == IEX_F32 && variant != 3 && variant != 7) return sddmm_split_bytes(dtype, p, variant == 12) ? 12 : 0;
   if (variant == 12) return 0;
   const bool any_order = (flags & IEX_SDDMM_ANY_COLUMN_ORDER) != 0;
   if (variant != 7 && sddmm_mfma_fits(dtype, p) && (variant == 3 || (!any_order && sddmm_mfma_wins(p)))) return 3;
@@ -515,7 +521,7 @@ size_t sddmm_workspace_bytes(int dtype, int flags, int m, int k, int n, int nonz
   void* const some_aligned = reinterpret_cast<void*>(size_t(256));
   SddmmParams p{m, k, n, nonzeros, batch, nullptr, nullptr, nullptr, some_aligned, some_aligned, nullptr,
                 (flags & IEX_SDDMM_SUM_OVER_BATCH) != 0, (flags & IEX_SDDMM_ACCUMULATE) != 0, (flags & IEX_SDDMM_PAD_OPERANDS) != 0};
-  if (dtype == IEX_F32 && variant != 3 && variant != 7) return sddmm_split_fits(dtype, p) && (variant == 12 || sddmm_split_wins(p)) ? sddmm_split_plan(p).bytes : 0;
+  if (dtype == IEX_F32 && variant != 3 && variant != 7) return sddmm_split_bytes(dtype, p, variant == 12);
   if (variant == 12) return 0;
   const bool any_order = (flags & IEX_SDDMM_ANY_COLUMN_ORDER) != 0;
   if (variant != 7 && sddmm_mfma_fits(dtype, p) && (variant == 3 || (!any_order && sddmm_mfma_wins(p)))) return sddmm_mfma_bytes(p);
@@ -564,9 +570,10 @@ int sddmm_dispatch(int dtype, int flags, int m, int k, int n, int nonzeros, cons
     }
     if (fits && room && (variant == 7 || sddmm_dense_wins(p))) return launch_sddmm_dense(dtype, p, workspace, s);
   }
-  if ((variant == 0 || variant == 12) && workspace && aligned(workspace, 256) && sddmm_split_fits(dtype, p) && (variant == 12 || sddmm_split_wins(p)) &&
-      workspace_bytes >= sddmm_split_plan(p).bytes)
-    return launch_sddmm_split(p, workspace, s);
+  if ((variant == 0 || variant == 12) && workspace && aligned(workspace, 256)) {
+    const size_t need = sddmm_split_bytes(dtype, p, variant == 12);
+    if (need && workspace_bytes >= need) return launch_sddmm_split(p, workspace, s);
+  }
   switch (dtype) {
     case IEX_F32: return launch_typed<float>(p, wpr, s);
     case IEX_F16: return launch_typed<__half>(p, wpr, s);

@@ -883,20 +883,24 @@ int launch_dense_path(const SpmmParams& p, int batch, const Choice& ch, hipStrea
 
 // ---- fp32 by parts: the dense form of A and B as three bf16 planes each, then their product on the bf16 matrix cores (gemm_split_device.cuh) ----
 struct SplitPlan {
-  int kp, np, parts, ld;   // ld: rows of the parts' sums
+  int kp, np, group, parts, ld;   // group: batch entries at a time; ld: rows of the parts' sums
   size_t a_at, b_at, sums_at, bytes;
 };
+// Batch entries' planes at a time, all that they hold together: enough to fill the chip many times over, and a call's memory does not grow with its batch.  (64 of
+// 4096 x 4096 at 80 % by 4096 x 4096: 6.5 GB of workspace, 0.6 this way.)
+constexpr size_t kSplitGroupBytes = (size_t)512 << 20;
 // the workspace: the ranges of the operands' entries, planes of A, planes of B, sums of the parts of K
 inline SplitPlan split_plan(const SpmmParams& p, int batch) {
   SplitPlan s;
   s.kp = round32(p.k);
   s.np = round8(p.n);
-  s.parts = gemm_split_parts(p.m, p.n, s.kp, batch);
+  s.group = (int)std::min<size_t>(batch, std::max<size_t>(1, kSplitGroupBytes / ((size_t)s.kp * s.np * 6)));
+  s.parts = gemm_split_parts(p.m, p.n, s.kp, s.group);
   s.ld = (p.n + 3) & ~3;
   s.a_at = kSplitRanges * 4;
   s.b_at = s.a_at + round256((size_t)p.m * s.kp * 6);
-  s.sums_at = s.b_at + round256((size_t)batch * s.kp * s.np * 6);
-  s.bytes = s.sums_at + (s.parts > 1 ? (size_t)s.parts * batch * p.m * s.ld * 4 : 0);
+  s.sums_at = s.b_at + round256((size_t)s.group * s.kp * s.np * 6);
+  s.bytes = s.sums_at + (s.parts > 1 ? (size_t)s.parts * s.group * p.m * s.ld * 4 : 0);
   return s;
 }
 // (canonical CSR; an operand's copies in the workspace, which is the caller's to allow; planes within a buffer's 4 GB; a vector of four columns for
@@ -910,9 +914,10 @@ inline bool split_path_fits(const SpmmParams& p) {
 // (gemm_split_seconds), the parts' sums at 4 TB/s; the row kernel gathers whole tiles of 256 columns at up to 30 TB/s, the fp32 matrix-core kernel
 // multiplies at 92 TFLOP/s.
 inline double split_path_seconds(const SpmmParams& p, int batch) {
-  const int kp = round32(p.k), parts = gemm_split_parts(p.m, p.n, kp, batch);
-  const double planes = 3.5e-6 + (6.0 * p.m * kp + 10.0 * batch * p.k * p.n) / 4.4e12;
-  return planes + gemm_split_seconds(p.m, p.n, kp, batch) + 4e-6 + (parts > 1 ? 4.0 * (parts + 1) * p.m * p.n * batch / 4e12 : 0.0);
+  const SplitPlan s = split_plan(p, batch);
+  const double planes = 3.5e-6 + (6.0 * p.m * s.kp + 10.0 * batch * p.k * p.n) / 4.4e12;
+  const double group = gemm_split_seconds(p.m, p.n, s.kp, s.group) + 4e-6 + (s.parts > 1 ? 4.0 * (s.parts + 1) * p.m * p.n * s.group / 4e12 : 0.0);
+  return planes + group * batch / s.group + 3.5e-6 * (ceil_div(batch, s.group) - 1);
 }
 inline bool split_path_wins(const SpmmParams& p, int batch) {
   // Row kernel: whole tiles of 256 columns (narrow ones to the next power of two) at 30 TB/s, 25 where a tile's slice of B outgrows an XCD's L2.
@@ -931,6 +936,13 @@ inline bool split_path_wins(const SpmmParams& p, int batch) {
   // 116 / 86): whoever looks at the names of the kernels finds that one there.
   if (p.n <= 256 && mfma_f32_variant<float, int>(p, batch, Choice{})) return false;
   return 1.1 * split_path_seconds(p, batch) < gather;
+}
+
+// What a call that goes this way wants of workspace; 0: it does not.
+inline size_t split_path_bytes(const SpmmParams& p, int batch, bool forced) {
+  if (!split_path_fits(p) || (!forced && !split_path_wins(p, batch))) return 0;
+  const size_t bytes = split_plan(p, batch).bytes;
+  return bytes <= kSplitWorkspaceMost ? bytes : 0;
 }
 
 // Behind the product: adds the parts of K up (bias, ReLU), or where an operand holds an infinity or a NaN, which a product of parts (and of the
@@ -975,34 +987,42 @@ __global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, co
   }
 }
 
-inline int launch_split_path(const SpmmParams& p, int batch, void* workspace, hipStream_t stream) {
-  const SplitPlan s = split_plan(p, batch);
+inline int launch_split_path(const SpmmParams& whole, int batch, void* workspace, hipStream_t stream) {
+  const SplitPlan s = split_plan(whole, batch);
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   unsigned* ranges = reinterpret_cast<unsigned*>(ws);
   float* sums = reinterpret_cast<float*>(ws + s.sums_at);
-  const long long plane_a = (long long)p.m * s.kp, plane_b = (long long)s.kp * s.np;
-  const SplitSparse a{p.m, s.kp, p.row_offsets, static_cast<const int*>(p.cols), static_cast<const float*>(p.values), plane_a, ws + s.a_at};
-  const SplitDense b{batch, p.k, p.n, static_cast<const float*>(p.dense), s.kp, s.np, s.np, 3 * plane_b, plane_b, ws + s.b_at};
-  if (int rc = launch_split_operands(a, b, ranges, stream)) return rc;
-  SplitParams g{};
-  g.M = p.m, g.N = p.n, g.K = s.kp;
-  g.A = ws + s.a_at, g.B = ws + s.b_at;
-  g.lda = s.kp, g.ldb = s.np;
-  g.plane_a = (unsigned)(plane_a * 2), g.plane_b = (unsigned)(plane_b * 2);
-  g.stride_b = 3 * plane_b;
-  if (s.parts > 1) {
-    g.C = sums, g.ldc = s.ld, g.stride_c = (long long)p.m * s.ld, g.stride_part = g.stride_c * batch;
-  } else {
-    g.C = static_cast<float*>(p.out), g.ldc = p.n, g.stride_c = (long long)p.m * p.n;
-    g.row_bias = p.bias, g.relu = p.relu;
+  const long long plane_a = (long long)whole.m * s.kp, plane_b = (long long)s.kp * s.np;
+  const SplitSparse a{whole.m, s.kp, whole.row_offsets, static_cast<const int*>(whole.cols), static_cast<const float*>(whole.values), plane_a, ws + s.a_at};
+  for (int first = 0; first < batch; first += s.group) {   // (A's planes stay; the other room is each group's in turn)
+    const int entries = std::min(s.group, batch - first);
+    SpmmParams p = whole;
+    p.dense = static_cast<const float*>(whole.dense) + (size_t)first * p.k * p.n;
+    p.out = static_cast<float*>(whole.out) + (size_t)first * p.m * p.n;
+    const SplitDense b{entries, p.k, p.n, static_cast<const float*>(p.dense), s.kp, s.np, s.np, 3 * plane_b, plane_b, ws + s.b_at};
+    if (int rc = first == 0 ? launch_split_operands(a, b, ranges, stream) : launch_split_operand(b, ranges, stream)) return rc;
+    SplitParams g{};
+    g.M = p.m, g.N = p.n, g.K = s.kp;
+    g.A = ws + s.a_at, g.B = ws + s.b_at;
+    g.lda = s.kp, g.ldb = s.np;
+    g.plane_a = (unsigned)(plane_a * 2), g.plane_b = (unsigned)(plane_b * 2);
+    g.stride_b = 3 * plane_b;
+    g.parts = s.parts;
+    if (s.parts > 1) {
+      g.C = sums, g.ldc = s.ld, g.stride_c = (long long)p.m * s.ld, g.stride_part = g.stride_c * entries;
+    } else {
+      g.C = static_cast<float*>(p.out), g.ldc = p.n, g.stride_c = (long long)p.m * p.n;
+      g.row_bias = p.bias, g.relu = p.relu;
+    }
+    g.ranges = ranges, g.slots_a = split_sparse_blocks(a), g.slots_b = split_dense_blocks(b), g.finite = 1;
+    if (int rc = gemm_split(g, false, entries, stream)) return rc;
+    note_kernel("spmm_split_finish_kernel");
+    const int tiles = ceil_div(p.n, kWave * 4);
+    hipLaunchKernelGGL(spmm_split_finish_kernel, dim3((unsigned)std::min<long long>(kFinishBlocks, (long long)p.m * tiles * entries)), dim3(256), 0, stream, p, ranges, sums,
+                       s.parts, s.ld, tiles, entries);
+    if (int rc = check_hip(hipGetLastError(), "spmm (fp32 by parts) launch")) return rc;
   }
-  g.ranges = ranges, g.slots_a = split_sparse_blocks(a), g.slots_b = split_dense_blocks(b), g.finite = 1;
-  if (int rc = gemm_split(g, false, batch, stream)) return rc;
-  note_kernel("spmm_split_finish_kernel");
-  const int tiles = ceil_div(p.n, kWave * 4);
-  hipLaunchKernelGGL(spmm_split_finish_kernel, dim3((unsigned)std::min<long long>(kFinishBlocks, (long long)p.m * tiles * batch)), dim3(256), 0, stream, p, ranges, sums,
-                     s.parts, s.ld, tiles, batch);
-  return check_hip(hipGetLastError(), "spmm (fp32 by parts) launch");
+  return 0;
 }
 
 template <typename T, typename IT>
@@ -1026,10 +1046,10 @@ int launch_typed(const SpmmParams& p, int batch, const Choice& given, hipStream_
     return launch_smallk<T, IT>(p, batch, stream);
   }
   if constexpr (std::is_same<T, float>::value && std::is_same<IT, int>::value) {
-    const bool room = ch.ws && aligned(ch.ws, 256);
-    if ((ch.variant == 12 || (ch.variant == 0 && !ch.beside_gather)) && room && split_path_fits(p) && (ch.variant == 12 || split_path_wins(p, batch)) &&
-        ch.ws_bytes >= split_plan(p, batch).bytes)
-      return launch_split_path(p, batch, ch.ws, stream);
+    if ((ch.variant == 12 || (ch.variant == 0 && !ch.beside_gather)) && ch.ws && aligned(ch.ws, 256)) {
+      const size_t need = split_path_bytes(p, batch, ch.variant == 12);
+      if (need && ch.ws_bytes >= need) return launch_split_path(p, batch, ch.ws, stream);
+    }
     if (const int arr = mfma_f32_variant<T, IT>(p, batch, ch)) {
       const bool split = ch.lpg != 8;   // (lanes-per-group code 8 = no role split, for tuning)
       // (a row's windows are the kernel's own affair; numbers that it never had are refused)
@@ -1213,9 +1233,9 @@ static size_t workspace_plan(int dtype, int itype, int flags, int m, int k, int 
   if (dtype == IEX_F32 && itype == IEX_I32 && (variant == 0 || variant == 12)) {
     const SpmmParams p{m, k, n, nonzeros, nullptr, nullptr, nullptr, nullptr, some_aligned, nullptr, some_aligned,
                        (flags & IEX_SPMM_PER_BATCH_VALUES) != 0, (flags & IEX_SPMM_ACCUMULATE) != 0, (flags & IEX_SPMM_RELU) != 0, (flags & IEX_SPMM_PAD_OPERANDS) != 0};
-    if (!split_path_fits(p) || (variant == 0 && ((flags & IEX_SPMM_BESIDE_GATHER_KERNEL) || !split_path_wins(p, batch)))) return 0;
-    *kind = 12;
-    return split_plan(p, batch).bytes;
+    const size_t bytes = variant == 0 && (flags & IEX_SPMM_BESIDE_GATHER_KERNEL) ? 0 : split_path_bytes(p, batch, variant == 12);
+    if (bytes) *kind = 12;
+    return bytes;
   }
   if (!(dtype == IEX_F16 || dtype == IEX_BF16) || !(itype == IEX_I32 || itype == IEX_I16)) return 0;
   if (variant != 0 && variant != 7 && variant != 10) return 0;

@@ -146,6 +146,31 @@ def test_where_it_is_taken_and_where_not():
     assert torch.equal(ops.spmm_sputnik_reuse_weight(shifted, row_indices, values, row_offsets, columns, 2048), taken)
 
 
+def test_a_batch_in_groups():
+    """The workspace does not grow with the batch: groups of entries share the room, the last one smaller; an infinity sends its own group to the row kernel."""
+    m, k, n, batch = 256, 8192, 4096, 6              # planes of an entry: 201 MB, so two at a time
+    w, csr, b = operands(m, k, n, 0.2, batch, seed=13)
+    size = lambda batch: _lib.load().iex_spmm_workspace_bytes(_lib.F32, _lib.I32, _lib.SPMM_PAD_OPERANDS | 12 << 16, m, k, n, csr[0].numel(), batch)
+    assert size(2) == size(6) == size(5000) > size(1)
+    b[3, 5, 7] = float("inf")
+    got = product(csr, b, m, 12)
+    assert _lib.last_kernels().count("gemm_split_kernel") == 3
+    for z in (0, 1, 4, 5):
+        assert error(got[z], w, b[z]) < 1.2e-7
+    assert torch.equal(got[3:4].isfinite(), product(csr, b[3:4].contiguous(), m, 1).isfinite())
+    uneven = product(csr, b[2:5].contiguous(), m, 12)     # two and one
+    assert torch.equal(uneven[2], got[4]) and error(uneven[2], w, b[4]) < 1.2e-7
+
+
+def test_no_more_workspace_than_its_bound():
+    size = lambda m, k, n, batch=1: _lib.load().iex_spmm_workspace_bytes(_lib.F32, _lib.I32, _lib.SPMM_PAD_OPERANDS | 12 << 16, m, k, n, m * k // 5, batch)
+    of_sddmm = lambda m, n, k: _lib.load().iex_sddmm_workspace_bytes(_lib.F32, _lib.SDDMM_PAD_OPERANDS | 12 << 16, m, k, n, m * n // 5, 1)
+    most = 4 << 30
+    for shape in ((4096, 4096, 4096, 64), (4096, 4096, 2048, 384), (11008, 4096, 8192, 64), (20000, 20000, 512)):
+        assert 0 < size(*shape) <= most
+    assert size(26000, 26000, 4096) == 0 and 0 < of_sddmm(11008, 4096, 32768) <= most and of_sddmm(30000, 30000, 16384) == 0
+
+
 def test_captured_and_replayed_between_other_work():
     w, csr, b = operands(1500, 2100, 600, 0.25, seed=6)
     values, row_indices, row_offsets, columns = csr
