@@ -203,6 +203,15 @@ Tensor workspace(size_t bytes, const Tensor& like) {
   return bytes ? at::empty({(int64_t)bytes}, like.options().dtype(at::kByte)) : Tensor();
 }
 
+// ... that a call can do without: nothing where there is no memory for it
+Tensor optional_workspace(size_t bytes, const Tensor& like) {
+  try {
+    return workspace(bytes, like);
+  } catch (const c10::OutOfMemoryError&) {
+    return Tensor();
+  }
+}
+
 // ---- SpMM ----------------------------------------------------------------------------------------------------------
 enum class Spmm { kSharedF32, kSharedHalf, kPerEntry, kAtomic };
 
@@ -259,10 +268,10 @@ Tensor spmm_call(const Tensor& b, const Tensor& row_indices, const Tensor& value
     use_tables(ws, known->tables_stream, column_indices, capturing());
     flags |= IEX_SPMM_TABLES_READY | IEX_SPMM_LISTS_READY;
   } else {
-    ws = workspace(ws_bytes, b);
+    ws = optional_workspace(ws_bytes, b);
   }
   if (aux.defined()) {
-    if (!plain(aux, 3 - flat) || aux.sizes() != out_shape || aux.scalar_type() != b.scalar_type() || aux.device() != b.device()) return Tensor();
+    if ((ws_bytes && !ws.defined()) || !plain(aux, 3 - flat) || aux.sizes() != out_shape || aux.scalar_type() != b.scalar_type() || aux.device() != b.device()) return Tensor();
     check(iex_spmm_aux(dtype, itype, flags, m, k, n, nonzeros, row_indices.const_data_ptr<int>(), values.const_data_ptr(),
                        row_offsets.const_data_ptr<int>(), column_indices.const_data_ptr(), b.const_data_ptr(), aux.const_data_ptr(), aux_mode,
                        out.data_ptr(), stream_of(b), batch, ws.defined() ? ws.data_ptr() : nullptr, ws_bytes,
@@ -317,7 +326,7 @@ Tensor sddmm(const Tensor& a, const Tensor& b, const Tensor& row_indices, const 
     use_tables(ws, known->tables_stream, column_indices, capturing());
     flags |= IEX_SDDMM_TABLES_READY | IEX_SDDMM_LISTS_READY;
   } else {
-    ws = workspace(ws_bytes, a);
+    ws = optional_workspace(ws_bytes, a);
   }
   check(iex_sddmm_ws(dtype, flags, m, k, n, nonzeros, row_indices.const_data_ptr<int>(), row_offsets.const_data_ptr<int>(),
                      column_indices.const_data_ptr<int>(), a.const_data_ptr(), b.const_data_ptr(), out.data_ptr(), stream_of(a), batch,
@@ -355,7 +364,7 @@ Tensor gemm(const Tensor& a, const Tensor& b, bool trans_b) {
   const c10::DeviceGuard guard(a.device());
   Tensor out = batched ? at::empty({batch, M, N}, a.options()) : at::empty({M, N}, a.options());
   const size_t ws_bytes = iex_gemm_workspace_bytes(dtype, trans_b, M, N, K, batch);
-  const Tensor ws = workspace(ws_bytes, a);
+  const Tensor ws = optional_workspace(ws_bytes, a);
   check(iex_gemm_ws(dtype, trans_b, M, N, K, a.const_data_ptr(), b.const_data_ptr(), out.data_ptr(), batch, a.dim() == 3 ? M * K : 0,
                     b.dim() == 3 ? N * K : 0, M * N, stream_of(a), ws.defined() ? ws.data_ptr() : nullptr, ws_bytes),
         "gemm");
@@ -372,7 +381,7 @@ Tensor gemm_transposed_a(const Tensor& a, const Tensor& b) {
   const c10::DeviceGuard guard(a.device());
   Tensor out = at::empty({M, N}, a.options());
   const size_t ws_bytes = iex_gemm_workspace_bytes(dtype, 2, M, N, K, 1);
-  const Tensor ws = workspace(ws_bytes, a);
+  const Tensor ws = optional_workspace(ws_bytes, a);
   check(iex_gemm_ws(dtype, 2, M, N, K, a.const_data_ptr(), b.const_data_ptr(), out.data_ptr(), 1, 0, 0, 0, stream_of(a),
                     ws.defined() ? ws.data_ptr() : nullptr, ws_bytes),
         "gemm");
@@ -531,7 +540,7 @@ struct WeightForm {
       form = layout.memory;
     }
     const size_t ws_bytes = iex_form_product_workspace_bytes(kind, m, k, n);
-    const Tensor ws = workspace(ws_bytes, x);
+    const Tensor ws = optional_workspace(ws_bytes, x);
     Tensor out = at::empty({m, n}, x.options());
     check(iex_form_product(dtype, kind, m, k, n, room, form.const_data_ptr(), x.const_data_ptr(), aux ? aux->const_data_ptr() : nullptr, mode,
                            out.data_ptr(), ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, stream_of(x)),
@@ -635,7 +644,8 @@ Tensor transposed_product(const Tensor& grad, const Tensor& values, const Tensor
   const auto known = note_of(row_offsets, column_indices, k);
   if (!bytes || !known || known->status != 0) return Tensor();   // (canonical CSR only)
   const c10::DeviceGuard guard(grad.device());
-  const Tensor ws = workspace(bytes, grad);
+  const Tensor ws = optional_workspace(bytes, grad);
+  if (!ws.defined()) return Tensor();
   Tensor out = at::empty({k, n}, grad.options());
   check(iex_spmm_transposed(dtype, column_indices.scalar_type() == at::kShort ? IEX_I16 : IEX_I32, m, k, n, nonzeros, values.const_data_ptr(),
                             row_offsets.const_data_ptr<int>(), column_indices.const_data_ptr(), grad.const_data_ptr(), out.data_ptr(), stream_of(grad),

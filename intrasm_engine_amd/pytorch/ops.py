@@ -162,6 +162,16 @@ def _dense_share_host(row_offsets, column_indices, k, dense_min=None):
     return int(count.item()) / nonzeros
 
 
+def _optional_workspace(nbytes, device, flags):
+    """Memory that a call can do without, None where there is none; a kernel asked for by name (``flags``) gets it or the allocator's error."""
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+    except torch.OutOfMemoryError:
+        if (flags >> 16) & 0xf:
+            raise
+        return None
+
+
 def _table_memory(nbytes, device):
     """Memory for tables that outlive the call: it is the current stream's, which the allocator has to be told where they
     are used on another one (:func:`_use_tables`)."""
@@ -557,7 +567,7 @@ def _spmm(b, row_indices, values, row_offsets, column_indices, m, *, per_batch_v
                 ws = tables
                 flags |= _lib.SPMM_TABLES_READY | _lib.SPMM_LISTS_READY
             else:
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=b.device) if ws_bytes else None
+                ws = _optional_workspace(ws_bytes, b.device, flags)
         # what is known about the pattern's row lengths (only what an earlier look left, unless the kernel that needs
         # it was asked for by name)
         if ((flags >> 16) & 0xf) == 11 and nonzeros > 0:
@@ -697,7 +707,7 @@ def _sddmm(a, b, row_indices, row_offsets, column_indices, *, sum_over_batch, dt
                 ws = tables
                 flags |= _lib.SDDMM_TABLES_READY | _lib.SDDMM_LISTS_READY
             else:
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
+                ws = _optional_workspace(ws_bytes, a.device, flags)
         rc = lib.iex_sddmm_ws(
             _DT[a.dtype], flags, m, k, n, nonzeros, row_indices.data_ptr(), row_offsets.data_ptr(),
             column_indices.data_ptr(), a.data_ptr(), b.data_ptr(), out.data_ptr(),
@@ -824,7 +834,7 @@ def gemm_mfma(a, b, trans_b=False, out=None):
         code = int(bool(trans_b)) | ((int(tile) & 0x1f) << 4)
         # room for the partial sums where the library would split K over two workgroups per tile (few tiles, long K)
         ws_bytes = lib.iex_gemm_workspace_bytes(_DT[a.dtype], code, M, N, K, batch)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
+        ws = _optional_workspace(ws_bytes, a.device, 0)
         rc = lib.iex_gemm_ws(_DT[a.dtype], code, M, N, K, a.data_ptr(), b.data_ptr(), out.data_ptr(), batch, sa, sb, M * N,
                              _stream_ptr(a.device), ws.data_ptr() if ws is not None else None, ws_bytes)
     _lib.check(rc, "gemm")

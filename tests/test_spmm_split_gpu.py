@@ -171,6 +171,41 @@ def test_no_more_workspace_than_its_bound():
     assert size(26000, 26000, 4096) == 0 and 0 < of_sddmm(11008, 4096, 32768) <= most and of_sddmm(30000, 30000, 16384) == 0
 
 
+def test_without_memory_for_the_workspace():
+    """Where the allocator has none left for it, the operators run on the kernels that take none, as they did before there were parts."""
+    m, k, n = 6144, 8192, 512
+    w, csr, b = operands(m, k, n, 0.2, seed=14)
+    values, row_indices, row_offsets, columns = csr
+    lhs, rhs = torch.randn(1, m, n, device="cuda"), torch.randn(1, k, n, device="cuda")
+    calls = {"native spmm": lambda: ops.spmm_sputnik_reuse_weight(b, row_indices, values, row_offsets, columns, m), "spmm": lambda: product(csr, b, m),
+             "native sddmm": lambda: ops.sddmm_sputnik_atomic_upd_weight(lhs, rhs, row_indices, row_offsets, columns),
+             "sddmm": lambda: pyops._sddmm(lhs, rhs, row_indices, row_offsets, columns, sum_over_batch=True, dtypes=(torch.float32,))}
+    want = {}
+    for name, call in calls.items():
+        want[name] = call().cpu()
+        assert "gemm_split_kernel" in _lib.last_kernels(), name
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    held = []
+    try:   # everything taken in pieces, one of them left for the results: nowhere room for the 360 MB of planes
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (256 << 20)) / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            while len(held) < 1000:
+                held.append(torch.empty(48 << 20, dtype=torch.uint8, device="cuda"))
+        held.pop()
+        for name, call in calls.items():
+            got = call()
+            assert "split" not in _lib.last_kernels(), name
+            assert float((got.cpu() - want[name]).norm() / want[name].norm()) < 2e-6, name
+            del got
+        with pytest.raises(torch.OutOfMemoryError):
+            product(csr, b, m, 12)
+    finally:
+        held.clear()
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
 def test_captured_and_replayed_between_other_work():
     w, csr, b = operands(1500, 2100, 600, 0.25, seed=6)
     values, row_indices, row_offsets, columns = csr
