@@ -240,7 +240,7 @@ int iex_spmm_sched(int dtype, int itype, int flags, int m, int k, int n, int non
                    const int* row_histogram);
 /* What that workspace would hold: 0 = nothing (not used), 7 = the dense form of A,
  * 10 = the tables and lists of family 10 (functions of the pattern only: a caller that keeps the workspace for a
- * pattern may say so with IEX_SPMM_TABLES_READY / IEX_SPMM_LISTS_READY on later calls). */
+ * pattern may say so with IEX_SPMM_TABLES_READY / IEX_SPMM_LISTS_READY on later calls), 12 = the parts of an fp32 product. */
 int iex_spmm_workspace_kind(int dtype, int itype, int flags, int m, int k, int n, int nonzeros, int batch);
 
 /* iex_spmm_ws for callers that cannot allocate device memory (code under hipGraph capture, tight serving
@@ -249,7 +249,8 @@ int iex_spmm_workspace_kind(int dtype, int itype, int flags, int m, int k, int n
  * IEX_SPMM_STATIC_SCRATCH_BYTES that the library itself holds on every GPU it runs on, from the moment the
  * library is loaded there until the process ends.  The call allocates and frees nothing (the first call on a
  * device looks the array's address up once).  A call whose workspace would exceed the array fails with
- * IEX_ERR_TOO_LARGE before anything is launched; a call that would not use a workspace runs as iex_spmm_ex.
+ * IEX_ERR_TOO_LARGE before anything is launched; a call that would not use a workspace runs as iex_spmm_ex, and so does
+ * every fp32 call that does not force family 12 (its bits are those of iex_spmm_ex, and it does not touch the array).
  * All calls on one GPU share that GPU's array: two calls whose work may overlap in time (different streams,
  * different threads) race on it -- order them, or give one of them iex_spmm_ws with memory of its own.  The
  * array keeps the previous call's contents; every kernel that reads it writes what it reads first

@@ -1223,7 +1223,7 @@ int spmm_dispatch(int dtype, int itype, int flags, int m, int k, int n, int nonz
 // Bytes of workspace with which iex_spmm_ws would take the dense-form path for this call (0: it
 // would not, whatever the workspace).  Pointers are taken to be 16-byte aligned.
 // kind: which family the workspace would serve (0 = none, 7 = dense form, 9 = partial sums of the k split, 10 = the
-// tables and lists of the dense-blocks kernel).
+// tables and lists of the dense-blocks kernel, 12 = the planes and sums of the fp32 product by parts).
 static size_t workspace_plan(int dtype, int itype, int flags, int m, int k, int n, int nonzeros, int batch, int* kind) {
   *kind = 0;
   if (m <= 0 || k <= 0 || n <= 0 || nonzeros <= 0 || batch <= 0) return 0;
@@ -1369,9 +1369,9 @@ int iex_spmm_static(int dtype, int itype, int flags, int m, int k, int n, int no
   // every call shares the array with whatever ran before it: nothing in it counts as "still there"
   flags &= ~(IEX_SPMM_TABLES_READY | IEX_SPMM_LISTS_READY);
   const size_t need = spmm_workspace_bytes(dtype, itype, flags, m, k, n, nonzeros, batch);
-  // a call that would not touch a workspace runs as iex_spmm_ex does (a forced family 7 fails there), and so does an fp32 one whose parts
-  // the array does not hold: the other families take none
-  if (need == 0 || (dtype == IEX_F32 && ((flags >> 16) & 0xf) == 0 && need > kStaticScratchBytes))
+  // a call that would not touch a workspace runs as iex_spmm_ex does (a forced family 7 fails there), and so does an fp32 one that does not ask for
+  // the product by parts: programs run such calls side by side, which the shared array would make a race
+  if (need == 0 || (dtype == IEX_F32 && ((flags >> 16) & 0xf) == 0))
     return spmm_dispatch(dtype, itype, flags, m, k, n, nonzeros, row_indices, values, row_offsets, column_indices, dense,
                          bias, out, stream, batch, nullptr, 0);
   IEX_REQUIRE(need <= kStaticScratchBytes, IEX_ERR_TOO_LARGE,

@@ -234,3 +234,18 @@ def test_static_scratch_too_small_for_the_parts(dev):
     _lib.check(lib.iex_spmm_static(_lib.F32, _lib.I32, _lib.SPMM_PAD_OPERANDS, m, k, n, columns.numel(), row_indices.data_ptr(), values.data_ptr(), row_offsets.data_ptr(),
                                    columns.data_ptr(), b.data_ptr(), None, out.data_ptr(), torch.cuda.current_stream().cuda_stream, 1), "static")
     assert "split" not in _lib.last_kernels() and error(out, w, b) < 2e-6
+
+
+def test_static_scratch_is_not_for_parts_that_it_would_hold(dev):
+    """iex_spmm_static's array is shared by all calls on the GPU.  fp32 calls never used it: programs may run them side by side."""
+    m, k, n = 2048, 2048, 512
+    w, csr, b = operands(m, k, n, 0.2, seed=7)
+    values, row_indices, row_offsets, columns = csr
+    lib, out, want = _lib.load(), torch.empty(1, m, n, device="cuda"), torch.empty(1, m, n, device="cuda")
+    assert 0 < lib.iex_spmm_workspace_bytes(_lib.F32, _lib.I32, _lib.SPMM_PAD_OPERANDS, m, k, n, columns.numel(), 1) <= lib.iex_spmm_static_scratch_bytes()
+    args = lambda out: (_lib.F32, _lib.I32, _lib.SPMM_PAD_OPERANDS, m, k, n, columns.numel(), row_indices.data_ptr(), values.data_ptr(), row_offsets.data_ptr(),
+                        columns.data_ptr(), b.data_ptr(), None, out.data_ptr(), torch.cuda.current_stream().cuda_stream, 1)
+    _lib.check(lib.iex_spmm_static(*args(out)), "static")
+    assert "split" not in _lib.last_kernels() and error(out, w, b) < 2e-6
+    _lib.check(lib.iex_spmm_ex(*args(want)), "plain")
+    assert torch.equal(out, want)
