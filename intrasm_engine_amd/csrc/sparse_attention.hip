@@ -6,10 +6,12 @@ namespace {
 
 // Entries of a 128 x 64 tile from which it counts as dense (fewer where only some groups of 32 rows have entries there).  A tile costs the matrix-core
 // path about 1100 (16-bit) and 8200 (fp32, HD = 64) clocks of a wavefront for 32 rows, an entry on its own about 20 and 40 beside its two rows from L2.  (16
-// heads x 1500 tokens, 175 scattered entries per tile, fp16: 45 us from 128 on, 30 from 224 on.  262 per tile, bf16, us from 224 / 288 / 512 on: 4 x 1000
-// of 128 20.5 / 14.4 / 13.1, 32 x 1000 of 32 21.8 / 17.3 / 16.4, of 64 27.2 / 25.2 / 24.8, of 128 42.7 / 43.5 / 43.5; 327 per tile, 32 x 800 of 128 37.8 / 37.9 / 41.5;
-// 655, 4 x 400 of 64 8.5 / - / 12.3.  8 x 1000, 260 per tile, fp32: 28 from 224 on, 22 from 400 on.)
+// heads x 1500 tokens, 175 scattered entries per tile, fp16: 45 us from 128 on, 30 from 224 on.  262 per tile, bf16, us from 224 / 288 / 448 on: 4 x 1000
+// of 128 20.4 / 13.8 / 12.7, 32 x 1000 of 32 20.8 / 16.3 / 15.5, of 64 25.8 / 24.2 / 23.2; 327 per tile, 32 x 800 of 128 36.9 / 36.9 / 39.6;
+// 655, 4 x 400 of 64 8.2 / 9.4 / 11.9.  8 x 1000, 260 per tile, fp32: 28 from 224 on, 22 from 400 on.)
 inline int dense_min(int dtype) { return dtype == IEX_F32 ? 800 : 288; }
+// ... and from which some launches take it for dense all the same (SparseAttentionShape::takes_either)
+inline int either_min(int dtype) { return dtype == IEX_F32 ? 800 : 224; }
 
 template <int TYPE, int HD, int QW, int KW>
 int launch(const SparseAttentionParams& p, hipStream_t stream) {
@@ -65,7 +67,7 @@ extern "C" int iex_mask_tables(int dtype, int m, int n, int nonzeros, const int*
   const MaskTables t = mask_tables_layout(m, n, nonzeros);
   note_kernel("mask_tables_kernel");
   hipLaunchKernelGGL(mask_tables_kernel, dim3(t.blocks), dim3(kMtWaves * kWave), mask_tables_lds_bytes(t.tiles), static_cast<hipStream_t>(stream), m, n,
-                     nonzeros, dense_min(dtype), row_offsets, column_indices, static_cast<unsigned char*>(tables));
+                     nonzeros, dense_min(dtype), either_min(dtype), row_offsets, column_indices, static_cast<unsigned char*>(tables));
   return check_hip(hipGetLastError(), "mask tables launch");
 }
 

@@ -8,6 +8,8 @@
 //
 // The mask's tables (made once per mask by mask_tables_kernel): per block of 128 rows the 64-column tiles that hold at
 // least dense_min / 4 entries for each group of 32 rows that has any there ("dense"), for each of them a 64-bit word per row, and per row the columns outside dense tiles.
+// Which tiles are better off as dense ones is not the same for every launch, and the tables are made before one is known: those between two limits stand at the
+// end of the list, their entries at the end of the rows' lists, and a launch takes them one way or the other.
 // A wavefront owns 32 queries, a workgroup QW wavefronts (fewer where the heads are few: more workgroups, and fewer tiles
 // that only some of its wavefronts want), or KW wavefronts share 32 queries, each with every KW-th tile and stages of its own
 // (8 heads x 1000 tokens, fp32: 27.8 -> 16 us), with more wavefronts beside them that do nothing but the other entries: their chains run
@@ -30,19 +32,21 @@ namespace iex {
 
 constexpr int kMaRows = 128, kMaCols = 64, kMaMaxTokens = 16384;
 constexpr int kMaEntries = 1 << 31;
+constexpr int kMaEither = 1 << 30;
 
 // Where the parts of a mask's tables lie in their memory.  They hold all that the kernel reads of the mask: a recorded launch
 // works on the mask as it was, whatever becomes of the index arrays.
 struct MaskTables {
   int blocks, tiles;            // blocks of 128 rows, tiles of 64 columns
-  size_t list, thin, thin_cols, bits, bytes;   // byte offsets and the total
+  size_t list, ends, thin, thin_cols, bits, bytes;   // byte offsets and the total
 };
 inline __host__ __device__ MaskTables mask_tables_layout(int m, int n, int nnz) {
   MaskTables t;
   t.blocks = (m + kMaRows - 1) / kMaRows;
   t.tiles = (n + kMaCols - 1) / kMaCols;
   t.list = 0;                                                              // int [blocks][tiles + 1]: how many; tile | wavefronts of 32 rows << 16
-  t.thin = (t.list + (size_t)t.blocks * (t.tiles + 1) * 4 + 7) / 8 * 8;    // int2 [blocks * 128]: where a row's begin (kMaEntries: it has entries); how many
+  t.ends = t.list + (size_t)t.blocks * (t.tiles + 1) * 4;                  // for launches that take the tiles at the list's end: int [blocks]: how many tiles; [blocks * 128]: how many entries of a row
+  t.thin = (t.ends + (size_t)t.blocks * (1 + kMaRows) * 4 + 7) / 8 * 8;    // int2 [blocks * 128]: where a row's begin (kMaEntries: it has entries); how many
   t.thin_cols = t.thin + (size_t)t.blocks * kMaRows * 8;                   // int [nnz]: row r's from row_offsets[r]
   t.bits = (t.thin_cols + (size_t)nnz * 4 + 255) / 256 * 256;              // u64 [blocks][tiles][128]: by position in the list
   t.bytes = t.bits + (size_t)t.blocks * t.tiles * kMaRows * 8;
@@ -53,16 +57,17 @@ inline __host__ __device__ MaskTables mask_tables_layout(int m, int n, int nnz) 
 constexpr int kMtWaves = 16;
 inline __host__ __device__ int mask_tables_lds_bytes(int tiles) { return tiles * 3 * 4 + kMtWaves * tiles * 8; }
 
-__global__ __launch_bounds__(kMtWaves * kWave) void mask_tables_kernel(int m, int n, int nnz, int dense_min, const int* __restrict__ row_offsets,
+__global__ __launch_bounds__(kMtWaves * kWave) void mask_tables_kernel(int m, int n, int nnz, int dense_min, int either_min, const int* __restrict__ row_offsets,
                                                                        const int* __restrict__ cols, unsigned char* __restrict__ ws) {
   extern __shared__ __align__(16) int mt_smem[];
   const MaskTables t = mask_tables_layout(m, n, nnz);
   const int tiles = t.tiles, rb = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int* count = mt_smem;             // [tiles]: entries; then the tile's position in the list, or -1
+  int* count = mt_smem;             // [tiles]: entries; then the tile's position in the list (| kMaEither), or -1
   int* groups = count + tiles;      // [tiles]: bit g: rows 32 g .. 32 g + 31 have entries there
   int* dense = groups + tiles;      // [tiles]: the list
   unsigned* map = reinterpret_cast<unsigned*>(dense + tiles) + wave * tiles * 2;   // [tiles * 2]: this wavefront's row, a bit per column
   int* list = reinterpret_cast<int*>(ws + t.list) + (size_t)rb * (tiles + 1);
+  int* ends = reinterpret_cast<int*>(ws + t.ends);
   int2* thin_of = reinterpret_cast<int2*>(ws + t.thin) + (size_t)rb * kMaRows;
   int* thin_cols = reinterpret_cast<int*>(ws + t.thin_cols);
   unsigned long long* bits = reinterpret_cast<unsigned long long*>(ws + t.bits) + (size_t)rb * tiles * kMaRows;
@@ -87,33 +92,40 @@ __global__ __launch_bounds__(kMtWaves * kWave) void mask_tables_kernel(int m, in
   }
   __syncthreads();
   if (wave == 0) {   // the list, in the order of the tiles
-    int had = 0;
-    for (int base = 0; base < tiles; base += kWave) {
-      const int tile = base + lane;
-      // (a tile costs every group of 32 rows that has entries there: a band's corner with entries of one group is worth it from a quarter on; fp32, 8 x 1544 of
-      // 32, band 512 + 16 scattered, 31.5 -> 23 us, 16 x 1179 of 64, band 64, 33.8 -> 27.7)
-      const bool is = tile < tiles && 4 * count[tile] >= dense_min * __popc((unsigned)groups[tile]) && count[tile] > 0;
-      const unsigned long long them = __ballot(is);
-      if (tile < tiles) count[tile] = -1;
-      if (is) {
-        const int at = had + __popcll(them & ((1ull << lane) - 1));
-        count[tile] = at;
-        dense[at] = tile;
-        list[1 + at] = tile | (groups[tile] << 16);
+    int had = 0, certain = 0;
+    for (int pass = 0; pass < 2; ++pass) {   // dense for all, for some
+      for (int base = 0; base < tiles; base += kWave) {
+        const int tile = base + lane;
+        // (a tile costs every group of 32 rows that has entries there: a band's corner with entries of one group is worth it from a quarter on; fp32, 8 x 1544 of
+        // 32, band 512 + 16 scattered, 31.5 -> 23 us, 16 x 1179 of 64, band 64, 33.8 -> 27.7)
+        const int there = tile < tiles ? count[tile] : 0, of = tile < tiles ? __popc((unsigned)groups[tile]) : 0;
+        const bool is = pass ? there == -2 : there > 0 && 4 * there >= dense_min * of;
+        const unsigned long long them = __ballot(is);
+        if (is) {
+          const int at = had + __popcll(them & ((1ull << lane) - 1));
+          count[tile] = at | (pass ? kMaEither : 0);
+          dense[at] = tile;
+          list[1 + at] = tile | (groups[tile] << 16);
+        } else if (pass == 0 && tile < tiles) {
+          count[tile] = there > 0 && 4 * there >= either_min * of ? -2 : -1;
+        }
+        had += __popcll(them);
       }
-      had += __popcll(them);
+      if (pass == 0) certain = had;
     }
     if (lane == 0) {
-      list[0] = had;
-      groups[0] = had;   // (the groups are done)
+      list[0] = certain;
+      ends[rb] = had;
+      groups[0] = certain | had << 16;   // (the groups are done)
     }
   }
   __syncthreads();
-  const int nd = groups[0];
+  const int nd = groups[0] >> 16;
+  const bool either_way = nd > (groups[0] & 0xffff);
   for (int r = wave; r < kMaRows; r += kMtWaves) {
     const int row = rb * kMaRows + r;
     for (int i = lane; i < 2 * tiles; i += kWave) map[i] = 0;
-    int thin = 0, begin = 0;
+    int thin = 0, both = 0, begin = 0;
     if (row < m) {
       const int start = row_offsets[row], end = row_offsets[row + 1];
       begin = start | (start < end ? kMaEntries : 0);
@@ -125,8 +137,17 @@ __global__ __launch_bounds__(kMtWaves * kWave) void mask_tables_kernel(int m, in
         if (to_thin) thin_cols[start + thin + __popcll(them & ((1ull << lane) - 1))] = col;
         thin += __popcll(them);
       }
+      both = thin;
+      if (either_way)
+        for (int j0 = start; j0 < end; j0 += kWave) {
+          const int j = j0 + lane, col = j < end ? cols[j] : -1;
+          const bool either = col >= 0 && count[col >> 6] >= kMaEither;
+          const unsigned long long them = __ballot(either);
+          if (either) thin_cols[start + both + __popcll(them & ((1ull << lane) - 1))] = col;
+          both += __popcll(them);
+        }
     }
-    if (lane == 0) thin_of[r] = int2{begin, thin};
+    if (lane == 0) thin_of[r] = int2{begin, both}, ends[t.blocks + rb * kMaRows + r] = thin;
     __builtin_amdgcn_wave_barrier();   // (the LDS operations of one wavefront execute in order)
     for (int s = lane; s < nd; s += kWave) {
       const int tile = dense[s];
@@ -161,6 +182,10 @@ struct SparseAttentionShape {
   }
   // wavefronts beside those KW, for the scattered entries alone
   static constexpr int extra(int kw) { return kw == 1 ? 0 : kw == 2 ? 6 : 4; }
+  // Tiles that may be taken either way as dense ones: where the same wavefronts do the other entries afterwards, 16 lanes to each.  (16-bit, us as entries / as tiles: 32 heads x 533 of 128,
+  // band 256 + 16 scattered 26.8 / 23.8; 32 x 677 of 128, causal, 64 + 32 35.6 / 30.7; 32 x 1000 of 128, 64 + 32 41.6 / 42.1, of 64 24.3 / 25.8, of 32 16.3 / 20.8; lists beside
+  // the tiles: 4 x 1000 of 128 13.8 / 20.4, 32 x 500 of 128 19.5 / 24.0, 12 x 1266 of 128 26.7 / 29.1)
+  static constexpr bool takes_either(int kw) { return kw == 1 && HD == 128; }
 };
 
 // LDS row of a key (or chunk permutation of a row): what keeps the operand reads of 16 consecutive lanes apart.
@@ -212,6 +237,7 @@ __global__ __launch_bounds__((QW * KW + SparseAttentionShape<TYPE, HD>::extra(KW
   constexpr int ES = Shape::ES, KEYS = Shape::KEYS, CPR = Shape::CPR, TILE = Shape::TILE, TLD = Shape::TLD;
   constexpr bool F32 = TYPE == 2;
   constexpr int XW = Shape::extra(KW);              // (wavefronts KW .. KW + XW - 1)
+  constexpr bool TAKE = Shape::takes_either(KW);    // tiles that are dense for some as dense ones
   constexpr int PER = kMaCols / KEYS;               // stages per tile of the mask
   constexpr int KB = KEYS / 32, DT = HD / 32;       // blocks of 32 keys, of 32 features
   constexpr int RPI = kWave / CPR;                  // rows per direct load
@@ -238,6 +264,7 @@ __global__ __launch_bounds__((QW * KW + SparseAttentionShape<TYPE, HD>::extra(KW
   const unsigned char* v = static_cast<const unsigned char*>(p.v) + at;
   const MaskTables mt = mask_tables_layout(T, T, p.nnz);
   const int* __restrict__ list = reinterpret_cast<const int*>(p.tables + mt.list) + (size_t)rb * (mt.tiles + 1);
+  const int* __restrict__ ends = reinterpret_cast<const int*>(p.tables + mt.ends);
   const unsigned char* bits = p.tables + mt.bits + ((size_t)rb * mt.tiles * kMaRows + (group0 + wave) * 32) * 8;
   const unsigned lds0 = (unsigned)(size_t)(lds_u8*)stages;
   const u32x4 k_buf = buffer_of(k, (size_t)T * HD * ES), v_buf = buffer_of(v, (size_t)T * HD * ES);   // (rows past the end: zeros)
@@ -346,7 +373,7 @@ __global__ __launch_bounds__((QW * KW + SparseAttentionShape<TYPE, HD>::extra(KW
 
   // ---- dense tiles that any of this workgroup's rows have entries in
   if (XW == 0 || kw < KW) {
-    const int count = uniform(list[0]), mine = ((1 << QW) - 1) << group0;
+    const int count = uniform(TAKE ? ends[rb] : list[0]), mine = ((1 << QW) - 1) << group0;
     int entry = 0;   // of the tile that `next` has found
     auto next = [&](int i) {
       while (i < count && (i % KW != kw || !(((entry = uniform(list[1 + i])) >> 16) & mine))) ++i;
@@ -377,7 +404,8 @@ __global__ __launch_bounds__((QW * KW + SparseAttentionShape<TYPE, HD>::extra(KW
   const int row0 = q0 + wave * 32;
   const int my_row = min(row0 + col, T - 1);
   const int2* thin_of = reinterpret_cast<const int2*>(p.tables + mt.thin);
-  const int my_count = row0 + col < T ? thin_of[my_row].y : 0;
+  auto thin_count = [&](int row) { return TAKE ? ends[mt.blocks + row] : thin_of[row].y; };
+  const int my_count = row0 + col < T ? thin_count(my_row) : 0;
   if (__ballot(my_count > 0)) {   // (uniform)
     constexpr int G = kWave / CPR, U = HD * ES >= 256 ? 4 : 8, E = 16 / ES;
     typedef int i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -386,7 +414,7 @@ __global__ __launch_bounds__((QW * KW + SparseAttentionShape<TYPE, HD>::extra(KW
     for (int r0 = (kw + XW) % (KW + XW) * G; r0 < 32; r0 += (KW + XW) * G) {
       const int row = row0 + r0 + sub, safe = min(row, T - 1);
       const int2 thin = thin_of[safe];
-      const int count = row < T ? thin.y : 0;
+      const int count = row < T ? TAKE ? thin_count(safe) : thin.y : 0;
       const int* at_cols = thin_cols + (thin.x & ~kMaEntries);   // (what follows the columns in the tables may be read, not used)
       int most = count;   // of the G rows
 #pragma unroll
@@ -519,7 +547,7 @@ __global__ __launch_bounds__((QW * KW + SparseAttentionShape<TYPE, HD>::extra(KW
       const unsigned these = todo >> r0 & (unsigned)((1ull << G) - 1);
       if (!these) continue;   // (uniform)
       if (these >> sub & 1) {
-        const int r = r0 + sub, row = row0 + r, nd = list[0], nt = thin_of[row].y, first = thin_of[row].x & ~kMaEntries;
+        const int r = r0 + sub, row = row0 + r, nd = TAKE ? ends[rb] : list[0], nt = thin_count(row), first = thin_of[row].x & ~kMaEntries;
         const u32x4 qv = *reinterpret_cast<const u32x4*>(q + ((size_t)row * CPR + part) * 16);
         auto entries = [&](auto each) {   // (the same for the CPR lanes of a row)
           for (int i = 0; i < nd; ++i) {

@@ -78,6 +78,32 @@ def test_lists_beside_tiles_that_few_rows_have(dev, dtype, tol, d, tokens, group
     assert np.linalg.norm(out.float().cpu().numpy() - want) <= tol * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("dtype, tol", [(torch.float16, 2e-3), (torch.float32, 1e-5)])
+def test_tiles_that_a_launch_takes_one_way_or_the_other(dev, dtype, tol):
+    """About 245 entries a tile, between the two limits of 16-bit tables: one mask, launches of either kind and heads of all sizes; an infinity stays with the rows
+    that attend to it."""
+    rng = np.random.default_rng(11)
+    tokens = 533
+    mask = _mask(tokens, 8, 16, rng)
+    mask[100:130] = _mask(tokens, 8, 0, rng)[100:130]     # rows without scattered entries among them
+    ro, ci, _ = W.csr_from_mask(mask)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    ri, ro, ci = t(W.swizzle_from_offsets(ro)), t(ro), t(ci)
+    for heads, d, wide in ((64, 128, True), (2, 128, False), (64, 64, True), (2, 64, False), (2, 32, False)):
+        q, k, v = (rng.standard_normal((2, tokens, d)).astype(np.float32) for _ in range(3))
+        operands = [t(x).to(dtype).repeat(heads // 2, 1, 1) for x in (q, k, v)]
+        out = sparse_attention(*operands, ri, ro, ci)
+        assert f", {d}, {4 if wide else 1}, " in _lib.last_kernels(), _lib.last_kernels()
+        want = _reference(mask, *(rounded(x, dtype).astype(np.float64) for x in (q, k, v)))
+        assert np.linalg.norm(out[-2:].float().cpu().numpy() - want) <= tol * np.linalg.norm(want)
+        assert torch.equal(out[:2], out[-2:])
+        operands[2][:, 300, 3] = float("inf")
+        odd = sparse_attention(*operands, ri, ro, ci)
+        assert torch.equal(odd[-1].isfinite().all(dim=1), t(~mask[:, 300]))
+        rest = ~mask[:, 300]
+        assert np.linalg.norm(odd[-1].float().cpu().numpy()[rest] - want[-1][rest]) <= tol * np.linalg.norm(want[-1][rest])
+
+
 def test_tables_follow_the_mask(dev):
     """A mask changed in place is looked at again; one that nobody may look at, and columns in another order, go by three kernels."""
     from intrasm_engine_amd.pytorch import ops as pyops
