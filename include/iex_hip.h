@@ -227,11 +227,14 @@ size_t iex_spmm_workspace_bytes(int dtype, int itype, int flags, int m, int k, i
  * sums of a row meet in LDS in a fixed order (no atomics: same bits from call to call).  The histogram and the
  * order of row_indices settle how many wavefronts a row HAS; into how many parts its sum is cut follows from the
  * row's own length, and a row with fewer wavefronts than parts lets one of them take all the parts.  So every row is
- * summed completely, and to the same bits, whatever the histogram and whatever the order of row_indices: a wrong
+ * summed completely, whatever the histogram and whatever the order of row_indices: a wrong
  * histogram or another order costs time only.  IEX_SPMM_FORCE_VARIANT(11) asks for this kernel and fails without a histogram
  * (bits 20..23 then force the chunks of 64 nonzeros a wavefront may get: 1 + log2, 0 = choose).
  * Where many rows fill the chip as it is, workgroups of four wavefronts serve one long row or four others each, n of no whole vectors too (family 11 with four
- * waves per row forced), to the same promise.  With nothing forced the histogram settles which of these arrangements runs, or one number for all rows.
+ * waves per row forced).
+ * Bits: another order of row_indices changes none.  With family 11 and its limit forced neither does another histogram; with nothing forced
+ * the histogram (or that there is none) settles which of these arrangements runs, with which limit, or one number of wavefronts for all rows, and
+ * with it how a row's sum is cut: same bits for the same histogram, last bits of fp32 sums for others.
  * No counterpart in the reference. */
 int iex_spmm_sched(int dtype, int itype, int flags, int m, int k, int n, int nonzeros,
                    const int* row_indices, const void* values, const int* row_offsets,

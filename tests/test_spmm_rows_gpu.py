@@ -129,6 +129,23 @@ def test_order_of_rows_and_histogram_change_no_bit(dev, sparsity, n):
         assert torch.equal(_call(c, dev, b_np, torch.float32, torch.int32, 11 << 16, hist), base)
 
 
+@pytest.mark.parametrize("m,k,n,sparsity", [(2048, 1024, 64, 0.9), (4500, 600, 128, 0.9), (1100, 2000, 512, 0.85), (2100, 1500, 130, 0.95)])
+def test_with_nothing_forced_the_histogram_settles_the_bits_and_the_order_does_not(oracle, dev, m, k, n, sparsity):
+    """Several nonzeros per gather and one, whole vectors and ragged rows: another order of the rows changes no bit, another histogram (the rule may then cut
+    the sums another way) or none at all leaves every row complete."""
+    c = W.config2_matrix(sparsity, m=m, k=k, seed=21)
+    rng = np.random.default_rng(22)
+    b_np = rng.standard_normal((1, k, n)).astype(np.float32)
+    want = oracle.spmm(b_np, c.row_indices, c.values, c.row_offsets, c.column_indices, c.m)
+    scale = oracle.spmm_abs_scale(b_np, c.row_indices, c.values, c.row_offsets, c.column_indices, c.m)
+    true_hist = _histogram(c.row_offsets)
+    for hist in (true_hist, [0] * 16, [m] * 16, [m, m // 2, 3] + [0] * 13, None):
+        base = _call(c, dev, b_np, torch.float32, torch.int32, 0, hist)
+        assert_close(base.cpu().numpy(), want, scale, 1e-5, f"histogram {hist and hist[:3]}")
+        for order in (rng.permutation(m).astype(np.int32), c.row_indices[::-1].copy()):
+            assert torch.equal(_call(c, dev, b_np, torch.float32, torch.int32, 0, hist, row_indices=order), base), hist and hist[:3]
+
+
 def test_forcing_it_without_a_histogram_is_refused(dev):
     c = W.config2_matrix(0.9, m=64, k=256, seed=1)
     ri, v, ro, ci = to_dev(c, dev)
