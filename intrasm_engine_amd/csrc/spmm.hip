@@ -932,9 +932,10 @@ inline bool split_path_wins(const SpmmParams& p, int batch) {
   const double columns = p.n <= 128 ? narrow : p.n - last + (last == 0 ? 0 : last <= 208 ? 216 : 256);
   const double gather = 5e-6 + (double)p.nnz * columns * batch * 4 / ((double)p.k * std::min(p.n, 256) > 1.1e6 ? 25e12 : 30e12);
   if (gather < 30e-6) return false;   // (what three launches and a short product take)
-  // Up to 256 columns the fp32 matrix-core kernel keeps the calls that its density rule gives it, although they are shorter this way (4096 x 4096, n = 256, 70 %
-  // 116 / 86): whoever looks at the names of the kernels finds that one there.
-  if (p.n <= 256 && mfma_f32_variant<float, int>(p, batch, Choice{})) return false;
+  // One tile of 128 columns is what the fp32 matrix-core kernel is good at, and it makes no copies: up to there it keeps the calls that its density rule gives it; from
+  // two tiles on they are shorter this way.  Us, that kernel / this way, n = 128 and n = 256: 8000 x 1000 at 60 % 30.8 / 41.8, 59 / 49; 11008 x 4096 at 72 %
+  // 171 / 164, 255 / 225; 4096 x 4096 at 72 % (n = 256, its 32-row tiles) 86 / 75, at 30 % 109 / 85; 4096 x 11008 at 72 % 220 / 214.
+  if (p.n <= 128 && mfma_f32_variant<float, int>(p, batch, Choice{})) return false;
   return 1.1 * split_path_seconds(p, batch) < gather;
 }
 
