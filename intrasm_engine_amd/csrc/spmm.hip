@@ -948,7 +948,8 @@ inline size_t split_path_bytes(const SpmmParams& p, int batch, bool forced) {
 
 // Behind the product: adds the parts of K up (bias, ReLU), or where an operand holds an infinity or a NaN, which a product of parts (and of the
 // dense form's zeros) spreads, or entries outside the range in which parts hold all 24 bits, computes it as the row kernel does, in as many workgroups as the
-// chip holds: results there are the row kernel's.  With K in one part it ends at once else (2 us).  Us a call, 4096 x 4096 at 80 %, n = 256 / at 90 %, n = 1024: row
+// chip holds: results there are the row kernel's.  Rows of one nonzero are its product, rounded once (by parts 2.59e-8 off in the 2-norm and 9.1e-8 at most, instead
+// of 2.53e-8 and 6.0e-8; rows of two and more are closer by parts).  With K in one part it ends at once else (2 us).  Us a call, 4096 x 4096 at 80 %, n = 256 / at 90 %, n = 1024: row
 // kernel 122 / 238, by parts 77 / 178, one infinity 159 / 394 (with the product computed all the same, and this kernel in 256 workgroups where K is in one part, 204 / 556).
 constexpr int kFinishBlocks = 1024;
 __global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, const unsigned* ranges, const float* sums, int parts, int ld, int tiles, int batch) {
@@ -960,18 +961,14 @@ __global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, co
       spmm_block<float, int, 4, kWave, 4, kSpmmUnroll, 1, true>(p, row, rest % tiles, rest / tiles, red);
       __syncthreads();
     }
-  } else if (parts > 1) {
+  } else {
     typedef float four __attribute__((ext_vector_type(4)));
     typedef four any4 __attribute__((aligned(4)));
     const int chunks = ld / 4;
     const size_t rows = (size_t)p.m * batch, part = rows * ld;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < rows * chunks; i += (size_t)gridDim.x * 256) {
-      const size_t zr = i / chunks;
-      const int c = (int)(i - zr * chunks) * 4;
-      const float* from = sums + zr * ld + c;
-      four x = *reinterpret_cast<const four*>(from);
-      for (int s = 1; s < parts; ++s) x += *reinterpret_cast<const four*>(from + s * part);
-      if (p.bias) x += p.bias[zr % p.m];
+    const int* cols = static_cast<const int*>(p.cols);
+    auto finish = [&](size_t zr, int row, int c, four x) {
+      if (p.bias) x += p.bias[row];
       if (p.relu) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) x[e] = fmaxf(x[e], 0.f);
@@ -983,6 +980,36 @@ __global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, co
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           if (c + e < p.n) out[e] = x[e];
+      }
+    };
+    // (a row of one nonzero: n >= 4, so the last chunk is read a few columns early)
+    auto alone = [&](size_t zr, int start, int c) {
+      const int at = min(c, p.n - 4), shift = c - at;
+      const four b = *reinterpret_cast<const any4*>(static_cast<const float*>(p.dense) + ((zr / p.m) * p.k + cols[start]) * p.n + at);
+      const float v = static_cast<const float*>(p.values)[start];
+      four x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = v * (shift == 0 ? b[e] : shift == 1 ? b[min(e + 1, 3)] : shift == 2 ? b[min(e + 2, 3)] : b[3]);
+      return x;
+    };
+    if (parts > 1) {
+      for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < rows * chunks; i += (size_t)gridDim.x * 256) {
+        const size_t zr = i / chunks;
+        const int c = (int)(i - zr * chunks) * 4, row = (int)(zr % p.m), start = p.row_offsets[row], end = p.row_offsets[row + 1];
+        const float* from = sums + zr * ld + c;
+        four x = *reinterpret_cast<const four*>(from);
+        for (int s = 1; s < parts; ++s) x += *reinterpret_cast<const four*>(from + s * part);
+        if (end - start == 1) x = alone(zr, start, c);
+        finish(zr, row, c, x);
+      }
+    } else {   // (the product has written all rows; those of one nonzero once more, by the wavefront that finds them)
+      for (size_t first = ((size_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kWave; first < rows; first += (size_t)gridDim.x * 4 * kWave) {
+        const size_t mine = min(first + lane_id(), rows - 1);
+        const int row = (int)(mine % p.m), start = p.row_offsets[row], end = p.row_offsets[row + 1];
+        for (unsigned long long them = __ballot(first + lane_id() < rows && end - start == 1); them; them &= them - 1) {
+          const int src = __ffsll(them) - 1, r = bcast_i(row, src), at = bcast_i(start, src);
+          for (int c = lane_id() * 4; c < p.n; c += kWave * 4) finish(first + src, r, c, alone(first + src, at, c));
+        }
       }
     }
   }

@@ -101,6 +101,22 @@ def test_entries_outside_the_range_of_the_parts(of_values, of_dense):
     assert error(got, w, b) <= max(1.05 * error(want, w, b), 1.2e-7)
 
 
+# (K in one part and in several; last chunks of one, two and three columns; more than a wavefront's columns)
+@pytest.mark.parametrize("m,k,n,batch", [(200, 320, 133, 2), (130, 4100, 262, 1), (70, 64, 4, 3), (300, 96, 519, 1)])
+def test_rows_of_one_nonzero_are_rounded_once(m, k, n, batch):
+    w, _, b = operands(m, k, n, 0.2, batch, seed=15)
+    w[1::3] = 0
+    w[torch.arange(1, m, 3), torch.randint(0, k, (len(range(1, m, 3)),))] = torch.randn(len(range(1, m, 3)), device="cuda")
+    csr, bias = dense_to_sparse(w), torch.randn(m, device="cuda")
+    got, want = product(csr, b, m, 12), torch.matmul(w.double(), b.double())
+    assert "gemm_split_kernel" in _lib.last_kernels()
+    one = (csr[2][1:] - csr[2][:-1] == 1).nonzero().view(-1)
+    assert len(one) >= m // 3 and torch.equal(got[:, one], want[:, one].float())
+    assert error(got, w, b) < 1.2e-7
+    with_bias = product(csr, b[:1].contiguous(), m, 12, bias=bias, relu=True)
+    assert torch.equal(with_bias[:, one], (want[:1, one].float() + bias[one, None]).relu())
+
+
 @pytest.mark.parametrize("of_rows,of_columns", [(-126, 0), (0, -126), (-64, -64), (-110, 0)])
 def test_rows_and_columns_of_widely_different_scales(of_rows, of_columns):
     """Every row and column from 1 down to 2^of_rows and 2^of_columns in steps of two powers: each result beside its own row's and column's scale."""
