@@ -161,11 +161,13 @@ int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream);
  * 11 = the row kernel with wavefronts per row by the row's own length (iex_spmm_sched only: see there); with four waves per row
  * forced too: a wavefront per row, four for rows of more than 64 << (code of bits 20..23 less one) nonzeros.
  * 12 = fp32 by parts: every entry of A's dense form and of the dense operand as three bf16 parts that hold all its 24 bits, the
- * six products of parts that reach into an fp32 result on the bf16 matrix cores (iex_spmm_ws only; chosen by itself for
- * large fp32 products with IEX_SPMM_PAD_OPERANDS, values shared by the batch, plain store, canonical CSR).  Its error against 64 bits is below that of a chain of
- * fp32 multiply-adds (2-norm, rows of two nonzeros and more; of a product alone, 2.6e-8 against 2.5e-8: rows of one nonzero are computed as that).  Where an operand holds an infinity or a NaN, or its entries are too large or small for the parts to be exact
- * (a magnitude but zero outside 2^-110 .. 2^126, a product of two outside 2^-120 .. 2^90), the row kernel computes the call
- * instead.  Where it cannot run (no workspace, other types) the row kernel does.
+ * six products of parts that reach into an fp32 result on the bf16 matrix cores (iex_spmm_ws and iex_spmm_sched; chosen by itself for
+ * large fp32 products with IEX_SPMM_PAD_OPERANDS, values shared by the batch, plain store, canonical CSR).  Error against 64 bits
+ * (2-norm, normal entries), by parts / by the row kernel: rows of 800 nonzeros 8.6e-8 / 2.6e-7, of 128 6.6e-8 / 1.1e-7, of 32
+ * 6.2e-8 / 6.7e-8, of 8 5.3e-8 / 5.4e-8, of two 3.6e-8 / 3.1e-8; rows of one nonzero are that product, rounded once.  Where an
+ * operand holds an infinity or a NaN, or its entries are too large or small for the parts to be exact (a magnitude but zero
+ * outside 2^-110 .. 2^126, a product of two outside 2^-120 .. 2^90), the row kernel computes the call instead.  Where it cannot
+ * run (no workspace, other types) the row kernel does.
  * Families 2-6 and 10 rely on strictly ascending column indices inside a row (canonical CSR, what
  * dense_to_sparse produces); family 1 accepts any order and duplicates -- force it for such
  * input.  Families 3-6 and 10 multiply explicit zeros with the dense operand, so a non-finite entry

@@ -74,74 +74,56 @@ __device__ __forceinline__ SplitRange split_dense_block(const SplitDense& s, int
 
 // As csr_to_dense_kernel (spmm_dense_device.cuh): a workgroup per row, the row (or 4096 columns of it) assembled in LDS in fp32, its parts taken on
 // the way out, every byte written once.  (4096 x 4096: 27 us, of which 20 are the bytes; two rows side by side the same, four 40.)
-constexpr int kPlanesSeg = 4096, kPlanesRows = 1, kPlanesWaves = 4;
+constexpr int kPlanesSeg = 4096, kPlanesWaves = 4;
 __device__ __forceinline__ SplitRange split_sparse_block(const SplitSparse& s, int block, int blocks) {
-  __shared__ __align__(16) float srow[kPlanesRows][kPlanesSeg];
+  __shared__ __align__(16) float srow[kPlanesSeg];
   const int lane = lane_id(), wave = uniform(threadIdx.x >> 6);
   const int* __restrict__ cols = s.cols;
   const float* __restrict__ values = s.values;
   uint16_t* __restrict__ dst = static_cast<uint16_t*>(s.dst);
   SplitExtent range;
   bool again = false;
-  for (int slot0 = block * kPlanesRows; slot0 < s.m; slot0 += blocks * kPlanesRows) {
-    int pos[kPlanesRows], end[kPlanesRows];   // this wavefront's quarter of each row's nonzeros, in whole chunks of 64
-#pragma unroll
-    for (int r = 0; r < kPlanesRows; ++r) {
-      const int row = min(slot0 + r, s.m - 1);
-      const int first = uniform(s.row_offsets[row]), last = slot0 + r < s.m ? uniform(s.row_offsets[row + 1]) : first;
-      const int share = ((max(last - first, 0) + kWave * kPlanesWaves - 1) / (kWave * kPlanesWaves)) * kWave;
-      pos[r] = min(first + wave * share, last);
-      end[r] = min(pos[r] + share, last);
-    }
+  for (int row = block; row < s.m; row += blocks) {
+    // this wavefront's quarter of the row's nonzeros, in whole chunks of 64
+    const int first = uniform(s.row_offsets[row]), last = uniform(s.row_offsets[row + 1]);
+    const int share = ((max(last - first, 0) + kWave * kPlanesWaves - 1) / (kWave * kPlanesWaves)) * kWave;
+    int pos = min(first + wave * share, last);
+    const int end = min(pos + share, last);
     for (int c0 = 0; c0 < s.ld; c0 += kPlanesSeg) {
       const int len = min(kPlanesSeg, s.ld - c0);   // a multiple of 32
       if (again) __syncthreads();   // the previous segment has been copied out
       again = true;
-#pragma unroll
-      for (int r = 0; r < kPlanesRows; ++r)
-        for (int i = threadIdx.x * 4; i < len; i += kPlanesWaves * kWave * 4) *reinterpret_cast<f32x4*>(srow[r] + i) = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = threadIdx.x * 4; i < len; i += kPlanesWaves * kWave * 4) *reinterpret_cast<f32x4*>(srow + i) = f32x4{0.f, 0.f, 0.f, 0.f};
       __syncthreads();
-      bool more[kPlanesRows], any = false;
+      for (bool more = pos < end; more;) {
+        int c[4];
+        float v[4];
 #pragma unroll
-      for (int r = 0; r < kPlanesRows; ++r) any |= more[r] = pos[r] < end[r];
-      while (any) {
-        any = false;
-        int c[kPlanesRows][4];
-        float v[kPlanesRows][4];
-#pragma unroll
-        for (int r = 0; r < kPlanesRows; ++r)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int j = max(min(pos[r] + u * kWave + lane, end[r] - 1), 0);   // (a row without nonzeros: entry 0, never used)
-            c[r][u] = cols[j] - c0;
-            v[r][u] = values[j];
-          }
-#pragma unroll
-        for (int r = 0; r < kPlanesRows; ++r) {
-          int taken = 0;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            // (the test on c keeps a row whose columns do not ascend inside the row's slice of LDS)
-            const bool mine = more[r] && pos[r] + u * kWave + lane < end[r] && c[r][u] < len && c[r][u] >= 0;
-            if (mine) {
-              srow[r][c[r][u]] = v[r][u];
-              range.add(v[r][u]);
-            }
-            taken += __popcll(__ballot(mine));
-          }
-          pos[r] += taken;
-          any |= more[r] = taken == 4 * kWave;   // a short take: the quarter ended or its next nonzero lies beyond this segment
+        for (int u = 0; u < 4; ++u) {
+          const int j = min(pos + u * kWave + lane, end - 1);
+          c[u] = cols[j] - c0;
+          v[u] = values[j];
         }
+        int taken = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          // (the test on c keeps a row whose columns do not ascend inside the row's slice of LDS)
+          const bool mine = pos + u * kWave + lane < end && c[u] < len && c[u] >= 0;
+          if (mine) {
+            srow[c[u]] = v[u];
+            range.add(v[u]);
+          }
+          taken += __popcll(__ballot(mine));
+        }
+        pos += taken;
+        more = taken == 4 * kWave;   // a short take: the quarter ended or its next nonzero lies beyond this segment
       }
       __syncthreads();
-#pragma unroll
-      for (int r = 0; r < kPlanesRows; ++r)
-        if (slot0 + r < s.m)
-          for (int i = threadIdx.x * 8; i < len; i += kPlanesWaves * kWave * 8) {
-            const f32x4 lo = *reinterpret_cast<const f32x4*>(srow[r] + i), hi = *reinterpret_cast<const f32x4*>(srow[r] + i + 4);
-            const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            store_parts(x, dst + (size_t)(slot0 + r) * s.ld + c0 + i, s.plane);
-          }
+      for (int i = threadIdx.x * 8; i < len; i += kPlanesWaves * kWave * 8) {
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(srow + i), hi = *reinterpret_cast<const f32x4*>(srow + i + 4);
+        const float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        store_parts(x, dst + (size_t)row * s.ld + c0 + i, s.plane);
+      }
     }
   }
   return range.range();
@@ -310,7 +292,7 @@ int split_dense_blocks(const SplitDense& s) {
   const long long chunks = (long long)s.batch * s.dst_rows * (s.dst_cols / 8);
   return (int)std::min<long long>(kSplitSlots, (chunks + 255) / 256);
 }
-int split_sparse_blocks(const SplitSparse& s) { return std::min(kSplitSparseSlots, ceil_div(s.m, kPlanesRows)); }
+int split_sparse_blocks(const SplitSparse& s) { return std::min(kSplitSparseSlots, s.m); }
 int launch_split_operands(const SplitSparse& a, const SplitDense& b, unsigned* ranges, hipStream_t stream) {
   return launch_operands(a, split_sparse_blocks(a), b, ranges, stream);
 }

@@ -949,7 +949,7 @@ inline size_t split_path_bytes(const SpmmParams& p, int batch, bool forced) {
 // Behind the product: adds the parts of K up (bias, ReLU), or where an operand holds an infinity or a NaN, which a product of parts (and of the
 // dense form's zeros) spreads, or entries outside the range in which parts hold all 24 bits, computes it as the row kernel does, in as many workgroups as the
 // chip holds: results there are the row kernel's.  Rows of one nonzero are its product, rounded once (by parts 2.59e-8 off in the 2-norm and 9.1e-8 at most, instead
-// of 2.53e-8 and 6.0e-8; rows of two and more are closer by parts).  With K in one part it ends at once else (2 us).  Us a call, 4096 x 4096 at 80 %, n = 256 / at 90 %, n = 1024: row
+// of 2.53e-8 and 6.0e-8).  With K in one part it ends at once else (2 us).  Us a call, 4096 x 4096 at 80 %, n = 256 / at 90 %, n = 1024: row
 // kernel 122 / 238, by parts 77 / 178, one infinity 159 / 394 (with the product computed all the same, and this kernel in 256 workgroups where K is in one part, 204 / 556).
 constexpr int kFinishBlocks = 1024;
 __global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, const unsigned* ranges, const float* sums, int parts, int ld, int tiles, int batch) {
