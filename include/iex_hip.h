@@ -164,7 +164,7 @@ int iex_copy_bytes(void* dst, const void* src, size_t nbytes, void* stream);
  * six products of parts that reach into an fp32 result on the bf16 matrix cores (iex_spmm_ws and iex_spmm_sched; chosen by itself for
  * large fp32 products with IEX_SPMM_PAD_OPERANDS, values shared by the batch, plain store, canonical CSR).  Error against 64 bits
  * (2-norm, normal entries), by parts / by the row kernel: rows of 800 nonzeros 8.6e-8 / 2.6e-7, of 128 6.6e-8 / 1.1e-7, of 32
- * 6.2e-8 / 6.7e-8, of 8 5.3e-8 / 5.4e-8, of two 3.6e-8 / 3.1e-8; rows of one nonzero are that product, rounded once.  Where an
+ * 6.2e-8 / 6.7e-8, of 8 5.3e-8 / 5.4e-8; shorter ones are a chain of multiply-adds as in the row kernel.  Where an
  * operand holds an infinity or a NaN, or its entries are too large or small for the parts to be exact (a magnitude but zero
  * outside 2^-110 .. 2^126, a product of two outside 2^-120 .. 2^90), the row kernel computes the call instead.  Where it cannot
  * run (no workspace, other types) the row kernel does.

@@ -948,10 +948,12 @@ inline size_t split_path_bytes(const SpmmParams& p, int batch, bool forced) {
 
 // Behind the product: adds the parts of K up (bias, ReLU), or where an operand holds an infinity or a NaN, which a product of parts (and of the
 // dense form's zeros) spreads, or entries outside the range in which parts hold all 24 bits, computes it as the row kernel does, in as many workgroups as the
-// chip holds: results there are the row kernel's.  Rows of one nonzero are its product, rounded once (by parts 2.59e-8 off in the 2-norm and 9.1e-8 at most, instead
-// of 2.53e-8 and 6.0e-8).  With K in one part it ends at once else (2 us).  Us a call, 4096 x 4096 at 80 %, n = 256 / at 90 %, n = 1024: row
+// chip holds: results there are the row kernel's.  Rows of up to kFewNonzeros are a chain of multiply-adds: three of nine products of parts are left out, which the roundings of
+// a longer chain outweigh (2-norm against 64 bits, nonzeros far apart, by parts / by the row kernel: one 2.59e-8 / 2.53e-8, two 3.6e-8 / 3.1e-8, four 4.5e-8 / 4.0e-8, seven
+// 5.1e-8 / 5.1e-8, eight 5.3e-8 / 5.4e-8, 32 6.2e-8 / 6.7e-8).  16 x 2048 rows, n = 512, half of them of seven nonzeros: 197 -> 219 us.
+// With K in one part it ends at once else (2 us).  Us a call, 4096 x 4096 at 80 %, n = 256 / at 90 %, n = 1024: row
 // kernel 122 / 238, by parts 77 / 178, one infinity 159 / 394 (with the product computed all the same, and this kernel in 256 workgroups where K is in one part, 204 / 556).
-constexpr int kFinishBlocks = 1024;
+constexpr int kFinishBlocks = 1024, kFewNonzeros = 7;
 __global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, const unsigned* ranges, const float* sums, int parts, int ld, int tiles, int batch) {
   __shared__ float red[spmm_lds_floats<4, 4, 1>()];
   if (ranges[kSplitVerdict] == 0) {
@@ -982,16 +984,32 @@ __global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, co
           if (c + e < p.n) out[e] = x[e];
       }
     };
-    // (a row of one nonzero: n >= 4, so the last chunk is read a few columns early)
-    auto alone = [&](size_t zr, int start, int c) {
+    // (a short row: n >= 4, so the last chunk is read a few columns early)
+    auto chain = [&](size_t zr, int start, int end, int c) {
       const int at = min(c, p.n - 4), shift = c - at;
-      const four b = *reinterpret_cast<const any4*>(static_cast<const float*>(p.dense) + ((zr / p.m) * p.k + cols[start]) * p.n + at);
-      const float v = static_cast<const float*>(p.values)[start];
-      four x;
+      const float* dense = static_cast<const float*>(p.dense) + (zr / p.m) * p.k * p.n + at;
+      four x = {0.f, 0.f, 0.f, 0.f};
+      for (int j0 = start; j0 < end; j0 += 4) {   // (four gathers in flight; past the end the last one's row, which is not added)
+        four b[4];
+        float v[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = v * (shift == 0 ? b[e] : shift == 1 ? b[min(e + 1, 3)] : shift == 2 ? b[min(e + 2, 3)] : b[3]);
+        for (int u = 0; u < 4; ++u) {
+          const int j = min(j0 + u, end - 1);
+          b[u] = *reinterpret_cast<const any4*>(dense + (size_t)cols[j] * p.n);
+          v[u] = static_cast<const float*>(p.values)[j];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = j0 + u < end ? fmaf(v[u], b[u][e], x[e]) : x[e];
+        }
+      }
+      const four y = x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = shift == 0 ? y[e] : shift == 1 ? y[min(e + 1, 3)] : shift == 2 ? y[min(e + 2, 3)] : y[3];
       return x;
     };
+    auto few = [](int start, int end) { return start < end && end - start <= kFewNonzeros; };
     if (parts > 1) {
       for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < rows * chunks; i += (size_t)gridDim.x * 256) {
         const size_t zr = i / chunks;
@@ -999,16 +1017,18 @@ __global__ __launch_bounds__(256) void spmm_split_finish_kernel(SpmmParams p, co
         const float* from = sums + zr * ld + c;
         four x = *reinterpret_cast<const four*>(from);
         for (int s = 1; s < parts; ++s) x += *reinterpret_cast<const four*>(from + s * part);
-        if (end - start == 1) x = alone(zr, start, c);
+        if (few(start, end)) x = chain(zr, start, end, c);
         finish(zr, row, c, x);
       }
-    } else {   // (the product has written all rows; those of one nonzero once more, by the wavefront that finds them)
-      for (size_t first = ((size_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kWave; first < rows; first += (size_t)gridDim.x * 4 * kWave) {
-        const size_t mine = min(first + lane_id(), rows - 1);
-        const int row = (int)(mine % p.m), start = p.row_offsets[row], end = p.row_offsets[row + 1];
-        for (unsigned long long them = __ballot(first + lane_id() < rows && end - start == 1); them; them &= them - 1) {
-          const int src = __ffsll(them) - 1, r = bcast_i(row, src), at = bcast_i(start, src);
-          for (int c = lane_id() * 4; c < p.n; c += kWave * 4) finish(first + src, r, c, alone(first + src, at, c));
+    } else {   // (the product has written all rows; short ones once more.  A wavefront looks at rows far apart, 64 at a time: short ones may stand side by side)
+      const size_t waves = (size_t)gridDim.x * 4;
+      for (size_t first = (size_t)blockIdx.x * 4 + uniform(threadIdx.x >> 6); first < rows; first += waves * kWave) {
+        const size_t mine = first + lane_id() * waves;
+        const int row = (int)(min(mine, rows - 1) % p.m), start = p.row_offsets[row], end = p.row_offsets[row + 1];
+        for (unsigned long long them = __ballot(mine < rows && few(start, end)); them; them &= them - 1) {
+          const int src = __ffsll(them) - 1, r = bcast_i(row, src), from = bcast_i(start, src), to = bcast_i(end, src);
+          const size_t zr = first + src * waves;
+          for (int c = lane_id() * 4; c < p.n; c += kWave * 4) finish(zr, r, c, chain(zr, from, to, c));
         }
       }
     }

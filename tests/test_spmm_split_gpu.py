@@ -101,8 +101,9 @@ def test_entries_outside_the_range_of_the_parts(of_values, of_dense):
     assert error(got, w, b) <= max(1.05 * error(want, w, b), 1.2e-7)
 
 
-# (2-norms, measured: 2 nonzeros 3.6e-8 / 3.1e-8, 8 5.3e-8 / 5.4e-8, 32 6.2e-8 / 6.7e-8, 256 7.1e-8 / 1.5e-7; bound: a fifth above up to 64, below from 128 on)
-@pytest.mark.parametrize("per_row", [2, 8, 32, 128, 800])
+# (2-norms; rows of up to seven nonzeros are a chain as in the row kernel, longer ones gain by parts: 8 5.3e-8 / 5.4e-8, 32 6.2e-8 / 6.7e-8, 256 7.1e-8 / 1.5e-7.  Bound: the norm of
+# 512 x 512 roundings is known to 1 / sqrt(2 * 512 * 512) = 1.4e-3 of itself, seven times that)
+@pytest.mark.parametrize("per_row", [1, 2, 5, 7, 8, 16, 32, 128, 800])
 def test_error_beside_the_row_kernels_by_the_length_of_rows(per_row):
     m, k, n = 512, 2048, 512
     g = torch.Generator("cuda").manual_seed(per_row)
@@ -111,11 +112,11 @@ def test_error_beside_the_row_kernels_by_the_length_of_rows(per_row):
     b = torch.randn(1, k, n, device="cuda", generator=g)
     csr = dense_to_sparse(w)
     by_parts, by_rows = error(product(csr, b, m, 12), w, b), error(product(csr, b, m, 1), w, b)
-    assert by_parts < (1.2 * by_rows if per_row < 128 else by_rows), (by_parts, by_rows)
+    assert by_parts <= 1.01 * by_rows, (by_parts, by_rows)
 
 
 # (K in one part and in several; last chunks of one, two and three columns; more than a wavefront's columns)
-@pytest.mark.parametrize("m,k,n,batch", [(200, 320, 133, 2), (130, 4100, 262, 1), (70, 64, 4, 3), (300, 96, 519, 1)])
+@pytest.mark.parametrize("m,k,n,batch", [(200, 320, 133, 2), (130, 4100, 262, 1), (70, 64, 4, 3), (300, 96, 519, 1), (9000, 64, 12, 1)])
 def test_rows_of_one_nonzero_are_rounded_once(m, k, n, batch):
     w, _, b = operands(m, k, n, 0.2, batch, seed=15)
     w[1::3] = 0
